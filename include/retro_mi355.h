@@ -258,6 +258,47 @@ int ri_wave_attention_part_f16(const void* q, const void* steady_k, const void* 
                                int BG, int gs, int nc, int es, float scale, void* workspace,
                                size_t workspace_bytes, ri_stream_t stream);
 
+/* The decode step of one layer over a device-resident cluster store: ri_score_select, then ri_wave_attention, with
+ * everything but the query, the steady zone's length and the output in one struct (host memory, read during the call)
+ * that a caller fills once per layer (steps 1-8 of compute(), cache_hub/retroinfer_cache.py:549-697).  Fields are the
+ * arguments of those two entry points under the same names; `half` selects IEEE half instead of bfloat16. */
+typedef struct ri_decode_step_t {
+  const void* centroids;
+  const uint8_t* mask;
+  const int32_t* cluster_size_i32;
+  const int32_t* cluster_start;
+  float* logits;
+  int32_t* ret_ids;
+  int32_t* est_ids;
+  int32_t* ret_tok_off;
+  int32_t* ret_start;
+  int32_t* meta;
+  const void* steady_k;
+  const void* steady_v;
+  const int32_t* static_len_dev;
+  const void* store_k;
+  const void* store_v;
+  const void* value_sum;
+  const void* cluster_size;
+  int32_t* valid_lengths;
+  void* score_workspace;
+  void* attn_workspace;
+  int64_t steady_stride;
+  int64_t store_stride;
+  size_t score_workspace_bytes;
+  size_t attn_workspace_bytes;
+  int BG, gs, nc, np, es, page, max_pages, half;
+  float scale;
+} ri_decode_step_t;
+int ri_decode_step(const ri_decode_step_t* step, const void* q, int static_len, void* out, ri_stream_t stream);
+
+/* Appends one token's K and V to the steady zone (cache_hub/retroinfer_cache.py:541-542):
+ * steady_k[g, pos, :] = key[g, :] and steady_v[g, pos, :] = value[g, :] for the BG groups, rows of 128 16-bit
+ * elements, `steady_stride` rows per group.  With pos_dev (device, int64) the position is read when the kernel runs
+ * and `pos` is ignored; a position outside [0, steady_stride) then writes nothing. */
+int ri_append_kv(const void* key, const void* value, void* steady_k, void* steady_v, int64_t steady_stride,
+                 int64_t pos, const int64_t* pos_dev, int BG, ri_stream_t stream);
+
 /* ri_wave_attention for callers that cannot allocate device memory: code running under HIP stream
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.
  * Same arguments and result as ri_wave_attention without the workspace: the arrival counters and the

@@ -10,6 +10,17 @@ _lib = None
 
 P, I, I64, F, SZ = C.c_void_p, C.c_int, C.c_int64, C.c_float, C.c_size_t
 
+
+class DecodeStep(C.Structure):
+    """ri_decode_step_t"""
+    _fields_ = [(n, P) for n in (
+        "centroids", "mask", "cluster_size_i32", "cluster_start", "logits", "ret_ids", "est_ids", "ret_tok_off",
+        "ret_start", "meta", "steady_k", "steady_v", "static_len_dev", "store_k", "store_v", "value_sum", "cluster_size",
+        "valid_lengths", "score_workspace", "attn_workspace")] + [
+        ("steady_stride", I64), ("store_stride", I64), ("score_workspace_bytes", SZ), ("attn_workspace_bytes", SZ)] + [
+        (n, I) for n in ("BG", "gs", "nc", "np", "es", "page", "max_pages", "half")] + [("scale", F)]
+
+
 # name -> (restype, argtypes); mirrors include/retro_mi355.h
 SIGNATURES = {
     "ri_status_string": (C.c_char_p, [I]),
@@ -38,6 +49,8 @@ SIGNATURES = {
     "ri_wave_attention_static_f16": (I, [P, P, P, I64, I, P, P, P, I64, P, I, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, F, P]),
     "ri_buffer_attention": (I, [P, P, P, I64, P, I, P, P, P, P, P, I, I, I, I, F, P, SZ, P]),
     "ri_buffer_attention_f16": (I, [P, P, P, I64, P, I, P, P, P, P, P, I, I, I, I, F, P, SZ, P]),
+    "ri_decode_step": (I, [P, P, I, P, P]),
+    "ri_append_kv": (I, [P, P, P, P, I64, I64, P, I, P]),
     "ri_lru_access_update": (I, [P, P, P, I, P, I, P, P, I, P, I, P, P, P] + [P] * 12 + [P, I, I, P] + [I] * 6 + [P]),
     "ri_gather_copy_vectors": (I, [P, P, P, P, P, P, P, I, I, I, I, I, I, P]),
     "ri_gather_copy_and_concat": (I, [P] * 17 + [I] * 7 + [P]),

@@ -149,6 +149,8 @@ class retroinfer_cache(KV_Cache):
         self.cluster_start = [zeros((BG, n_centroids), torch.int32, dev(l)) for l in L]
         self.cluster_size_i32 = [zeros((BG, n_centroids), torch.int32, dev(l)) for l in L]
         self.store_rows = [[0] * BG for _ in L]  # rows of the store in use, per group
+        self._plans = {}                         # (layer, buffer) -> DecodeStepPlan of the device-resident step
+        self._row_shape = (batch_size, 1, self.kv_head, self.head_dim)
         self._centred_keys = {}                  # (device, tokens) -> buffer of centred keys for the clustering
         if self.kv_residency == "device":
             self._init_device_store()
@@ -469,6 +471,7 @@ class retroinfer_cache(KV_Cache):
                                                 km.counts.cpu().contiguous())
         torch.cuda.set_device(self.layer_mapping[str(0)])
         self.n_centroids += ncu
+        self._plans.clear()
         self.logits = torch.zeros((BG, self.group_size, self.n_centroids), dtype=torch.float32,
                                   device=self.layer_mapping[str(0)])
         self.static_pattern_total = sps + spe
@@ -492,6 +495,19 @@ class retroinfer_cache(KV_Cache):
         self.context += 1
         self.static_pattern_total += 1
 
+    def _append(self, key_states, value_states, layer_idx, pos_dev=None):
+        """The token's K and V rows into the steady zone with one launch; False when the rows are not as a layer hands
+        them over (another type, layout or shape, a full zone): torch's copies then convert, broadcast or raise."""
+        k, v = self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx]
+        for row, zone in ((key_states, k), (value_states, v)):
+            if not (row.is_cuda and row.dtype == zone.dtype and row.shape == self._row_shape and row.is_contiguous()
+                    and zone.is_contiguous() and row.data_ptr() % 16 == 0):
+                return False
+        if self.static_pattern_total >= k.shape[2]:
+            return False
+        kernels.append_kv(key_states, value_states, k, v, self.static_pattern_total, pos_dev)
+        return True
+
     def decode_update_kv_cache(self, key_states, value_states, layer_idx):
         """Appends the new token's K/V to the steady zone (reference: retroinfer_cache.py:527-546)."""
         last = layer_idx == self.layer_num - 1
@@ -499,15 +515,17 @@ class retroinfer_cache(KV_Cache):
             capturing = torch.cuda.is_current_stream_capturing()
             if not capturing:
                 self.prepare_token()
-            self.steady_zone_keys[layer_idx].index_copy_(2, self.steady_pos_dev, key_states.transpose(1, 2))
-            self.steady_zone_values[layer_idx].index_copy_(2, self.steady_pos_dev, value_states.transpose(1, 2))
+            if not self._append(key_states, value_states, layer_idx, self.steady_pos_dev):
+                self.steady_zone_keys[layer_idx].index_copy_(2, self.steady_pos_dev, key_states.transpose(1, 2))
+                self.steady_zone_values[layer_idx].index_copy_(2, self.steady_pos_dev, value_states.transpose(1, 2))
             # (the device-side position moves on after the last layer's attention, in compute())
             if last and not capturing:
                 self.token_replayed()
             return None, None
         self.prepare_token()
-        self.steady_zone_keys[layer_idx][:, :, self.static_pattern_total] = key_states[:, 0]
-        self.steady_zone_values[layer_idx][:, :, self.static_pattern_total] = value_states[:, 0]
+        if not self._append(key_states, value_states, layer_idx):
+            self.steady_zone_keys[layer_idx][:, :, self.static_pattern_total] = key_states[:, 0]
+            self.steady_zone_values[layer_idx][:, :, self.static_pattern_total] = value_states[:, 0]
         if last:
             self.context += 1
             self.static_pattern_total += 1
@@ -574,6 +592,11 @@ class retroinfer_cache(KV_Cache):
 
     def _compute_device(self, queries, layer_idx, static_len, buf):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
+        if queries.is_cuda and queries.dtype == self.dtype and queries.is_contiguous() and \
+                queries.numel() == BG * gs * D and not kernels.PROFILER_RANGES:
+            out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
+            self._plan(layer_idx, buf).run(queries, static_len, out)
+            return out
         self._select(queries, layer_idx, buf, True)
         out = torch.empty((BG, gs, D), dtype=self.dtype, device=queries.device)
         es = self.es_cluster_num
@@ -585,6 +608,26 @@ class retroinfer_cache(KV_Cache):
             ret_tok_off=self.ret_tok_off, ret_start=self.ret_start,
             static_len_dev=self.steady_len_dev if self.device_positions else None)
         return out.view(self.batch_size, 1, self.num_heads, D)
+
+    def _plan(self, layer, buf):
+        """The layer's step as one prepared call.  It is prepared again when any buffer has moved since (buffers are
+        attributes that the index growth and callers replace)."""
+        t = (self.centroids[layer], self.centroids_mask[layer], self.cluster_size_i32[layer], self.cluster_start[layer],
+             self.logits, self.ret_ids[buf], self.est_ids[buf], self.ret_tok_off, self.ret_start, self.meta,
+             self.steady_zone_keys[layer], self.steady_zone_values[layer], self.list_keys[layer],
+             self.list_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
+        key = [x.data_ptr() for x in t]
+        key += (self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size)
+        plan = self._plans.get((layer, buf))
+        if plan is None or not plan.valid(key):
+            names = ("centroids", "mask", "cluster_size_i32", "cluster_start", "logits", "ret_ids", "est_ids",
+                     "ret_tok_off", "ret_start", "meta", "steady_k", "steady_v", "store_k", "store_v", "value_sum",
+                     "cluster_size", "valid_lengths")
+            tensors = dict(zip(names, t), static_len_dev=self.steady_len_dev if self.device_positions else None)
+            plan = self._plans[(layer, buf)] = kernels.DecodeStepPlan(
+                key, self.dtype, tensors, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
+                self.RSQRT_DIM)
+        return plan
 
     def block_cache_stats(self, layer_idx):
         """(hit blocks, miss blocks) of the layer's last look-up, summed over the groups (host residency)."""

@@ -1,0 +1,51 @@
+// The decode step of one layer as two calls with few arguments (gfx950): appending the new token's K/V to the
+// steady zone, and scoring + selection + attention over a device-resident cluster store.
+//
+// A short context's step is bound by what the host spends on it, not by the GPU: through torch's slice copies and one
+// wrapper call per stage a layer-step took 46 us of host time, of which the launches are 1 us each.  The addresses and
+// sizes of a layer do not change from token to token, so the caller keeps them in one struct and hands over its address.
+#include "ri_common.h"
+
+// ------------------------------------------------------------------------------------
+// append: steady_k/v[g, pos] = key/value[g]; 16 lanes per 256-byte row, grid.y = K, V.
+// One launch for both tensors (a slice copy each: 2.4-4.9 us per launch); the row's position is an argument
+// or is read from the device, so that a captured call follows the position that the device keeps.
+// ------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void append_kernel(const uint4* __restrict__ key, const uint4* __restrict__ value,
+                                                     uint4* __restrict__ steady_k, uint4* __restrict__ steady_v,
+                                                     int64_t stride, int64_t pos, const int64_t* __restrict__ pos_dev,
+                                                     int BG) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int g = i >> 4, piece = i & 15;
+  if (g >= BG) return;
+  const uint4 v = (blockIdx.y ? value : key)[i];
+  if (pos_dev) pos = *pos_dev;
+  if (pos < 0 || pos >= stride) return;   // the steady zone is full: nothing is written past its end
+  (blockIdx.y ? steady_v : steady_k)[((size_t)g * stride + pos) * 16 + piece] = v;
+}
+
+extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, void* steady_v, int64_t steady_stride,
+                            int64_t pos, const int64_t* pos_dev, int BG, ri_stream_t stream) {
+  if (!key || !value || !steady_k || !steady_v || BG <= 0 || steady_stride <= 0) return RI_ERR_ARG;
+  if (!pos_dev && (pos < 0 || pos >= steady_stride)) return RI_ERR_ARG;
+  if (ri_any_misaligned16(key, value, steady_k, steady_v)) return RI_ERR_ARG;
+  append_kernel<<<dim3((BG * 16 + 255) / 256, 2), 256, 0, (hipStream_t)stream>>>(
+      (const uint4*)key, (const uint4*)value, (uint4*)steady_k, (uint4*)steady_v, steady_stride, pos, pos_dev, BG);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int static_len, void* out, ri_stream_t stream) {
+  if (!s) return RI_ERR_ARG;
+  auto* select = s->half ? ri_score_select_f16 : ri_score_select;
+  auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
+  const int rc = select(q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,
+                        s->ret_ids, s->est_ids, s->ret_tok_off, s->ret_start, nullptr, 0, s->meta, s->BG, s->gs, s->nc,
+                        s->np, s->es, s->page, s->max_pages, s->scale, s->score_workspace, s->score_workspace_bytes,
+                        stream);
+  if (rc) return rc;
+  return attend(q, s->steady_k, s->steady_v, s->steady_stride, static_len, s->static_len_dev, s->store_k, s->store_v,
+                s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta, s->est_ids,
+                s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out, s->valid_lengths, s->BG,
+                s->gs, s->nc, s->es, s->scale, s->attn_workspace, s->attn_workspace_bytes, stream);
+}

@@ -6,12 +6,13 @@ against the reference runs unchanged; the second block exposes the fused MI355X 
 Tensors only provide memory and the current stream; all arithmetic happens in the library.
 """
 import contextlib
+import ctypes
 import functools
 import math
 
 import torch
 
-from ._lib import lib, check
+from ._lib import DecodeStep, lib, check
 
 # 16-bit element types of the reference's operators and cache (batch_gemm_softmax.cu:185-197,
 # gather_copy.cu:63-67): every wrapper takes either and calls the entry point of that type (name or name_f16).
@@ -57,7 +58,9 @@ def _ranged(name):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """hipStream_t of the current device's current stream (torch.cuda.current_stream().cuda_stream without the
+    Stream object around it: 0.3 instead of 2.7 us of a decode step's host time)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
@@ -74,6 +77,7 @@ def _need(t, dtype, name, cuda=True):
 
 
 _workspaces = {}
+_workspace_generation = 0  # moves on whenever a scratch tensor is replaced: holders of an address look again
 _retired_workspaces = []   # superseded scratch tensors: captured HIP graphs may still hold their addresses
 
 
@@ -95,6 +99,8 @@ def _workspace(nbytes, device, tag):
             nbytes = max(nbytes, w.numel() * 3 // 2)
         w = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
         _workspaces[key] = w
+        global _workspace_generation
+        _workspace_generation += 1
     return w
 
 
@@ -381,6 +387,51 @@ def wave_attention(q, steady_k, steady_v, static_len, store_k, store_v, row_src,
                                   _p(est_centroids), _p(value_sum), _p(cluster_size_bf16), _p(out),
                                   _p(valid_lengths), BG, gs, nc, es, float(scale), _p(ws), ws.numel(), _stream()),
           "wave_attention")
+
+
+class DecodeStepPlan:
+    """score_select + wave_attention of one layer over a device-resident store as one call (ri_decode_step): the
+    addresses and sizes, which stay the same from token to token, are checked and laid down once.  `tensors`: the
+    fields of ri_decode_step_t that are addresses (None: not given); `key` is what the holder compares to see whether
+    they still are what it would hand over now."""
+
+    def __init__(self, key, dtype, tensors, nprobe, es, page, max_pages, scale):
+        c = tensors["centroids"]
+        BG, nc, _ = c.shape
+        gs = tensors["logits"].shape[1]
+        for nm in ("centroids", "steady_k", "steady_v", "store_k", "store_v", "value_sum", "cluster_size"):
+            _need(tensors[nm], dtype, nm)
+        device = c.device
+        tensors = dict(tensors,
+                       score_workspace=_workspace(lib().ri_score_select_workspace_bytes(BG, gs, nc), device, "score0"),
+                       attn_workspace=_workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), device, "attn0"))
+        self.key, self.generation = key, _workspace_generation
+        self._tensors = tensors
+        self._step = DecodeStep(
+            steady_stride=tensors["steady_k"].shape[-2], store_stride=tensors["store_k"].shape[-2],
+            score_workspace_bytes=tensors["score_workspace"].numel(),
+            attn_workspace_bytes=tensors["attn_workspace"].numel(), BG=BG, gs=gs, nc=nc, np=nprobe, es=es, page=page,
+            max_pages=max_pages, half=int(dtype == torch.float16), scale=scale,
+            **{nm: _p(t) for nm, t in tensors.items()})
+        self._address = ctypes.addressof(self._step)
+        self._call = lib().ri_decode_step
+
+    def valid(self, key):
+        return self.key == key and self.generation == _workspace_generation
+
+    def run(self, q, static_len, out):
+        status = self._call(self._address, q.data_ptr(), static_len, out.data_ptr(), _stream())
+        if status:
+            check(status, "decode_step")
+
+
+def append_kv(key, value, steady_k, steady_v, pos, pos_dev=None):
+    """steady[g, pos] = row g of key / value [BG, 128] (any shape of BG * 128 elements), one launch for both."""
+    stride = steady_k.shape[-2]
+    status = lib().ri_append_kv(key.data_ptr(), value.data_ptr(), steady_k.data_ptr(), steady_v.data_ptr(), stride, pos,
+                                _p(pos_dev), steady_k.numel() // (stride * 128), _stream())
+    if status:
+        check(status, "append_kv")
 
 
 @_ranged("flash_attention")
