@@ -17,6 +17,9 @@ __host__ __device__ __forceinline__ float ri_bf16_to_f32(uint16_t v) {
   return x.f;
 }
 __host__ __device__ __forceinline__ uint16_t ri_f32_to_bf16(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(uint16_t, (__bf16)f);   // one conversion instruction; the code below is three and a branch
+#endif
   union { uint32_t u; float f; } x;
   x.f = f;
   if ((x.u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((x.u >> 16) | 0x40u);

@@ -43,21 +43,21 @@ __device__ __forceinline__ void score_body(
   const int c0 = tile * SCORE_TILE + wave * (16 * TPW);
 
   const uint16_t* cg = cent + (size_t)g * nc * RI_DIM;
-  uint4 a[TPW][4];
+  // Rows past the last centroid and query heads past gs read a valid row instead (their columns are never used): a load
+  // under a condition is a branch of its own, and the compiler waited for everything before the last query pieces.
+  uint4 a[TPW][4], bq[4];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
-    const int row = c0 + t * 16 + r;
-    const bool ok = row < nc;
-    const uint16_t* p = cg + (size_t)row * RI_DIM + h * 8;
+    const uint16_t* p = cg + (size_t)min(c0 + t * 16 + r, nc - 1) * RI_DIM + h * 8;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) a[t][kk] = ok ? ri_ld16(p + kk * 32) : ri_zero16();
+    for (int kk = 0; kk < 4; ++kk) a[t][kk] = ri_ld16(p + kk * 32);
   }
-  uint4 bq[4];
   {
-    const uint16_t* p = q + ((size_t)g * gs + r) * RI_DIM + h * 8;
+    const uint16_t* p = q + ((size_t)g * gs + min(r, gs - 1)) * RI_DIM + h * 8;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) bq[kk] = (r < gs) ? ri_ld16(p + kk * 32) : ri_zero16();
+    for (int kk = 0; kk < 4; ++kk) bq[kk] = ri_ld16(p + kk * 32);
   }
+  __builtin_amdgcn_sched_barrier(0);   // every load is in flight before the first product
 
   f32x4_t acc[TPW];
 #pragma unroll
