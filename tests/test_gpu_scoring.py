@@ -326,3 +326,32 @@ def test_misaligned_rows_are_rejected(dev):
     k = torch.empty(1 * 40 * 128 + 8, dtype=torch.bfloat16, device=dev)[1:1 + 40 * 128].view(1, 40, 1, 128)
     with pytest.raises(RuntimeError, match="invalid argument"):
         kernels.weighted_flash_decoding(q.view(1, 1, 4, 128).to(dev), k, k)
+
+
+@pytest.mark.parametrize("BG,gs,nc,nprobe,es", [
+    (2, 4, 8, 1, 7), (3, 16, 8, 8, 0), (2, 5, 64, 64, 0), (2, 4, 72, 65, 7), (2, 3, 256, 256, 0), (2, 12, 264, 200, 40),
+    (2, 8, 512, 512, 0), (2, 4, 512, 129, 383),                            # the workgroup scores its own centroids
+    (2, 4, 520, 512, 8), (2, 16, 1024, 1, 900), (2, 7, 1032, 300, 0), (2, 4, 2048, 513, 1000),
+    (2, 12, 2056, 1024, 100), (2, 4, 4096, 1024, 3072), (1, 1, 8192, 1024, 4000), (1, 3, 8192, 700, 700),   # own score sums
+    (2, 4, 8192, 1024, 100), (1, 9, 4104, 130, 900), (1, 4, 8200, 1023, 1), (1, 4, 16384, 1024, 0),   # keys handed in
+    (1, 4, 16392, 1023, 100), (1, 4, 16384, 1025, 100),                    # one bin per key
+])
+def test_score_select_dispatch_edges(dev, BG, gs, nc, nprobe, es):
+    """Both sides of every line between the selection's variants, with the longest probe lists of each."""
+    test_score_select(dev, BG, gs, nc, nprobe, es, 3000 + nc)
+    test_score_select(dev, BG, gs, nc, nprobe, es, 3001 + nc, dt=torch.float16)
+
+
+@pytest.mark.parametrize("nc,gs", [(256, 4), (512, 4), (1024, 4), (4096, 4), (8192, 4), (16384, 4), (16392, 4)])
+def test_score_select_all_scores_equal(dev, nc, gs):
+    """One score for every cluster: the zones are the lowest ids, in every variant."""
+    from retrievalattention_amd import kernels
+    nprobe, es = nc // 9, nc // 5
+    q = torch.zeros(2, gs, 128, dtype=torch.bfloat16, device=dev)
+    cent = torch.randn(2, nc, 128, generator=torch.Generator().manual_seed(nc)).to(torch.bfloat16).to(dev)
+    i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)
+    ret, est = i32(2, nprobe), i32(2, es)
+    kernels.score_select(q, cent, None, None, None, torch.empty(2, gs, nc, device=dev), None, None, ret, est, None, None,
+                         None, nprobe, es, 8, 16, 1.0)
+    assert torch.equal(ret.cpu(), torch.arange(nprobe, dtype=torch.int32).expand(2, -1))
+    assert torch.equal(est.cpu(), torch.arange(nprobe, nprobe + es, dtype=torch.int32).expand(2, -1))
