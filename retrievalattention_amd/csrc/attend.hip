@@ -1,34 +1,35 @@
 // Weighted flash decoding for the wave index (gfx950).
 //
-// One kernel serves every attention call of the decode step.  A workgroup (4 waves) takes
-// one split of one group's rows; a wave owns a contiguous run of rows and walks it in batches
+// One kernel serves every attention call of the decode step.  A workgroup (8 waves) takes
+// one split of one group's rows; a wave owns a contiguous run of rows of one kind and walks it in batches
 // of 64 rows = 4 chunks of 16.  For a batch it first fetches one row descriptor per lane
-// (where the row lives), then issues every K and V load of the batch before it computes, so
-// that a short kernel keeps enough bytes in flight to load HBM:
-//   * key/value rows ("KV" splits): scores = scale * q·k on bf16 MFMA 16x16x32 with the
+// (where the row lives); a chunk's loads are requested while the chunk before it is computed:
+//   * key/value rows: scores = scale * q·k on bf16 MFMA 16x16x32 with the
 //     query heads as the A rows and 16 key rows as the B columns, so each lane ends up with
 //     the scores of one key row for four heads;
-//   * estimation rows ("EST" splits): the score of a cluster is the logit already computed
+//   * estimation rows: the score of a cluster is the logit already computed
 //     by the scoring kernel, the "value" row is the cluster's value sum and the softmax
 //     denominator is weighted by the cluster size.
 // P·V runs on the matrix cores too: the chunk's probabilities go to LDS as bf16 [head][row], the 16 x 128
 // value tile row-major, and eight MFMA 16x16x16 (B operands read with LDS transpose loads) add the chunk
-// to fp32 accumulators that hold, per lane, four heads of one dimension per 16-wide tile.  Every
-// workgroup writes a (max, denominator, numerator) partial; the workgroup that finishes last for a group
-// merges the partials (and an optional previous result) with the log-sum-exp rule and writes the
-// output, so the whole call is one launch.
+// to fp32 accumulators that hold, per lane, four heads of one dimension per 16-wide tile.  A group with few
+// rows has one workgroup, which writes the output; otherwise every workgroup writes a (max, denominator, numerator)
+// partial, and the workgroup that finishes last for a group merges the partials (and an optional previous result) with
+// the log-sum-exp rule and writes the output, so the whole call is one launch.
 //
 // Semantics follow the weighted_flash_decoding call sites at
 // cache_hub/retroinfer_cache.py:611-617 and :666-674.
+#include <math.h>
 #include <stdint.h>
-#include <stdlib.h>
 
 #include <mutex>
 
 #include "attend_common.h"
 #include "ri_common.h"
 
-#define ATT_FLAG_A 0x40000000  // descriptor bit: row lives in region A
+#define ATT_WAVES 8                // waves of a workgroup
+#define ATT_FLAG_A 0x40000000     // descriptor bit: row lives in region A
+#define ATT_SKIP (int)0x80000000  // descriptor bit (the sign): the row is read but not attended
 
 struct AttendParams {
   const uint16_t* q;  // [BG, gs, 128]
@@ -70,8 +71,8 @@ struct AttendParams {
   float* part_ml;   // [BG, S, GS_PAD, 2]
   float* part_acc;  // [BG, S, GS_PAD, 128]
   int* counters;    // [BG]
-  int S_kv;
-  int S_es;
+  int S;     // workgroups per group
+  int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
   int gs;
   float scale;
   // epilogue
@@ -90,88 +91,156 @@ __device__ __forceinline__ void wave_rows(int total, int nwaves, int wid, int* r
   *r1 = min(total, *r0 + rpw);
 }
 
+// The output rows of head j: A / L merged with an earlier part (its output po, its log-sum-exp pl) under the maximum M.
+// Lane l holds dims 2l and 2l + 1.
+template <bool HALF>
+__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, float M, float L, float A0, float A1) {
+  const int lane = threadIdx.x & 63;
+  const size_t o = (size_t)g * P.gs + j;
+  if (P.prev_lse) {
+    const float pl = P.prev_lse[o];
+    if (pl != -INFINITY) {  // an empty earlier part carries no weight, whatever its output holds
+      float p0, p1;
+      ri_unpack2<HALF>(*reinterpret_cast<const uint32_t*>(P.prev_out + o * RI_DIM + 2 * lane), p0, p1);
+      const float M2 = fmaxf(M, pl);
+      const float f = M == -INFINITY ? 0.f : __expf(M - M2), fp = __expf(pl - M2);
+      L = L * f + fp;
+      A0 = A0 * f + fp * p0;
+      A1 = A1 * f + fp * p1;
+      M = M2;
+    }
+  }
+  // nothing attended at all (an empty part): zeros and a log-sum-exp of -inf, not 0/0
+  const bool any = L > 0.f;
+  *reinterpret_cast<uint32_t*>(P.out + o * RI_DIM + 2 * lane) =
+      (uint32_t)ri_f32_to_e16<HALF>(any ? A0 / L : 0.f) | ((uint32_t)ri_f32_to_e16<HALF>(any ? A1 / L : 0.f) << 16);
+  if (lane == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
+}
+
 // Merges the S split partials of group g (and the optional previous result) and writes the
 // output: wave w of the calling workgroup takes heads w, w+NW, ...; lanes first cover the splits
 // (statistics), then two dims each.
-template <int GS_PAD, int NW, bool HALF>
-__device__ __forceinline__ void combine_group(const AttendParams& P, int g, int S, int lenA, int lenB) {
-  const int gs = P.gs;
+// The partials come from the memory side, where a load takes about a microsecond and one compute unit gets 20 KB per
+// microsecond: every wave requests the statistics of all its heads and then eight splits of all of them at a time.
+// (One head after the other: 13600 cycles for 16 heads over 3 splits.)
+template <int GS_PAD, bool HALF>
+__device__ __forceinline__ void combine_group(const AttendParams& P, int g) {
+  constexpr int NW = ATT_WAVES;
+  constexpr int HPW = (GS_PAD + NW - 1) / NW;   // heads of a wave
+  constexpr int U = HPW > 2 ? 4 : 8;            // splits requested at a time
+  const int gs = P.gs, S = P.S;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int j = wave; j < gs; j += NW) {
-    const float* ml = P.part_ml + ((size_t)g * S * GS_PAD + j) * 2;
-    const float* pa = P.part_acc + ((size_t)g * S * GS_PAD + j) * RI_DIM + 2 * lane;
-    // every load of the merge is issued up front: the statistics (one split per lane) and the
-    // first CB_PRE splits' numerators; their latencies overlap instead of adding up
-    constexpr int CB_PRE = 24;
-    float2 ms = make_float2(-INFINITY, 0.f);
-    if (lane < S) ms = ri_ld_partial(ml + (size_t)lane * GS_PAD * 2);
-    float2 a2[CB_PRE];
+  if (wave >= gs) return;
+  const float* ml = P.part_ml + (size_t)g * S * GS_PAD * 2;
+  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + 2 * lane;
+  float2 ms[HPW];
 #pragma unroll
-    for (int u = 0; u < CB_PRE; ++u)
-      a2[u] = (u < S) ? ri_ld_partial(pa + (size_t)u * GS_PAD * RI_DIM) : make_float2(0.f, 0.f);
-    const float pl = P.prev_lse ? P.prev_lse[(size_t)g * gs + j] : -INFINITY;
-    uint32_t po = 0u;
-    if (P.prev_lse) po = *reinterpret_cast<const uint32_t*>(P.prev_out + ((size_t)g * gs + j) * RI_DIM + 2 * lane);
-    float M = fmaxf(ms.x, pl);
+  for (int k = 0; k < HPW; ++k)
+    ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * 2);
+  float2 a[U][HPW];
+  const auto request = [&](int s0) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-    const float f = (ms.x == -INFINITY) ? 0.f : __expf(ms.x - M);
-    float L = ms.y * f;
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
-    float A0 = 0.f, A1 = 0.f;
-    if (P.prev_lse && pl != -INFINITY) {  // an empty earlier part carries no weight, whatever its output holds
-      const float fp = __expf(pl - M);
-      float p0, p1;
-      ri_unpack2<HALF>(po, p0, p1);
-      L += fp;
-      A0 = fp * p0;
-      A1 = fp * p1;
-    }
+      for (int k = 0; k < HPW; ++k)
+        a[u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * RI_DIM);
+  };
+  request(0);
+  float f[HPW], M[HPW], L[HPW], A0[HPW], A1[HPW];
 #pragma unroll
-    for (int u = 0; u < CB_PRE; ++u) {
-      const float fs = __shfl(f, u);
-      A0 += a2[u].x * fs;
-      A1 += a2[u].y * fs;
-    }
-    for (int s0 = CB_PRE; s0 < S; s0 += 8) {
-      float2 b2[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        b2[u] = (s0 + u < S) ? ri_ld_partial(pa + (size_t)(s0 + u) * GS_PAD * RI_DIM)
-                             : make_float2(0.f, 0.f);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float fs = __shfl(f, (s0 + u) & 63);
-        A0 += b2[u].x * fs;
-        A1 += b2[u].y * fs;
-      }
-    }
-    // nothing attended at all (an empty part): zeros and a log-sum-exp of -inf, not 0/0
-    const bool any = L > 0.f;
-    const uint32_t o = (uint32_t)ri_f32_to_e16<HALF>(any ? A0 / L : 0.f) |
-                       ((uint32_t)ri_f32_to_e16<HALF>(any ? A1 / L : 0.f) << 16);
-    *reinterpret_cast<uint32_t*>(P.out + ((size_t)g * gs + j) * RI_DIM + 2 * lane) = o;
-    if (lane == 0 && P.lse_out) P.lse_out[(size_t)g * gs + j] = M + __logf(L);
+  for (int k = 0; k < HPW; ++k) {
+    const float m = lane < S ? ms[k].x : -INFINITY;
+    M[k] = ri_row_max(m);
+    M[k] = fmaxf(M[k], __shfl_xor(M[k], 16));
+    M[k] = fmaxf(M[k], __shfl_xor(M[k], 32));
+    f[k] = m == -INFINITY ? 0.f : __expf(m - M[k]);
+    L[k] = ri_row_sum(ms[k].y * f[k]);
+    L[k] += __shfl_xor(L[k], 16);
+    L[k] += __shfl_xor(L[k], 32);
+    A0[k] = A1[k] = 0.f;
   }
-  if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
+  for (int s0 = 0; s0 < S; s0 += U) {   // (a split past the last has no weight: f of its lane is 0)
+    if (s0) request(s0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < HPW; ++k) {
+        const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[k]), (s0 + u) & 63));
+        const float w = s0 + u < S ? fs : 0.f;
+        A0[k] += a[u][k].x * w;
+        A1[k] += a[u][k].y * w;
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < HPW; ++k)
+    if (wave + k * NW < gs) write_head<HALF>(P, g, wave + k * NW, M[k], L[k], A0[k], A1[k]);
 }
 
 #define ATT_DESC_MAX 64  // rows of one wave whose descriptors are staged in LDS at a time (32 and 128 measured slower)
 
-// PF = chunks (of 16 rows) in flight per wave: the loads of chunk j+PF are issued before chunk j
-// is computed.  Launched with PF = 1: with eight to twelve waves per compute unit one chunk ahead already
-// keeps the memory system busy, and the deeper pipelines only add registers and ramp (step time at 32 groups
-// of 4 heads: 52.8 us with one chunk ahead, 53.4 with two, 56.0 with three).
-//
-// NW = waves per workgroup (4 or 8).  The waves of a workgroup merge in LDS, so a group split over S workgroups
-// hands S partials to its last arriver whatever NW is: eight-wave workgroups halve the partials (and the
-// arrivals) of a launch with the same number of waves per compute unit.
+// A wave's LDS: value tile, probabilities, rescale factors, row descriptors and weights.
+struct WaveLds {
+  uint16_t* vt;
+  uint16_t* pb;
+  float* al;
+  int* dsc;
+  float* w;
+};
+
+// Rows [r0, r1) of one wave in batches of 64.  `stage(row, weight)` returns where the row lives (a descriptor) and may set
+// the row's weight; `load(d, dv, k, v)` requests the score operand and the four value rows of a chunk, `score` turns
+// the operand into the scores of this lane's heads.
+// The next chunk is requested as soon as the registers of this one are free (keys after their products, values after
+// they are in LDS), so that its loads run under the softmax and the P.V products without a second set of registers.
+template <int GS_PAD, bool HALF, typename K, typename Stage, typename Load, typename Score>
+__device__ __forceinline__ void attend_rows(WaveState<GS_PAD>& st, const WaveLds& sh, int r0, int r1, Stage&& stage,
+                                            Load&& load, Score&& score) {
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 15, h = lane >> 4;
+  for (int s0 = r0; s0 < r1; s0 += ATT_DESC_MAX) {
+    const int s1 = min(r1, s0 + ATT_DESC_MAX);
+    {
+      float w = 1.f;
+      // (a row past the last repeats it, marked: every load has a valid address and no load sits under a condition)
+      const int d = stage(min(s0 + lane, s1 - 1), w);
+      sh.dsc[lane] = s0 + lane < s1 ? d : d | ATT_SKIP;
+      sh.w[lane] = w;
+    }
+    ri_wave_sync();
+    const int nch = (s1 - s0 + 15) >> 4;
+    K k;
+    uint4 v[4];
+    int dk, dv[4];
+    const auto issue = [&](int j) {
+      dk = sh.dsc[j * 16 + n];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dv[i] = sh.dsc[j * 16 + h + 4 * i];
+      load(dk & ~ATT_SKIP, dv, k, v);
+    };
+    issue(0);
+    for (int j = 0; j < nch; ++j) {
+      const bool valid = dk >= 0;
+      float sv[GS_PAD / 4], w = sh.w[j * 16 + n];
+      score(k, sv, w);
+      if (__builtin_amdgcn_ballot_w64(valid) != ~0ull) {   // rows that are not attended must not bring NaN into P.V
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (dv[i] < 0) v[i] = ri_zero16();
+      }
+      chunk_values(v, sh.vt, lane);
+      if (j + 1 < nch) issue(j + 1);
+      chunk_update<GS_PAD, HALF>(st, sv, valid, w, sh.vt, sh.pb, sh.al, lane);
+    }
+  }
+}
+
+// The eight waves of a workgroup merge in LDS, so a group split over S workgroups hands S partials to its last arriver.
 // The rank tables of the retrieval zone (np + 1 token offsets, np first rows) live in dynamic LDS, sized by
 // the launch, so that any number of probes the selection accepts can be attended.
 // HALF: q, K, V, value sums, cluster sizes, weights and outputs are IEEE half instead of bfloat16.
-template <int GS_PAD, int NW, int PF, bool HALF>
-__global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(AttendParams P) {
+template <int GS_PAD, bool HALF>
+__global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams P) {
+  constexpr int NW = ATT_WAVES;
   constexpr int NH = GS_PAD / 4;
   constexpr int NT = 64 * NW;
   __shared__ __attribute__((aligned(16))) uint16_t sh_vt[NW][16 * ATT_VT_STRIDE];
@@ -197,9 +266,9 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
   const int g = blockIdx.y;
   const int split = blockIdx.x;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, h = lane >> 4;
-  const int gs = P.gs;
+  const int gs = P.gs, S = P.S;
 
   WaveState<GS_PAD> st;
 #pragma unroll
@@ -207,24 +276,21 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) st.acc[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
-  uint16_t* vt = sh_vt[wave];
-  uint16_t* pb = sh_pb[wave];
-  float* al_sh = sh_al[wave];
+  const WaveLds sh = {sh_vt[wave], sh_pb[wave], sh_al[wave], sh_desc[wave], sh_w[wave]};
   // P rows of heads that do not exist stay zero; alpha of such heads must not scale by garbage
-  for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(pb)[i] = 0u;
-  if (lane < 16) al_sh[lane] = 1.f;
-  int* dsc = sh_desc[wave];
-  float* wsh = sh_w[wave];
+  for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(sh.pb)[i] = 0u;
+  if (lane < 16) sh.al[lane] = 1.f;
   const int lenB = P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  const int lenA_all = P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
+  const int lenA = P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
 
-  // Estimation rows whose scores are not handed in are key/value rows of their own: key = centroid,
-  // value = value sum, weight = cluster size, located through the id list.
-  const bool est_split = split >= P.S_kv;
-  if (!est_split || P.est_cent) {
-    // ---------------- key/value rows ----------------
-    // rank tables (requested together with everything else the prologue loads: no dependent round trip)
-    const bool tab = !est_split && P.ret_off != nullptr;
+  const int wid = split * NW + wave;            // wave of the group
+  const bool kv_wave = wid < P.W_kv;
+  const bool kv_wg = split * NW < P.W_kv;       // the workgroup has waves with key/value rows
+  const int W_es = S * NW - P.W_kv;
+
+  // ---------------- prologue: query and rank tables to LDS ----------------
+  if (kv_wg || P.est_cent) {
+    const bool tab = kv_wg && P.ret_off != nullptr;
     // every global load of the prologue is requested before the first of them is consumed
     // (up to 1023 probes the table entries pass through registers, TAB_U per thread; longer tables are
     // staged by a plain loop after the query)
@@ -235,8 +301,8 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
 #pragma unroll
       for (int u = 0; u < TAB_U; ++u) {
         const int i = threadIdx.x + u * NT;
-        t_off[u] = (i <= P.np) ? P.ret_off[(size_t)g * (P.np + 1) + i] : 0;
-        t_st[u] = (i < P.np) ? P.ret_start[(size_t)g * P.np + i] : 0;
+        t_off[u] = P.ret_off[(size_t)g * (P.np + 1) + min(i, P.np)];
+        t_st[u] = P.ret_start[(size_t)g * P.np + min(i, P.np - 1)];
       }
     }
     // A operand: query heads through LDS (read again per chunk: registers go to the loads);
@@ -244,8 +310,8 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
     static_assert(GS_PAD * (RI_DIM / 8) <= NT, "one piece of the query per thread");
     {
       const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
-      uint4 qv = ri_zero16();
-      if (head < gs) qv = ri_ld16(P.q + ((size_t)g * gs + head) * RI_DIM + piece * 8);
+      uint4 qv = ri_ld16(P.q + ((size_t)g * gs + min(head, gs - 1)) * RI_DIM + piece * 8);
+      if (head >= gs) qv = ri_zero16();
       if (head < GS_PAD) *reinterpret_cast<uint4*>(&sh_q[head][piece * 8]) = qv;
     }
     if (tab_fast) {
@@ -261,189 +327,112 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
         if (i < P.np) sh_rst[i] = P.ret_start[(size_t)g * P.np + i];
       }
     }
-    // (the row count is consumed only now: the loads above went out together with its load)
-    const int lenA = est_split ? 0 : lenA_all;
-    const int total = est_split ? P.es : lenA_all + lenB;
+    __syncthreads();
+  }
+
+  if (kv_wave || P.est_cent) {
+    // ---------------- rows with keys ----------------
+    // Estimation rows whose scores are not handed in are key/value rows of their own: key = centroid,
+    // value = value sum, weight = cluster size, located through the id list.
+    const bool est = !kv_wave;
     int r0, r1;
-    if (est_split)
-      wave_rows(total, P.S_es * NW, (split - P.S_kv) * NW + wave, &r0, &r1);
-    else
-      wave_rows(total, P.S_kv * NW, split * NW + wave, &r0, &r1);
+    if (est) wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
+    else wave_rows(lenA + lenB, P.W_kv, wid, &r0, &r1);
     const uint16_t* qrow = &sh_q[n % GS_PAD][h * 8];
     const uint16_t* kA = P.kA + (size_t)g * P.strideA * RI_DIM;
     const uint16_t* vA = P.vA + (size_t)g * P.strideA * RI_DIM;
-    const uint16_t* kB = est_split ? P.est_cent + (size_t)g * P.nc * RI_DIM : P.kB + (size_t)g * P.strideB * RI_DIM;
-    const uint16_t* vB = est_split ? P.value_sum + (size_t)g * P.nc * RI_DIM : P.vB + (size_t)g * P.strideB * RI_DIM;
-    const int32_t* rs = est_split ? P.est_ids + (size_t)g * P.es
-                                  : (P.row_src ? P.row_src + (size_t)g * P.rs_stride : nullptr);
-    const uint16_t* wB = (!est_split && P.weightB) ? P.weightB + (size_t)g * P.weight_stride : nullptr;
-    const uint16_t* wsrc = est_split ? P.csize + (size_t)g * P.nc : nullptr;  // weight by source row
+    const uint16_t* kB = est ? P.est_cent + (size_t)g * P.nc * RI_DIM : P.kB + (size_t)g * P.strideB * RI_DIM;
+    const uint16_t* vB = est ? P.value_sum + (size_t)g * P.nc * RI_DIM : P.vB + (size_t)g * P.strideB * RI_DIM;
+    const int32_t* rs = est ? P.est_ids + (size_t)g * P.es
+                            : (P.row_src ? P.row_src + (size_t)g * P.rs_stride : nullptr);
+    const uint16_t* wB = (!est && P.weightB) ? P.weightB + (size_t)g * P.weight_stride : nullptr;
+    const uint16_t* wsrc = est ? P.csize + (size_t)g * P.nc : nullptr;  // weight by source row
     const int r_first = ri_head_reg<GS_PAD>(h);
-    bool q_ready = false;
-    if (tab) {  // the tables are searched while the rows are located
-      __syncthreads();
-      q_ready = true;
-    }
-
-    for (int s0 = r0; s0 < r1; s0 += ATT_DESC_MAX) {
-      const int s1 = min(r1, s0 + ATT_DESC_MAX);
-      // stage the descriptors of rows [s0, s1): where each row lives (-1 = padding row)
-      for (int i = lane; i < ATT_DESC_MAX; i += 64) {
-        const int row = s0 + i;
-        int d = -1;
-        float w = 1.f;
-        if (row < s1) {
-          if (row < lenA) {
-            d = row | ATT_FLAG_A;
-          } else {
-            const int rb = row - lenA;
-            if (tab) {
-              // the last rank whose first row is <= rb (ranks of empty clusters share a first row
-              // with the next rank, which is the one found)
-              int lo = 0, hi = P.np;
-              while (lo + 1 < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (sh_roff[mid] <= rb) lo = mid; else hi = mid;
-              }
-              d = sh_rst[lo] + rb - sh_roff[lo];
-            } else {
-              d = rs ? rs[rb] : rb;
-              if (!est_split && P.row_src && (d < P.src_lo || d >= P.src_hi)) d = -1;
+    const int lead = est ? 0 : lenA;
+    struct Keys { uint4 k[4]; };
+    attend_rows<GS_PAD, HALF, Keys>(
+        st, sh, r0, r1,
+        [&](int row, float& w) {
+          if (row < lead) return row | ATT_FLAG_A;
+          const int rb = row - lead;
+          int d;
+          if (!est && P.ret_off) {
+            // the last rank whose first row is <= rb (ranks of empty clusters share a first row
+            // with the next rank, which is the one found)
+            int lo = 0, hi = P.np;
+            while (lo + 1 < hi) {
+              const int mid = (lo + hi) >> 1;
+              if (sh_roff[mid] <= rb) lo = mid; else hi = mid;
             }
-            if (wB) w = ri_e16_to_f32<HALF>(wB[rb]);
-            if (wsrc) w = ri_e16_to_f32<HALF>(wsrc[d]);
+            d = sh_rst[lo] + rb - sh_roff[lo];
+          } else {
+            d = rs ? rs[rb] : rb;
+            if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d |= ATT_SKIP;
           }
-        }
-        dsc[i] = d;
-        wsh[i] = w;
-      }
-      if (!q_ready) { __syncthreads(); q_ready = true; }  // sh_q complete (also orders dsc writes)
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const int nch = (s1 - s0 + 15) >> 4;
-      uint4 bk[PF][4], v[PF][4];
-      auto issue = [&](int slot_unused, uint4* bks, uint4* vs_, int j) {
-        (void)slot_unused;
-        const int dk = dsc[j * 16 + n];
-        const uint16_t* kp = ((dk & ATT_FLAG_A) ? kA : kB) + (size_t)(dk & ~ATT_FLAG_A) * RI_DIM + h * 8;
+          if (wB) w = ri_e16_to_f32<HALF>(wB[rb]);
+          if (wsrc) w = ri_e16_to_f32<HALF>(wsrc[d]);
+          return d;
+        },
+        [&](int dk, const int* dv, Keys& k, uint4* v) {
+          const uint16_t* kp = ((dk & ATT_FLAG_A) ? kA : kB) + (size_t)(dk & ~ATT_FLAG_A) * RI_DIM + h * 8;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) bks[kk] = (dk >= 0) ? ri_ld16(kp + kk * 32) : ri_zero16();
+          for (int kk = 0; kk < 4; ++kk) k.k[kk] = ri_ld16(kp + kk * 32);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int dv = dsc[j * 16 + h + 4 * i];
-          const uint16_t* vp = ((dv & ATT_FLAG_A) ? vA : vB) + (size_t)(dv & ~ATT_FLAG_A) * RI_DIM + n * 8;
-          vs_[i] = (dv >= 0) ? ri_ld16(vp) : ri_zero16();
-        }
-      };
-      auto compute = [&](const uint4* bks, const uint4* vs_, int j) {
-        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const uint4 qv = *reinterpret_cast<const uint4*>(qrow + kk * 32);
-          acc = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, qv),
-                                                              __builtin_bit_cast(f16x8_t, bks[kk]), acc, 0, 0, 0)
-                     : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(qv), ri_as_bf16x8(bks[kk]), acc, 0, 0, 0);
-        }
-        float sv[NH];
-#pragma unroll
-        for (int i = 0; i < NH; ++i) {
-          float x;
-          if (GS_PAD == 16) {
-            x = acc[i];
-          } else {  // register r_first + i without dynamic indexing
-            const int r = r_first + i;
-            x = r == 0 ? acc[0] : (r == 1 ? acc[1] : (r == 2 ? acc[2] : acc[3]));
+          for (int i = 0; i < 4; ++i) {
+            const int d = dv[i] & ~ATT_SKIP;
+            v[i] = ri_ld16(((d & ATT_FLAG_A) ? vA : vB) + (size_t)(d & ~ATT_FLAG_A) * RI_DIM + n * 8);
           }
-          sv[i] = x * P.scale;
-        }
-        const bool valid = dsc[j * 16 + n] >= 0;
-        const float w = wsh[j * 16 + n];
-        chunk_update<GS_PAD, HALF>(st, sv, valid, w, vs_, vt, pb, al_sh, lane);
-      };
+        },
+        [&](const Keys& k, float* sv, float&) {
+          f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < PF; ++s)
-        if (s < nch) issue(s, bk[s], v[s], s);
-      for (int j0 = 0; j0 < nch; j0 += PF) {
-#pragma unroll
-        for (int s = 0; s < PF; ++s) {
-          const int j = j0 + s;
-          if (j < nch) {
-            compute(bk[s], v[s], j);
-            if (j + PF < nch) issue(s, bk[s], v[s], j + PF);
+          for (int kk = 0; kk < 4; ++kk) {
+            const uint4 qv = *reinterpret_cast<const uint4*>(qrow + kk * 32);
+            acc = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, qv),
+                                                                __builtin_bit_cast(f16x8_t, k.k[kk]), acc, 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(qv), ri_as_bf16x8(k.k[kk]), acc, 0, 0, 0);
           }
-        }
-      }
-    }
-    if (!q_ready) __syncthreads();  // keep the barrier count uniform for waves without rows
+#pragma unroll
+          for (int i = 0; i < NH; ++i) {
+            float x;
+            if (GS_PAD == 16) {
+              x = acc[i];
+            } else {  // register r_first + i without dynamic indexing
+              const int r = r_first + i;
+              x = r == 0 ? acc[0] : (r == 1 ? acc[1] : (r == 2 ? acc[2] : acc[3]));
+            }
+            sv[i] = x * P.scale;
+          }
+        });
   } else {
-    // ---------------- estimation rows ----------------
-    const int es = P.es;
+    // ---------------- estimation rows with their logits at hand ----------------
     int r0, r1;
-    wave_rows(es, P.S_es * NW, (split - P.S_kv) * NW + wave, &r0, &r1);
-    const int32_t* ids = P.est_ids + (size_t)g * es;
+    wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
+    const int32_t* ids = P.est_ids + (size_t)g * P.es;
     const uint16_t* vs = P.value_sum + (size_t)g * P.nc * RI_DIM;
     const uint16_t* cs = P.csize + (size_t)g * P.nc;
     const float* lg = P.logits + (size_t)g * gs * P.nc;
-
-    for (int s0 = r0; s0 < r1; s0 += ATT_DESC_MAX) {
-      const int s1 = min(r1, s0 + ATT_DESC_MAX);
-      for (int i = lane; i < ATT_DESC_MAX; i += 64) {
-        const int row = s0 + i;
-        int d = -1;
-        float w = 0.f;
-        if (row < s1) {
-          d = ids[row];
-          w = ri_e16_to_f32<HALF>(cs[d]);
-        }
-        dsc[i] = d;
-        wsh[i] = w;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const int nch = (s1 - s0 + 15) >> 4;
-      float sc[PF][NH];
-      uint4 v[PF][4];
-      auto issue = [&](float* scs, uint4* vs_, int j) {
-        const int ck = dsc[j * 16 + n];
+    struct Logits { float x[NH]; uint16_t size; };
+    attend_rows<GS_PAD, HALF, Logits>(
+        st, sh, r0, r1, [&](int row, float&) { return ids[row]; },
+        [&](int dk, const int* dv, Logits& k, uint4* v) {
 #pragma unroll
-        for (int i = 0; i < NH; ++i) {
-          const int head = ri_head_of<GS_PAD>(h, i);
-          scs[i] = (ck >= 0 && head < gs) ? lg[(size_t)head * P.nc + ck] : -INFINITY;
-        }
+          for (int i = 0; i < NH; ++i) k.x[i] = lg[(size_t)min(ri_head_of<GS_PAD>(h, i), gs - 1) * P.nc + dk];
+          k.size = cs[dk];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int cv = dsc[j * 16 + h + 4 * i];
-          vs_[i] = (cv >= 0) ? ri_ld16(vs + (size_t)cv * RI_DIM + n * 8) : ri_zero16();
-        }
-      };
+          for (int i = 0; i < 4; ++i) v[i] = ri_ld16(vs + (size_t)(dv[i] & ~ATT_SKIP) * RI_DIM + n * 8);
+        },
+        [&](const Logits& k, float* sv, float& w) {
 #pragma unroll
-      for (int s = 0; s < PF; ++s)
-        if (s < nch) issue(sc[s], v[s], s);
-      for (int j0 = 0; j0 < nch; j0 += PF) {
-#pragma unroll
-        for (int s = 0; s < PF; ++s) {
-          const int j = j0 + s;
-          if (j < nch) {
-            const bool valid = dsc[j * 16 + n] >= 0;
-            const float w = wsh[j * 16 + n];
-            chunk_update<GS_PAD, HALF>(st, sc[s], valid, w, v[s], vt, pb, al_sh, lane);
-            if (j + PF < nch) issue(sc[s], v[s], j + PF);
-          }
-        }
-      }
-    }
+          for (int i = 0; i < NH; ++i) sv[i] = ri_head_of<GS_PAD>(h, i) < gs ? k.x[i] : -INFINITY;
+          w = ri_e16_to_f32<HALF>(k.size);
+        });
   }
 
   // ---------------- wave partial -> LDS ----------------
 #pragma unroll
   for (int i = 0; i < NH; ++i) {
-    float l = st.l[i];
-    l += __shfl_xor(l, 1);
-    l += __shfl_xor(l, 2);
-    l += __shfl_xor(l, 4);
-    l += __shfl_xor(l, 8);
+    const float l = ri_row_sum(st.l[i]);
     if (n == 0) {
       sh_m[wave][ri_head_of<GS_PAD>(h, i)] = st.m[i];
       sh_l[wave][ri_head_of<GS_PAD>(h, i)] = l;
@@ -460,27 +449,39 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
   }
   __syncthreads();
 
-  // ---------------- merge the waves, write the split partial ----------------
-  const int S = P.S_kv + P.S_es;
-  for (int idx = threadIdx.x; idx < GS_PAD * RI_DIM; idx += NT) {
-    const int j = idx / RI_DIM, d = idx % RI_DIM;
-    float M = sh_m[0][j];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, sh_m[w][j]);
-    float a = 0.f, l = 0.f;
+  // ---------------- merge the waves: wave w takes heads w, w + NW, ..., a lane two dims ----------------
+  for (int j = wave; j < gs; j += NW) {
+    float m[NW], M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float f = (sh_m[w][j] == -INFINITY) ? 0.f : __expf(sh_m[w][j] - M);
-      a += acc_of(w)[j * RI_DIM + d] * f;
+      m[w] = sh_m[w][j];
+      M = fmaxf(M, m[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = m[w] == -INFINITY ? 0.f : __expf(m[w] - M);
+      const float2 x = *reinterpret_cast<const float2*>(acc_of(w) + j * RI_DIM + 2 * lane);
+      a0 += x.x * f;
+      a1 += x.y * f;
       l += sh_l[w][j] * f;
+    }
+    if (S == 1) {   // the workgroup has the whole group: no partial leaves it
+      write_head<HALF>(P, g, j, M, l, a0, a1);
+      continue;
     }
     const size_t o = ((size_t)g * S + split) * GS_PAD + j;
     // device-coherent stores: another workgroup of this launch reads them
-    __hip_atomic_store(&P.part_acc[o * RI_DIM + d], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (d == 0) {
-      __hip_atomic_store(&P.part_ml[o * 2], M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&P.part_ml[o * 2 + 1], l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + 2 * lane]),
+                       (uint64_t)__float_as_uint(a0) | (uint64_t)__float_as_uint(a1) << 32, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_ml[o * 2]),
+                         (uint64_t)__float_as_uint(M) | (uint64_t)__float_as_uint(l) << 32, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (S == 1) {
+    if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
+    return;
   }
 
   // ---------------- last workgroup of the group merges all splits ----------------
@@ -509,7 +510,8 @@ __global__ __launch_bounds__(64 * NW, GS_PAD == 16 ? 1 : 3) void attend_kernel(A
     sh_last = (__hip_atomic_fetch_add(&P.counters[g], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1);
   __syncthreads();
   if (!sh_last) return;
-  combine_group<GS_PAD, NW, HALF>(P, g, S, lenA_all, lenB);
+  combine_group<GS_PAD, HALF>(P, g);
+  if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
   // ready for the next launch (every arrival of this launch has been counted; launches that share the
   // workspace do not overlap)
   if (threadIdx.x == 0) __hip_atomic_store(&P.counters[g], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -533,53 +535,32 @@ static size_t attn_workspace_bytes(int BG, int gs) {
 extern "C" size_t ri_flash_decoding_workspace_bytes(int BG, int gs) { return attn_workspace_bytes(BG, gs); }
 extern "C" size_t ri_wave_attention_workspace_bytes(int BG, int gs) { return attn_workspace_bytes(BG, gs); }
 
-// Bytes a launch with S = S_kv + S_es splits per group really uses: the counter area, then the
+// Bytes a launch with S splits per group really uses: the counter area, then the
 // (max, denominator) pairs and the numerators of BG * S partials.
 static size_t attn_scratch_used(int BG, int gp, int S) {
   return RI_MAX_GROUPS * sizeof(int) + (size_t)BG * S * gp * (2 + RI_DIM) * sizeof(float);
 }
 
 static void carve_workspace(AttendParams& P, void* workspace, int BG, int gp) {
-  const int S = P.S_kv + P.S_es;
   P.counters = (int*)workspace;
   P.part_ml = (float*)((char*)workspace + RI_MAX_GROUPS * sizeof(int));
-  P.part_acc = P.part_ml + (size_t)BG * S * gp * 2;
+  P.part_acc = P.part_ml + (size_t)BG * P.S * gp * 2;
 }
 
 template <bool HALF>
-static void launch_attend_t(const AttendParams& P, dim3 grid, int gp, int nw, size_t tab_bytes, hipStream_t s) {
-  if (nw == 8 && gp == 4) attend_kernel<4, 8, 1, HALF><<<grid, 512, tab_bytes, s>>>(P);
-  else if (nw == 8 && gp == 8) attend_kernel<8, 8, 1, HALF><<<grid, 512, tab_bytes, s>>>(P);
-  else if (gp == 4) attend_kernel<4, 4, 1, HALF><<<grid, 256, tab_bytes, s>>>(P);
-  else if (gp == 8) attend_kernel<8, 4, 1, HALF><<<grid, 256, tab_bytes, s>>>(P);
-  else attend_kernel<16, 4, 1, HALF><<<grid, 256, tab_bytes, s>>>(P);
+static void launch_attend_t(const AttendParams& P, dim3 grid, int gp, size_t tab_bytes, hipStream_t s) {
+  if (gp == 4) attend_kernel<4, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
+  else if (gp == 8) attend_kernel<8, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
+  else attend_kernel<16, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
 }
 
-static int launch_attend(AttendParams& P, int BG, int gs, int nw, bool half, hipStream_t s) {
-  const int S = P.S_kv + P.S_es;
-  const dim3 grid(S, BG);
+static int launch_attend(AttendParams& P, int BG, int gs, bool half, hipStream_t s) {
+  const dim3 grid(P.S, BG);
   const size_t tab_bytes = P.ret_off ? (size_t)(2 * P.np + 1) * sizeof(int) : 0;
-  if (half) launch_attend_t<true>(P, grid, gs_pad_of(gs), nw, tab_bytes, s);
-  else launch_attend_t<false>(P, grid, gs_pad_of(gs), nw, tab_bytes, s);
+  if (half) launch_attend_t<true>(P, grid, gs_pad_of(gs), tab_bytes, s);
+  else launch_attend_t<false>(P, grid, gs_pad_of(gs), tab_bytes, s);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
-}
-
-// Waves per workgroup of a launch.  Eight for groups of up to four query heads: half the split partials and
-// arrivals per group at the same number of waves per compute unit (32 groups of 4 heads over 8192 clusters:
-// 18.7 against 19.3 us per launch).  Four otherwise: with eight or more heads the wave partials of an
-// eight-wave workgroup take so much LDS that only one workgroup fits a compute unit (64 groups of 8 heads over
-// 16384 clusters: 71 against 53 us).  RI_ATTEND_WAVES=4|8 in the environment overrides the choice for groups of
-// up to eight heads (read once, for measurements).
-static int attend_waves(int gs) {
-  static const int forced = [] {
-    const char* e = getenv("RI_ATTEND_WAVES");
-    return e ? atoi(e) : 0;
-  }();
-  const int gp = gs_pad_of(gs);
-  if (gp == 16) return 4;
-  if (forced == 4 || forced == 8) return forced;
-  return gp == 4 ? 8 : 4;
 }
 
 // Memory traffic of one estimation row: its value-sum row, the 32-byte sector around its cluster size, and
@@ -587,36 +568,27 @@ static int attend_waves(int gs) {
 // its centroid row.
 static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_here ? 256 : 32 * gs); }
 
-// Split plan: about two workgroups per compute unit in total (an even load over the 256 CUs,
-// all resident at once), at least 128 rows per workgroup, the budget shared between the
-// key/value rows and the estimation rows in proportion to the memory traffic of a row, es_row_bytes
-// against the 512 bytes of a K and a V row (the launch is bound by its traffic: weighing a key/value
-// row twice an estimation row, by its arithmetic, left the estimation workgroups finishing last,
-// 20.2 against 19.5 us at 32 groups of 4 heads and 60.4 against 54.9 us at 64 groups of 8).
-static void plan_splits(int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int nw, int* S_kv, int* S_es) {
-  // eight waves per compute unit while the launch is short (latency counts); twelve once every
-  // wave has more than 128 rows to stream (throughput counts)
-  const int64_t all_rows = (kv_rows + es_rows) * BG;
-  const int target_wgs = (all_rows > 512 * 512 ? 768 : 512) * 4 / nw;
-  int per_group = target_wgs / BG;
-  if (per_group < 1) per_group = 1;
-  if (per_group > RI_MAX_SPLITS) per_group = RI_MAX_SPLITS;
-  const int64_t rows = kv_rows + es_rows;
-  int64_t by_rows = (rows + 32 * nw - 1) / (32 * nw);
-  if (by_rows < 1) by_rows = 1;
-  if (per_group > by_rows) per_group = (int)by_rows;
-  if (es_rows <= 0) {
-    *S_kv = per_group;
-    *S_es = 0;
-    return;
-  }
-  if (per_group < 2) per_group = 2;
-  const int64_t wk = kv_rows * 512, we = es_rows * es_row_bytes;
-  int kv = (int)((wk * per_group + (wk + we) / 2) / (wk + we));
-  if (kv < 1) kv = 1;
-  if (kv > per_group - 1) kv = per_group - 1;
-  *S_kv = kv;
-  *S_es = per_group - kv;
+// Split plan of a launch: workgroups per group, and the waves of a group that take key/value rows, shared with the
+// estimation rows in proportion to the memory traffic of a row, es_row_bytes against the 512 bytes of a K and a V row.
+//  * One workgroup of eight waves per compute unit: 64 groups of 8 heads over 16384 clusters 54.7 us, two per unit or
+//    three of four waves 55.3 .. 60 us; 11 groups, 29000 rows: 38.0 against 41.9 .. 45.
+//  * A compute unit reads about 25 KB per microsecond, so more workgroups stream a group's rows faster, but the last
+//    one to arrive reads the partials of all of them at that same rate: the sum of both is least near
+//    sqrt(bytes of the group / bytes of a partial), flat towards fewer (12 groups of 7 heads, 3550 rows: 15 workgroups
+//    11.6 us, 21: 12.0).
+//  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
+//    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
+static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs) {
+  const int64_t rows = kv_rows + es_rows, wk = kv_rows * 512, we = es_rows * es_row_bytes;
+  int64_t per_group = 256 / BG;
+  per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
+  per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
+  per_group = min(per_group, (int64_t)RI_MAX_SPLITS);
+  if (rows * gs_pad_of(gs) <= 384 * 4 || per_group < 1) per_group = 1;
+  const int waves = (int)per_group * ATT_WAVES;
+  P.S = (int)per_group;
+  P.W_kv = waves;
+  if (es_rows > 0) P.W_kv = (int)min(max((wk * waves + (wk + we) / 2) / (wk + we), (int64_t)1), (int64_t)(waves - 1));
 }
 
 static int flash_decoding_impl(const void* q, const void* k, const void* v, const void* weight,
@@ -640,8 +612,7 @@ static int flash_decoding_impl(const void* q, const void* k, const void* v, cons
   P.lenB_const = S;
   P.weightB = (const uint16_t*)weight;
   P.weight_stride = S;
-  const int nw = attend_waves(gs);
-  plan_splits(S, 0, 0, BG, nw, &P.S_kv, &P.S_es);
+  plan_splits(P, S, 0, 0, BG, gs);
   P.gs = gs;
   P.scale = scale;
   P.prev_out = (const uint16_t*)prev_out;
@@ -649,7 +620,7 @@ static int flash_decoding_impl(const void* q, const void* k, const void* v, cons
   P.out = (uint16_t*)out;
   P.lse_out = lse_out;
   carve_workspace(P, workspace, BG, gp);
-  return launch_attend(P, BG, gs, nw, half, (hipStream_t)stream);
+  return launch_attend(P, BG, gs, half, (hipStream_t)stream);
 }
 
 extern "C" int ri_weighted_flash_decoding(const void* q, const void* k, const void* v, const void* weight,
@@ -737,16 +708,15 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   // the retrieved-token count is only known on the device: size the split for the row table
   // capacity scaled by the usual fill (a quarter) or for 16 tokens per rank, the estimation zone by
   // its exact size
-  const int nw = attend_waves(gs);
-  plan_splits(static_len + (row_src ? row_src_stride / 4 : np * 16), es, est_row_bytes(gs, est_centroids != nullptr), BG,
-              nw, &P.S_kv, &P.S_es);
-  if (scratch_bytes < attn_scratch_used(BG, gp, P.S_kv + P.S_es)) return RI_ERR_WORKSPACE;
+  plan_splits(P, static_len + (row_src ? row_src_stride / 4 : np * 16), es,
+              est_row_bytes(gs, est_centroids != nullptr), BG, gs);
+  if (scratch_bytes < attn_scratch_used(BG, gp, P.S)) return RI_ERR_WORKSPACE;
   carve_workspace(P, scratch, BG, gp);
   if (clear_counters) {
     attend_clear_counters_kernel<<<(BG + 255) / 256, 256, 0, stream>>>(P.counters, BG);
     RI_HIP_CHECK_LAUNCH();
   }
-  return launch_attend(P, BG, gs, nw, half, stream);
+  return launch_attend(P, BG, gs, half, stream);
 }
 
 // Clears the arrival counters at the head of an attention workspace with a small kernel on `stream` (no
@@ -967,10 +937,9 @@ static int ri_buffer_attention_any(const void* q, const void* buf_k, const void*
   P.scale = scale;
   P.out = (uint16_t*)out;
   // the valid lengths are only known on the device: size the split for a quarter of the buffer
-  const int nw = attend_waves(gs);
-  plan_splits(max_len / 4 + 64, es, est_row_bytes(gs, false), BG, nw, &P.S_kv, &P.S_es);
+  plan_splits(P, max_len / 4 + 64, es, est_row_bytes(gs, false), BG, gs);
   carve_workspace(P, workspace, BG, gp);
-  return launch_attend(P, BG, gs, nw, half, (hipStream_t)stream);
+  return launch_attend(P, BG, gs, half, (hipStream_t)stream);
 }
 
 extern "C" int ri_buffer_attention(const void* q, const void* buf_k, const void* buf_v, int64_t buf_stride,

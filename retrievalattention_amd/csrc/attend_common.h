@@ -37,55 +37,65 @@ __device__ __forceinline__ uint16_t ri_p_to_e16(float x) {
   return __builtin_bit_cast(uint16_t, b);
 }
 
-// One chunk of 16 rows.
+// maximum / sum over the 16 lanes of a row, in every lane (register moves within the row, no LDS crossbar)
+__device__ __forceinline__ float ri_row_max(float x) {
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, true)));   // quad_perm 1,0,3,2
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, true)));   // quad_perm 2,3,0,1
+  x = fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, true)));  // half row mirrored
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, true)));  // row mirrored
+}
+__device__ __forceinline__ float ri_row_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, true));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, true));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, true));
+  return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ void ri_wave_sync() {   // LDS written by this wave is read by this wave
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The value rows h, h+4, h+8, h+12 of a chunk (dims 8n..8n+7, as loaded) -> row-major 16 x 128 tile in LDS.
+__device__ __forceinline__ void chunk_values(const uint4 v[4], uint16_t* vt, int lane) {
+  const int n = lane & 15, h = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(vt + (h + 4 * i) * ATT_VT_STRIDE + 8 * n) = v[i];
+}
+
+// One chunk of 16 rows whose value tile is in LDS.
 //   sv[NH]  scores of the heads this lane keeps for row n = lane%16 (lane group h = lane/16)
-//   v[4]    value rows h, h+4, h+8, h+12 of the chunk, dims 8n..8n+7 (as loaded from memory)
-// Softmax bookkeeping in fp32 per lane; P goes to LDS as bf16 [head][row], the value tile to LDS
-// row-major; P·V = 8 MFMA 16x16x16 whose B operands come from LDS transpose reads
+// Softmax bookkeeping in fp32 per lane; P goes to LDS as bf16 [head][row]; P·V = 8 MFMA 16x16x16 whose B
+// operands come from LDS transpose reads
 // (ds_read_b64_tr_b16: lane l of a 16-lane group receives element l%4 of the 8-byte pieces
 // addressed by lanes l/4, l/4+4, l/4+8, l/4+12 — four consecutive rows of one column).
 template <int GS_PAD, bool HALF>
 __device__ __forceinline__ void chunk_update(WaveState<GS_PAD>& st, const float* sv, bool valid, float w,
-                                             const uint4 v[4], uint16_t* vt, uint16_t* pb, float* al_sh,
-                                             int lane) {
+                                             const uint16_t* vt, uint16_t* pb, float* al_sh, int lane) {
   constexpr int NH = GS_PAD / 4;
   const int n = lane & 15, h = lane >> 4;
-  // value tile -> LDS
-#pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(vt + (h + 4 * i) * ATT_VT_STRIDE + 8 * n) = v[i];
   float al[NH];
   bool rescale = false;
 #pragma unroll
   for (int i = 0; i < NH; ++i) {
     const float s = valid ? sv[i] : -INFINITY;
-    float cm = s;
-    cm = fmaxf(cm, __shfl_xor(cm, 1));
-    cm = fmaxf(cm, __shfl_xor(cm, 2));
-    cm = fmaxf(cm, __shfl_xor(cm, 4));
-    cm = fmaxf(cm, __shfl_xor(cm, 8));
-    const float mn = fmaxf(st.m[i], cm);
-    float p;
-    if (mn == -INFINITY) {
-      al[i] = 1.f;
-      p = 0.f;
-    } else {
-      al[i] = __expf(st.m[i] - mn);  // exp(-inf) = 0 for the first chunk
-      p = valid ? __expf(s - mn) : 0.f;
-    }
+    const float mn = fmaxf(st.m[i], ri_row_max(s));
+    // (no valid row so far: the maximum is -inf; exp(-inf) = 0 for the first chunk that has one)
+    al[i] = mn == -INFINITY ? 1.f : __expf(st.m[i] - mn);
+    const float p = valid ? __expf(s - mn) : 0.f;
     rescale |= (al[i] != 1.f);
     st.l[i] = st.l[i] * al[i] + w * p;
     st.m[i] = mn;
     pb[ri_head_of<GS_PAD>(h, i) * 16 + n] = ri_p_to_e16<HALF>(p);
   }
   // the running maximum rarely moves after the first chunks: rescale only when some head's did
-  const bool any_rescale = __any(rescale);
+  const bool any_rescale = __builtin_amdgcn_ballot_w64(rescale) != 0;
   if (any_rescale && n == 0) {
 #pragma unroll
     for (int i = 0; i < NH; ++i) al_sh[ri_head_of<GS_PAD>(h, i)] = al[i];
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  ri_wave_sync();
   if (any_rescale) {
     const float4 a4 = *reinterpret_cast<const float4*>(al_sh + 4 * h);
 #pragma unroll
@@ -106,8 +116,7 @@ __device__ __forceinline__ void chunk_update(WaveState<GS_PAD>& st, const float*
     else
       st.acc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa, vb, st.acc[dt], 0, 0, 0);
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();  // the tile and P are rewritten by the next chunk
+  ri_wave_sync();   // the tile and P are rewritten by the next chunk
 }
 
 // The partials were written by other workgroups of the same launch; they are read with

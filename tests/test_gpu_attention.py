@@ -336,3 +336,12 @@ def test_wave_attention_part_that_attends_nothing(dev):
     assert torch.equal(merged, full)
     ref = attention.weighted_flash_decoding(q.cpu(), store_k.cpu(), store_v.cpu(), None, None, None)[0]
     _close(full.cpu(), ref)
+
+
+@pytest.mark.parametrize("gs,S", [(4, 1), (4, 15), (4, 16), (4, 17), (3, 64), (4, 65), (4, 127), (4, 129), (4, 384),
+                                  (4, 385), (5, 191), (8, 192), (7, 193), (9, 96), (16, 97), (12, 640), (4, 4097)])
+def test_split_plan_edges(dev, gs, S):
+    """Rows around the chunk (16), the wave batch (64) and the line between one workgroup per group and several, with
+    previous partials and ragged lengths."""
+    test_weighted_flash_decoding(dev, 2, gs, S, True, True, True)
+    test_weighted_flash_decoding(dev, 3, gs, S, False, False, False, dt=torch.float16)
