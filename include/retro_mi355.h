@@ -441,6 +441,17 @@ int ri_kmeans_update_f16(const void* data, const int32_t* counts, const int32_t*
                          int64_t head_rows, int normalize, void* workspace, size_t workspace_bytes,
                          ri_stream_t stream);
 
+/* ri_kmeans_build_lists followed by ri_kmeans_update in one launch, for at most 16384 tokens per problem: the same
+ * means bit for bit.  counts [P, nc], offsets [P, nc+1] and members [P, N] are written as ri_kmeans_build_lists writes
+ * them, or all three are NULL. */
+int ri_kmeans_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
+                            int32_t* offsets, int32_t* members, int P, int N, int nc, int seg,
+                            int64_t head_rows, int normalize, ri_stream_t stream);
+/* ri_kmeans_update_direct on IEEE half instead of bfloat16. */
+int ri_kmeans_update_direct_f16(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
+                                int32_t* offsets, int32_t* members, int P, int N, int nc, int seg,
+                                int64_t head_rows, int normalize, ri_stream_t stream);
+
 /* Per-cluster value sums: replaces triton_index_add (cache_hub/kmeans.py:176-221).
  * value_sum[p,c,:] = bf16(Σ member value rows), Σ in the same fixed order as above. */
 int ri_kmeans_value_sum(const void* values, const int32_t* counts, const int32_t* offsets,

@@ -37,23 +37,32 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices):
     centroids = torch.index_select(key, 1, init_indices).contiguous()
     nseg, ncs = N // S, nc // S
     P = G * S
-    assign = torch.empty((P, max(nseg, 1)), dtype=torch.int32, device=dev)
-    counts = torch.empty((P, ncs), dtype=torch.int32, device=dev)
-    offsets = torch.empty((P, ncs + 1), dtype=torch.int32, device=dev)
-    members = torch.empty((P, max(nseg, 1)), dtype=torch.int32, device=dev)
-    if nseg > 0:
+    if nseg > 0 and num_iters > 1:
+        assign = torch.empty((P, nseg), dtype=torch.int32, device=dev)
+        direct = nseg <= kernels.KMEANS_DIRECT_MAX_TOKENS
+        if not direct:
+            counts = torch.empty((P, ncs), dtype=torch.int32, device=dev)
+            offsets = torch.empty((P, ncs + 1), dtype=torch.int32, device=dev)
+            members = torch.empty((P, nseg), dtype=torch.int32, device=dev)
         for _ in range(num_iters - 1):
             kernels.kmeans_assign(key, centroids, assign, P, nseg, ncs, S, N)
-            kernels.kmeans_build_lists(assign, counts, offsets, members, P, nseg, ncs)
-            kernels.kmeans_update(key, counts, offsets, members, centroids, P, nseg, ncs, S, N, True)
+            if direct:
+                kernels.kmeans_update_direct(key, assign, centroids, P, nseg, ncs, S, N, True)
+            else:
+                kernels.kmeans_build_lists(assign, counts, offsets, members, P, nseg, ncs)
+                kernels.kmeans_update(key, counts, offsets, members, centroids, P, nseg, ncs, S, N, True)
     r = KMeansResult()
     r.assign = torch.empty((G, N), dtype=torch.int32, device=dev)
     r.counts = torch.empty((G, nc), dtype=torch.int32, device=dev)
     r.offsets = torch.empty((G, nc + 1), dtype=torch.int32, device=dev)
     r.members = torch.empty((G, N), dtype=torch.int32, device=dev)
     kernels.kmeans_assign(key, centroids, r.assign, G, N, nc, 1, N)
-    kernels.kmeans_build_lists(r.assign, r.counts, r.offsets, r.members, G, N, nc)
-    kernels.kmeans_update(key, r.counts, r.offsets, r.members, centroids, G, N, nc, 1, N, False)
+    if N <= kernels.KMEANS_DIRECT_MAX_TOKENS:
+        kernels.kmeans_update_direct(key, r.assign, centroids, G, N, nc, 1, N, False,
+                                     (r.counts, r.offsets, r.members))
+    else:
+        kernels.kmeans_build_lists(r.assign, r.counts, r.offsets, r.members, G, N, nc)
+        kernels.kmeans_update(key, r.counts, r.offsets, r.members, centroids, G, N, nc, 1, N, False)
     r.centroids = centroids
     return r
 

@@ -8,18 +8,6 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void* km_lds_ptr;
 typedef const __attribute__((address_space(1))) void* km_glb_ptr;
 
-#define KM_WAVES 4        // waves per workgroup sharing one centroid tile
-// The assignment kernel comes in two tilings (KM_TT 32-token MFMA columns per wave held in registers,
-// KM_CT centroid rows per LDS tile):
-//   4 x 128  long centroid loops (more than KM_WIDE_MIN_NC centroids per problem): most reuse of every LDS read,
-//            256 VGPRs and 64 KiB of LDS, two workgroups per CU;
-//   2 x 32   short loops (the segmented iterations: 512 centroids per problem): the load of the tokens in
-//            front of the loop is a large part of the kernel, and 126 VGPRs / 16 KiB let four workgroups per
-//            CU overlap one's loads with the others' MFMAs.
-// Measured with 8 x 131072 tokens: 512 centroids per problem 125.6 against 135.4 us, 1024: 228 against 252,
-// 2048: 433 against 457, 4096: 836 against 845, 8192: 1639 against 1611 us.
-#define KM_WIDE_MIN_NC 4096
-
 // 16 bytes per lane from global memory straight into LDS: lane l lands at lds_base + 16 l
 // (lds_base: byte address inside the workgroup's LDS, the same in every lane).  The wait for the
 // data is the caller's (s_waitcnt vmcnt): issued as inline assembly so that LDS reads of other
@@ -34,26 +22,28 @@ __device__ __forceinline__ size_t km_row0(int p, int seg, int64_t head_rows, int
 }
 
 // ------------------------------------------------------------------------------------
-// assign: grid (ceil(N / (KM_WAVES * 32 * KM_TT)), P), KM_WAVES waves; a wave keeps KM_TT columns of 32
+// assign: grid (ceil(N / (KM_W * 32 * KM_TT)), P), KM_W waves; a wave keeps KM_TT columns of 32
 // tokens in registers for the whole kernel (KM_TT independent accumulator chains).  Centroid
-// tiles of KM_CT rows go through two LDS buffers shared by all waves of the workgroup: the next
-// tile is requested from global memory straight into the other buffer (no registers, no LDS
-// stores) before the MFMAs of the current one, one wait and one barrier per tile.  (On the full-size
-// pass 4 token columns x 4 waves measured fastest against 2x4, 2x8, 2x12, 3x8, and 128-row tiles
-// against 64 and 256, with clocks warmed up and runs interleaved.)
+// tiles of KM_CT rows go through KM_NB LDS buffers shared by all waves of the workgroup: a tile
+// is requested from global memory straight into its buffer (no registers, no LDS
+// stores) KM_NB - 1 tiles ahead, one wait and one barrier per tile.
 // MFMA 32x32x16: A = centroid rows, B = token columns; accumulator i of lane l is
 // row (i/4)*8 + (l/32)*4 + i%4, column l%32.  nc is a multiple of 32; the last tile may hold
-// fewer sub-tiles.
-// ------------------------------------------------------------------------------------
+// fewer sub-tiles.  (Which tiling serves which shape: km_assign below.)
 // HALF: keys and centroids are IEEE half instead of bfloat16.
-template <int KM_TT, int KM_CT, bool HALF>
-__global__ __launch_bounds__(KM_WAVES * 64) void km_assign_kernel(const uint16_t* __restrict__ data,
-                                                                  const uint16_t* __restrict__ cent,
-                                                                  int32_t* __restrict__ assign, int N, int nc,
-                                                                  int seg, int64_t head_rows) {
-  static_assert(KM_CT % (4 * KM_WAVES) == 0 && KM_CT % 32 == 0, "a tile is whole 1 KiB wave loads and whole sub-tiles");
-  constexpr int KM_WG_TOKENS = KM_WAVES * 32 * KM_TT;
-  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[2][KM_CT][RI_DIM];
+// ------------------------------------------------------------------------------------
+template <int V>
+__device__ __forceinline__ void km_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory"); }
+
+template <int KM_TT, int KM_CT, int KM_W, int KM_NB, bool HALF>
+__global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __restrict__ data,
+                                                              const uint16_t* __restrict__ cent,
+                                                              int32_t* __restrict__ assign, int N, int nc,
+                                                              int seg, int64_t head_rows) {
+  static_assert(KM_CT % (4 * KM_W) == 0 && KM_CT % 32 == 0, "a tile is whole 1 KiB wave loads and whole sub-tiles");
+  constexpr int KM_WG_TOKENS = KM_W * 32 * KM_TT;
+  constexpr int L = KM_CT / 4 / KM_W;   // loads of a wave per tile
+  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[KM_NB][KM_CT][RI_DIM];
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 31, hh = lane >> 5;
@@ -69,32 +59,30 @@ __global__ __launch_bounds__(KM_WAVES * 64) void km_assign_kernel(const uint16_t
   const uint32_t sh_base = (uint32_t)(uintptr_t)(km_lds_ptr)&sh_c[0][0][0];
   auto tile_load = [&](int ct, int buf) {
 #pragma unroll
-    for (int u = 0; u < KM_CT / 4 / KM_WAVES; ++u) {
-      const int row4 = (wave + u * KM_WAVES) * 4;      // first of the four rows of this instruction
-      const int row = row4 + ld_row;
-      if (ct + row4 < nc) {  // uniform: nc is a multiple of 32
-        const uint16_t* g = cp + (size_t)(ct + row) * RI_DIM + ((ld_piece ^ (row & 15)) * 8);
-        km_lds_dma16(g, __builtin_amdgcn_readfirstlane(sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2)));
-      }
+    for (int u = 0; u < L; ++u) {
+      const int row4 = (wave + u * KM_W) * 4;      // first of the four rows of this instruction
+      const int row = min(ct + row4, nc - 4) + ld_row;   // (rows past the last repeat it: the count of loads is fixed)
+      const uint16_t* g = cp + (size_t)row * RI_DIM + ((ld_piece ^ ((row4 + ld_row) & 15)) * 8);
+      km_lds_dma16(g, __builtin_amdgcn_readfirstlane(sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2)));
     }
   };
-  tile_load(0, 0);
   uint4 b[KM_TT][8];
 #pragma unroll
   for (int tt = 0; tt < KM_TT; ++tt) {
-    const int tok = t0 + tt * 32 + r;
-    const uint16_t* q = dp + (size_t)tok * RI_DIM + hh * 8;
+    const uint16_t* q = dp + (size_t)min(t0 + tt * 32 + r, N - 1) * RI_DIM + hh * 8;
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) b[tt][kk] = (tok < N) ? ri_ld16(q + kk * 16) : ri_zero16();
+    for (int kk = 0; kk < 8; ++kk) b[tt][kk] = ri_ld16(q + kk * 16);
   }
+  const int tiles = (nc + KM_CT - 1) / KM_CT;
+#pragma unroll
+  for (int t = 0; t < KM_NB - 1; ++t) tile_load(t * KM_CT, t);
   // (the token registers are consumed here so that the compiler's own wait for their loads sits
   // in front of the loop and not inside it, where it would also wait for the tile in flight)
+  km_wait_vm<(KM_NB - 1) * L>();
 #pragma unroll
   for (int tt = 0; tt < KM_TT; ++tt)
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) asm volatile("" : : "v"(b[tt][kk].x));
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+    for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[tt][kk].x), "+v"(b[tt][kk].y), "+v"(b[tt][kk].z), "+v"(b[tt][kk].w));
 
   float best[KM_TT];
   int bidx[KM_TT];
@@ -104,9 +92,10 @@ __global__ __launch_bounds__(KM_WAVES * 64) void km_assign_kernel(const uint16_t
     bidx[tt] = 0;
   }
   int buf = 0;
-  for (int ct = 0; ct < nc; ct += KM_CT, buf ^= 1) {
-    const int nxt = ct + KM_CT;
-    if (nxt < nc) tile_load(nxt, buf ^ 1);
+  for (int ct = 0; ct < nc; ct += KM_CT) {
+    km_wait_vm<(KM_NB - 2) * L>();   // this tile's loads of this wave have landed ...
+    asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
+    tile_load(ct + (KM_NB - 1) * KM_CT, buf == 0 ? KM_NB - 1 : buf - 1);
 #pragma unroll
     for (int half = 0; half < KM_CT / 32; ++half) {
       if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
@@ -146,9 +135,9 @@ __global__ __launch_bounds__(KM_WAVES * 64) void km_assign_kernel(const uint16_t
         }
       }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    buf = buf + 1 == KM_NB ? 0 : buf + 1;
   }
+  km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's)
 #pragma unroll
   for (int tt = 0; tt < KM_TT; ++tt) {
     const float ob = __shfl_xor(best[tt], 32);
@@ -451,30 +440,36 @@ __global__ __launch_bounds__(256) void km_counts_kernel(const int32_t* __restric
 // ------------------------------------------------------------------------------------
 #define KM_BLK 256
 
-// Rows k0 .. k1-1 of a list added in list order.  Sixteen rows per round: the lanes fetch the round's
-// member ids with one load, the ids are broadcast from the lanes, and the sixteen row loads are all
-// in flight before the first add; a short last round adds +0 for its missing rows, which changes no
-// sum.  (Two dependent round trips per sixteen rows instead of two per row for a list's tail.)
-template <bool HALF>
-__device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const int32_t* __restrict__ mem, int k0,
-                                            int k1, float& s0, float& s1) {
+// Rows k0 .. k1-1 of a list added in list order, U per round: the lanes fetch the round's
+// member ids with one load, the ids are broadcast from the lanes, and the row loads (in eights; a short last eight
+// repeats its last row) are all in flight before the first add; a missing row adds +0, which changes no sum.  (Two
+// dependent round trips per U rows instead of two per row for a list's tail.)
+template <bool HALF, int U, typename Id>
+__device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const Id* mem, int k0, int k1, float& s0,
+                                            float& s1) {
+  static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
-  for (int k = k0; k < k1; k += 16) {
-    const int n = min(16, k1 - k);
-    const int id = (lane < n) ? mem[k + lane] : 0;
-    uint32_t v[16];
+  for (int k = k0; k < k1; k += U) {
+    const int n = min(U, k1 - k);
+    const int id = (int)mem[k + min(lane, n - 1)];
+    uint32_t v[U];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int r = __builtin_amdgcn_readlane(id, j);
-      v[j] = (j < n) ? rp[(size_t)r * (RI_DIM / 2)] : 0u;
-    }
+    for (int e = 0; e < U; e += 8)
+      if (e < n) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      float x0, x1;
-      ri_unpack2<HALF>(v[j], x0, x1);   // a missing row reads as the word 0 = (+0, +0) in either type
-      s0 += x0;
-      s1 += x1;
-    }
+        for (int j = e; j < e + 8; ++j) v[j] = rp[(size_t)__builtin_amdgcn_readlane(id, j) * (RI_DIM / 2)];
+      }
+#pragma unroll
+    for (int e = 0; e < U; e += 8)
+      if (e < n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) {
+          float x0, x1;
+          ri_unpack2<HALF>(j < n ? v[j] : 0u, x0, x1);   // the word 0 is (+0, +0) in either type
+          s0 += x0;
+          s1 += x1;
+        }
+      }
   }
 }
 
@@ -545,7 +540,7 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
     int s, o, j;
     if (km_slot_owner(off, nc, slot, s, o, j) < 0) return;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1);
+    km_sum_rows<HALF, 32>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1);
     partial[((size_t)p * cap + slot) * 64 + lane] = make_float2(s0, s1);
     return;
   }
@@ -559,7 +554,7 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1);
+  km_sum_rows<HALF, 32>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1);
   km_finish<MEAN, HALF>(s0, s1, s, normalize, op);
 }
 
@@ -598,6 +593,156 @@ __global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __re
   }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
   km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op);
+}
+
+// ------------------------------------------------------------------------------------
+// update straight from the assignment, for problems of at most KM_DIRECT_MAX tokens (the segments of the segmented
+// iterations): list sort, list-ordered sums and means in one launch, no lists in memory.
+// grid (ceil(nc / CPW), P), eight waves: a workgroup owns CPW consecutive clusters.  Every wave takes a contiguous run of
+// the problem's tokens, compacts those of the workgroup's clusters into LDS (in token order), counts them, and after a
+// scan in (cluster, wave) order scatters them to the workgroup's list in LDS, ranking equal clusters inside a round of 64
+// with ballots: the stable order of the list kernels, hence the same sums.  Then a wave sums whole clusters of at most
+// KM_BLK rows; the blocks of longer ones are spread over the waves and folded in block order.
+// Reading all assignments of the problem per workgroup (4 N bytes) is what the split costs: 32 KB at 8192 tokens, about a
+// microsecond.  128 x 8192 tokens, 512 clusters each: 56 us, bound by reading the keys, against 13 + 70 + 5 us of list
+// sort, sums and fold; 8 x 8192: 9.6 us against 12 + 11 + 4.5.
+// counts / offsets / members (CSR, as km_sort_small_kernel writes them) only when asked for.
+// ------------------------------------------------------------------------------------
+#define KM_DIRECT_WAVES 8
+#define KM_DIRECT_MAX 16384
+
+template <bool HALF, int CPW>
+__global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
+    const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int seg,
+    int64_t head_rows, int normalize) {
+  constexpr int NW = KM_DIRECT_WAVES, SLOTS = CPW * NW;
+  static_assert(SLOTS <= NW * 64, "one (cluster, wave) counter per thread");
+  __shared__ int32_t sh_run[NW][CPW], sh_off[CPW + 1], sh_w[NW], sh_below[NW];
+  extern __shared__ __attribute__((aligned(16))) uint32_t sh_buf[];   // rounds * 512 words: compacted tokens, later block sums
+  // (last problem first: its keys are what the assignment pass has just left in the memory-side cache)
+  const int p = gridDim.y - 1 - blockIdx.y, c0 = blockIdx.x * CPW;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rounds = (N + NW * 64 - 1) / (NW * 64);   // 64-token rounds per wave
+  uint32_t* const mine = sh_buf + wave * rounds * 64;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(sh_buf + NW * rounds * 64);
+  int32_t* run = sh_run[wave];
+  if (lane < CPW) run[lane] = 0;
+  km_wave_lds_sync();
+  const int32_t* as = assign + (size_t)p * N;
+  int cnt = 0, below = 0;   // tokens of this wave in the workgroup's clusters, in lower ones
+  for (int r0 = 0; r0 < rounds; r0 += 8) {
+    int32_t a[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = as[min((wave * rounds + r0 + u) * 64 + lane, N - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = (wave * rounds + r0 + u) * 64 + lane;
+      const bool ok = r0 + u < rounds && i < N;
+      const int loc = a[u] - c0;
+      const bool in = ok && (unsigned)loc < (unsigned)CPW;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+      if (members) below += __popcll(__builtin_amdgcn_ballot_w64(ok && loc < 0));
+      if (in) {
+        mine[__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, cnt))] =
+            (uint32_t)loc << 16 | (uint32_t)i;
+        atomicAdd(&run[loc], 1);
+      }
+      cnt += __popcll(m);
+    }
+  }
+  if (lane == 0) sh_below[wave] = below;
+  __syncthreads();
+  {   // exclusive scan in (cluster, wave) order
+    const int c = tid / NW, w = tid % NW;
+    const int v = tid < SLOTS ? sh_run[w][c] : 0;
+    const int inc = (int)ri_wave_incl_scan((uint32_t)v);
+    if (lane == 63) sh_w[wave] = inc;
+    __syncthreads();
+    int ex = inc - v;
+#pragma unroll
+    for (int x = 0; x < NW; ++x)
+      if (x < wave) ex += sh_w[x];
+    if (tid < SLOTS) {
+      sh_run[w][c] = ex;
+      if (w == 0) sh_off[c] = ex;
+      if (tid == SLOTS - 1) sh_off[CPW] = ex + v;
+    }
+  }
+  __syncthreads();
+  const uint64_t lower = (1ull << lane) - 1ull;
+  for (int k = 0; k < cnt; k += 64) {
+    const bool ok = k + lane < cnt;
+    const uint32_t e = mine[min(k + lane, cnt - 1)];
+    const int c = (int)(e >> 16);
+    uint64_t peers = __builtin_amdgcn_ballot_w64(ok);   // lanes of this round with the same cluster
+#pragma unroll
+    for (int b = 1; b < CPW; b <<= 1) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(ok && (c & b));
+      peers &= (c & b) ? m : ~m;
+    }
+    const int start = run[c];
+    km_wave_lds_sync();  // every lane has read the running position before the leader advances it
+    if (ok) {
+      list[start + __popcll(peers & lower)] = (uint16_t)(e & 0xffffu);
+      if (lane == 63 - __clzll((long long)peers)) run[c] = start + __popcll(peers);
+    }
+    km_wave_lds_sync();
+  }
+  __syncthreads();
+
+  if (members) {
+    int base = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) base += sh_below[w];
+    for (int k = tid; k < sh_off[CPW]; k += NW * 64) members[(size_t)p * N + base + k] = list[k];
+    if (tid < CPW && c0 + tid < nc) {
+      offsets[(size_t)p * (nc + 1) + c0 + tid] = base + sh_off[tid];
+      counts[(size_t)p * nc + c0 + tid] = sh_off[tid + 1] - sh_off[tid];
+    }
+    if (tid == 0 && c0 + CPW >= nc) offsets[(size_t)p * (nc + 1) + nc] = N;
+  }
+  const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM) + lane;
+  uint32_t* op = reinterpret_cast<uint32_t*>(cent + ((size_t)p * nc + c0) * RI_DIM) + lane;
+  // Work items for the waves in turn: the blocks of the long lists first (early iterations have lists of thousands), then
+  // the short lists; no barrier between them.  Block sums go to LDS: the compacted tokens are dead, and the blocks of
+  // lists longer than KM_BLK are at most 2 N / KM_BLK of 512 bytes.
+  float2* const part = reinterpret_cast<float2*>(sh_buf);
+  const int my_o = sh_off[min(lane, CPW - 1)], my_s = lane < CPW ? sh_off[min(lane, CPW - 1) + 1] - my_o : 0;
+  const int my_nb = my_s > KM_BLK ? (my_s + KM_BLK - 1) / KM_BLK : 0;
+  const int nb_incl = (int)ri_wave_incl_scan((uint32_t)my_nb);
+  const int nblocks = __builtin_amdgcn_readlane(nb_incl, 63);
+  for (int k = wave; k < nblocks; k += NW) {
+    const int c = __ffsll((long long)__builtin_amdgcn_ballot_w64(nb_incl > k)) - 1;
+    const int o = __builtin_amdgcn_readlane(my_o, c), s = __builtin_amdgcn_readlane(my_s, c);
+    const int b = k - (__builtin_amdgcn_readlane(nb_incl, c) - __builtin_amdgcn_readlane(my_nb, c));
+    float s0 = 0.f, s1 = 0.f;
+    km_sum_rows<HALF, 64>(rp, list, o + b * KM_BLK, o + min(s, (b + 1) * KM_BLK), s0, s1);
+    part[k * 64 + lane] = make_float2(s0, s1);
+  }
+  // (the wave after the last block's takes the first short list)
+  for (int c = (wave - nblocks) & (NW - 1); c < CPW; c += NW) {   // (a cluster past the last has no tokens; an empty one keeps its centroid)
+    const int o = __builtin_amdgcn_readlane(my_o, c), s = __builtin_amdgcn_readlane(my_s, c);
+    if (s == 0 || s > KM_BLK) continue;
+    float s0 = 0.f, s1 = 0.f;
+    km_sum_rows<HALF, 32>(rp, list, o, o + s, s0, s1);
+    km_finish<true, HALF>(s0, s1, s, normalize, op + c * (RI_DIM / 2));
+  }
+  if (nblocks == 0) return;   // uniform over the workgroup
+  __syncthreads();
+  uint64_t big = __builtin_amdgcn_ballot_w64(my_nb > 0);
+  for (int i = 0; big; big &= big - 1, ++i) {   // a wave folds every eighth long list in block order
+    if ((i & (NW - 1)) != wave) continue;
+    const int c = __ffsll((long long)big) - 1;
+    const int s = __builtin_amdgcn_readlane(my_s, c), nb = __builtin_amdgcn_readlane(my_nb, c);
+    const float2* pp = part + (__builtin_amdgcn_readlane(nb_incl, c) - nb) * 64 + lane;
+    float2 t = pp[0];
+    for (int b = 1; b < nb; ++b) {
+      t.x += pp[b * 64].x;
+      t.y += pp[b * 64].y;
+    }
+    km_finish<true, HALF>(t.x, t.y, s, normalize, op + c * (RI_DIM / 2));
+  }
 }
 
 // out[p, i, :] = in[p, members[p, i], :]; 16 lanes per row
@@ -646,15 +791,25 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
                      int64_t head_rows, ri_stream_t stream) {
   int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
   if (rc) return rc;
-  if (nc > KM_WIDE_MIN_NC) {
-    constexpr int wg_tokens = KM_WAVES * 32 * 4;
-    km_assign_kernel<4, 128, HALF><<<dim3((N + wg_tokens - 1) / wg_tokens, P), KM_WAVES * 64, 0, (hipStream_t)stream>>>(
-        (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows);
-  } else {
-    constexpr int wg_tokens = KM_WAVES * 32 * 2;
-    km_assign_kernel<2, 32, HALF><<<dim3((N + wg_tokens - 1) / wg_tokens, P), KM_WAVES * 64, 0, (hipStream_t)stream>>>(
-        (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows);
-  }
+#define KM_ASSIGN_LAUNCH(TT, CT, W, NB)                                                                                  \
+  km_assign_kernel<TT, CT, W, NB, HALF><<<dim3((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, (hipStream_t)stream>>>( \
+      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows)
+  const long long wgs128 = (long long)P * ((N + 127) / 128), wgs256 = (long long)P * ((N + 255) / 256);
+  const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
+  // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
+  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
+  // against 18.9 with two columns; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
+  if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
+  else if (wgs256 <= 512) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
+  // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
+  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves; 4 x 65536, 4096: 219 against
+  // 232), provided the last round of these large workgroups is not mostly empty.
+  else if (nc > 1024 && wgs1024 * 100 >= rounds1024 * 256 * 87) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
+  // Otherwise the load of the tokens in front of the loop is a large part of the kernel, and 126 registers and 32 KB of
+  // LDS let four workgroups per compute unit overlap one's loads with the others' products (128 x 8192 tokens, 512
+  // centroids: 132 us; 137 with two buffers, 137 with four columns and tiles of 128).
+  else KM_ASSIGN_LAUNCH(2, 32, 4, 4);
+#undef KM_ASSIGN_LAUNCH
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
@@ -788,6 +943,52 @@ extern "C" int ri_kmeans_update_f16(const void* data, const int32_t* counts, con
                                     ri_stream_t stream) {
   return km_update<true>(data, counts, offsets, members, centroids, P, N, nc, seg, head_rows, normalize, workspace,
                          workspace_bytes, stream);
+}
+
+template <bool HALF>
+static int km_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
+                            int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize,
+                            ri_stream_t stream) {
+  if (!data || !assign || !centroids || (!counts != !members) || (!offsets != !members)) return RI_ERR_ARG;
+  if (ri_any_misaligned16(data, centroids)) return RI_ERR_ARG;
+  int rc = km_check(P, N, nc);
+  if (rc) return rc;
+  if (N > KM_DIRECT_MAX || seg <= 0 || P % seg != 0) return RI_ERR_ARG;
+  const int rounds = (N + KM_DIRECT_WAVES * 64 - 1) / (KM_DIRECT_WAVES * 64);
+  // tokens compacted (4 bytes) and listed (2 bytes); block sums of a long cluster (512 bytes per KM_BLK rows) fit there too
+  const size_t lds = (size_t)rounds * KM_DIRECT_WAVES * 64 * 6 + 512;
+#define KM_DIRECT_LAUNCH(CPW)                                                                                         \
+  do {                                                                                                                \
+    km_direct_kernel<HALF, CPW><<<dim3((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>(   \
+        (const uint16_t*)data, assign, (uint16_t*)centroids, counts, offsets, members, N, nc, seg, head_rows,         \
+        normalize);                                                                                                   \
+  } while (0)
+  // As many workgroups as are resident at once (four of 512 threads, as many as the LDS of a compute unit holds): more
+  // of them read the assignments more often and wait for a second round (24 x 8119 tokens, 512 clusters each: 8
+  // clusters per workgroup 20.1 us, 16: 16.2, 32: 19.0; 8 x 8192: 8 clusters 9.6, 64: 21.6; 128 x 8192: 32 clusters
+  // 57.6, 64: 61.2, 16: 66.9).
+  const long long resident = 256 * (long long)min((size_t)4, (160 * 1024) / (lds + 2560));
+  const auto fits = [&](int cpw) { return (long long)P * ((nc + cpw - 1) / cpw) <= resident; };
+  if (fits(8)) KM_DIRECT_LAUNCH(8);
+  else if (fits(16)) KM_DIRECT_LAUNCH(16);
+  else KM_DIRECT_LAUNCH(32);
+#undef KM_DIRECT_LAUNCH
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_kmeans_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
+                                       int32_t* offsets, int32_t* members, int P, int N, int nc, int seg,
+                                       int64_t head_rows, int normalize, ri_stream_t stream) {
+  return km_update_direct<false>(data, assign, centroids, counts, offsets, members, P, N, nc, seg, head_rows, normalize,
+                                 stream);
+}
+
+extern "C" int ri_kmeans_update_direct_f16(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
+                                           int32_t* offsets, int32_t* members, int P, int N, int nc, int seg,
+                                           int64_t head_rows, int normalize, ri_stream_t stream) {
+  return km_update_direct<true>(data, assign, centroids, counts, offsets, members, P, N, nc, seg, head_rows, normalize,
+                                stream);
 }
 
 template <bool HALF>

@@ -533,6 +533,17 @@ def kmeans_update(data, counts, offsets, members, centroids, P, N, nc, seg, head
                                  head_rows, int(bool(normalize)), _p(ws), ws.numel(), _stream()), "kmeans_update")
 
 
+KMEANS_DIRECT_MAX_TOKENS = 16384   # ri_kmeans_update_direct: tokens per problem
+
+
+def kmeans_update_direct(data, assign, centroids, P, N, nc, seg, head_rows, normalize, lists=None):
+    """Lists and means in one launch; lists: (counts, offsets, members) to be written as well."""
+    counts, offsets, members = lists or (None, None, None)
+    check(_fn("ri_kmeans_update_direct", data.dtype)(_p(data), _p(assign), _p(centroids), _p(counts), _p(offsets),
+                                                     _p(members), P, N, nc, seg, head_rows, int(bool(normalize)),
+                                                     _stream()), "kmeans_update_direct")
+
+
 def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot=0):
     ws = _workspace(lib().ri_kmeans_reduce_workspace_bytes(P, N, nc), values.device, f"kmeans_reduce{slot}")
     check(_fn("ri_kmeans_value_sum", values.dtype)(_p(values), _p(counts), _p(offsets), _p(members), _p(value_sum), P, N, nc,

@@ -273,3 +273,38 @@ def test_segment_k_means_teacher_forced(dev, G, N, nc, S, seed, dt=torch.bfloat1
 @pytest.mark.parametrize("G,N,nc,S,seed", [(2, 4096, 256, 4, 10), (2, 3001, 192, 3, 12)])
 def test_segment_k_means_teacher_forced_float16(dev, G, N, nc, S, seed):
     test_segment_k_means_teacher_forced(dev, G, N, nc, S, seed, dt=torch.float16)
+
+
+@pytest.mark.parametrize("P,N,nc,kind", [
+    (3, 1, 32, "even"), (2, 63, 32, "even"), (4, 64, 64, "one"), (2, 513, 96, "even"), (1, 8192, 512, "skew"),
+    (130, 700, 512, "even"), (2, 4100, 1024, "even"), (1, 16384, 512, "one"), (1, 16384, 1024, "skew"), (1, 16383, 32, "even"),
+    (16, 8192, 512, "skew"), (64, 1000, 512, "skew"), (100, 2000, 512, "one"),
+])
+def test_update_direct_equals_lists_and_update(dev, P, N, nc, kind):
+    """Lists and means in one launch against the separate launches, bit for bit: every number of clusters per workgroup,
+    lists longer than a block, a single list, problems that do not fill a round of the waves."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(N + nc)
+    a = torch.randint(0, nc, (P, N), generator=g, dtype=torch.int32)
+    if kind == "one":
+        a[:] = nc // 3
+    elif kind == "skew":
+        big = torch.rand(P, N, generator=g)
+        a[big < 0.5] = 7
+        a[big > 0.8] = nc - 1
+    a = a.to(dev)
+    for dt in (torch.bfloat16, torch.float16):
+        rows = torch.randn(P, N, 128, generator=g).to(dt).to(dev)
+        cent = torch.randn(P, nc, 128, generator=g).to(dt).to(dev)
+        i32 = lambda *s: torch.full(s, -1, dtype=torch.int32, device=dev)
+        lists, got = (i32(P, nc), i32(P, nc + 1), i32(P, N)), (i32(P, nc), i32(P, nc + 1), i32(P, N))
+        kernels.kmeans_build_lists(a, *lists, P, N, nc)
+        for normalize in (True, False):
+            want, direct = cent.clone(), cent.clone()
+            kernels.kmeans_update(rows, *lists, want, P, N, nc, 1, N, normalize)
+            kernels.kmeans_update_direct(rows, a, direct, P, N, nc, 1, N, normalize, got if normalize else None)
+            assert torch.equal(want.view(torch.int16), direct.view(torch.int16))
+        for x, y in zip(lists, got):
+            assert torch.equal(x, y)
+    with pytest.raises(RuntimeError):
+        kernels.kmeans_update_direct(rows, a, cent, P, kernels.KMEANS_DIRECT_MAX_TOKENS + 1, nc, 1, N, True)
