@@ -508,6 +508,41 @@ int ri_lru_access_update(const int32_t* ret_ids, const int32_t* sizes, const int
  * out[p, i, :] = in[p, members[p, i], :] — K/V rows permuted into cluster-contiguous order. */
 int ri_permute_rows(const void* in, const int32_t* members, void* out, int P, int N,
                     int64_t in_stride_rows, int64_t out_stride_rows, ri_stream_t stream);
+/* The same with strides in elements on the side that is read (multiples of 8): rows need not be contiguous. */
+int ri_permute_rows_strided(const void* in, int64_t in_head_stride, int64_t in_row_stride, const int32_t* members,
+                            void* out, int P, int N, int64_t out_stride_rows, ri_stream_t stream);
+
+/* ri_kmeans_value_sum over values whose heads and rows lie head_stride and row_stride elements apart
+   (multiples of 8).  With store, value row members[p][i] is also copied to row p * store_stride_rows + i of it
+   (what ri_permute_rows would write), while it is there for the sum. */
+int ri_kmeans_value_rows(const void* values, int64_t head_stride, int64_t row_stride, const int32_t* counts,
+                         const int32_t* offsets, const int32_t* members, void* value_sum, void* store,
+                         int64_t store_stride_rows, int P, int N, int nc, void* workspace, size_t workspace_bytes,
+                         ri_stream_t stream);
+int ri_kmeans_value_rows_f16(const void* values, int64_t head_stride, int64_t row_stride, const int32_t* counts,
+                             const int32_t* offsets, const int32_t* members, void* value_sum, void* store,
+                             int64_t store_stride_rows, int P, int N, int nc, void* workspace, size_t workspace_bytes,
+                             ri_stream_t stream);
+
+/* Initial centroids: row trunc(c * (N / nc) + N / nc / 2) of every problem, in float32 (kmeans.py:234-236). */
+int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_stream_t stream);
+
+/* ---- prefill around the clustering (retroinfer_cache.py:384-436) ----
+   ri_prefill_split: keys[h][i] = key[first + i][h] for i < N, and the steady zone of both tensors: rows 0..n_start-1
+   of every head from tokens start0.., the following n_end from tokens end0..  Strides in elements, multiples of 8.
+   ri_prefill_center: keys[h][i] -= mean[h], in the element type.
+   ri_prefill_index: out = centroids + mean, mask = (count == 0), sizes as elements and as int32, first rows. */
+int ri_prefill_split(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                     int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
+                     int end0, int n_end, int H, void* keys, void* steady_k, void* steady_v, int64_t steady_stride,
+                     ri_stream_t stream);
+int ri_prefill_center(void* keys, const void* mean, int H, int N, ri_stream_t stream);
+int ri_prefill_center_f16(void* keys, const void* mean, int H, int N, ri_stream_t stream);
+int ri_prefill_index(const void* centroids, const void* mean, const int32_t* counts, const int32_t* offsets, void* out,
+                     uint8_t* mask, void* size16, int32_t* size, int32_t* start, int H, int nc, ri_stream_t stream);
+int ri_prefill_index_f16(const void* centroids, const void* mean, const int32_t* counts, const int32_t* offsets,
+                         void* out, uint8_t* mask, void* size16, int32_t* size, int32_t* start, int H, int nc,
+                         ri_stream_t stream);
 
 /* ------------------------------------------------------------------------------------
  * Host wave buffer (LRU block cache manager + K/V re-organisation) and its thread pool

@@ -67,6 +67,15 @@ SIGNATURES = {
     "ri_kmeans_value_sum": (I, [P, P, P, P, P, I, I, I, P, SZ, P]),
     "ri_kmeans_value_sum_f16": (I, [P, P, P, P, P, I, I, I, P, SZ, P]),
     "ri_permute_rows": (I, [P, P, P, I, I, I64, I64, P]),
+    "ri_permute_rows_strided": (I, [P, I64, I64, P, P, I, I, I64, P]),
+    "ri_kmeans_value_rows": (I, [P, I64, I64, P, P, P, P, P, I64, I, I, I, P, SZ, P]),
+    "ri_kmeans_value_rows_f16": (I, [P, I64, I64, P, P, P, P, P, I64, I, I, I, P, SZ, P]),
+    "ri_kmeans_init": (I, [P, P, I, I, I, P]),
+    "ri_prefill_split": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, I64, P]),
+    "ri_prefill_center": (I, [P, P, I, I, P]),
+    "ri_prefill_center_f16": (I, [P, P, I, I, P]),
+    "ri_prefill_index": (I, [P] * 9 + [I, I, P]),
+    "ri_prefill_index_f16": (I, [P] * 9 + [I, I, P]),
     "ri_threadpool_create": (P, [I]),
     "ri_threadpool_create_pinned": (P, [I, I]),
     "ri_threadpool_pinned_workers": (I, [P]),

@@ -33,8 +33,10 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices):
     dev = key.device
     nc, S = num_centroids, num_segments
     if init_indices is None:
-        init_indices = init_centroid_indices(N, nc, dev)
-    centroids = torch.index_select(key, 1, init_indices).contiguous()
+        centroids = torch.empty((G, nc, D), dtype=key.dtype, device=dev)
+        kernels.kmeans_init(key, centroids, G, N, nc)
+    else:
+        centroids = torch.index_select(key, 1, init_indices).contiguous()
     nseg, ncs = N // S, nc // S
     P = G * S
     if nseg > 0 and num_iters > 1:
@@ -76,9 +78,12 @@ _MAX_GRAPHS = 4
 
 
 def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1, init_indices=None,
-                        reuse_graph=False):
+                        reuse_graph=False, value_sum=None, value_store=None, store_stride=0):
     """Runs the clustering and returns a KMeansResult (no dense cluster lists, no host copy).
-    key/value [G, N, 128] bfloat16 or float16 contiguous device tensors.
+    key/value [G, N, 128] bfloat16 or float16 device tensors, keys contiguous.
+
+    value_sum: [G, nc, 128] tensor for the sums (else a new one).  value_store: where the value rows are also
+    written cluster by cluster, store_stride rows from group to group.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and the same
     shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -96,7 +101,6 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     nc, S = num_centroids, num_segments
     if (nc // S) % 32 != 0 or nc % 32 != 0:
         raise AssertionError("centroids per segment must be a multiple of 32")  # kmeans.py:99
-    value = value.contiguous()
     r = None
     if reuse_graph and not torch.cuda.is_current_stream_capturing():
         gkey = (key.data_ptr(), tuple(key.shape), str(key.device), nc, num_iters, S,
@@ -122,8 +126,9 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
                 _SEEN.popitem(last=False)
     if r is None:
         r = _cluster(key, nc, num_iters, S, init_indices)
-    r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device)
-    kernels.kmeans_value_sum(value, r.counts, r.offsets, r.members, r.value_sum, G, N, nc)
+    r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device) if value_sum is None else value_sum
+    kernels.kmeans_value_sum(kernels.aligned_rows(value), r.counts, r.offsets, r.members, r.value_sum, G, N, nc,
+                             store=value_store, store_stride=store_stride)
     return r
 
 

@@ -328,9 +328,14 @@ class retroinfer_cache(KV_Cache):
             if prev is not None:
                 self.wave_buffer[prev].construction_sync()
 
-        self.temp_keys = key_states[0, vs + sps:seq_len - spe].transpose(0, 1).contiguous()      # [H, N, D]
-        self.temp_values = value_states[0, vs + sps:seq_len - spe].transpose(0, 1).contiguous()
+        # the sequence's K and V stay where they are: heads are taken apart once, for the clustering, and the
+        # store is filled straight from the strided rows
+        keys, values = kernels.aligned_rows(key_states[0]), kernels.aligned_rows(value_states[0])     # [T, H, D]
+        lo = vs + sps
+        head_keys = keys[lo:seq_len - spe].transpose(0, 1)                                            # [H, N, D]
+        head_values = values[lo:seq_len - spe].transpose(0, 1)
         if cpu_organise:
+            self.temp_keys, self.temp_values = head_keys.contiguous(), head_values.contiguous()
             self.mainevents[dkey].record()
             with torch.cuda.stream(self.copystream):
                 self.mainevents[dkey].wait()
@@ -338,50 +343,45 @@ class retroinfer_cache(KV_Cache):
                 self.offload_values[:, :valid_length].copy_(self.temp_values, non_blocking=True)
                 self.copyevents[dkey].record()
 
-        for zone, src in ((self.steady_zone_keys, key_states), (self.steady_zone_values, value_states)):
-            zone[layer_idx][batch_idx, :, :sps] = src[0, vs:vs + sps].transpose(0, 1)
-            zone[layer_idx][batch_idx, :, sps:spt] = src[0, seq_len - spe:seq_len].transpose(0, 1)
-
-        mean_key = torch.mean(self.temp_keys, dim=1, keepdim=True)
         # the centred keys go to a buffer that keeps its address from call to call: the clustering of
         # every further layer and sequence of this length then replays one captured graph
         ck = self._centred_keys.get((dkey, valid_length))
         if ck is None:
             if len(self._centred_keys) >= 2:
                 self._centred_keys.clear()
-            ck = torch.empty_like(self.temp_keys)
+            ck = torch.empty((H, valid_length, head_dim), dtype=keys.dtype, device=keys.device)
             self._centred_keys[(dkey, valid_length)] = ck
-        torch.sub(self.temp_keys, mean_key, out=ck)
-        km = segment_k_means_csr(ck, self.temp_values, self.n_centroids, num_segments=self.n_segment,
-                                 reuse_graph=True)   # results are copied out below, before the next call
-        self.centroids[layer_idx][rows].copy_(km.centroids + mean_key)
-        self.value_sum[layer_idx][rows].copy_(km.value_sum)
-        self.centroids_mask[layer_idx][rows].copy_(km.counts == 0)
-        self.cluster_size[layer_idx][rows].copy_(km.counts.to(self.dtype))
+        kernels.prefill_split(keys, values, lo, valid_length, vs, sps, seq_len - spe, spe, ck,
+                              self.steady_zone_keys[layer_idx][batch_idx], self.steady_zone_values[layer_idx][batch_idx])
+        mean_key = torch.mean(ck, dim=1, keepdim=True)
+        kernels.prefill_center(ck, mean_key)
 
-        # clusters sit in the store in id order, tokens ascending inside (device: permute below; host:
-        # WaveBufferCPU's organisation)
-        self.cluster_start[layer_idx][rows].copy_(km.offsets[:, :self.n_centroids])
-        self.cluster_size_i32[layer_idx][rows].copy_(km.counts)
-        for h in range(H):
-            self.store_rows[layer_idx][batch_idx * H + h] = valid_length
+        # cluster-contiguous store built on the device (stands in for organize_kv on the host): values while
+        # their sums are taken, keys afterwards; clusters in id order, tokens ascending inside
+        store_k = store_v = None
+        stride = 0
         if self.kv_residency == "device":
-            # cluster-contiguous store built on the device (stands in for organize_kv on the host)
-            lk = self.list_keys[layer_idx][batch_idx]
-            lv = self.list_values[layer_idx][batch_idx]
-            kernels.permute_rows(self.temp_keys, km.members, lk, H, valid_length, valid_length, self.list_stride)
-            kernels.permute_rows(self.temp_values, km.members, lv, H, valid_length, valid_length, self.list_stride)
+            store_k, store_v = self.list_keys[layer_idx][batch_idx], self.list_values[layer_idx][batch_idx]
+            stride = self.list_stride
         elif dev_organise:
-            # the same permutation on the device into a staging buffer, then one copy per tensor into
-            # the pinned store on the copy stream (no host-side re-organisation, no dense cluster lists)
+            # into a staging buffer, then one copy per tensor into the pinned store on the copy stream (no
+            # host-side re-organisation, no dense cluster lists)
             self.copyevents[dkey].synchronize()   # the previous copy has left the staging buffers
-            if getattr(self, "stage_keys", None) is None or self.stage_keys.device != self.temp_keys.device:
+            if getattr(self, "stage_keys", None) is None or self.stage_keys.device != keys.device:
                 n_in = self.input_length - self.static_pattern_total
-                self.stage_keys = torch.empty((H, n_in, self.head_dim), dtype=self.dtype, device=self.temp_keys.device)
+                self.stage_keys = torch.empty((H, n_in, self.head_dim), dtype=self.dtype, device=keys.device)
                 self.stage_values = torch.empty_like(self.stage_keys)
-            n_st = self.stage_keys.shape[1]
-            kernels.permute_rows(self.temp_keys, km.members, self.stage_keys, H, valid_length, valid_length, n_st)
-            kernels.permute_rows(self.temp_values, km.members, self.stage_values, H, valid_length, valid_length, n_st)
+            store_k, store_v, stride = self.stage_keys, self.stage_values, self.stage_keys.shape[1]
+        km = segment_k_means_csr(ck, head_values, self.n_centroids, num_segments=self.n_segment,
+                                 reuse_graph=True,   # results are consumed below, before the next call
+                                 value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride)
+        kernels.prefill_index(km.centroids, mean_key, km.counts, km.offsets, self.centroids[layer_idx][rows],
+                              self.centroids_mask[layer_idx][rows], self.cluster_size[layer_idx][rows],
+                              self.cluster_size_i32[layer_idx][rows], self.cluster_start[layer_idx][rows])
+        self.store_rows[layer_idx][rows] = [valid_length] * H
+        if store_k is not None:
+            kernels.permute_rows_strided(head_keys, km.members, store_k, H, valid_length, stride)
+        if dev_organise:
             self.mainevents[dkey].record()
             with torch.cuda.stream(self.copystream):
                 self.mainevents[dkey].wait()
@@ -390,7 +390,7 @@ class retroinfer_cache(KV_Cache):
                 self.list_values[layer_idx][batch_idx, :, :valid_length].copy_(self.stage_values[:, :valid_length],
                                                                                non_blocking=True)
                 self.copyevents[dkey].record()
-        else:
+        elif cpu_organise:
             self.cluster_size_cpu = km.counts.cpu().contiguous()
             self.clusters_cpu = csr_to_dense(km.counts, km.offsets, km.members).cpu().contiguous()
 

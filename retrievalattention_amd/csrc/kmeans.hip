@@ -444,9 +444,10 @@ __global__ __launch_bounds__(256) void km_counts_kernel(const int32_t* __restric
 // member ids with one load, the ids are broadcast from the lanes, and the row loads (in eights; a short last eight
 // repeats its last row) are all in flight before the first add; a missing row adds +0, which changes no sum.  (Two
 // dependent round trips per U rows instead of two per row for a list's tail.)
-template <bool HALF, int U, typename Id>
+// pitch: words between rows.  With wp the rows are also copied: row k of the list to wp + k * 64.
+template <bool HALF, int U, bool COPY = false, typename Id>
 __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const Id* mem, int k0, int k1, float& s0,
-                                            float& s1) {
+                                            float& s1, size_t pitch = RI_DIM / 2, uint32_t* __restrict__ wp = nullptr) {
   static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
   for (int k = k0; k < k1; k += U) {
@@ -457,7 +458,7 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
     for (int e = 0; e < U; e += 8)
       if (e < n) {
 #pragma unroll
-        for (int j = e; j < e + 8; ++j) v[j] = rp[(size_t)__builtin_amdgcn_readlane(id, j) * (RI_DIM / 2)];
+        for (int j = e; j < e + 8; ++j) v[j] = rp[(size_t)__builtin_amdgcn_readlane(id, j) * pitch];
       }
 #pragma unroll
     for (int e = 0; e < U; e += 8)
@@ -468,6 +469,7 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
           ri_unpack2<HALF>(j < n ? v[j] : 0u, x0, x1);   // the word 0 is (+0, +0) in either type
           s0 += x0;
           s1 += x1;
+          if (COPY && j < n) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
         }
       }
   }
@@ -522,25 +524,32 @@ __device__ __forceinline__ int km_slot_owner(const int32_t* __restrict__ off, in
 // grid (item workgroups + ceil(nc / 4), P), four waves each.  The first item_wgs workgroups take
 // one slot per wave (blocks of long lists, their fp32 sums go to partial[p][slot]); the others one
 // cluster per wave.
-template <bool MEAN, bool HALF>
-__global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restrict__ rows,
+// COPY (sums of value rows): every row is also written where its list puts it, row off + k of problem p to
+// copy + (p * copy_stride + off + k) * 128: the cluster-contiguous store, without a second pass over the rows.
+template <bool MEAN, bool HALF, bool COPY>
+__global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restrict__ rows, size_t pitch,
                                                         const int32_t* __restrict__ counts,
                                                         const int32_t* __restrict__ offsets,
                                                         const int32_t* __restrict__ members,
                                                         uint16_t* __restrict__ out, float2* __restrict__ partial,
                                                         int item_wgs, int cap, int N, int nc, int seg,
-                                                        int64_t head_rows, int normalize) {
+                                                        int64_t head_stride, int normalize,
+                                                        uint16_t* __restrict__ copy, int64_t copy_stride) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int32_t* off = offsets + (size_t)p * (nc + 1);
-  const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM) + lane;
+  // (head_stride and pitch in words: the rows of a head need not be contiguous)
+  const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows) + (size_t)(p / seg) * head_stride +
+                       (size_t)(p % seg) * N * pitch + lane;
+  uint32_t* wp = COPY ? reinterpret_cast<uint32_t*>(copy) + (size_t)p * copy_stride * (RI_DIM / 2) + lane : nullptr;
   if ((int)blockIdx.x < item_wgs) {
     const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (slot >= cap) return;
     int s, o, j;
     if (km_slot_owner(off, nc, slot, s, o, j) < 0) return;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, 32>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1);
+    km_sum_rows<HALF, 32, COPY>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1, pitch,
+                                COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr);
     partial[((size_t)p * cap + slot) * 64 + lane] = make_float2(s0, s1);
     return;
   }
@@ -554,7 +563,8 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF, 32>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1);
+  km_sum_rows<HALF, 32, COPY>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1, pitch,
+                              COPY ? wp + (size_t)off[c] * (RI_DIM / 2) : nullptr);
   km_finish<MEAN, HALF>(s0, s1, s, normalize, op);
 }
 
@@ -745,17 +755,27 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
   }
 }
 
-// out[p, i, :] = in[p, members[p, i], :]; 16 lanes per row
+// out[p, i, :] = in[p, members[p, i], :]; 16 lanes per row; strides in 16-byte pieces
 __global__ __launch_bounds__(256) void km_permute_kernel(const uint4* __restrict__ in,
                                                          const int32_t* __restrict__ members,
-                                                         uint4* __restrict__ out, int N, int64_t in_stride,
-                                                         int64_t out_stride) {
+                                                         uint4* __restrict__ out, int N, int64_t in_head,
+                                                         int64_t in_row, int64_t out_head) {
   const int p = blockIdx.y;
   const int i = blockIdx.x * 16 + (threadIdx.x >> 4);
   const int piece = threadIdx.x & 15;
   if (i >= N) return;
   const int32_t src = members[(size_t)p * N + i];
-  out[((size_t)p * out_stride + i) * 16 + piece] = in[((size_t)p * in_stride + src) * 16 + piece];
+  out[(size_t)p * out_head + (size_t)i * 16 + piece] = in[(size_t)p * in_head + (size_t)src * in_row + piece];
+}
+
+// centroids[g, c] = data[g, idx(c)], idx(c) = trunc(c * ratio + half) in fp32 (kmeans.py:234-236); 16 lanes per row
+__global__ __launch_bounds__(256) void km_init_kernel(const uint4* __restrict__ data, uint4* __restrict__ cent, int N,
+                                                      int nc, float ratio, float half) {
+  const int c = blockIdx.x * 16 + (threadIdx.x >> 4), piece = threadIdx.x & 15;
+  if (c >= nc) return;
+  const float x = (float)c * ratio;   // (two roundings: built without fp contraction)
+  const int row = min((int)(x + half), N - 1);
+  cent[((size_t)blockIdx.y * nc + c) * 16 + piece] = data[((size_t)blockIdx.y * N + row) * 16 + piece];
 }
 
 // ------------------------------------------------------------------------------------
@@ -897,18 +917,20 @@ extern "C" size_t ri_kmeans_reduce_workspace_bytes(int P, int N, int nc) {
   return (size_t)P * (size_t)km_item_cap(N) * RI_DIM * sizeof(float) + 256;
 }
 
-template <bool MEAN, bool HALF>
-static int km_reduce(const void* rows, const int32_t* counts, const int32_t* offsets, const int32_t* members,
-                     void* out, int P, int N, int nc, int seg, int64_t head_rows, int normalize, void* workspace,
-                     size_t workspace_bytes, hipStream_t s) {
+// head_stride and row_stride in elements
+template <bool MEAN, bool HALF, bool COPY>
+static int km_reduce(const void* rows, int64_t head_stride, int64_t row_stride, const int32_t* counts,
+                     const int32_t* offsets, const int32_t* members, void* out, int P, int N, int nc, int seg,
+                     int normalize, void* copy, int64_t copy_stride, void* workspace, size_t workspace_bytes,
+                     hipStream_t s) {
   if (workspace_bytes < ri_kmeans_reduce_workspace_bytes(P, N, nc)) return RI_ERR_WORKSPACE;
   const int cap = km_item_cap(N);
   float2* partial = (float2*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   const int item_wgs = (cap + 3) / 4;
   if ((long long)item_wgs + (nc + 3) / 4 > 0x7fffffffLL) return RI_ERR_ARG;
-  km_reduce_kernel<MEAN, HALF><<<dim3(item_wgs + (nc + 3) / 4, P), 256, 0, s>>>(
-      (const uint16_t*)rows, counts, offsets, members, (uint16_t*)out, partial, item_wgs, cap, N, nc, seg, head_rows,
-      normalize);
+  km_reduce_kernel<MEAN, HALF, COPY><<<dim3(item_wgs + (nc + 3) / 4, P), 256, 0, s>>>(
+      (const uint16_t*)rows, (size_t)row_stride / 2, counts, offsets, members, (uint16_t*)out, partial, item_wgs, cap, N,
+      nc, seg, head_stride / 2, normalize, (uint16_t*)copy, copy_stride);
   RI_HIP_CHECK_LAUNCH();
   km_reduce_fold_kernel<MEAN, HALF><<<dim3(item_wgs, P), 256, 0, s>>>(offsets, partial, (uint16_t*)out, cap, nc,
                                                                       normalize);
@@ -925,8 +947,8 @@ static int km_update(const void* data, const int32_t* counts, const int32_t* off
   int rc = km_check(P, N, nc);
   if (rc) return rc;
   if (seg <= 0 || P % seg != 0) return RI_ERR_ARG;
-  return km_reduce<true, HALF>(data, counts, offsets, members, centroids, P, N, nc, seg, head_rows, normalize,
-                               workspace, workspace_bytes, (hipStream_t)stream);
+  return km_reduce<true, HALF, false>(data, head_rows * RI_DIM, RI_DIM, counts, offsets, members, centroids, P, N, nc, seg,
+                                      normalize, nullptr, 0, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int ri_kmeans_update(const void* data, const int32_t* counts, const int32_t* offsets,
@@ -992,36 +1014,79 @@ extern "C" int ri_kmeans_update_direct_f16(const void* data, const int32_t* assi
 }
 
 template <bool HALF>
-static int km_value_sum(const void* values, const int32_t* counts, const int32_t* offsets, const int32_t* members,
-                        void* value_sum, int P, int N, int nc, void* workspace, size_t workspace_bytes,
-                        ri_stream_t stream) {
+static int km_value_rows(const void* values, int64_t head_stride, int64_t row_stride, const int32_t* counts,
+                         const int32_t* offsets, const int32_t* members, void* value_sum, void* store,
+                         int64_t store_stride_rows, int P, int N, int nc, void* workspace, size_t workspace_bytes,
+                         ri_stream_t stream) {
   if (!values || !counts || !offsets || !members || !value_sum || !workspace) return RI_ERR_ARG;
-  if (ri_any_misaligned16(values, value_sum, workspace)) return RI_ERR_ARG;
+  if (ri_any_misaligned16(values, value_sum, store, workspace)) return RI_ERR_ARG;
   int rc = km_check(P, N, nc);
   if (rc) return rc;
-  return km_reduce<false, HALF>(values, counts, offsets, members, value_sum, P, N, nc, 1, (int64_t)N, 0, workspace,
-                                workspace_bytes, (hipStream_t)stream);
+  if (head_stride < 0 || row_stride < RI_DIM || (head_stride | row_stride) % 8 != 0) return RI_ERR_ARG;
+  if (store && store_stride_rows < N) return RI_ERR_ARG;
+  return store ? km_reduce<false, HALF, true>(values, head_stride, row_stride, counts, offsets, members, value_sum, P, N, nc,
+                                              1, 0, store, store_stride_rows, workspace, workspace_bytes,
+                                              (hipStream_t)stream)
+               : km_reduce<false, HALF, false>(values, head_stride, row_stride, counts, offsets, members, value_sum, P, N,
+                                               nc, 1, 0, nullptr, 0, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" int ri_kmeans_value_rows(const void* values, int64_t head_stride, int64_t row_stride, const int32_t* counts,
+                                    const int32_t* offsets, const int32_t* members, void* value_sum, void* store,
+                                    int64_t store_stride_rows, int P, int N, int nc, void* workspace,
+                                    size_t workspace_bytes, ri_stream_t stream) {
+  return km_value_rows<false>(values, head_stride, row_stride, counts, offsets, members, value_sum, store,
+                              store_stride_rows, P, N, nc, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ri_kmeans_value_rows_f16(const void* values, int64_t head_stride, int64_t row_stride,
+                                        const int32_t* counts, const int32_t* offsets, const int32_t* members,
+                                        void* value_sum, void* store, int64_t store_stride_rows, int P, int N, int nc,
+                                        void* workspace, size_t workspace_bytes, ri_stream_t stream) {
+  return km_value_rows<true>(values, head_stride, row_stride, counts, offsets, members, value_sum, store,
+                             store_stride_rows, P, N, nc, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ri_kmeans_value_sum(const void* values, const int32_t* counts, const int32_t* offsets,
                                    const int32_t* members, void* value_sum, int P, int N, int nc, void* workspace,
                                    size_t workspace_bytes, ri_stream_t stream) {
-  return km_value_sum<false>(values, counts, offsets, members, value_sum, P, N, nc, workspace, workspace_bytes, stream);
+  return km_value_rows<false>(values, (int64_t)N * RI_DIM, RI_DIM, counts, offsets, members, value_sum, nullptr, 0, P, N, nc,
+                              workspace, workspace_bytes, stream);
 }
 
 extern "C" int ri_kmeans_value_sum_f16(const void* values, const int32_t* counts, const int32_t* offsets,
                                        const int32_t* members, void* value_sum, int P, int N, int nc, void* workspace,
                                        size_t workspace_bytes, ri_stream_t stream) {
-  return km_value_sum<true>(values, counts, offsets, members, value_sum, P, N, nc, workspace, workspace_bytes, stream);
+  return km_value_rows<true>(values, (int64_t)N * RI_DIM, RI_DIM, counts, offsets, members, value_sum, nullptr, 0, P, N, nc,
+                             workspace, workspace_bytes, stream);
+}
+
+extern "C" int ri_permute_rows_strided(const void* in, int64_t in_head_stride, int64_t in_row_stride,
+                                       const int32_t* members, void* out, int P, int N, int64_t out_stride_rows,
+                                       ri_stream_t stream) {
+  if (!in || !members || !out || P <= 0 || N <= 0 || P > 65535 || in_head_stride < 0 || in_row_stride < RI_DIM ||
+      (in_head_stride | in_row_stride) % 8 != 0 || out_stride_rows < N)
+    return RI_ERR_ARG;
+  if (ri_any_misaligned16(in, out)) return RI_ERR_ARG;
+  km_permute_kernel<<<dim3((N + 15) / 16, P), 256, 0, (hipStream_t)stream>>>(
+      (const uint4*)in, members, (uint4*)out, N, in_head_stride / 8, in_row_stride / 8, out_stride_rows * (RI_DIM / 8));
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
 }
 
 extern "C" int ri_permute_rows(const void* in, const int32_t* members, void* out, int P, int N,
                                int64_t in_stride_rows, int64_t out_stride_rows, ri_stream_t stream) {
-  if (!in || !members || !out || P <= 0 || N <= 0 || P > 65535 || in_stride_rows < N || out_stride_rows < N)
-    return RI_ERR_ARG;
-  if (ri_any_misaligned16(in, out)) return RI_ERR_ARG;
-  km_permute_kernel<<<dim3((N + 15) / 16, P), 256, 0, (hipStream_t)stream>>>(
-      (const uint4*)in, members, (uint4*)out, N, in_stride_rows, out_stride_rows);
+  if (in_stride_rows < N) return RI_ERR_ARG;
+  return ri_permute_rows_strided(in, in_stride_rows * RI_DIM, RI_DIM, members, out, P, N, out_stride_rows, stream);
+}
+
+extern "C" int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_stream_t stream) {
+  if (!data || !centroids || ri_any_misaligned16(data, centroids)) return RI_ERR_ARG;
+  int rc = km_check(P, N, nc);
+  if (rc) return rc;
+  const double ratio = (double)N / nc;
+  km_init_kernel<<<dim3((nc + 15) / 16, P), 256, 0, (hipStream_t)stream>>>((const uint4*)data, (uint4*)centroids, N, nc,
+                                                                           (float)ratio, (float)(ratio / 2));
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

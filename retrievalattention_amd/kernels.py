@@ -544,10 +544,64 @@ def kmeans_update_direct(data, assign, centroids, P, N, nc, seg, head_rows, norm
                                                      _stream()), "kmeans_update_direct")
 
 
-def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot=0):
+def _rows_ok(t):
+    return t.stride(-1) == 1 and t.stride(-2) % 8 == 0 and t.stride(-3) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
+def aligned_rows(t):
+    """t if its 128-element rows can be read 16 bytes at a time where they lie, else a contiguous copy."""
+    return t if _rows_ok(t) else t.clone(memory_format=torch.contiguous_format)
+
+
+def _row_strides(t, what):
+    """Strides in elements of the two outer dimensions of [., ., 128] rows read 16 bytes at a time."""
+    if not _rows_ok(t):
+        raise ValueError(f"{what}: rows must be contiguous and 16-byte aligned")
+    return t.stride(0), t.stride(1)
+
+
+def kmeans_init(data, centroids, P, N, nc):
+    check(lib().ri_kmeans_init(_p(data), _p(centroids), P, N, nc, _stream()), "kmeans_init")
+
+
+def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot=0, store=None, store_stride=0):
+    """values [P, N, 128], strided or not; store: the cluster-contiguous value rows are written there as well."""
     ws = _workspace(lib().ri_kmeans_reduce_workspace_bytes(P, N, nc), values.device, f"kmeans_reduce{slot}")
-    check(_fn("ri_kmeans_value_sum", values.dtype)(_p(values), _p(counts), _p(offsets), _p(members), _p(value_sum), P, N, nc,
-                                    _p(ws), ws.numel(), _stream()), "kmeans_value_sum")
+    head, row = _row_strides(values, "kmeans_value_sum")
+    check(_fn("ri_kmeans_value_rows", values.dtype)(_p(values), head, row, _p(counts), _p(offsets), _p(members),
+                                                    _p(value_sum), _p(store), store_stride, P, N, nc, _p(ws), ws.numel(),
+                                                    _stream()), "kmeans_value_sum")
+
+
+def permute_rows_strided(src, members, dst, P, N, out_stride_rows):
+    """permute_rows from [P, N, 128] rows with strides of their own."""
+    head, row = _row_strides(src, "permute_rows")
+    check(lib().ri_permute_rows_strided(_p(src), head, row, _p(members), _p(dst), P, N, out_stride_rows, _stream()),
+          "permute_rows")
+
+
+def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, steady_k, steady_v):
+    """keys/values [T, H, 128]; out [H, N, 128]; steady_k/v [H, rows, 128]."""
+    kr, kh = _row_strides(keys, "prefill_split")
+    vr, vh = _row_strides(values, "prefill_split")
+    T, H = keys.shape[0], keys.shape[1]
+    if first + N > T or start0 + n_start > T or end0 + n_end > T or n_start + n_end > steady_k.shape[1]:
+        raise ValueError("prefill_split: rows outside the sequence")
+    if not keys.dtype == values.dtype == out.dtype == steady_k.dtype == steady_v.dtype:
+        raise TypeError("prefill_split: keys, values and the cache must have the same element type")
+    check(lib().ri_prefill_split(_p(keys), _p(values), kr, kh, vr, vh, first, N, start0, n_start, end0, n_end, H, _p(out),
+                                 _p(steady_k), _p(steady_v), steady_k.stride(0) // 128, _stream()), "prefill_split")
+
+
+def prefill_center(keys, mean):
+    H, N, _ = keys.shape
+    check(_fn("ri_prefill_center", keys.dtype)(_p(keys), _p(mean), H, N, _stream()), "prefill_center")
+
+
+def prefill_index(centroids, mean, counts, offsets, out, mask, size16, size, start):
+    H, nc, _ = centroids.shape
+    check(_fn("ri_prefill_index", centroids.dtype)(_p(centroids), _p(mean), _p(counts), _p(offsets), _p(out), _p(mask),
+                                                   _p(size16), _p(size), _p(start), H, nc, _stream()), "prefill_index")
 
 
 def permute_rows(src, members, dst, P, N, in_stride_rows, out_stride_rows):

@@ -1,0 +1,61 @@
+"""The passes around the prefill clustering against torch, bit for bit: heads taken apart, keys centred, initial
+centroids, value rows summed and stored, index entries (GPU)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,nc,fused", [(1, 1, 32, False), (2, 63, 32, True), (3, 65, 64, False), (8, 1000, 96, True),
+                                          (2, 20001, 1088, False)])
+def test_prefill_passes(dev, dtype, H, N, nc, fused):
+    from retrievalattention_amd import kernels
+    from retrievalattention_amd.cache_hub.kmeans import init_centroid_indices
+    g = torch.Generator().manual_seed(H * N + nc)
+    vs, sps, spe = 5, 3, 17
+    T = vs + sps + N + spe
+    if fused:      # keys and values as slices of one projection: rows further apart than their heads fill
+        kv = torch.randn(T, 2, H, 128, generator=g).to(dtype).to(dev)
+        K, V = kv[:, 0], kv[:, 1]
+    else:
+        K, V = (torch.randn(T, H, 128, generator=g).to(dtype).to(dev) for _ in range(2))
+    lo = vs + sps
+    hk, hv = K[lo:lo + N].transpose(0, 1), V[lo:lo + N].transpose(0, 1)
+    ck = torch.empty((H, N, 128), dtype=dtype, device=dev)
+    zk, zv = (torch.zeros((H, sps + spe + 2, 128), dtype=dtype, device=dev) for _ in range(2))
+    kernels.prefill_split(K, V, lo, N, vs, sps, lo + N, spe, ck, zk, zv)
+    assert torch.equal(ck, hk)
+    for z, src in ((zk, K), (zv, V)):
+        ref = torch.cat((src[vs:lo], src[lo + N:], torch.zeros_like(src[:2])))
+        assert torch.equal(z, ref.transpose(0, 1))
+
+    mean = torch.mean(ck, dim=1, keepdim=True)
+    centred = ck - mean
+    kernels.prefill_center(ck, mean)
+    assert torch.equal(ck, centred)
+
+    cent = torch.empty((H, nc, 128), dtype=dtype, device=dev)
+    kernels.kmeans_init(ck, cent, H, N, nc)
+    assert torch.equal(cent, ck[:, init_centroid_indices(N, nc, dev)])
+
+    assign = torch.randint(0, nc - 1, (H, N), generator=g, dtype=torch.int32)      # the last cluster stays empty
+    assign[:, : N // 2] = 3                                                        # one list beyond a block of sums
+    assign = assign.to(dev)
+    counts, offsets, members = (torch.empty(s, dtype=torch.int32, device=dev) for s in ((H, nc), (H, nc + 1), (H, N)))
+    kernels.kmeans_build_lists(assign, counts, offsets, members, H, N, nc)
+    sums, ref_sums = (torch.empty((H, nc, 128), dtype=dtype, device=dev) for _ in range(2))
+    store, store_k = (torch.zeros((H, N + 7, 128), dtype=dtype, device=dev) for _ in range(2))
+    kernels.kmeans_value_sum(hv.contiguous(), counts, offsets, members, ref_sums, H, N, nc)
+    kernels.kmeans_value_sum(hv, counts, offsets, members, sums, H, N, nc, store=store, store_stride=N + 7)
+    kernels.permute_rows_strided(hk, members, store_k, H, N, N + 7)
+    at = members.long()[:, :, None].expand(-1, -1, 128)
+    assert torch.equal(sums, ref_sums)
+    for st, src in ((store, hv), (store_k, hk)):
+        assert torch.equal(st[:, :N], torch.gather(src, 1, at)) and not st[:, N:].any()
+
+    out, mask = torch.empty_like(cent), torch.empty((H, nc), dtype=torch.bool, device=dev)
+    size16, size, start = torch.empty((H, nc), dtype=dtype, device=dev), torch.empty_like(counts), torch.empty_like(counts)
+    kernels.prefill_index(cent, mean, counts, offsets, out, mask, size16, size, start)
+    assert torch.equal(out, cent + mean) and torch.equal(mask, counts == 0) and torch.equal(size16, counts.to(dtype))
+    assert torch.equal(size, counts) and torch.equal(start, offsets[:, :nc])
