@@ -621,6 +621,50 @@ __global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __re
 #define KM_DIRECT_WAVES 8
 #define KM_DIRECT_MAX 16384
 
+#define KM_DIRECT_SHORT 128   // longer lists are summed in blocks and folded, as lists of several blocks are
+// Rows k0 .. k1-1 of a list in LDS added in list order, U per round: ids come with one LDS read and are broadcast from the
+// lanes as buffer offsets, the loads of a round (in eights; a short last eight repeats its last row, and adds +0 for it,
+// which changes no sum) are all in flight before the first add.  A wave's own chain bounds a list: two instructions fetch
+// a row and two per dim add it (an address per row in 64 bits, and a select per row, made it ten; 8 x 8192 tokens, 512
+// clusters: 10.6 -> 9.6 us; 128 x 8192: 67.6 -> 61.6).  WHOLE: two dims per lane, else one (two waves share the row).
+template <bool HALF, int U, bool WHOLE>
+__device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint32_t byte, const uint16_t* list, int k0, int k1,
+                                              float& s0, float& s1) {
+  static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
+  const int lane = threadIdx.x & 63;
+  const auto add = [&](uint32_t w) {
+    float x0, x1;
+    ri_unpack2<HALF>(w, x0, x1);
+    s0 += x0;
+    if (WHOLE) s1 += x1;
+  };
+  for (int k = k0; k < k1; k += U) {
+    const int n = min(U, k1 - k);
+    const int off = (int)list[k + min(lane, n - 1)] * (RI_DIM * 2);
+    uint32_t v[U];
+#pragma unroll
+    for (int e = 0; e < U; e += 8)
+      if (e < n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) {
+          const int so = __builtin_amdgcn_readlane(off, j);
+          v[j] = WHOLE ? __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so, 0)
+                       : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, byte, so, 0);
+        }
+      }
+#pragma unroll
+    for (int e = 0; e < U; e += 8) {
+      if (e + 8 <= n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) add(v[j]);
+      } else if (e < n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) add(j < n ? v[j] : 0u);   // the word 0 is (+0, +0) in either type
+      }
+    }
+  }
+}
+
 template <bool HALF, int CPW>
 __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
     const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
@@ -712,30 +756,41 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
     }
     if (tid == 0 && c0 + CPW >= nc) offsets[(size_t)p * (nc + 1) + nc] = N;
   }
-  const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM) + lane;
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM), 0, N * RI_DIM * 2, 0x00020000);
   uint32_t* op = reinterpret_cast<uint32_t*>(cent + ((size_t)p * nc + c0) * RI_DIM) + lane;
   // Work items for the waves in turn: the blocks of the long lists first (early iterations have lists of thousands), then
-  // the short lists; no barrier between them.  Block sums go to LDS: the compacted tokens are dead, and the blocks of
-  // lists longer than KM_BLK are at most 2 N / KM_BLK of 512 bytes.
-  float2* const part = reinterpret_cast<float2*>(sh_buf);
+  // the short lists; no barrier between them.  Block sums go to LDS: the compacted tokens are dead, and lists longer than
+  // KM_DIRECT_SHORT have at most N / KM_DIRECT_SHORT blocks of 512 bytes.  A block of 256 rows is a long chain, so
+  // its two halves go to two waves while every wave gets one at most (with more blocks that would only be twice the
+  // loads): the four early iterations of 8 x 8192 tokens 104 -> 84 us together, three of 128 x 8192 267 -> 216.
+  float* const part = reinterpret_cast<float*>(sh_buf);
   const int my_o = sh_off[min(lane, CPW - 1)], my_s = lane < CPW ? sh_off[min(lane, CPW - 1) + 1] - my_o : 0;
-  const int my_nb = my_s > KM_BLK ? (my_s + KM_BLK - 1) / KM_BLK : 0;
+  const int my_nb = my_s > KM_DIRECT_SHORT ? (my_s + KM_BLK - 1) / KM_BLK : 0;
   const int nb_incl = (int)ri_wave_incl_scan((uint32_t)my_nb);
   const int nblocks = __builtin_amdgcn_readlane(nb_incl, 63);
-  for (int k = wave; k < nblocks; k += NW) {
-    const int c = __ffsll((long long)__builtin_amdgcn_ballot_w64(nb_incl > k)) - 1;
+  const int halves = 2 * nblocks <= NW ? 2 : 1, items = halves * nblocks;
+  for (int k = wave; k < items; k += NW) {
+    const int blk = halves == 2 ? k >> 1 : k;
+    const int c = __ffsll((long long)__builtin_amdgcn_ballot_w64(nb_incl > blk)) - 1;
     const int o = __builtin_amdgcn_readlane(my_o, c), s = __builtin_amdgcn_readlane(my_s, c);
-    const int b = k - (__builtin_amdgcn_readlane(nb_incl, c) - __builtin_amdgcn_readlane(my_nb, c));
+    const int b = blk - (__builtin_amdgcn_readlane(nb_incl, c) - __builtin_amdgcn_readlane(my_nb, c));
+    const int k0 = o + b * KM_BLK, k1 = o + min(s, (b + 1) * KM_BLK);
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, 64>(rp, list, o + b * KM_BLK, o + min(s, (b + 1) * KM_BLK), s0, s1);
-    part[k * 64 + lane] = make_float2(s0, s1);
+    if (halves == 2) {
+      km_sum_listed<HALF, 64, false>(rp, (k & 1) * RI_DIM + lane * 2, list, k0, k1, s0, s1);
+      part[k * 64 + lane] = s0;
+    } else {
+      km_sum_listed<HALF, 64, true>(rp, lane * 4, list, k0, k1, s0, s1);
+      reinterpret_cast<float2*>(part)[k * 64 + lane] = make_float2(s0, s1);
+    }
   }
   // (the wave after the last block's takes the first short list)
-  for (int c = (wave - nblocks) & (NW - 1); c < CPW; c += NW) {   // (a cluster past the last has no tokens; an empty one keeps its centroid)
+  for (int c = (wave - items) & (NW - 1); c < CPW; c += NW) {   // (a cluster past the last has no tokens; an empty one keeps its centroid)
     const int o = __builtin_amdgcn_readlane(my_o, c), s = __builtin_amdgcn_readlane(my_s, c);
-    if (s == 0 || s > KM_BLK) continue;
+    if (s == 0 || s > KM_DIRECT_SHORT) continue;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, 32>(rp, list, o, o + s, s0, s1);
+    km_sum_listed<HALF, 32, true>(rp, lane * 4, list, o, o + s, s0, s1);
     km_finish<true, HALF>(s0, s1, s, normalize, op + c * (RI_DIM / 2));
   }
   if (nblocks == 0) return;   // uniform over the workgroup
@@ -745,7 +800,7 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
     if ((i & (NW - 1)) != wave) continue;
     const int c = __ffsll((long long)big) - 1;
     const int s = __builtin_amdgcn_readlane(my_s, c), nb = __builtin_amdgcn_readlane(my_nb, c);
-    const float2* pp = part + (__builtin_amdgcn_readlane(nb_incl, c) - nb) * 64 + lane;
+    const float2* pp = reinterpret_cast<const float2*>(part) + (__builtin_amdgcn_readlane(nb_incl, c) - nb) * 64 + lane;
     float2 t = pp[0];
     for (int b = 1; b < nb; ++b) {
       t.x += pp[b * 64].x;

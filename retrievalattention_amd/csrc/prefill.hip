@@ -7,8 +7,10 @@
 
 // ------------------------------------------------------------------------------------
 // split: keys[h, i] = K[first + i, h] for the clustered range, and the steady rows of K and V.
-// 16 lanes per row, a workgroup moves 64 rows of one head.  Heads vary fastest over the workgroups, so those in
-// flight together read whole tokens.  Workgroups behind the clustered range move the steady rows.
+// 16 lanes per row, a workgroup moves 16 rows of one head: occupancy keeps more loads in flight than several rows per
+// thread do (8 heads of 8K / 128K tokens: 6.7 / 93 us; two or four rows per thread 19 / 105).  Heads vary fastest over
+// the workgroups, so those in flight together read whole tokens.  Workgroups behind the clustered range move the steady
+// rows.
 // ------------------------------------------------------------------------------------
 struct SplitParams {
   const uint4* k;
@@ -18,22 +20,15 @@ struct SplitParams {
   uint4* zone_v;
   int64_t k_row, k_head, v_row, v_head;   // pieces between tokens and between heads
   int64_t zone_stride;                    // rows between heads
-  int first, N, start0, end0, n_start, n_end, H, blocks;   // blocks: of 64 clustered rows
+  int first, N, start0, end0, n_start, n_end, H, blocks;   // blocks: of 16 clustered rows
 };
 
 __global__ __launch_bounds__(256) void split_kernel(SplitParams P) {
   const int h = blockIdx.x % P.H, blk = blockIdx.x / P.H;
   const int piece = threadIdx.x & 15, sub = threadIdx.x >> 4;
   if (blk < P.blocks) {
-    const int i0 = blk * 64 + sub;
-    const uint4* kp = P.k + h * P.k_head + P.first * P.k_row + piece;
-    uint4* out = P.keys + (int64_t)h * P.N * 16 + piece;
-    uint4 x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = kp[min(i0 + 16 * u, P.N - 1) * P.k_row];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + 16 * u < P.N) out[(int64_t)(i0 + 16 * u) * 16] = x[u];
+    const int i = blk * 16 + sub;
+    if (i < P.N) P.keys[((int64_t)h * P.N + i) * 16 + piece] = P.k[h * P.k_head + (P.first + (int64_t)i) * P.k_row + piece];
     return;
   }
   const int i = (blk - P.blocks) * 16 + sub;
@@ -55,7 +50,7 @@ extern "C" int ri_prefill_split(const void* key, const void* value, int64_t key_
       steady_stride < n_start + n_end || key_row_stride < 0 || key_head_stride < 0 || value_row_stride < 0 ||
       value_head_stride < 0 || (key_row_stride | key_head_stride | value_row_stride | value_head_stride) % 8 != 0)
     return RI_ERR_ARG;
-  const int blocks = N / 64 + (N % 64 != 0);
+  const int blocks = N / 16 + (N % 16 != 0);
   const int64_t wgs = ((int64_t)blocks + ((int64_t)n_start + n_end + 15) / 16) * H;
   if (wgs > 0x7fffffffLL) return RI_ERR_ARG;
   const SplitParams P = {(const uint4*)key, (const uint4*)value, (uint4*)keys, (uint4*)steady_k, (uint4*)steady_v,
@@ -68,7 +63,7 @@ extern "C" int ri_prefill_split(const void* key, const void* value, int64_t key_
 
 // ------------------------------------------------------------------------------------
 // center: keys[h, i] -= mean[h] (16-bit arithmetic: both operands widened, the difference rounded), in place.
-// grid (rows / 64, H), 16 lanes per row, four rows per thread.
+// grid (ceil(rows / 16), H), 16 lanes per row.
 // ------------------------------------------------------------------------------------
 template <bool HALF>
 __device__ __forceinline__ uint32_t sub2(uint32_t a, uint32_t b) {
@@ -80,23 +75,16 @@ __device__ __forceinline__ uint32_t sub2(uint32_t a, uint32_t b) {
 
 template <bool HALF>
 __global__ __launch_bounds__(256) void center_kernel(uint4* __restrict__ keys, const uint4* __restrict__ mean, int N) {
-  const int piece = threadIdx.x & 15;
-  uint4* kp = keys + (size_t)blockIdx.y * N * 16 + piece;
-  const uint4 m = mean[(size_t)blockIdx.y * 16 + piece];
-  const int i0 = blockIdx.x * 64 + (threadIdx.x >> 4);
-  uint4 x[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) x[u] = kp[(size_t)min(i0 + 16 * u, N - 1) * 16];
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (i0 + 16 * u < N)
-      kp[(size_t)(i0 + 16 * u) * 16] = make_uint4(sub2<HALF>(x[u].x, m.x), sub2<HALF>(x[u].y, m.y),
-                                                  sub2<HALF>(x[u].z, m.z), sub2<HALF>(x[u].w, m.w));
+  const int i = blockIdx.x * 16 + (threadIdx.x >> 4), piece = threadIdx.x & 15;
+  if (i >= N) return;
+  uint4* kp = keys + ((size_t)blockIdx.y * N + i) * 16 + piece;
+  const uint4 x = *kp, m = mean[(size_t)blockIdx.y * 16 + piece];
+  *kp = make_uint4(sub2<HALF>(x.x, m.x), sub2<HALF>(x.y, m.y), sub2<HALF>(x.z, m.z), sub2<HALF>(x.w, m.w));
 }
 
 static int prefill_center(void* keys, const void* mean, int H, int N, bool half, ri_stream_t stream) {
   if (!keys || !mean || ri_any_misaligned16(keys, mean) || H <= 0 || H > 65535 || N <= 0) return RI_ERR_ARG;
-  const dim3 grid((N + 63) / 64, H);
+  const dim3 grid(N / 16 + (N % 16 != 0), H);
   if (half) center_kernel<true><<<grid, 256, 0, (hipStream_t)stream>>>((uint4*)keys, (const uint4*)mean, N);
   else center_kernel<false><<<grid, 256, 0, (hipStream_t)stream>>>((uint4*)keys, (const uint4*)mean, N);
   RI_HIP_CHECK_LAUNCH();
