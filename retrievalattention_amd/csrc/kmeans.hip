@@ -154,15 +154,17 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
 // ------------------------------------------------------------------------------------
 // inverted lists
 // ------------------------------------------------------------------------------------
-// Inverted lists are a stable sort of the token ids by cluster id: one or two least-significant-
-// digit counting passes of at most 9 bits.  A pass is three launches: per-chunk digit histograms
-// (one wave per chunk of KM_SORT_CHUNK tokens, wave-private LDS counters), an exclusive scan of
-// the [digit][chunk] table per problem, and a scatter in which every wave walks its chunk in
-// token order, ranks equal digits inside each 64-token round with ballots and keeps running
-// positions in LDS.  Stability makes every list ascending without any per-list sort, and no
-// global atomics are involved, so the result does not depend on scheduling.
+// Inverted lists are a stable sort of the token ids by cluster id.  Ids of at most 9 bits take one counting pass, three
+// launches: per-chunk digit histograms (KM_SORT_CHUNK tokens, LDS counters), an exclusive scan of the [digit][chunk]
+// table per problem, and a scatter in which every wave walks its part of a chunk in token order, ranks equal digits
+// inside each 64-token round with ballots and keeps running positions in LDS.  Longer ids take that pass over their upper
+// digit and one launch that sorts every bucket of it by the lower digit in a workgroup and writes offsets and counts on
+// the way.  Stability makes every list ascending without any per-list sort, and no global atomics are involved, so the
+// result does not depend on scheduling.  Every launch is a short serial chain, so chunks are shared by four waves and
+// tables are read in one round trip (all launches of 4 x 48787 tokens, 3040 clusters: 16.0 us; two passes of three
+// launches with a wave per chunk, a search of the bounds and their differences: 38.5; 8 x 131072, 8192: 25.2 and 62.8).
 #define KM_SORT_CHUNK 1024
-#define KM_SORT_ROUNDS (KM_SORT_CHUNK / 64)
+#define KM_SORT_ROUNDS (KM_SORT_CHUNK / 256)   // 64-token rounds of each of the four waves of a chunk
 #define KM_SORT_MAX_BINS 512
 
 __device__ __forceinline__ void km_wave_lds_sync() {
@@ -171,31 +173,23 @@ __device__ __forceinline__ void km_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// chunk_hist[p][digit][chunk] = tokens of the chunk whose key has that digit
+// chunk_hist[p][digit][chunk] = tokens of the chunk whose key has that digit; a workgroup per chunk
 __global__ __launch_bounds__(256) void km_sort_hist_kernel(const int32_t* __restrict__ keys,
                                                            int32_t* __restrict__ chunk_hist, int N, int nchunks,
                                                            int shift, int bits) {
-  __shared__ int32_t sh[4][KM_SORT_MAX_BINS];
-  const int p = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int chunk = blockIdx.x * 4 + wave;
-  const int bins = 1 << bits;
-  if (chunk >= nchunks) return;
-  int32_t* h = sh[wave];
-  for (int b = lane; b < bins; b += 64) h[b] = 0;
-  km_wave_lds_sync();
-  const int base = chunk * KM_SORT_CHUNK;
+  __shared__ int32_t h[KM_SORT_MAX_BINS];
+  const int p = blockIdx.y, chunk = blockIdx.x, bins = 1 << bits;
+  const int i0 = chunk * KM_SORT_CHUNK + threadIdx.x;
   int32_t k[KM_SORT_ROUNDS];
 #pragma unroll
-  for (int r = 0; r < KM_SORT_ROUNDS; ++r) {
-    const int i = base + r * 64 + lane;
-    k[r] = (i < N) ? keys[(size_t)p * N + i] : -1;
-  }
+  for (int r = 0; r < KM_SORT_ROUNDS; ++r) k[r] = keys[(size_t)p * N + min(i0 + r * 256, N - 1)];
+  for (int b = threadIdx.x; b < bins; b += 256) h[b] = 0;
+  __syncthreads();
 #pragma unroll
   for (int r = 0; r < KM_SORT_ROUNDS; ++r)
-    if (base + r * 64 + lane < N) atomicAdd(&h[(k[r] >> shift) & (bins - 1)], 1);
-  km_wave_lds_sync();
-  for (int b = lane; b < bins; b += 64) chunk_hist[((size_t)p * bins + b) * nchunks + chunk] = h[b];
+    if (i0 + r * 256 < N) atomicAdd(&h[(k[r] >> shift) & (bins - 1)], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < bins; b += 256) chunk_hist[((size_t)p * bins + b) * nchunks + chunk] = h[b];
 }
 
 // in-place exclusive prefix sum over the n = bins * nchunks entries of each problem.
@@ -211,35 +205,31 @@ __global__ __launch_bounds__(1024) void km_sort_scan_kernel(int32_t* __restrict_
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (threadIdx.x == 0) sh_carry = 0;
   __syncthreads();
-  for (int base = 0; base < n; base += 4096) {
-    const int i0 = base + threadIdx.x * 4;
-    int32_t v[4], run = 0;
+  // sixteen rows of 64 entries per wave and round: a table of 128 digits and 128 chunks is one round trip
+  for (int base = 0; base < n; base += 16 * 1024) {
+    const int i0 = base + wave * 1024 + lane;
+    int32_t v[16], x[16], run = 0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      v[u] = (i0 + u < n) ? a[i0 + u] : 0;
-      run += v[u];
-    }
-    int32_t inc = run;
+    for (int u = 0; u < 16; ++u) v[u] = a[min(i0 + u * 64, n - 1)];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int32_t o = __shfl_up(inc, d);
-      if (lane >= d) inc += o;
+    for (int u = 0; u < 16; ++u) {
+      if (i0 + u * 64 >= n) v[u] = 0;
+      const int32_t inc = (int32_t)ri_wave_incl_scan((uint32_t)v[u]);
+      x[u] = run + inc - v[u];
+      run += __builtin_amdgcn_readlane(inc, 63);
     }
-    if (lane == 63) sh_w[wave] = inc;
+    if (lane == 0) sh_w[wave] = run;
     __syncthreads();
-    int32_t woff = 0, tot = 0;
+    int32_t ex = sh_carry, tot = 0;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
-      const int32_t x = sh_w[w];
-      if (w < wave) woff += x;
-      tot += x;
+      const int32_t y = sh_w[w];
+      if (w < wave) ex += y;
+      tot += y;
     }
-    int32_t ex = sh_carry + woff + inc - run;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (i0 + u < n) a[i0 + u] = ex;
-      ex += v[u];
-    }
+    for (int u = 0; u < 16; ++u)
+      if (i0 + u * 64 < n) a[i0 + u * 64] = ex + x[u];
     __syncthreads();
     if (threadIdx.x == 0) sh_carry += tot;
     __syncthreads();
@@ -257,48 +247,61 @@ __global__ __launch_bounds__(1024) void km_sort_scan_kernel(int32_t* __restrict_
   }
 }
 
-// toks == nullptr: token id = position (first pass); out_keys == nullptr: last pass
+// A workgroup per chunk; its four waves take 256 consecutive tokens each and count their digits first, so that each knows
+// where it starts.  low >= 0: token << low | the id's low bits, else the token.
 __global__ __launch_bounds__(256) void km_sort_scatter_kernel(const int32_t* __restrict__ keys,
-                                                              const int32_t* __restrict__ toks,
                                                               const int32_t* __restrict__ chunk_hist,
-                                                              int32_t* __restrict__ out_keys,
                                                               int32_t* __restrict__ out_toks, int N, int nchunks,
-                                                              int shift, int bits) {
+                                                              int shift, int bits, int low) {
   __shared__ int32_t sh[4][KM_SORT_MAX_BINS];
-  const int p = blockIdx.y;
+  const int p = blockIdx.y, chunk = blockIdx.x, bins = 1 << bits;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int chunk = blockIdx.x * 4 + wave;
-  const int bins = 1 << bits;
-  if (chunk >= nchunks) return;
+  const int i0 = chunk * KM_SORT_CHUNK + wave * (KM_SORT_CHUNK / 4) + lane;
   int32_t* run = sh[wave];
-  for (int b = lane; b < bins; b += 64) run[b] = chunk_hist[((size_t)p * bins + b) * nchunks + chunk];
-  const int base = chunk * KM_SORT_CHUNK;
-  int32_t k[KM_SORT_ROUNDS], t[KM_SORT_ROUNDS];
+  int32_t k[KM_SORT_ROUNDS];
 #pragma unroll
-  for (int r = 0; r < KM_SORT_ROUNDS; ++r) {
-    const int i = base + r * 64 + lane;
-    k[r] = (i < N) ? keys[(size_t)p * N + i] : 0;
-    t[r] = (i < N && toks) ? toks[(size_t)p * N + i] : i;
-  }
+  for (int r = 0; r < KM_SORT_ROUNDS; ++r) k[r] = keys[(size_t)p * N + min(i0 + r * 64, N - 1)];
+  for (int b = lane; b < bins; b += 64) run[b] = 0;
+  int32_t first[KM_SORT_MAX_BINS / 256];
+#pragma unroll
+  for (int u = 0; u < KM_SORT_MAX_BINS / 256; ++u)
+    first[u] = chunk_hist[((size_t)p * bins + min((int)threadIdx.x + u * 256, bins - 1)) * nchunks + chunk];
   km_wave_lds_sync();
+#pragma unroll
+  for (int r = 0; r < KM_SORT_ROUNDS; ++r)
+    if (i0 + r * 64 < N) atomicAdd(&run[(k[r] >> shift) & (bins - 1)], 1);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < KM_SORT_MAX_BINS / 256; ++u) {
+    const int b = threadIdx.x + u * 256;
+    if (b < bins) {
+      int32_t at = first[u];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const int32_t n = sh[w][b];
+        sh[w][b] = at;
+        at += n;
+      }
+    }
+  }
+  __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
   for (int r = 0; r < KM_SORT_ROUNDS; ++r) {
-    const bool valid = base + r * 64 + lane < N;
+    const int i = i0 + r * 64;
+    const bool valid = i < N;
     const int bin = (k[r] >> shift) & (bins - 1);
-    uint64_t peers = __ballot(valid);  // lanes of this round with the same digit
-    for (int b = 0; b < bits; ++b) {
-      const bool bit = (bin >> b) & 1;
-      const uint64_t m = __ballot(valid && bit);
-      peers &= bit ? m : ~m;
+    uint64_t peers = __builtin_amdgcn_ballot_w64(valid);  // lanes of this round with the same digit
+    for (int b = 1; b < bins; b <<= 1) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(valid && (bin & b));
+      peers &= (bin & b) ? m : ~m;
     }
     const int start = run[bin];
     km_wave_lds_sync();  // every lane has read the running position before the leader advances it
     if (valid) {
-      const int pos = start + __popcll(peers & below);
       if (lane == 63 - __clzll((long long)peers)) run[bin] = start + __popcll(peers);
-      out_toks[(size_t)p * N + pos] = t[r];
-      if (out_keys) out_keys[(size_t)p * N + pos] = k[r];
+      out_toks[(size_t)p * N + start + __popcll(peers & below)] =
+          low < 0 ? i : (int32_t)((uint32_t)i << low | (uint32_t)(k[r] & ((1 << low) - 1)));
     }
     km_wave_lds_sync();
   }
@@ -328,14 +331,14 @@ __global__ __launch_bounds__(KM_SMALL_WAVES * 64) void km_sort_small_kernel(cons
   int32_t* run = sh[wave];
   for (int b = lane; b < bins; b += 64) run[b] = 0;
   km_wave_lds_sync();
-  int32_t k[KM_SORT_ROUNDS];
+  int32_t k[KM_SORT_CHUNK / 64];
 #pragma unroll
-  for (int r = 0; r < KM_SORT_ROUNDS; ++r) {
+  for (int r = 0; r < KM_SORT_CHUNK / 64; ++r) {
     const int i = base + r * 64 + lane;
     k[r] = (r < rounds && i < N) ? (keys[(size_t)p * N + i] & (bins - 1)) : -1;
   }
 #pragma unroll
-  for (int r = 0; r < KM_SORT_ROUNDS; ++r)
+  for (int r = 0; r < KM_SORT_CHUNK / 64; ++r)
     if (k[r] >= 0) atomicAdd(&run[k[r]], 1);
   __syncthreads();
   // exclusive scan in (digit, wave) order: thread t owns digit t / 2, waves 8 (t % 2) .. + 7
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(KM_SMALL_WAVES * 64) void km_sort_small_kernel(cons
   __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
-  for (int r = 0; r < KM_SORT_ROUNDS; ++r) {
+  for (int r = 0; r < KM_SORT_CHUNK / 64; ++r) {
     if (r < rounds) {   // uniform
       const bool valid = k[r] >= 0;
       const int bin = valid ? k[r] : 0;
@@ -398,28 +401,101 @@ __global__ __launch_bounds__(KM_SMALL_WAVES * 64) void km_sort_small_kernel(cons
   }
 }
 
-// CSR offsets from the sorted members: position i starts every cluster in (key[i-1], key[i]]
-__global__ __launch_bounds__(256) void km_bounds_kernel(const int32_t* __restrict__ assign,
-                                                        const int32_t* __restrict__ members,
-                                                        int32_t* __restrict__ offsets, int N, int nc) {
-  const int p = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= N) return;
-  const int32_t* as = assign + (size_t)p * N;
-  const int32_t* mem = members + (size_t)p * N;
-  int32_t* off = offsets + (size_t)p * (nc + 1);
-  const int c = min(max(as[mem[i]], 0), nc - 1);
-  const int cprev = (i > 0) ? min(max(as[mem[i - 1]], 0), nc - 1) : -1;
-  for (int k = cprev + 1; k <= c; ++k) off[k] = i;
-  if (i == N - 1)
-    for (int k = c + 1; k <= nc; ++k) off[k] = N;
-}
+// Second half of a two-digit sort: one workgroup per bucket of 2^bits consecutive clusters.  The bucket's tokens (as the
+// scatter left them: ascending) are counted per (cluster, wave), each wave over its own stretch of them, and placed in
+// (cluster, wave) order by the same ballot ranking; the counters' scan is the bucket's part of offsets and counts.
+// packed: the entries carry the cluster's low bits; where token and bits do not fit one word, the assignment is read again.
+#define KM_BUCKET_WAVES 8
+#define KM_BUCKET_HELD 4   // rounds of 64 tokens per wave kept in registers between the two walks
 
-__global__ __launch_bounds__(256) void km_counts_kernel(const int32_t* __restrict__ offsets,
-                                                        int32_t* __restrict__ counts, int nc) {
-  const int p = blockIdx.y;
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c < nc) counts[(size_t)p * nc + c] = offsets[(size_t)p * (nc + 1) + c + 1] - offsets[(size_t)p * (nc + 1) + c];
+__global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
+    const int32_t* __restrict__ assign, const int32_t* __restrict__ toks, const int32_t* __restrict__ chunk_hist,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int nchunks,
+    int bits, int buckets, int bins, bool packed) {
+  constexpr int NW = KM_BUCKET_WAVES, HELD = KM_BUCKET_HELD;
+  __shared__ int32_t sh_run[KM_SORT_MAX_BINS][NW];
+  __shared__ int32_t sh_w[NW];
+  const int p = blockIdx.y, bucket = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int C = 1 << bits, c0 = bucket << bits;
+  const int32_t* first = chunk_hist + (size_t)p * bins * nchunks;
+  const int start = first[(size_t)bucket * nchunks];
+  const int end = bucket + 1 < buckets ? first[(size_t)(bucket + 1) * nchunks] : N;
+  const int rounds = (end - start + NW * 64 - 1) / (NW * 64);   // of 64 tokens per wave
+  const int32_t* as = assign + (size_t)p * N;
+  const int32_t* tk = toks + (size_t)p * N;
+  const int i0 = start + wave * rounds * 64 + lane;
+  for (int k = tid; k < C * NW; k += NW * 64) (&sh_run[0][0])[k] = 0;
+  int32_t t[HELD], c[HELD];
+  const auto fetch = [&](int r0) {   // four rounds' tokens and clusters; -1: none
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) t[u] = tk[min(i0 + (r0 + u) * 64, N - 1)];
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) {
+      c[u] = (packed ? t[u] : as[t[u]]) & (C - 1);
+      if (packed) t[u] = (int32_t)((uint32_t)t[u] >> bits);
+    }
+#pragma unroll
+    for (int u = 0; u < HELD; ++u)
+      if (r0 + u >= rounds || i0 + (r0 + u) * 64 >= end) c[u] = -1;
+  };
+  __syncthreads();
+  for (int r0 = 0; r0 < rounds; r0 += HELD) {
+    fetch(r0);
+#pragma unroll
+    for (int u = 0; u < HELD; ++u)
+      if (c[u] >= 0) atomicAdd(&sh_run[c[u]][wave], 1);
+  }
+  __syncthreads();
+  int carry = start;
+  for (int k0 = 0; k0 < C * NW; k0 += NW * 64) {   // exclusive scan in (cluster, wave) order
+    const int k = k0 + tid;
+    const int v = k < C * NW ? (&sh_run[0][0])[k] : 0;
+    const int inc = (int)ri_wave_incl_scan((uint32_t)v);
+    if (lane == 63) sh_w[wave] = inc;
+    __syncthreads();
+    int ex = carry + inc - v;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      if (w < wave) ex += sh_w[w];
+      carry += sh_w[w];
+    }
+    const int cl = c0 + k / NW;
+    // a cluster's count: from its first wave's position to its last wave's end, eight lanes on
+    const int past = __shfl_down(ex + v, NW - 1);
+    if (k < C * NW) {
+      (&sh_run[0][0])[k] = ex;
+      if (k % NW == 0 && cl < nc) {
+        offsets[(size_t)p * (nc + 1) + cl] = ex;
+        counts[(size_t)p * nc + cl] = past - ex;
+      }
+    }
+    __syncthreads();
+  }
+  if (bucket == buckets - 1 && tid == 0) offsets[(size_t)p * (nc + 1) + nc] = N;
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int r0 = 0; r0 < rounds; r0 += HELD) {
+    if (rounds > HELD) fetch(r0);
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) {
+      if (r0 + u < rounds) {
+        const bool ok = c[u] >= 0;
+        const int cl = ok ? c[u] : 0;
+        uint64_t peers = __builtin_amdgcn_ballot_w64(ok);   // lanes of this round with the same cluster
+        for (int b = 1; b < C; b <<= 1) {
+          const uint64_t m = __builtin_amdgcn_ballot_w64(ok && (cl & b));
+          peers &= (cl & b) ? m : ~m;
+        }
+        const int at = sh_run[cl][wave];
+        km_wave_lds_sync();   // every lane has read the running position before the leader advances it
+        if (ok) {
+          members[(size_t)p * N + at + __popcll(peers & below)] = t[u];
+          if (lane == 63 - __clzll((long long)peers)) sh_run[cl][wave] = at + __popcll(peers);
+        }
+        km_wave_lds_sync();
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------
@@ -440,38 +516,55 @@ __global__ __launch_bounds__(256) void km_counts_kernel(const int32_t* __restric
 // ------------------------------------------------------------------------------------
 #define KM_BLK 256
 
-// Rows k0 .. k1-1 of a list added in list order, U per round: the lanes fetch the round's
-// member ids with one load, the ids are broadcast from the lanes, and the row loads (in eights; a short last eight
-// repeats its last row) are all in flight before the first add; a missing row adds +0, which changes no sum.  (Two
-// dependent round trips per U rows instead of two per row for a list's tail.)
+// Rows k0 .. k1-1 of a list added in list order, U per round: the lanes fetch the round's member ids with one load and
+// make row addresses of them, which are broadcast from the lanes as scalar bases; the row loads (in eights; a short last
+// eight repeats its last row, and adds +0 for it, which changes no sum) are all in flight before the first add.  The
+// wave's instructions bound this as much as the bytes: three fetch a row (address arithmetic per row took seven, and a
+// select per row is left to the last eight: 8 x 131072 tokens, 8192 clusters 71.3 -> 57.0 us, with 64 rows in flight 67.4;
+// half the tokens in seven clusters of 4 x 20000 tokens 27.7 -> 19.7).
 // pitch: words between rows.  With wp the rows are also copied: row k of the list to wp + k * 64.
-template <bool HALF, int U, bool COPY = false, typename Id>
-__device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const Id* mem, int k0, int k1, float& s0,
+template <bool HALF, int U, bool COPY = false>
+__device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const int32_t* mem, int k0, int k1, float& s0,
                                             float& s1, size_t pitch = RI_DIM / 2, uint32_t* __restrict__ wp = nullptr) {
   static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
+  const auto add = [&](uint32_t w) {
+    float x0, x1;
+    ri_unpack2<HALF>(w, x0, x1);
+    s0 += x0;
+    s1 += x1;
+  };
   for (int k = k0; k < k1; k += U) {
     const int n = min(U, k1 - k);
-    const int id = (int)mem[k + min(lane, n - 1)];
+    const uint64_t at = (uint64_t)(rp + (size_t)mem[k + min(lane, n - 1)] * pitch);
+    const uint32_t lo = (uint32_t)at, hi = (uint32_t)(at >> 32);
     uint32_t v[U];
 #pragma unroll
     for (int e = 0; e < U; e += 8)
       if (e < n) {
 #pragma unroll
-        for (int j = e; j < e + 8; ++j) v[j] = rp[(size_t)__builtin_amdgcn_readlane(id, j) * pitch];
+        for (int j = e; j < e + 8; ++j) {
+          const uint64_t row = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32 |
+                               (uint32_t)__builtin_amdgcn_readlane(lo, j);
+          v[j] = reinterpret_cast<const uint32_t*>(row)[(uint32_t)lane];
+        }
       }
 #pragma unroll
-    for (int e = 0; e < U; e += 8)
-      if (e < n) {
+    for (int e = 0; e < U; e += 8) {
+      if (e + 8 <= n) {
 #pragma unroll
         for (int j = e; j < e + 8; ++j) {
-          float x0, x1;
-          ri_unpack2<HALF>(j < n ? v[j] : 0u, x0, x1);   // the word 0 is (+0, +0) in either type
-          s0 += x0;
-          s1 += x1;
+          add(v[j]);
+          if (COPY) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
+        }
+      } else if (e < n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) {
+          add(j < n ? v[j] : 0u);   // the word 0 is (+0, +0) in either type
           if (COPY && j < n) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
         }
       }
+    }
   }
 }
 
@@ -540,7 +633,7 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
   const int32_t* off = offsets + (size_t)p * (nc + 1);
   // (head_stride and pitch in words: the rows of a head need not be contiguous)
   const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows) + (size_t)(p / seg) * head_stride +
-                       (size_t)(p % seg) * N * pitch + lane;
+                       (size_t)(p % seg) * N * pitch;
   uint32_t* wp = COPY ? reinterpret_cast<uint32_t*>(copy) + (size_t)p * copy_stride * (RI_DIM / 2) + lane : nullptr;
   if ((int)blockIdx.x < item_wgs) {
     const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -843,11 +936,19 @@ static int km_check(int P, int N, int nc) {
 
 static int km_sort_chunks(int N) { return (N + KM_SORT_CHUNK - 1) / KM_SORT_CHUNK; }
 
-// digit widths of the list sort: one pass when the cluster ids fit 9 bits, else two of about half each
-static void km_sort_bits(int nc, int& lo_bits, int& hi_bits) {
+// Digits of the list sort: one when the cluster ids fit 9 bits, else an upper one, whose buckets are sorted by a workgroup
+// each, and a lower one of 5 bits, or more where the upper one would have more than 9 or its table more than one round of
+// the scan.  (131072 tokens, 8192 clusters: 128 buckets of 64 clusters.)
+static void km_sort_bits(int N, int nc, int& lo_bits, int& hi_bits) {
   int total_bits = 1;
   while ((1 << total_bits) < nc) ++total_bits;
-  lo_bits = total_bits <= 9 ? total_bits : (total_bits + 1) / 2;
+  lo_bits = 0;
+  hi_bits = total_bits;
+  if (total_bits <= 9) return;
+  lo_bits = 5;
+  while (total_bits - lo_bits > 9 ||
+         (lo_bits < 7 && ((long long)km_sort_chunks(N) << (total_bits - lo_bits)) > 16 * 1024))
+    ++lo_bits;
   hi_bits = total_bits - lo_bits;
 }
 
@@ -901,48 +1002,38 @@ extern "C" int ri_kmeans_assign_f16(const void* data, const void* centroids, int
 
 extern "C" size_t ri_kmeans_workspace_bytes(int P, int N, int nc) {
   if (P <= 0 || N <= 0 || nc <= 0) return 0;
-  // digit table [P, 512, chunks] + one (key, token) staging pair [P, N] for the two-pass case
-  return ((size_t)P * KM_SORT_MAX_BINS * km_sort_chunks(N) + 2 * (size_t)P * N) * sizeof(int32_t);
+  // digit table [P, 512, chunks] + the tokens by bucket [P, N] for ids of two digits
+  return ((size_t)P * KM_SORT_MAX_BINS * km_sort_chunks(N) + (size_t)P * N) * sizeof(int32_t);
 }
 
 static int km_build_lists(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P, int N,
                           int nc, void* workspace, hipStream_t s) {
   const int nchunks = km_sort_chunks(N);
   int32_t* chunk_hist = (int32_t*)workspace;
-  int32_t* tmp_key = chunk_hist + (size_t)P * KM_SORT_MAX_BINS * nchunks;
-  int32_t* tmp_tok = tmp_key + (size_t)P * N;
+  int32_t* toks = chunk_hist + (size_t)P * KM_SORT_MAX_BINS * nchunks;
   int lo_bits, hi_bits;
-  km_sort_bits(nc, lo_bits, hi_bits);
-  if (hi_bits == 0 && N <= KM_SMALL_MAX) {
-    km_sort_small_kernel<<<P, KM_SMALL_WAVES * 64, 0, s>>>(assign, offsets, counts, members, N, nc, lo_bits);
+  km_sort_bits(N, nc, lo_bits, hi_bits);
+  if (lo_bits == 0 && N <= KM_SMALL_MAX) {
+    km_sort_small_kernel<<<P, KM_SMALL_WAVES * 64, 0, s>>>(assign, offsets, counts, members, N, nc, hi_bits);
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }
-  const dim3 cgrid((nchunks + 3) / 4, P);
-  // pass over the low digit (the only one when the ids fit 9 bits)
-  km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, N, nchunks, 0, lo_bits);
+  const dim3 cgrid(nchunks, P);
+  km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, N, nchunks, lo_bits, hi_bits);
   RI_HIP_CHECK_LAUNCH();
-  // one pass and no cluster id beyond nc: the scan itself yields offsets and counts
-  const bool direct = hi_bits == 0;
-  km_sort_scan_kernel<<<P, 1024, 0, s>>>(chunk_hist, (1 << lo_bits) * nchunks, direct ? offsets : nullptr,
-                                         direct ? counts : nullptr, nchunks, nc, N);
+  // (a single digit: the scan itself yields offsets and counts)
+  const bool single = lo_bits == 0;
+  km_sort_scan_kernel<<<P, 1024, 0, s>>>(chunk_hist, nchunks << hi_bits, single ? offsets : nullptr,
+                                         single ? counts : nullptr, nchunks, nc, N);
   RI_HIP_CHECK_LAUNCH();
-  km_sort_scatter_kernel<<<cgrid, 256, 0, s>>>(assign, nullptr, chunk_hist, hi_bits ? tmp_key : nullptr,
-                                               hi_bits ? tmp_tok : members, N, nchunks, 0, lo_bits);
+  const bool packed = (uint64_t)N << lo_bits <= 1ull << 32;
+  km_sort_scatter_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, single ? members : toks, N, nchunks, lo_bits, hi_bits,
+                                               single || !packed ? -1 : lo_bits);
   RI_HIP_CHECK_LAUNCH();
-  if (hi_bits) {
-    km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(tmp_key, chunk_hist, N, nchunks, lo_bits, hi_bits);
-    RI_HIP_CHECK_LAUNCH();
-    km_sort_scan_kernel<<<P, 1024, 0, s>>>(chunk_hist, (1 << hi_bits) * nchunks, nullptr, nullptr, nchunks, nc, N);
-    RI_HIP_CHECK_LAUNCH();
-    km_sort_scatter_kernel<<<cgrid, 256, 0, s>>>(tmp_key, tmp_tok, chunk_hist, nullptr, members, N, nchunks,
-                                                 lo_bits, hi_bits);
-    RI_HIP_CHECK_LAUNCH();
-  }
-  if (!direct) {
-    km_bounds_kernel<<<dim3((N + 255) / 256, P), 256, 0, s>>>(assign, members, offsets, N, nc);
-    RI_HIP_CHECK_LAUNCH();
-    km_counts_kernel<<<dim3((nc + 255) / 256, P), 256, 0, s>>>(offsets, counts, nc);
+  if (!single) {
+    const int buckets = ((nc - 1) >> lo_bits) + 1;
+    km_bucket_kernel<<<dim3(buckets, P), KM_BUCKET_WAVES * 64, 0, s>>>(assign, toks, chunk_hist, counts, offsets, members, N,
+                                                                       nc, nchunks, lo_bits, buckets, 1 << hi_bits, packed);
     RI_HIP_CHECK_LAUNCH();
   }
   return RI_OK;

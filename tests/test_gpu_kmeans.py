@@ -220,6 +220,23 @@ def test_build_lists_is_a_stable_sort(dev, P, N, nc, seed):
         assert np.array_equal(offsets[p].cpu().numpy(), np.concatenate([[0], np.cumsum(cnt)]))
 
 
+@pytest.mark.parametrize("P,N,nc", [(3, 1000, 544), (2, 40001, 1056), (1, 300000, 8192), (2, 70000, 40000), (1, 3000, 262144)])
+def test_build_lists_by_buckets(dev, P, N, nc):
+    """Ids of two digits: the least and the most clusters, a scan of several rounds, buckets whose counters need several,
+    one bucket with most of the tokens and buckets without any."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(N)
+    assign = torch.randint(0, max(nc - 700, 1), (P, N), generator=g, dtype=torch.int32)
+    assign[0, N // 3:] = nc - 1
+    counts, offsets, members = (torch.full(s, -1, dtype=torch.int32, device=dev) for s in ((P, nc), (P, nc + 1), (P, N)))
+    kernels.kmeans_build_lists(assign.to(dev), counts, offsets, members, P, N, nc)
+    for p in range(P):
+        cnt = torch.bincount(assign[p], minlength=nc)
+        assert torch.equal(members[p].cpu().long(), torch.argsort(assign[p], stable=True))
+        assert torch.equal(counts[p].cpu().long(), cnt)
+        assert torch.equal(offsets[p].cpu().long(), torch.cat((torch.zeros(1, dtype=torch.int64), torch.cumsum(cnt, 0))))
+
+
 @pytest.mark.parametrize("G,N,nc,S,seed", [(2, 4096, 256, 4, 0), (1, 8192, 512, 1, 1), (2, 3001, 192, 3, 2)])
 def test_segment_k_means_teacher_forced(dev, G, N, nc, S, seed, dt=torch.bfloat16):
     """Whole driver against the oracle, iteration by iteration: every step is checked on the
