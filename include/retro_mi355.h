@@ -504,6 +504,34 @@ int ri_lru_access_update(const int32_t* ret_ids, const int32_t* sizes, const int
                          int BG, int np, int ncl, int buffer_size, int capacity, int block,
                          ri_stream_t stream);
 
+/* ri_lru_access_update in two launches, with its arguments in one struct (host memory, read during the call) that a
+ * caller fills once per layer: ri_lru_access writes the hit and miss lists, the row table and meta, which is all that
+ * staging and attention wait for; ri_lru_stage_update evicts and admits, and copies the missed rows from the host store
+ * [BG, host_stride, 128] to the staging rows of [BG, cache_stride, 128] in the same launch.  Both have to run, in this
+ * order, before the next call on the same state; the row table is required. */
+typedef struct ri_lru_t {
+  const int32_t *ret_ids, *sizes, *starts, *blk_off;
+  int32_t *stamp, *order, *blk_ids, *free_list, *free_count, *epoch;
+  int32_t *hit_ids, *hit_sizes, *hit_cumsum, *hit_num;
+  int32_t *miss_ids, *miss_sizes, *miss_cumsum, *miss_num;
+  int32_t *upd_buf, *upd_sizes, *upd_cache, *upd_num;
+  int32_t *row_src, *meta;
+  const void *host_k, *host_v;
+  void *cache_k, *cache_v;
+  int64_t host_stride, cache_stride;
+  int row_src_stride, stage_row0, np, ncl, meta_stride, blk_off_stride, stamp_stride, blk_ids_stride, buffer_size,
+      capacity, block, BG;
+} ri_lru_t;
+int ri_lru_access(const ri_lru_t* lru, ri_stream_t stream);
+int ri_lru_stage_update(const ri_lru_t* lru, ri_stream_t stream);
+
+/* The decode step of one layer over a host-resident store with the device-side block cache (compute(),
+ * cache_hub/retroinfer_cache.py:549-697): ri_score_select, ri_lru_access, ri_lru_stage_update, ri_wave_attention over the
+ * row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`, store_k / store_v are the cache tensors of
+ * `lru` and ret_tok_off, ret_start, cluster_start are not used. */
+int ri_host_step(const ri_decode_step_t* step, const ri_lru_t* lru, const void* q, int static_len, void* out,
+                 ri_stream_t stream);
+
 /* Device-side replacement of WaveBufferCPU::organize_kv (wave_buffer_cpu.cpp:545-567):
  * out[p, i, :] = in[p, members[p, i], :] — K/V rows permuted into cluster-contiguous order. */
 int ri_permute_rows(const void* in, const int32_t* members, void* out, int P, int N,

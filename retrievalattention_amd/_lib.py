@@ -21,6 +21,17 @@ class DecodeStep(C.Structure):
         (n, I) for n in ("BG", "gs", "nc", "np", "es", "page", "max_pages", "half")] + [("scale", F)]
 
 
+class Lru(C.Structure):
+    """ri_lru_t"""
+    _fields_ = [(n, P) for n in (
+        "ret_ids", "sizes", "starts", "blk_off", "stamp", "order", "blk_ids", "free_list", "free_count", "epoch", "hit_ids",
+        "hit_sizes", "hit_cumsum", "hit_num", "miss_ids", "miss_sizes", "miss_cumsum", "miss_num", "upd_buf", "upd_sizes",
+        "upd_cache", "upd_num", "row_src", "meta", "host_k", "host_v", "cache_k", "cache_v")] + [
+        ("host_stride", I64), ("cache_stride", I64)] + [(n, I) for n in (
+            "row_src_stride", "stage_row0", "np", "ncl", "meta_stride", "blk_off_stride", "stamp_stride", "blk_ids_stride",
+            "buffer_size", "capacity", "block", "BG")]
+
+
 # name -> (restype, argtypes); mirrors include/retro_mi355.h
 SIGNATURES = {
     "ri_status_string": (C.c_char_p, [I]),
@@ -51,6 +62,9 @@ SIGNATURES = {
     "ri_buffer_attention_f16": (I, [P, P, P, I64, P, I, P, P, P, P, P, I, I, I, I, F, P, SZ, P]),
     "ri_decode_step": (I, [P, P, I, P, P]),
     "ri_append_kv": (I, [P, P, P, P, I64, I64, P, I, P]),
+    "ri_lru_access": (I, [P, P]),
+    "ri_lru_stage_update": (I, [P, P]),
+    "ri_host_step": (I, [P, P, P, I, P, P]),
     "ri_lru_access_update": (I, [P, P, P, I, P, I, P, P, I, P, I, P, P, P] + [P] * 12 + [P, I, I, P] + [I] * 6 + [P]),
     "ri_gather_copy_vectors": (I, [P, P, P, P, P, P, P, I, I, I, I, I, I, P]),
     "ri_gather_copy_and_concat": (I, [P] * 17 + [I] * 7 + [P]),

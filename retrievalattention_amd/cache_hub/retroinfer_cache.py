@@ -629,6 +629,27 @@ class retroinfer_cache(KV_Cache):
                 self.RSQRT_DIM)
         return plan
 
+    def _host_plan(self, layer, buf):
+        """_plan for a host-resident store with the device-side block cache."""
+        lru = self.device_lru[layer]
+        _, _, row_src, meta = self.layouts[buf if self.use_cluster_estimation else 0]
+        t = (self.centroids[layer], self.centroids_mask[layer], self.logits, self.ret_ids[buf], self.est_ids[buf], meta,
+             self.steady_zone_keys[layer], self.steady_zone_values[layer], self.cache_keys[layer],
+             self.cache_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
+        other = (self.cluster_size_i32[layer], self.cluster_start[layer], row_src, self.list_keys[layer],
+                 self.list_values[layer])
+        key = [x.data_ptr() for x in t] + [x.data_ptr() for x in other]
+        key += (lru, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size)
+        plan = self._plans.get((layer, buf))
+        if plan is None or not plan.valid(key):
+            names = ("centroids", "mask", "logits", "ret_ids", "est_ids", "meta", "steady_k", "steady_v", "store_k",
+                     "store_v", "value_sum", "cluster_size", "valid_lengths")
+            plan = self._plans[(layer, buf)] = kernels.HostStepPlan(
+                key, self.dtype, dict(zip(names, t)), self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
+                self.RSQRT_DIM, lru, other[0], other[1], self._lists(layer), row_src, other[3], other[4],
+                self.cache_size * self.page_size)
+        return plan
+
     def block_cache_stats(self, layer_idx):
         """(hit blocks, miss blocks) of the layer's last look-up, summed over the groups (host residency)."""
         miss = int(self.miss_num_units[layer_idx].sum())
@@ -664,6 +685,12 @@ class retroinfer_cache(KV_Cache):
                                search_next):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
         es = self.es_cluster_num
+        if search_here and not search_next and not self.overlap_miss_staging and not kernels.PROFILER_RANGES and \
+                queries.is_cuda and queries.dtype == self.dtype and queries.is_contiguous() and \
+                queries.numel() == BG * gs * D:
+            out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
+            self._host_plan(layer_idx, buf).run(queries, static_len, out)
+            return out
         q = queries.view(BG, gs, D)
         rows = self.cache_blocks * self.page_size
         stage0 = self.cache_size * self.page_size

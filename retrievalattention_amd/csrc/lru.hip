@@ -1,6 +1,6 @@
 // Device-side block cache manager for a host-resident cluster store (gfx950).
 //
-// Does on the GPU, in one launch and without a host round trip, what the reference does on CPU
+// Does on the GPU, without a host round trip, what the reference does on CPU
 // worker threads between the top-k search and the gather:
 //   BufferManager::batch_access  (library/retroinfer/retroinfer_kernels/src/wave_buffer_cpu.cpp:190-257)
 //     walk the retrieved clusters in rank order, stop when their blocks no longer fit the
@@ -18,35 +18,23 @@
 // first.  Eviction takes whole clusters from the least recent end until the request is covered, hits of the
 // current step included (:140-142; their blocks have been listed for this step's attention, which runs
 // before the admission copy overwrites them).  The victims are found without sorting: a radix selection over
-// the step ages (four 8-bit digits) gives the boundary step, and inside that step the clusters are ranked by
+// the step ages (8-bit digits) gives the boundary step, and inside that step the clusters are ranked by
 // their order through an LDS table indexed by it.
+//
+// A group's workgroup is one serial chain of scans and dependent loads.  Everything the attention waits for (hits,
+// misses, row table) is its first half; the second (eviction, admission) only has to be done before the admission copy.
+// So the two are also launched apart, the second beside the copy of the missed rows from the host, which is bound by the
+// link and leaves the compute units idle (32 groups, 3840 clusters, 10 MB of misses: access and update in one launch in
+// front of the copy 27.8 + 200 us, access alone 7 and both others together 187).
 #include "ri_common.h"
 
 #define LRU_THREADS 1024
 #define LRU_WAVES (LRU_THREADS / 64)
 #define LRU_DIGIT 256
+#define LRU_COPIES 8        // of the age histogram: a step's clusters share their age
+#define LRU_HELD 4          // clusters per thread whose stamps and blocks stay in registers
 
-struct LruParams {
-  const int32_t* ret_ids;   // [BG, np] cluster ids in rank order
-  const int32_t* sizes;     // [BG, meta_stride] tokens per cluster
-  const int32_t* starts;    // [BG, meta_stride] first row of the cluster in the host store
-  const int32_t* blk_off;   // [BG, blk_off_stride] exclusive prefix of ceil(size / block)
-  int32_t* stamp;           // [BG, stamp_stride] 0 = not resident, else last step that touched it
-  int32_t* order;           // [BG, stamp_stride] order inside that step (larger = more recent)
-  int32_t* blk_ids;         // [BG, blk_ids_stride] cache block ids of resident clusters, at blk_off
-  int32_t* free_list;       // [BG, capacity] free block ids, the first free_count are valid
-  int32_t* free_count;      // [BG]
-  int32_t* epoch;           // [BG] step counter
-  int32_t *hit_ids, *hit_sizes, *hit_cumsum, *hit_num;
-  int32_t *miss_ids, *miss_sizes, *miss_cumsum, *miss_num;
-  int32_t *upd_buf, *upd_sizes, *upd_cache, *upd_num;
-  // optional row table for attention in place: row of every retrieved token in a tensor that holds the
-  // cache blocks first and the staging area of the misses behind them; then no hit list is emitted
-  int32_t* row_src;  // [BG, row_src_stride] or null
-  int32_t* meta;     // [BG, 4]: {clusters kept, tokens, blocks, 0} or null
-  int row_src_stride, stage_row0;
-  int np, ncl, meta_stride, blk_off_stride, stamp_stride, blk_ids_stride, buffer_size, capacity, block;
-};
+enum { LRU_BOTH, LRU_ACCESS, LRU_UPDATE };
 
 // exclusive prefix sums of N values over the 1024 threads; totals in tot.  Wave scans on DPP, the sixteen
 // wave totals scanned by the lanes of every wave (one LDS read, one DPP scan, two lane reads).
@@ -73,18 +61,19 @@ __device__ __forceinline__ void lru_scan(const int (&v)[N], int (&pre)[N], int (
 }
 
 // R: ranks of the probe list a thread owns (thread t: ranks [t*R, t*R + R)); 1 up to 1023 probes, 4 up to 4096.
-template <int R>
-__global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
+// LRU_UPDATE sees the state that LRU_ACCESS left: the hits carry this step's stamp, so every rank finds itself as before.
+template <int R, int PHASE>
+__device__ __forceinline__ void lru_group(const ri_lru_t& P, int g) {
   constexpr int NPMAX = LRU_THREADS * R;
+  constexpr bool ACCESS = PHASE != LRU_UPDATE, UPDATE = PHASE != LRU_ACCESS;
   __shared__ int sh_scan[7 * LRU_WAVES];
-  __shared__ int sh_hist[LRU_DIGIT];
+  __shared__ __attribute__((aligned(16))) int sh_hist[UPDATE ? LRU_DIGIT * LRU_COPIES : 4];
   __shared__ int sh_cut[2];  // selected digit, blocks freed by clusters with a larger one
   // token offsets and sources of the ranks for the row table; later the blocks of the boundary step's
   // clusters by their order inside the step (2 * NPMAX entries: hits below, admitted misses above)
   __shared__ int sh_tab[2 * NPMAX];
   int* const sh_off = sh_tab;
   int* const sh_src = sh_tab + NPMAX;
-  const int g = blockIdx.x;
   const int tid = threadIdx.x;
   const int block = P.block;
   const int32_t* sizes = P.sizes + (size_t)g * P.meta_stride;
@@ -98,6 +87,30 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
   const int E = P.epoch[g] + 1;
   const int F0 = P.free_count[g];
   const int rb = tid * R;
+  if (PHASE == LRU_UPDATE && P.miss_num[g] == 0) {   // (uniform) nothing to admit
+    if (tid == 0) {
+      P.upd_num[g] = 0;
+      P.epoch[g] = E;
+    }
+    return;
+  }
+  // thread t owns the ids [t*K, t*K + K) for the eviction; up to LRU_HELD of them stay in registers
+  const int K = (P.ncl + LRU_THREADS - 1) / LRU_THREADS;
+  const bool held = K <= LRU_HELD;   // uniform
+  const int c0 = tid * K, c1 = min(P.ncl, c0 + K);
+  int h_stamp[LRU_HELD], h_nb[LRU_HELD];
+  auto hold = [&]() {
+#pragma unroll
+    for (int i = 0; i < LRU_HELD; ++i) {
+      const int cc = min(c0 + i, P.ncl - 1);
+      h_stamp[i] = stamp[cc];
+      h_nb[i] = boff[cc + 1] - boff[cc];
+    }
+#pragma unroll
+    for (int i = 0; i < LRU_HELD; ++i)
+      if (c0 + i >= c1) h_stamp[i] = 0;
+  };
+  if (PHASE == LRU_UPDATE && held) hold();   // (in flight under the ranks' own loads)
 
   // ---- access: every rank looks at its cluster ----
   // (everything the rank needs to know about its cluster is requested in one go: loads issued after a
@@ -178,7 +191,7 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
   int hit_tok[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) hit_tok[i] = 0;
-  if (!P.row_src) {
+  if (ACCESS && !P.row_src) {
     int vh[1] = {0}, ph[1], th[1];
 #pragma unroll
     for (int i = 0; i < R; ++i) vh[0] += hit[i] ? sz[i] : 0;
@@ -210,90 +223,110 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
     for (int i = 0; i < R; ++i) { adm_pre[i] = a; a += adm[i] ? nb[i] : 0; }
   }
 
-  const bool rows = P.row_src != nullptr;
-  if (rows) {
-    // row table: every thread takes tokens t, t + 1024, ... and finds the rank that owns them by
-    // bisection over the token offsets of the ranks (clusters that were dropped have no tokens)
+  if (ACCESS) {
+    const bool rows = P.row_src != nullptr;
+    if (rows) {
+      // row table: every thread takes tokens t, t + 1024, ... and finds the rank that owns them by
+      // bisection over the token offsets of the ranks (clusters that were dropped have no tokens)
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        sh_off[rb + i] = tok_pre[i];
+        sh_src[rb + i] = hit[i] ? -(boff_c[i] + 1) : P.stage_row0 + mt_pre[i];  // hits: where their block ids are
+      }
+      __syncthreads();
+      int32_t* table = P.row_src + (size_t)g * P.row_src_stride;
+      for (int t = tid; t < t5[1]; t += LRU_THREADS) {
+        int lo_r = 0, hi_r = min(NPMAX, P.np);  // first rank whose offset exceeds t (ranks past the list hold the total)
+        while (lo_r < hi_r) {
+          const int mid = (lo_r + hi_r) >> 1;
+          if (sh_off[mid] > t) hi_r = mid; else lo_r = mid + 1;
+        }
+        const int r = lo_r - 1, i = t - sh_off[r], src = sh_src[r];
+        table[t] = src < 0 ? bids[-src - 1 + i / block] * block + i % block : src + i;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      sh_off[rb + i] = tok_pre[i];
-      sh_src[rb + i] = hit[i] ? -(boff_c[i] + 1) : P.stage_row0 + mt_pre[i];  // hits: where their block ids are
-    }
-    __syncthreads();
-    int32_t* table = P.row_src + (size_t)g * P.row_src_stride;
-    for (int t = tid; t < t5[1]; t += LRU_THREADS) {
-      int lo_r = 0, hi_r = min(NPMAX, P.np);  // first rank whose offset exceeds t (ranks past the list hold the total)
-      while (lo_r < hi_r) {
-        const int mid = (lo_r + hi_r) >> 1;
-        if (sh_off[mid] > t) hi_r = mid; else lo_r = mid + 1;
+      if (hit[i]) {
+        const int32_t* ids = bids + boff_c[i];
+        if (!rows) {
+          for (int j = 0; j < nb[i]; ++j) {
+            P.hit_ids[lo + hb_pre[i] + j] = ids[j];
+            P.hit_sizes[lo + hb_pre[i] + j] = (j == nb[i] - 1) ? sz[i] - (nb[i] - 1) * block : block;
+            P.hit_cumsum[lo + hb_pre[i] + j] = hit_tok[i] + j * block;
+          }
+        }
+        stamp[c[i]] = E;
+        order[c[i]] = nhits - 1 - hit_idx[i];   // hits are moved to the front in reverse rank order
       }
-      const int r = lo_r - 1, i = t - sh_off[r], src = sh_src[r];
-      table[t] = src < 0 ? bids[-src - 1 + i / block] * block + i % block : src + i;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    if (hit[i]) {
-      const int32_t* ids = bids + boff_c[i];
-      if (!rows) {
+      if (miss[i]) {
+        const int row = start_c[i];
         for (int j = 0; j < nb[i]; ++j) {
-          P.hit_ids[lo + hb_pre[i] + j] = ids[j];
-          P.hit_sizes[lo + hb_pre[i] + j] = (j == nb[i] - 1) ? sz[i] - (nb[i] - 1) * block : block;
-          P.hit_cumsum[lo + hb_pre[i] + j] = hit_tok[i] + j * block;
+          P.miss_ids[lo + mb_pre[i] + j] = row + j * block;
+          P.miss_sizes[lo + mb_pre[i] + j] = (j == nb[i] - 1) ? sz[i] - (nb[i] - 1) * block : block;
+          P.miss_cumsum[lo + mb_pre[i] + j] = mt_pre[i] + j * block;
         }
       }
-      stamp[c[i]] = E;
-      order[c[i]] = nhits - 1 - hit_idx[i];   // hits are moved to the front in reverse rank order
     }
-    if (miss[i]) {
-      const int row = start_c[i];
-      for (int j = 0; j < nb[i]; ++j) {
-        P.miss_ids[lo + mb_pre[i] + j] = row + j * block;
-        P.miss_sizes[lo + mb_pre[i] + j] = (j == nb[i] - 1) ? sz[i] - (nb[i] - 1) * block : block;
-        P.miss_cumsum[lo + mb_pre[i] + j] = mt_pre[i] + j * block;
+    if (tid == 0) {
+      P.hit_num[g] = rows ? 0 : t5[0];
+      P.miss_num[g] = t5[2];
+      if (P.meta) {
+        P.meta[g * 4 + 0] = t5[4];
+        P.meta[g * 4 + 1] = t5[1];
+        P.meta[g * 4 + 2] = t5[0] + t5[2];
+        P.meta[g * 4 + 3] = 0;
       }
     }
   }
-  if (tid == 0) {
-    P.hit_num[g] = rows ? 0 : t5[0];
-    P.miss_num[g] = t5[2];
-    if (P.meta) {
-      P.meta[g * 4 + 0] = t5[4];
-      P.meta[g * 4 + 1] = t5[1];
-      P.meta[g * 4 + 2] = t5[0] + t5[2];
-      P.meta[g * 4 + 3] = 0;
-    }
-  }
-  __syncthreads();  // the hits carry this step's stamp and order before anybody looks for victims
+  if (!UPDATE) return;
+  if (PHASE == LRU_BOTH) __syncthreads();  // the hits carry this step's stamp and order before anybody looks for victims
 
   // ---- eviction: free (need - F0) blocks from the least recently used clusters ----
   const int to_free = need - F0;  // uniform
   int F = F0;
   if (to_free > 0) {
-    // thread t owns the ids [t*K, t*K + K)
-    const int K = (P.ncl + LRU_THREADS - 1) / LRU_THREADS;
-    const int c0 = tid * K, c1 = min(P.ncl, c0 + K);
+    if (PHASE == LRU_BOTH && held) hold();
+    // fn(cluster, stamp, blocks) for every resident cluster of this thread, in id order
+    auto resident = [&](auto&& fn) {
+      if (held) {
+#pragma unroll
+        for (int i = 0; i < LRU_HELD; ++i)
+          if (h_stamp[i] != 0) fn(c0 + i, h_stamp[i], h_nb[i]);
+      } else {
+        for (int cc = c0; cc < c1; ++cc) {
+          const int st = stamp[cc];
+          if (st != 0) fn(cc, st, boff[cc + 1] - boff[cc]);
+        }
+      }
+    };
     // boundary step: the age A such that every resident cluster older than A goes and the clusters of age A
-    // cover the remaining `rem` blocks; radix selection over the four bytes of the age, oldest first
+    // cover the remaining `rem` blocks; radix selection over the bytes of the age, oldest first.  No age has a byte
+    // above the step number's: the first 255 steps take one round.
     uint32_t sel_mask = 0, sel_val = 0;
     int rem = to_free;
-    for (int b = 3; b >= 0; --b) {
-      if (tid < LRU_DIGIT) sh_hist[tid] = 0;
+    for (int b = (31 - __clz(E)) >> 3; b >= 0; --b) {
+#pragma unroll
+      for (int i = 0; i < LRU_DIGIT * LRU_COPIES / LRU_THREADS; ++i) sh_hist[i * LRU_THREADS + tid] = 0;
       if (tid == 0) { sh_cut[0] = 0; sh_cut[1] = 0; }
       __syncthreads();
-      for (int cc = c0; cc < c1; ++cc) {
-        const int st = stamp[cc];
-        if (st == 0) continue;
+      resident([&](int, int st, int nbc) {
         const uint32_t age = (uint32_t)(E - st);
-        if ((age & sel_mask) == sel_val) atomicAdd(&sh_hist[(age >> (8 * b)) & 255u], boff[cc + 1] - boff[cc]);
-      }
+        if ((age & sel_mask) == sel_val)
+          atomicAdd(&sh_hist[((age >> (8 * b)) & 255u) * LRU_COPIES + (tid & (LRU_COPIES - 1))], nbc);
+      });
       __syncthreads();
       if (tid < 64) {
         // lane l holds the digits 255 - 4l .. 252 - 4l (oldest first); the lane whose running total crosses
         // rem holds the boundary digit
         int h[4], sum = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { h[i] = sh_hist[255 - (4 * tid + i)]; sum += h[i]; }
+        for (int i = 0; i < 4; ++i) {
+          const int4* hp = reinterpret_cast<const int4*>(sh_hist + (255 - (4 * tid + i)) * LRU_COPIES);
+          const int4 x = hp[0], y = hp[1];
+          h[i] = x.x + x.y + x.z + x.w + y.x + y.y + y.z + y.w;
+          sum += h[i];
+        }
         const int incl = (int)ri_wave_incl_scan((uint32_t)sum);
         int acc = incl - sum;
         if (acc < rem && rem <= incl) {
@@ -310,15 +343,15 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
       sel_val |= (uint32_t)sh_cut[0] << (8 * b);
       sel_mask |= 255u << (8 * b);
       rem -= sh_cut[1];
+      __syncthreads();
     }
     const uint32_t cut = sel_val;   // boundary age; rem blocks are still wanted from the clusters of that age
     // the clusters of the boundary step, least recent first = ascending order inside the step
     for (int i = tid; i < 2 * NPMAX; i += LRU_THREADS) sh_tab[i] = 0;
     __syncthreads();
-    for (int cc = c0; cc < c1; ++cc) {
-      const int st = stamp[cc];
-      if (st != 0 && (uint32_t)(E - st) == cut) sh_tab[min(max(order[cc], 0), 2 * NPMAX - 1)] = boff[cc + 1] - boff[cc];
-    }
+    resident([&](int cc, int st, int nbc) {
+      if ((uint32_t)(E - st) == cut) sh_tab[min(max(order[cc], 0), 2 * NPMAX - 1)] = nbc;
+    });
     __syncthreads();
     {
       // exclusive prefix of the table in place: thread t owns the entries [t * 2R, t * 2R + 2R)
@@ -333,16 +366,14 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
     __syncthreads();
     int ev = 0;
     uint64_t ev_bits = 0;  // K <= 64 ids per thread
-    for (int cc = c0; cc < c1; ++cc) {
-      const int st = stamp[cc];
-      if (st == 0) continue;
+    resident([&](int cc, int st, int nbc) {
       const uint32_t age = (uint32_t)(E - st);
       const bool out = age > cut || (age == cut && sh_tab[min(max(order[cc], 0), 2 * NPMAX - 1)] < rem);
       if (out) {
         ev_bits |= 1ull << (cc - c0);
-        ev += boff[cc + 1] - boff[cc];
+        ev += nbc;
       }
-    }
+    });
     int ve[1] = {ev}, pe[1], te[1];
     lru_scan<1>(ve, pe, te, sh_scan);
     int w = F0 + pe[0];
@@ -388,6 +419,53 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(LruParams P) {
   }
 }
 
+template <int R, int PHASE>
+__global__ __launch_bounds__(LRU_THREADS) void lru_kernel(ri_lru_t P) {
+  lru_group<R, PHASE>(P, blockIdx.x);
+}
+
+// grid (1 + X, groups): workgroup 0 of a group updates the cache's books, the others copy the group's missed rows from the
+// host store into the staging rows, eight items of at most `block` rows at a time (16 lanes per row).
+template <int R>
+__global__ __launch_bounds__(LRU_THREADS) void lru_stage_kernel(ri_lru_t P) {
+  const int g = blockIdx.y;
+  if (blockIdx.x == 0) {
+    lru_group<R, LRU_UPDATE>(P, g);
+    return;
+  }
+  const int n = P.miss_num[g];
+  const size_t lists = (size_t)g * P.buffer_size;
+  const int sub = threadIdx.x >> 7, vec = (threadIdx.x & 127) >> 4, piece = threadIdx.x & 15;
+  for (int j = (blockIdx.x - 1) * 8 + sub; j < n; j += (gridDim.x - 1) * 8) {
+    const int rows = P.miss_sizes[lists + j];
+    const size_t src = (size_t)g * P.host_stride + P.miss_ids[lists + j];
+    const size_t dst = (size_t)g * P.cache_stride + P.stage_row0 + P.miss_cumsum[lists + j];
+    for (int r = vec; r < rows; r += 8) {
+      const uint4 k = reinterpret_cast<const uint4*>(P.host_k)[(src + r) * 16 + piece];
+      const uint4 v = reinterpret_cast<const uint4*>(P.host_v)[(src + r) * 16 + piece];
+      reinterpret_cast<uint4*>(P.cache_k)[(dst + r) * 16 + piece] = k;
+      reinterpret_cast<uint4*>(P.cache_v)[(dst + r) * 16 + piece] = v;
+    }
+  }
+}
+
+static int lru_check(const ri_lru_t& P) {
+  // (a cache without blocks has an empty free list: its pointer may be null)
+  if (!P.ret_ids || !P.sizes || !P.starts || !P.blk_off || !P.stamp || !P.order || !P.blk_ids ||
+      (!P.free_list && P.capacity > 0) || !P.free_count || !P.epoch || !P.hit_ids || !P.hit_sizes || !P.hit_cumsum ||
+      !P.hit_num || !P.miss_ids || !P.miss_sizes || !P.miss_cumsum || !P.miss_num || !P.upd_buf || !P.upd_sizes ||
+      !P.upd_cache || !P.upd_num)
+    return RI_ERR_ARG;
+  if (P.BG <= 0 || P.np <= 0 || P.np > 4 * LRU_THREADS || P.ncl <= 0 || P.ncl > 64 * LRU_THREADS || P.buffer_size <= 0 ||
+      P.capacity < 0 || P.block <= 0)
+    return RI_ERR_ARG;
+  if (P.meta_stride < P.ncl || P.blk_off_stride < P.ncl + 1 || P.stamp_stride < P.ncl || P.blk_ids_stride <= 0)
+    return RI_ERR_ARG;
+  if (P.row_src && (!P.meta || P.row_src_stride < P.buffer_size * P.block || P.stage_row0 < P.capacity * P.block))
+    return RI_ERR_ARG;
+  return RI_OK;
+}
+
 extern "C" int ri_lru_access_update(const int32_t* ret_ids, const int32_t* sizes, const int32_t* starts,
                                     int meta_stride, const int32_t* blk_off, int blk_off_stride, int32_t* stamp,
                                     int32_t* order, int stamp_stride, int32_t* blk_ids, int blk_ids_stride, int32_t* free_list,
@@ -397,25 +475,46 @@ extern "C" int ri_lru_access_update(const int32_t* ret_ids, const int32_t* sizes
                                     int32_t* upd_cache, int32_t* upd_num, int32_t* row_src, int row_src_stride,
                                     int stage_row0, int32_t* meta, int BG, int np, int ncl, int buffer_size,
                                     int capacity, int block, ri_stream_t stream) {
-  // (a cache without blocks has an empty free list: its pointer may be null)
-  if (!ret_ids || !sizes || !starts || !blk_off || !stamp || !order || !blk_ids || (!free_list && capacity > 0) || !free_count ||
-      !epoch ||
-      !hit_ids || !hit_sizes || !hit_cumsum || !hit_num || !miss_ids || !miss_sizes || !miss_cumsum || !miss_num ||
-      !upd_buf || !upd_sizes || !upd_cache || !upd_num)
-    return RI_ERR_ARG;
-  if (BG <= 0 || np <= 0 || np > 4 * LRU_THREADS || ncl <= 0 || ncl > 64 * LRU_THREADS || buffer_size <= 0 ||
-      capacity < 0 || block <= 0)
-    return RI_ERR_ARG;
-  if (meta_stride < ncl || blk_off_stride < ncl + 1 || stamp_stride < ncl || blk_ids_stride <= 0) return RI_ERR_ARG;
-  if (row_src && (!meta || row_src_stride < buffer_size * block || stage_row0 < capacity * block)) return RI_ERR_ARG;
-  LruParams P = {ret_ids, sizes, starts, blk_off, stamp, order, blk_ids, free_list, free_count, epoch,
-                 hit_ids, hit_sizes, hit_cumsum, hit_num, miss_ids, miss_sizes, miss_cumsum, miss_num,
-                 upd_buf, upd_sizes, upd_cache, upd_num, row_src, meta, row_src_stride, stage_row0,
-                 np, ncl, meta_stride, blk_off_stride, stamp_stride, blk_ids_stride, buffer_size, capacity, block};
+  const ri_lru_t P = {ret_ids, sizes, starts, blk_off, stamp, order, blk_ids, free_list, free_count, epoch,
+                      hit_ids, hit_sizes, hit_cumsum, hit_num, miss_ids, miss_sizes, miss_cumsum, miss_num,
+                      upd_buf, upd_sizes, upd_cache, upd_num, row_src, meta, nullptr, nullptr, nullptr, nullptr, 0, 0,
+                      row_src_stride, stage_row0, np, ncl, meta_stride, blk_off_stride, stamp_stride, blk_ids_stride,
+                      buffer_size, capacity, block, BG};
+  const int rc = lru_check(P);
+  if (rc) return rc;
   if (np < LRU_THREADS)
-    lru_kernel<1><<<BG, LRU_THREADS, 0, (hipStream_t)stream>>>(P);
+    lru_kernel<1, LRU_BOTH><<<BG, LRU_THREADS, 0, (hipStream_t)stream>>>(P);
   else
-    lru_kernel<4><<<BG, LRU_THREADS, 0, (hipStream_t)stream>>>(P);
+    lru_kernel<4, LRU_BOTH><<<BG, LRU_THREADS, 0, (hipStream_t)stream>>>(P);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_lru_access(const ri_lru_t* s, ri_stream_t stream) {
+  if (!s) return RI_ERR_ARG;
+  const int rc = lru_check(*s);
+  if (rc) return rc;
+  if (s->np < LRU_THREADS)
+    lru_kernel<1, LRU_ACCESS><<<s->BG, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
+  else
+    lru_kernel<4, LRU_ACCESS><<<s->BG, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_lru_stage_update(const ri_lru_t* s, ri_stream_t stream) {
+  if (!s) return RI_ERR_ARG;
+  const int rc = lru_check(*s);
+  if (rc) return rc;
+  if (!s->row_src || !s->host_k || !s->host_v || !s->cache_k || !s->cache_v || s->host_stride <= 0 || s->BG > 65535 ||
+      s->cache_stride < (int64_t)s->stage_row0 + (int64_t)s->buffer_size * s->block)
+    return RI_ERR_ARG;
+  if (ri_any_misaligned16(s->host_k, s->host_v, s->cache_k, s->cache_v)) return RI_ERR_ARG;
+  // A workgroup takes eight blocks at a time.  Many per group, most of them without work: the groups then start one after
+  // the other, and the link carries 54.9 GB/s; with at most sixteen, all groups' reads are mixed and it carries 50.0.
+  const dim3 grid(1 + min(64, (s->buffer_size + 7) / 8), s->BG);
+  if (s->np < LRU_THREADS) lru_stage_kernel<1><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
+  else lru_stage_kernel<4><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

@@ -49,3 +49,26 @@ extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int stat
                 s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out, s->valid_lengths, s->BG,
                 s->gs, s->nc, s->es, s->scale, s->attn_workspace, s->attn_workspace_bytes, stream);
 }
+
+extern "C" int ri_host_step(const ri_decode_step_t* s, const ri_lru_t* lru, const void* q, int static_len, void* out,
+                            ri_stream_t stream) {
+  if (!s || !lru) return RI_ERR_ARG;
+  auto* select = s->half ? ri_score_select_f16 : ri_score_select;
+  auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
+  int rc = select(q, s->centroids, s->mask, nullptr, nullptr, s->logits, nullptr, nullptr, s->ret_ids, s->est_ids, nullptr,
+                  nullptr, nullptr, 0, nullptr, s->BG, s->gs, s->nc, s->np, s->es, s->page, s->max_pages, s->scale,
+                  s->score_workspace, s->score_workspace_bytes, stream);
+  if (rc) return rc;
+  if ((rc = ri_lru_access(lru, stream))) return rc;
+  if ((rc = ri_lru_stage_update(lru, stream))) return rc;
+  rc = attend(q, s->steady_k, s->steady_v, s->steady_stride, static_len, s->static_len_dev, s->store_k, s->store_v,
+              s->store_stride, lru->row_src, lru->row_src_stride, nullptr, nullptr, 0, s->meta, s->est_ids,
+              s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out, s->valid_lengths, s->BG, s->gs,
+              s->nc, s->es, s->scale, s->attn_workspace, s->attn_workspace_bytes, stream);
+  if (rc) return rc;
+  const size_t stage = (size_t)lru->stage_row0 * RI_DIM * 2;
+  return ri_gather_copy_and_scatter((const char*)lru->cache_k + stage, lru->cache_k, (const char*)lru->cache_v + stage,
+                                    lru->cache_v, lru->upd_buf, lru->upd_sizes, lru->upd_cache, lru->upd_num, lru->BG,
+                                    (int)lru->cache_stride, (int)(lru->cache_stride / lru->block), lru->buffer_size, 0,
+                                    stream);
+}

@@ -12,7 +12,7 @@ import math
 
 import torch
 
-from ._lib import DecodeStep, lib, check
+from ._lib import DecodeStep, Lru, lib, check
 
 # 16-bit element types of the reference's operators and cache (batch_gemm_softmax.cu:185-197,
 # gather_copy.cu:63-67): every wrapper takes either and calls the entry point of that type (name or name_f16).
@@ -425,6 +425,28 @@ class DecodeStepPlan:
             check(status, "decode_step")
 
 
+class HostStepPlan(DecodeStepPlan):
+    """The same over a host-resident store with the device-side block cache (ri_host_step).  `tensors` as above with the
+    cache tensors as store_k / store_v; lru: DeviceLru of the layer; lists: as for its access_update; host_k, host_v
+    [.., rows, 128] pinned; stage_row0: first staging row of the cache tensors."""
+
+    def __init__(self, key, dtype, tensors, nprobe, es, page, max_pages, scale, lru, sizes, starts, lists, row_src, host_k,
+                 host_v, stage_row0):
+        rows = tensors["store_k"].numel() // (lru.BG * 128)
+        tensors = dict(tensors, store_k=tensors["store_k"].view(lru.BG, rows, 128),
+                       store_v=tensors["store_v"].view(lru.BG, rows, 128))
+        super().__init__(key, dtype, tensors, nprobe, es, page, max_pages, scale)
+        self._lru = lru.prepared(tensors["ret_ids"], sizes, starts, lists, row_src, stage_row0, tensors["meta"], host_k,
+                                 host_v, tensors["store_k"], tensors["store_v"])
+        self._lru_address = ctypes.addressof(self._lru)
+        self._call = lib().ri_host_step
+
+    def run(self, q, static_len, out):
+        status = self._call(self._address, self._lru_address, q.data_ptr(), static_len, out.data_ptr(), _stream())
+        if status:
+            check(status, "host_step")
+
+
 def append_kv(key, value, steady_k, steady_v, pos, pos_dev=None):
     """steady[g, pos] = row g of key / value [BG, 128] (any shape of BG * 128 elements), one launch for both."""
     stride = steady_k.shape[-2]
@@ -512,6 +534,24 @@ class DeviceLru:
             _p(self.free_count), _p(self.epoch), *[_p(t) for t in lists], _p(row_src),
             0 if row_src is None else row_src.shape[1], stage_row0, _p(meta), BG, np_, ncl, self.buffer_size,
             self.capacity, self.block, _stream()), "lru_access_update")
+
+
+    def prepared(self, ret_ids, sizes, starts, lists, row_src, stage_row0, meta, host_k, host_v, cache_k, cache_v):
+        """The arguments of access_update and of the copy of the misses, host_k/v [.., rows, 128] to the staging rows of
+        cache_k/v [BG, rows, 128], for ri_lru_access and ri_lru_stage_update."""
+        names = [f"{a}_{b}" for a in ("hit", "miss") for b in ("ids", "sizes", "cumsum", "num")] + [
+            "upd_buf", "upd_sizes", "upd_cache", "upd_num"]
+        tensors = dict(zip(names, lists), ret_ids=ret_ids, sizes=sizes, starts=starts, blk_off=self.blk_off,
+                       stamp=self.stamp, order=self.order, blk_ids=self.blk_ids, free_list=self.free_list,
+                       free_count=self.free_count, epoch=self.epoch, row_src=row_src, meta=meta, host_k=host_k,
+                       host_v=host_v, cache_k=cache_k, cache_v=cache_v)
+        s = Lru(host_stride=host_k.shape[-2], cache_stride=cache_k.shape[-2], row_src_stride=row_src.shape[1],
+                stage_row0=stage_row0, np=ret_ids.shape[1], ncl=sizes.shape[1], meta_stride=sizes.stride(0),
+                blk_off_stride=self.blk_off.shape[1], stamp_stride=self.stamp.shape[1],
+                blk_ids_stride=self.blk_ids.shape[1], buffer_size=self.buffer_size, capacity=self.capacity,
+                block=self.block, BG=self.BG, **{nm: _p(t) for nm, t in tensors.items()})
+        s.tensors = tensors   # (alive as long as their addresses are)
+        return s
 
 
 def kmeans_assign(data, centroids, assign, P, N, nc, seg, head_rows):

@@ -159,3 +159,53 @@ def test_bad_arguments(dev):
     assert l.ri_lru_access_update(p, p, p, 8, p, 9, p, p, 8, p, 8, p, p, p, *ptrs, None, 0, 0, None, 1, 4097, 8, 4, 4, 8, None) == -1   # np too large
     assert l.ri_lru_access_update(p, p, p, 4, p, 9, p, p, 8, p, 8, p, p, p, *ptrs, None, 0, 0, None, 1, 2, 8, 4, 4, 8, None) == -1      # stride < ncl
     assert l.ri_lru_access_update(None, p, p, 8, p, 9, p, p, 8, p, 8, p, p, p, *ptrs, None, 0, 0, None, 1, 2, 8, 4, 4, 8, None) == -1
+
+
+@pytest.mark.parametrize("ncl,nprobe,capacity,buffer_size", [(300, 20, 60, 48), (4097, 60, 500, 400), (9000, 1100, 3000, 5000),
+                                                             (200, 10, 0, 64)])
+def test_access_and_stage_update_equal_the_one_launch(dev, ncl, nprobe, capacity, buffer_size):
+    """Access and update apart: same lists, row table and books as in one launch, with ages of one to three bytes, and the
+    missed rows in the staging rows."""
+    import ctypes
+    from retrievalattention_amd import kernels
+    from retrievalattention_amd._lib import lib
+    BG, block = 2, 8
+    g = torch.Generator().manual_seed(ncl)
+    sz = torch.randint(0, 30, (BG, ncl), generator=g, dtype=torch.int32).to(dev)
+    st = (torch.cumsum(sz.long(), 1) - sz.long()).to(torch.int32)
+    n = int(sz.sum(1).max())
+    max_blocks = int(((sz + block - 1) // block).sum(1).max()) + 1
+    host = [torch.randn(BG, n, 128, generator=g).to(torch.bfloat16).pin_memory() for _ in range(2)]
+    stage0 = capacity * block
+    cache = [torch.zeros(BG, stage0 + buffer_size * block, 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    sides = []
+    for _ in range(2):
+        lru = kernels.DeviceLru(BG, ncl, max_blocks, capacity, buffer_size, block, dev)
+        lru.set_sizes(sz)
+        lists = [torch.zeros((BG,) if i % 4 == 3 else (BG, buffer_size), dtype=torch.int32, device=dev) for i in range(12)]
+        row_src = torch.zeros(BG, buffer_size * block, dtype=torch.int32, device=dev)
+        sides.append((lru, lists, row_src, torch.zeros(BG, 4, dtype=torch.int32, device=dev)))
+    hot = torch.randperm(ncl, generator=g)[:4 * nprobe]
+    ids = torch.zeros(BG, nprobe, dtype=torch.int32, device=dev)
+    lru, lists, row_src, meta = sides[1]
+    s = lru.prepared(ids, sz, st, lists, row_src, stage0, meta, *host, *cache)
+    for step in range(12):
+        for b in range(BG):
+            ids[b] = hot[torch.randperm(hot.numel(), generator=g)[:nprobe]]
+        if step in (4, 8):
+            for side in sides:
+                side[0].epoch += 300 if step == 4 else 70000
+        sides[0][0].access_update(ids, sz, st, sides[0][1], row_src=sides[0][2], stage_row0=stage0, meta=sides[0][3])
+        for fn in (lib().ri_lru_access, lib().ri_lru_stage_update):
+            assert fn(ctypes.addressof(s), kernels._stream()) == 0
+        for x, y in zip(sides[0][1] + list(sides[0][2:]), lists + [row_src, meta]):
+            assert torch.equal(x, y), step
+        for name in ("stamp", "blk_ids", "free_list", "free_count", "epoch"):
+            assert torch.equal(getattr(sides[0][0], name), getattr(lru, name)), (step, name)
+        resident = lru.stamp > 0
+        assert torch.equal(sides[0][0].order[resident], lru.order[resident])
+        for b in range(BG):
+            for j in range(int(lists[7][b])):
+                row, k, at = (int(lists[4 + x][b, j]) for x in range(3))
+                for h, c in zip(host, cache):
+                    assert torch.equal(c[b, stage0 + at:stage0 + at + k].cpu(), h[b, row:row + k])
