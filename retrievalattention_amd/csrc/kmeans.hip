@@ -971,12 +971,18 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   km_assign_kernel<TT, CT, W, NB, HALF><<<dim3((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, (hipStream_t)stream>>>( \
       (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows)
   const long long wgs128 = (long long)P * ((N + 127) / 128), wgs256 = (long long)P * ((N + 255) / 256);
+  const long long wgs768 = (long long)P * ((N + 767) / 768);
   const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
   // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
   // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
   // against 18.9 with two columns; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
   if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
   else if (wgs256 <= 512) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
+  // One workgroup per compute unit that gives each wave three or four columns, where the fullest unit has that many
+  // columns per wave to do anyway: the same work with more reuse of every LDS read (16 x 8200 tokens, 512 centroids: 25.8
+  // us against 28.7 for the last line's; 4 x 48719, 3072: 124 against 135; 20 x 9757, 608: 37.8 against 40.4).
+  else if (nc >= 512 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
+  else if (nc >= 512 && wgs256 > 768 && wgs1024 <= 256) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
   // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
   // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves; 4 x 65536, 4096: 219 against
   // 232), provided the last round of these large workgroups is not mostly empty.

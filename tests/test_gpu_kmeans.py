@@ -72,6 +72,25 @@ def test_assign_update_valuesum(dev, P, N, nc, seed, dt=torch.bfloat16):
         assert torch.equal(vsum[p].cpu(), okm.value_sum(vals[p], A[p].astype(np.int64), nc))
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("P,N,nc", [(5, 1001, 32), (8, 8193, 544), (16, 8200, 544), (20, 9757, 608), (33, 8200, 512),
+                                    (3, 100000, 1056), (4, 65500, 1056)])
+def test_assign_tilings(dev, P, N, nc, dt):
+    """One size for every tiling of the assignment, with a remainder of tokens and of centroids."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator(device=dev).manual_seed(N)
+    data = torch.randn(P, N, 128, generator=g, device=dev).to(dt)
+    cent = torch.nn.functional.normalize(torch.randn(P, nc, 128, generator=g, device=dev), dim=-1).to(dt)
+    assign = torch.full((P, N), -1, dtype=torch.int32, device=dev)
+    kernels.kmeans_assign(data, cent, assign, P, N, nc, 1, N)
+    for p in range(P):
+        s = data[p].double() @ cent[p].double().T
+        best, at = s.max(dim=1)
+        mine = s.gather(1, assign[p].long()[:, None])[:, 0]
+        assert bool((best - mine <= 1e-5).all())            # (fp32 sums of products may swap near-ties)
+        assert float((at != assign[p]).float().mean()) < 1e-3
+
+
 @pytest.mark.parametrize("P,N,nc,seed", [(3, 1000, 64, 10), (2, 8192, 512, 11), (1, 4100, 1024, 12), (4, 37, 32, 13)])
 def test_assign_update_valuesum_float16(dev, P, N, nc, seed):
     """IEEE half keys, values and centroids (the reference's harnesses default to fp16, simple_test.py:29):
