@@ -76,6 +76,14 @@ def _need(t, dtype, name, cuda=True):
         raise ValueError(f"{name}: expected a contiguous tensor")
 
 
+def _need_all(tensors, dtype, names):
+    """_need for device tensors of one type: one look at each while nothing is wrong."""
+    for t in tensors:
+        if t.dtype is not dtype or not t.is_cuda or not t.is_contiguous():
+            for x, nm in zip(tensors, names):
+                _need(x, dtype, nm)
+
+
 _workspaces = {}
 _workspace_generation = 0  # moves on whenever a scratch tensor is replaced: holders of an address look again
 _retired_workspaces = []   # superseded scratch tensors: captured HIP graphs may still hold their addresses
@@ -88,7 +96,7 @@ def _workspace(nbytes, device, tag):
     address, so handing the block back to the allocator would let that replay write into someone else's
     memory.  Growing (or first use) during a capture is refused: the allocation would land in the graph's
     private pool and its zero fill would become a memset node of the graph."""
-    key = (str(device), tag)
+    key = (device, tag)
     w = _workspaces.get(key)
     if w is None or w.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
@@ -142,9 +150,8 @@ def batch_gemm_softmax(A, B, D, Norm, Sum, Softmax, batch_count, m, n, k, alpha=
     """batch_gemm_softmax.cu:201-209.  A [bc, m, k], B [bc, n, k]; D/Softmax [bc, m, n]."""
     if A.dtype not in _DT:
         raise RuntimeError("Only Half and BFloat16 are supported")      # batch_gemm_softmax.cu:196
-    for t, nm in ((A, "A"), (B, "B"), (D, "D"), (Softmax, "Softmax")):
-        _need(t, A.dtype, nm)
-    _need(Norm, torch.float32, "Norm"); _need(Sum, torch.float32, "Sum")
+    _need_all((A, B, D, Softmax), A.dtype, ("A", "B", "D", "Softmax"))
+    _need_all((Norm, Sum), torch.float32, ("Norm", "Sum"))
     ntiles = (n + 255) // 256
     if A.numel() < batch_count * m * k or B.numel() < batch_count * n * k or \
             D.numel() < batch_count * m * n or Softmax.numel() < batch_count * m * n or \
@@ -160,9 +167,8 @@ def gather_copy_vectors(key_data, key_buffer, value_data, value_buffer, src_meta
     """gather_copy.cu:288-292.  The rows are moved as 16-bit elements: Half or BFloat16 (gather_copy.cu:63-67)."""
     if key_data.dtype not in _DT:
         raise RuntimeError("Only Half and BFloat16 are supported")
-    for t, nm in ((key_data, "key_data"), (key_buffer, "key_buffer"), (value_data, "value_data"),
-                  (value_buffer, "value_buffer"), (src_metadata, "src_metadata"), (dst_metadata, "dst_metadata")):
-        _need(t, key_data.dtype, nm)
+    _need_all((key_data, key_buffer, value_data, value_buffer, src_metadata, dst_metadata), key_data.dtype,
+              ("key_data", "key_buffer", "value_data", "value_buffer", "src_metadata", "dst_metadata"))
     _need(data_offsets, torch.int64, "data_offsets")
     if key_data.numel() < groups * data_length * 128 or key_buffer.numel() < groups * buffer_length * 128 or \
             data_offsets.numel() < groups * index_size or src_metadata.numel() < groups * data_length or \
@@ -211,6 +217,11 @@ def gather_copy_and_scatter(key_data, key_buffer, value_data, value_buffer, s_of
           "gather_copy_and_scatter")
 
 
+@functools.lru_cache(maxsize=64)
+def _flash_workspace_bytes(BG, gs):
+    return lib().ri_flash_decoding_workspace_bytes(BG, gs)
+
+
 @_ranged("flash_attention")
 def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_lse=None, cache_seqlens=None,
                             return_softmax_lse=False):
@@ -222,10 +233,10 @@ def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_ls
     if one != 1 or D != 128 or k.shape[2] != 1:
         raise ValueError("weighted_flash_decoding: expected q [BG,1,gs,128], k/v [BG,S,1,128]")
     dt = q.dtype
-    for t, nm in ((q, "q"), (k, "k"), (v, "v")):
-        _need(t, dt, nm)
     if weight is not None:
-        _need(weight, dt, "weight")
+        _need_all((q, k, v, weight), dt, ("q", "k", "v", "weight"))
+    else:
+        _need_all((q, k, v), dt, ("q", "k", "v"))
     if previous_out is not None:
         _need(previous_out, dt, "previous_out")
         _need(previous_lse, torch.float32, "previous_lse")
@@ -233,8 +244,7 @@ def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_ls
         _need(cache_seqlens, torch.int32, "cache_seqlens")
     out = torch.empty_like(q)
     lse = torch.empty((BG, gs), dtype=torch.float32, device=q.device) if return_softmax_lse else None
-    nb = lib().ri_flash_decoding_workspace_bytes(BG, gs)
-    ws = _workspace(nb, q.device, "attn")
+    ws = _workspace(_flash_workspace_bytes(BG, gs), q.device, "attn")
     check(_fn("ri_weighted_flash_decoding", dt)(_p(q), _p(k), _p(v), _p(weight), _p(cache_seqlens), _p(previous_out),
                                            _p(previous_lse), _p(out), _p(lse), BG, gs, S, S,
                                            1.0 / math.sqrt(D), _p(ws), ws.numel(), _stream()),
