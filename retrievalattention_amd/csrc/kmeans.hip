@@ -35,6 +35,26 @@ __device__ __forceinline__ size_t km_row0(int p, int seg, int64_t head_rows, int
 template <int V>
 __device__ __forceinline__ void km_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory"); }
 
+// One step of three searches for m: i0, i1, i2 become I0, I1, I2 where those scores equal it.  The hardware wants two
+// instructions between a comparison and the select that reads its mask; in one chain of fifteen, which the compiler makes
+// of every way to write this, they are idle (62 issue slots per search, 31 here).  With one or two token columns per wave
+// that delays the next products (8 x 8192 tokens, 512 centroids: 12.3 -> 11.7 us; 24 x 8119, 512: 30.0 -> 29.0; 4 x
+// 9000, 288: 8.05 -> 7.61); with three or four they are the other columns' and nothing changes (8 x 32768, 2048: 112.8
+// and 113 us), or the three more registers cost (16 x 8200, 512: 24.8 and 25.9), so the chain stays there.
+// (The scores have been read by the maximum before: no matrix result is outstanding when this runs.)
+template <int I0, int I1, int I2>
+__device__ __forceinline__ void km_first_of(const f32x16_t& x, float m, int& i0, int& i1, int& i2) {
+  uint64_t e0, e1, e2;
+  asm("v_cmp_eq_f32_e64 %3, %6, %9\n\t"
+      "v_cmp_eq_f32_e64 %4, %7, %9\n\t"
+      "v_cmp_eq_f32_e64 %5, %8, %9\n\t"
+      "v_cndmask_b32_e64 %0, %0, %10, %3\n\t"
+      "v_cndmask_b32_e64 %1, %1, %11, %4\n\t"
+      "v_cndmask_b32_e64 %2, %2, %12, %5"
+      : "+v"(i0), "+v"(i1), "+v"(i2), "=&s"(e0), "=&s"(e1), "=&s"(e2)
+      : "v"(x[I0]), "v"(x[I1]), "v"(x[I2]), "v"(m), "n"(I0), "n"(I1), "n"(I2));
+}
+
 template <int KM_TT, int KM_CT, int KM_W, int KM_NB, bool HALF>
 __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __restrict__ data,
                                                               const uint16_t* __restrict__ cent,
@@ -125,8 +145,18 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
           const bool upd = m > best[tt];
           if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
             int sel = 15;
+            if constexpr (KM_TT <= 2) {
+              int s1 = 15, s2 = 15;
+              km_first_of<4, 9, 14>(acc[tt], m, sel, s1, s2);
+              km_first_of<3, 8, 13>(acc[tt], m, sel, s1, s2);
+              km_first_of<2, 7, 12>(acc[tt], m, sel, s1, s2);
+              km_first_of<1, 6, 11>(acc[tt], m, sel, s1, s2);
+              km_first_of<0, 5, 10>(acc[tt], m, sel, s1, s2);
+              sel = min(min(sel, s1), s2);
+            } else {
 #pragma unroll
-            for (int i = 14; i >= 0; --i) sel = (acc[tt][i] == m) ? i : sel;
+              for (int i = 14; i >= 0; --i) sel = (acc[tt][i] == m) ? i : sel;
+            }
             if (upd) {
               best[tt] = m;
               bidx[tt] = ct + half * 32 + (sel >> 2) * 8 + hh * 4 + (sel & 3);

@@ -91,6 +91,28 @@ def test_assign_tilings(dev, P, N, nc, dt):
         assert float((at != assign[p]).float().mean()) < 1e-3
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("P,N,nc", [(5, 1001, 32), (8, 8193, 544), (16, 8200, 544), (20, 9757, 608), (33, 8200, 512),
+                                    (3, 100000, 1056)])
+def test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt):
+    """Small whole numbers: every score is exact in fp32, and every centroid appears again four rows on (the other half
+    of the wave), 32 rows on (the next sub-tile) or in place of one before it, so that most maxima are tied."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator(device=dev).manual_seed(N)
+    data = torch.randint(-2, 3, (P, N, 128), generator=g, device=dev).to(dt)
+    cent = torch.randint(-2, 3, (P, nc, 128), generator=g, device=dev).to(dt)
+    cent[:, 4:nc:8] = cent[:, 0:nc - 4:8]
+    cent[:, 33:nc:64] = cent[:, 1:nc - 32:64]
+    cent[:, nc - 1] = cent[:, 2]
+    assign = torch.full((P, N), -1, dtype=torch.int32, device=dev)
+    kernels.kmeans_assign(data, cent, assign, P, N, nc, 1, N)
+    ids = torch.arange(nc, device=dev)
+    for p in range(P):
+        s = data[p].double() @ cent[p].double().T
+        first = torch.where(s == s.max(dim=1, keepdim=True)[0], ids, nc).amin(dim=1)
+        assert torch.equal(assign[p].long(), first)
+
+
 @pytest.mark.parametrize("P,N,nc,seed", [(3, 1000, 64, 10), (2, 8192, 512, 11), (1, 4100, 1024, 12), (4, 37, 32, 13)])
 def test_assign_update_valuesum_float16(dev, P, N, nc, seed):
     """IEEE half keys, values and centroids (the reference's harnesses default to fp16, simple_test.py:29):
