@@ -552,6 +552,21 @@ int ri_kmeans_value_rows_f16(const void* values, int64_t head_stride, int64_t ro
                              int64_t store_stride_rows, int P, int N, int nc, void* workspace, size_t workspace_bytes,
                              ri_stream_t stream);
 
+/* The last step of a prefill: ri_kmeans_value_rows with a store, and for the keys (raw rows, strides as the values')
+   the same store and the means, not normalised, of the rows minus mean[p] in the element type: what ri_kmeans_update
+   gives over the centred keys and ri_permute_rows_strided over the raw ones.  One segment per head; centroids of
+   empty clusters stay as they are.  workspace_bytes: twice ri_kmeans_reduce_workspace_bytes. */
+int ri_kmeans_store_rows(const void* values, int64_t v_head_stride, int64_t v_row_stride, const void* keys,
+                         int64_t k_head_stride, int64_t k_row_stride, const void* mean, const int32_t* counts,
+                         const int32_t* offsets, const int32_t* members, void* value_sum, void* centroids,
+                         void* value_store, void* key_store, int64_t store_stride_rows, int P, int N, int nc,
+                         void* workspace, size_t workspace_bytes, ri_stream_t stream);
+int ri_kmeans_store_rows_f16(const void* values, int64_t v_head_stride, int64_t v_row_stride, const void* keys,
+                             int64_t k_head_stride, int64_t k_row_stride, const void* mean, const int32_t* counts,
+                             const int32_t* offsets, const int32_t* members, void* value_sum, void* centroids,
+                             void* value_store, void* key_store, int64_t store_stride_rows, int P, int N, int nc,
+                             void* workspace, size_t workspace_bytes, ri_stream_t stream);
+
 /* Initial centroids: row trunc(c * (N / nc) + N / nc / 2) of every problem, in float32 (kmeans.py:234-236). */
 int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_stream_t stream);
 

@@ -27,8 +27,9 @@ class KMeansResult:
     __slots__ = ("centroids", "value_sum", "assign", "counts", "offsets", "members")
 
 
-def _cluster(key, num_centroids, num_iters, num_segments, init_indices):
-    """Everything of the clustering that reads the keys: centroids, assignment, inverted lists."""
+def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_means=True):
+    """Everything of the clustering that reads the keys: centroids, assignment, inverted lists.  final_means off: the
+    caller takes the last means over the lists."""
     G, N, D = key.shape
     dev = key.device
     nc, S = num_centroids, num_segments
@@ -64,7 +65,8 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices):
                                      (r.counts, r.offsets, r.members))
     else:
         kernels.kmeans_build_lists(r.assign, r.counts, r.offsets, r.members, G, N, nc)
-        kernels.kmeans_update(key, r.counts, r.offsets, r.members, centroids, G, N, nc, 1, N, False)
+        if final_means:
+            kernels.kmeans_update(key, r.counts, r.offsets, r.members, centroids, G, N, nc, 1, N, False)
     r.centroids = centroids
     return r
 
@@ -78,12 +80,14 @@ _MAX_GRAPHS = 4
 
 
 def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1, init_indices=None,
-                        reuse_graph=False, value_sum=None, value_store=None, store_stride=0):
+                        reuse_graph=False, value_sum=None, value_store=None, store_stride=0, key_rows=None, key_mean=None,
+                        key_store=None):
     """Runs the clustering and returns a KMeansResult (no dense cluster lists, no host copy).
     key/value [G, N, 128] bfloat16 or float16 device tensors, keys contiguous.
 
     value_sum: [G, nc, 128] tensor for the sums (else a new one).  value_store: where the value rows are also
-    written cluster by cluster, store_stride rows from group to group.
+    written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
+    key_rows, the [G, N, 128] keys before key_mean was subtracted.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and the same
     shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -103,13 +107,13 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
         raise AssertionError("centroids per segment must be a multiple of 32")  # kmeans.py:99
     r = None
     if reuse_graph and not torch.cuda.is_current_stream_capturing():
-        gkey = (key.data_ptr(), tuple(key.shape), str(key.device), nc, num_iters, S,
+        gkey = (key.data_ptr(), tuple(key.shape), str(key.device), nc, num_iters, S, key_store is None,
                 None if init_indices is None else init_indices.data_ptr())
         hit = _GRAPHS.get(gkey)
         if hit is None and gkey in _SEEN:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
-                res = _cluster(key, nc, num_iters, S, init_indices)
+                res = _cluster(key, nc, num_iters, S, init_indices, key_store is None)
             hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph)
             _GRAPHS[gkey] = hit
             while len(_GRAPHS) > _MAX_GRAPHS:
@@ -125,8 +129,12 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
             while len(_SEEN) > 64:
                 _SEEN.popitem(last=False)
     if r is None:
-        r = _cluster(key, nc, num_iters, S, init_indices)
+        r = _cluster(key, nc, num_iters, S, init_indices, key_store is None)
     r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device) if value_sum is None else value_sum
+    if key_store is not None:
+        kernels.kmeans_store_rows(kernels.aligned_rows(value), key_rows, key_mean, r.counts, r.offsets, r.members,
+                                  r.value_sum, r.centroids, value_store, key_store, G, N, nc, store_stride)
+        return r
     kernels.kmeans_value_sum(kernels.aligned_rows(value), r.counts, r.offsets, r.members, r.value_sum, G, N, nc,
                              store=value_store, store_stride=store_stride)
     return r

@@ -356,8 +356,8 @@ class retroinfer_cache(KV_Cache):
         mean_key = torch.mean(ck, dim=1, keepdim=True)
         kernels.prefill_center(ck, mean_key)
 
-        # cluster-contiguous store built on the device (stands in for organize_kv on the host): values while
-        # their sums are taken, keys afterwards; clusters in id order, tokens ascending inside
+        # cluster-contiguous store built on the device (stands in for organize_kv on the host) while the last sums
+        # are taken; clusters in id order, tokens ascending inside
         store_k = store_v = None
         stride = 0
         if self.kv_residency == "device":
@@ -374,13 +374,12 @@ class retroinfer_cache(KV_Cache):
             store_k, store_v, stride = self.stage_keys, self.stage_values, self.stage_keys.shape[1]
         km = segment_k_means_csr(ck, head_values, self.n_centroids, num_segments=self.n_segment,
                                  reuse_graph=True,   # results are consumed below, before the next call
-                                 value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride)
+                                 value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride,
+                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k)
         kernels.prefill_index(km.centroids, mean_key, km.counts, km.offsets, self.centroids[layer_idx][rows],
                               self.centroids_mask[layer_idx][rows], self.cluster_size[layer_idx][rows],
                               self.cluster_size_i32[layer_idx][rows], self.cluster_start[layer_idx][rows])
         self.store_rows[layer_idx][rows] = [valid_length] * H
-        if store_k is not None:
-            kernels.permute_rows_strided(head_keys, km.members, store_k, H, valid_length, stride)
         if dev_organise:
             self.mainevents[dkey].record()
             with torch.cuda.stream(self.copystream):

@@ -553,9 +553,11 @@ __global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
 // select per row is left to the last eight: 8 x 131072 tokens, 8192 clusters 71.3 -> 57.0 us, with 64 rows in flight 67.4;
 // half the tokens in seven clusters of 4 x 20000 tokens 27.7 -> 19.7).
 // pitch: words between rows.  With wp the rows are also copied: row k of the list to wp + k * 64.
-template <bool HALF, int U, bool COPY = false>
+// CENTER: the sum is of the rows minus `mean` (this lane's two dims), as ri_prefill_center leaves them.
+template <bool HALF, int U, bool COPY = false, bool CENTER = false>
 __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const int32_t* mem, int k0, int k1, float& s0,
-                                            float& s1, size_t pitch = RI_DIM / 2, uint32_t* __restrict__ wp = nullptr) {
+                                            float& s1, size_t pitch = RI_DIM / 2, uint32_t* __restrict__ wp = nullptr,
+                                            uint32_t mean = 0u) {
   static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
   const auto add = [&](uint32_t w) {
@@ -564,6 +566,7 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
     s0 += x0;
     s1 += x1;
   };
+  const auto term = [&](uint32_t w) { return CENTER ? ri_sub2<HALF>(w, mean) : w; };
   for (int k = k0; k < k1; k += U) {
     const int n = min(U, k1 - k);
     const uint64_t at = (uint64_t)(rp + (size_t)mem[k + min(lane, n - 1)] * pitch);
@@ -584,13 +587,13 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
       if (e + 8 <= n) {
 #pragma unroll
         for (int j = e; j < e + 8; ++j) {
-          add(v[j]);
+          add(term(v[j]));
           if (COPY) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
         }
       } else if (e < n) {
 #pragma unroll
         for (int j = e; j < e + 8; ++j) {
-          add(j < n ? v[j] : 0u);   // the word 0 is (+0, +0) in either type
+          add(j < n ? term(v[j]) : 0u);   // the word 0 is (+0, +0) in either type
           if (COPY && j < n) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
         }
       }
@@ -649,15 +652,14 @@ __device__ __forceinline__ int km_slot_owner(const int32_t* __restrict__ off, in
 // cluster per wave.
 // COPY (sums of value rows): every row is also written where its list puts it, row off + k of problem p to
 // copy + (p * copy_stride + off + k) * 128: the cluster-contiguous store, without a second pass over the rows.
-template <bool MEAN, bool HALF, bool COPY>
-__global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restrict__ rows, size_t pitch,
-                                                        const int32_t* __restrict__ counts,
-                                                        const int32_t* __restrict__ offsets,
-                                                        const int32_t* __restrict__ members,
-                                                        uint16_t* __restrict__ out, float2* __restrict__ partial,
-                                                        int item_wgs, int cap, int N, int nc, int seg,
-                                                        int64_t head_stride, int normalize,
-                                                        uint16_t* __restrict__ copy, int64_t copy_stride) {
+template <bool MEAN, bool HALF, bool COPY, bool CENTER>
+__device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows, size_t pitch,
+                                               const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
+                                               const int32_t* __restrict__ members, uint16_t* __restrict__ out,
+                                               float2* __restrict__ partial, int item_wgs, int cap, int N, int nc,
+                                               int seg, int64_t head_stride, int normalize,
+                                               uint16_t* __restrict__ copy, int64_t copy_stride,
+                                               const uint16_t* __restrict__ mean) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int32_t* off = offsets + (size_t)p * (nc + 1);
@@ -665,14 +667,15 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
   const uint32_t* rp = reinterpret_cast<const uint32_t*>(rows) + (size_t)(p / seg) * head_stride +
                        (size_t)(p % seg) * N * pitch;
   uint32_t* wp = COPY ? reinterpret_cast<uint32_t*>(copy) + (size_t)p * copy_stride * (RI_DIM / 2) + lane : nullptr;
+  const uint32_t mw = CENTER ? reinterpret_cast<const uint32_t*>(mean)[p * (RI_DIM / 2) + lane] : 0u;
   if ((int)blockIdx.x < item_wgs) {
     const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (slot >= cap) return;
     int s, o, j;
     if (km_slot_owner(off, nc, slot, s, o, j) < 0) return;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, 32, COPY>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1, pitch,
-                                COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr);
+    km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1,
+                                        pitch, COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
     partial[((size_t)p * cap + slot) * 64 + lane] = make_float2(s0, s1);
     return;
   }
@@ -686,18 +689,54 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF, 32, COPY>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1, pitch,
-                              COPY ? wp + (size_t)off[c] * (RI_DIM / 2) : nullptr);
+  km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1, pitch,
+                                      COPY ? wp + (size_t)off[c] * (RI_DIM / 2) : nullptr, mw);
   km_finish<MEAN, HALF>(s0, s1, s, normalize, op);
+}
+
+template <bool MEAN, bool HALF, bool COPY>
+__global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restrict__ rows, size_t pitch,
+                                                        const int32_t* __restrict__ counts,
+                                                        const int32_t* __restrict__ offsets,
+                                                        const int32_t* __restrict__ members,
+                                                        uint16_t* __restrict__ out, float2* __restrict__ partial,
+                                                        int item_wgs, int cap, int N, int nc, int seg,
+                                                        int64_t head_stride, int normalize,
+                                                        uint16_t* __restrict__ copy, int64_t copy_stride) {
+  km_reduce_rows<MEAN, HALF, COPY, false>(rows, pitch, counts, offsets, members, out, partial, item_wgs, cap, N, nc, seg,
+                                          head_stride, normalize, copy, copy_stride, nullptr);
+}
+
+// Value sums with the value store (z = 0) and means of the centred keys with the key store (z = 1): the last step of a
+// prefill.  The keys are read raw, from where the model left them, and centred on the way to their sum, so that the
+// store needs no pass of its own.  Bound by the bytes: 8 x 131072 tokens, 1.07 GB in 211 us = 5.1 TB/s, the rate of a
+// copy (keys 51 us, values 102 and the copy of the keys 98 in launches of their own).
+struct KmStoreArgs {
+  const uint16_t* rows;
+  uint16_t *out, *copy;
+  float2* partial;
+  size_t pitch;          // words
+  int64_t head_stride;   // words
+};
+template <bool HALF>
+__global__ __launch_bounds__(256) void km_store_kernel(KmStoreArgs V, KmStoreArgs K, const uint16_t* __restrict__ mean,
+                                                       const int32_t* __restrict__ counts,
+                                                       const int32_t* __restrict__ offsets,
+                                                       const int32_t* __restrict__ members, int item_wgs, int cap, int N,
+                                                       int nc, int64_t copy_stride) {
+  if (blockIdx.z == 0)
+    km_reduce_rows<false, HALF, true, false>(V.rows, V.pitch, counts, offsets, members, V.out, V.partial, item_wgs, cap, N,
+                                             nc, 1, V.head_stride, 0, V.copy, copy_stride, nullptr);
+  else
+    km_reduce_rows<true, HALF, true, true>(K.rows, K.pitch, counts, offsets, members, K.out, K.partial, item_wgs, cap, N,
+                                           nc, 1, K.head_stride, 0, K.copy, copy_stride, mean);
 }
 
 // grid (item workgroups, P): the wave of a long list's first slot adds the block sums in block
 // order and finishes the cluster
 template <bool MEAN, bool HALF>
-__global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __restrict__ offsets,
-                                                             const float2* __restrict__ partial,
-                                                             uint16_t* __restrict__ out, int cap, int nc,
-                                                             int normalize) {
+__device__ __forceinline__ void km_fold(const int32_t* __restrict__ offsets, const float2* __restrict__ partial,
+                                        uint16_t* __restrict__ out, int cap, int nc, int normalize) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -726,6 +765,21 @@ __global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __re
   }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
   km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op);
+}
+
+template <bool MEAN, bool HALF>
+__global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __restrict__ offsets,
+                                                             const float2* __restrict__ partial,
+                                                             uint16_t* __restrict__ out, int cap, int nc,
+                                                             int normalize) {
+  km_fold<MEAN, HALF>(offsets, partial, out, cap, nc, normalize);
+}
+
+template <bool HALF>
+__global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmStoreArgs K,
+                                                            const int32_t* __restrict__ offsets, int cap, int nc) {
+  if (blockIdx.z == 0) km_fold<false, HALF>(offsets, V.partial, V.out, cap, nc, 0);
+  else km_fold<true, HALF>(offsets, K.partial, K.out, cap, nc, 0);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1227,6 +1281,60 @@ extern "C" int ri_kmeans_value_rows_f16(const void* values, int64_t head_stride,
                                         void* workspace, size_t workspace_bytes, ri_stream_t stream) {
   return km_value_rows<true>(values, head_stride, row_stride, counts, offsets, members, value_sum, store,
                              store_stride_rows, P, N, nc, workspace, workspace_bytes, stream);
+}
+
+template <bool HALF>
+static int km_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
+                         const void* mean, const int32_t* counts, const int32_t* offsets, const int32_t* members,
+                         void* value_sum, void* centroids, void* value_store, void* key_store, int64_t store_stride_rows,
+                         int P, int N, int nc, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  if (!values || !keys || !mean || !counts || !offsets || !members || !value_sum || !centroids || !value_store ||
+      !key_store || !workspace)
+    return RI_ERR_ARG;
+  if (ri_any_misaligned16(values, value_sum, value_store, workspace) ||
+      ri_any_misaligned16(keys, centroids, key_store, mean))
+    return RI_ERR_ARG;
+  int rc = km_check(P, N, nc);
+  if (rc) return rc;
+  if (v_head < 0 || k_head < 0 || v_row < RI_DIM || k_row < RI_DIM || (v_head | v_row | k_head | k_row) % 8 != 0 ||
+      store_stride_rows < N)
+    return RI_ERR_ARG;
+  const size_t each = ri_kmeans_reduce_workspace_bytes(P, N, nc);
+  if (workspace_bytes < 2 * each) return RI_ERR_WORKSPACE;
+  const int cap = km_item_cap(N), item_wgs = (cap + 3) / 4;
+  if ((long long)item_wgs + (nc + 3) / 4 > 0x7fffffffLL) return RI_ERR_ARG;
+  float2* const partial = (float2*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  const KmStoreArgs V = {(const uint16_t*)values, (uint16_t*)value_sum, (uint16_t*)value_store, partial,
+                         (size_t)v_row / 2, v_head / 2};
+  const KmStoreArgs K = {(const uint16_t*)keys, (uint16_t*)centroids, (uint16_t*)key_store,
+                         partial + (size_t)P * cap * (RI_DIM / 2), (size_t)k_row / 2, k_head / 2};
+  km_store_kernel<HALF><<<dim3(item_wgs + (nc + 3) / 4, P, 2), 256, 0, s>>>(V, K, (const uint16_t*)mean, counts, offsets,
+                                                                            members, item_wgs, cap, N, nc,
+                                                                            store_stride_rows);
+  RI_HIP_CHECK_LAUNCH();
+  km_store_fold_kernel<HALF><<<dim3(item_wgs, P, 2), 256, 0, s>>>(V, K, offsets, cap, nc);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_kmeans_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,
+                                    int64_t k_row, const void* mean, const int32_t* counts, const int32_t* offsets,
+                                    const int32_t* members, void* value_sum, void* centroids, void* value_store,
+                                    void* key_store, int64_t store_stride_rows, int P, int N, int nc, void* workspace,
+                                    size_t workspace_bytes, ri_stream_t stream) {
+  return km_store_rows<false>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum,
+                              centroids, value_store, key_store, store_stride_rows, P, N, nc, workspace, workspace_bytes,
+                              (hipStream_t)stream);
+}
+
+extern "C" int ri_kmeans_store_rows_f16(const void* values, int64_t v_head, int64_t v_row, const void* keys,
+                                        int64_t k_head, int64_t k_row, const void* mean, const int32_t* counts,
+                                        const int32_t* offsets, const int32_t* members, void* value_sum, void* centroids,
+                                        void* value_store, void* key_store, int64_t store_stride_rows, int P, int N,
+                                        int nc, void* workspace, size_t workspace_bytes, ri_stream_t stream) {
+  return km_store_rows<true>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum,
+                             centroids, value_store, key_store, store_stride_rows, P, N, nc, workspace, workspace_bytes,
+                             (hipStream_t)stream);
 }
 
 extern "C" int ri_kmeans_value_sum(const void* values, const int32_t* counts, const int32_t* offsets,

@@ -66,20 +66,12 @@ extern "C" int ri_prefill_split(const void* key, const void* value, int64_t key_
 // grid (ceil(rows / 16), H), 16 lanes per row.
 // ------------------------------------------------------------------------------------
 template <bool HALF>
-__device__ __forceinline__ uint32_t sub2(uint32_t a, uint32_t b) {
-  float a0, a1, b0, b1;
-  ri_unpack2<HALF>(a, a0, a1);
-  ri_unpack2<HALF>(b, b0, b1);
-  return (uint32_t)ri_f32_to_e16<HALF>(a0 - b0) | ((uint32_t)ri_f32_to_e16<HALF>(a1 - b1) << 16);
-}
-
-template <bool HALF>
 __global__ __launch_bounds__(256) void center_kernel(uint4* __restrict__ keys, const uint4* __restrict__ mean, int N) {
   const int i = blockIdx.x * 16 + (threadIdx.x >> 4), piece = threadIdx.x & 15;
   if (i >= N) return;
   uint4* kp = keys + ((size_t)blockIdx.y * N + i) * 16 + piece;
   const uint4 x = *kp, m = mean[(size_t)blockIdx.y * 16 + piece];
-  *kp = make_uint4(sub2<HALF>(x.x, m.x), sub2<HALF>(x.y, m.y), sub2<HALF>(x.z, m.z), sub2<HALF>(x.w, m.w));
+  *kp = make_uint4(ri_sub2<HALF>(x.x, m.x), ri_sub2<HALF>(x.y, m.y), ri_sub2<HALF>(x.z, m.z), ri_sub2<HALF>(x.w, m.w));
 }
 
 static int prefill_center(void* keys, const void* mean, int H, int N, bool half, ri_stream_t stream) {

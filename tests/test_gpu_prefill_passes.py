@@ -54,6 +54,15 @@ def test_prefill_passes(dev, dtype, H, N, nc, fused):
     for st, src in ((store, hv), (store_k, hk)):
         assert torch.equal(st[:, :N], torch.gather(src, 1, at)) and not st[:, N:].any()
 
+    # sums, means and both stores in one pass against the passes by themselves
+    means, both = cent.clone(), cent.clone()
+    kernels.kmeans_update(ck, counts, offsets, members, means, H, N, nc, 1, N, False)
+    sums.zero_()
+    stores = [torch.zeros_like(store) for _ in range(2)]
+    kernels.kmeans_store_rows(hv, hk, mean, counts, offsets, members, sums, both, *stores, H, N, nc, N + 7)
+    assert torch.equal(both, means) and torch.equal(sums, ref_sums)
+    assert torch.equal(stores[0], store) and torch.equal(stores[1], store_k)
+
     out, mask = torch.empty_like(cent), torch.empty((H, nc), dtype=torch.bool, device=dev)
     size16, size, start = torch.empty((H, nc), dtype=dtype, device=dev), torch.empty_like(counts), torch.empty_like(counts)
     kernels.prefill_index(cent, mean, counts, offsets, out, mask, size16, size, start)
