@@ -451,6 +451,9 @@ int ri_kmeans_update_direct(const void* data, const int32_t* assign, void* centr
 int ri_kmeans_update_direct_f16(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
                                 int32_t* offsets, int32_t* members, int P, int N, int nc, int seg,
                                 int64_t head_rows, int normalize, ri_stream_t stream);
+/* Its lists alone, in the same launch form (at most 16384 tokens per problem). */
+int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P, int N,
+                           int nc, ri_stream_t stream);
 
 /* Per-cluster value sums: replaces triton_index_add (cache_hub/kmeans.py:176-221).
  * value_sum[p,c,:] = bf16(Σ member value rows), Σ in the same fixed order as above. */

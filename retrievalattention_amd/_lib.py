@@ -84,6 +84,7 @@ SIGNATURES = {
     "ri_permute_rows_strided": (I, [P, I64, I64, P, P, I, I, I64, P]),
     "ri_kmeans_value_rows": (I, [P, I64, I64, P, P, P, P, P, I64, I, I, I, P, SZ, P]),
     "ri_kmeans_value_rows_f16": (I, [P, I64, I64, P, P, P, P, P, I64, I, I, I, P, SZ, P]),
+    "ri_kmeans_lists_direct": (I, [P, P, P, P, I, I, I, P]),
     "ri_kmeans_store_rows": (I, [P, I64, I64, P, I64, I64] + [P] * 8 + [I64, I, I, I, P, SZ, P]),
     "ri_kmeans_store_rows_f16": (I, [P, I64, I64, P, I64, I64] + [P] * 8 + [I64, I, I, I, P, SZ, P]),
     "ri_kmeans_init": (I, [P, P, I, I, I, P]),

@@ -60,7 +60,9 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_me
     r.offsets = torch.empty((G, nc + 1), dtype=torch.int32, device=dev)
     r.members = torch.empty((G, N), dtype=torch.int32, device=dev)
     kernels.kmeans_assign(key, centroids, r.assign, G, N, nc, 1, N)
-    if N <= kernels.KMEANS_DIRECT_MAX_TOKENS:
+    if N <= kernels.KMEANS_DIRECT_MAX_TOKENS and not final_means:
+        kernels.kmeans_lists_direct(r.assign, r.counts, r.offsets, r.members, G, N, nc)
+    elif N <= kernels.KMEANS_DIRECT_MAX_TOKENS:
         kernels.kmeans_update_direct(key, r.assign, centroids, G, N, nc, 1, N, False,
                                      (r.counts, r.offsets, r.members))
     else:

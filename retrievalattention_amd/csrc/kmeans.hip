@@ -793,7 +793,8 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 // Reading all assignments of the problem per workgroup (4 N bytes) is what the split costs: 32 KB at 8192 tokens, about a
 // microsecond.  128 x 8192 tokens, 512 clusters each: 56 us, bound by reading the keys, against 13 + 70 + 5 us of list
 // sort, sums and fold; 8 x 8192: 9.6 us against 12 + 11 + 4.5.
-// counts / offsets / members (CSR, as km_sort_small_kernel writes them) only when asked for.
+// counts / offsets / members (CSR, as km_sort_small_kernel writes them) only when asked for, and then alone if there is
+// no `cent`: the last pass of a prefill, whose means come with the stores (8 x 8192 tokens, whole prefill 367 -> 363 us).
 // ------------------------------------------------------------------------------------
 #define KM_DIRECT_WAVES 8
 #define KM_DIRECT_MAX 16384
@@ -932,6 +933,7 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
       counts[(size_t)p * nc + c0 + tid] = sh_off[tid + 1] - sh_off[tid];
     }
     if (tid == 0 && c0 + CPW >= nc) offsets[(size_t)p * (nc + 1) + nc] = N;
+    if (!cent) return;
   }
   const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM), 0, N * RI_DIM * 2, 0x00020000);
@@ -1204,14 +1206,9 @@ extern "C" int ri_kmeans_update_f16(const void* data, const int32_t* counts, con
 }
 
 template <bool HALF>
-static int km_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
+static int km_direct_launch(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
                             int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize,
                             ri_stream_t stream) {
-  if (!data || !assign || !centroids || (!counts != !members) || (!offsets != !members)) return RI_ERR_ARG;
-  if (ri_any_misaligned16(data, centroids)) return RI_ERR_ARG;
-  int rc = km_check(P, N, nc);
-  if (rc) return rc;
-  if (N > KM_DIRECT_MAX || seg <= 0 || P % seg != 0) return RI_ERR_ARG;
   const int rounds = (N + KM_DIRECT_WAVES * 64 - 1) / (KM_DIRECT_WAVES * 64);
   // tokens compacted (4 bytes) and listed (2 bytes); block sums of a long cluster (512 bytes per KM_BLK rows) fit there too
   const size_t lds = (size_t)rounds * KM_DIRECT_WAVES * 64 * 6 + 512;
@@ -1233,6 +1230,28 @@ static int km_update_direct(const void* data, const int32_t* assign, void* centr
 #undef KM_DIRECT_LAUNCH
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
+}
+
+template <bool HALF>
+static int km_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
+                            int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize,
+                            ri_stream_t stream) {
+  if (!data || !assign || !centroids || (!counts != !members) || (!offsets != !members)) return RI_ERR_ARG;
+  if (ri_any_misaligned16(data, centroids)) return RI_ERR_ARG;
+  int rc = km_check(P, N, nc);
+  if (rc) return rc;
+  if (N > KM_DIRECT_MAX || seg <= 0 || P % seg != 0) return RI_ERR_ARG;
+  return km_direct_launch<HALF>(data, assign, centroids, counts, offsets, members, P, N, nc, seg, head_rows, normalize,
+                                stream);
+}
+
+extern "C" int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P,
+                                      int N, int nc, ri_stream_t stream) {
+  if (!assign || !counts || !offsets || !members) return RI_ERR_ARG;
+  int rc = km_check(P, N, nc);
+  if (rc) return rc;
+  if (N > KM_DIRECT_MAX) return RI_ERR_ARG;
+  return km_direct_launch<false>(nullptr, assign, nullptr, counts, offsets, members, P, N, nc, 1, N, 0, stream);
 }
 
 extern "C" int ri_kmeans_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts,

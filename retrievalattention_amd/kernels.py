@@ -594,6 +594,12 @@ def kmeans_update_direct(data, assign, centroids, P, N, nc, seg, head_rows, norm
                                                      _stream()), "kmeans_update_direct")
 
 
+def kmeans_lists_direct(assign, counts, offsets, members, P, N, nc):
+    """The lists alone, for at most KMEANS_DIRECT_MAX_TOKENS tokens per problem."""
+    check(lib().ri_kmeans_lists_direct(_p(assign), _p(counts), _p(offsets), _p(members), P, N, nc, _stream()),
+          "kmeans_lists_direct")
+
+
 def _rows_ok(t):
     return t.stride(-1) == 1 and t.stride(-2) % 8 == 0 and t.stride(-3) % 8 == 0 and t.data_ptr() % 16 == 0
 

@@ -44,6 +44,10 @@ def test_prefill_passes(dev, dtype, H, N, nc, fused):
     assign = assign.to(dev)
     counts, offsets, members = (torch.empty(s, dtype=torch.int32, device=dev) for s in ((H, nc), (H, nc + 1), (H, N)))
     kernels.kmeans_build_lists(assign, counts, offsets, members, H, N, nc)
+    if N <= kernels.KMEANS_DIRECT_MAX_TOKENS:
+        lists = [torch.full_like(t, -1) for t in (counts, offsets, members)]
+        kernels.kmeans_lists_direct(assign, *lists, H, N, nc)
+        assert all(torch.equal(a, b) for a, b in zip(lists, (counts, offsets, members)))
     sums, ref_sums = (torch.empty((H, nc, 128), dtype=dtype, device=dev) for _ in range(2))
     store, store_k = (torch.zeros((H, N + 7, 128), dtype=dtype, device=dev) for _ in range(2))
     kernels.kmeans_value_sum(hv.contiguous(), counts, offsets, members, ref_sums, H, N, nc)
