@@ -104,11 +104,13 @@ def test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt):
     cent[:, 4:nc:8] = cent[:, 0:nc - 4:8]
     cent[:, 33:nc:64] = cent[:, 1:nc - 32:64]
     cent[:, nc - 1] = cent[:, 2]
+    cent[:, nc // 2 + 1] = float("nan")      # scores that are no number never win, and a token without others gets 0
+    data[0, N // 2] = float("nan")
     assign = torch.full((P, N), -1, dtype=torch.int32, device=dev)
     kernels.kmeans_assign(data, cent, assign, P, N, nc, 1, N)
     ids = torch.arange(nc, device=dev)
     for p in range(P):
-        s = data[p].double() @ cent[p].double().T
+        s = (data[p].double() @ cent[p].double().T).nan_to_num(nan=-1e9)
         first = torch.where(s == s.max(dim=1, keepdim=True)[0], ids, nc).amin(dim=1)
         assert torch.equal(assign[p].long(), first)
 
