@@ -967,7 +967,9 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   // One compute unit reads about 20 KB per microsecond, whatever it reads.  Its own scoring therefore pays up to 512
   // clusters (128 KB of centroids: 10.2 us against 10.9 for two launches; 1024 clusters: 15.7 against 11.0), its own
   // score sums up to about 112 KB of logits (8 groups of 4 heads, 4096 clusters: 14.4 against 15.5 us; 32 groups of
-  // 4 heads, 8192 clusters: 26.7 against 26.1).
+  // 4 heads, 8192 clusters: 26.7 against 26.1).  Past 4096 clusters a thread holds eight of them: with more than four
+  // heads that is 64 logits in registers, and many compute units are the faster ones again (4 .. 32 groups of 5 and 6
+  // heads, 4104 .. 5728 clusters: 16.1 .. 22.6 us with dist_kernel, 20.0 .. 26.2 without).
   if (nc <= 512) {
     if (nc <= 256) launch_select_heads<256, 1, SEL_SCORE>(P, BG, half, s);
     else launch_select_heads<512, 1, SEL_SCORE>(P, BG, half, s);
@@ -976,12 +978,12 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   }
   int rc = ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, scale, half, s);
   if (rc) return rc;
-  if (nc * gs <= 28 * 1024 && nc <= 8192 && np <= SEL_THREADS) {
+  if (nc * gs <= 28 * 1024 && nc <= (gs <= 4 ? 8192 : 4096) && np <= SEL_THREADS) {
     // as few waves as the clusters and the probes leave room for: what a wave does once costs all of them
     if (nc <= 1024 && np <= 512) launch_select_heads<512, 2, SEL_LOGITS>(P, BG, half, s);
     else if (nc <= 2048 && np <= 512) launch_select_heads<512, 4, SEL_LOGITS>(P, BG, half, s);
     else if (nc <= 4096) launch_select_heads<SEL_THREADS, 4, SEL_LOGITS>(P, BG, half, s);
-    else launch_select<SEL_THREADS, 8, 4, SEL_LOGITS>(P, BG, half, s);   // gs <= 3 here: 7 K logits per head at most
+    else launch_select<SEL_THREADS, 8, 4, SEL_LOGITS>(P, BG, half, s);   // gs <= 4 here, the heads this one holds
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }

@@ -355,3 +355,12 @@ def test_score_select_all_scores_equal(dev, nc, gs):
                          None, nprobe, es, 8, 16, 1.0)
     assert torch.equal(ret.cpu(), torch.arange(nprobe, dtype=torch.int32).expand(2, -1))
     assert torch.equal(est.cpu(), torch.arange(nprobe, nprobe + es, dtype=torch.int32).expand(2, -1))
+
+
+@pytest.mark.parametrize("gs", [5, 6])
+@pytest.mark.parametrize("nc", [4104, 4768, 4776, 5728, 5736])
+def test_score_select_every_head_counts(dev, gs, nc):
+    """More than four heads past 4096 clusters, on both sides of 28 K logits per group (5728 clusters of 5 heads, 4776 of
+    6): the selection must not make score sums here with the variant that holds four heads."""
+    test_score_select(dev, 2, gs, nc, nc // 56, nc // 4, 3100 + nc + gs)
+    test_score_select(dev, 2, gs, nc, nc // 56, nc // 4, 3200 + nc + gs, dt=torch.float16)
