@@ -81,9 +81,11 @@ __device__ __forceinline__ void chunk_update(WaveState<GS_PAD>& st, const float*
   for (int i = 0; i < NH; ++i) {
     const float s = valid ? sv[i] : -INFINITY;
     const float mn = fmaxf(st.m[i], ri_row_max(s));
-    // (no valid row so far: the maximum is -inf; exp(-inf) = 0 for the first chunk that has one)
-    al[i] = mn == -INFINITY ? 1.f : __expf(st.m[i] - mn);
-    const float p = valid ? __expf(s - mn) : 0.f;
+    // No finite score so far (no valid row, a head that does not exist, keys with infinite elements): relative to 0 such
+    // scores weigh exp(-inf) = 0, as the rows that are not valid always do; relative to -inf they would weigh NaN.
+    const bool none = mn == -INFINITY;
+    al[i] = none ? 1.f : __expf(st.m[i] - mn);
+    const float p = __expf(s - (none ? 0.f : mn));
     rescale |= (al[i] != 1.f);
     st.l[i] = st.l[i] * al[i] + w * p;
     st.m[i] = mn;

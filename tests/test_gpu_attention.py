@@ -345,3 +345,50 @@ def test_split_plan_edges(dev, gs, S):
     previous partials and ragged lengths."""
     test_weighted_flash_decoding(dev, 2, gs, S, True, True, True)
     test_weighted_flash_decoding(dev, 3, gs, S, False, False, False, dt=torch.float16)
+
+
+def _hide_rows(gen, S, runs):
+    """Row numbers of a group whose scores are to be -inf: the first rows of every 64 (the batch of a wave), whole batches,
+    and single rows; the last row stays."""
+    hidden = (torch.arange(S) % 64 < 16) | (torch.arange(S) // 64 % 3 == 1) if runs else torch.zeros(S, dtype=torch.bool)
+    hidden |= torch.rand(S, generator=gen) < 0.1
+    hidden[-1] = False
+    return hidden
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gs,S,runs", [(4, 40, True), (4, 1000, True), (7, 130, False), (8, 3001, True), (12, 640, True)])
+def test_infinite_key_elements(dev, gs, S, runs, dt):
+    """A key with an infinite element scores -inf for queries of the other sign: it has no weight, also where no finite
+    score has come before it."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(gs * S)
+    q, k, v = _rand((2, gs, 128), g, dt=dt), _rand((2, S, 128), g, dt=dt), _rand((2, S, 128), g, dt=dt)
+    q[:, :, 5] = q[:, :, 5].abs() + 0.5
+    for b in range(2):
+        k[b, _hide_rows(g, S, runs), 5] = float("-inf")
+    out, lse = kernels.weighted_flash_decoding(q.view(2, 1, gs, 128).to(dev), k.view(2, S, 1, 128).to(dev),
+                                               v.view(2, S, 1, 128).to(dev), return_softmax_lse=True)
+    ro, rl = attention.weighted_flash_decoding(q, k, v)
+    _close(out.cpu().view(2, gs, 128), ro)
+    assert torch.allclose(lse.cpu(), rl, atol=2e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gs,es", [(3, 200), (4, 1500), (16, 64)])
+def test_infinite_logits_of_the_estimation_zone(dev, gs, es, dt):
+    from retrievalattention_amd import kernels
+    BG, nc, n = 2, 2048, 48
+    g = torch.Generator().manual_seed(gs * es)
+    q, k, v = _rand((BG, gs, 128), g, dt=dt), _rand((BG, n, 128), g, dt=dt), _rand((BG, n, 128), g, dt=dt)
+    vsum, size = _rand((BG, nc, 128), g, 4.0, dt=dt), torch.randint(1, 33, (BG, nc), generator=g).to(dt)
+    logits = torch.randn(BG, gs, nc, generator=g)
+    ids = torch.stack([torch.randperm(nc, generator=g)[:es].sort().values for _ in range(BG)])
+    for b in range(BG):
+        logits[b][:, ids[b, _hide_rows(g, es, True)]] = float("-inf")
+    out = torch.empty(BG, gs, 128, dtype=dt, device=dev)
+    kernels.buffer_attention(q.to(dev), k.to(dev), v.to(dev), torch.full((BG,), n, dtype=torch.int32, device=dev),
+                             ids.to(torch.int32).to(dev), logits.to(dev), vsum.to(dev), size.to(dev), out, es,
+                             1 / math.sqrt(128))
+    eo, el = attention.estimation(logits, ids, vsum, size)
+    _close(out.cpu(), attention.weighted_flash_decoding(q, k, v, None, eo.to(dt), el.float())[0])
