@@ -184,7 +184,8 @@ int ri_weighted_flash_decoding_f16(const void* q, const void* k, const void* v, 
  *   [0, steady_stride]) and static_len only sizes the split: a captured launch then stays valid while
  *   the steady zone grows token by token
  *   store_k/v  [BG, store_stride, 128]: cluster-contiguous K/V
- *   row_src [BG, row_src_stride]: store row of every retrieved token; or NULL with ret_tok_off
+ *   row_src [BG, row_src_stride]: store row of every retrieved token, a negative entry for none (padding: not
+ *   attended, nothing is read for it); or NULL with ret_tok_off
  *   [BG, np+1] and ret_start [BG, np]: rank r's tokens are the store rows ret_start[r] + i
  *   meta, est_ids, logits: as written by ri_score_select (or meta by ri_lru_access_update)
  *   est_centroids [BG, nc, 128] bf16: given instead of logits (exactly one of the two is NULL when
@@ -225,7 +226,8 @@ int ri_wave_attention_f16(const void* q, const void* steady_k, const void* stead
 /* One part of a wave attention over a row table (host-resident store, block cache managed on the device;
  * cache_hub/retroinfer_cache.py:629-674, where the reference overlaps the transfer of missed blocks with
  * other work on its copy stream): as ri_wave_attention with row_src, but of the table's rows only those
- * whose source row lies in [src_row_lo, src_row_hi) are attended (the window may be empty: a block cache of
+ * whose source row lies in [src_row_lo, src_row_hi) are attended; an entry outside the window need not be a row
+ * of the store at all (the window may be empty: a block cache of
  * zero blocks has no cached rows).  (prev_out [BG, gs, 128] bf16, prev_lse
  * [BG, gs] fp32), both or neither, is an earlier part's result that is merged in (log-sum-exp rule);
  * lse_out [BG, gs] fp32 or NULL receives this part's log-sum-exp.  static_len = 0 leaves the steady zone

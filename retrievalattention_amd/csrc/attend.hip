@@ -46,8 +46,9 @@ struct AttendParams {
   int64_t strideB;
   const int32_t* row_src;
   int rs_stride;
-  // with a row table: only rows whose source row lies in [src_lo, src_hi) are attended, the others are
-  // skipped like padding rows (a second launch takes them, merging this one's result as its previous one)
+  // with a row table: only rows whose source row lies in [src_lo, src_hi), src_lo >= 0, are attended; the others are
+  // skipped like padding rows (a second launch takes them, merging this one's result as its previous one).  Their entries
+  // may be anything: row 0 is read in their place.
   int src_lo, src_hi;
   // or, without a row table: rank r of np clusters covers rows [ret_off[r], ret_off[r+1]) of region B,
   // stored contiguously from row ret_start[r] (ret_off has np + 1 entries, constant from the last kept rank on)
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams 
             d = sh_rst[lo] + rb - sh_roff[lo];
           } else {
             d = rs ? rs[rb] : rb;
-            if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d |= ATT_SKIP;
+            if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d = ATT_SKIP;   // row 0, not attended
           }
           if (wB) w = ri_e16_to_f32<HALF>(wB[rb]);
           if (wsrc) w = ri_e16_to_f32<HALF>(wsrc[d]);
@@ -677,12 +678,13 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   P.strideA = steady_stride;
   P.lenA = static_len;
   P.lenA_ptr = static_len_dev;
-  P.kB = (const uint16_t*)store_k;
-  P.vB = (const uint16_t*)store_v;
+  // (a store without rows: its table has only entries that are skipped, and the row read for them is the query's)
+  P.kB = (const uint16_t*)(store_stride > 0 ? store_k : q);
+  P.vB = (const uint16_t*)(store_stride > 0 ? store_v : q);
   P.strideB = store_stride;
   P.row_src = row_src;
   P.rs_stride = row_src_stride;
-  P.src_lo = src_lo;
+  P.src_lo = max(src_lo, 0);   // an entry below 0 is padding in every window
   P.src_hi = src_hi;
   P.prev_out = (const uint16_t*)prev_out;
   P.prev_lse = prev_lse;

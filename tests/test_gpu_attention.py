@@ -392,3 +392,46 @@ def test_infinite_logits_of_the_estimation_zone(dev, gs, es, dt):
                              1 / math.sqrt(128))
     eo, el = attention.estimation(logits, ids, vsum, size)
     _close(out.cpu(), attention.weighted_flash_decoding(q, k, v, None, eo.to(dt), el.float())[0])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gs,n", [(4, 40), (3, 700), (8, 2100)])
+def test_row_table_entries_that_are_no_rows(dev, gs, n, dt):
+    """A negative entry of a row table is padding, and so is whatever lies outside the row window of a part: neither is
+    attended and neither is taken for an address."""
+    from types import SimpleNamespace
+    from retrievalattention_amd import kernels
+    BG, ntok, nc = 2, 3000, 8
+    g = torch.Generator().manual_seed(gs * n)
+    q, steady = _rand((BG, gs, 128), g, dt=dt), _rand((BG, 9, 128), g, dt=dt)
+    k, v = _rand((BG, ntok, 128), g, dt=dt), _rand((BG, ntok, 128), g, dt=dt)
+    rows = torch.randint(0, ntok, (BG, n), generator=g, dtype=torch.int32)
+    kind = torch.randint(0, 6, (BG, n), generator=g)
+    kind[:, :33] = 0   # two whole chunks and one row more
+    none = {0: -1, 1: -2 ** 31, 2: -2 ** 30 - 7}
+    beyond = {3: 2 ** 31 - 1, 4: ntok + 2 ** 20}
+    table, window = rows.clone(), rows.clone()
+    for i, x in list(none.items()) + list(beyond.items()):
+        window[kind == i] = x
+        if i in none:
+            table[kind == i] = x
+    meta = torch.tensor([[1, n, 0, 0]] * BG, dtype=torch.int32, device=dev)
+    vsum, size = torch.zeros(BG, nc, 128, dtype=dt, device=dev), torch.ones(BG, nc, dtype=dt, device=dev)
+    scale = 1 / math.sqrt(128)
+    qd, sd, kd, vd = (t.to(dev) for t in (q, steady, k, v))
+    out, part, empty = (torch.empty(BG, gs, 128, dtype=dt, device=dev) for _ in range(3))
+    vl = torch.empty(BG, dtype=torch.int32, device=dev)
+    kernels.wave_attention(qd, sd, sd, 9, kd, vd, table.to(dev), meta, None, None, vsum, size, out, vl, 0, scale)
+    kernels.wave_attention_part(qd, sd, sd, 9, kd, vd, window.to(dev), 0, ntok, meta, None, None, vsum, size, part, None,
+                                0, scale)
+    for got, keep in ((out, kind > 2), (part, kind > 4)):
+        for b in range(BG):
+            at = rows[b, keep[b]].long()
+            ref = attention.weighted_flash_decoding(q[b:b + 1], torch.cat((steady[b], k[b, at]))[None],
+                                                    torch.cat((steady[b], v[b, at]))[None])[0]
+            _close(got[b].cpu(), ref[0])
+    # a store without rows: every entry is skipped, the steady zone remains
+    hollow = [SimpleNamespace(shape=(BG, 0, 128), data_ptr=t.data_ptr) for t in (kd, vd)]
+    kernels.wave_attention_part(qd, sd, sd, 9, *hollow, window.to(dev), 0, 0, meta, None, None, vsum, size, empty, None, 0,
+                                scale)
+    _close(empty.cpu(), attention.weighted_flash_decoding(q, steady, steady)[0])
