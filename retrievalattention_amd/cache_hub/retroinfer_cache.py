@@ -488,9 +488,20 @@ class retroinfer_cache(KV_Cache):
         if self.fold_due():
             self._update_kv_cache()
 
+    def _require_room(self, layer_idx=0):
+        """Refuses a token for which the steady zone has no row left (more tokens than max_new_length announced, or a
+        fold that was due).  The position of a captured or indexed append is only known on the device, where it is
+        too late to refuse."""
+        rows = self.steady_zone_keys[layer_idx].shape[2]
+        if self.static_pattern_total >= rows:
+            raise IndexError(f"the steady zone is full: no row {self.static_pattern_total} for this token in a zone of "
+                             f"{rows} rows")
+
     def token_replayed(self):
         """Host-side bookkeeping for one token decoded by replaying captured steps (device_positions):
-        the replay advanced the device-side position, this advances the host counters."""
+        the replay advanced the device-side position, this advances the host counters.  Raises when the zone had no row
+        for that token: its K/V was not written."""
+        self._require_room()
         self.context += 1
         self.static_pattern_total += 1
 
@@ -515,6 +526,7 @@ class retroinfer_cache(KV_Cache):
             if not capturing:
                 self.prepare_token()
             if not self._append(key_states, value_states, layer_idx, self.steady_pos_dev):
+                self._require_room(layer_idx)
                 self.steady_zone_keys[layer_idx].index_copy_(2, self.steady_pos_dev, key_states.transpose(1, 2))
                 self.steady_zone_values[layer_idx].index_copy_(2, self.steady_pos_dev, value_states.transpose(1, 2))
             # (the device-side position moves on after the last layer's attention, in compute())
