@@ -507,11 +507,13 @@ class retroinfer_cache(KV_Cache):
 
     def _append(self, key_states, value_states, layer_idx, pos_dev=None):
         """The token's K and V rows into the steady zone with one launch; False when the rows are not as a layer hands
-        them over (another type, layout or shape, a full zone): torch's copies then convert, broadcast or raise."""
+        them over (another type, layout, shape or device, a full zone): torch's copies then convert, broadcast or
+        raise."""
         k, v = self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx]
         for row, zone in ((key_states, k), (value_states, v)):
-            if not (row.is_cuda and row.dtype == zone.dtype and row.shape == self._row_shape and row.is_contiguous()
-                    and zone.is_contiguous() and row.data_ptr() % 16 == 0):
+            if not (row.is_cuda and row.get_device() == zone.get_device() and row.dtype == zone.dtype
+                    and row.shape == self._row_shape and row.is_contiguous() and zone.is_contiguous()
+                    and row.data_ptr() % 16 == 0):
                 return False
         if self.static_pattern_total >= k.shape[2]:
             return False
@@ -601,10 +603,16 @@ class retroinfer_cache(KV_Cache):
         return self._compute_staged(queries, layer_idx, queries_next, static_len, buf, nbuf, search_here,
                                     search_next)
 
+    def _prepared_takes(self, queries, layer_idx):
+        """Whether a prepared call can read the queries where they are (otherwise the operators one by one, which
+        convert or raise)."""
+        return queries.is_cuda and queries.get_device() == self.centroids[layer_idx].get_device() and \
+            queries.dtype == self.dtype and queries.is_contiguous() and \
+            queries.numel() == self.batch_groups * self.group_size * self.head_dim and not kernels.PROFILER_RANGES
+
     def _compute_device(self, queries, layer_idx, static_len, buf):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
-        if queries.is_cuda and queries.dtype == self.dtype and queries.is_contiguous() and \
-                queries.numel() == BG * gs * D and not kernels.PROFILER_RANGES:
+        if self._prepared_takes(queries, layer_idx):
             out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
             self._plan(layer_idx, buf).run(queries, static_len, out)
             return out
@@ -696,9 +704,8 @@ class retroinfer_cache(KV_Cache):
                                search_next):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
         es = self.es_cluster_num
-        if search_here and not search_next and not self.overlap_miss_staging and not kernels.PROFILER_RANGES and \
-                queries.is_cuda and queries.dtype == self.dtype and queries.is_contiguous() and \
-                queries.numel() == BG * gs * D:
+        if search_here and not search_next and not self.overlap_miss_staging and \
+                self._prepared_takes(queries, layer_idx):
             out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
             self._host_plan(layer_idx, buf).run(queries, static_len, out)
             return out
