@@ -635,14 +635,16 @@ class retroinfer_cache(KV_Cache):
              self.logits, self.ret_ids[buf], self.est_ids[buf], self.ret_tok_off, self.ret_start, self.meta,
              self.steady_zone_keys[layer], self.steady_zone_values[layer], self.list_keys[layer],
              self.list_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
+        length = self.steady_len_dev if self.device_positions else None
         key = [x.data_ptr() for x in t]
-        key += (self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size)
+        key += (None if length is None else length.data_ptr(), self.nprobe, self.es_cluster_num, self.page_size,
+                self.buffer_size)
         plan = self._plans.get((layer, buf))
         if plan is None or not plan.valid(key):
             names = ("centroids", "mask", "cluster_size_i32", "cluster_start", "logits", "ret_ids", "est_ids",
                      "ret_tok_off", "ret_start", "meta", "steady_k", "steady_v", "store_k", "store_v", "value_sum",
                      "cluster_size", "valid_lengths")
-            tensors = dict(zip(names, t), static_len_dev=self.steady_len_dev if self.device_positions else None)
+            tensors = dict(zip(names, t), static_len_dev=length)
             plan = self._plans[(layer, buf)] = kernels.DecodeStepPlan(
                 key, self.dtype, tensors, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
                 self.RSQRT_DIM)
@@ -657,7 +659,8 @@ class retroinfer_cache(KV_Cache):
              self.cache_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
         other = (self.cluster_size_i32[layer], self.cluster_start[layer], row_src, self.list_keys[layer],
                  self.list_values[layer])
-        key = [x.data_ptr() for x in t] + [x.data_ptr() for x in other]
+        lists = self._lists(layer)
+        key = [x.data_ptr() for x in (*t, *other, *lists, *lru.state())]
         key += (lru, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size)
         plan = self._plans.get((layer, buf))
         if plan is None or not plan.valid(key):
@@ -665,7 +668,7 @@ class retroinfer_cache(KV_Cache):
                      "store_v", "value_sum", "cluster_size", "valid_lengths")
             plan = self._plans[(layer, buf)] = kernels.HostStepPlan(
                 key, self.dtype, dict(zip(names, t)), self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
-                self.RSQRT_DIM, lru, other[0], other[1], self._lists(layer), row_src, other[3], other[4],
+                self.RSQRT_DIM, lru, other[0], other[1], lists, row_src, other[3], other[4],
                 self.cache_size * self.page_size)
         return plan
 

@@ -525,6 +525,10 @@ class DeviceLru:
         self.free_count = torch.full((BG,), capacity, dtype=torch.int32, device=device)
         self.epoch = i32(BG)
 
+    def state(self):
+        """The tensors whose addresses a prepared call holds."""
+        return self.blk_off, self.stamp, self.order, self.blk_ids, self.free_list, self.free_count, self.epoch
+
     def set_sizes(self, sizes_i32):
         """sizes_i32 [BG, ncl]: recompute the block offsets (offsets of existing clusters do not move
         when clusters are appended)."""

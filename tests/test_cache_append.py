@@ -1,4 +1,5 @@
-"""The host side of appending a token to the steady zone (CPU): what is refused, and which rows take which way."""
+"""The host side of a decode step (CPU): which tokens the steady zone refuses, which tensors take which way, and when a
+prepared call is prepared again."""
 import pytest
 import torch
 
@@ -86,3 +87,49 @@ def test_native_calls_take_tensors_of_one_device(monkeypatch, row_device, zone_d
                     lambda: c._compute_host_in_place(q, 0, None, 69, 0, 1, True, False)):
         with pytest.raises(Taken, match="prepared" if native else "general"):
             compute()
+
+
+@pytest.mark.parametrize("residency", ["device", "host"])
+def test_prepared_call_follows_its_buffers(monkeypatch, residency):
+    """Replacing any buffer whose address a prepared call holds prepares it again, once."""
+    prepared = []
+
+    class Plan:
+        def __init__(self, key, *a):
+            self.key = key
+            prepared.append(self)
+
+        def valid(self, key):
+            return self.key == key
+
+    monkeypatch.setattr(kernels, "DecodeStepPlan", Plan)
+    monkeypatch.setattr(kernels, "HostStepPlan", Plan)
+    new = lambda: torch.zeros(4, dtype=torch.int32)
+    per_layer = ["centroids", "centroids_mask", "cluster_size_i32", "cluster_start", "value_sum", "cluster_size",
+                 "steady_zone_keys", "steady_zone_values", "list_keys", "list_values", "ret_ids", "est_ids", "valid_lengths"]
+    single = ["logits"]
+    if residency == "device":
+        single += ["ret_tok_off", "ret_start", "meta", "steady_len_dev"]
+    else:
+        per_layer += ["cache_keys", "cache_values", "hit_unit_idices", "hit_unit_sizes", "hit_unit_sizes_cumsum",
+                      "hit_num_units", "miss_unit_idices", "miss_unit_sizes", "miss_unit_sizes_cumsum", "miss_num_units",
+                      "update_buffer_indices", "update_unit_sizes", "update_cache_indices", "update_num_units"]
+    c = _cache(monkeypatch, 70, 69, device_positions=residency == "device", _plans={}, nprobe=2, es_cluster_num=3,
+               page_size=8, buffer_size=16, cache_size=1, dtype=torch.bfloat16, use_cluster_estimation=False, RSQRT_DIM=1.0)
+    c.__dict__.update({n: [new()] for n in per_layer}, **{n: new() for n in single})
+    c.layouts = [[new() for _ in range(4)]]
+    lru = kernels.DeviceLru(2, 8, 16, 4, 4, 8, "cpu")
+    c.device_lru = [lru]
+    plan = c._plan if residency == "device" else c._host_plan
+    replace = [lambda n=n: setattr(c, n, [new()]) for n in per_layer] + [lambda n=n: setattr(c, n, new()) for n in single]
+    if residency == "host":
+        replace += [lambda i=i: c.layouts[0].__setitem__(i, new()) for i in (2, 3)]
+        replace += [lambda n=n: setattr(lru, n, getattr(lru, n).clone())
+                    for n in ("blk_off", "stamp", "order", "blk_ids", "free_list", "free_count", "epoch")]
+    keep = [plan(0, 0)]
+    for i, move in enumerate(replace):
+        held = {**c.__dict__, **lru.__dict__, "layouts": list(c.layouts[0])}   # (the old buffers keep their addresses)
+        keep.append(held)
+        move()
+        assert plan(0, 0) is prepared[-1] and plan(0, 0) is prepared[-1]
+        assert len(prepared) == i + 2, i
