@@ -73,7 +73,7 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_me
     return r
 
 
-# Captured clusterings, newest last: (key pointer, shape, parameters) -> (graph, result).  A clustering is
+# Captured clusterings, newest last: (key pointer, type, shape, parameters) -> (graph, result).  A clustering is
 # about a hundred short launches; replayed as one HIP graph it loses the gaps between them.  The graph
 # reads the key tensor afresh on every replay, so only the address has to stay the same, not the content.
 _GRAPHS = collections.OrderedDict()
@@ -91,8 +91,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
     key_rows, the [G, N, 128] keys before key_mean was subtracted.
 
-    reuse_graph (off unless asked for): the second call with keys at the same address and the same
-    shape and parameters captures the launches into a HIP graph, and later such calls replay it.
+    reuse_graph (off unless asked for): the second call with keys at the same address and of the same
+    type, shape and parameters captures the launches into a HIP graph, and later such calls replay it.
     Results of replayed calls live in the graph's own memory: THEY ARE OVERWRITTEN by the next replay
     for the same key tensor, so only a caller that consumes or copies them before its next call may
     turn this on (prefill_update_kv_cache does: it copies everything into the cache's tensors at once;
@@ -109,7 +109,7 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
         raise AssertionError("centroids per segment must be a multiple of 32")  # kmeans.py:99
     r = None
     if reuse_graph and not torch.cuda.is_current_stream_capturing():
-        gkey = (key.data_ptr(), tuple(key.shape), str(key.device), nc, num_iters, S, key_store is None,
+        gkey = (key.data_ptr(), key.dtype, tuple(key.shape), str(key.device), nc, num_iters, S, key_store is None,
                 None if init_indices is None else init_indices.data_ptr())
         hit = _GRAPHS.get(gkey)
         if hit is None and gkey in _SEEN:
