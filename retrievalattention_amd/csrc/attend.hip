@@ -249,8 +249,9 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams 
   __shared__ float sh_al[NW][16];
   __shared__ float sh_m[NW][GS_PAD];
   __shared__ float sh_l[NW][GS_PAD];
-  // the waves' numerators for the merge: up to eight heads they are laid over the wave's own value tile (dead
-  // once its rows are done), which keeps a four-wave workgroup under 40 KB of LDS (four per compute unit)
+  // the waves' numerators for the merge: up to eight heads they are laid over the wave's own value tile (dead once its
+  // rows are done), which keeps a workgroup at 48 KB of LDS, so that the two its registers leave room for fit a compute
+  // unit (sixteen heads: 116 KB, one workgroup)
   constexpr bool ACC_OVER_VT = GS_PAD * RI_DIM * sizeof(float) <= 16 * ATT_VT_STRIDE * sizeof(uint16_t);
   __shared__ float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
   auto acc_of = [&](int w) -> float* {
@@ -572,7 +573,10 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 // Split plan of a launch: workgroups per group, and the waves of a group that take key/value rows, shared with the
 // estimation rows in proportion to the memory traffic of a row, es_row_bytes against the 512 bytes of a K and a V row.
 //  * One workgroup of eight waves per compute unit: 64 groups of 8 heads over 16384 clusters 54.7 us, two per unit or
-//    three of four waves 55.3 .. 60 us; 11 groups, 29000 rows: 38.0 against 41.9 .. 45.
+//    three of four waves 55.3 .. 60 us; 11 groups, 29000 rows: 38.0 against 41.9 .. 45.  256 / BG rounds down, which
+//    leaves units without work between 86 and 255 groups (4 heads over 8192 clusters: 100 groups 33.8 us, 128: 42.0, 160:
+//    58.6, 200: 67.0, 256: 88.8), and is still ahead of the two or more workgroups of four waves per group that it
+//    replaced (42.4, 46.7, 78.7, 86.8, 101.8 us).
 //  * A compute unit reads about 25 KB per microsecond, so more workgroups stream a group's rows faster, but the last
 //    one to arrive reads the partials of all of them at that same rate: the sum of both is least near
 //    sqrt(bytes of the group / bytes of a partial), flat towards fewer (12 groups of 7 heads, 3550 rows: 15 workgroups
