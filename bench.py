@@ -575,7 +575,8 @@ def bench_host(args, cfg, cache, queries, L, nprobe, es, static_len, config_name
         "value": B / (cfg["L"] * t_warm), "unit": "tokens/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": t_warm * 1e3, "us_per_layer_step": t_warm * 1e6, "cold_us_per_layer_step": t_cold * 1e6,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": DT_NAME, "data": "synthetic",
-        "config": {"workload": f"{args.config}: {cfg['desc']}; clustered K/V in pinned host memory, block cache of "
+        "config": {"workload": f"{config_name or args.config}: {cfg['desc'].replace(' (device-resident variant)', '')}; "
+                               f"clustered K/V in pinned host memory, block cache of "
                                f"{cache.cache_size if hasattr(cache, 'cache_size') else '?'} blocks per group, "
                                f"block cache manager on the {cache.block_cache}, miss staging "
                                f"{'beside' if cache.overlap_miss_staging else 'before'} the attention, nprobe {nprobe}, "
