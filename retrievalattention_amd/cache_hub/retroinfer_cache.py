@@ -510,13 +510,14 @@ class retroinfer_cache(KV_Cache):
         them over (another type, layout, shape or device, a full zone): torch's copies then convert, broadcast or
         raise."""
         k, v = self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx]
+        device = k.get_device()
+        if device < 0 or self.static_pattern_total >= k.shape[2]:
+            return False
         for row, zone in ((key_states, k), (value_states, v)):
-            if not (row.is_cuda and row.get_device() == zone.get_device() and row.dtype == zone.dtype
+            if not (row.get_device() == device and zone.get_device() == device and row.dtype == zone.dtype
                     and row.shape == self._row_shape and row.is_contiguous() and zone.is_contiguous()
                     and row.data_ptr() % 16 == 0):
                 return False
-        if self.static_pattern_total >= k.shape[2]:
-            return False
         kernels.append_kv(key_states, value_states, k, v, self.static_pattern_total, pos_dev)
         return True
 
@@ -606,14 +607,14 @@ class retroinfer_cache(KV_Cache):
     def _prepared_takes(self, queries, layer_idx):
         """Whether a prepared call can read the queries where they are (otherwise the operators one by one, which
         convert or raise)."""
-        return queries.is_cuda and queries.get_device() == self.centroids[layer_idx].get_device() and \
-            queries.dtype == self.dtype and queries.is_contiguous() and \
-            queries.numel() == self.batch_groups * self.group_size * self.head_dim and not kernels.PROFILER_RANGES
+        return queries.get_device() == self.centroids[layer_idx].get_device() and queries.dtype == self.dtype and \
+            queries.is_contiguous() and not kernels.PROFILER_RANGES and \
+            queries.numel() == self.batch_groups * self.group_size * self.head_dim
 
     def _compute_device(self, queries, layer_idx, static_len, buf):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
         if self._prepared_takes(queries, layer_idx):
-            out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
+            out = queries.new_empty((self.batch_size, 1, self.num_heads, D))
             self._plan(layer_idx, buf).run(queries, static_len, out)
             return out
         self._select(queries, layer_idx, buf, True)
@@ -709,7 +710,7 @@ class retroinfer_cache(KV_Cache):
         es = self.es_cluster_num
         if search_here and not search_next and not self.overlap_miss_staging and \
                 self._prepared_takes(queries, layer_idx):
-            out = torch.empty((self.batch_size, 1, self.num_heads, D), dtype=self.dtype, device=queries.device)
+            out = queries.new_empty((self.batch_size, 1, self.num_heads, D))
             self._host_plan(layer_idx, buf).run(queries, static_len, out)
             return out
         q = queries.view(BG, gs, D)

@@ -54,6 +54,9 @@ class _OnDevice:
     def data_ptr(self):
         return 256
 
+    def new_empty(self, shape):
+        return torch.empty(shape, dtype=self.dtype)
+
     def numel(self):
         return self.shape.numel()
 
