@@ -83,10 +83,10 @@ class retroinfer_cache(KV_Cache):
         # host-resident store with the device-side manager: attend the rows already in the block cache
         # (with the steady and estimation zones) while the missed blocks are still crossing the host link
         # on the copy stream, then the staged rows (reference: retroinfer_cache.py:629-657 overlaps that
-        # transfer with other work of the step).  Off by default: the attention over the hits is ~30 us
+        # transfer with other work of the step).  Off by default: the attention over the hits is ~15 us
         # of a step whose miss staging takes hundreds, and the second launch and the stream join cost
-        # more than the overlap returns (measured at B=8, 8 KV heads, 120K tokens: 287 vs 270 us per
-        # layer-step at 70 % hits, 93 vs 66 us with every block a hit)
+        # more than the overlap returns (measured at B=16, 4 KV heads, 60K tokens: 269 vs 243 us per
+        # layer-step at 69 % hits, 74 vs 54 us with every block a hit)
         self.overlap_miss_staging = bool(overlap_miss_staging)
         # the reference's NVTX ranges (retroinfer_cache.py:558-678) as roctx ranges of the same names
         self.profiler_ranges = bool(profiler_ranges)
