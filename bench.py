@@ -257,7 +257,7 @@ def kmeans_cpu_baseline(cfg, iters=10):
                       f"{t_seg + t_glob:.1f} s of CPU work",
             "extrapolation": f"{Hkv} heads x ({S} segments x segment sweep + {N // sample} x final-pass sample): linear "
                              f"in tokens, segments and heads",
-            "note": "the checker's restatement (float64 scores, numpy), not a tuned CPU implementation"}
+            "note": "the oracle's restatement (float64 scores, numpy), not a tuned CPU implementation"}
 
 
 def cpu_baseline(cache, cfg, queries, nprobe, es, static_len, max_seconds=10.0, max_samples=100, min_samples=3):
@@ -554,7 +554,7 @@ def bench_host(args, cfg, cache, queries, L, nprobe, es, static_len, config_name
         cpu = {"value": B / (cfg["L"] * t_cpu), "unit": "tokens/s", "us_per_layer_step": t_cpu * 1e6,
                "cores": torch.get_num_threads(), "kind": "port",
                "sample": f"median of {n} full-shape decode layer-steps of layer 0 (oracle/pipeline.py)",
-               "note": "the checker's restatement, not a tuned CPU implementation: float64 matrix products and a "
+               "note": "the oracle's restatement, not a tuned CPU implementation: float64 matrix products and a "
                        "Python loop over the groups",
                "max_abs_vs_gpu": float(d.max()), "mean_abs_vs_gpu": float(d.mean())}
     link = max((v["host_link_GBps"] for v in drift.values()), default=0.0)
@@ -830,7 +830,7 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
                                   "cores": torch.get_num_threads(), "kind": "port",
                                   "sample": f"median of {n} full-shape decode layer-steps of layer 0 (oracle/pipeline.py)" +
                                             (", about 10 s of CPU work" if extras else ""),
-                                  "note": "the checker's restatement, not a tuned CPU implementation: float64 matrix "
+                                  "note": "the oracle's restatement, not a tuned CPU implementation: float64 matrix "
                                           "products and a Python loop over the groups",
                                   "max_abs_vs_gpu": float(d.max()), "mean_abs_vs_gpu": float(d.mean())}
     return result

@@ -1,7 +1,7 @@
 """CPU restatement of RetroInfer's wave-index path (reference: wennitao/RetrievalAttention).
 
 TEST INFRASTRUCTURE ONLY.  Nothing under this package is part of the product: it is the
-checker that tests/, __graft_entry__.smoke() and the cpu_baseline leg of bench.py compare the
+oracle that tests/, __graft_entry__.smoke() and the cpu_baseline leg of bench.py compare the
 HIP kernels against.  The product (retrievalattention_amd/) never imports it.
 
 Every function cites the reference file:line it follows.  The 16-bit element type (bfloat16 or IEEE

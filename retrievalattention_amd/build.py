@@ -18,7 +18,7 @@ CPP_SOURCES = ["wavebuf.cpp"]
 ARCH = "gfx950"
 # -ffp-contract=off: products and sums round separately unless the source says fmaf, which
 # keeps the k-means reductions reproducible on a CPU.  The packed-fp32 feature is disabled
-# because some of its instruction forms have been unreliable on this hardware pool.
+# because some of its instruction forms have been unreliable on this hardware.
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 # per-file additions: the k-means assignment reads every MFMA accumulator in its argmax
