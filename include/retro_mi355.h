@@ -579,11 +579,28 @@ int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_s
    ri_prefill_split: keys[h][i] = key[first + i][h] for i < N, and the steady zone of both tensors: rows 0..n_start-1
    of every head from tokens start0.., the following n_end from tokens end0..  Strides in elements, multiples of 8.
    ri_prefill_center: keys[h][i] -= mean[h], in the element type.
+   ri_prefill_mean: mean[h] = the mean of key[first .. first + N - 1][h], summed in fp32 in a fixed order and rounded once:
+   the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144 tokens, and 2 GiB of them together; beyond that
+   ri_prefill_mean_workspace_bytes is 0 and the call refuses.
+   ri_prefill_split_centred: ri_prefill_split with mean[h] taken off the rows of keys, as ri_prefill_center does.
    ri_prefill_index: out = centroids + mean, mask = (count == 0), sizes as elements and as int32, first rows. */
 int ri_prefill_split(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
                      int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
                      int end0, int n_end, int H, void* keys, void* steady_k, void* steady_v, int64_t steady_stride,
                      ri_stream_t stream);
+int ri_prefill_split_centred(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                             int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
+                             int end0, int n_end, int H, const void* mean, void* keys, void* steady_k, void* steady_v,
+                             int64_t steady_stride, ri_stream_t stream);
+int ri_prefill_split_centred_f16(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                                 int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0,
+                                 int n_start, int end0, int n_end, int H, const void* mean, void* keys, void* steady_k,
+                                 void* steady_v, int64_t steady_stride, ri_stream_t stream);
+size_t ri_prefill_mean_workspace_bytes(int H, int N);
+int ri_prefill_mean(const void* key, int64_t key_row_stride, int64_t key_head_stride, int first, int N, int H, void* mean,
+                    void* workspace, size_t workspace_bytes, ri_stream_t stream);
+int ri_prefill_mean_f16(const void* key, int64_t key_row_stride, int64_t key_head_stride, int first, int N, int H,
+                        void* mean, void* workspace, size_t workspace_bytes, ri_stream_t stream);
 int ri_prefill_center(void* keys, const void* mean, int H, int N, ri_stream_t stream);
 int ri_prefill_center_f16(void* keys, const void* mean, int H, int N, ri_stream_t stream);
 int ri_prefill_index(const void* centroids, const void* mean, const int32_t* counts, const int32_t* offsets, void* out,

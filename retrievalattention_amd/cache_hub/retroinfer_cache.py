@@ -351,10 +351,13 @@ class retroinfer_cache(KV_Cache):
                 self._centred_keys.clear()
             ck = torch.empty((H, valid_length, head_dim), dtype=keys.dtype, device=keys.device)
             self._centred_keys[(dkey, valid_length)] = ck
+        mean_key = kernels.prefill_mean(keys, lo, valid_length)
         kernels.prefill_split(keys, values, lo, valid_length, vs, sps, seq_len - spe, spe, ck,
-                              self.steady_zone_keys[layer_idx][batch_idx], self.steady_zone_values[layer_idx][batch_idx])
-        mean_key = torch.mean(ck, dim=1, keepdim=True)
-        kernels.prefill_center(ck, mean_key)
+                              self.steady_zone_keys[layer_idx][batch_idx], self.steady_zone_values[layer_idx][batch_idx],
+                              mean_key)
+        if mean_key is None:
+            mean_key = torch.mean(ck, dim=1, keepdim=True)
+            kernels.prefill_center(ck, mean_key)
 
         # cluster-contiguous store built on the device (stands in for organize_kv on the host) while the last sums
         # are taken; clusters in id order, tokens ascending inside

@@ -654,8 +654,25 @@ def permute_rows_strided(src, members, dst, P, N, out_stride_rows):
           "permute_rows")
 
 
-def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, steady_k, steady_v):
-    """keys/values [T, H, 128]; out [H, N, 128]; steady_k/v [H, rows, 128]."""
+def prefill_mean(keys, first, N):
+    """Mean [H, 1, 128] of keys[first:first + N] ([T, H, 128]) per head, the bits of torch.mean over the heads' own rows;
+    None for shapes the kernel does not take."""
+    H = keys.shape[1]
+    nbytes = lib().ri_prefill_mean_workspace_bytes(H, N)
+    if nbytes == 0:
+        return None
+    kr, kh = _row_strides(keys, "prefill_mean")
+    if first + N > keys.shape[0]:
+        raise ValueError("prefill_mean: rows outside the sequence")
+    mean = torch.empty((H, 1, 128), dtype=keys.dtype, device=keys.device)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=keys.device)
+    check(_fn("ri_prefill_mean", keys.dtype)(_p(keys), kr, kh, first, N, H, _p(mean), _p(ws), nbytes, _stream()),
+          "prefill_mean")
+    return mean
+
+
+def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, steady_k, steady_v, mean=None):
+    """keys/values [T, H, 128]; out [H, N, 128], less mean [H, 1, 128] where given; steady_k/v [H, rows, 128]."""
     kr, kh = _row_strides(keys, "prefill_split")
     vr, vh = _row_strides(values, "prefill_split")
     T, H = keys.shape[0], keys.shape[1]
@@ -663,8 +680,12 @@ def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, ste
         raise ValueError("prefill_split: rows outside the sequence")
     if not keys.dtype == values.dtype == out.dtype == steady_k.dtype == steady_v.dtype:
         raise TypeError("prefill_split: keys, values and the cache must have the same element type")
-    check(lib().ri_prefill_split(_p(keys), _p(values), kr, kh, vr, vh, first, N, start0, n_start, end0, n_end, H, _p(out),
-                                 _p(steady_k), _p(steady_v), steady_k.stride(0) // 128, _stream()), "prefill_split")
+    lead = (_p(keys), _p(values), kr, kh, vr, vh, first, N, start0, n_start, end0, n_end, H)
+    tail = (_p(out), _p(steady_k), _p(steady_v), steady_k.stride(0) // 128, _stream())
+    if mean is None:
+        check(lib().ri_prefill_split(*lead, *tail), "prefill_split")
+    else:
+        check(_fn("ri_prefill_split_centred", keys.dtype)(*lead, _p(mean), *tail), "prefill_split")
 
 
 def prefill_center(keys, mean):

@@ -72,3 +72,33 @@ def test_prefill_passes(dev, dtype, H, N, nc, fused):
     kernels.prefill_index(cent, mean, counts, offsets, out, mask, size16, size, start)
     assert torch.equal(out, cent + mean) and torch.equal(mask, counts == 0) and torch.equal(size16, counts.to(dtype))
     assert torch.equal(size, counts) and torch.equal(start, offsets[:, :nc])
+
+
+# where the order of the sum changes (one part, four, eight, sixteen ...; one head has a rule of its own), and around it
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N", [(1, 1), (1, 1020), (1, 1021), (1, 8193), (1, 16384), (1, 16385), (1, 40007), (2, 3),
+                                 (2, 510), (3, 511), (8, 4094), (5, 4095), (4, 32752), (2, 32753), (8, 65504), (2, 65505),
+                                 (32, 2049), (1, 262144), (2, 131009), (2, 262144)])
+def test_prefill_mean(dev, dtype, H, N):
+    from retrievalattention_amd import kernels
+    g = torch.Generator(device=dev).manual_seed(H + N)
+    vs, sps, spe = 5, 3, 17
+    T = vs + sps + N + spe
+    kv = torch.randn(T, 2, H, 128, generator=g, device=dev)
+    kv = ((kv + 0.1) * torch.where(torch.arange(128, device=dev) < 4, 8.0, 1.0)).to(dtype)
+    K, V = (kv[:, 0], kv[:, 1]) if N % 2 else (kv[:, 0].contiguous(), kv[:, 1].contiguous())
+    lo = vs + sps
+    ck, ref = (torch.empty((H, N, 128), dtype=dtype, device=dev) for _ in range(2))
+    zones = [torch.zeros((H, sps + spe, 128), dtype=dtype, device=dev) for _ in range(4)]
+    kernels.prefill_split(K, V, lo, N, vs, sps, lo + N, spe, ref, *zones[:2])
+    mean = kernels.prefill_mean(K, lo, N)
+    assert torch.equal(mean, torch.mean(ref, dim=1, keepdim=True))
+    kernels.prefill_center(ref, mean)
+    kernels.prefill_split(K, V, lo, N, vs, sps, lo + N, spe, ck, *zones[2:], mean)
+    assert torch.equal(ck, ref) and torch.equal(zones[0], zones[2]) and torch.equal(zones[1], zones[3])
+
+
+def test_prefill_mean_leaves_other_shapes(dev):
+    from retrievalattention_amd import kernels
+    assert kernels.prefill_mean(torch.empty((40, 33, 128), dtype=torch.bfloat16, device=dev), 0, 40) is None
+    assert kernels.prefill_mean(torch.empty((262145, 1, 128), dtype=torch.bfloat16, device=dev), 0, 262145) is None
