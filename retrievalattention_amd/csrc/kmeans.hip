@@ -9,11 +9,11 @@ typedef __attribute__((address_space(3))) void* km_lds_ptr;
 typedef const __attribute__((address_space(1))) void* km_glb_ptr;
 
 // 16 bytes per lane from global memory straight into LDS: lane l lands at lds_base + 16 l
-// (lds_base: byte address inside the workgroup's LDS, the same in every lane).  The wait for the
-// data is the caller's (s_waitcnt vmcnt): issued as inline assembly so that LDS reads of other
+// (lds_base: byte address inside the workgroup's LDS, the same in every lane, as `base` is; `at`: the lane's byte offset).
+// The wait for the data is the caller's (s_waitcnt vmcnt): issued as inline assembly so that LDS reads of other
 // buffers are not made to wait for it.
-__device__ __forceinline__ void km_lds_dma16(const void* g, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds_base) : "memory", "m0");
+__device__ __forceinline__ void km_lds_dma16(const void* base, uint32_t at, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(at), "s"(base), "s"(lds_base) : "memory", "m0");
 }
 
 // first data row of problem p: problems are `seg` consecutive N-row slices of each head
@@ -35,24 +35,56 @@ __device__ __forceinline__ size_t km_row0(int p, int seg, int64_t head_rows, int
 template <int V>
 __device__ __forceinline__ void km_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory"); }
 
-// One step of three searches for m: i0, i1, i2 become I0, I1, I2 where those scores equal it.  The hardware wants two
-// instructions between a comparison and the select that reads its mask; in one chain of fifteen, which the compiler makes
-// of every way to write this, they are idle (62 issue slots per search, 31 here).  With one or two token columns per wave
-// that delays the next products (8 x 8192 tokens, 512 centroids: 12.3 -> 11.7 us; 24 x 8119, 512: 30.0 -> 29.0; 4 x
-// 9000, 288: 8.05 -> 7.61); with three or four they are the other columns' and nothing changes (8 x 32768, 2048: 112.8
-// and 113 us), or the three more registers cost (16 x 8200, 512: 24.8 and 25.9), so the chain stays there.
-// (The scores have been read by the maximum before: no matrix result is outstanding when this runs.)
-template <int I0, int I1, int I2>
-__device__ __forceinline__ void km_first_of(const f32x16_t& x, float m, int& i0, int& i1, int& i2) {
-  uint64_t e0, e1, e2;
-  asm("v_cmp_eq_f32_e64 %3, %6, %9\n\t"
-      "v_cmp_eq_f32_e64 %4, %7, %9\n\t"
-      "v_cmp_eq_f32_e64 %5, %8, %9\n\t"
-      "v_cndmask_b32_e64 %0, %0, %10, %3\n\t"
-      "v_cndmask_b32_e64 %1, %1, %11, %4\n\t"
-      "v_cndmask_b32_e64 %2, %2, %12, %5"
-      : "+v"(i0), "+v"(i1), "+v"(i2), "=&s"(e0), "=&s"(e1), "=&s"(e2)
-      : "v"(x[I0]), "v"(x[I1]), "v"(x[I2]), "v"(m), "n"(I0), "n"(I1), "n"(I2));
+// base + the row, past the lane's first one in a sub-tile, of the first of a lane's sixteen scores that equals m: the half
+// that holds m is selected, then its half, down to one score.  low8 and low4 are the maxima of best and the first eight
+// and four scores, high4 of best and scores 8 .. 11; m is above best in every lane whose answer counts.  26 instructions,
+// of which four compare; comparing and selecting one score after the other takes 30, and leaves two slots idle between
+// each comparison and the select that reads its mask.  Written out because the compiler turns a select between two scores
+// into a search by index.  (The hardware wants two slots between a comparison and a select that reads it.  The scores have
+// been read by the maxima before: no matrix result is outstanding when this runs.)
+__device__ __forceinline__ int km_first_of(const f32x16_t& x, float m, float best, float low8, float low4, float high4,
+                                           int base) {
+  float y0, y1, y2, y3, y4, y5, y6, y7, t;
+  uint64_t e, e8;
+  int row;
+  asm volatile(
+      "v_cmp_eq_f32_e64 %8, %25, %26\n\t"
+      "s_nop 1\n\t"
+      "v_cndmask_b32_e64 %0, %17, %9, %8\n\t"
+      "v_cndmask_b32_e64 %1, %18, %10, %8\n\t"
+      "v_cndmask_b32_e64 %2, %19, %11, %8\n\t"
+      "v_cndmask_b32_e64 %3, %20, %12, %8\n\t"
+      "v_cndmask_b32_e64 %4, %21, %13, %8\n\t"
+      "v_cndmask_b32_e64 %5, %22, %14, %8\n\t"
+      "v_cndmask_b32_e64 %6, %23, %15, %8\n\t"
+      "v_cndmask_b32_e64 %7, %24, %16, %8"
+      : "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7), "=&s"(e8)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]),
+        "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(low8), "v"(m));
+  // (accumulator i is row (i / 4) * 8 + i % 4)
+  asm volatile(
+      "v_cndmask_b32_e64 %8, %13, %12, %10\n\t"
+      "v_cmp_eq_f32_e64 %11, %8, %15\n\t"
+      "v_cndmask_b32_e64 %9, 16, 0, %10\n\t"
+      "s_nop 0\n\t"
+      "v_cndmask_b32_e64 %0, %4, %0, %11\n\t"
+      "v_cndmask_b32_e64 %1, %5, %1, %11\n\t"
+      "v_cndmask_b32_e64 %2, %6, %2, %11\n\t"
+      "v_cndmask_b32_e64 %3, %7, %3, %11\n\t"
+      "v_max3_f32 %8, %14, %0, %1\n\t"
+      "v_cmp_eq_f32_e64 %10, %8, %15\n\t"
+      "v_cndmask_b32_e64 %4, 8, 0, %11\n\t"
+      "s_nop 0\n\t"
+      "v_cndmask_b32_e64 %0, %2, %0, %10\n\t"
+      "v_cmp_eq_f32_e64 %11, %0, %15\n\t"
+      "v_cndmask_b32_e64 %5, 2, 0, %10\n\t"
+      "v_add3_u32 %9, %9, %4, %5\n\t"
+      "v_cndmask_b32_e64 %6, 1, 0, %11\n\t"
+      "v_add3_u32 %9, %9, %6, %16"
+      : "+v"(y0), "+v"(y1), "+v"(y2), "+v"(y3), "+v"(y4), "+v"(y5), "+v"(y6), "+v"(y7), "=&v"(t), "=&v"(row), "+s"(e8),
+        "=&s"(e)
+      : "v"(low4), "v"(high4), "v"(best), "v"(m), "v"(base));
+  return row;
 }
 
 template <int KM_TT, int KM_CT, int KM_W, int KM_NB, bool HALF>
@@ -65,7 +97,7 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
   constexpr int L = KM_CT / 4 / KM_W;   // loads of a wave per tile
   __shared__ __attribute__((aligned(1024))) uint16_t sh_c[KM_NB][KM_CT][RI_DIM];
   const int p = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, hh = lane >> 5;
   const int t0 = blockIdx.x * KM_WG_TOKENS + wave * (32 * KM_TT);
   const uint16_t* dp = data + km_row0(p, seg, head_rows, N) * RI_DIM;
@@ -75,15 +107,17 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
   // per wave instruction: lane l lands at byte l * 16 of the instruction's LDS window, and which
   // global piece it fetches is free, so the 16-byte pieces of row w are stored at piece ^ (w & 15):
   // the 16 lanes of a ds_read_b128 phase then hit 16 different piece positions (all 64 banks once).
-  const int ld_row = lane >> 4, ld_piece = lane & 15;
+  // (A wave's rows start at the same place of sixteen in every instruction, so a lane's offset never changes and the rest
+  // of the address is scalar.)
+  static_assert(KM_W % 4 == 0, "an instruction's first row modulo 16 is the wave's");
+  const uint32_t ld_at = (lane >> 4) * (RI_DIM * 2) + (((lane & 15) ^ ((wave * 4 + (lane >> 4)) & 15)) * 16);
   const uint32_t sh_base = (uint32_t)(uintptr_t)(km_lds_ptr)&sh_c[0][0][0];
   auto tile_load = [&](int ct, int buf) {
 #pragma unroll
     for (int u = 0; u < L; ++u) {
       const int row4 = (wave + u * KM_W) * 4;      // first of the four rows of this instruction
-      const int row = min(ct + row4, nc - 4) + ld_row;   // (rows past the last repeat it: the count of loads is fixed)
-      const uint16_t* g = cp + (size_t)row * RI_DIM + ((ld_piece ^ ((row4 + ld_row) & 15)) * 8);
-      km_lds_dma16(g, __builtin_amdgcn_readfirstlane(sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2)));
+      const int row = min(ct + row4, nc - 4);      // (rows past the last repeat it: the count of loads is fixed)
+      km_lds_dma16(cp + (size_t)row * RI_DIM, ld_at, sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2));
     }
   };
   uint4 b[KM_TT][8];
@@ -111,63 +145,60 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
     best[tt] = -INFINITY;
     bidx[tt] = 0;
   }
-  int buf = 0;
-  for (int ct = 0; ct < nc; ct += KM_CT) {
-    km_wait_vm<(KM_NB - 2) * L>();   // this tile's loads of this wave have landed ...
-    asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
-    tile_load(ct + (KM_NB - 1) * KM_CT, buf == 0 ? KM_NB - 1 : buf - 1);
+  const uint16_t* row_at[8];   // this lane's pieces of its row of a sub-tile
 #pragma unroll
-    for (int half = 0; half < KM_CT / 32; ++half) {
-      if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
-        f32x16_t acc[KM_TT];
+  for (int kk = 0; kk < 8; ++kk) row_at[kk] = &sh_c[0][r][((kk * 2 + hh) ^ (r & 15)) * 8];
+  for (int ct0 = 0; ct0 < nc; ct0 += KM_NB * KM_CT) {
 #pragma unroll
-        for (int tt = 0; tt < KM_TT; ++tt)
+    for (int buf = 0; buf < KM_NB; ++buf) {   // (unrolled: the buffer is in the offset of every LDS read)
+      const int ct = ct0 + buf * KM_CT;
+      if (ct >= nc) break;
+      km_wait_vm<(KM_NB - 2) * L>();   // this tile's loads of this wave have landed ...
+      asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
+      tile_load(ct + (KM_NB - 1) * KM_CT, buf == 0 ? KM_NB - 1 : buf - 1);
 #pragma unroll
-          for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          const uint4 a = *reinterpret_cast<const uint4*>(&sh_c[buf][half * 32 + r][((kk * 2 + hh) ^ (r & 15)) * 8]);
+      for (int half = 0; half < KM_CT / 32; ++half) {
+        if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
+          f32x16_t acc[KM_TT];
 #pragma unroll
           for (int tt = 0; tt < KM_TT; ++tt)
-            acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
-                                                                    __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
-                           : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
-                                                                     0, 0);
-        }
-        // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
-        // equal to their maximum is the lowest row; the index search only runs when some lane
-        // of the wave improves on its best (about half of the sub-tiles of a full-size pass)
 #pragma unroll
-        for (int tt = 0; tt < KM_TT; ++tt) {
-          // (from the best so far, which is no NaN: eight instructions; from the first score the compiler makes it ten.
-          // 4 x 48719 tokens, 3072 centroids 120.5 -> 119.3 us, 128 x 8192, 512 133.7 -> 132.8, in half 138.8 -> 135.9)
-          float m = best[tt];
+            for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) m = fmaxf(m, acc[tt][i]);
-          const bool upd = m > best[tt];
-          if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
-            int sel = 15;
-            if constexpr (KM_TT <= 2) {
-              int s1 = 15, s2 = 15;
-              km_first_of<4, 9, 14>(acc[tt], m, sel, s1, s2);
-              km_first_of<3, 8, 13>(acc[tt], m, sel, s1, s2);
-              km_first_of<2, 7, 12>(acc[tt], m, sel, s1, s2);
-              km_first_of<1, 6, 11>(acc[tt], m, sel, s1, s2);
-              km_first_of<0, 5, 10>(acc[tt], m, sel, s1, s2);
-              sel = min(min(sel, s1), s2);
-            } else {
+          for (int kk = 0; kk < 8; ++kk) {
+            const uint4 a = *reinterpret_cast<const uint4*>(row_at[kk] + (buf * KM_CT + half * 32) * RI_DIM);
 #pragma unroll
-              for (int i = 14; i >= 0; --i) sel = (acc[tt][i] == m) ? i : sel;
+            for (int tt = 0; tt < KM_TT; ++tt)
+              acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                                      __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
+                             : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
+                                                                       0, 0);
+          }
+          // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
+          // equal to their maximum is the lowest row; the index search only runs when some lane
+          // of the wave improves on its best (about half of the sub-tiles of a full-size pass)
+#pragma unroll
+          for (int tt = 0; tt < KM_TT; ++tt) {
+            // (both halves from the best so far, which is no NaN: nine instructions)
+            float low8 = best[tt], high8 = best[tt], low4 = best[tt], high4 = best[tt];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              low8 = fmaxf(low8, acc[tt][i]);
+              high8 = fmaxf(high8, acc[tt][8 + i]);
+              if (i == 3) low4 = low8, high4 = high8;
             }
-            if (upd) {
+            float m;
+            asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(low8), "v"(high8));   // (no NaN: the compiler would quiet one first)
+            const bool upd = m > best[tt];
+            if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+              const int at = km_first_of(acc[tt], m, best[tt], low8, low4, high4, hh * 4 + ct + half * 32);
+              bidx[tt] = upd ? at : bidx[tt];
               best[tt] = m;
-              bidx[tt] = ct + half * 32 + (sel >> 2) * 8 + hh * 4 + (sel & 3);
             }
           }
         }
       }
     }
-    buf = buf + 1 == KM_NB ? 0 : buf + 1;
   }
   km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's)
 #pragma unroll
@@ -1062,22 +1093,24 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   const long long wgs768 = (long long)P * ((N + 767) / 768);
   const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
   // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
-  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
-  // against 18.9 with two columns; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
+  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 10.9 us
+  // against 18.9 with two columns at the time; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
   if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
   else if (wgs256 <= 512) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
   // One workgroup per compute unit that gives each wave three or four columns, where the fullest unit has that many
   // columns per wave to do anyway: the same work with more reuse of every LDS read (16 x 8200 tokens, 512 centroids: 25.8
-  // us against 28.7 for the last line's; 4 x 48719, 3072: 124 against 135; 20 x 9757, 608: 37.8 against 40.4).
+  // us against 28.7 for the last line's when they were compared; 4 x 48719, 3072: 124 against 135; 20 x 9757, 608: 37.8
+  // against 40.4; now 23.1, 119.6 and 34.8).
   else if (nc >= 512 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
   else if (nc >= 512 && wgs256 > 768 && wgs1024 <= 256) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
   // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
-  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves; 4 x 65536, 4096: 219 against
-  // 232), provided the last round of these large workgroups is not mostly empty.
+  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves, now 1532; 4 x 65536, 4096: 219
+  // against 232, now 202), provided the last round of these large workgroups is not mostly empty.
   else if (nc > 1024 && wgs1024 * 100 >= rounds1024 * 256 * 87) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
   // Otherwise the load of the tokens in front of the loop is a large part of the kernel, and 126 registers and 32 KB of
   // LDS let four workgroups per compute unit overlap one's loads with the others' products (128 x 8192 tokens, 512
-  // centroids: 132 us; 137 with two buffers, 137 with four columns and tiles of 128).
+  // centroids: 114.8 us, four columns and tiles of 128: 140.5, of 32: 119.7, eight waves 118.3, three buffers 114.5, tiles
+  // of 64 116.3 and 124.9, three columns 131).
   else KM_ASSIGN_LAUNCH(2, 32, 4, 4);
 #undef KM_ASSIGN_LAUNCH
   RI_HIP_CHECK_LAUNCH();

@@ -115,6 +115,29 @@ def test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt):
         assert torch.equal(assign[p].long(), first)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("P,N,nc", [(5, 1001, 32), (8, 8193, 544), (16, 8200, 544), (20, 9757, 608), (33, 8200, 512),
+                                    (2, 32768, 2048)])
+def test_assign_finds_every_row(dev, P, N, nc, dt):
+    """Scores that are exact (tokens that pick out one dimension of the centroids), with the maximum in every row of a
+    sub-tile, with ties, with centroids that are no numbers (never chosen) and infinities: the first of the largest."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(nc + N)
+    cent = torch.randint(-9, 10, (P, nc, 128), generator=g).float()
+    dim = torch.randint(0, 128, (P, N), generator=g)
+    cent[:, :, 64:] = torch.randint(-2, 1, (P, nc, 64), generator=g).float()     # ties everywhere
+    cent[:, torch.arange(64) % nc, torch.arange(64)] = 20.                       # row c is the best of dimension c
+    cent[1, 7] = float("nan")
+    cent[0, :, 100] = -float("inf")      # (0 * inf is no number either: every other token of the problem has none)
+    keys = torch.zeros(P, N, 128).scatter_(2, dim[..., None], 1.0)
+    got = torch.full((P, N), -1, dtype=torch.int32, device=dev)
+    kernels.kmeans_assign(keys.to(dt).to(dev), cent.to(dt).to(dev), got, P, N, nc, 1, N)
+    score = torch.gather(cent.transpose(1, 2), 1, dim[..., None].expand(P, N, nc))
+    score[0] = -float("inf")
+    score = torch.nan_to_num(score, nan=-float("inf"), neginf=-float("inf"))
+    assert np.array_equal(got.cpu().numpy(), score.numpy().argmax(axis=2))
+
+
 @pytest.mark.parametrize("P,N,nc,seed", [(3, 1000, 64, 10), (2, 8192, 512, 11), (1, 4100, 1024, 12), (4, 37, 32, 13)])
 def test_assign_update_valuesum_float16(dev, P, N, nc, seed):
     """IEEE half keys, values and centroids (the reference's harnesses default to fp16, simple_test.py:29):
