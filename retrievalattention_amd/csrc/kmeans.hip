@@ -21,8 +21,18 @@ __device__ __forceinline__ size_t km_row0(int p, int seg, int64_t head_rows, int
   return (size_t)(p / seg) * (size_t)head_rows + (size_t)(p % seg) * (size_t)N;
 }
 
+// Workgroups go to the eight chiplets in turn, each with an L2 of its own.  A launch over P problems of T workgroups each
+// has the grid (T << sh, P >> sh), problem p = (y << sh) + x % (1 << sh), with 1 << sh the largest power of two up to eight
+// that divides P: up to eight problems run beside each other, each on its own chiplets, and what the workgroups of a
+// problem share (its centroids, its assignment) is fetched by as few of them as can be.  Nine iterations of 8 x 8192
+// tokens, 512 centroids: 244 -> 216 us (with eight heads of 8192 tokens the keys, too, stay in the L2 of their chiplet from
+// pass to pass), of 24 x 8119 420 -> 404, of 128 x 8192 1552 -> 1516, of 4 x 8120 184 -> 177; 17 x 7000 314 and 313 (an odd
+// P runs as before).
+static int km_together(int P) { return P % 8 == 0 ? 3 : P % 4 == 0 ? 2 : P % 2 == 0 ? 1 : 0; }
+static dim3 km_grid(int T, int P) { return dim3((unsigned)T << km_together(P), P >> km_together(P)); }
+
 // ------------------------------------------------------------------------------------
-// assign: grid (ceil(N / (KM_W * 32 * KM_TT)), P), KM_W waves; a wave keeps KM_TT columns of 32
+// assign: grid km_grid(ceil(N / (KM_W * 32 * KM_TT)), P), KM_W waves; a wave keeps KM_TT columns of 32
 // tokens in registers for the whole kernel (KM_TT independent accumulator chains).  Centroid
 // tiles of KM_CT rows go through KM_NB LDS buffers shared by all waves of the workgroup: a tile
 // is requested from global memory straight into its buffer (no registers, no LDS
@@ -91,15 +101,15 @@ template <int KM_TT, int KM_CT, int KM_W, int KM_NB, bool HALF>
 __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __restrict__ data,
                                                               const uint16_t* __restrict__ cent,
                                                               int32_t* __restrict__ assign, int N, int nc,
-                                                              int seg, int64_t head_rows) {
+                                                              int seg, int64_t head_rows, int sh) {
   static_assert(KM_CT % (4 * KM_W) == 0 && KM_CT % 32 == 0, "a tile is whole 1 KiB wave loads and whole sub-tiles");
   constexpr int KM_WG_TOKENS = KM_W * 32 * KM_TT;
   constexpr int L = KM_CT / 4 / KM_W;   // loads of a wave per tile
   __shared__ __attribute__((aligned(1024))) uint16_t sh_c[KM_NB][KM_CT][RI_DIM];
-  const int p = blockIdx.y;
+  const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, hh = lane >> 5;
-  const int t0 = blockIdx.x * KM_WG_TOKENS + wave * (32 * KM_TT);
+  const int t0 = (blockIdx.x >> sh) * KM_WG_TOKENS + wave * (32 * KM_TT);
   const uint16_t* dp = data + km_row0(p, seg, head_rows, N) * RI_DIM;
   const uint16_t* cp = cent + (size_t)p * nc * RI_DIM;
 
@@ -818,7 +828,7 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 // ------------------------------------------------------------------------------------
 // update straight from the assignment, for problems of at most KM_DIRECT_MAX tokens (the segments of the segmented
 // iterations): list sort, list-ordered sums and means in one launch, no lists in memory.
-// grid (ceil(nc / CPW), P), eight waves: a workgroup owns CPW consecutive clusters.  Every wave takes a contiguous run of
+// grid km_grid(ceil(nc / CPW), P), eight waves: a workgroup owns CPW consecutive clusters.  Every wave takes a contiguous run of
 // the problem's tokens, compacts those of the workgroup's clusters into LDS (in token order), counts them, and after a
 // scan in (cluster, wave) order scatters them to the workgroup's list in LDS, ranking equal clusters inside a round of 64
 // with ballots: the stable order of the list kernels, hence the same sums.  Then a wave sums whole clusters of at most
@@ -880,13 +890,13 @@ template <bool HALF, int CPW>
 __global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
     const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int seg,
-    int64_t head_rows, int normalize) {
+    int64_t head_rows, int normalize, int sh) {
   constexpr int NW = KM_DIRECT_WAVES, SLOTS = CPW * NW;
   static_assert(SLOTS <= NW * 64, "one (cluster, wave) counter per thread");
   __shared__ int32_t sh_run[NW][CPW], sh_off[CPW + 1], sh_w[NW], sh_below[NW];
   extern __shared__ __attribute__((aligned(16))) uint32_t sh_buf[];   // rounds * 512 words: compacted tokens, later block sums
   // (last problem first: its keys are what the assignment pass has just left in the memory-side cache)
-  const int p = gridDim.y - 1 - blockIdx.y, c0 = blockIdx.x * CPW;
+  const int p = ((gridDim.y - 1 - blockIdx.y) << sh) + (blockIdx.x & ((1 << sh) - 1)), c0 = (blockIdx.x >> sh) * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rounds = (N + NW * 64 - 1) / (NW * 64);   // 64-token rounds per wave
   uint32_t* const mine = sh_buf + wave * rounds * 64;
@@ -1087,8 +1097,8 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
   if (rc) return rc;
 #define KM_ASSIGN_LAUNCH(TT, CT, W, NB)                                                                                  \
-  km_assign_kernel<TT, CT, W, NB, HALF><<<dim3((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, (hipStream_t)stream>>>( \
-      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows)
+  km_assign_kernel<TT, CT, W, NB, HALF><<<km_grid((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, (hipStream_t)stream>>>( \
+      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P))
   const long long wgs128 = (long long)P * ((N + 127) / 128), wgs256 = (long long)P * ((N + 255) / 256);
   const long long wgs768 = (long long)P * ((N + 767) / 768);
   const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
@@ -1249,9 +1259,9 @@ static int km_direct_launch(const void* data, const int32_t* assign, void* centr
   const size_t lds = (size_t)rounds * KM_DIRECT_WAVES * 64 * 6 + 512;
 #define KM_DIRECT_LAUNCH(CPW)                                                                                         \
   do {                                                                                                                \
-    km_direct_kernel<HALF, CPW><<<dim3((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>(   \
+    km_direct_kernel<HALF, CPW><<<km_grid((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>( \
         (const uint16_t*)data, assign, (uint16_t*)centroids, counts, offsets, members, N, nc, seg, head_rows,         \
-        normalize);                                                                                                   \
+        normalize, km_together(P));                                                                                                   \
   } while (0)
   // As many workgroups as are resident at once (four of 512 threads, as many as the LDS of a compute unit holds): more
   // of them read the assignments more often and wait for a second round (24 x 8119 tokens, 512 clusters each: 8
