@@ -603,12 +603,7 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
                                             uint32_t mean = 0u) {
   static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
-  const auto add = [&](uint32_t w) {
-    float x0, x1;
-    ri_unpack2<HALF>(w, x0, x1);
-    s0 += x0;
-    s1 += x1;
-  };
+  const auto add = [&](uint32_t w) { ri_add2<HALF>(w, s0, s1); };
   const auto term = [&](uint32_t w) { return CENTER ? ri_sub2<HALF>(w, mean) : w; };
   for (int k = k0; k < k1; k += U) {
     const int n = min(U, k1 - k);
@@ -843,51 +838,77 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 #define KM_DIRECT_MAX 16384
 
 #define KM_DIRECT_SHORT 128   // longer lists are summed in blocks and folded, as lists of several blocks are
-// Rows k0 .. k1-1 of a list in LDS added in list order, U per round: ids come with one LDS read and are broadcast from the
-// lanes as buffer offsets, the loads of a round (in eights; a short last eight repeats its last row, and adds +0 for it,
-// which changes no sum) are all in flight before the first add.  A wave's own chain bounds a list: two instructions fetch
-// a row and two per dim add it (an address per row in 64 bits, and a select per row, made it ten; 8 x 8192 tokens, 512
-// clusters: 10.6 -> 9.6 us; 128 x 8192: 67.6 -> 61.6).  WHOLE: two dims per lane, else one (two waves share the row).
+// Rows k0 .. k1-1 of a list in LDS added in list order, U in flight: ids come with one LDS read per U and are broadcast
+// from the lanes as buffer offsets; a row's register takes the row U further on as soon as it is added (in eights; past the
+// last row that is repeated, and +0 is added for it, which changes no sum).  A wave's own chain bounds a list: two
+// instructions fetch a row and two per dim add it, one in half (an address per row in 64 bits, and a select per row, made
+// it ten; 8 x 8192 tokens, 512 clusters: 10.6 -> 9.6 us; 128 x 8192: 67.6 -> 61.6).  Requests beside the additions instead
+// of U rows at a time, nine updates of Lloyd iterations together: 128 x 8192 tokens 543 -> 517 us (half 626 -> 512, where
+// 80 registers instead of 82 also make room for a third workgroup), 24 x 8119 183 -> 175 (216 -> 166), 8 x 8192 107 -> 104.
+// WHOLE: two dims per lane, else one (two waves share the row).
 template <bool HALF, int U, bool WHOLE>
 __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint32_t byte, const uint16_t* list, int k0, int k1,
                                               float& s0, float& s1) {
   static_assert(U <= 64 && U % 8 == 0, "an id per lane, rows in eights");
   const int lane = threadIdx.x & 63;
   const auto add = [&](uint32_t w) {
-    float x0, x1;
-    ri_unpack2<HALF>(w, x0, x1);
-    s0 += x0;
-    if (WHOLE) s1 += x1;
+    if (WHOLE) ri_add2<HALF>(w, s0, s1);
+    else ri_add_lo<HALF>(w, s0);
   };
-  for (int k = k0; k < k1; k += U) {
-    const int n = min(U, k1 - k);
-    const int off = (int)list[k + min(lane, n - 1)] * (RI_DIM * 2);
-    uint32_t v[U];
+  uint32_t v[U];
+  int off;
+  const auto ids = [&](int k) { off = (int)list[min(k + lane, k1 - 1)] * (RI_DIM * 2); };
+  const auto fetch = [&](int e) {
 #pragma unroll
-    for (int e = 0; e < U; e += 8)
-      if (e < n) {
+    for (int j = e; j < e + 8; ++j) {
+      const int so = __builtin_amdgcn_readlane(off, j);
+      v[j] = WHOLE ? __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so, 0)
+                   : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, byte, so, 0);
+    }
+  };
+  const auto add8 = [&](int e) {
 #pragma unroll
-        for (int j = e; j < e + 8; ++j) {
-          const int so = __builtin_amdgcn_readlane(off, j);
-          v[j] = WHOLE ? __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so, 0)
-                       : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, byte, so, 0);
-        }
-      }
+    for (int j = e; j < e + 8; ++j) add(v[j]);
+  };
+  const auto rest = [&](int k) {
 #pragma unroll
     for (int e = 0; e < U; e += 8) {
-      if (e + 8 <= n) {
+      if (k + e + 8 <= k1) {
+        add8(e);
+      } else if (k + e < k1) {
 #pragma unroll
-        for (int j = e; j < e + 8; ++j) add(v[j]);
-      } else if (e < n) {
-#pragma unroll
-        for (int j = e; j < e + 8; ++j) add(j < n ? v[j] : 0u);   // the word 0 is (+0, +0) in either type
+        for (int j = e; j < e + 8; ++j) add(k + j < k1 ? v[j] : 0u);   // the word 0 is (+0, +0) in either type
       }
     }
+  };
+  int k = k0;
+  ids(k);
+  if (k + U < k1) {
+#pragma unroll
+    for (int e = 0; e < U; e += 8) fetch(e);
+    // (no branch around a load here: the compiler counts the loads behind the ones it waits for, and takes those that may
+    // not have been made for not made)
+    do {
+      k += U;
+      ids(k);
+#pragma unroll
+      for (int e = 0; e < U; e += 8) {
+        add8(e);
+        fetch(e);
+        __builtin_amdgcn_sched_barrier(0);   // (else the next loads move up, into registers of their own)
+      }
+    } while (k + U < k1);
+    rest(k);
+  } else {
+#pragma unroll
+    for (int e = 0; e < U; e += 8)
+      if (k + e < k1) fetch(e);
+    rest(k);
   }
 }
 
 template <bool HALF, int CPW>
-__global__ __launch_bounds__(KM_DIRECT_WAVES * 64) void km_direct_kernel(
+__global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
     const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int seg,
     int64_t head_rows, int normalize, int sh) {

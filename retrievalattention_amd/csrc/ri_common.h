@@ -80,6 +80,19 @@ __device__ __forceinline__ void ri_unpack2(uint32_t w, float& lo, float& hi) {
     hi = __uint_as_float(w & 0xffff0000u);
   }
 }
+// s0 += the low element, s1 += the high one, each rounded once.  Halves as x * 1 + s, the same number: one instruction
+// where a conversion and an addition are two (the compiler makes the two of it).
+template <bool HALF>
+__device__ __forceinline__ void ri_add_lo(uint32_t w, float& s) {
+  if (HALF) asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(s) : "v"(w));
+  else s += __uint_as_float(w << 16);
+}
+template <bool HALF>
+__device__ __forceinline__ void ri_add2(uint32_t w, float& s0, float& s1) {
+  ri_add_lo<HALF>(w, s0);
+  if (HALF) asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s1) : "v"(w));
+  else s1 += __uint_as_float(w & 0xffff0000u);
+}
 // a - b on packed pairs: both operands widened, the differences rounded
 template <bool HALF>
 __device__ __forceinline__ uint32_t ri_sub2(uint32_t a, uint32_t b) {
