@@ -19,10 +19,11 @@
 // the one before, so a chain cannot be split: the rows in flight are what fills the link to memory).  Heads vary fastest:
 // workgroups next to each other read whole tokens.
 // mean_fold_kernel: a workgroup per head and 32 dims puts the chains together.
-// 8 heads of 8192 / 131072 tokens and 4 of 48719: 7.5 + 3, 69 + 4.6 and 20.6 + 4.6 us, where torch.mean took 54, 168 and
-// 157.  The long ones are bound by the rows (268 MB at 3.9 TB/s), the short ones by the rows in flight: there are only
-// H S waves.  And the mean is known before the heads are taken apart, so that pass centres them: 6.2 / 78 / 15.7 us for
-// both, where a copy (6.7 / 91 / 15.7) and a pass over it (12 / 77 / 16) were needed.
+// Chains and fold, 8 heads of 8192 / 131072 tokens and 4 of 48719: 8.3, 44 and 14.7 us, where torch.mean took 54, 168 and
+// 157 (with a branch around each of the loads 10.5, 73 and 25).  Bound by the rows where they are many (268 MB at 6.1
+// TB/s, some of it from the memory-side cache), else by the rows in flight: there are only H S waves.  And the mean is known
+// before the heads are taken apart, so that pass centres them: 6.2 / 78 / 15.7 us for both, where a copy (6.7 / 91 / 15.7)
+// and a pass over it (12 / 77 / 16) were needed.
 // ------------------------------------------------------------------------------------
 #define MEAN_DEEP 64
 #define MEAN_MAX_C 256
@@ -56,29 +57,37 @@ __global__ __launch_bounds__(64) void mean_chain_kernel(const uint32_t* __restri
       --left;
     }
   };
-  const auto add = [&](uint32_t w) {
-    float x0, x1;
-    ri_unpack2<HALF>(w, x0, x1);
-    s0 += x0;
-    s1 += x1;
-  };
+  const auto add = [&](int j) { ri_add2<HALF>(v[j], s0, s1); };
+  int i = 0;
+  if (n >= MEAN_DEEP) {
 #pragma unroll
-  for (int e = 0; e < MEAN_DEEP; e += 8)
-    if (e < n) fetch(e);
-  for (int i = 0; i < n; i += MEAN_DEEP) {
+    for (int e = 0; e < MEAN_DEEP; e += 8) fetch(e);
+    // (no branch around a load here: the compiler counts the loads behind the ones it waits for, and takes those that may
+    // not have been made for not made)
+    for (; i + 2 * MEAN_DEEP <= n; i += MEAN_DEEP)
+#pragma unroll
+      for (int e = 0; e < MEAN_DEEP; e += 8) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) add(j);
+        fetch(e);
+      }
+    i += MEAN_DEEP;
 #pragma unroll
     for (int e = 0; e < MEAN_DEEP; e += 8) {
-      if (i + e + 8 <= n) {
 #pragma unroll
-        for (int j = e; j < e + 8; ++j) add(v[j]);
-      } else {
-#pragma unroll
-        for (int j = e; j < e + 8; ++j)
-          if (i + j < n) add(v[j]);
-      }
-      if (i + MEAN_DEEP + e < n) fetch(e);
+      for (int j = e; j < e + 8; ++j) add(j);
+      if (i + e < n) fetch(e);
     }
+  } else {
+#pragma unroll
+    for (int e = 0; e < MEAN_DEEP; e += 8)
+      if (e < n) fetch(e);
   }
+#pragma unroll
+  for (int e = 0; e < MEAN_DEEP; e += 8)
+#pragma unroll
+    for (int j = e; j < e + 8; ++j)
+      if (i + j < n) add(j);
   chains[((size_t)h * S + r) * (RI_DIM / 2) + lane] = make_float2(s0, s1);
 }
 
