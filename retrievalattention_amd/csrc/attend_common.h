@@ -51,12 +51,6 @@ __device__ __forceinline__ float ri_row_sum(float x) {
   return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, true));
 }
 
-__device__ __forceinline__ void ri_wave_sync() {   // LDS written by this wave is read by this wave
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The value rows h, h+4, h+8, h+12 of a chunk (dims 8n..8n+7, as loaded) -> row-major 16 x 128 tile in LDS.
 __device__ __forceinline__ void chunk_values(const uint4 v[4], uint16_t* vt, int lane) {
   const int n = lane & 15, h = lane >> 4;

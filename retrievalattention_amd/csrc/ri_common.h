@@ -126,6 +126,34 @@ __host__ __device__ __forceinline__ uint32_t ri_bf16_sort_key(uint16_t b) {
   return (b & 0x8000u) ? (uint32_t)(~b & 0xffffu) : (uint32_t)(b | 0x8000u);
 }
 
+__device__ __forceinline__ void ri_wave_sync() {   // LDS written by this wave is read by this wave
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sixteen rows of 128 elements as operands of MFMA 16x16x32 (lane l: row l % 16, dims 32 kk + 8 (l / 16) ..).  They are
+// loaded four whole rows per instruction (lane l: piece l % 16 of row 4 i + l / 16) and turned in 4 KiB of the wave's LDS,
+// because a compute unit takes a cycle and more per row that sixteen neighbouring lanes of a load touch: rows per lane
+// stream 14.5 bytes per cycle from the L2, whole rows 43 to 56 (one workgroup, 128 .. 512 KB).  Scoring and selection of 8
+// groups of 4 heads and 512 clusters 10.2 -> 8.0 us, of 16 and 1024 11.6 -> 10.8, of 12 of 7 heads and 1856 13.5 -> 13.0;
+// where all compute units stream, memory bounds it (32 of 8192: 26).  The attention, whose rows are few per wave and in a
+// chain, gains nothing by it and loads its keys by lanes.  Piece p of row r lies at place p ^ r of its row: both accesses
+// hit all banks once.
+__device__ __forceinline__ void ri_rows_put(uint4* sh, const uint4 (&v)[4]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 4 * i + (lane >> 4);
+    sh[row * 16 + ((lane & 15) ^ row)] = v[i];
+  }
+}
+__device__ __forceinline__ void ri_rows_get(const uint4* sh, uint4 (&o)[4]) {
+  const int r = threadIdx.x & 15, h = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) o[kk] = sh[r * 16 + ((h + 4 * kk) ^ r)];
+}
+
 // Rows of bf16 matrices are read and written 16 bytes at a time: their base pointers must be
 // 16-byte aligned (a null pointer counts as aligned: optional arguments are checked elsewhere).
 static inline bool ri_misaligned16(const void* p) { return ((uintptr_t)p & 15u) != 0; }

@@ -46,9 +46,9 @@ __device__ __forceinline__ void score_body(
   uint4 a[TPW][4], bq[4];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
-    const uint16_t* p = cg + (size_t)min(c0 + t * 16 + r, nc - 1) * RI_DIM + h * 8;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) a[t][kk] = ri_ld16(p + kk * 32);
+    for (int i = 0; i < 4; ++i)
+      a[t][i] = ri_ld16(cg + (size_t)min(c0 + t * 16 + 4 * i + h, nc - 1) * RI_DIM + r * 8);
   }
   {
     const uint16_t* p = q + ((size_t)g * gs + min(r, gs - 1)) * RI_DIM + h * 8;
@@ -57,15 +57,21 @@ __device__ __forceinline__ void score_body(
   }
   __builtin_amdgcn_sched_barrier(0);   // every load is in flight before the first product
 
+  __shared__ __attribute__((aligned(16))) uint4 sh_rows[NWV][256];
   f32x4_t acc[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
+    uint4 at[4];
+    ri_rows_put(sh_rows[wave], a[t]);
+    ri_wave_sync();
+    ri_rows_get(sh_rows[wave], at);
+    ri_wave_sync();   // (a wave's LDS accesses happen in order: the next rows need not wait for these)
     acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
-      acc[t] = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a[t][kk]),
+      acc[t] = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, at[kk]),
                                                              __builtin_bit_cast(f16x8_t, bq[kk]), acc[t], 0, 0, 0)
-                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(a[t][kk]), ri_as_bf16x8(bq[kk]),
+                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(at[kk]), ri_as_bf16x8(bq[kk]),
                                                               acc[t], 0, 0, 0);
   }
 

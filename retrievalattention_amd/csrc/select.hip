@@ -555,6 +555,7 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(SelectArgs P) {
   __shared__ uint32_t sh_fine[2][64], sh_scan[3][16], sh_sel[4], sh_tot[3], sh_ret[NT];
   __shared__ __attribute__((aligned(16))) uint16_t sh_p[SRC == SEL_SCORE ? IDS * GSM : 8];
   __shared__ float sh_a[SRC == SEL_SCORE ? NW : 1][16], sh_b[SRC == SEL_SCORE ? NW : 1][16];
+  __shared__ __attribute__((aligned(16))) uint4 sh_rows[SRC == SEL_SCORE ? NW : 1][SRC == SEL_SCORE ? 256 : 1];
   const int g = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nc = P.nc, np = P.np, es = P.es, k2 = np + es, gs = P.gs;
@@ -593,9 +594,9 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(SelectArgs P) {
       // the last centroid and heads past gs read a valid row (never used)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const uint16_t* p = cg + (size_t)min(16 * (wave + NW * t) + r, nc - 1) * RI_DIM + h * 8;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) a[t][kk] = ri_ld16(p + kk * 32);
+        for (int i = 0; i < 4; ++i)
+          a[t][i] = ri_ld16(cg + (size_t)min(16 * (wave + NW * t) + 4 * i + h, nc - 1) * RI_DIM + r * 8);
       }
       {
         const uint16_t* p = P.q + ((size_t)g * gs + min(r, gs - 1)) * RI_DIM + h * 8;
@@ -606,12 +607,17 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(SelectArgs P) {
       f32x4_t acc[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
+        uint4 at[4];
+        ri_rows_put(sh_rows[wave], a[t]);
+        ri_wave_sync();
+        ri_rows_get(sh_rows[wave], at);
+        ri_wave_sync();   // (a wave's LDS accesses happen in order: the next rows need not wait for these)
         f32x4_t x = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
-          x = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a[t][kk]),
+          x = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, at[kk]),
                                                             __builtin_bit_cast(f16x8_t, bq[kk]), x, 0, 0, 0)
-                   : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(a[t][kk]), ri_as_bf16x8(bq[kk]), x, 0, 0, 0);
+                   : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(at[kk]), ri_as_bf16x8(bq[kk]), x, 0, 0, 0);
         acc[t] = x * P.scale;
       }
       // softmax statistics: every wave's maximum and sum relative to it, folded by every lane for its head
@@ -964,9 +970,10 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   const SelectArgs P = {keys, (const uint16_t*)q, (const uint16_t*)centroids, logits, tmax, tsum, mask,
                         cluster_size_i32, cluster_start, (uint16_t*)dist, cI, ret_ids, est_ids, ret_tok_off, ret_start,
                         row_src, meta, row_src_stride, gs, nc, ntiles, np, es, page, max_pages, scale};
-  // One compute unit reads about 20 KB per microsecond, whatever it reads.  Its own scoring therefore pays up to 512
-  // clusters (128 KB of centroids: 10.2 us against 10.9 for two launches; 1024 clusters: 15.7 against 11.0), its own
-  // score sums up to about 112 KB of logits (8 groups of 4 heads, 4096 clusters: 14.4 against 15.5 us; 32 groups of
+  // One compute unit reads 20 KB per microsecond from memory and up to 100 from its L2.  Its own scoring therefore pays up to
+  // 512 clusters (8 groups of 4 heads: 8.0 us; 640 clusters 10.3 against 10.0 for two launches, 16 groups of 1024 11.8
+  // against 10.7; for 128 groups of 8 heads it is still ahead there, 14.0 against 16.0, but not by what the rule would
+  // cost), its own score sums up to about 112 KB of logits (8 groups of 4 heads, 4096 clusters: 14.4 against 15.5 us; 32 groups of
   // 4 heads, 8192 clusters: 26.7 against 26.1).  Past 4096 clusters a thread holds eight of them: with more than four
   // heads that is 64 logits in registers, and many compute units are the faster ones again (4 .. 32 groups of 5 and 6
   // heads, 4104 .. 5728 clusters: 16.1 .. 22.6 us with dist_kernel, 20.0 .. 26.2 without).
