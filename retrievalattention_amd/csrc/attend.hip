@@ -27,496 +27,9 @@
 #include "attend_common.h"
 #include "ri_common.h"
 
-#define ATT_WAVES 8                // waves of a workgroup
-#define ATT_FLAG_A 0x40000000     // descriptor bit: row lives in region A
-#define ATT_SKIP (int)0x80000000  // descriptor bit (the sign): the row is read but not attended
-
-struct AttendParams {
-  const uint16_t* q;  // [BG, gs, 128]
-  // region A: rows [0, lenA) at kA/vA + (g*strideA + row)*128
-  const uint16_t* kA;
-  const uint16_t* vA;
-  int64_t strideA;
-  int lenA;
-  const int32_t* lenA_ptr;  // when given: lenA is read here at launch time (clamped to [0, strideA])
-  // region B: rows [0, lenB(g)) at kB/vB + (g*strideB + src(row))*128,
-  // src(row) = row_src ? row_src[g*rs_stride + row] : row
-  const uint16_t* kB;
-  const uint16_t* vB;
-  int64_t strideB;
-  const int32_t* row_src;
-  int rs_stride;
-  // with a row table: only rows whose source row lies in [src_lo, src_hi), src_lo >= 0, are attended; the others are
-  // skipped like padding rows (a second launch takes them, merging this one's result as its previous one).  Their entries
-  // may be anything: row 0 is read in their place.
-  int src_lo, src_hi;
-  // or, without a row table: rank r of np clusters covers rows [ret_off[r], ret_off[r+1]) of region B,
-  // stored contiguously from row ret_start[r] (ret_off has np + 1 entries, constant from the last kept rank on)
-  const int32_t* ret_off;
-  const int32_t* ret_start;
-  int np;
-  const int32_t* lenB_ptr;  // lenB(g) = lenB_ptr ? lenB_ptr[g*lenB_ptr_stride] : lenB_const
-  int lenB_ptr_stride;
-  int lenB_const;
-  const uint16_t* weightB;  // [BG, weight_stride] bf16 per region-B row, or null
-  int weight_stride;
-  // estimation rows
-  const int32_t* est_ids;     // [BG, es]
-  const float* logits;        // [BG, gs, nc] scores of the estimation rows, or null:
-  const uint16_t* est_cent;   // [BG, nc, 128] then the scores are computed here from the centroid rows
-  const uint16_t* value_sum;  // [BG, nc, 128]
-  const uint16_t* csize;      // [BG, nc] bf16
-  int nc;
-  int es;
-  // partials and the per-group arrival counters (zero between launches)
-  float* part_ml;   // [BG, S, GS_PAD, 2]
-  float* part_acc;  // [BG, S, GS_PAD, 128]
-  int* counters;    // [BG]
-  int S;     // workgroups per group
-  int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
-  int gs;
-  float scale;
-  // epilogue
-  const uint16_t* prev_out;  // [BG, gs, 128] or null
-  const float* prev_lse;     // [BG, gs] or null
-  uint16_t* out;             // [BG, gs, 128]
-  float* lse_out;            // [BG, gs] or null
-  int32_t* valid_lengths;    // [BG] or null: lenA + lenB(g)
-};
-
-// rows of a wave: the group's `total` rows are cut into `nwaves` runs of a multiple of 16 rows
-__device__ __forceinline__ void wave_rows(int total, int nwaves, int wid, int* r0, int* r1) {
-  int rpw = (total + nwaves - 1) / nwaves;
-  rpw = (rpw + 15) & ~15;
-  *r0 = min(total, wid * rpw);
-  *r1 = min(total, *r0 + rpw);
-}
-
-// The output rows of head j: A / L merged with an earlier part (its output po, its log-sum-exp pl) under the maximum M.
-// Lane l holds dims 2l and 2l + 1.
-template <bool HALF>
-__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, float M, float L, float A0, float A1) {
-  const int lane = threadIdx.x & 63;
-  const size_t o = (size_t)g * P.gs + j;
-  if (P.prev_lse) {
-    const float pl = P.prev_lse[o];
-    if (pl != -INFINITY) {  // an empty earlier part carries no weight, whatever its output holds
-      float p0, p1;
-      ri_unpack2<HALF>(*reinterpret_cast<const uint32_t*>(P.prev_out + o * RI_DIM + 2 * lane), p0, p1);
-      const float M2 = fmaxf(M, pl);
-      const float f = M == -INFINITY ? 0.f : __expf(M - M2), fp = __expf(pl - M2);
-      L = L * f + fp;
-      A0 = A0 * f + fp * p0;
-      A1 = A1 * f + fp * p1;
-      M = M2;
-    }
-  }
-  // nothing attended at all (an empty part): zeros and a log-sum-exp of -inf, not 0/0
-  const bool any = L > 0.f;
-  *reinterpret_cast<uint32_t*>(P.out + o * RI_DIM + 2 * lane) =
-      (uint32_t)ri_f32_to_e16<HALF>(any ? A0 / L : 0.f) | ((uint32_t)ri_f32_to_e16<HALF>(any ? A1 / L : 0.f) << 16);
-  if (lane == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
-}
-
-// Merges the S split partials of group g (and the optional previous result) and writes the
-// output: wave w of the calling workgroup takes heads w, w+NW, ...; lanes first cover the splits
-// (statistics), then two dims each.
-// The partials come from the memory side, where a load takes about a microsecond and one compute unit gets 20 KB per
-// microsecond: every wave requests the statistics of all its heads and then eight splits of all of them at a time.
-// (One head after the other: 13600 cycles for 16 heads over 3 splits.)
-template <int GS_PAD, bool HALF>
-__device__ __forceinline__ void combine_group(const AttendParams& P, int g) {
-  constexpr int NW = ATT_WAVES;
-  constexpr int HPW = (GS_PAD + NW - 1) / NW;   // heads of a wave
-  constexpr int U = HPW > 2 ? 4 : 8;            // splits requested at a time
-  const int gs = P.gs, S = P.S;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave >= gs) return;
-  const float* ml = P.part_ml + (size_t)g * S * GS_PAD * 2;
-  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + 2 * lane;
-  float2 ms[HPW];
-#pragma unroll
-  for (int k = 0; k < HPW; ++k)
-    ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * 2);
-  float2 a[U][HPW];
-  const auto request = [&](int s0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int k = 0; k < HPW; ++k)
-        a[u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * RI_DIM);
-  };
-  request(0);
-  float f[HPW], M[HPW], L[HPW], A0[HPW], A1[HPW];
-#pragma unroll
-  for (int k = 0; k < HPW; ++k) {
-    const float m = lane < S ? ms[k].x : -INFINITY;
-    M[k] = ri_row_max(m);
-    M[k] = fmaxf(M[k], __shfl_xor(M[k], 16));
-    M[k] = fmaxf(M[k], __shfl_xor(M[k], 32));
-    f[k] = m == -INFINITY ? 0.f : __expf(m - M[k]);
-    L[k] = ri_row_sum(ms[k].y * f[k]);
-    L[k] += __shfl_xor(L[k], 16);
-    L[k] += __shfl_xor(L[k], 32);
-    A0[k] = A1[k] = 0.f;
-  }
-  for (int s0 = 0; s0 < S; s0 += U) {   // (a split past the last has no weight: f of its lane is 0)
-    if (s0) request(s0);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int k = 0; k < HPW; ++k) {
-        const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[k]), (s0 + u) & 63));
-        const float w = s0 + u < S ? fs : 0.f;
-        A0[k] += a[u][k].x * w;
-        A1[k] += a[u][k].y * w;
-      }
-  }
-#pragma unroll
-  for (int k = 0; k < HPW; ++k)
-    if (wave + k * NW < gs) write_head<HALF>(P, g, wave + k * NW, M[k], L[k], A0[k], A1[k]);
-}
-
-#define ATT_DESC_MAX 64  // rows of one wave whose descriptors are staged in LDS at a time (32 and 128 measured slower)
-
-// A wave's LDS: value tile, probabilities, rescale factors, row descriptors and weights.
-struct WaveLds {
-  uint16_t* vt;
-  uint16_t* pb;
-  float* al;
-  int* dsc;
-  float* w;
-};
-
-// Rows [r0, r1) of one wave in batches of 64.  `stage(row, weight)` returns where the row lives (a descriptor) and may set
-// the row's weight; `load(d, dv, k, v)` requests the score operand and the four value rows of a chunk, `score` turns
-// the operand into the scores of this lane's heads.
-// The next chunk is requested as soon as the registers of this one are free (keys after their products, values after
-// they are in LDS), so that its loads run under the softmax and the P.V products without a second set of registers.
-template <int GS_PAD, bool HALF, typename K, typename Stage, typename Load, typename Score>
-__device__ __forceinline__ void attend_rows(WaveState<GS_PAD>& st, const WaveLds& sh, int r0, int r1, Stage&& stage,
-                                            Load&& load, Score&& score) {
-  const int lane = threadIdx.x & 63;
-  const int n = lane & 15, h = lane >> 4;
-  for (int s0 = r0; s0 < r1; s0 += ATT_DESC_MAX) {
-    const int s1 = min(r1, s0 + ATT_DESC_MAX);
-    {
-      float w = 1.f;
-      // (a row past the last repeats it, marked: every load has a valid address and no load sits under a condition)
-      const int d = stage(min(s0 + lane, s1 - 1), w);
-      sh.dsc[lane] = s0 + lane < s1 ? d : d | ATT_SKIP;
-      sh.w[lane] = w;
-    }
-    ri_wave_sync();
-    const int nch = (s1 - s0 + 15) >> 4;
-    K k;
-    uint4 v[4];
-    int dk, dv[4];
-    const auto issue = [&](int j) {
-      dk = sh.dsc[j * 16 + n];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dv[i] = sh.dsc[j * 16 + h + 4 * i];
-      load(dk & ~ATT_SKIP, dv, k, v);
-    };
-    issue(0);
-    for (int j = 0; j < nch; ++j) {
-      const bool valid = dk >= 0;
-      float sv[GS_PAD / 4], w = sh.w[j * 16 + n];
-      score(k, sv, w);
-      if (__builtin_amdgcn_ballot_w64(valid) != ~0ull) {   // rows that are not attended must not bring NaN into P.V
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (dv[i] < 0) v[i] = ri_zero16();
-      }
-      chunk_values(v, sh.vt, lane);
-      if (j + 1 < nch) issue(j + 1);
-      chunk_update<GS_PAD, HALF>(st, sv, valid, w, sh.vt, sh.pb, sh.al, lane);
-    }
-  }
-}
-
-// The eight waves of a workgroup merge in LDS, so a group split over S workgroups hands S partials to its last arriver.
-// The rank tables of the retrieval zone (np + 1 token offsets, np first rows) live in dynamic LDS, sized by
-// the launch, so that any number of probes the selection accepts can be attended.
-// HALF: q, K, V, value sums, cluster sizes, weights and outputs are IEEE half instead of bfloat16.
 template <int GS_PAD, bool HALF>
 __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams P) {
-  constexpr int NW = ATT_WAVES;
-  constexpr int NH = GS_PAD / 4;
-  constexpr int NT = 64 * NW;
-  __shared__ __attribute__((aligned(16))) uint16_t sh_vt[NW][16 * ATT_VT_STRIDE];
-  __shared__ __attribute__((aligned(16))) uint16_t sh_pb[NW][16 * 16];
-  __shared__ float sh_al[NW][16];
-  __shared__ float sh_m[NW][GS_PAD];
-  __shared__ float sh_l[NW][GS_PAD];
-  // the waves' numerators for the merge: up to eight heads they are laid over the wave's own value tile (dead once its
-  // rows are done), which keeps a workgroup at 48 KB of LDS, so that the two its registers leave room for fit a compute
-  // unit (sixteen heads: 116 KB, one workgroup)
-  constexpr bool ACC_OVER_VT = GS_PAD * RI_DIM * sizeof(float) <= 16 * ATT_VT_STRIDE * sizeof(uint16_t);
-  __shared__ float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
-  auto acc_of = [&](int w) -> float* {
-    return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : &sh_acc_own[ACC_OVER_VT ? 0 : w][0][0];
-  };
-  __shared__ __attribute__((aligned(16))) uint16_t sh_q[GS_PAD][RI_DIM];
-  __shared__ int sh_desc[NW][ATT_DESC_MAX];
-  __shared__ float sh_w[NW][ATT_DESC_MAX];
-  __shared__ int sh_last;
-  extern __shared__ __attribute__((aligned(16))) int sh_tab[];
-  int* const sh_roff = sh_tab;              // [np + 1]
-  int* const sh_rst = sh_tab + P.np + 1;    // [np]
-
-  const int g = blockIdx.y;
-  const int split = blockIdx.x;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = lane & 15, h = lane >> 4;
-  const int gs = P.gs, S = P.S;
-
-  WaveState<GS_PAD> st;
-#pragma unroll
-  for (int i = 0; i < NH; ++i) { st.m[i] = -INFINITY; st.l[i] = 0.f; }
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) st.acc[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-  const WaveLds sh = {sh_vt[wave], sh_pb[wave], sh_al[wave], sh_desc[wave], sh_w[wave]};
-  // P rows of heads that do not exist stay zero; alpha of such heads must not scale by garbage
-  for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(sh.pb)[i] = 0u;
-  if (lane < 16) sh.al[lane] = 1.f;
-  const int lenB = P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  const int lenA = P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
-
-  const int wid = split * NW + wave;            // wave of the group
-  const bool kv_wave = wid < P.W_kv;
-  const bool kv_wg = split * NW < P.W_kv;       // the workgroup has waves with key/value rows
-  const int W_es = S * NW - P.W_kv;
-
-  // ---------------- prologue: query and rank tables to LDS ----------------
-  if (kv_wg || P.est_cent) {
-    const bool tab = kv_wg && P.ret_off != nullptr;
-    // every global load of the prologue is requested before the first of them is consumed
-    // (up to 1023 probes the table entries pass through registers, TAB_U per thread; longer tables are
-    // staged by a plain loop after the query)
-    constexpr int TAB_U = 1024 / NT;
-    const bool tab_fast = tab && P.np < 1024;
-    int t_off[TAB_U], t_st[TAB_U];
-    if (tab_fast) {
-#pragma unroll
-      for (int u = 0; u < TAB_U; ++u) {
-        const int i = threadIdx.x + u * NT;
-        t_off[u] = P.ret_off[(size_t)g * (P.np + 1) + min(i, P.np)];
-        t_st[u] = P.ret_start[(size_t)g * P.np + min(i, P.np - 1)];
-      }
-    }
-    // A operand: query heads through LDS (read again per chunk: registers go to the loads);
-    // row m of the MFMA holds head m % GS_PAD, zero if >= gs
-    static_assert(GS_PAD * (RI_DIM / 8) <= NT, "one piece of the query per thread");
-    {
-      const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
-      uint4 qv = ri_ld16(P.q + ((size_t)g * gs + min(head, gs - 1)) * RI_DIM + piece * 8);
-      if (head >= gs) qv = ri_zero16();
-      if (head < GS_PAD) *reinterpret_cast<uint4*>(&sh_q[head][piece * 8]) = qv;
-    }
-    if (tab_fast) {
-#pragma unroll
-      for (int u = 0; u < TAB_U; ++u) {
-        const int i = threadIdx.x + u * NT;
-        if (i <= P.np) sh_roff[i] = t_off[u];
-        if (i < P.np) sh_rst[i] = t_st[u];
-      }
-    } else if (tab) {
-      for (int i = threadIdx.x; i <= P.np; i += NT) {
-        sh_roff[i] = P.ret_off[(size_t)g * (P.np + 1) + i];
-        if (i < P.np) sh_rst[i] = P.ret_start[(size_t)g * P.np + i];
-      }
-    }
-    __syncthreads();
-  }
-
-  if (kv_wave || P.est_cent) {
-    // ---------------- rows with keys ----------------
-    // Estimation rows whose scores are not handed in are key/value rows of their own: key = centroid,
-    // value = value sum, weight = cluster size, located through the id list.
-    const bool est = !kv_wave;
-    int r0, r1;
-    if (est) wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
-    else wave_rows(lenA + lenB, P.W_kv, wid, &r0, &r1);
-    const uint16_t* qrow = &sh_q[n % GS_PAD][h * 8];
-    const uint16_t* kA = P.kA + (size_t)g * P.strideA * RI_DIM;
-    const uint16_t* vA = P.vA + (size_t)g * P.strideA * RI_DIM;
-    const uint16_t* kB = est ? P.est_cent + (size_t)g * P.nc * RI_DIM : P.kB + (size_t)g * P.strideB * RI_DIM;
-    const uint16_t* vB = est ? P.value_sum + (size_t)g * P.nc * RI_DIM : P.vB + (size_t)g * P.strideB * RI_DIM;
-    const int32_t* rs = est ? P.est_ids + (size_t)g * P.es
-                            : (P.row_src ? P.row_src + (size_t)g * P.rs_stride : nullptr);
-    const uint16_t* wB = (!est && P.weightB) ? P.weightB + (size_t)g * P.weight_stride : nullptr;
-    const uint16_t* wsrc = est ? P.csize + (size_t)g * P.nc : nullptr;  // weight by source row
-    const int r_first = ri_head_reg<GS_PAD>(h);
-    const int lead = est ? 0 : lenA;
-    struct Keys { uint4 k[4]; };
-    attend_rows<GS_PAD, HALF, Keys>(
-        st, sh, r0, r1,
-        [&](int row, float& w) {
-          if (row < lead) return row | ATT_FLAG_A;
-          const int rb = row - lead;
-          int d;
-          if (!est && P.ret_off) {
-            // the last rank whose first row is <= rb (ranks of empty clusters share a first row
-            // with the next rank, which is the one found)
-            int lo = 0, hi = P.np;
-            while (lo + 1 < hi) {
-              const int mid = (lo + hi) >> 1;
-              if (sh_roff[mid] <= rb) lo = mid; else hi = mid;
-            }
-            d = sh_rst[lo] + rb - sh_roff[lo];
-          } else {
-            d = rs ? rs[rb] : rb;
-            if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d = ATT_SKIP;   // row 0, not attended
-          }
-          if (wB) w = ri_e16_to_f32<HALF>(wB[rb]);
-          if (wsrc) w = ri_e16_to_f32<HALF>(wsrc[d]);
-          return d;
-        },
-        [&](int dk, const int* dv, Keys& k, uint4* v) {
-          const uint16_t* kp = ((dk & ATT_FLAG_A) ? kA : kB) + (size_t)(dk & ~ATT_FLAG_A) * RI_DIM + h * 8;
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) k.k[kk] = ri_ld16(kp + kk * 32);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int d = dv[i] & ~ATT_SKIP;
-            v[i] = ri_ld16(((d & ATT_FLAG_A) ? vA : vB) + (size_t)(d & ~ATT_FLAG_A) * RI_DIM + n * 8);
-          }
-        },
-        [&](const Keys& k, float* sv, float&) {
-          f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            const uint4 qv = *reinterpret_cast<const uint4*>(qrow + kk * 32);
-            acc = HALF ? __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, qv),
-                                                                __builtin_bit_cast(f16x8_t, k.k[kk]), acc, 0, 0, 0)
-                       : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(qv), ri_as_bf16x8(k.k[kk]), acc, 0, 0, 0);
-          }
-#pragma unroll
-          for (int i = 0; i < NH; ++i) {
-            float x;
-            if (GS_PAD == 16) {
-              x = acc[i];
-            } else {  // register r_first + i without dynamic indexing
-              const int r = r_first + i;
-              x = r == 0 ? acc[0] : (r == 1 ? acc[1] : (r == 2 ? acc[2] : acc[3]));
-            }
-            sv[i] = x * P.scale;
-          }
-        });
-  } else {
-    // ---------------- estimation rows with their logits at hand ----------------
-    int r0, r1;
-    wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
-    const int32_t* ids = P.est_ids + (size_t)g * P.es;
-    const uint16_t* vs = P.value_sum + (size_t)g * P.nc * RI_DIM;
-    const uint16_t* cs = P.csize + (size_t)g * P.nc;
-    const float* lg = P.logits + (size_t)g * gs * P.nc;
-    struct Logits { float x[NH]; uint16_t size; };
-    attend_rows<GS_PAD, HALF, Logits>(
-        st, sh, r0, r1, [&](int row, float&) { return ids[row]; },
-        [&](int dk, const int* dv, Logits& k, uint4* v) {
-#pragma unroll
-          for (int i = 0; i < NH; ++i) k.x[i] = lg[(size_t)min(ri_head_of<GS_PAD>(h, i), gs - 1) * P.nc + dk];
-          k.size = cs[dk];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = ri_ld16(vs + (size_t)(dv[i] & ~ATT_SKIP) * RI_DIM + n * 8);
-        },
-        [&](const Logits& k, float* sv, float& w) {
-#pragma unroll
-          for (int i = 0; i < NH; ++i) sv[i] = ri_head_of<GS_PAD>(h, i) < gs ? k.x[i] : -INFINITY;
-          w = ri_e16_to_f32<HALF>(k.size);
-        });
-  }
-
-  // ---------------- wave partial -> LDS ----------------
-#pragma unroll
-  for (int i = 0; i < NH; ++i) {
-    const float l = ri_row_sum(st.l[i]);
-    if (n == 0) {
-      sh_m[wave][ri_head_of<GS_PAD>(h, i)] = st.m[i];
-      sh_l[wave][ri_head_of<GS_PAD>(h, i)] = l;
-    }
-  }
-  // accumulators are already summed over rows: lane (n, h) register i holds head 4h+i, dim 16*dt+n
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int head = 4 * h + i;
-    if (head < GS_PAD) {
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) acc_of(wave)[head * RI_DIM + 16 * dt + n] = st.acc[dt][i];
-    }
-  }
-  __syncthreads();
-
-  // ---------------- merge the waves: wave w takes heads w, w + NW, ..., a lane two dims ----------------
-  for (int j = wave; j < gs; j += NW) {
-    float m[NW], M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      m[w] = sh_m[w][j];
-      M = fmaxf(M, m[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float f = m[w] == -INFINITY ? 0.f : __expf(m[w] - M);
-      const float2 x = *reinterpret_cast<const float2*>(acc_of(w) + j * RI_DIM + 2 * lane);
-      a0 += x.x * f;
-      a1 += x.y * f;
-      l += sh_l[w][j] * f;
-    }
-    if (S == 1) {   // the workgroup has the whole group: no partial leaves it
-      write_head<HALF>(P, g, j, M, l, a0, a1);
-      continue;
-    }
-    const size_t o = ((size_t)g * S + split) * GS_PAD + j;
-    // device-coherent stores: another workgroup of this launch reads them
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + 2 * lane]),
-                       (uint64_t)__float_as_uint(a0) | (uint64_t)__float_as_uint(a1) << 32, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    if (lane == 0)
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_ml[o * 2]),
-                         (uint64_t)__float_as_uint(M) | (uint64_t)__float_as_uint(l) << 32, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (S == 1) {
-    if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
-    return;
-  }
-
-  // ---------------- last workgroup of the group merges all splits ----------------
-  // Hand-off of the partials between workgroups of one launch, without fences:
-  //  * the partial was written above with agent-scope atomic stores: on gfx950 those are write-through
-  //    stores (sc1) that complete in the memory-side cache every compute unit shares, not in this
-  //    compute unit's L1 or this chiplet's L2;
-  //  * s_waitcnt(0) returns when all of this wave's stores have been acknowledged there, the barrier
-  //    makes that true for the whole workgroup, and only then does one thread announce the arrival with
-  //    an agent-scope atomic increment (performed at the same shared level);
-  //  * the workgroup that sees the count complete reads the partials with agent-scope atomic loads
-  //    (combine_group), which bypass the non-coherent cache levels.
-  // So every partial is globally visible before its arrival can be counted, and the reader cannot hit a
-  // stale line.  The C++ memory model would express this with a release increment and an acquire on the
-  // last arriver; at agent scope those compile to a write-back and an invalidate of the whole L2, which
-  // was measured at +15 us per launch (35.2 us instead of 20.0 us at the benchmark shape), while the
-  // data that must be ordered is only this workgroup's own 2 KB.  The asm statement keeps the compiler
-  // from moving the stores below the wait.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
-#error "the partial hand-off below relies on gfx950 cache behaviour: build this file for gfx950 only"
-#endif
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0)
-    sh_last = (__hip_atomic_fetch_add(&P.counters[g], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1);
-  __syncthreads();
-  if (!sh_last) return;
-  combine_group<GS_PAD, HALF>(P, g);
-  if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
-  // ready for the next launch (every arrival of this launch has been counted; launches that share the
-  // workspace do not overlap)
-  if (threadIdx.x == 0) __hip_atomic_store(&P.counters[g], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  attend_group<GS_PAD, HALF, false>(P, blockIdx.y, blockIdx.x, AttendKept{});
 }
 
 // ------------------------------------------------------------------------------------
@@ -583,12 +96,13 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 //    11.6 us, 21: 12.0).
 //  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
 //    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
-static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs) {
+static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
+                        int max_splits = RI_MAX_SPLITS) {
   const int64_t rows = kv_rows + es_rows, wk = kv_rows * 512, we = es_rows * es_row_bytes;
   int64_t per_group = 256 / BG;
   per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
-  per_group = min(per_group, (int64_t)RI_MAX_SPLITS);
+  per_group = min(per_group, (int64_t)max_splits);
   if (rows * gs_pad_of(gs) <= 384 * 4 || per_group < 1) per_group = 1;
   const int waves = (int)per_group * ATT_WAVES;
   P.S = (int)per_group;
@@ -646,26 +160,14 @@ extern "C" int ri_weighted_flash_decoding_f16(const void* q, const void* k, cons
                              scale, workspace, workspace_bytes, true, stream);
 }
 
-// Shared body of ri_wave_attention and ri_wave_attention_static.  `scratch` holds the arrival
-// counters and the split partials; with scratch_bytes == 0 the caller vouches for its size through
-// scratch_limit (the static array) and the counters are cleared by a fill kernel first.
-__global__ void attend_clear_counters_kernel(int* counters, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) counters[i] = 0;
-}
-
-static int wave_attention_impl(const void* q, const void* steady_k, const void* steady_v, int64_t steady_stride,
-                               int static_len, const int32_t* static_len_dev, const void* store_k,
-                               const void* store_v, int64_t store_stride, const int32_t* row_src,
-                               int row_src_stride, const int32_t* ret_tok_off, const int32_t* ret_start, int np,
-                               const int32_t* meta, const int32_t* est_ids, const float* logits,
-                               const void* est_centroids, const void* value_sum, const void* cluster_size_bf16,
-                               void* out, int32_t* valid_lengths, int BG, int gs, int nc, int es, float scale,
-                               void* scratch, size_t scratch_bytes, bool clear_counters, bool half, hipStream_t stream,
-                               int src_lo = INT32_MIN, int src_hi = INT32_MAX, const void* prev_out = nullptr,
-                               const float* prev_lse = nullptr, float* lse_out = nullptr) {
+int ri_prepare_wave_attention(AttendParams* out_params, const void* q, const void* steady_k, const void* steady_v,
+                              int64_t steady_stride, int static_len, const int32_t* static_len_dev, const void* store_k,
+                              const void* store_v, int64_t store_stride, const int32_t* row_src, int row_src_stride,
+                              const int32_t* ret_tok_off, const int32_t* ret_start, int np, const int32_t* meta,
+                              const int32_t* est_ids, const float* logits, const void* est_centroids, const void* value_sum,
+                              const void* cluster_size_bf16, void* out, int32_t* valid_lengths, int BG, int gs, int nc,
+                              int es, float scale, void* scratch, size_t scratch_bytes, bool one_workgroup) {
   if (!q || !steady_k || !steady_v || !store_k || !store_v || !meta || !out || !scratch) return RI_ERR_ARG;
-  if ((prev_out == nullptr) != (prev_lse == nullptr) || ri_misaligned16(prev_out)) return RI_ERR_ARG;
   if (ri_any_misaligned16(q, steady_k, steady_v, store_k, store_v, value_sum, est_centroids, out, scratch))
     return RI_ERR_ARG;
   if (!row_src && (!ret_tok_off || !ret_start || np <= 0 || np > RI_MAX_PROBES)) return RI_ERR_ARG;
@@ -688,11 +190,7 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   P.strideB = store_stride;
   P.row_src = row_src;
   P.rs_stride = row_src_stride;
-  P.src_lo = max(src_lo, 0);   // an entry below 0 is padding in every window
-  P.src_hi = src_hi;
-  P.prev_out = (const uint16_t*)prev_out;
-  P.prev_lse = prev_lse;
-  P.lse_out = lse_out;
+  P.src_hi = INT32_MAX;   // (an entry below 0 is padding in every window)
   if (!row_src) {
     P.ret_off = ret_tok_off;
     P.ret_start = ret_start;
@@ -715,9 +213,43 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   // capacity scaled by the usual fill (a quarter) or for 16 tokens per rank, the estimation zone by
   // its exact size
   plan_splits(P, static_len + (row_src ? row_src_stride / 4 : np * 16), es,
-              est_row_bytes(gs, est_centroids != nullptr), BG, gs);
+              est_row_bytes(gs, est_centroids != nullptr), BG, gs, one_workgroup ? 1 : RI_MAX_SPLITS);
   if (scratch_bytes < attn_scratch_used(BG, gp, P.S)) return RI_ERR_WORKSPACE;
   carve_workspace(P, scratch, BG, gp);
+  *out_params = P;
+  return RI_OK;
+}
+
+// Shared body of ri_wave_attention and ri_wave_attention_static.  `scratch` holds the arrival
+// counters and the split partials; with scratch_bytes == 0 the caller vouches for its size through
+// scratch_limit (the static array) and the counters are cleared by a fill kernel first.
+__global__ void attend_clear_counters_kernel(int* counters, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) counters[i] = 0;
+}
+
+static int wave_attention_impl(const void* q, const void* steady_k, const void* steady_v, int64_t steady_stride,
+                               int static_len, const int32_t* static_len_dev, const void* store_k,
+                               const void* store_v, int64_t store_stride, const int32_t* row_src,
+                               int row_src_stride, const int32_t* ret_tok_off, const int32_t* ret_start, int np,
+                               const int32_t* meta, const int32_t* est_ids, const float* logits,
+                               const void* est_centroids, const void* value_sum, const void* cluster_size_bf16,
+                               void* out, int32_t* valid_lengths, int BG, int gs, int nc, int es, float scale,
+                               void* scratch, size_t scratch_bytes, bool clear_counters, bool half, hipStream_t stream,
+                               int src_lo = INT32_MIN, int src_hi = INT32_MAX, const void* prev_out = nullptr,
+                               const float* prev_lse = nullptr, float* lse_out = nullptr) {
+  if ((prev_out == nullptr) != (prev_lse == nullptr) || ri_misaligned16(prev_out)) return RI_ERR_ARG;
+  AttendParams P;
+  const int rc = ri_prepare_wave_attention(&P, q, steady_k, steady_v, steady_stride, static_len, static_len_dev, store_k,
+                                           store_v, store_stride, row_src, row_src_stride, ret_tok_off, ret_start, np, meta,
+                                           est_ids, logits, est_centroids, value_sum, cluster_size_bf16, out, valid_lengths,
+                                           BG, gs, nc, es, scale, scratch, scratch_bytes, false);
+  if (rc) return rc;
+  P.src_lo = max(src_lo, 0);
+  P.src_hi = src_hi;
+  P.prev_out = (const uint16_t*)prev_out;
+  P.prev_lse = prev_lse;
+  P.lse_out = lse_out;
   if (clear_counters) {
     attend_clear_counters_kernel<<<(BG + 255) / 256, 256, 0, stream>>>(P.counters, BG);
     RI_HIP_CHECK_LAUNCH();

@@ -4,7 +4,8 @@
 // A short context's step is bound by what the host spends on it, not by the GPU: through torch's slice copies and one
 // wrapper call per stage a layer-step took 46 us of host time, of which the launches are 1 us each.  The addresses and
 // sizes of a layer do not change from token to token, so the caller keeps them in one struct and hands over its address.
-#include "ri_common.h"
+#include "attend_common.h"
+#include "select_body.h"
 
 // ------------------------------------------------------------------------------------
 // append: steady_k/v[g, pos] = key/value[g]; 16 lanes per 256-byte row, grid.y = K, V.
@@ -35,8 +36,60 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
   return RI_OK;
 }
 
+// ------------------------------------------------------------------------------------
+// step: scoring, selection and attention of a group by one workgroup, for short contexts.
+// With up to 512 clusters the selection is one workgroup per group that scores for itself, and with few rows the attention
+// is, too: as one kernel the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
+// host as well.  What bounds it is the chain of either half on one compute unit.  8 groups of 4 heads, 512 clusters, 331
+// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110 KB of LDS (124 with 8 heads): one workgroup
+// per compute unit, hence at most 256 groups; sixteen heads would not fit.
+// ------------------------------------------------------------------------------------
+#define STEP_CLUSTERS 512
+
+template <int GSM, bool HALF>
+__global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(SelectArgs S, AttendParams A) {
+  static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
+  __shared__ float sh_logits[STEP_CLUSTERS * GSM];
+  __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS];
+  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, true>(S, blockIdx.x, SelectKept{sh_logits, sh_est, sh_off, sh_start});
+  lds_barrier();
+  attend_group<GSM, HALF, true>(A, blockIdx.x, 0, AttendKept{sh_logits, sh_est, sh_off, sh_start});
+}
+
+// Short: what one workgroup scores for itself (select.hip), and no more rows than one workgroup attends as fast as several
+// (with the launch left out; 8 groups of 4 heads: 446 rows 14.4 us either way, 557 rows 15.8 against 15.4; 64 groups of 8
+// heads: 446 rows 16.7 against 17.1).
+#define STEP_ROWS 448
+static bool step_is_short(const ri_decode_step_t* s, int static_len) {
+  const long long rows = (long long)static_len + (long long)s->np * 16 + s->es;
+  return s->nc <= STEP_CLUSTERS && s->gs <= 8 && s->BG <= 256 && rows <= STEP_ROWS && s->cluster_size_i32 &&
+         s->cluster_start;
+}
+
+static int step_short(const ri_decode_step_t* s, const void* q, int static_len, void* out, hipStream_t stream) {
+  SelectArgs S;
+  int rc = ri_prepare_select(&S, q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,
+                             s->ret_ids, s->est_ids, s->ret_tok_off, s->ret_start, nullptr, 0, s->meta, s->BG, s->gs, s->nc,
+                             s->np, s->es, s->page, s->max_pages, s->scale, s->score_workspace, s->score_workspace_bytes);
+  if (rc) return rc;
+  if (s->attn_workspace && s->attn_workspace_bytes < ri_wave_attention_workspace_bytes(s->BG, s->gs)) return RI_ERR_WORKSPACE;
+  AttendParams A;
+  rc = ri_prepare_wave_attention(&A, q, s->steady_k, s->steady_v, s->steady_stride, static_len, s->static_len_dev, s->store_k,
+                                 s->store_v, s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta,
+                                 s->est_ids, s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out,
+                                 s->valid_lengths, s->BG, s->gs, s->nc, s->es, s->scale, s->attn_workspace,
+                                 s->attn_workspace_bytes, true);
+  if (rc) return rc;
+  auto* kernel = s->gs <= 4 ? (s->half ? step_kernel<4, true> : step_kernel<4, false>)
+                            : (s->half ? step_kernel<8, true> : step_kernel<8, false>);
+  kernel<<<s->BG, 64 * ATT_WAVES, 0, stream>>>(S, A);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
 extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int static_len, void* out, ri_stream_t stream) {
   if (!s) return RI_ERR_ARG;
+  if (step_is_short(s, static_len)) return step_short(s, q, static_len, out, (hipStream_t)stream);
   auto* select = s->half ? ri_score_select_f16 : ri_score_select;
   auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
   const int rc = select(q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,

@@ -21,3 +21,53 @@ def test_append_kv(dev, BG, stride, pos, on_device):
     if not on_device:
         with pytest.raises(RuntimeError):
             kernels.append_kv(k, v, zk, zv, stride)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BG,gs,nc,np_,es,static,pages,on_device", [
+    (1, 1, 8, 1, 0, 0, 100, False), (2, 4, 8, 3, 5, 1, 100, True), (3, 5, 40, 7, 33, 17, 100, False),
+    (5, 8, 256, 4, 60, 70, 2, True), (4, 3, 264, 10, 100, 69, 100, False), (8, 4, 512, 9, 118, 98, 100, False),
+    (2, 7, 504, 12, 150, 100, 3, True), (256, 2, 16, 2, 3, 5, 100, False), (257, 2, 16, 2, 3, 5, 100, False),
+    (2, 4, 512, 13, 118, 98, 100, False)])
+def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
+    """The step that one workgroup per group makes (and, past its limits, the launches one by one) against scoring +
+    selection and attention called by themselves: the same lists; outputs differ only where those split a group's rows,
+    by roundings of the 16-bit probabilities and of the output, each at most 2^-8 of a value (2^-11 in half), of which a
+    norm over the output sees a fraction."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(BG * nc + gs)
+    rn = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)
+    size = torch.randint(0, 30, (BG, nc), generator=g, dtype=torch.int32)
+    size[:, 0] = 0
+    start = (size.cumsum(1) - size).int().to(dev)
+    rows = int(size.sum(1).max()) + 1
+    mask = (size == 0).to(dev)
+    size16, size = size.to(dtype).to(dev), size.to(dev)
+    q, cent, vs = rn(BG, gs, 128), rn(BG, nc, 128), rn(BG, nc, 128)
+    zone = static + 3
+    sk, sv, store_k, store_v = rn(BG, zone, 128), rn(BG, zone, 128), rn(BG, rows, 128), rn(BG, rows, 128)
+    length = torch.tensor([static], dtype=torch.int32, device=dev) if on_device else None
+
+    def fresh():
+        i32 = lambda *s: torch.full(s, -5, dtype=torch.int32, device=dev)
+        return dict(logits=torch.zeros(BG, gs, nc, device=dev), ret_ids=i32(BG, np_), est_ids=i32(BG, max(es, 1)),
+                    ret_tok_off=i32(BG, np_ + 1), ret_start=i32(BG, np_), meta=i32(BG, 4), valid_lengths=i32(BG))
+    a, b = fresh(), fresh()
+    scale = 128 ** -0.5
+    est = lambda d: d["est_ids"] if es else None
+    kernels.score_select(q, cent, mask, size, start, a["logits"], None, None, a["ret_ids"], est(a), a["ret_tok_off"], None,
+                         a["meta"], np_, es, 8, pages, scale, ret_start=a["ret_start"])
+    want, got = torch.empty(BG, gs, 128, dtype=dtype, device=dev), torch.empty(BG, gs, 128, dtype=dtype, device=dev)
+    kernels.wave_attention(q, sk, sv, static, store_k, store_v, None, a["meta"], est(a), a["logits"] if es else None, vs,
+                           size16, want, a["valid_lengths"], es, scale, ret_tok_off=a["ret_tok_off"],
+                           ret_start=a["ret_start"], static_len_dev=length)
+    plan = kernels.DecodeStepPlan(None, dtype, dict(
+        b, est_ids=est(b), centroids=cent, mask=mask, cluster_size_i32=size, cluster_start=start, steady_k=sk, steady_v=sv,
+        static_len_dev=length, store_k=store_k, store_v=store_v, value_sum=vs, cluster_size=size16), np_, es, 8, pages, scale)
+    for _ in range(2):
+        plan.run(q, static, got)
+    for name in a:
+        if es or name != "est_ids":
+            assert torch.equal(a[name], b[name]), name
+    wf, gf = want.float(), got.float()
+    assert (wf - gf).norm() <= (4e-3 if dtype == torch.bfloat16 else 5e-4) * wf.norm()
