@@ -130,23 +130,56 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
       km_lds_dma16(cp + (size_t)row * RI_DIM, ld_at, sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2));
     }
   };
+  // Tokens as operands: lane: token r, dims 16 kk + 8 hh.  A load whose lanes touch 32 tokens keeps the compute unit's address
+  // path busy for 64 cycles, one of four whole tokens for 18; with eight waves that start together that is in front of the
+  // first product.  Their tokens are loaded whole and turned in the wave's part of the last tile buffer, which no tile is on
+  // its way to yet, 16 at a time, piece k of token t at place k ^ t of its row (8 x 8192 tokens, 512 centroids: 11.4 -> 10.3
+  // us, 16 x 8200 22.8 -> 20.8, 4 x 15000, 928 17.0 -> 16.0; 4 x 48719, 3072 120.6 and 121.4; four columns of long loops the
+  // same, so they stay).  The small tiles of four
+  // waves leave room for eight tokens at a time, and other workgroups run beside: as operands (128 x 8192: 121.9 us, turned
+  // 124.1).
+  constexpr int WR = KM_CT / KM_W;
+  constexpr bool TURN = WR == 16 && KM_TT < 4;
   uint4 b[KM_TT][8];
 #pragma unroll
   for (int tt = 0; tt < KM_TT; ++tt) {
     const uint16_t* q = dp + (size_t)min(t0 + tt * 32 + r, N - 1) * RI_DIM + hh * 8;
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) b[tt][kk] = ri_ld16(q + kk * 16);
+    for (int i = 0; i < 8; ++i)
+      b[tt][i] = TURN ? ri_ld16(dp + (size_t)min(t0 + tt * 32 + 4 * i + (lane >> 4), N - 1) * RI_DIM + (lane & 15) * 8)
+                      : ri_ld16(q + i * 16);
   }
   const int tiles = (nc + KM_CT - 1) / KM_CT;
 #pragma unroll
   for (int t = 0; t < KM_NB - 1; ++t) tile_load(t * KM_CT, t);
-  // (the token registers are consumed here so that the compiler's own wait for their loads sits
-  // in front of the loop and not inside it, where it would also wait for the tile in flight)
+  // (The token registers are consumed here so that the compiler's own wait for their loads sits in front of the loop and not
+  // inside it, where it would also wait for the tile in flight.)
+  uint4* const turn = reinterpret_cast<uint4*>(&sh_c[KM_NB - 1][wave * WR][0]);
   km_wait_vm<(KM_NB - 1) * L>();
 #pragma unroll
-  for (int tt = 0; tt < KM_TT; ++tt)
+  for (int tt = 0; tt < KM_TT; ++tt) {
+    if (TURN) {
+      uint4 o[8];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = 4 * i + (lane >> 4);
+          turn[row * 16 + ((lane & 15) ^ row)] = b[tt][w * 4 + i];
+        }
+        ri_wave_sync();
+        if (r >> 4 == w) {
+#pragma unroll
+          for (int kk = 0; kk < 8; ++kk) o[kk] = turn[(r & 15) * 16 + ((kk * 2 + hh) ^ (r & 15))];
+        }
+        ri_wave_sync();   // (a wave's LDS accesses happen in order)
+      }
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) b[tt][kk] = o[kk];
+    }
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[tt][kk].x), "+v"(b[tt][kk].y), "+v"(b[tt][kk].z), "+v"(b[tt][kk].w));
+  }
 
   float best[KM_TT];
   int bidx[KM_TT];
@@ -1124,14 +1157,14 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   const long long wgs768 = (long long)P * ((N + 767) / 768);
   const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
   // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
-  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 10.9 us
-  // against 18.9 with two columns at the time; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
+  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
+  // against 18.9 with two columns when they were compared, now 10.3; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
   if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
   else if (wgs256 <= 512) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
   // One workgroup per compute unit that gives each wave three or four columns, where the fullest unit has that many
   // columns per wave to do anyway: the same work with more reuse of every LDS read (16 x 8200 tokens, 512 centroids: 25.8
   // us against 28.7 for the last line's when they were compared; 4 x 48719, 3072: 124 against 135; 20 x 9757, 608: 37.8
-  // against 40.4; now 23.1, 119.6 and 34.8).
+  // against 40.4; now 20.8, 121 and 33.6).
   else if (nc >= 512 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
   else if (nc >= 512 && wgs256 > 768 && wgs1024 <= 256) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
   // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
