@@ -251,12 +251,10 @@ __device__ __forceinline__ void combine_group(const AttendParams& P, int g) {
   for (int k = 0; k < HPW; ++k) {
     const float m = lane < S ? ms[k].x : -INFINITY;
     M[k] = ri_row_max(m);
-    M[k] = fmaxf(M[k], __shfl_xor(M[k], 16));
-    M[k] = fmaxf(M[k], __shfl_xor(M[k], 32));
+    M[k] = ri_xor_max<32>(ri_xor_max<16>(M[k]));
     f[k] = m == -INFINITY ? 0.f : __expf(m - M[k]);
     L[k] = ri_row_sum(ms[k].y * f[k]);
-    L[k] += __shfl_xor(L[k], 16);
-    L[k] += __shfl_xor(L[k], 32);
+    L[k] = ri_xor_sum<32>(ri_xor_sum<16>(L[k]));
     A0[k] = A1[k] = 0.f;
   }
   for (int s0 = 0; s0 < S; s0 += U) {   // (a split past the last has no weight: f of its lane is 0)

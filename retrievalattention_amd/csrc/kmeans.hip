@@ -679,10 +679,7 @@ __device__ __forceinline__ void km_finish(float s0, float s1, int count, int nor
     s0 = s0 / cnt;
     s1 = s1 / cnt;
     if (normalize) {
-      float sq = s0 * s0 + s1 * s1;  // two roundings: built without fp contraction
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
-      const float nrm = sqrtf(sq);
+      const float nrm = sqrtf(ri_wave_sum(s0 * s0 + s1 * s1));  // two roundings: built without fp contraction
       s0 = s0 / nrm;
       s1 = s1 / nrm;
     }

@@ -89,8 +89,7 @@ __device__ __forceinline__ void score_body(
   }
   __shared__ float sh_max[NWV][16];
   __shared__ float sh_sum[NWV][16];
-  lmax = fmaxf(lmax, __shfl_xor(lmax, 16));
-  lmax = fmaxf(lmax, __shfl_xor(lmax, 32));
+  lmax = ri_xor_max<32>(ri_xor_max<16>(lmax));
   float lsum = 0.f;
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
@@ -99,8 +98,7 @@ __device__ __forceinline__ void score_body(
     for (int i = 0; i < 4; ++i)
       if (cbase + i < nc) lsum += __expf(acc[t][i] - lmax);
   }
-  lsum += __shfl_xor(lsum, 16);
-  lsum += __shfl_xor(lsum, 32);
+  lsum = ri_xor_sum<32>(ri_xor_sum<16>(lsum));
   if (h == 0) {
     sh_max[wave][r] = lmax;
     sh_sum[wave][r] = lsum;

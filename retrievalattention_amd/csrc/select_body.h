@@ -50,28 +50,6 @@ struct SelectArgs {
 // Barrier over LDS traffic only: global stores issued before it stay in flight (__syncthreads waits for them as well).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// {a, b} = this lane's value and that of lane (lane ^ D), in either order; register moves only
-template <int D>
-__device__ __forceinline__ void lane_pair(uint32_t v, uint32_t& a, uint32_t& b) {
-  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-  a = v;
-  if constexpr (D == 1) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true);   // quad_perm 1,0,3,2
-  if constexpr (D == 2) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true);   // quad_perm 2,3,0,1
-  if constexpr (D == 4) {
-    const int m = __builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true);                      // half row mirrored: ^ 7
-    b = (uint32_t)__builtin_amdgcn_update_dpp(0, m, 0x1B, 0xf, 0xf, true);                            // quad_perm 3,2,1,0: ^ 3
-  }
-  if constexpr (D == 8) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, true);  // row_ror:8
-  if constexpr (D == 16) {   // rows 1 and 3 of one copy against rows 0 and 2 of the other
-    const u32x2_t p = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_permlane16_swap(v, v, false, false));
-    a = p.x; b = p.y;
-  }
-  if constexpr (D == 32) {
-    const u32x2_t p = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_permlane32_swap(v, v, false, false));
-    a = p.x; b = p.y;
-  }
-}
-
 // lanes whose bit K and bit D are equal: those that keep the larger value of an exchange over 2^D in a merge of 2^K
 constexpr uint64_t keep_mask(int K, int D) {
   uint64_t m = 0;
@@ -96,7 +74,7 @@ __device__ __forceinline__ void bitonic_step(uint32_t& v, bool active, uint32_t*
     }
   } else if (active) {
     uint32_t a, b;
-    lane_pair<(1 << LD)>(v, a, b);
+    ri_lane_pair<(1 << LD)>(v, a, b);
     const uint32_t hi = max(a, b), lo = min(a, b);
     uint64_t keep = keep_mask(LK, LD);   // (bit LK of a lane is 0 when LK >= 6: bit LK of tid is the wave's)
     if (LK >= 6 && ((wave >> (LK >= 6 ? LK - 6 : 0)) & 1)) keep = ~keep;
@@ -214,15 +192,13 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
         if (16 * (wave + NW * t) + 4 * h < nc)   // nc % 4 == 0: the four rows are valid together
 #pragma unroll
           for (int i = 0; i < 4; ++i) lmax = fmaxf(lmax, acc[t][i]);
-      lmax = fmaxf(lmax, __shfl_xor(lmax, 16));
-      lmax = fmaxf(lmax, __shfl_xor(lmax, 32));
+      lmax = ri_xor_max<32>(ri_xor_max<16>(lmax));
 #pragma unroll
       for (int t = 0; t < 4; ++t)
         if (16 * (wave + NW * t) + 4 * h < nc)
 #pragma unroll
           for (int i = 0; i < 4; ++i) lsum += __expf(acc[t][i] - lmax);
-      lsum += __shfl_xor(lsum, 16);
-      lsum += __shfl_xor(lsum, 32);
+      lsum = ri_xor_sum<32>(ri_xor_sum<16>(lsum));
       if (h == 0) {
         sh_a[wave][r] = lmax;
         sh_b[wave][r] = lsum;
