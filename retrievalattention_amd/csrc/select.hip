@@ -75,12 +75,14 @@ __global__ __launch_bounds__(256) void dist_kernel(const float* __restrict__ log
   float d[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < GSM; ++j) {
+    // (uniform; of sixteen the compiler moves every load behind its branch, so there the heads past gs count for nothing)
+    if (GSM <= 8 && j >= gs) break;
     const float x[4] = {x4[j].x, x4[j].y, x4[j].z, x4[j].w};
     const float m = sh_m[j], iz = sh_iz[j];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float p = ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[i]) - m) * iz);
-      d[i] += j < gs ? p : 0.f;
+      d[i] += GSM <= 8 || j < gs ? p : 0.f;
     }
   }
   uint16_t bits[4], key[4];

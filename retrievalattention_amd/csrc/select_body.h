@@ -256,11 +256,13 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       for (int i = 0; i < E; ++i) d[i] = 0.f;
 #pragma unroll
       for (int j = 0; j < GSM; ++j) {
+        // (uniform; of sixteen the compiler moves every load behind its branch, so there the heads past gs count for nothing)
+        if (GSM <= 8 && j >= gs) break;
         const float m = sh_a[0][j], iz = sh_b[0][j];
 #pragma unroll
         for (int i = 0; i < E; ++i) {
           const float p = ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[j][i / V][i % V]) - m) * iz);
-          d[i] += j < gs ? p : 0.f;
+          d[i] += GSM <= 8 || j < gs ? p : 0.f;
         }
       }
     }
