@@ -113,13 +113,20 @@ struct SelectKept {
 // GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well.
 template <int NT, int E, int GSM, bool HALF, int SRC, bool KEEP>
 __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K) {
-  static_assert(!KEEP || SRC == SEL_SCORE, "the logits are at hand where they are made");
+  static_assert(!KEEP || (SRC == SEL_SCORE && GSM <= 8), "the logits are in LDS");
   constexpr int NW = NT / 64, IDS = NT * E;
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
   constexpr int SHIFT = 16 - (LOGT + 2), FB = 1 << SHIFT;   // lower bits of a key, fine bins
   __shared__ __attribute__((aligned(16))) uint32_t hist[4 * NT];   // coarse bins; later the exchange area of the sort
   __shared__ uint32_t sh_fine[2][64], sh_scan[3][16], sh_sel[4], sh_tot[3], sh_ret[NT];
-  __shared__ __attribute__((aligned(16))) uint16_t sh_p[SRC == SEL_SCORE ? IDS * GSM : 8];
+  // Sizes and first rows of all clusters, requested with the first loads: the ones of the retrieval zone are only known
+  // after the sort, and a round trip for them there is a tenth of the kernel.  (With more clusters that is more than it saves:
+  // 16 groups of 1024 10.4 us either way.)
+  constexpr bool STAGED = SRC == SEL_SCORE;
+  constexpr bool OWN = GSM <= 8;   // who computes the probabilities, see below
+  __shared__ __attribute__((aligned(16))) int32_t sh_size[STAGED ? IDS : 4], sh_row[STAGED ? IDS : 4];
+  __shared__ __attribute__((aligned(16))) float sh_x[SRC == SEL_SCORE && OWN && !KEEP ? IDS * GSM : 4];
+  __shared__ __attribute__((aligned(16))) uint16_t sh_p[SRC == SEL_SCORE && !OWN ? IDS * GSM : 8];
   __shared__ float sh_a[SRC == SEL_SCORE ? NW : 1][16], sh_b[SRC == SEL_SCORE ? NW : 1][16];
   __shared__ __attribute__((aligned(16))) uint4 sh_rows[SRC == SEL_SCORE ? NW : 1][SRC == SEL_SCORE ? 256 : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -131,6 +138,12 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   if (tid < 128) sh_fine[tid >> 6][lane] = 0u;
   if (tid < 3) sh_tot[tid] = 0u;
   sh_ret[tid] = 0u;
+
+  int32_t own_size = 0, own_row = 0;
+  if (STAGED && P.cluster_size) {
+    own_size = P.cluster_size[(size_t)g * nc + min(tid, nc - 1)];
+    if (P.cluster_start) own_row = P.cluster_start[(size_t)g * nc + min(tid, nc - 1)];
+  }
 
   // ---- this thread's keys, two per word ----
   uint32_t kw[(E + 1) / 2];
@@ -203,8 +216,24 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
         sh_a[wave][r] = lmax;
         sh_b[wave][r] = lsum;
       }
+      // The products leave a cluster's heads to neighbouring lanes: with up to eight of them half of the lanes or more have
+      // nothing, so the scores go through LDS to the thread that owns the cluster, which computes gs probabilities (8 groups
+      // of 4 heads, 512 clusters with the sizes at hand: 7.9 -> 7.7 us, 256: 6.9 -> 6.6); with more heads the lanes that have
+      // the scores compute sixteen each (8 groups of 12: 8.4, the other way 9.3).
+      float* const xs = KEEP ? K.logits : sh_x;   // [cluster][GSM]
+      if (OWN) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int c = 16 * (wave + NW * t) + 4 * h;
+          if (r < gs && c < nc)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) xs[(c + i) * GSM + r] = acc[t][i];
+        }
+      }
+      sh_size[tid] = own_size;
+      sh_row[tid] = own_row;
       lds_barrier();
-      float m = sh_a[0][r], z = 0.f;
+      float m = sh_a[0][r], z = 0.f;   // of head r
 #pragma unroll
       for (int w = 1; w < NW; ++w) m = fmaxf(m, sh_a[w][r]);
 #pragma unroll
@@ -213,25 +242,39 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
         z += (mw == -INFINITY) ? 0.f : sh_b[w][r] * __expf(mw - m);   // a wave past the last centroid holds nothing
       }
       const float iz = 1.0f / z;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int c = 16 * (wave + NW * t) + 4 * h;
-        if (r < gs && c < nc) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            sh_p[(c + i) * GSM + r] = ri_f32_to_e16<HALF>(__expf(ri_round_e16<HALF>(acc[t][i]) - m) * iz);
-          if (KEEP)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) K.logits[(c + i) * GSM + r] = acc[t][i];
-          *reinterpret_cast<f32x4_t*>(P.logits + ((size_t)g * gs + r) * nc + c) = acc[t];
-        }
-      }
-      lds_barrier();
       d[0] = 0.f;
+      if constexpr (OWN) {
+        float x[GSM];
 #pragma unroll
-      for (int j = 0; j < GSM; ++j) {
-        const float p = ri_e16_to_f32<HALF>(sh_p[cc * GSM + j]);
-        d[0] += j < gs ? p : 0.f;
+        for (int j = 0; j < GSM; j += 4) {
+          const float4 v = *reinterpret_cast<const float4*>(xs + cc * GSM + j);
+          x[j] = v.x; x[j + 1] = v.y; x[j + 2] = v.z; x[j + 3] = v.w;
+        }
+#pragma unroll
+        for (int j = 0; j < GSM; ++j) {
+          if (j >= gs) break;   // uniform
+          const float mj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), j));
+          const float izj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iz), j));
+          d[0] += ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[j]) - mj) * izj);
+          if (cbeg < nc) P.logits[((size_t)g * gs + j) * nc + cbeg] = x[j];
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int c = 16 * (wave + NW * t) + 4 * h;
+          if (r < gs && c < nc) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              sh_p[(c + i) * GSM + r] = ri_f32_to_e16<HALF>(__expf(ri_round_e16<HALF>(acc[t][i]) - m) * iz);
+            *reinterpret_cast<f32x4_t*>(P.logits + ((size_t)g * gs + r) * nc + c) = acc[t];
+          }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < GSM; ++j) {
+          const float p = ri_e16_to_f32<HALF>(sh_p[cc * GSM + j]);
+          d[0] += j < gs ? p : 0.f;
+        }
       }
     } else {
       constexpr int V = E < 4 ? E : 4;   // columns per load
@@ -405,20 +448,20 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   const auto id_of = [](uint32_t pair) { return (int)(0xffffu - (pair & 0xffffu)); };
   // (the sizes and first rows are requested for the unsorted entries, so that the loads behind the sort find them near)
   int32_t warm_size = 0, warm_start = 0;
-  if (in && P.cluster_size) {
+  if (!STAGED && in && P.cluster_size) {
     warm_size = P.cluster_size[(size_t)g * nc + id_of(v)];
     if (P.cluster_start) warm_start = P.cluster_start[(size_t)g * nc + id_of(v)];
   }
   int n = 64;
   while (n < np) n <<= 1;
   block_sort_desc<LOGT>(v, n, hist);
-  asm volatile("" : : "v"(warm_size), "v"(warm_start));
+  if (!STAGED) asm volatile("" : : "v"(warm_size), "v"(warm_start));
   const int my_c = id_of(v);
   uint32_t sz = 0;
   int32_t st = 0;
   if (in && P.cluster_size) {
-    sz = (uint32_t)P.cluster_size[(size_t)g * nc + my_c];
-    if (P.cluster_start) st = P.cluster_start[(size_t)g * nc + my_c];
+    sz = (uint32_t)(STAGED ? sh_size[my_c] : P.cluster_size[(size_t)g * nc + my_c]);
+    if (P.cluster_start) st = STAGED ? sh_row[my_c] : P.cluster_start[(size_t)g * nc + my_c];
   }
 
   // ---- token layout of the retrieved clusters with the page cut-off ----
