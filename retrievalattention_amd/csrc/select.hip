@@ -499,10 +499,13 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   // One compute unit reads 20 KB per microsecond from memory and up to 100 from its L2.  Its own scoring therefore pays up to
   // 512 clusters (8 groups of 4 heads: 8.0 us; 640 clusters 10.3 against 10.0 for two launches, 16 groups of 1024 11.8
   // against 10.7; for 128 groups of 8 heads it is still ahead there, 14.0 against 16.0, but not by what the rule would
-  // cost), its own score sums up to about 112 KB of logits (8 groups of 4 heads, 4096 clusters: 14.4 against 15.5 us; 32 groups of
-  // 4 heads, 8192 clusters: 26.7 against 26.1).  Past 4096 clusters a thread holds eight of them: with more than four
-  // heads that is 64 logits in registers, and many compute units are the faster ones again (4 .. 32 groups of 5 and 6
-  // heads, 4104 .. 5728 clusters: 16.1 .. 22.6 us with dist_kernel, 20.0 .. 26.2 without).
+  // cost), its own score sums up to about 112 KB of logits of up to four heads (8 groups of 4, 4096 clusters: 14.4 against
+  // 15.5 us; 32 groups of 4, 7168 clusters 24.5 either way, 8192 28.1 against 27.4; one head, 8192 clusters 16.3 against
+  // 17.3).  Past 4096 clusters a thread holds eight of them: with more than four heads that is 64 logits in registers, and
+  // many compute units are the faster ones again (4 .. 32 groups of 5 and 6 heads, 4104 .. 5728 clusters: 16.1 .. 22.6 us
+  // with dist_kernel, 20.0 .. 26.2 without; 8 heads, 4096 clusters 15.9 without, 16.4 with); so it is past 2048 with more
+  // than eight (8 groups of 9 heads, 3000 clusters 16.2 us with dist_kernel, 18.3 without; 16 of 16, 2048 16.6 without,
+  // 17.7 with).
   if (nc <= 512) {
     if (nc <= 256) launch_select_heads<256, 1, SEL_SCORE>(P, BG, half, s);
     else launch_select_heads<512, 1, SEL_SCORE>(P, BG, half, s);
@@ -511,7 +514,7 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   }
   rc = ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, scale, half, s);
   if (rc) return rc;
-  if (nc * gs <= 28 * 1024 && nc <= (gs <= 4 ? 8192 : 4096) && np <= SEL_THREADS) {
+  if (nc <= (gs <= 4 ? min(8192, 28 * 1024 / gs) : gs <= 8 ? 4096 : 2048) && np <= SEL_THREADS) {
     // as few waves as the clusters and the probes leave room for: what a wave does once costs all of them
     if (nc <= 1024 && np <= 512) launch_select_heads<512, 2, SEL_LOGITS>(P, BG, half, s);
     else if (nc <= 2048 && np <= 512) launch_select_heads<512, 4, SEL_LOGITS>(P, BG, half, s);
