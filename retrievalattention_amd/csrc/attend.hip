@@ -29,7 +29,7 @@
 
 template <int GS_PAD, bool HALF>
 __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams P) {
-  attend_group<GS_PAD, HALF, false>(P, blockIdx.y, blockIdx.x, AttendKept{});
+  attend_group<GS_PAD, HALF, false>(P, blockIdx.x, blockIdx.y, AttendKept{});
 }
 
 // ------------------------------------------------------------------------------------
@@ -70,7 +70,10 @@ static void launch_attend_t(const AttendParams& P, dim3 grid, int gp, size_t tab
 }
 
 static int launch_attend(AttendParams& P, int BG, int gs, bool half, hipStream_t s) {
-  const dim3 grid(P.S, BG);
+  // Groups vary fastest: workgroups go to the eight chiplets in turn, and with eight splits that vary fastest the chiplets
+  // of the last ones have estimation rows only, the others none (32 groups of 16 heads over 4096 clusters 15.2 -> 13.9 us, of
+  // 4 over 1024 8.5 -> 8.2, of 8 over 16384 26.6 -> 25.9; elsewhere up to 2 %).
+  const dim3 grid(BG, P.S);
   const size_t tab_bytes = P.ret_off ? (size_t)(2 * P.np + 1) * sizeof(int) : 0;
   if (half) launch_attend_t<true>(P, grid, gs_pad_of(gs), tab_bytes, s);
   else launch_attend_t<false>(P, grid, gs_pad_of(gs), tab_bytes, s);
@@ -94,6 +97,9 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 //    one to arrive reads the partials of all of them at that same rate: the sum of both is least near
 //    sqrt(bytes of the group / bytes of a partial), flat towards fewer (12 groups of 7 heads, 3550 rows: 15 workgroups
 //    11.6 us, 21: 12.0).
+//  * The last one reads the partials eight at a time, so one or two past a multiple of eight cost a round trip: 9 -> 8
+//    workgroups 8.5 -> 7.9 us (16 groups of 4 heads, 623 rows), 17 -> 16 12.1 -> 11.5 (12 groups of 7, 3488), 25 -> 24 10.6 ->
+//    10.2 (4 of 4, 4350), 34 -> 32 14.1 -> 13.7 (2 of 8, 15100).  More than a fifth is not worth giving up.
 //  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
 //    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
 static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
@@ -103,6 +109,7 @@ static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int e
   per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
   per_group = min(per_group, (int64_t)max_splits);
+  if (per_group > 8 && per_group % 8 * 5 <= per_group) per_group -= per_group % 8;
   if (rows * gs_pad_of(gs) <= 384 * 4 || per_group < 1) per_group = 1;
   const int waves = (int)per_group * ATT_WAVES;
   P.S = (int)per_group;
