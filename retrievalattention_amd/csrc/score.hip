@@ -26,7 +26,7 @@ __device__ __forceinline__ uint16_t score_f32_to_16(float f) { return ri_f32_to_
 // Softmax partials of the 256 columns with one barrier: every wave reduces its own columns to a maximum and a
 // sum of exponentials relative to that maximum, and after the barrier one thread per head folds the wave pairs
 // (max of the maxima, sums rescaled by exp(m_w - M)).
-template <bool HALF, int TPW>
+template <bool HALF, int TPW, bool STREAM>
 __device__ __forceinline__ void score_body(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cent, float* __restrict__ logits,
     uint16_t* __restrict__ logits_bf16, float* __restrict__ tile_max, float* __restrict__ tile_sum,
@@ -125,11 +125,12 @@ __device__ __forceinline__ void score_body(
     if (r < gs && cbase < nc) {  // nc % 4 == 0, so the four columns are valid together
       const size_t o = ((size_t)g * gs + r) * nc + cbase;
       if (logits) {
-        // streaming store: the 4 MB of logits leave the cache as they are written instead of waiting, dirty,
-        // for the write-back at the end of the kernel (about 1 us per step at 32 groups of 8192 centroids)
+        // streaming store (STREAM): logits that leave the cache as they are written do not wait, dirty, for the write-back
+        // at the end of the kernel (about 1 us per step at 32 groups of 8192 centroids)
         typedef float score_f4 __attribute__((ext_vector_type(4)));
         const score_f4 val = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
-        __builtin_nontemporal_store(val, reinterpret_cast<score_f4*>(logits + o));
+        if (STREAM) __builtin_nontemporal_store(val, reinterpret_cast<score_f4*>(logits + o));
+        else *reinterpret_cast<score_f4*>(logits + o) = val;
       }
       if (logits_bf16) {
         uint2 pk;
@@ -141,12 +142,12 @@ __device__ __forceinline__ void score_body(
   }
 }
 
-template <bool HALF, int TPW>
+template <bool HALF, int TPW, bool STREAM>
 __global__ __launch_bounds__(1024 / TPW) void score_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cent, float* __restrict__ logits,
     uint16_t* __restrict__ logits16, float* __restrict__ tile_max, float* __restrict__ tile_sum,
     int gs, int nc, int ntiles, float scale) {
-  score_body<HALF, TPW>(q, cent, logits, logits16, tile_max, tile_sum, gs, nc, ntiles, scale);
+  score_body<HALF, TPW, STREAM>(q, cent, logits, logits16, tile_max, tile_sum, gs, nc, ntiles, scale);
 }
 
 // Row statistics and softmax, a workgroup per row: every wave reduces the row's partials, with the workgroup's first 8
@@ -202,7 +203,7 @@ static int batch_gemm_softmax_impl(const void* A, const void* B, void* D, float*
   const int ntiles = (n + SCORE_TILE - 1) / SCORE_TILE;
   // fp32 logits are not part of this interface: the partial statistics come from the fp32
   // accumulators inside the kernel, the softmax from the 16-bit D, as in the reference.
-  score_kernel<HALF, 4><<<dim3(ntiles, batch_count), 256, 0, s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
+  score_kernel<HALF, 4, false><<<dim3(ntiles, batch_count), 256, 0, s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
                                                                   (uint16_t*)D, Norm, Sum, m, n, ntiles, alpha);
   RI_HIP_CHECK_LAUNCH();
   const int threads = min(1024, (n / 8 + 63) / 64 * 64);
@@ -230,12 +231,13 @@ int ri_launch_score(const void* q, const void* centroids, float* logits, float* 
                     int BG, int gs, int nc, float scale, bool half, hipStream_t s) {
   const int ntiles = (nc + SCORE_TILE - 1) / SCORE_TILE;
   const uint16_t *qq = (const uint16_t*)q, *cc = (const uint16_t*)centroids;
-  if (half)
-    score_kernel<true, 4><<<dim3(ntiles, BG), 256, 0, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc,
-                                                           ntiles, scale);
-  else
-    score_kernel<false, 4><<<dim3(ntiles, BG), 256, 0, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc,
-                                                            ntiles, scale);
+  // Up to 32 MB of centroids the logits are better left where the next kernels find them (whole steps: 8 groups of 8 heads,
+  // 4096 centroids 25.9 -> 25.0 us, 16 of 16, 2048 32.0 -> 30.9, 12 of 7, 1856 24.8 -> 24.4; 16 of 4, 8192 34.7 either way);
+  // with more the write-back is longer than that (32 of 4, 8192 46.1 streamed, 46.4 not).
+  const bool stream = (size_t)BG * nc > 128 * 1024;
+  auto* kernel = half ? (stream ? score_kernel<true, 4, true> : score_kernel<true, 4, false>)
+                      : (stream ? score_kernel<false, 4, true> : score_kernel<false, 4, false>);
+  kernel<<<dim3(ntiles, BG), 256, 0, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc, ntiles, scale);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
