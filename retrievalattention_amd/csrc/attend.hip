@@ -99,7 +99,8 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 //    11.6 us, 21: 12.0).
 //  * The last one reads the partials eight at a time, so one or two past a multiple of eight cost a round trip: 9 -> 8
 //    workgroups 8.5 -> 7.9 us (16 groups of 4 heads, 623 rows), 17 -> 16 12.1 -> 11.5 (12 groups of 7, 3488), 25 -> 24 10.6 ->
-//    10.2 (4 of 4, 4350), 34 -> 32 14.1 -> 13.7 (2 of 8, 15100).  More than a fifth is not worth giving up.
+//    10.2 (4 of 4, 4350), 34 -> 32 14.1 -> 13.7 (2 of 8, 15100).  More than a fifth is not worth giving up, nor
+//    any of them once a wave has more than four chunks (24 groups of 3, 24200 rows: 10 -> 8 took 1.5 % of the step).
 //  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
 //    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
 static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
@@ -109,7 +110,7 @@ static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int e
   per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
   per_group = min(per_group, (int64_t)max_splits);
-  if (per_group > 8 && per_group % 8 * 5 <= per_group) per_group -= per_group % 8;
+  if (per_group > 8 && per_group % 8 * 5 <= per_group && rows <= 64 * ATT_WAVES * per_group) per_group -= per_group % 8;
   if (rows * gs_pad_of(gs) <= 384 * 4 || per_group < 1) per_group = 1;
   const int waves = (int)per_group * ATT_WAVES;
   P.S = (int)per_group;
