@@ -875,6 +875,9 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 // it ten; 8 x 8192 tokens, 512 clusters: 10.6 -> 9.6 us; 128 x 8192: 67.6 -> 61.6).  Requests beside the additions instead
 // of U rows at a time, nine updates of Lloyd iterations together: 128 x 8192 tokens 543 -> 517 us (half 626 -> 512, where
 // 80 registers instead of 82 also make room for a third workgroup), 24 x 8119 183 -> 175 (216 -> 166), 8 x 8192 107 -> 104.
+// The offsets of eight rows are read from the lanes before the additions that free their registers: a load right behind
+// the readlane that makes its offset waits five issues for it (the same nine updates 101 -> 99, 128 x 8192 507 -> 503, 4 x
+// 15000 tokens, 928 clusters 155 -> 145).
 // WHOLE: two dims per lane, else one (two waves share the row).
 template <bool HALF, int U, bool WHOLE>
 __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint32_t byte, const uint16_t* list, int k0, int k1,
@@ -886,15 +889,22 @@ __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint3
     else ri_add_lo<HALF>(w, s0);
   };
   uint32_t v[U];
-  int off;
+  int off, so[8];
   const auto ids = [&](int k) { off = (int)list[min(k + lane, k1 - 1)] * (RI_DIM * 2); };
-  const auto fetch = [&](int e) {
+  const auto offsets = [&](int e) {
 #pragma unroll
-    for (int j = e; j < e + 8; ++j) {
-      const int so = __builtin_amdgcn_readlane(off, j);
-      v[j] = WHOLE ? __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so, 0)
-                   : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, byte, so, 0);
-    }
+    for (int j = 0; j < 8; ++j) so[j] = __builtin_amdgcn_readlane(off, e + j);
+  };
+  const auto request = [&](int e) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[e + j] = WHOLE ? __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so[j], 0)
+                       : (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rows, byte, so[j], 0);
+  };
+  const auto fetch = [&](int e) {
+    offsets(e);
+    __builtin_amdgcn_sched_barrier(0);
+    request(e);
   };
   const auto add8 = [&](int e) {
 #pragma unroll
@@ -923,8 +933,11 @@ __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint3
       ids(k);
 #pragma unroll
       for (int e = 0; e < U; e += 8) {
+        offsets(e);
+        __builtin_amdgcn_sched_barrier(0);   // (else each goes to the load it is for)
         add8(e);
-        fetch(e);
+        __builtin_amdgcn_sched_barrier(0);
+        request(e);
         __builtin_amdgcn_sched_barrier(0);   // (else the next loads move up, into registers of their own)
       }
     } while (k + U < k1);
