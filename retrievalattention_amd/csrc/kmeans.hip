@@ -856,11 +856,15 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 // grid km_grid(ceil(nc / CPW), P), eight waves: a workgroup owns CPW consecutive clusters.  Every wave takes a contiguous run of
 // the problem's tokens, compacts those of the workgroup's clusters into LDS (in token order), counts them, and after a
 // scan in (cluster, wave) order scatters them to the workgroup's list in LDS, ranking equal clusters inside a round of 64
-// with ballots: the stable order of the list kernels, hence the same sums.  Then a wave sums whole clusters of at most
+// with ballots: the stable order of the list kernels, hence the same sums.  The run is read four tokens to a lane, up to
+// 1024 requested at once; a token costs three instructions (its cluster in a byte, all others' flagged), positions come
+// from one wave scan per 512 and only the few hits are looped over.  A ballot, a rank and a branch for every 64 tokens
+// were most of a late update: 8 x 8192 tokens, 512 clusters 8.2 -> 7.5 us, 4 x 15000, 928 clusters 10.8 -> 9.2, 1 x 16384
+// 8.5 -> 6.9, 128 x 8192 52.0 -> 49.8.  Then a wave sums whole clusters of at most
 // KM_BLK rows; the blocks of longer ones are spread over the waves and folded in block order.
 // Reading all assignments of the problem per workgroup (4 N bytes) is what the split costs: 32 KB at 8192 tokens, about a
-// microsecond.  128 x 8192 tokens, 512 clusters each: 56 us, bound by reading the keys, against 13 + 70 + 5 us of list
-// sort, sums and fold; 8 x 8192: 9.6 us against 12 + 11 + 4.5.
+// microsecond.  128 x 8192 tokens, 512 clusters each: 50 us, bound by reading the keys, against 13 + 70 + 5 us of list
+// sort, sums and fold; 8 x 8192: 7.5 us against 12 + 11 + 4.5.
 // counts / offsets / members (CSR, as km_sort_small_kernel writes them) only when asked for, and then alone if there is
 // no `cent`: the last pass of a prefill, whose means come with the stores (8 x 8192 tokens, whole prefill 367 -> 363 us).
 // ------------------------------------------------------------------------------------
@@ -950,65 +954,104 @@ __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint3
   }
 }
 
+// four consecutive assignments; a problem's first one lies on four bytes only
+typedef int32_t km_quad __attribute__((ext_vector_type(4), aligned(4)));
+// tokens of a wave's run: whole quads of 64 lanes
+__host__ __device__ constexpr int km_direct_run(int N) {
+  return (N + KM_DIRECT_WAVES * 256 - 1) / (KM_DIRECT_WAVES * 256) * 256;
+}
+
 template <bool HALF, int CPW>
 __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
     const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
     int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int seg,
     int64_t head_rows, int normalize, int sh) {
-  constexpr int NW = KM_DIRECT_WAVES, SLOTS = CPW * NW;
-  static_assert(SLOTS <= NW * 64, "one (cluster, wave) counter per thread");
-  __shared__ int32_t sh_run[NW][CPW], sh_off[CPW + 1], sh_w[NW], sh_below[NW];
-  extern __shared__ __attribute__((aligned(16))) uint32_t sh_buf[];   // rounds * 512 words: compacted tokens, later block sums
+  constexpr int NW = KM_DIRECT_WAVES, E = CPW * NW / 64;   // E: (cluster, wave) counters per lane
+  static_assert((CPW & (CPW - 1)) == 0 && CPW * NW % 64 == 0 && CPW <= 64, "counters dealt to the lanes, a cluster in a byte");
+  __shared__ int32_t sh_run[CPW * NW], sh_at[NW][CPW], sh_off[CPW + 1], sh_below[NW];
+  extern __shared__ __attribute__((aligned(16))) uint32_t sh_buf[];   // NW * run_len words: compacted tokens, later block sums
   // (last problem first: its keys are what the assignment pass has just left in the memory-side cache)
   const int p = ((gridDim.y - 1 - blockIdx.y) << sh) + (blockIdx.x & ((1 << sh) - 1)), c0 = (blockIdx.x >> sh) * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rounds = (N + NW * 64 - 1) / (NW * 64);   // 64-token rounds per wave
-  uint32_t* const mine = sh_buf + wave * rounds * 64;
-  uint16_t* const list = reinterpret_cast<uint16_t*>(sh_buf + NW * rounds * 64);
-  int32_t* run = sh_run[wave];
-  if (lane < CPW) run[lane] = 0;
+  const int run_len = km_direct_run(N);
+  uint32_t* const mine = sh_buf + wave * run_len;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(sh_buf + NW * run_len);
+  if (lane < CPW) sh_run[lane * NW + wave] = 0;
   km_wave_lds_sync();
   const int32_t* as = assign + (size_t)p * N;
-  int cnt = 0, below = 0;   // tokens of this wave in the workgroup's clusters, in lower ones
-  for (int r0 = 0; r0 < rounds; r0 += 8) {
-    int32_t a[8];
+  const int t1 = min((wave + 1) * run_len, N);
+  int cnt = 0, below = 0;   // tokens of this wave in the workgroup's clusters, (per lane) in lower ones
+  for (int t0 = wave * run_len; t0 < t1; t0 += 1024) {
+    // four quads of consecutive tokens per lane, all requested before the first is looked at
+    km_quad a[4];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] = as[min((wave * rounds + r0 + u) * 64 + lane, N - 1)];
+    for (int q = 0; q < 4; ++q) {
+      const int i = t0 + q * 256 + lane * 4;
+      if (t0 + q * 256 + 256 <= t1) {
+        a[q] = *reinterpret_cast<const km_quad*>(as + i);
+      } else if (t0 + q * 256 < t1) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = (wave * rounds + r0 + u) * 64 + lane;
-      const bool ok = r0 + u < rounds && i < N;
-      const int loc = a[u] - c0;
-      const bool in = ok && (unsigned)loc < (unsigned)CPW;
-      const uint64_t m = __builtin_amdgcn_ballot_w64(in);
-      if (members) below += __popcll(__builtin_amdgcn_ballot_w64(ok && loc < 0));
-      if (in) {
-        mine[__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, cnt))] =
-            (uint32_t)loc << 16 | (uint32_t)i;
-        atomicAdd(&run[loc], 1);
+        for (int j = 0; j < 4; ++j) {
+          const int x = as[min(i + j, N - 1)];
+          a[q][j] = i + j < t1 ? x : 0x7fffffff;
+        }
+      } else {
+        a[q] = km_quad(0x7fffffff);
       }
-      cnt += __popcll(m);
     }
-  }
-  if (lane == 0) sh_below[wave] = below;
-  __syncthreads();
-  {   // exclusive scan in (cluster, wave) order
-    const int c = tid / NW, w = tid % NW;
-    const int v = tid < SLOTS ? sh_run[w][c] : 0;
-    const int inc = (int)ri_wave_incl_scan((uint32_t)v);
-    if (lane == 63) sh_w[wave] = inc;
-    __syncthreads();
-    int ex = inc - v;
 #pragma unroll
-    for (int x = 0; x < NW; ++x)
-      if (x < wave) ex += sh_w[x];
-    if (tid < SLOTS) {
-      sh_run[w][c] = ex;
-      if (w == 0) sh_off[c] = ex;
-      if (tid == SLOTS - 1) sh_off[CPW] = ex + v;
+    for (int q0 = 0; q0 < 4; q0 += 2) {
+      if (t0 + q0 * 256 >= t1) break;
+      uint32_t loc[2], hit[2], at[2];   // a byte per token: its cluster from c0 on, CPW for all others
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        loc[q] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t d = (uint32_t)(a[q0 + q][j] - c0);
+          loc[q] |= min(d, (uint32_t)CPW) << (8 * j);
+          if (members) below += (int)(d >> 31);
+        }
+        hit[q] = ~loc[q] & (uint32_t)CPW * 0x01010101u;
+      }
+      // positions of a lane's first hits in both quads, in one scan (at most 256 each)
+      const uint32_t n = (uint32_t)__popc(hit[0]) | (uint32_t)__popc(hit[1]) << 16, inc = ri_wave_incl_scan(n);
+      const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+      at[0] = cnt + ((inc - n) & 0xffffu);
+      at[1] = cnt + (int)(all & 0xffffu) + ((inc - n) >> 16);
+      cnt += (int)(all & 0xffffu) + (int)(all >> 16);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        for (uint32_t h = hit[q]; h; h &= h - 1) {
+          const int j = (__ffs((int)h) - 1) >> 3;
+          const uint32_t c = loc[q] >> (8 * j) & (uint32_t)(CPW - 1);
+          mine[at[q]++] = c << 16 | (uint32_t)(t0 + (q0 + q) * 256 + lane * 4 + j);
+          atomicAdd(&sh_run[c * NW + wave], 1);
+        }
+      }
     }
   }
+  if (members) {
+    below = (int)ri_wave_incl_scan((uint32_t)below);
+    if (lane == 63) sh_below[wave] = below;
+  }
   __syncthreads();
+  int32_t* const run = sh_at[wave];
+  {   // exclusive scan in (cluster, wave) order; every wave makes it, and keeps the positions of its own tokens
+    int v[E], sum = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) sum += v[e] = sh_run[lane * E + e];
+    int ex = (int)ri_wave_incl_scan((uint32_t)sum) - sum;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int c = (lane * E + e) / NW, w = (lane * E + e) % NW;
+      if (w == wave) run[c] = ex;
+      if (w == 0 && wave == 0) sh_off[c] = ex;
+      ex += v[e];
+    }
+    if (wave == 0 && lane == 63) sh_off[CPW] = ex;
+  }
+  km_wave_lds_sync();
   const uint64_t lower = (1ull << lane) - 1ull;
   for (int k = 0; k < cnt; k += 64) {
     const bool ok = k + lane < cnt;
@@ -1318,9 +1361,8 @@ template <bool HALF>
 static int km_direct_launch(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
                             int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize,
                             ri_stream_t stream) {
-  const int rounds = (N + KM_DIRECT_WAVES * 64 - 1) / (KM_DIRECT_WAVES * 64);
   // tokens compacted (4 bytes) and listed (2 bytes); block sums of a long cluster (512 bytes per KM_BLK rows) fit there too
-  const size_t lds = (size_t)rounds * KM_DIRECT_WAVES * 64 * 6 + 512;
+  const size_t lds = (size_t)km_direct_run(N) * KM_DIRECT_WAVES * 6 + 512;
 #define KM_DIRECT_LAUNCH(CPW)                                                                                         \
   do {                                                                                                                \
     km_direct_kernel<HALF, CPW><<<km_grid((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>( \
@@ -1329,8 +1371,9 @@ static int km_direct_launch(const void* data, const int32_t* assign, void* centr
   } while (0)
   // As many workgroups as are resident at once (four of 512 threads, as many as the LDS of a compute unit holds): more
   // of them read the assignments more often and wait for a second round (24 x 8119 tokens, 512 clusters each: 8
-  // clusters per workgroup 20.1 us, 16: 16.2, 32: 19.0; 8 x 8192: 8 clusters 9.6, 64: 21.6; 128 x 8192: 32 clusters
-  // 57.6, 64: 61.2, 16: 66.9).
+  // clusters per workgroup 15.6 us, 16: 13.3, 32: 14.9; 8 x 8192: 7.5, 7.8, 10.3; 128 x 8192: 68.3, 53.3, 49.8).  Sixteen
+  // waves for 16 clusters where eight have too few workgroups: late updates 7.5 -> 7.2, early ones 14.0 -> 17.5 (two
+  // long lists in one workgroup wait for one compute unit's cache), so not taken.
   const long long resident = 256 * (long long)min((size_t)4, (160 * 1024) / (lds + 2560));
   const auto fits = [&](int cpw) { return (long long)P * ((nc + cpw - 1) / cpw) <= resident; };
   if (fits(8)) KM_DIRECT_LAUNCH(8);

@@ -391,3 +391,12 @@ def test_update_direct_equals_lists_and_update(dev, P, N, nc, kind):
             assert torch.equal(x, y)
     with pytest.raises(RuntimeError):
         kernels.kmeans_update_direct(rows, a, cent, P, kernels.KMEANS_DIRECT_MAX_TOKENS + 1, nc, 1, N, True)
+
+
+# Ends of the runs that the eight waves read four tokens to a lane (256, 512 and 1024 at a time, run lengths in 256s), rows
+# of assignments that begin on four bytes only, and the three widths of a workgroup (by the number of problems).
+@pytest.mark.parametrize("P", [1, 20, 70])
+@pytest.mark.parametrize("N", [3, 255, 257, 511, 1025, 2047, 2049, 4095, 4099, 6145, 8193])
+def test_update_direct_at_the_ends_of_runs(dev, P, N):
+    for kind in ("even", "skew"):
+        test_update_direct_equals_lists_and_update(dev, P, N, 512, kind)
