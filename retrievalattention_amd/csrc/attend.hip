@@ -27,8 +27,24 @@
 #include "attend_common.h"
 #include "ri_common.h"
 
+// (what the first loads want stands before the struct: in registers at the start; 32 groups of 4 heads over 8192 clusters 16.5
+// -> 16.3 us, 12 groups of 7 heads over 1856 in half 9.34 -> 9.14)
 template <int GS_PAD, bool HALF>
-__global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(AttendParams P) {
+__global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(const int32_t* ret_off, const int32_t* ret_start,
+                                                                   const int32_t* lenB_ptr, const uint16_t* q, int np, int gs,
+                                                                   int S, int W_kv, int lenB_ptr_stride, int lenA,
+                                                                   AttendParams A) {
+  AttendParams P = A;
+  P.ret_off = ret_off;
+  P.ret_start = ret_start;
+  P.lenB_ptr = lenB_ptr;
+  P.q = q;
+  P.np = np;
+  P.gs = gs;
+  P.S = S;
+  P.W_kv = W_kv;
+  P.lenB_ptr_stride = lenB_ptr_stride;
+  P.lenA = lenA;
   attend_group<GS_PAD, HALF, false>(P, blockIdx.x, blockIdx.y, AttendKept{});
 }
 
@@ -64,9 +80,9 @@ static void carve_workspace(AttendParams& P, void* workspace, int BG, int gp) {
 
 template <bool HALF>
 static void launch_attend_t(const AttendParams& P, dim3 grid, int gp, size_t tab_bytes, hipStream_t s) {
-  if (gp == 4) attend_kernel<4, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
-  else if (gp == 8) attend_kernel<8, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
-  else attend_kernel<16, HALF><<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P);
+  auto* kernel = gp == 4 ? attend_kernel<4, HALF> : gp == 8 ? attend_kernel<8, HALF> : attend_kernel<16, HALF>;
+  kernel<<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P.ret_off, P.ret_start, P.lenB_ptr, P.q, P.np, P.gs, P.S, P.W_kv,
+                                                 P.lenB_ptr_stride, P.lenA, P);
 }
 
 static int launch_attend(AttendParams& P, int BG, int gs, bool half, hipStream_t s) {

@@ -429,8 +429,30 @@ __global__ __launch_bounds__(SEL_THREADS) void select_kernel(
   }
 }
 
+// What the first loads want stands before the struct: those arguments are in registers at the start (32 groups of 4 heads over
+// 8192 clusters, with the attention's: a step 44.5 -> 43.9 us; 16 groups, 1024 clusters 17.7 -> 17.3; 12 of 7 heads, 1856
+// clusters in half 20.6 -> 20.2).
 template <int NT, int E, int GSM, bool HALF, int SRC>
-__global__ __launch_bounds__(NT) void select_radix_kernel(SelectArgs P) {
+__global__ __launch_bounds__(NT) void select_radix_kernel(const void* a, const void* b, const void* c,
+                                                          const uint8_t* mask, int nc, int gs, int np, int es, int ntiles,
+                                                          SelectArgs A) {
+  SelectArgs P = A;
+  if (SRC == SEL_KEYS) {
+    P.keys = (uint16_t*)a;
+  } else if (SRC == SEL_LOGITS) {
+    P.logits = (float*)a;
+    P.tile_max = (float*)b;
+    P.tile_sum = (float*)c;
+  } else {
+    P.cent = (const uint16_t*)a;
+    P.q = (const uint16_t*)b;
+  }
+  P.mask = mask;
+  P.nc = nc;
+  P.gs = gs;
+  P.np = np;
+  P.es = es;
+  P.ntiles = ntiles;
   select_group<NT, E, GSM, HALF, SRC, false>(P, blockIdx.x, SelectKept{});
 }
 
@@ -447,8 +469,10 @@ extern "C" size_t ri_score_select_workspace_bytes(int BG, int gs, int nc) {
 
 template <int NT, int E, int GSM, int SRC>
 static void launch_select(const SelectArgs& P, int BG, bool half, hipStream_t s) {
-  if (half) select_radix_kernel<NT, E, GSM, true, SRC><<<BG, NT, 0, s>>>(P);
-  else select_radix_kernel<NT, E, GSM, false, SRC><<<BG, NT, 0, s>>>(P);
+  const void* a = SRC == SEL_KEYS ? (const void*)P.keys : SRC == SEL_LOGITS ? (const void*)P.logits : (const void*)P.cent;
+  const void* b = SRC == SEL_LOGITS ? (const void*)P.tile_max : (const void*)P.q;
+  auto* kernel = half ? select_radix_kernel<NT, E, GSM, true, SRC> : select_radix_kernel<NT, E, GSM, false, SRC>;
+  kernel<<<BG, NT, 0, s>>>(a, b, P.tile_sum, P.mask, P.nc, P.gs, P.np, P.es, P.ntiles, P);
 }
 template <int NT, int E, int SRC>
 static void launch_select_heads(const SelectArgs& P, int BG, bool half, hipStream_t s) {
