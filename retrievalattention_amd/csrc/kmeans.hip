@@ -199,6 +199,20 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
       km_wait_vm<(KM_NB - 2) * L>();   // this tile's loads of this wave have landed ...
       asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
       tile_load(ct + (KM_NB - 1) * KM_CT, buf == 0 ? KM_NB - 1 : buf - 1);
+      // Operands from LDS: each is requested AHEAD products before its own, into the register that a product has just read, across
+      // sub-tiles where a tile has several.  (The compiler has two on their way and waits for each; as many more as the
+      // registers hold.  8 x 8192 tokens, 512 centroids: 10.2 -> 9.3 us, 16 x 8200 22.4 -> 20.7, 4 x 48719, 3072 119 -> 118,
+      // 128 x 8192 120.6 -> 117.6, 8 x 131072, 8192 1531 -> 1512.)
+      constexpr int AHEAD = KM_TT == 2 ? 3 : KM_CT == 32 ? 0 : KM_TT == 4 ? 4 : 8;
+      uint4 rows[AHEAD ? AHEAD : 1];
+      const auto operand = [&](int at) {
+        return *reinterpret_cast<const uint4*>(row_at[at % 8] + (buf * KM_CT + at / 8 * 32) * RI_DIM);
+      };
+      if (AHEAD) {
+#pragma unroll
+        for (int kk = 0; kk < AHEAD; ++kk) rows[kk] = operand(kk);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int half = 0; half < KM_CT / 32; ++half) {
         if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
@@ -209,13 +223,18 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
             for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
 #pragma unroll
           for (int kk = 0; kk < 8; ++kk) {
-            const uint4 a = *reinterpret_cast<const uint4*>(row_at[kk] + (buf * KM_CT + half * 32) * RI_DIM);
+            const int at = half * 8 + kk;
+            const uint4 a = AHEAD ? rows[at % (AHEAD ? AHEAD : 1)] : operand(at);
 #pragma unroll
             for (int tt = 0; tt < KM_TT; ++tt)
               acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
                                                                       __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
                              : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
                                                                        0, 0);
+            if (AHEAD) {
+              if (at + AHEAD < KM_CT / 4) rows[at % (AHEAD ? AHEAD : 1)] = operand(at + AHEAD);
+              __builtin_amdgcn_sched_barrier(0);
+            }
           }
           // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
           // equal to their maximum is the lowest row; the index search only runs when some lane
@@ -1211,23 +1230,26 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
   // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
   // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
-  // against 18.9 with two columns when they were compared, now 10.3; 2 x 1708 tokens, 96 centroids: 4.9 against 6.7).
+  // against 18.9 with two columns when they were compared, now 8.7 against 11.8; 2 x 1708 tokens, 96 centroids: 4.9
+  // against 6.7).
   if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
-  else if (wgs256 <= 512) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
-  // One workgroup per compute unit that gives each wave three or four columns, where the fullest unit has that many
-  // columns per wave to do anyway: the same work with more reuse of every LDS read (16 x 8200 tokens, 512 centroids: 25.8
-  // us against 28.7 for the last line's when they were compared; 4 x 48719, 3072: 124 against 135; 20 x 9757, 608: 37.8
-  // against 40.4; now 20.8, 121 and 33.6).
-  else if (nc >= 512 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
-  else if (nc >= 512 && wgs256 > 768 && wgs1024 <= 256) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
+  // A little more than those two per compute unit is a second round for a few: three columns per wave then do it in one
+  // round, the longer the loop the further (16 x 8200 tokens, 528 workgroups of one column, 512 centroids: 20.2 us against
+  // 21.0, 16 x 9200, 576: 23.6 against 22.9; 8 x 20000, 632, 1024: 39.8 against 40.4, 8 x 24000, 752: 44.9 against 43.7;
+  // 4 x 48719, 764, 3072: 115 against 118).
+  else if (nc >= 512 && wgs256 > 512 && wgs256 <= 440 + nc / 5 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
+  // (up to three of them: 22 x 8192 tokens, 512 centroids: 24.4 us against 25.4 with two columns, 26.5 with three; 24 x 8119:
+  // 25.2 against 25.7; 24 x 8192, 256: 16.4 either way; 28 x 8192: 30.8 against 30.0)
+  else if (wgs256 <= 768) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
   // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
-  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves, now 1532; 4 x 65536, 4096: 219
-  // against 232, now 202), provided the last round of these large workgroups is not mostly empty.
-  else if (nc > 1024 && wgs1024 * 100 >= rounds1024 * 256 * 87) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
-  // Otherwise the load of the tokens in front of the loop is a large part of the kernel, and 126 registers and 32 KB of
+  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves, now 1512; 4 x 61440, 3840: 177
+  // against 178 with two columns, 4 x 51000, 3200: 136 against 139, 4 x 65536, 2048: 104.2 against 102.7), provided the
+  // last round of these large workgroups is not mostly empty.
+  else if (nc > 2048 && (wgs1024 <= 256 || wgs1024 * 100 >= rounds1024 * 256 * 87)) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
+  // Otherwise the load of the tokens in front of the loop is a large part of the kernel, and 128 registers and 32 KB of
   // LDS let four workgroups per compute unit overlap one's loads with the others' products (128 x 8192 tokens, 512
-  // centroids: 114.8 us, four columns and tiles of 128: 140.5, of 32: 119.7, eight waves 118.3, three buffers 114.5, tiles
-  // of 64 116.3 and 124.9, three columns 131).
+  // centroids: 111.3 us, one column 124, four 130, three 142, two in eight waves and tiles of 128 136; 32 x 8192: 31.6,
+  // 32.7, 34.6, 43.9, 36.5).
   else KM_ASSIGN_LAUNCH(2, 32, 4, 4);
 #undef KM_ASSIGN_LAUNCH
   RI_HIP_CHECK_LAUNCH();
