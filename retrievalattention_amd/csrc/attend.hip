@@ -30,21 +30,18 @@
 // (what the first loads want stands before the struct: in registers at the start; 32 groups of 4 heads over 8192 clusters 16.5
 // -> 16.3 us, 12 groups of 7 heads over 1856 in half 9.34 -> 9.14)
 template <int GS_PAD, bool HALF>
-__global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(const int32_t* ret_off, const int32_t* ret_start,
-                                                                   const int32_t* lenB_ptr, const uint16_t* q, int np, int gs,
-                                                                   int S, int W_kv, int lenB_ptr_stride, int lenA,
-                                                                   AttendParams A) {
+__global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, ri_int4 n, ri_int2 len, AttendParams A) {
   AttendParams P = A;
-  P.ret_off = ret_off;
-  P.ret_start = ret_start;
-  P.lenB_ptr = lenB_ptr;
-  P.q = q;
-  P.np = np;
-  P.gs = gs;
-  P.S = S;
-  P.W_kv = W_kv;
-  P.lenB_ptr_stride = lenB_ptr_stride;
-  P.lenA = lenA;
+  P.ret_off = ri_global<const int32_t>(in[0]);
+  P.ret_start = ri_global<const int32_t>(in[1]);
+  P.lenB_ptr = ri_global<const int32_t>(in[2]);
+  P.q = ri_global<const uint16_t>(in[3]);
+  P.np = n[0];
+  P.gs = n[1];
+  P.S = n[2];
+  P.W_kv = n[3];
+  P.lenB_ptr_stride = len[0];
+  P.lenA = len[1];
   attend_group<GS_PAD, HALF, false>(P, blockIdx.x, blockIdx.y, AttendKept{});
 }
 
@@ -81,8 +78,8 @@ static void carve_workspace(AttendParams& P, void* workspace, int BG, int gp) {
 template <bool HALF>
 static void launch_attend_t(const AttendParams& P, dim3 grid, int gp, size_t tab_bytes, hipStream_t s) {
   auto* kernel = gp == 4 ? attend_kernel<4, HALF> : gp == 8 ? attend_kernel<8, HALF> : attend_kernel<16, HALF>;
-  kernel<<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(P.ret_off, P.ret_start, P.lenB_ptr, P.q, P.np, P.gs, P.S, P.W_kv,
-                                                 P.lenB_ptr_stride, P.lenA, P);
+  kernel<<<grid, 64 * ATT_WAVES, tab_bytes, s>>>(ri_pack_ptrs(P.ret_off, P.ret_start, P.lenB_ptr, P.q),
+                                                 (ri_int4){P.np, P.gs, P.S, P.W_kv}, (ri_int2){P.lenB_ptr_stride, P.lenA}, P);
 }
 
 static int launch_attend(AttendParams& P, int BG, int gs, bool half, hipStream_t s) {

@@ -218,6 +218,20 @@ __device__ __forceinline__ float ri_wave_sum(float x) {
   return ri_xor_sum<1>(ri_xor_sum<2>(ri_xor_sum<4>(ri_xor_sum<8>(ri_xor_sum<16>(ri_xor_sum<32>(x))))));
 }
 
+// Kernel arguments that are wanted at once: the first fourteen words are in registers when a wave starts, but none of a struct;
+// as vectors they are few arguments for the host to lay out (about 20 ns each).
+typedef uint64_t ri_ptr4 __attribute__((ext_vector_type(4)));
+typedef int ri_int4 __attribute__((ext_vector_type(4)));
+typedef int ri_int2 __attribute__((ext_vector_type(2)));
+// (through a global pointer: from an integer alone the compiler makes loads that ask where the address lies)
+template <typename T>
+__device__ __forceinline__ T* ri_global(uint64_t p) {
+  return (T*)(__attribute__((address_space(1))) T*)p;
+}
+static inline ri_ptr4 ri_pack_ptrs(const void* a, const void* b, const void* c, const void* d) {
+  return (ri_ptr4){(uint64_t)a, (uint64_t)b, (uint64_t)c, (uint64_t)d};
+}
+
 // ---- shared between score.hip and select.hip ----
 #define RI_SCORE_TILE 256          // centroids per softmax partial
 int ri_launch_score(const void* q, const void* centroids, float* logits, float* tile_max, float* tile_sum,

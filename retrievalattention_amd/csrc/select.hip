@@ -433,25 +433,23 @@ __global__ __launch_bounds__(SEL_THREADS) void select_kernel(
 // 8192 clusters, with the attention's: a step 44.5 -> 43.9 us; 16 groups, 1024 clusters 17.7 -> 17.3; 12 of 7 heads, 1856
 // clusters in half 20.6 -> 20.2).
 template <int NT, int E, int GSM, bool HALF, int SRC>
-__global__ __launch_bounds__(NT) void select_radix_kernel(const void* a, const void* b, const void* c,
-                                                          const uint8_t* mask, int nc, int gs, int np, int es, int ntiles,
-                                                          SelectArgs A) {
+__global__ __launch_bounds__(NT) void select_radix_kernel(ri_ptr4 in, ri_int4 n, int ntiles, SelectArgs A) {
   SelectArgs P = A;
   if (SRC == SEL_KEYS) {
-    P.keys = (uint16_t*)a;
+    P.keys = ri_global<uint16_t>(in[0]);
   } else if (SRC == SEL_LOGITS) {
-    P.logits = (float*)a;
-    P.tile_max = (float*)b;
-    P.tile_sum = (float*)c;
+    P.logits = ri_global<float>(in[0]);
+    P.tile_max = ri_global<float>(in[1]);
+    P.tile_sum = ri_global<float>(in[2]);
   } else {
-    P.cent = (const uint16_t*)a;
-    P.q = (const uint16_t*)b;
+    P.cent = ri_global<const uint16_t>(in[0]);
+    P.q = ri_global<const uint16_t>(in[1]);
   }
-  P.mask = mask;
-  P.nc = nc;
-  P.gs = gs;
-  P.np = np;
-  P.es = es;
+  P.mask = ri_global<const uint8_t>(in[3]);
+  P.nc = n[0];
+  P.gs = n[1];
+  P.np = n[2];
+  P.es = n[3];
   P.ntiles = ntiles;
   select_group<NT, E, GSM, HALF, SRC, false>(P, blockIdx.x, SelectKept{});
 }
@@ -472,7 +470,7 @@ static void launch_select(const SelectArgs& P, int BG, bool half, hipStream_t s)
   const void* a = SRC == SEL_KEYS ? (const void*)P.keys : SRC == SEL_LOGITS ? (const void*)P.logits : (const void*)P.cent;
   const void* b = SRC == SEL_LOGITS ? (const void*)P.tile_max : (const void*)P.q;
   auto* kernel = half ? select_radix_kernel<NT, E, GSM, true, SRC> : select_radix_kernel<NT, E, GSM, false, SRC>;
-  kernel<<<BG, NT, 0, s>>>(a, b, P.tile_sum, P.mask, P.nc, P.gs, P.np, P.es, P.ntiles, P);
+  kernel<<<BG, NT, 0, s>>>(ri_pack_ptrs(a, b, P.tile_sum, P.mask), (ri_int4){P.nc, P.gs, P.np, P.es}, P.ntiles, P);
 }
 template <int NT, int E, int SRC>
 static void launch_select_heads(const SelectArgs& P, int BG, bool half, hipStream_t s) {

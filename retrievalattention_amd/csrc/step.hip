@@ -49,22 +49,20 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
 template <int GSM, bool HALF>
-__global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(const uint16_t* cent, const uint16_t* q, const uint8_t* mask,
-                                                              const int32_t* size, int nc, int gs, int np, int es, float scale,
-                                                              SelectArgs S0, AttendParams A0) {
+__global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int4 n, float scale, SelectArgs S0, AttendParams A0) {
   static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
   __shared__ float sh_logits[STEP_CLUSTERS * GSM];
   __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS];
   SelectArgs S = S0;
   AttendParams A = A0;
-  S.cent = cent;
-  S.q = A.q = q;
-  S.mask = mask;
-  S.cluster_size = size;
-  S.nc = A.nc = nc;
-  S.gs = A.gs = gs;
-  S.np = A.np = np;
-  S.es = A.es = es;
+  S.cent = ri_global<const uint16_t>(in[0]);
+  S.q = A.q = ri_global<const uint16_t>(in[1]);
+  S.mask = ri_global<const uint8_t>(in[2]);
+  S.cluster_size = ri_global<const int32_t>(in[3]);
+  S.nc = A.nc = n[0];
+  S.gs = A.gs = n[1];
+  S.np = A.np = n[2];
+  S.es = A.es = n[3];
   S.scale = A.scale = scale;
   select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, true>(S, blockIdx.x, SelectKept{sh_logits, sh_est, sh_off, sh_start});
   lds_barrier();
@@ -97,7 +95,8 @@ static int step_short(const ri_decode_step_t* s, const void* q, int static_len, 
   if (rc) return rc;
   auto* kernel = s->gs <= 4 ? (s->half ? step_kernel<4, true> : step_kernel<4, false>)
                             : (s->half ? step_kernel<8, true> : step_kernel<8, false>);
-  kernel<<<s->BG, 64 * ATT_WAVES, 0, stream>>>(S.cent, S.q, S.mask, S.cluster_size, S.nc, S.gs, S.np, S.es, S.scale, S, A);
+  kernel<<<s->BG, 64 * ATT_WAVES, 0, stream>>>(ri_pack_ptrs(S.cent, S.q, S.mask, S.cluster_size),
+                                               (ri_int4){S.nc, S.gs, S.np, S.es}, S.scale, S, A);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
