@@ -26,6 +26,7 @@
 
 #include "attend_common.h"
 #include "ri_common.h"
+#include "step_route.h"
 
 // (what the first loads want stands before the struct: in registers at the start; 32 groups of 4 heads over 8192 clusters 16.5
 // -> 16.3 us, 12 groups of 7 heads over 1856 in half 9.34 -> 9.14)
@@ -51,8 +52,6 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, r
 #define RI_MAX_SPLITS 64
 #define RI_MAX_PROBES 4096  // rank tables of a launch: (2 * np + 1) * 4 bytes of LDS (what the selection lays out)
 #define RI_MAX_GROUPS 4096  // size of the counter area at the head of the workspace
-
-static inline int gs_pad_of(int gs) { return gs <= 4 ? 4 : (gs <= 8 ? 8 : 16); }
 
 static size_t attn_workspace_bytes(int BG, int gs) {
   if (BG <= 0 || BG > RI_MAX_GROUPS || gs <= 0 || gs > 16) return 0;
@@ -124,7 +123,7 @@ static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int e
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
   per_group = min(per_group, (int64_t)max_splits);
   if (per_group > 8 && per_group % 8 * 5 <= per_group && rows <= 64 * ATT_WAVES * per_group) per_group -= per_group % 8;
-  if (rows * gs_pad_of(gs) <= 384 * 4 || per_group < 1) per_group = 1;
+  if (attend_alone(rows, gs, BG) || per_group < 1) per_group = 1;
   const int waves = (int)per_group * ATT_WAVES;
   P.S = (int)per_group;
   P.W_kv = waves;

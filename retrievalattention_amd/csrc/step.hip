@@ -6,6 +6,7 @@
 // sizes of a layer do not change from token to token, so the caller keeps them in one struct and hands over its address.
 #include "attend_common.h"
 #include "select_body.h"
+#include "step_route.h"
 
 // ------------------------------------------------------------------------------------
 // append: steady_k/v[g, pos] = key/value[g]; 16 lanes per 256-byte row, grid.y = K, V.
@@ -44,8 +45,6 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
 // rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110 KB of LDS (124 with 8 heads): one workgroup
 // per compute unit, hence at most 256 groups; sixteen heads would not fit.
 // ------------------------------------------------------------------------------------
-#define STEP_CLUSTERS 512
-
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
 template <int GSM, bool HALF>
@@ -67,16 +66,6 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, true>(S, blockIdx.x, SelectKept{sh_logits, sh_est, sh_off, sh_start});
   lds_barrier();
   attend_group<GSM, HALF, true>(A, blockIdx.x, 0, AttendKept{sh_logits, sh_est, sh_off, sh_start});
-}
-
-// Short: what one workgroup scores for itself (select.hip), and no more rows than one workgroup attends as fast as several
-// (with the launch left out; 8 groups of 4 heads: 446 rows 14.4 us either way, 557 rows 15.8 against 15.4; 64 groups of 8
-// heads: 446 rows 16.7 against 17.1).
-#define STEP_ROWS 448
-static bool step_is_short(const ri_decode_step_t* s, int static_len) {
-  const long long rows = (long long)static_len + (long long)s->np * 16 + s->es;
-  return s->nc <= STEP_CLUSTERS && s->gs <= 8 && s->BG <= 256 && rows <= STEP_ROWS && s->cluster_size_i32 &&
-         s->cluster_start;
 }
 
 static int step_short(const ri_decode_step_t* s, const void* q, int static_len, void* out, hipStream_t stream) {

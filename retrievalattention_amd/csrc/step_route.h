@@ -1,0 +1,38 @@
+// Which decode steps one workgroup per group makes in one launch (step_kernel) and which are scoring + selection and
+// attention in launches of their own.  Host code only.
+#pragma once
+#include <stdint.h>
+
+#include "../../include/retro_mi355.h"
+
+// Heads of a group as the kernels pad them.
+static inline int gs_pad_of(int gs) { return gs <= 4 ? 4 : (gs <= 8 ? 8 : 16); }
+
+// Groups that an attention launch gives one workgroup each: few rows (fewer the more heads share their arithmetic), or no
+// compute unit left for a second one.
+static inline bool attend_alone(int64_t rows, int gs, int BG) { return rows * gs_pad_of(gs) <= 384 * 4 || BG > 128; }
+
+// Short: what one workgroup scores for itself (select.hip), and usually (16 tokens per retrieved cluster) no more rows than
+// one workgroup attends as fast as several: 8 groups of 8 heads 424 rows 14.6 us against 15.5, 488: 14.8 / 15.7, 552: 15.9 /
+// 15.5; of 4 heads 488: 13.8 / 15.0, 552: 15.4 / 14.8; one group of 8 heads 488: 14.5 / 15.0, 552: 15.6 / 14.9.
+// The rows are not known here when the kernel reads the zone's length from the device, as a captured step does until the
+// zone is full, and never what the retrieved clusters hold:
+//  * Where the attention by itself would be one workgroup per group all the same, one launch is faster whatever they turn
+//    out to be.  8 groups of 4 heads captured with 331 rows: then 12.3 us against 14.2, at 1354 rows 22.3 / 24.4, with 512
+//    tokens in each of 9 clusters 53.6 / 55.6; 128 groups 13.9 / 16.3 and 25.7 / 27.8.
+//  * Elsewhere the other route has more workgroups, so the rows that the zone can hold decide, and those of the clusters are
+//    bounded by the page limit and the store.  8 groups of 8 heads captured with 331 rows: then 13.1 us against 15.5, at 458
+//    rows 15.0 / 15.5, but at 762 18.1 / 16.6, 962: 20.1 / 17.8, 1354: 24.4 / 18.8; with 64 tokens in each of 9 clusters (763
+//    rows) 18.5 / 16.8, with 512: 64.9 / 28.5.  At twice the limit the most crowded clusters cost what usual ones save.
+#define STEP_CLUSTERS 512
+#define STEP_ROWS 448
+#define STEP_ROWS_CROWDED (2 * STEP_ROWS)
+static inline bool step_is_short(const ri_decode_step_t* s, int static_len) {
+  if (s->nc > STEP_CLUSTERS || s->gs > 8 || s->BG > 256 || !s->cluster_size_i32 || !s->cluster_start) return false;
+  const int64_t usual = (int64_t)s->np * 16 + s->es;
+  if (static_len + usual > STEP_ROWS) return false;
+  if (attend_alone(static_len + usual, s->gs, s->BG)) return true;
+  const int64_t zone = s->static_len_dev ? s->steady_stride : static_len;
+  const int64_t pages = (int64_t)s->max_pages * s->page, held = pages < s->store_stride ? pages : s->store_stride;
+  return zone + usual <= STEP_ROWS && zone + s->es + held <= STEP_ROWS_CROWDED;
+}

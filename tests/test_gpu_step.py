@@ -28,7 +28,8 @@ def test_append_kv(dev, BG, stride, pos, on_device):
     (1, 1, 8, 1, 0, 0, 100, False), (2, 4, 8, 3, 5, 1, 100, True), (3, 5, 40, 7, 33, 17, 100, False),
     (5, 8, 256, 4, 60, 70, 2, True), (4, 3, 264, 10, 100, 69, 100, False), (8, 4, 512, 9, 118, 98, 100, False),
     (2, 7, 504, 12, 150, 100, 3, True), (256, 2, 16, 2, 3, 5, 100, False), (257, 2, 16, 2, 3, 5, 100, False),
-    (2, 4, 512, 13, 118, 98, 100, False)])
+    (2, 4, 512, 13, 118, 98, 100, False), (2, 4, 512, 13, 118, 98, 40, False), (3, 8, 512, 9, 118, 98, 72, False),
+    (3, 8, 512, 9, 118, 98, 76, True)])
 def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
     """The step that one workgroup per group makes (and, past its limits, the launches one by one) against scoring +
     selection and attention called by themselves: the same lists; outputs differ only where those split a group's rows,

@@ -1,0 +1,63 @@
+"""Which decode steps one workgroup per group makes (csrc/step_route.h, host code: compiled here by g++)."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from retrievalattention_amd._lib import DecodeStep
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def is_short(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    where = tmp_path_factory.mktemp("route")
+    (where / "route.cpp").write_text('#include "step_route.h"\nextern "C" int is_short(const ri_decode_step_t* s, int n) '
+                                     '{ return step_is_short(s, n); }\n')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I",
+                    os.path.join(ROOT, "retrievalattention_amd", "csrc"), str(where / "route.cpp"), "-o",
+                    str(where / "route.so")], check=True)
+    call = ctypes.CDLL(str(where / "route.so")).is_short
+
+    def short(static_len, zone=323, on_device=False, BG=8, gs=4, nc=512, np=9, es=118, page=8, max_pages=72, store=8192,
+              sizes=True):
+        step = DecodeStep(BG=BG, gs=gs, nc=nc, np=np, es=es, page=page, max_pages=max_pages, steady_stride=zone,
+                          store_stride=store, static_len_dev=1 if on_device else None,
+                          cluster_size_i32=1 if sizes else None, cluster_start=1 if sizes else None)
+        return bool(call(ctypes.byref(step), static_len))
+    return short
+
+
+def test_limits(is_short):
+    assert is_short(98) and is_short(98, gs=8)
+    assert not is_short(98, nc=520) and not is_short(98, gs=9) and not is_short(98, BG=257) and not is_short(98, sizes=False)
+    assert is_short(186) and not is_short(187)                      # 448 rows
+    assert is_short(186, BG=256) and not is_short(187, BG=256)
+
+
+@pytest.mark.parametrize("gs", [1, 4, 5, 8])
+def test_length_on_the_device_grows_to_the_zone(is_short, gs):
+    """A captured step serves every length up to the zone's: only where the attention by itself would have one workgroup
+    as well (384 rows of up to four heads, 192 of eight, more than 128 groups) does the length at hand decide."""
+    alone = gs <= 4
+    for zone in (69 + 256, 69 + 1024):
+        assert is_short(69, zone=zone, on_device=True, gs=gs) == alone
+        assert is_short(122, zone=zone, on_device=True, gs=gs) == alone
+        assert not is_short(123, zone=zone, on_device=True, gs=gs)
+        assert is_short(123, zone=zone, on_device=False, gs=gs)
+        assert is_short(123, zone=zone, on_device=True, gs=gs, BG=129)
+    assert is_short(123, zone=186, on_device=True, gs=gs) and not is_short(123, zone=187, on_device=True, gs=gs)
+    assert is_short(69, zone=1093, on_device=True, gs=gs, nc=128, np=2, es=30)
+
+
+@pytest.mark.parametrize("gs", [4, 8])
+def test_clusters_may_hold_what_the_page_limit_lets_them(is_short, gs):
+    at = 170   # 432 rows if the clusters have their usual size
+    assert is_short(at, gs=gs, max_pages=76) and not is_short(at, gs=gs, max_pages=77)     # 896 rows at most
+    assert is_short(at, gs=gs, max_pages=1 << 30, store=608) and not is_short(at, gs=gs, max_pages=1 << 30, store=609)
+    assert is_short(at, gs=gs, max_pages=1 << 30, BG=129)
+    assert is_short(98, gs=gs, max_pages=1 << 30) == (gs == 4)
