@@ -358,7 +358,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   // rows are done), which keeps a workgroup at 48 KB of LDS, so that the two its registers leave room for fit a compute
   // unit (sixteen heads: 116 KB, one workgroup)
   constexpr bool ACC_OVER_VT = GS_PAD * RI_DIM * sizeof(float) <= 16 * ATT_VT_STRIDE * sizeof(uint16_t);
-  __shared__ float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
+  __shared__ __attribute__((aligned(16))) float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
+  static_assert(__alignof__(sh_acc_own) == 16 && __alignof__(sh_vt) == 16, "read two dims at a time");
   auto acc_of = [&](int w) -> float* {
     return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : &sh_acc_own[ACC_OVER_VT ? 0 : w][0][0];
   };

@@ -97,7 +97,8 @@ __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(
 template <bool HALF, int Y>
 __global__ __launch_bounds__(512) void mean_fold_kernel(const float4* __restrict__ chains, uint16_t* __restrict__ mean, int C,
                                                         float inv) {
-  __shared__ float sums[MEAN_MAX_C][32];
+  __shared__ __attribute__((aligned(16))) float sums[MEAN_MAX_C][32];
+  static_assert(__alignof__(sums) == 16, "written four dims at a time");
   const int h = blockIdx.y, quad = threadIdx.x & 7;
   const float4* in = chains + (size_t)h * 4 * Y * C * (RI_DIM / 4) + blockIdx.x * 8 + quad;
   for (int c = threadIdx.x >> 3; c < C; c += 64) {

@@ -50,7 +50,8 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
 template <int GSM, bool HALF>
 __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int4 n, float scale, SelectArgs S0, AttendParams A0) {
   static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
-  __shared__ float sh_logits[STEP_CLUSTERS * GSM];
+  __shared__ __attribute__((aligned(16))) float sh_logits[STEP_CLUSTERS * GSM];
+  static_assert(__alignof__(sh_logits) == 16, "read four heads at a time");
   __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS];
   SelectArgs S = S0;
   AttendParams A = A0;
