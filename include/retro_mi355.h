@@ -579,8 +579,8 @@ int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_s
    ri_prefill_split: keys[h][i] = key[first + i][h] for i < N, and the steady zone of both tensors: rows 0..n_start-1
    of every head from tokens start0.., the following n_end from tokens end0..  Strides in elements, multiples of 8.
    ri_prefill_center: keys[h][i] -= mean[h], in the element type.
-   ri_prefill_mean: mean[h] = the mean of key[first .. first + N - 1][h], summed in fp32 in a fixed order and rounded once:
-   the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144 tokens, and 2 GiB of them together; beyond that
+   ri_prefill_mean: mean[h] = the mean of key[first .. first + N - 1][h], summed in fp32 in a fixed order; the sum times 1 / N
+   is rounded to half, or to fp32 and then to bfloat16: the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144 tokens, and 2 GiB of them together; beyond that
    ri_prefill_mean_workspace_bytes is 0 and the call refuses.
    ri_prefill_split_centred: ri_prefill_split with mean[h] taken off the rows of keys, as ri_prefill_center does.
    ri_prefill_index: out = centroids + mean, mask = (count == 0), sizes as elements and as int32, first rows. */

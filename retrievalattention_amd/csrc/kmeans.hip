@@ -1234,9 +1234,10 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   // against 6.7).
   if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
   // A little more than those two per compute unit is a second round for a few: three columns per wave then do it in one
-  // round, the longer the loop the further (16 x 8200 tokens, 528 workgroups of one column, 512 centroids: 20.2 us against
-  // 21.0, 16 x 9200, 576: 23.6 against 22.9; 8 x 20000, 632, 1024: 39.8 against 40.4, 8 x 24000, 752: 44.9 against 43.7;
-  // 4 x 48719, 764, 3072: 115 against 118).
+  // round, the longer the loop the further.  By centroids, workgroups of one column and us with three columns / one: 512
+  // centroids, 520 21.5 / 22.2, 576 22.7 / 22.8; 768, 520 27.9 / 29.8, 576 30.6 / 31.4, 624 32.5 / 31.9; 1024, 520 35.9 / 39.0,
+  // 640 41.2 / 41.2, 688 43.1 / 42.8; 1536, 520 51.0 / 56.2, 720 63.0 / 63.1, 752 66.6 / 65.4; 2048, 520 65.9 / 74.3, 752 84.3 /
+  // 85.2; 3072, 520 95.5 / 109.2, 752 121.6 / 123.6.  (92 shapes of 4, 8 and 16 problems; the ones between lie between.)
   else if (nc >= 512 && wgs256 > 512 && wgs256 <= 440 + nc / 5 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
   // (up to three of them: 22 x 8192 tokens, 512 centroids: 24.4 us against 25.4 with two columns, 26.5 with three; 24 x 8119:
   // 25.2 against 25.7; 24 x 8192, 256: 16.4 either way; 28 x 8192: 30.8 against 30.0)

@@ -13,17 +13,19 @@
 // order of j; of the Y C sums left, those of a c (r = c Y + y) as a tree over y; these into Y sums over c = y', y' + Y ...
 // in order, and those as a tree.  Y and C are mean_order's.  It is the order in which torch 2.10 adds on this device
 // (torch.mean(keys, dim=1) over [H, N, 128]), found from its sums over chosen inputs, so that an index built with
-// torch.mean and one built here are the same to the bit; the product with 1 / N is rounded once, to the element type.
+// torch.mean and one built here are the same to the bit.  The product with 1 / N is torch's as well: in half rounded once, to
+// the element type, in bfloat16 first to fp32.
 //
 // mean_chain_kernel: a wave per chain and head, two dims per lane, MEAN_DEEP rows of it in flight (an addition waits for
 // the one before, so a chain cannot be split: the rows in flight are what fills the link to memory).  Heads vary fastest:
 // workgroups next to each other read whole tokens.
 // mean_fold_kernel: a workgroup per head and 32 dims puts the chains together.
-// Chains and fold, 8 heads of 8192 / 131072 tokens and 4 of 48719: 8.3, 44 and 14.7 us, where torch.mean took 54, 168 and
-// 157 (with a branch around each of the loads 10.5, 73 and 25).  Bound by the rows where they are many (268 MB at 6.1
-// TB/s, some of it from the memory-side cache), else by the rows in flight: there are only H S waves.  And the mean is known
-// before the heads are taken apart, so that pass centres them: 6.2 / 78 / 15.7 us for both, where a copy (6.7 / 91 / 15.7)
-// and a pass over it (12 / 77 / 16) were needed.
+// Inside a prefill, 8 heads of 8192 / 131072 tokens and 4 of 48719: chains 6.6, 69 and 11.2 us, fold 2.4, 4.8 and 4.5, where
+// torch.mean took 54, 168 and 157.  Bound by the rows in flight, there are only H S waves of 256 bytes a row: 268 MB at 3.9
+// TB/s, where reading alone reaches 5.7.  (Over the same rows again and again, some of them in the memory-side cache: 8.3, 44
+// and 14.7 us for both; with a branch around each of the loads 10.5, 73 and 25.)  And the mean is known before the heads are
+// taken apart, so that pass centres them: 5.8 / 79 / 16.1 us for both, where a copy (6.7 / 91 / 15.7) and a pass over it (12 /
+// 77 / 16) were needed.
 // ------------------------------------------------------------------------------------
 #define MEAN_DEEP 64
 #define MEAN_MAX_C 256
@@ -132,7 +134,7 @@ __global__ __launch_bounds__(512) void mean_fold_kernel(const float4* __restrict
   for (int o = Y / 2; o > 0; o >>= 1)
 #pragma unroll
     for (int y = 0; y < o; ++y) t[y] += t[y + o];
-  // (the product of two 24-bit numbers is exact in 53 bits: one rounding)
+  // (half: the product of two 24-bit numbers is exact in 53 bits, one rounding; bfloat16: to fp32, then to the element type)
   mean[h * RI_DIM + blockIdx.x * 32 + threadIdx.x] =
       HALF ? __builtin_bit_cast(uint16_t, (_Float16)((double)t[0] * (double)inv)) : ri_f32_to_bf16(t[0] * inv);
 }

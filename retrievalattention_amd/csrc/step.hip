@@ -42,8 +42,8 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
 // With up to 512 clusters the selection is one workgroup per group that scores for itself, and with few rows the attention
 // is, too: as one kernel the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
 // host as well.  What bounds it is the chain of either half on one compute unit.  8 groups of 4 heads, 512 clusters, 331
-// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110 KB of LDS (124 with 8 heads): one workgroup
-// per compute unit, hence at most 256 groups; sixteen heads would not fit.
+// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110060 bytes of LDS (119532 with 8 heads): one
+// workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.  step_route.h says which steps take it.
 // ------------------------------------------------------------------------------------
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
