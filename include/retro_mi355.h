@@ -457,6 +457,18 @@ int ri_kmeans_update_direct_f16(const void* data, const int32_t* assign, void* c
 int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P, int N,
                            int nc, ri_stream_t stream);
 
+/* `updates` times ri_kmeans_assign and the normalised update of that assignment, then (last != 0) one more assignment:
+ * the same centroids and the same assign [P, N] bit for bit.  Between the passes the library keeps, in the workspace, what
+ * a token's best and second best scores were and which centroids have moved, and scores again only where the best can have
+ * changed.  centroids [P, nc, 128] as the clustering starts from them (nc % 32 == 0); workspace:
+ * ri_kmeans_iterate_workspace_bytes, no initialisation needed. */
+size_t ri_kmeans_iterate_workspace_bytes(int P, int N, int nc);
+int ri_kmeans_iterate(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg, int64_t head_rows,
+                      int updates, int last, void* workspace, size_t workspace_bytes, ri_stream_t stream);
+/* ri_kmeans_iterate on IEEE half instead of bfloat16. */
+int ri_kmeans_iterate_f16(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                          int64_t head_rows, int updates, int last, void* workspace, size_t workspace_bytes,
+                          ri_stream_t stream);
 /* Per-cluster value sums: replaces triton_index_add (cache_hub/kmeans.py:176-221).
  * value_sum[p,c,:] = bf16(Σ member value rows), Σ in the same fixed order as above. */
 int ri_kmeans_value_sum(const void* values, const int32_t* counts, const int32_t* offsets,

@@ -78,6 +78,9 @@ SIGNATURES = {
     "ri_kmeans_update_f16": (I, [P, P, P, P, P, I, I, I, I, I64, I, P, SZ, P]),
     "ri_kmeans_update_direct": (I, [P, P, P, P, P, P, I, I, I, I, I64, I, P]),
     "ri_kmeans_update_direct_f16": (I, [P, P, P, P, P, P, I, I, I, I, I64, I, P]),
+    "ri_kmeans_iterate_workspace_bytes": (SZ, [I, I, I]),
+    "ri_kmeans_iterate": (I, [P, P, P, I, I, I, I, I64, I, I, P, SZ, P]),
+    "ri_kmeans_iterate_f16": (I, [P, P, P, I, I, I, I, I64, I, I, P, SZ, P]),
     "ri_kmeans_value_sum": (I, [P, P, P, P, P, I, I, I, P, SZ, P]),
     "ri_kmeans_value_sum_f16": (I, [P, P, P, P, P, I, I, I, P, SZ, P]),
     "ri_permute_rows": (I, [P, P, P, I, I, I64, I64, P]),

@@ -40,26 +40,19 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_me
         centroids = torch.index_select(key, 1, init_indices).contiguous()
     nseg, ncs = N // S, nc // S
     P = G * S
+    assign = None
     if nseg > 0 and num_iters > 1:
         assign = torch.empty((P, nseg), dtype=torch.int32, device=dev)
-        direct = nseg <= kernels.KMEANS_DIRECT_MAX_TOKENS
-        if not direct:
-            counts = torch.empty((P, ncs), dtype=torch.int32, device=dev)
-            offsets = torch.empty((P, ncs + 1), dtype=torch.int32, device=dev)
-            members = torch.empty((P, nseg), dtype=torch.int32, device=dev)
-        for _ in range(num_iters - 1):
-            kernels.kmeans_assign(key, centroids, assign, P, nseg, ncs, S, N)
-            if direct:
-                kernels.kmeans_update_direct(key, assign, centroids, P, nseg, ncs, S, N, True)
-            else:
-                kernels.kmeans_build_lists(assign, counts, offsets, members, P, nseg, ncs)
-                kernels.kmeans_update(key, counts, offsets, members, centroids, P, nseg, ncs, S, N, True)
+        kernels.kmeans_iterate(key, centroids, assign, P, nseg, ncs, S, N, num_iters - 1, S == 1)
     r = KMeansResult()
-    r.assign = torch.empty((G, N), dtype=torch.int32, device=dev)
     r.counts = torch.empty((G, nc), dtype=torch.int32, device=dev)
     r.offsets = torch.empty((G, nc + 1), dtype=torch.int32, device=dev)
     r.members = torch.empty((G, N), dtype=torch.int32, device=dev)
-    kernels.kmeans_assign(key, centroids, r.assign, G, N, nc, 1, N)
+    if assign is not None and S == 1:   # (the segment is the sequence: the last pass over all centroids was one of them)
+        r.assign = assign
+    else:
+        r.assign = torch.empty((G, N), dtype=torch.int32, device=dev)
+        kernels.kmeans_assign(key, centroids, r.assign, G, N, nc, 1, N)
     if N <= kernels.KMEANS_DIRECT_MAX_TOKENS and not final_means:
         kernels.kmeans_lists_direct(r.assign, r.counts, r.offsets, r.members, G, N, nc)
     elif N <= kernels.KMEANS_DIRECT_MAX_TOKENS:

@@ -97,39 +97,116 @@ __device__ __forceinline__ int km_first_of(const f32x16_t& x, float m, float bes
   return row;
 }
 
-template <int KM_TT, int KM_CT, int KM_W, int KM_NB, bool HALF>
-__global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __restrict__ data,
-                                                              const uint16_t* __restrict__ cent,
-                                                              int32_t* __restrict__ assign, int N, int nc,
-                                                              int seg, int64_t head_rows, int sh) {
-  static_assert(KM_CT % (4 * KM_W) == 0 && KM_CT % 32 == 0, "a tile is whole 1 KiB wave loads and whole sub-tiles");
-  constexpr int KM_WG_TOKENS = KM_W * 32 * KM_TT;
-  constexpr int L = KM_CT / 4 / KM_W;   // loads of a wave per tile
-  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[KM_NB][KM_CT][RI_DIM];
-  const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 31, hh = lane >> 5;
-  const int t0 = (blockIdx.x >> sh) * KM_WG_TOKENS + wave * (32 * KM_TT);
-  const uint16_t* dp = data + km_row0(p, seg, head_rows, N) * RI_DIM;
-  const uint16_t* cp = cent + (size_t)p * nc * RI_DIM;
+// The same with the largest of the other fifteen scores and of what low8, low4, high8 and high4 started from, in `second`:
+// what each halving leaves behind.  Ten instructions more.
+__device__ __forceinline__ int km_first_two(const f32x16_t& x, float m, float low8, float high8, float low4, float high4,
+                                            int base, float& second) {
+  float y0, y1, y2, y3, y4, y5, y6, y7, t, u;
+  uint64_t e, e8;
+  int row;
+  asm volatile(
+      "v_cmp_eq_f32_e64 %9, %26, %28\n\t"
+      "s_nop 1\n\t"
+      "v_cndmask_b32_e64 %0, %18, %10, %9\n\t"
+      "v_cndmask_b32_e64 %1, %19, %11, %9\n\t"
+      "v_cndmask_b32_e64 %2, %20, %12, %9\n\t"
+      "v_cndmask_b32_e64 %3, %21, %13, %9\n\t"
+      "v_cndmask_b32_e64 %4, %22, %14, %9\n\t"
+      "v_cndmask_b32_e64 %5, %23, %15, %9\n\t"
+      "v_cndmask_b32_e64 %6, %24, %16, %9\n\t"
+      "v_cndmask_b32_e64 %7, %25, %17, %9\n\t"
+      "v_cndmask_b32_e64 %8, %26, %27, %9"
+      : "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7), "=&v"(second), "=&s"(e8)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]),
+        "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(low8), "v"(high8), "v"(m));
+  asm volatile(
+      "v_cndmask_b32_e64 %5, %14, %13, %8\n\t"
+      "v_cmp_eq_f32_e64 %9, %5, %15\n\t"
+      "v_cndmask_b32_e64 %7, 16, 0, %8\n\t"
+      "v_max3_f32 %6, %4, %10, %11\n\t"
+      "v_max_f32_e32 %6, %6, %12\n\t"
+      "v_cndmask_b32_e64 %0, %4, %0, %9\n\t"
+      "v_cndmask_b32_e64 %1, %10, %1, %9\n\t"
+      "v_cndmask_b32_e64 %2, %11, %2, %9\n\t"
+      "v_cndmask_b32_e64 %3, %12, %3, %9\n\t"
+      "v_cndmask_b32_e64 %5, %5, %6, %9\n\t"
+      "v_cndmask_b32_e64 %4, 8, 0, %9"
+      : "+&v"(y0), "+&v"(y1), "+&v"(y2), "+&v"(y3), "+&v"(y4), "=&v"(t), "=&v"(u), "=&v"(row), "+s"(e8), "=&s"(e)
+      : "v"(y5), "v"(y6), "v"(y7), "v"(low4), "v"(high4), "v"(m));
+  asm volatile(
+      "v_max_f32_e32 %4, %0, %1\n\t"
+      "v_cmp_eq_f32_e64 %8, %4, %11\n\t"
+      "v_add_u32_e32 %7, %7, %10\n\t"
+      "v_max_f32_e32 %5, %2, %3\n\t"
+      "v_cndmask_b32_e64 %0, %2, %0, %8\n\t"
+      "v_cmp_eq_f32_e64 %9, %0, %11\n\t"
+      "v_cndmask_b32_e64 %1, %3, %1, %8\n\t"
+      "v_cndmask_b32_e64 %4, %4, %5, %8\n\t"
+      "v_cndmask_b32_e64 %5, 2, 0, %8\n\t"
+      "v_cndmask_b32_e64 %1, %0, %1, %9\n\t"
+      "v_max3_f32 %6, %6, %12, %4\n\t"
+      "v_cndmask_b32_e64 %4, 1, 0, %9\n\t"
+      "v_max_f32_e32 %6, %6, %1\n\t"
+      "v_add3_u32 %7, %7, %5, %4\n\t"
+      "v_add_u32_e32 %7, %7, %13"
+      : "+&v"(y0), "+&v"(y1), "+&v"(y2), "+&v"(y3), "=&v"(y5), "=&v"(y6), "+&v"(second), "+&v"(row), "=&s"(e8), "=&s"(e)
+      : "v"(y4), "v"(m), "v"(t), "v"(base));
+  return row;
+}
 
-  // A tile goes from global memory straight into LDS, 16 bytes per lane and 1 KiB (four rows)
-  // per wave instruction: lane l lands at byte l * 16 of the instruction's LDS window, and which
-  // global piece it fetches is free, so the 16-byte pieces of row w are stored at piece ^ (w & 15):
-  // the 16 lanes of a ds_read_b128 phase then hit 16 different piece positions (all 64 banks once).
-  // (A wave's rows start at the same place of sixteen in every instruction, so a lane's offset never changes and the rest
-  // of the address is scalar.)
-  static_assert(KM_W % 4 == 0, "an instruction's first row modulo 16 is the wave's");
-  const uint32_t ld_at = (lane >> 4) * (RI_DIM * 2) + (((lane & 15) ^ ((wave * 4 + (lane >> 4)) & 15)) * 16);
-  const uint32_t sh_base = (uint32_t)(uintptr_t)(km_lds_ptr)&sh_c[0][0][0];
-  auto tile_load = [&](int ct, int buf) {
-#pragma unroll
-    for (int u = 0; u < L; ++u) {
-      const int row4 = (wave + u * KM_W) * 4;      // first of the four rows of this instruction
-      const int row = min(ct + row4, nc - 4);      // (rows past the last repeat it: the count of loads is fixed)
-      km_lds_dma16(cp + (size_t)row * RI_DIM, ld_at, sh_base + (uint32_t)((buf * KM_CT + row4) * RI_DIM * 2));
-    }
-  };
+// ------------------------------------------------------------------------------------
+// What the passes of one clustering know of each other (ri_kmeans_iterate): a pass looks only where a token's centroid can
+// have changed since the one before.  A word per cluster, as the last update left it: KM_MOVED: it wrote the centroid; KM_UNIT:
+// some update did, so that the centroid's norm is one; KM_FRESH: this was the first; above them the tokens of the cluster.
+// ------------------------------------------------------------------------------------
+#define KM_MOVED 1
+#define KM_UNIT 2
+#define KM_FRESH 4
+#define KM_SIZE_SHIFT 3
+#define KM_OPEN_WGS 768     // three to a compute unit
+#define KM_OPEN_PARTS 8
+// How a pass goes about a problem.  KM_ALL: every centroid is scored.  KM_KEYS: most tokens came to a centroid that no update
+// had written before, a key as it is, with a norm far above one; those that are left of them are scored first, and no unit
+// vector scores above a token's norm.  KM_NEW: the centroids that the last update wrote are scored; of the others none but a
+// token's own scores above its bound.
+enum { KM_ALL, KM_KEYS, KM_NEW };
+struct KmBounds {
+  float* best;            // [P, N] the score of the token's centroid
+  float* bound;           // [P, N] no other centroid scores above it
+  const int32_t* state;   // [P, nc]
+  uint8_t* touched;       // [P, nc] a token has come or gone since the last update
+  const uint16_t* order;  // [P, nc] the centroids that are scored first, then the others, each ascending
+  const ri_int2* plan;    // [P] KM_ALL .. KM_NEW, how many are scored first
+  int32_t* open;          // [P, N] tokens of this pass that have to look at all centroids
+  int32_t* open_count;    // [P]
+  int32_t* partial;       // [KM_OPEN_WGS, 3, tokens of a block]
+  int32_t* arrived;       // [KM_OPEN_WGS] zero between launches
+  const int32_t* odd;     // [P] a centroid that an update wrote has no norm of one (see km_finish)
+  int P;
+};
+__device__ __forceinline__ void km_settle(const KmBounds& B, int32_t* assign, size_t t, size_t first_centroid, int id, int old,
+                                          float best, float bound) {
+  assign[t] = id;
+  B.best[t] = best;
+  B.bound[t] = bound;
+  if (id != old) B.touched[first_centroid + old] = B.touched[first_centroid + id] = 1;
+}
+
+// the value of the lane 32 on
+__device__ __forceinline__ float km_other(float x, int hh) {
+  uint32_t a, b;
+  ri_lane_pair<32>(__float_as_uint(x), a, b);
+  return __uint_as_float(hh ? a : b);
+}
+
+// One workgroup's turn over centroids for its tokens: W waves of TT columns of 32 tokens, which stay in registers.
+// LISTED: the centroids are those at `list` (LDS), else consecutive rows.
+template <int TT, int CT, int W, int NB, bool HALF, bool LISTED>
+struct KmScan {
+  static_assert(CT % (4 * W) == 0 && CT % 32 == 0, "a tile is whole 1 KiB wave loads and whole sub-tiles");
+  static_assert(W % 4 == 0, "an instruction's first row modulo 16 is the wave's");
+  static constexpr int TOKENS = W * 32 * TT;
+  static constexpr int L = CT / 4 / W;   // loads of a wave per tile
   // Tokens as operands: lane: token r, dims 16 kk + 8 hh.  A load whose lanes touch 32 tokens keeps the compute unit's address
   // path busy for 64 cycles, one of four whole tokens for 18; with eight waves that start together that is in front of the
   // first product.  Their tokens are loaded whole and turned in the wave's part of the last tile buffer, which no tile is on
@@ -138,141 +215,464 @@ __global__ __launch_bounds__(KM_W * 64) void km_assign_kernel(const uint16_t* __
   // same, so they stay).  The small tiles of four
   // waves leave room for eight tokens at a time, and other workgroups run beside: as operands (128 x 8192: 121.9 us, turned
   // 124.1).
-  constexpr int WR = KM_CT / KM_W;
-  constexpr bool TURN = WR == 16 && KM_TT < 4;
-  uint4 b[KM_TT][8];
+  static constexpr int WR = CT / W;
+  static constexpr bool TURN = WR == 16 && TT < 4;
+  // Operands from LDS: each is requested AHEAD products before its own, into the register that a product has just read, across
+  // sub-tiles where a tile has several.  (The compiler has two on their way and waits for each; as many more as the
+  // registers hold.  8 x 8192 tokens, 512 centroids: 10.2 -> 9.3 us, 16 x 8200 22.4 -> 20.7, 4 x 48719, 3072 119 -> 118,
+  // 128 x 8192 120.6 -> 117.6, 8 x 131072, 8192 1531 -> 1512.)
+  static constexpr int AHEAD = TT == 2 ? 3 : CT == 32 ? 0 : TT == 4 ? 4 : 8;
+
+  uint16_t (*sh)[CT][RI_DIM];   // [NB] tile buffers
+  const uint16_t* cp;           // the problem's centroids
+  const uint16_t* list;
+  int nc, lane, wave, r, hh;
+  uint32_t next[L];             // LISTED: this lane's rows of the tile that is requested next
+  uint4 b[TT][8];
+  float best[TT], second[TT];
+  int at[TT];                   // where best was scored: the centroid, or its place in the list
+
+  __device__ __forceinline__ KmScan(uint16_t (*sh_c)[CT][RI_DIM], const uint16_t* centroids, int n)
+      : sh(sh_c), cp(centroids), list(nullptr), nc(n), lane(threadIdx.x & 63),
+        wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), r(lane & 31), hh(lane >> 5) {}
+
+  // A tile goes from global memory straight into LDS, 16 bytes per lane and 1 KiB (four rows)
+  // per wave instruction: lane l lands at byte l * 16 of the instruction's LDS window, and which
+  // global piece it fetches is free, so the 16-byte pieces of row w are stored at piece ^ (w & 15):
+  // the 16 lanes of a ds_read_b128 phase then hit 16 different piece positions (all 64 banks once).
+  // (A wave's rows start at the same place of sixteen in every instruction, so a lane's offset never changes and the rest
+  // of the address is scalar; the rows of a list are the lane's own.)
+  __device__ __forceinline__ void tile_rows(int ct, int end) {
 #pragma unroll
-  for (int tt = 0; tt < KM_TT; ++tt) {
-    const uint16_t* q = dp + (size_t)min(t0 + tt * 32 + r, N - 1) * RI_DIM + hh * 8;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      b[tt][i] = TURN ? ri_ld16(dp + (size_t)min(t0 + tt * 32 + 4 * i + (lane >> 4), N - 1) * RI_DIM + (lane & 15) * 8)
-                      : ri_ld16(q + i * 16);
+    for (int u = 0; u < L; ++u) next[u] = list[min(ct + (wave + u * W) * 4 + (lane >> 4), end - 1)];
   }
-  const int tiles = (nc + KM_CT - 1) / KM_CT;
+  __device__ __forceinline__ void tile_load(int ct, int buf) {
+    const uint32_t piece = ((lane & 15) ^ ((wave * 4 + (lane >> 4)) & 15)) * 16;
+    const uint32_t sh_base = (uint32_t)(uintptr_t)(km_lds_ptr)&sh[0][0][0];
 #pragma unroll
-  for (int t = 0; t < KM_NB - 1; ++t) tile_load(t * KM_CT, t);
+    for (int u = 0; u < L; ++u) {
+      const int row4 = (wave + u * W) * 4;      // first of the four rows of this instruction
+      const uint32_t to = sh_base + (uint32_t)((buf * CT + row4) * RI_DIM * 2);
+      if (LISTED) {
+        km_lds_dma16(cp, next[u] * (RI_DIM * 2) + piece, to);
+      } else {
+        const int row = min(ct + row4, nc - 4);      // (rows past the last repeat it: the count of loads is fixed)
+        km_lds_dma16(cp + (size_t)row * RI_DIM, (lane >> 4) * (RI_DIM * 2) + piece, to);
+      }
+    }
+  }
+  __device__ __forceinline__ void start(int from, int end) {
+    if (LISTED) tile_rows(from, end);
+#pragma unroll
+    for (int t = 0; t < NB - 1; ++t) {
+      tile_load(from + t * CT, t);
+      if (LISTED) tile_rows(from + (t + 1) * CT, end);
+    }
+  }
+  __device__ __forceinline__ void nothing_yet() {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      best[tt] = second[tt] = -INFINITY;
+      at[tt] = 0;
+    }
+  }
+  // rows t0 .. of dp, the last one `last` (open: the rows named there)
+  __device__ __forceinline__ void request_tokens(const uint16_t* dp, int t0, int last, const int32_t* open = nullptr) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      const int tok = min(t0 + tt * 32 + r, last);
+      const uint16_t* q = dp + (size_t)(open ? open[tok] : tok) * RI_DIM + hh * 8;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        b[tt][i] = TURN ? ri_ld16(dp + (size_t)min(t0 + tt * 32 + 4 * i + (lane >> 4), last) * RI_DIM + (lane & 15) * 8)
+                        : ri_ld16(q + i * 16);
+    }
+  }
   // (The token registers are consumed here so that the compiler's own wait for their loads sits in front of the loop and not
   // inside it, where it would also wait for the tile in flight.)
-  uint4* const turn = reinterpret_cast<uint4*>(&sh_c[KM_NB - 1][wave * WR][0]);
-  km_wait_vm<(KM_NB - 1) * L>();
+  __device__ __forceinline__ void take_tokens() {
+    uint4* const turn = reinterpret_cast<uint4*>(&sh[NB - 1][wave * WR][0]);
+    km_wait_vm<(NB - 1) * L>();
 #pragma unroll
-  for (int tt = 0; tt < KM_TT; ++tt) {
-    if (TURN) {
-      uint4 o[8];
+    for (int tt = 0; tt < TT; ++tt) {
+      if (TURN) {
+        uint4 o[8];
 #pragma unroll
-      for (int w = 0; w < 2; ++w) {
+        for (int w = 0; w < 2; ++w) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = 4 * i + (lane >> 4);
-          turn[row * 16 + ((lane & 15) ^ row)] = b[tt][w * 4 + i];
+          for (int i = 0; i < 4; ++i) {
+            const int row = 4 * i + (lane >> 4);
+            turn[row * 16 + ((lane & 15) ^ row)] = b[tt][w * 4 + i];
+          }
+          ri_wave_sync();
+          if (r >> 4 == w) {
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) o[kk] = turn[(r & 15) * 16 + ((kk * 2 + hh) ^ (r & 15))];
+          }
+          ri_wave_sync();   // (a wave's LDS accesses happen in order)
         }
-        ri_wave_sync();
-        if (r >> 4 == w) {
 #pragma unroll
-          for (int kk = 0; kk < 8; ++kk) o[kk] = turn[(r & 15) * 16 + ((kk * 2 + hh) ^ (r & 15))];
-        }
-        ri_wave_sync();   // (a wave's LDS accesses happen in order)
+        for (int kk = 0; kk < 8; ++kk) b[tt][kk] = o[kk];
       }
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) b[tt][kk] = o[kk];
+      for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[tt][kk].x), "+v"(b[tt][kk].y), "+v"(b[tt][kk].z), "+v"(b[tt][kk].w));
+    }
+  }
+  // centroids (or places of the list) from .. end-1 against the tokens; track: with the second best
+  __device__ __forceinline__ void score(int from, int end, bool track) {
+    const uint16_t* row_at[8];   // this lane's pieces of its row of a sub-tile
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) row_at[kk] = &sh[0][r][((kk * 2 + hh) ^ (r & 15)) * 8];
+    for (int ct0 = from; ct0 < end; ct0 += NB * CT) {
+#pragma unroll
+      for (int buf = 0; buf < NB; ++buf) {   // (unrolled: the buffer is in the offset of every LDS read)
+        const int ct = ct0 + buf * CT;
+        if (ct >= end) break;
+        km_wait_vm<(NB - 2) * L>();   // this tile's loads of this wave have landed ...
+        asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
+        tile_load(ct + (NB - 1) * CT, buf == 0 ? NB - 1 : buf - 1);
+        if (LISTED) tile_rows(ct + NB * CT, end);
+        uint4 rows[AHEAD ? AHEAD : 1];
+        const auto operand = [&](int k) {
+          return *reinterpret_cast<const uint4*>(row_at[k % 8] + (buf * CT + k / 8 * 32) * RI_DIM);
+        };
+        if (AHEAD) {
+#pragma unroll
+          for (int kk = 0; kk < AHEAD; ++kk) rows[kk] = operand(kk);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int half = 0; half < CT / 32; ++half) {
+          if (ct + half * 32 < end) {  // uniform: only the last tile can lack sub-tiles
+            f32x16_t acc[TT];
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+              const int k = half * 8 + kk;
+              const uint4 a = AHEAD ? rows[k % (AHEAD ? AHEAD : 1)] : operand(k);
+#pragma unroll
+              for (int tt = 0; tt < TT; ++tt)
+                acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                                        __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
+                               : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
+                                                                         0, 0);
+              if (AHEAD) {
+                if (k + AHEAD < CT / 4) rows[k % (AHEAD ? AHEAD : 1)] = operand(k + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+            }
+            if (LISTED && ct + half * 32 + 32 > end) {   // uniform: rows past the last score nothing
+              const int left = end - (ct + half * 32) - hh * 4;
+#pragma unroll
+              for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[tt][i] = i / 4 * 8 + i % 4 < left ? acc[tt][i] : -INFINITY;
+            }
+            // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
+            // equal to their maximum is the lowest row; the index search only runs when some lane
+            // of the wave improves on its best (about half of the sub-tiles of a full-size pass)
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+              // (both halves from a score seen before, which is no NaN: nine instructions.  From the second best where that is
+              // wanted: it then is the larger of the two wherever the best stays.)
+              float low8 = track ? second[tt] : best[tt], high8 = low8, low4 = low8, high4 = low8;
+#pragma unroll
+              for (int i = 0; i < 8; ++i) {
+                low8 = fmaxf(low8, acc[tt][i]);
+                high8 = fmaxf(high8, acc[tt][8 + i]);
+                if (i == 3) low4 = low8, high4 = high8;
+              }
+              float m;
+              asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(low8), "v"(high8));   // (no NaN: the compiler would quiet one first)
+              const bool upd = m > best[tt];
+              if (!track) {
+                if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+                  const int k = km_first_of(acc[tt], m, best[tt], low8, low4, high4, hh * 4 + ct + half * 32);
+                  at[tt] = upd ? k : at[tt];
+                  best[tt] = m;
+                }
+              } else if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+                float s;
+                const int k = km_first_two(acc[tt], m, low8, high8, low4, high4, hh * 4 + ct + half * 32, s);
+                asm("v_max_f32_e32 %0, %1, %2" : "=v"(s) : "v"(s), "v"(best[tt]));
+                second[tt] = upd ? s : m;
+                at[tt] = upd ? k : at[tt];
+                best[tt] = upd ? m : best[tt];
+              } else {
+                second[tt] = m;
+              }
+            }
+          }
+        }
+      }
     }
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[tt][kk].x), "+v"(b[tt][kk].y), "+v"(b[tt][kk].z), "+v"(b[tt][kk].w));
+    for (int tt = 0; tt < TT; ++tt) asm volatile("" : "+v"(best[tt]), "+v"(at[tt]));   // (one register each, whichever way out)
+    km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's, or that another turn fills)
   }
+  // both halves of a wave have scored every other four rows for the same tokens: best, its place and second best of all
+  __device__ __forceinline__ void merged(int tt, float& top, int& place, float& next_best) {
+    const float ob = km_other(best[tt], hh);
+    const int oi = __float_as_int(km_other(__int_as_float(at[tt]), hh));
+    const bool other = ob > best[tt] || (ob == best[tt] && oi < at[tt]);
+    next_best = fmaxf(fminf(ob, best[tt]), ri_xor_max<32>(second[tt]));
+    top = other ? ob : best[tt];
+    place = other ? oi : at[tt];
+  }
+};
 
-  float best[KM_TT];
-  int bidx[KM_TT];
+template <int TT, int CT, int W, int NB, bool HALF>
+__global__ __launch_bounds__(W * 64) void km_assign_kernel(const uint16_t* __restrict__ data, const uint16_t* __restrict__ cent,
+                                                           int32_t* __restrict__ assign, int N, int nc, int seg,
+                                                           int64_t head_rows, int sh) {
+  typedef KmScan<TT, CT, W, NB, HALF, false> Scan;
+  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[NB][CT][RI_DIM];
+  const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
+  Scan s(sh_c, cent + (size_t)p * nc * RI_DIM, nc);
+  const int t0 = (blockIdx.x >> sh) * Scan::TOKENS + s.wave * (32 * TT);
+  s.request_tokens(data + km_row0(p, seg, head_rows, N) * RI_DIM, t0, N - 1);
+  s.start(0, nc);
+  s.take_tokens();
+  s.nothing_yet();
+  s.score(0, nc, false);
 #pragma unroll
-  for (int tt = 0; tt < KM_TT; ++tt) {
-    best[tt] = -INFINITY;
-    bidx[tt] = 0;
+  for (int tt = 0; tt < TT; ++tt) {
+    float top, second;
+    int place;
+    s.merged(tt, top, place, second);
+    const int tok = t0 + tt * 32 + s.r;
+    if (s.hh == 0 && tok < N) assign[(size_t)p * N + tok] = place;
   }
-  const uint16_t* row_at[8];   // this lane's pieces of its row of a sub-tile
+}
+
+// A pass of a clustering that knows the pass before (KmBounds), grid (ceil(N / TOKENS), P).  The clusters that no token has
+// joined or left keep their centroids, most keys win against unit vectors by their norm, and a token whose second best score
+// is known needs no more than the centroids that were written since: the same scores, hence the same assignment, of far fewer
+// products.  8 x 131072 tokens, 8192 centroids, us of ten passes: 10 x 1524 -> 1524 (all), 1308, 585, 105 and 73 + 391 (keys
+// left: 81, 38, 4 and 0.1 %; a fifth of the tokens is left open by the last), 1700 (all, with the second best: its search is
+// what a full pass loses by it), 1481 + 67, 722 + 61, 463 + 54 and 324 + 40 (90, 46, 28 and 19 % of the centroids written, 3 to
+// 1.6 % of the tokens open).  Two columns of tokens and small tiles: with a short list the load of the tokens is the launch, and
+// three workgroups per compute unit overlap it (19 % of 8192: 324, of which 55 are the bytes; four columns, 8 waves: 393;
+// one column: 450).  The problems' workgroups are dealt over all chiplets, unlike those of a plain pass: problems take unequal
+// time (12943 -> 14059 with a problem to a chiplet).
+template <int TT, int CT, int W, int NB, bool HALF>
+__global__ __launch_bounds__(W * 64, TT == 2 ? 3 : 2) void km_assign_again_kernel(
+    const uint16_t* __restrict__ data, const uint16_t* __restrict__ cent, int32_t* __restrict__ assign, int N, int nc, int seg,
+    int64_t head_rows, KmBounds B) {
+  typedef KmScan<TT, CT, W, NB, HALF, true> Scan;
+  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[NB][CT][RI_DIM];
+  __shared__ int sh_open[W + 1];   // uncertain tokens of every wave, then where the workgroup's go
+  extern __shared__ __attribute__((aligned(16))) uint16_t list[];   // the centroids in the order they are scored
+  const int p = blockIdx.y, wg0 = blockIdx.x * Scan::TOKENS;
+  const size_t first_token = (size_t)p * N, first_centroid = (size_t)p * nc;
+  Scan s(sh_c, cent + first_centroid * RI_DIM, nc);
+  s.list = list;
+  const int t0 = wg0 + s.wave * (32 * TT);
+  s.request_tokens(data + km_row0(p, seg, head_rows, N) * RI_DIM, t0, N - 1);
+  const int mode = B.plan[p].x, n1 = B.plan[p].y;
+  const uint4* const order = reinterpret_cast<const uint4*>(B.order + first_centroid);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < nc / 8; i += W * 64) reinterpret_cast<uint4*>(list)[i] = order[i];
+  s.nothing_yet();
+  if (mode == KM_NEW) {   // (scores up to the bound are of no interest)
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) row_at[kk] = &sh_c[0][r][((kk * 2 + hh) ^ (r & 15)) * 8];
-  for (int ct0 = 0; ct0 < nc; ct0 += KM_NB * KM_CT) {
+    for (int tt = 0; tt < TT; ++tt) {
+      s.best[tt] = s.second[tt] = B.bound[first_token + min(t0 + tt * 32 + s.r, N - 1)];
+      s.at[tt] = nc - 1;   // (unless one does: uncertain below)
+    }
+  }
+  __syncthreads();
+  s.start(0, max(n1, 1));
+  s.take_tokens();
+  bool track = mode != KM_KEYS;
+  for (int part = 0, from = 0, end = n1;; part = 1, from = mode == KM_KEYS ? n1 : 0, end = nc) {
+    s.score(from, end, track);
+    const bool whole = part == 1 || mode == KM_ALL;
+    int rr = s.r;
+    asm volatile("" : "+v"(rr));   // (what follows from it is computed here and not kept through the loop)
+    int id[TT], old[TT];
+    float top[TT], bound[TT];
+    uint32_t sure = 0;
+    int uncertain = 0;
 #pragma unroll
-    for (int buf = 0; buf < KM_NB; ++buf) {   // (unrolled: the buffer is in the offset of every LDS read)
-      const int ct = ct0 + buf * KM_CT;
-      if (ct >= nc) break;
-      km_wait_vm<(KM_NB - 2) * L>();   // this tile's loads of this wave have landed ...
-      asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
-      tile_load(ct + (KM_NB - 1) * KM_CT, buf == 0 ? KM_NB - 1 : buf - 1);
-      // Operands from LDS: each is requested AHEAD products before its own, into the register that a product has just read, across
-      // sub-tiles where a tile has several.  (The compiler has two on their way and waits for each; as many more as the
-      // registers hold.  8 x 8192 tokens, 512 centroids: 10.2 -> 9.3 us, 16 x 8200 22.4 -> 20.7, 4 x 48719, 3072 119 -> 118,
-      // 128 x 8192 120.6 -> 117.6, 8 x 131072, 8192 1531 -> 1512.)
-      constexpr int AHEAD = KM_TT == 2 ? 3 : KM_CT == 32 ? 0 : KM_TT == 4 ? 4 : 8;
-      uint4 rows[AHEAD ? AHEAD : 1];
-      const auto operand = [&](int at) {
-        return *reinterpret_cast<const uint4*>(row_at[at % 8] + (buf * KM_CT + at / 8 * 32) * RI_DIM);
-      };
-      if (AHEAD) {
+    for (int tt = 0; tt < TT; ++tt) {
+      int place;
+      s.merged(tt, top[tt], place, bound[tt]);
+      const int tok = t0 + tt * 32 + rr;
+      const size_t t = first_token + min(tok, N - 1);
+      old[tt] = assign[t];
+      id[tt] = top[tt] > -INFINITY ? list[place] : 0;
+      bool ok = true;
+      if (part == 1) {
+        ok = !(top[tt] == bound[tt]) || top[tt] == -INFINITY;   // (a tie across the two turns: not in the order of ids)
+      } else if (mode == KM_NEW) {
+        // its own centroid, where that was not written, scores what it did
+        const float limit = B.bound[t], own = B.best[t];
+        if (!(B.state[first_centroid + old[tt]] & KM_MOVED)) {
+          const bool stay = own > top[tt] || (own == top[tt] && old[tt] < id[tt]);
+          bound[tt] = fmaxf(bound[tt], fminf(own, top[tt]));
+          id[tt] = stay ? old[tt] : id[tt];
+          top[tt] = stay ? own : top[tt];
+        }
+        ok = top[tt] > limit;
+      } else if (mode == KM_KEYS) {
+        // |x c| <= |x| |c|, and a centroid that an update has written is a unit vector rounded to 16 bits (and this sum,
+        // like the scores, to 32: far inside the hundredth)
+        float sq = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < AHEAD; ++kk) rows[kk] = operand(kk);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float lo, hi;
+            uint32_t word = (&s.b[tt][kk].x)[i];
+            asm volatile("" : "+v"(word));   // (here, and not ahead of the loop: the registers are full)
+            ri_unpack2<HALF>(word, lo, hi);
+            sq = fmaf(lo, lo, fmaf(hi, hi, sq));
+          }
+        ok = top[tt] > 1.01f * sqrtf(ri_xor_sum<32>(sq)) + 1e-17f && !B.odd[p];   // (1e-17: squares too small for a float)
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if (ok) sure |= 1u << tt;
+      uncertain += __popcll(__builtin_amdgcn_ballot_w64(!ok && s.hh == 0 && tok < N));
+    }
+    // Where most of a workgroup's tokens are uncertain it looks at the other centroids itself; else one addition in memory
+    // reserves the places of all of its open tokens (one address takes an addition every 40 ns or so: one per wave and column
+    // was 20 us of 8 x 20000 tokens).
+    if (s.lane == 0) sh_open[s.wave] = uncertain;
+    __syncthreads();
+    int all = 0, at = 0;
 #pragma unroll
-      for (int half = 0; half < KM_CT / 32; ++half) {
-        if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
-          f32x16_t acc[KM_TT];
+    for (int w = 0; w < W; ++w) {
+      if (w < s.wave) at += sh_open[w];
+      all += sh_open[w];
+    }
+    all = __builtin_amdgcn_readfirstlane(all);
+    if (!whole) {
+      if (4 * all > 3 * min(Scan::TOKENS, N - wg0)) {
+        __syncthreads();
+        track = true;
+        if (mode == KM_NEW) s.nothing_yet();
+        s.start(mode == KM_KEYS ? n1 : 0, nc);
+        continue;
+      }
+    }
+    if (all) {
+      if (threadIdx.x == 0) sh_open[W] = atomicAdd(&B.open_count[p], all);
+      __syncthreads();
+      at += sh_open[W];
+    }
 #pragma unroll
-          for (int tt = 0; tt < KM_TT; ++tt)
+    for (int tt = 0; tt < TT; ++tt) {
+      const int tok = t0 + tt * 32 + rr;
+      const bool mine = s.hh == 0 && tok < N, ok = sure >> tt & 1;
+      if (mine && ok) km_settle(B, assign, first_token + tok, first_centroid, id[tt], old[tt], top[tt], bound[tt]);
+      const uint64_t left = __builtin_amdgcn_ballot_w64(mine && !ok);
+      if (mine && !ok) B.open[first_token + at + __popcll(left & ((1ull << s.lane) - 1ull))] = tok;
+      at += __popcll(left);
+    }
+    return;
+  }
+}
+
+template <bool HALF>
+using KmOpenScan = KmScan<2, 32, 4, 4, HALF, false>;
+
+// The tokens that a pass left open (a few in a hundred), against all centroids, grid KM_OPEN_WGS: blocks of a problem's open tokens, each cut into
+// as many parts of the centroids as there are workgroups for; the last of a block's parts to arrive puts them together.
+// (What the others wrote reaches it by write-through stores that are complete before they arrive.)  Bound by the matrix cores
+// where there are many (210000 of 8 x 131072, 8192 centroids: 391 us, a full pass's rate), else by its chain: 400 tokens of
+// eight problems, 640 centroids: 10.5 us, 17 while the parts were put together one after the other.
+template <bool HALF>
+__global__ __launch_bounds__(256) void km_assign_open_kernel(const uint16_t* __restrict__ data,
+                                                                const uint16_t* __restrict__ cent, int32_t* __restrict__ assign,
+                                                                int N, int nc, int seg, int64_t head_rows, KmBounds B) {
+  typedef KmOpenScan<HALF> Scan;
+  constexpr int TT = 2;
+  static_assert(!Scan::TURN && Scan::TOKENS == 4 * 32 * TT, "tokens by name");
+  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[4][32][RI_DIM];
+  __shared__ int sh_last;
+  const int lane = threadIdx.x & 63;
+  // blocks of every problem, a lane per problem
+  const int blocks = lane < B.P ? (B.open_count[lane] + Scan::TOKENS - 1) / Scan::TOKENS : 0;
+  const int incl = (int)ri_wave_incl_scan((uint32_t)blocks), items = __builtin_amdgcn_readlane(incl, 63);
+  if (items == 0) return;
+  const int parts = min(max((int)gridDim.x / items, 1), min(KM_OPEN_PARTS, nc / 32));
+  for (int w = blockIdx.x; w < items * parts; w += gridDim.x) {
+    const int item = w / parts, part = w % parts;
+    const int p = __ffsll((long long)__builtin_amdgcn_ballot_w64(incl > item)) - 1;
+    const int block = item - (__builtin_amdgcn_readlane(incl, p) - __builtin_amdgcn_readlane(blocks, p));
+    const size_t first_token = (size_t)p * N, first_centroid = (size_t)p * nc;
+    const int32_t* const open = B.open + first_token;
+    const int n = __builtin_amdgcn_readfirstlane(B.open_count[p]);
+    const int from = (int)((int64_t)(nc / 32) * part / parts) * 32, end = (int)((int64_t)(nc / 32) * (part + 1) / parts) * 32;
+    Scan s(sh_c, cent + first_centroid * RI_DIM, nc);
+    const int t0 = block * Scan::TOKENS + s.wave * (32 * TT);
+    s.request_tokens(data + km_row0(p, seg, head_rows, N) * RI_DIM, t0, n - 1, open);
+    s.start(from, end);
+    s.take_tokens();
+    s.nothing_yet();
+    s.score(from, end, true);
+    int last = 1;
+    int32_t* const mine = B.partial + (size_t)w * 3 * Scan::TOKENS + s.wave * (32 * TT) + s.r;
+    if (parts > 1) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
+      for (int tt = 0; tt < TT; ++tt) {
+        float top, second;
+        int place;
+        s.merged(tt, top, place, second);
+        if (s.hh == 0) {
+          __hip_atomic_store(mine + tt * 32, __float_as_int(top), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(mine + tt * 32 + Scan::TOKENS, __float_as_int(second), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(mine + tt * 32 + 2 * Scan::TOKENS, place, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      km_wait_vm<0>();
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        int32_t* const arrived = B.arrived + item;
+        last = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        if (last) __hip_atomic_store(arrived, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh_last = last;
+      }
+      __syncthreads();
+      last = __builtin_amdgcn_readfirstlane(sh_last);
+    }
+    if (last) {
 #pragma unroll
-          for (int kk = 0; kk < 8; ++kk) {
-            const int at = half * 8 + kk;
-            const uint4 a = AHEAD ? rows[at % (AHEAD ? AHEAD : 1)] : operand(at);
+      for (int tt = 0; tt < TT; ++tt) {
+        float top, second;
+        int place;
+        s.merged(tt, top, place, second);
+        const int at = t0 + tt * 32 + s.r;
+        if (s.hh == 0 && at < n) {
+          if (parts > 1) {
+            top = second = -INFINITY;
+            place = 0;
+            int32_t v[KM_OPEN_PARTS][3];   // (all on their way before the first is looked at)
 #pragma unroll
-            for (int tt = 0; tt < KM_TT; ++tt)
-              acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
-                                                                      __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
-                             : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
-                                                                       0, 0);
-            if (AHEAD) {
-              if (at + AHEAD < KM_CT / 4) rows[at % (AHEAD ? AHEAD : 1)] = operand(at + AHEAD);
-              __builtin_amdgcn_sched_barrier(0);
+            for (int q = 0; q < KM_OPEN_PARTS; ++q)
+#pragma unroll
+              for (int k = 0; k < 3; ++k)
+                v[q][k] = __hip_atomic_load(mine + ((ptrdiff_t)(min(q, parts - 1) - part) * 3 + k) * Scan::TOKENS + tt * 32,
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int q = 0; q < KM_OPEN_PARTS; ++q) {   // (ascending centroids: a tie stays where it is)
+              if (q >= parts) break;
+              const float a = __int_as_float(v[q][0]);
+              second = fmaxf(fmaxf(second, __int_as_float(v[q][1])), fminf(top, a));
+              place = a > top ? v[q][2] : place;
+              top = fmaxf(top, a);
             }
           }
-          // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
-          // equal to their maximum is the lowest row; the index search only runs when some lane
-          // of the wave improves on its best (about half of the sub-tiles of a full-size pass)
-#pragma unroll
-          for (int tt = 0; tt < KM_TT; ++tt) {
-            // (both halves from the best so far, which is no NaN: nine instructions)
-            float low8 = best[tt], high8 = best[tt], low4 = best[tt], high4 = best[tt];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              low8 = fmaxf(low8, acc[tt][i]);
-              high8 = fmaxf(high8, acc[tt][8 + i]);
-              if (i == 3) low4 = low8, high4 = high8;
-            }
-            float m;
-            asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(low8), "v"(high8));   // (no NaN: the compiler would quiet one first)
-            const bool upd = m > best[tt];
-            if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
-              const int at = km_first_of(acc[tt], m, best[tt], low8, low4, high4, hh * 4 + ct + half * 32);
-              bidx[tt] = upd ? at : bidx[tt];
-              best[tt] = m;
-            }
-          }
+          const int tok = open[at];
+          km_settle(B, assign, first_token + tok, first_centroid, place, assign[first_token + tok], top, second);
         }
       }
     }
-  }
-  km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's)
-#pragma unroll
-  for (int tt = 0; tt < KM_TT; ++tt) {
-    const float ob = __shfl_xor(best[tt], 32);
-    const int oi = __shfl_xor(bidx[tt], 32);
-    if (ob > best[tt] || (ob == best[tt] && oi < bidx[tt])) {
-      best[tt] = ob;
-      bidx[tt] = oi;
-    }
-    const int tok = t0 + tt * 32 + r;
-    if (hh == 0 && tok < N) assign[(size_t)p * N + tok] = bidx[tt];
+    __syncthreads();   // (the tile buffers, and sh_last)
   }
 }
 
@@ -691,14 +1091,17 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
   }
 }
 
+// odd (where it is asked for): set if the squares underflow or are no numbers, so that the result's norm need not be one
 template <bool MEAN, bool HALF>
-__device__ __forceinline__ void km_finish(float s0, float s1, int count, int normalize, uint32_t* op) {
+__device__ __forceinline__ void km_finish(float s0, float s1, int count, int normalize, uint32_t* op,
+                                          int32_t* odd = nullptr) {
   if (MEAN) {
     const float cnt = (float)count;
     s0 = s0 / cnt;
     s1 = s1 / cnt;
     if (normalize) {
       const float nrm = sqrtf(ri_wave_sum(s0 * s0 + s1 * s1));  // two roundings: built without fp contraction
+      if (odd && !(nrm >= 1e-15f)) *odd = 1;
       s0 = s0 / nrm;
       s1 = s1 / nrm;
     }
@@ -734,6 +1137,71 @@ __device__ __forceinline__ int km_slot_owner(const int32_t* __restrict__ off, in
   return lo;
 }
 
+// What an update of a clustering reads and writes of KmBounds (state == nullptr: every cluster is summed, nothing is kept)
+struct KmMoves {
+  int32_t* state;
+  uint8_t* touched;
+  uint16_t* order;
+  ri_int2* plan;
+  int32_t *open_count, *odd;
+  int first;   // nothing is known of the clusters yet
+};
+__device__ __forceinline__ int32_t km_next_state(int32_t state, int size, int touched) {
+  const int moved = touched && size > 0;   // (an empty cluster keeps its centroid)
+  return size << KM_SIZE_SHIFT | (state & KM_UNIT) | (moved ? KM_MOVED | KM_UNIT | (state & KM_UNIT ? 0 : KM_FRESH) : 0);
+}
+
+// How the next pass goes about problem p, by one workgroup of 256; a thread takes nc / 256 consecutive centroids (up to 64: a
+// bit of a word each).
+__device__ __forceinline__ void km_plan(const KmMoves& M, int p, int N, int nc) {
+  __shared__ int sums[3][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int each = (nc + 1023) / 1024 * 4, c0 = min((int)threadIdx.x * each, nc), n = min(each, nc - c0);
+  const int4* const state = reinterpret_cast<const int4*>(M.state + (size_t)p * nc + c0);
+  const bool known = !M.first && M.plan[p].x != KM_KEYS;
+  uint64_t moved = 0, keys = 0;
+  int fresh = 0;
+#pragma unroll 8
+  for (int i = 0; i < n; i += 4) {
+    const int4 e = state[i / 4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int w = (&e.x)[j];
+      moved |= (uint64_t)(w & KM_MOVED ? 1 : 0) << (i + j);
+      keys |= (uint64_t)(w & KM_UNIT ? 0 : 1) << (i + j);
+      fresh += w & KM_FRESH ? w >> KM_SIZE_SHIFT : 0;
+    }
+  }
+  // (both counts in one scan: at most 16384 each)
+  const uint32_t both = (uint32_t)__popcll(moved) | (uint32_t)__popcll(keys) << 16, incl = ri_wave_incl_scan(both);
+  const int fresh_incl = (int)ri_wave_incl_scan((uint32_t)fresh);
+  if (lane == 63) {
+    sums[0][wave] = (int)incl;
+    sums[1][wave] = fresh_incl;
+  }
+  __syncthreads();
+  uint32_t all = 0, before = incl - both;
+  int all_fresh = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) before += (uint32_t)sums[0][w];
+    all += (uint32_t)sums[0][w];
+    all_fresh += sums[1][w];
+  }
+  const int all_keys = (int)(all >> 16);
+  const int mode = 2 * (int64_t)all_fresh >= N ? all_keys > 0 ? KM_KEYS : KM_ALL : known ? KM_NEW : KM_ALL;
+  const int n1 = mode == KM_ALL ? nc : mode == KM_KEYS ? all_keys : (int)(all & 0xffffu);
+  const uint64_t first = mode == KM_ALL ? 0ull : mode == KM_KEYS ? keys : moved;
+  int at1 = mode == KM_ALL ? 0 : mode == KM_KEYS ? (int)(before >> 16) : (int)(before & 0xffffu);
+  int at2 = mode == KM_ALL ? c0 : n1 + c0 - at1;
+  uint16_t* const order = M.order + (size_t)p * nc;
+  for (int i = 0; i < n; ++i) order[first >> i & 1 ? at1++ : at2++] = (uint16_t)(c0 + i);
+  if (threadIdx.x == 0) {
+    M.plan[p] = (ri_int2){mode, n1};
+    M.open_count[p] = 0;
+  }
+}
+
 // grid (item workgroups + ceil(nc / 4), P), four waves each.  The first item_wgs workgroups take
 // one slot per wave (blocks of long lists, their fp32 sums go to partial[p][slot]); the others one
 // cluster per wave.
@@ -746,7 +1214,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
                                                float2* __restrict__ partial, int item_wgs, int cap, int N, int nc,
                                                int seg, int64_t head_stride, int normalize,
                                                uint16_t* __restrict__ copy, int64_t copy_stride,
-                                               const uint16_t* __restrict__ mean) {
+                                               const uint16_t* __restrict__ mean, const KmMoves& M = KmMoves{}) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int32_t* off = offsets + (size_t)p * (nc + 1);
@@ -759,7 +1227,8 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
     const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (slot >= cap) return;
     int s, o, j;
-    if (km_slot_owner(off, nc, slot, s, o, j) < 0) return;
+    const int c = km_slot_owner(off, nc, slot, s, o, j);
+    if (c < 0 || (M.state && !M.first && !M.touched[(size_t)p * nc + c])) return;
     float s0 = 0.f, s1 = 0.f;
     km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1,
                                         pitch, COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
@@ -769,6 +1238,12 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
   const int c = ((int)blockIdx.x - item_wgs) * 4 + (threadIdx.x >> 6);
   if (c >= nc) return;
   const int s = counts[(size_t)p * nc + c];
+  if (M.state) {   // (touched is cleared by the fold's launch)
+    const size_t at = (size_t)p * nc + c;
+    const int touched = M.first || M.touched[at];
+    if (lane == 0) M.state[at] = km_next_state(M.first ? 0 : M.state[at], s, touched);
+    if (!touched) return;   // the tokens of the update before, in the same order: it has their mean
+  }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
   if (s == 0) {
     if (!MEAN) *op = 0u;  // empty cluster: zero value sum; the centroid is left untouched
@@ -778,7 +1253,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
   float s0 = 0.f, s1 = 0.f;
   km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1, pitch,
                                       COPY ? wp + (size_t)off[c] * (RI_DIM / 2) : nullptr, mw);
-  km_finish<MEAN, HALF>(s0, s1, s, normalize, op);
+  km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);
 }
 
 template <bool MEAN, bool HALF, bool COPY>
@@ -789,9 +1264,9 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
                                                         uint16_t* __restrict__ out, float2* __restrict__ partial,
                                                         int item_wgs, int cap, int N, int nc, int seg,
                                                         int64_t head_stride, int normalize,
-                                                        uint16_t* __restrict__ copy, int64_t copy_stride) {
+                                                        uint16_t* __restrict__ copy, int64_t copy_stride, KmMoves M) {
   km_reduce_rows<MEAN, HALF, COPY, false>(rows, pitch, counts, offsets, members, out, partial, item_wgs, cap, N, nc, seg,
-                                          head_stride, normalize, copy, copy_stride, nullptr);
+                                          head_stride, normalize, copy, copy_stride, nullptr, M);
 }
 
 // Value sums with the value store (z = 0) and means of the centred keys with the key store (z = 1): the last step of a
@@ -823,14 +1298,17 @@ __global__ __launch_bounds__(256) void km_store_kernel(KmStoreArgs V, KmStoreArg
 // order and finishes the cluster
 template <bool MEAN, bool HALF>
 __device__ __forceinline__ void km_fold(const int32_t* __restrict__ offsets, const float2* __restrict__ partial,
-                                        uint16_t* __restrict__ out, int cap, int nc, int normalize) {
+                                        uint16_t* __restrict__ out, int cap, int nc, int normalize,
+                                        const KmMoves& M = KmMoves{}) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (M.state)
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < nc; c += gridDim.x * 256) M.touched[(size_t)p * nc + c] = 0;
   if (slot >= cap) return;
   int s, o, j;
   const int c = km_slot_owner(offsets + (size_t)p * (nc + 1), nc, slot, s, o, j);
-  if (c < 0 || j != 0) return;
+  if (c < 0 || j != 0 || (M.state && !(M.state[(size_t)p * nc + c] & KM_MOVED))) return;
   const int nb = (s + KM_BLK - 1) / KM_BLK;
   const float2* pp = partial + ((size_t)p * cap + slot) * 64 + lane;
   float2 t = pp[0];
@@ -851,15 +1329,16 @@ __device__ __forceinline__ void km_fold(const int32_t* __restrict__ offsets, con
     t.y += v.y;
   }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
-  km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op);
+  km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op, M.state ? M.odd + p : nullptr);
 }
 
 template <bool MEAN, bool HALF>
 __global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __restrict__ offsets,
                                                              const float2* __restrict__ partial,
                                                              uint16_t* __restrict__ out, int cap, int nc,
-                                                             int normalize) {
-  km_fold<MEAN, HALF>(offsets, partial, out, cap, nc, normalize);
+                                                             int normalize, KmMoves M, int N) {
+  if (M.state && blockIdx.x == gridDim.x - 1) km_plan(M, blockIdx.y, N, nc);   // (a workgroup of its own: no slot is left)
+  km_fold<MEAN, HALF>(offsets, partial, out, cap, nc, normalize, M);
 }
 
 template <bool HALF>
@@ -1218,12 +1697,10 @@ static int km_assign_args(const void* data, const void* centroids, const int32_t
 }
 
 template <bool HALF>
-static int km_assign(const void* data, const void* centroids, int32_t* assign, int P, int N, int nc, int seg,
-                     int64_t head_rows, ri_stream_t stream) {
-  int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
-  if (rc) return rc;
+static void km_assign_launch(const void* data, const void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                             int64_t head_rows, hipStream_t stream) {
 #define KM_ASSIGN_LAUNCH(TT, CT, W, NB)                                                                                  \
-  km_assign_kernel<TT, CT, W, NB, HALF><<<km_grid((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, (hipStream_t)stream>>>( \
+  km_assign_kernel<TT, CT, W, NB, HALF><<<km_grid((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, stream>>>( \
       (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P))
   const long long wgs128 = (long long)P * ((N + 127) / 128), wgs256 = (long long)P * ((N + 255) / 256);
   const long long wgs768 = (long long)P * ((N + 767) / 768);
@@ -1253,6 +1730,25 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
   // 32.7, 34.6, 43.9, 36.5).
   else KM_ASSIGN_LAUNCH(2, 32, 4, 4);
 #undef KM_ASSIGN_LAUNCH
+}
+
+// a pass that knows the one before, and the tokens that it left open
+template <bool HALF>
+static void km_assign_again(const void* data, const void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                            int64_t head_rows, const KmBounds& B, hipStream_t stream) {
+  typedef KmScan<2, 32, 4, 4, HALF, true> Scan;
+  km_assign_again_kernel<2, 32, 4, 4, HALF><<<dim3((N + Scan::TOKENS - 1) / Scan::TOKENS, P), 256, (size_t)nc * 2, stream>>>(
+      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, B);
+  km_assign_open_kernel<HALF><<<KM_OPEN_WGS, 256, 0, stream>>>((const uint16_t*)data, (const uint16_t*)centroids,
+                                                                         assign, N, nc, seg, head_rows, B);
+}
+
+template <bool HALF>
+static int km_assign(const void* data, const void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                     int64_t head_rows, ri_stream_t stream) {
+  int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
+  if (rc) return rc;
+  km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, (hipStream_t)stream);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
@@ -1335,7 +1831,7 @@ template <bool MEAN, bool HALF, bool COPY>
 static int km_reduce(const void* rows, int64_t head_stride, int64_t row_stride, const int32_t* counts,
                      const int32_t* offsets, const int32_t* members, void* out, int P, int N, int nc, int seg,
                      int normalize, void* copy, int64_t copy_stride, void* workspace, size_t workspace_bytes,
-                     hipStream_t s) {
+                     hipStream_t s, const KmMoves& M = KmMoves{}) {
   if (workspace_bytes < ri_kmeans_reduce_workspace_bytes(P, N, nc)) return RI_ERR_WORKSPACE;
   const int cap = km_item_cap(N);
   float2* partial = (float2*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
@@ -1343,10 +1839,10 @@ static int km_reduce(const void* rows, int64_t head_stride, int64_t row_stride, 
   if ((long long)item_wgs + (nc + 3) / 4 > 0x7fffffffLL) return RI_ERR_ARG;
   km_reduce_kernel<MEAN, HALF, COPY><<<dim3(item_wgs + (nc + 3) / 4, P), 256, 0, s>>>(
       (const uint16_t*)rows, (size_t)row_stride / 2, counts, offsets, members, (uint16_t*)out, partial, item_wgs, cap, N,
-      nc, seg, head_stride / 2, normalize, (uint16_t*)copy, copy_stride);
+      nc, seg, head_stride / 2, normalize, (uint16_t*)copy, copy_stride, M);
   RI_HIP_CHECK_LAUNCH();
-  km_reduce_fold_kernel<MEAN, HALF><<<dim3(item_wgs, P), 256, 0, s>>>(offsets, partial, (uint16_t*)out, cap, nc,
-                                                                      normalize);
+  km_reduce_fold_kernel<MEAN, HALF><<<dim3(item_wgs + (M.state ? 1 : 0), P), 256, 0, s>>>(offsets, partial, (uint16_t*)out,
+                                                                                          cap, nc, normalize, M, N);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
@@ -1441,6 +1937,119 @@ extern "C" int ri_kmeans_update_direct_f16(const void* data, const int32_t* assi
                                            int64_t head_rows, int normalize, ri_stream_t stream) {
   return km_update_direct<true>(data, assign, centroids, counts, offsets, members, P, N, nc, seg, head_rows, normalize,
                                 stream);
+}
+
+// ------------------------------------------------------------------------------------
+// the iterations of a clustering
+// ------------------------------------------------------------------------------------
+// Whether passes know the ones before.  They read every token again (8 x 131072: 55 us), which short passes are bound by
+// anyway, and each is one launch more (5 us, 10 with a few tokens open).  Ten assignments and nine updates, us without / with,
+// by problems, tokens and centroids, keys in clusters (as many as centroids) with four large dimensions | without any structure:
+// 8 x 16400, 512: 486 / 569 | 432 / 510; 8 x 20000, 640: 611 / 648 | 529 / 588; 1 x 65536, 2048: 687 / 753 | 518 / 645; 8 x
+// 20000, 1248: 807 / 775 | 727 / 610; 8 x 32768, 1024: 971 / 947 | 861 / 860; 2 x 65536, 2048: 976 / 890 | 824 / 798; 1 x
+// 131072, 2720: 1161 / 1045 | 1010 / 1074; 4 x 32768, 2048: 893 / 785 | 818 / 647; 2 x 65536, 4096: 1422 / 1094 | 1343 / 921;
+// 8 x 65536, 1376: 1922 / 1640 | 1810 / 1828; 1 x 131072, 8192: 2563 / 1804 | 2365 / 1455; 8 x 131072, 8192: 15863 / 9751 |
+// two of those 4125 / 2345.  So from 2^28 scores a pass on.  (Up to 16384 tokens the lists never leave a workgroup, and a pass is
+// bound by its keys.  64 problems: a lane each where the open tokens are dealt out; 16384 centroids: their order in LDS.)
+static bool km_bounded(int P, int N, int nc) {
+  return N > KM_DIRECT_MAX && P <= 64 && nc <= 16384 && (int64_t)P * N * nc >= 1ll << 28;
+}
+
+__global__ __launch_bounds__(KM_OPEN_WGS + 64) void km_clear_kernel(int32_t* p, int n) {
+  if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
+}
+
+static size_t km_align256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+struct KmIterateSpace {
+  size_t state, touched, best, bound, order, plan, open, open_count, partial, cleared, counts, offsets, members, lists, reduce, all;
+};
+static KmIterateSpace km_iterate_space(int P, int N, int nc) {
+  KmIterateSpace w;
+  size_t at = 0;
+  const auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += km_align256(bytes);
+    return here;
+  };
+  const size_t tokens = (size_t)P * N, clusters = (size_t)P * nc;
+  const bool bounded = km_bounded(P, N, nc), lists = N > KM_DIRECT_MAX;
+  w.state = take(bounded ? clusters * 4 : 0);
+  w.touched = take(bounded ? clusters : 0);
+  w.best = take(bounded ? tokens * 4 : 0);
+  w.bound = take(bounded ? tokens * 4 : 0);
+  w.order = take(bounded ? clusters * 2 : 0);
+  w.plan = take(bounded ? (size_t)P * 8 : 0);
+  w.open = take(bounded ? tokens * 4 : 0);
+  w.open_count = take(bounded ? (size_t)P * 4 : 0);
+  w.partial = take(bounded ? (size_t)KM_OPEN_WGS * 3 * KmOpenScan<false>::TOKENS * 4 : 0);
+  w.cleared = take(bounded ? (size_t)(KM_OPEN_WGS + P) * 4 : 0);   // arrivals, odd
+  w.counts = take(lists ? clusters * 4 : 0);
+  w.offsets = take(lists ? (clusters + P) * 4 : 0);
+  w.members = take(lists ? tokens * 4 : 0);
+  w.lists = take(lists ? ri_kmeans_workspace_bytes(P, N, nc) : 0);
+  w.reduce = take(lists ? ri_kmeans_reduce_workspace_bytes(P, N, nc) : 0);
+  w.all = at + 256;
+  return w;
+}
+
+extern "C" size_t ri_kmeans_iterate_workspace_bytes(int P, int N, int nc) {
+  if (P <= 0 || N <= 0 || nc <= 0) return 0;
+  return km_iterate_space(P, N, nc).all;
+}
+
+template <bool HALF>
+static int km_iterate(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg, int64_t head_rows,
+                      int updates, int last, void* workspace, size_t workspace_bytes, ri_stream_t stream) {
+  int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
+  if (rc) return rc;
+  if (updates < 0 || !workspace || (N > KM_DIRECT_MAX && nc > (1 << 18))) return RI_ERR_ARG;   // (lists of two digits)
+  const KmIterateSpace w = km_iterate_space(P, N, nc);
+  if (workspace_bytes < w.all) return RI_ERR_WORKSPACE;
+  const bool bounded = km_bounded(P, N, nc);
+  hipStream_t s = (hipStream_t)stream;
+  char* const base = (char*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  const KmBounds B = {(float*)(base + w.best), (float*)(base + w.bound), (const int32_t*)(base + w.state),
+                      (uint8_t*)(base + w.touched), (const uint16_t*)(base + w.order), (const ri_int2*)(base + w.plan),
+                      (int32_t*)(base + w.open), (int32_t*)(base + w.open_count), (int32_t*)(base + w.partial),
+                      (int32_t*)(base + w.cleared), (const int32_t*)(base + w.cleared) + KM_OPEN_WGS, P};
+  KmMoves M = {bounded ? (int32_t*)(base + w.state) : nullptr, B.touched, (uint16_t*)(base + w.order), (ri_int2*)(base + w.plan),
+               B.open_count, B.arrived + KM_OPEN_WGS, 1};
+  if (bounded) {
+    km_clear_kernel<<<1, KM_OPEN_WGS + 64, 0, s>>>(B.arrived, KM_OPEN_WGS + P);
+    RI_HIP_CHECK_LAUNCH();
+  }
+  for (int i = 0; i < updates + (last ? 1 : 0); ++i) {
+    if (bounded && i > 0) km_assign_again<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, B, s);
+    else km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, s);
+    RI_HIP_CHECK_LAUNCH();
+    if (i == updates) break;
+    if (N <= KM_DIRECT_MAX) {
+      rc = km_direct_launch<HALF>(data, assign, centroids, nullptr, nullptr, nullptr, P, N, nc, seg, head_rows, 1, stream);
+      if (rc) return rc;
+      continue;
+    }
+    int32_t *const counts = (int32_t*)(base + w.counts), *const offsets = (int32_t*)(base + w.offsets),
+            *const members = (int32_t*)(base + w.members);
+    rc = km_build_lists(assign, counts, offsets, members, P, N, nc, base + w.lists, s);
+    if (rc) return rc;
+    M.first = i == 0;
+    rc = km_reduce<true, HALF, false>(data, head_rows * RI_DIM, RI_DIM, counts, offsets, members, centroids, P, N, nc, seg, 1,
+                                      nullptr, 0, base + w.reduce, ri_kmeans_reduce_workspace_bytes(P, N, nc), s, M);
+    if (rc) return rc;
+  }
+  return RI_OK;
+}
+
+extern "C" int ri_kmeans_iterate(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                                 int64_t head_rows, int updates, int last, void* workspace, size_t workspace_bytes,
+                                 ri_stream_t stream) {
+  return km_iterate<false>(data, centroids, assign, P, N, nc, seg, head_rows, updates, last, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ri_kmeans_iterate_f16(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg,
+                                     int64_t head_rows, int updates, int last, void* workspace, size_t workspace_bytes,
+                                     ri_stream_t stream) {
+  return km_iterate<true>(data, centroids, assign, P, N, nc, seg, head_rows, updates, last, workspace, workspace_bytes, stream);
 }
 
 template <bool HALF>

@@ -604,6 +604,14 @@ def kmeans_lists_direct(assign, counts, offsets, members, P, N, nc):
           "kmeans_lists_direct")
 
 
+def kmeans_iterate(data, centroids, assign, P, N, nc, seg, head_rows, updates, last):
+    """`updates` rounds of kmeans_assign and a normalised update, then one more assignment if `last`."""
+    nbytes = lib().ri_kmeans_iterate_workspace_bytes(P, N, nc)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=data.device)
+    check(_fn("ri_kmeans_iterate", data.dtype)(_p(data), _p(centroids), _p(assign), P, N, nc, seg, head_rows, updates,
+                                               int(bool(last)), _p(ws), nbytes, _stream()), "kmeans_iterate")
+
+
 def _rows_ok(t):
     return t.stride(-1) == 1 and t.stride(-2) % 8 == 0 and t.stride(-3) % 8 == 0 and t.data_ptr() % 16 == 0
 

@@ -408,3 +408,68 @@ def test_update_direct_equals_lists_and_update(dev, P, N, nc, kind):
 def test_update_direct_at_the_ends_of_runs(dev, P, N):
     for kind in ("even", "skew"):
         test_update_direct_equals_lists_and_update(dev, P, N, 512, kind)
+
+
+def _passes_one_by_one(keys, cent, seg, updates, last):
+    """What ri_kmeans_iterate stands for: plain assignments and updates."""
+    from retrievalattention_amd import kernels
+    G, N, _ = keys.shape
+    n, nc, P = N // seg, cent.shape[1] // seg, G * seg
+    assign, members = (torch.empty(P, n, dtype=torch.int32, device=keys.device) for _ in range(2))
+    counts = torch.empty(P, nc, dtype=torch.int32, device=keys.device)
+    offsets = torch.empty(P, nc + 1, dtype=torch.int32, device=keys.device)
+    for i in range(updates + last):
+        kernels.kmeans_assign(keys, cent, assign, P, n, nc, seg, N)
+        if i < updates:
+            kernels.kmeans_build_lists(assign, counts, offsets, members, P, n, nc)
+            kernels.kmeans_update(keys, counts, offsets, members, cent, P, n, nc, seg, N, True)
+    return assign, cent
+
+
+# The smallest problems whose passes know of each other, with remainders of tokens and of the list's last sub-tile; the most
+# centroids, the most problems, segments with tokens left over; and shapes on the other side of the line.
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("kind", ["mixture", "normal", "ties", "odd"])
+@pytest.mark.parametrize("G,N,nc,seg", [(3, 45001, 2080, 1), (1, 17001, 16384, 1), (64, 16385, 288, 1), (2, 50003, 8192, 2),
+                                        (1, 20001, 64, 1), (2, 3001, 192, 3)])
+def test_iterate_equals_its_passes(dev, G, N, nc, seg, kind, dt):
+    """Bit for bit the centroids and the assignment of the passes run one by one."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator(device=dev).manual_seed(N + nc)
+    keys = torch.randn(G, N, 128, generator=g, device=dev)
+    if kind == "mixture":      # clusters of keys with a few large dimensions: the largest keys take every token at first
+        centres = torch.randn(G, max(N // 16, 1), 128, generator=g, device=dev)
+        centres[:, :, :4] *= 8
+        label = torch.randint(centres.shape[1], (G, N), generator=g, device=dev)
+        keys = torch.gather(centres, 1, label[..., None].expand(G, N, 128)) + 0.3 * keys
+    elif kind == "ties":       # small whole numbers in few dimensions: keys and scores come many times over
+        keys = torch.randint(-2, 3, (G, N, 128), generator=g, device=dev).float()
+        keys[:, :, 6:] = 0
+    elif kind == "odd":        # keys without a norm of any size (their mean's is no number), infinities, and no numbers
+        keys[:, ::3] *= 1e-30 if dt == torch.bfloat16 else 0
+        keys[:, 5::4001] = float("inf")
+        keys[:, 9::5003, 7] = float("nan")
+    keys = keys.to(dt).contiguous()
+    start = torch.empty(G, nc, 128, dtype=dt, device=dev)
+    kernels.kmeans_init(keys, start, G, N, nc)
+    for updates, last in ((9, True), (4, False), (0, True)):
+        want, cent = _passes_one_by_one(keys, start.clone(), seg, updates, last)
+        mine = start.clone()
+        got = torch.full_like(want, -1)
+        kernels.kmeans_iterate(keys, mine, got, G * seg, N // seg, nc // seg, seg, N, updates, last)
+        assert torch.equal(got, want)
+        assert torch.equal(mine.view(torch.int16), cent.view(torch.int16))
+
+
+def test_iterate_refuses(dev):
+    from retrievalattention_amd import _lib
+    lib = _lib.lib()
+    keys = torch.zeros(1, 64, 128, dtype=torch.bfloat16, device=dev)
+    cent = torch.zeros(1, 32, 128, dtype=torch.bfloat16, device=dev)
+    assign = torch.empty(1, 64, dtype=torch.int32, device=dev)
+    nbytes = lib.ri_kmeans_iterate_workspace_bytes(1, 64, 32)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    call = lambda nc=32, updates=1, room=nbytes, p=ws.data_ptr(): lib.ri_kmeans_iterate(
+        keys.data_ptr(), cent.data_ptr(), assign.data_ptr(), 1, 64, nc, 1, 64, updates, 1, p, room, 0)
+    assert call() == 0
+    assert call(nc=33) != 0 and call(updates=-1) != 0 and call(room=nbytes - 1) != 0 and call(p=None) != 0
