@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, r
   P.W_kv = n[3];
   P.lenB_ptr_stride = len[0];
   P.lenA = len[1];
-  attend_group<GS_PAD, HALF, false>(P, blockIdx.x, blockIdx.y, AttendKept{});
+  attend_group<GS_PAD, HALF, KEPT_NONE>(P, blockIdx.x, blockIdx.y, AttendKept{});
 }
 
 // ------------------------------------------------------------------------------------
@@ -116,14 +116,14 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 //  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
 //    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
 static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
-                        int max_splits = RI_MAX_SPLITS) {
+                        int max_splits = RI_MAX_SPLITS, bool several = false) {
   const int64_t rows = kv_rows + es_rows, wk = kv_rows * 512, we = es_rows * es_row_bytes;
   int64_t per_group = 256 / BG;
   per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
   per_group = min(per_group, (int64_t)max_splits);
   if (per_group > 8 && per_group % 8 * 5 <= per_group && rows <= 64 * ATT_WAVES * per_group) per_group -= per_group % 8;
-  if (attend_alone(rows, gs, BG) || per_group < 1) per_group = 1;
+  if ((!several && attend_alone(rows, gs, BG)) || per_group < 1) per_group = 1;
   const int waves = (int)per_group * ATT_WAVES;
   P.S = (int)per_group;
   P.W_kv = waves;
@@ -186,7 +186,7 @@ int ri_prepare_wave_attention(AttendParams* out_params, const void* q, const voi
                               const int32_t* ret_tok_off, const int32_t* ret_start, int np, const int32_t* meta,
                               const int32_t* est_ids, const float* logits, const void* est_centroids, const void* value_sum,
                               const void* cluster_size_bf16, void* out, int32_t* valid_lengths, int BG, int gs, int nc,
-                              int es, float scale, void* scratch, size_t scratch_bytes, bool one_workgroup) {
+                              int es, float scale, void* scratch, size_t scratch_bytes, int plan) {
   if (!q || !steady_k || !steady_v || !store_k || !store_v || !meta || !out || !scratch) return RI_ERR_ARG;
   if (ri_any_misaligned16(q, steady_k, steady_v, store_k, store_v, value_sum, est_centroids, out, scratch))
     return RI_ERR_ARG;
@@ -233,7 +233,7 @@ int ri_prepare_wave_attention(AttendParams* out_params, const void* q, const voi
   // capacity scaled by the usual fill (a quarter) or for 16 tokens per rank, the estimation zone by
   // its exact size
   plan_splits(P, static_len + (row_src ? row_src_stride / 4 : np * 16), es,
-              est_row_bytes(gs, est_centroids != nullptr), BG, gs, one_workgroup ? 1 : RI_MAX_SPLITS);
+              est_row_bytes(gs, est_centroids != nullptr), BG, gs, plan == ATT_ONE ? 1 : RI_MAX_SPLITS, plan == ATT_SEVERAL);
   if (scratch_bytes < attn_scratch_used(BG, gp, P.S)) return RI_ERR_WORKSPACE;
   carve_workspace(P, scratch, BG, gp);
   *out_params = P;
@@ -263,7 +263,7 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   const int rc = ri_prepare_wave_attention(&P, q, steady_k, steady_v, steady_stride, static_len, static_len_dev, store_k,
                                            store_v, store_stride, row_src, row_src_stride, ret_tok_off, ret_start, np, meta,
                                            est_ids, logits, est_centroids, value_sum, cluster_size_bf16, out, valid_lengths,
-                                           BG, gs, nc, es, scale, scratch, scratch_bytes, false);
+                                           BG, gs, nc, es, scale, scratch, scratch_bytes, ATT_PLAN);
   if (rc) return rc;
   P.src_lo = max(src_lo, 0);
   P.src_hi = src_hi;

@@ -336,15 +336,28 @@ __device__ __forceinline__ void attend_rows(WaveState<GS_PAD>& st, const WaveLds
 // The rank tables of the retrieval zone (np + 1 token offsets, np first rows) live in dynamic LDS, sized by
 // the launch, so that any number of probes the selection accepts can be attended.
 // HALF: q, K, V, value sums, cluster sizes, weights and outputs are IEEE half instead of bfloat16.
-// KEPT: the workgroup has just made the selection, whose tables, ids and logits are in LDS (K); it has the whole group.
+// KEPT: the workgroup has just made the selection, whose tables and ids are in LDS (K), from KEPT_LOGITS on the logits too.
+// KEPT_ALL: it has the whole group.
+enum { KEPT_NONE, KEPT_TABLES, KEPT_LOGITS, KEPT_ALL };
 struct AttendKept {
   const float* logits;   // [nc][GS_PAD]
   const int* est;        // [es]
   int* off;              // [np + 1]
   int* start;            // [np]
+  uint4 q;               // this thread's piece of the query (att_query_piece), requested ahead of the selection
+  int lenA;              // the steady zone's rows
 };
 
-template <int GS_PAD, bool HALF, bool KEPT>
+// piece threadIdx.x % 16 of the query of head threadIdx.x / 16
+__device__ __forceinline__ uint4 att_query_piece(const AttendParams& P, int g) {
+  const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
+  return ri_ld16(P.q + ((size_t)g * P.gs + min(head, P.gs - 1)) * RI_DIM + piece * 8);
+}
+__device__ __forceinline__ int att_steady_rows(const AttendParams& P) {
+  return P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
+}
+
+template <int GS_PAD, bool HALF, int KEPT>
 __device__ __forceinline__ void attend_group(const AttendParams& P, const int g, const int split, const AttendKept& K) {
   constexpr int NW = ATT_WAVES;
   constexpr int NH = GS_PAD / 4;
@@ -374,7 +387,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, h = lane >> 4;
-  const int gs = P.gs, S = KEPT ? 1 : P.S;
+  const int gs = P.gs, S = KEPT == KEPT_ALL ? 1 : P.S;
 
   WaveState<GS_PAD> st;
 #pragma unroll
@@ -387,7 +400,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(sh.pb)[i] = 0u;
   if (lane < 16) sh.al[lane] = 1.f;
   const int lenB = KEPT ? K.off[P.np] : P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  const int lenA = P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
+  const int lenA = KEPT ? K.lenA : att_steady_rows(P);
 
   const int wid = split * NW + wave;            // wave of the group
   const bool kv_wave = wid < P.W_kv;
@@ -416,7 +429,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
     static_assert(GS_PAD * (RI_DIM / 8) <= NT, "one piece of the query per thread");
     {
       const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
-      uint4 qv = ri_ld16(P.q + ((size_t)g * gs + min(head, gs - 1)) * RI_DIM + piece * 8);
+      uint4 qv = KEPT ? K.q : att_query_piece(P, g);
       if (head >= gs) qv = ri_zero16();
       if (head < GS_PAD) *reinterpret_cast<uint4*>(&sh_q[head][piece * 8]) = qv;
     }
@@ -433,7 +446,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
         if (i < P.np) sh_rst[i] = P.ret_start[(size_t)g * P.np + i];
       }
     }
-    __syncthreads();
+    if (KEPT) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (the selection's stores stay in flight)
+    else __syncthreads();
   }
 
   if (kv_wave || (!KEPT && P.est_cent)) {
@@ -525,7 +539,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
 #pragma unroll
           for (int i = 0; i < NH; ++i) {
             const int head = min(ri_head_of<GS_PAD>(h, i), gs - 1);
-            k.x[i] = KEPT ? K.logits[dk * GS_PAD + head] : lg[(size_t)head * P.nc + dk];
+            k.x[i] = KEPT >= KEPT_LOGITS ? K.logits[dk * GS_PAD + head] : lg[(size_t)head * P.nc + dk];
           }
           k.size = cs[dk];
 #pragma unroll
@@ -592,7 +606,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
     if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
     return;
   }
-  if constexpr (!KEPT) {
+  if constexpr (KEPT != KEPT_ALL) {
 
   // ---------------- last workgroup of the group merges all splits ----------------
   // Hand-off of the partials between workgroups of one launch, without fences:
@@ -628,12 +642,13 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   }
 }
 
-// Checks the arguments of ri_wave_attention and lays them down with their split plan (attend.hip).  one_workgroup: a group
-// is not split.
+// Checks the arguments of ri_wave_attention and lays them down with their split plan (attend.hip), as the launch plans it by
+// itself, or with one workgroup per group, or without the rule that leaves a few rows to one.
+enum { ATT_PLAN, ATT_ONE, ATT_SEVERAL };
 int ri_prepare_wave_attention(AttendParams* P, const void* q, const void* steady_k, const void* steady_v,
                               int64_t steady_stride, int static_len, const int32_t* static_len_dev, const void* store_k,
                               const void* store_v, int64_t store_stride, const int32_t* row_src, int row_src_stride,
                               const int32_t* ret_tok_off, const int32_t* ret_start, int np, const int32_t* meta,
                               const int32_t* est_ids, const float* logits, const void* est_centroids, const void* value_sum,
                               const void* cluster_size_bf16, void* out, int32_t* valid_lengths, int BG, int gs, int nc,
-                              int es, float scale, void* scratch, size_t scratch_bytes, bool one_workgroup);
+                              int es, float scale, void* scratch, size_t scratch_bytes, int plan);

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(ri_ptr4 in, ri_int4 n,
   P.np = n[2];
   P.es = n[3];
   P.ntiles = ntiles;
-  select_group<NT, E, GSM, HALF, SRC, false>(P, blockIdx.x, SelectKept{});
+  select_group<NT, E, GSM, HALF, SRC, KEEP_NONE>(P, blockIdx.x, SelectKept{});
 }
 
 // ------------------------------------------------------------------------------------
@@ -503,6 +503,21 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
   return RI_OK;
 }
 
+static int launch_dist(const SelectArgs& P, int BG, bool half, hipStream_t s) {
+  const dim3 grid((P.nc + DIST_IDS - 1) / DIST_IDS, BG);
+  auto* kernel = P.gs <= 4   ? (half ? dist_kernel<4, true> : dist_kernel<4, false>)
+                 : P.gs <= 8 ? (half ? dist_kernel<8, true> : dist_kernel<8, false>)
+                             : (half ? dist_kernel<16, true> : dist_kernel<16, false>);
+  kernel<<<grid, 256, 0, s>>>(P.logits, P.tile_max, P.tile_sum, P.mask, P.keys, P.dist_out, P.gs, P.nc, P.ntiles);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+int ri_launch_select_inputs(const SelectArgs& P, int BG, bool half, bool keys, hipStream_t s) {
+  const int rc = ri_launch_score(P.q, P.cent, P.logits, P.tile_max, P.tile_sum, BG, P.gs, P.nc, P.scale, half, s);
+  return rc || !keys ? rc : launch_dist(P, BG, half, s);
+}
+
 static int score_select_impl(const void* q, const void* centroids, const uint8_t* mask,
                              const int32_t* cluster_size_i32, const int32_t* cluster_start, float* logits, void* dist,
                              int64_t* cI, int32_t* ret_ids, int32_t* est_ids, int32_t* ret_tok_off, int32_t* ret_start,
@@ -545,19 +560,7 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }
-  const dim3 dgrid((nc + DIST_IDS - 1) / DIST_IDS, BG);
-#define RI_DIST_LAUNCH(GSM)                                                                                       \
-  do {                                                                                                            \
-    if (half)                                                                                                     \
-      dist_kernel<GSM, true><<<dgrid, 256, 0, s>>>(logits, tmax, tsum, mask, keys, (uint16_t*)dist, gs, nc, ntiles); \
-    else                                                                                                          \
-      dist_kernel<GSM, false><<<dgrid, 256, 0, s>>>(logits, tmax, tsum, mask, keys, (uint16_t*)dist, gs, nc, ntiles); \
-  } while (0)
-  if (gs <= 4) RI_DIST_LAUNCH(4);
-  else if (gs <= 8) RI_DIST_LAUNCH(8);
-  else RI_DIST_LAUNCH(16);
-#undef RI_DIST_LAUNCH
-  RI_HIP_CHECK_LAUNCH();
+  if ((rc = launch_dist(P, BG, half, s))) return rc;
   const int per_thread = (nc + SEL_THREADS - 1) / SEL_THREADS;
 #define RI_SELECT_LAUNCH_T(E8, R, BPT)                                                                               \
   select_kernel<E8, R, BPT><<<BG, SEL_THREADS, 0, s>>>(keys, cluster_size_i32, cluster_start, cI, ret_ids, est_ids,  \

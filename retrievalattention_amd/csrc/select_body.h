@@ -104,16 +104,22 @@ __device__ __forceinline__ uint32_t wave_offset(const uint32_t* sh, uint32_t* to
 
 // Where the rest of a workgroup that goes on with the attention finds the selection (LDS).
 struct SelectKept {
-  float* logits;   // [nc][GSM]
+  float* logits;   // [nc][GSM]: SEL_SCORE
   int* est;        // [es]
   int* off;        // [np + 1]
   int* start;      // [np]
+  int* ids;        // [np] KEEP_TABLES
+  int* meta;       // [4] KEEP_TABLES
 };
+enum { KEEP_NONE, KEEP_TABLES, KEEP_ALL };
 
-// GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well.
-template <int NT, int E, int GSM, bool HALF, int SRC, bool KEEP>
+// GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well, with
+// KEEP_TABLES in place of memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
+template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP>
 __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K) {
-  static_assert(!KEEP || (SRC == SEL_SCORE && GSM <= 8), "the logits are in LDS");
+  static_assert(KEEP == KEEP_NONE || SRC != SEL_SCORE || GSM <= 8, "the logits are in LDS");
+  static_assert(KEEP != KEEP_ALL || SRC == SEL_SCORE, "what is not kept is in memory");
+  constexpr bool STORE = KEEP != KEEP_TABLES;
   constexpr int NW = NT / 64, IDS = NT * E;
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
   constexpr int SHIFT = 16 - (LOGT + 2), FB = 1 << SHIFT;   // lower bits of a key, fine bins
@@ -256,7 +262,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
           const float mj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), j));
           const float izj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iz), j));
           d[0] += ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[j]) - mj) * izj);
-          if (cbeg < nc) P.logits[((size_t)g * gs + j) * nc + cbeg] = x[j];
+          if (STORE && cbeg < nc) P.logits[((size_t)g * gs + j) * nc + cbeg] = x[j];
         }
       } else {
 #pragma unroll
@@ -501,25 +507,26 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   // ---- all global stores ----
   // (behind every load: a load's wait covers the stores in front of it)
   if (in) {
-    P.ret_ids[(size_t)g * np + tid] = my_c;
-    if (P.cI) P.cI[(size_t)g * k2 + tid] = my_c;
+    if (STORE) P.ret_ids[(size_t)g * np + tid] = my_c;
+    else K.ids[tid] = my_c;
+    if (STORE && P.cI) P.cI[(size_t)g * k2 + tid] = my_c;
   }
   {
     uint32_t at = est_first;
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       if ((est_bits >> i) & 1u) {
-        P.est_ids[(size_t)g * es + at] = cbeg + i;
+        if (STORE) P.est_ids[(size_t)g * es + at] = cbeg + i;
         if (KEEP) K.est[at] = cbeg + i;
-        if (P.cI) P.cI[(size_t)g * k2 + np + at] = cbeg + i;
+        if (STORE && P.cI) P.cI[(size_t)g * k2 + np + at] = cbeg + i;
         ++at;
       }
     }
   }
   if (!P.cluster_size) return;
   if (in) {
-    P.ret_tok_off[(size_t)g * (np + 1) + tid] = (int32_t)((tid < nkeep) ? tok : T_ret);
-    if (P.ret_start) P.ret_start[(size_t)g * np + tid] = st;
+    if (STORE) P.ret_tok_off[(size_t)g * (np + 1) + tid] = (int32_t)((tid < nkeep) ? tok : T_ret);
+    if (STORE && P.ret_start) P.ret_start[(size_t)g * np + tid] = st;
     if (KEEP) {
       K.off[tid] = (int)((tid < nkeep) ? tok : T_ret);
       K.start[tid] = st;
@@ -527,13 +534,14 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   }
   if (tid == 0) {
     if (KEEP) K.off[np] = (int)T_ret;
-    P.ret_tok_off[(size_t)g * (np + 1) + np] = (int32_t)T_ret;
-    P.meta[g * 4 + 0] = nkeep;
-    P.meta[g * 4 + 1] = (int32_t)T_ret;
-    P.meta[g * 4 + 2] = (int32_t)pages;
-    P.meta[g * 4 + 3] = 0;
+    int32_t* const meta = STORE ? P.meta + g * 4 : K.meta;
+    if (STORE) P.ret_tok_off[(size_t)g * (np + 1) + np] = (int32_t)T_ret;
+    meta[0] = nkeep;
+    meta[1] = (int32_t)T_ret;
+    meta[2] = (int32_t)pages;
+    meta[3] = 0;
   }
-  if (P.row_src && P.cluster_start && keep) {   // row table: each kept cluster writes the rows of its tokens
+  if (STORE && P.row_src && P.cluster_start && keep) {   // row table: each kept cluster writes the rows of its tokens
     int32_t* dst = P.row_src + (size_t)g * P.row_src_stride + tok;
     const int room = P.row_src_stride - (int)tok;
     for (int k = 0; k < (int)sz && k < room; ++k) dst[k] = st + k;
@@ -546,3 +554,6 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
                       int32_t* ret_ids, int32_t* est_ids, int32_t* ret_tok_off, int32_t* ret_start, int32_t* row_src,
                       int row_src_stride, int32_t* meta, int BG, int gs, int nc, int np, int es, int page, int max_pages,
                       float scale, void* workspace, size_t workspace_bytes);
+
+// Scoring, and the scores' sums and keys if `keys` (select.hip)
+int ri_launch_select_inputs(const SelectArgs& P, int BG, bool half, bool keys, hipStream_t s);

@@ -37,22 +37,42 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
   return RI_OK;
 }
 
+// What a selection with KEEP_TABLES left in LDS goes to memory, by one of the workgroups that made it and when its rows are
+// attended.
+__device__ __forceinline__ void store_selection(const SelectArgs& S, int g, const SelectKept& K) {
+  const int np = S.np, es = S.es, tid = threadIdx.x;
+  for (int i = tid; i < np; i += 64 * ATT_WAVES) {
+    S.ret_ids[(size_t)g * np + i] = K.ids[i];
+    S.ret_start[(size_t)g * np + i] = K.start[i];
+  }
+  for (int i = tid; i <= np; i += 64 * ATT_WAVES) S.ret_tok_off[(size_t)g * (np + 1) + i] = K.off[i];
+  for (int i = tid; i < es; i += 64 * ATT_WAVES) S.est_ids[(size_t)g * es + i] = K.est[i];
+  if (tid < 4) S.meta[g * 4 + tid] = K.meta[tid];
+}
+
 // ------------------------------------------------------------------------------------
-// step: scoring, selection and attention of a group by one workgroup, for short contexts.
-// With up to 512 clusters the selection is one workgroup per group that scores for itself, and with few rows the attention
-// is, too: as one kernel the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
+// step: scoring, selection and attention of a group in one launch, for short contexts.
+// With up to 512 clusters the selection is one workgroup per group that scores for itself: as one kernel with the attention
+// the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
 // host as well.  What bounds it is the chain of either half on one compute unit.  8 groups of 4 heads, 512 clusters, 331
 // rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110060 bytes of LDS (119532 with 8 heads): one
-// workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.  step_route.h says which steps take it.
+// workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.
+// SPLIT: several workgroups per group, which all make the same selection and attend a part of the rows each (see
+// select_attend_kernel): with the query and the zone's length requested ahead of the selection and its results stored behind
+// the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 523 / 843 / 1099 rows:
+// 15.0 / 17.3 / 19.8 / 22.7 us with one workgroup, 14.6 / 14.6 / 14.8 / 16.5 with several (16.3 .. 18.8 in two launches); the
+// retrieval of 10 % of the clusters, 8 groups of 8 heads 20.7 -> 19.0 (two launches -> SPLIT), 16 of 4 20.8 -> 19.4, 128 of 8
+// 33.6 -> 31.7.  step_route.h says which step takes which form.
 // ------------------------------------------------------------------------------------
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
-template <int GSM, bool HALF>
+template <int GSM, bool HALF, bool SPLIT>
 __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int4 n, float scale, SelectArgs S0, AttendParams A0) {
   static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
   __shared__ __attribute__((aligned(16))) float sh_logits[STEP_CLUSTERS * GSM];
   static_assert(__alignof__(sh_logits) == 16, "read four heads at a time");
-  __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS];
+  __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS], sh_ids[SPLIT ? STEP_CLUSTERS : 1],
+      sh_meta[4];
   SelectArgs S = S0;
   AttendParams A = A0;
   S.cent = ri_global<const uint16_t>(in[0]);
@@ -64,12 +84,83 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.np = A.np = n[2];
   S.es = A.es = n[3];
   S.scale = A.scale = scale;
-  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, true>(S, blockIdx.x, SelectKept{sh_logits, sh_est, sh_off, sh_start});
+  const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta};
+  const AttendKept known = {sh_logits, sh_est, sh_off, sh_start, att_query_piece(A, blockIdx.x), att_steady_rows(A)};
+  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, SPLIT ? KEEP_TABLES : KEEP_ALL>(S, blockIdx.x, kept);
   lds_barrier();
-  attend_group<GSM, HALF, true>(A, blockIdx.x, 0, AttendKept{sh_logits, sh_est, sh_off, sh_start});
+  attend_group<GSM, HALF, SPLIT ? KEPT_LOGITS : KEPT_ALL>(A, blockIdx.x, SPLIT ? blockIdx.y : 0, known);
+  if (SPLIT && blockIdx.y == 0) {
+    store_selection(S, blockIdx.x, kept);
+    const int nc = S.nc;
+    for (int j = 0; j < S.gs; ++j)
+      if ((int)threadIdx.x < nc) S.logits[((size_t)blockIdx.x * S.gs + j) * nc + threadIdx.x] = sh_logits[threadIdx.x * GSM + j];
+  }
 }
 
-static int step_short(const ri_decode_step_t* s, const void* q, int static_len, void* out, hipStream_t stream) {
+// ------------------------------------------------------------------------------------
+// select + attend, behind the scoring: the attention's workgroups of a group each make the group's selection and go on with its
+// tables in LDS.  The compute units that repeat it would wait for it otherwise; a launch, and the tables' way through memory, are
+// left out.  The query's pieces and the zone's length are requested ahead of the selection, and one of the workgroups stores its
+// results when its rows are attended (a load's wait covers the stores in front of it): without both 19.0, 47.5 and 26.2 us in
+// the first, second and third of these steps (captured, 4 layers a graph; in launches of their own -> joined): 16 groups of 4
+// heads, 1024 clusters 21.0 -> 18.9; 32 of 4, 8192 48.8 -> 47.0; 12 of 7, 1920 27.5 -> 25.6; 64 of 8, 16384 139.9 -> 138.2; 8 of
+// 4, 2048 22.3 -> 20.2; 1 of 4, 8192 27.5 -> 25.8; 8 of 8, 4096 28.0 -> 25.9; 32 of 16, 4096 41.2 -> 38.6; 4 of 12, 8192 35.0 ->
+// 33.2; 16 of 1, 1920 22.2 -> 20.0; 320 of 8, 1280 70.2 -> 65.2; 512 of 4, 1024 71.2 -> 68.0.
+// What bounds it is the selection's chain (see select_body.h), then what bounds the attention.
+// ------------------------------------------------------------------------------------
+template <int E, int GSM, bool HALF, int SRC>
+__global__ __launch_bounds__(64 * ATT_WAVES, 2) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int4 m, SelectArgs S0,
+                                                                          AttendParams A0) {
+  extern __shared__ __attribute__((aligned(16))) int sh_kept[];
+  SelectArgs S = S0;
+  AttendParams A = A0;
+  if (SRC == SEL_KEYS) {
+    S.keys = ri_global<uint16_t>(in[0]);
+  } else {
+    S.logits = ri_global<float>(in[0]);
+    S.tile_max = ri_global<float>(in[1]);
+    S.tile_sum = ri_global<float>(in[2]);
+  }
+  S.mask = ri_global<const uint8_t>(in[3]);
+  S.nc = A.nc = n[0];
+  S.gs = A.gs = n[1];
+  S.np = A.np = n[2];
+  S.es = A.es = n[3];
+  S.ntiles = m[0];
+  A.S = m[1];
+  A.W_kv = m[2];
+  const int np = S.np, g = blockIdx.x;
+  int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
+  const SelectKept kept = {nullptr, est, off, start, ids, meta};
+  const AttendKept known = {nullptr, est, off, start, att_query_piece(A, g), att_steady_rows(A)};
+  select_group<64 * ATT_WAVES, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept);
+  lds_barrier();
+  attend_group<GSM, HALF, KEPT_TABLES>(A, g, blockIdx.y, known);
+  if (blockIdx.y == 0) store_selection(S, g, kept);
+}
+
+template <int E, int SRC>
+static void launch_select_attend(const SelectArgs& S, const AttendParams& A, int BG, bool half, hipStream_t stream) {
+  const void* a = SRC == SEL_KEYS ? (const void*)S.keys : (const void*)S.logits;
+  auto* kernel = S.gs <= 4   ? (half ? select_attend_kernel<E, 4, true, SRC> : select_attend_kernel<E, 4, false, SRC>)
+                 : S.gs <= 8 ? (half ? select_attend_kernel<E, 8, true, SRC> : select_attend_kernel<E, 8, false, SRC>)
+                             : (half ? select_attend_kernel<E, 16, true, SRC> : select_attend_kernel<E, 16, false, SRC>);
+  const size_t lds = (size_t)(4 + 3 * S.np + 1 + S.es) * sizeof(int);
+  kernel<<<dim3(BG, A.S), 64 * ATT_WAVES, lds, stream>>>(ri_pack_ptrs(a, S.tile_max, S.tile_sum, S.mask),
+                                                         (ri_int4){S.nc, S.gs, S.np, S.es}, (ri_int4){S.ntiles, A.S, A.W_kv, 0}, S,
+                                                         A);
+}
+
+template <bool SPLIT>
+static void launch_step(const SelectArgs& S, const AttendParams& A, int BG, bool half, hipStream_t stream) {
+  auto* kernel = S.gs <= 4 ? (half ? step_kernel<4, true, SPLIT> : step_kernel<4, false, SPLIT>)
+                           : (half ? step_kernel<8, true, SPLIT> : step_kernel<8, false, SPLIT>);
+  kernel<<<dim3(BG, A.S), 64 * ATT_WAVES, 0, stream>>>(ri_pack_ptrs(S.cent, S.q, S.mask, S.cluster_size),
+                                                       (ri_int4){S.nc, S.gs, S.np, S.es}, S.scale, S, A);
+}
+
+// The step in one launch (nc <= STEP_CLUSTERS, up to eight heads), or in scoring and one more.
+static int step_joined(const ri_decode_step_t* s, const void* q, int static_len, bool alone, void* out, hipStream_t stream) {
   SelectArgs S;
   int rc = ri_prepare_select(&S, q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,
                              s->ret_ids, s->est_ids, s->ret_tok_off, s->ret_start, nullptr, 0, s->meta, s->BG, s->gs, s->nc,
@@ -81,19 +172,36 @@ static int step_short(const ri_decode_step_t* s, const void* q, int static_len, 
                                  s->store_v, s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta,
                                  s->est_ids, s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out,
                                  s->valid_lengths, s->BG, s->gs, s->nc, s->es, s->scale, s->attn_workspace,
-                                 s->attn_workspace_bytes, true);
+                                 s->attn_workspace_bytes, alone ? ATT_ONE : S.nc <= STEP_CLUSTERS ? ATT_SEVERAL : ATT_PLAN);
   if (rc) return rc;
-  auto* kernel = s->gs <= 4 ? (s->half ? step_kernel<4, true> : step_kernel<4, false>)
-                            : (s->half ? step_kernel<8, true> : step_kernel<8, false>);
-  kernel<<<s->BG, 64 * ATT_WAVES, 0, stream>>>(ri_pack_ptrs(S.cent, S.q, S.mask, S.cluster_size),
-                                               (ri_int4){S.nc, S.gs, S.np, S.es}, S.scale, S, A);
+  if (S.nc <= STEP_CLUSTERS) {
+    if (alone) launch_step<false>(S, A, s->BG, s->half, stream);
+    else launch_step<true>(S, A, s->BG, s->half, stream);
+    RI_HIP_CHECK_LAUNCH();
+    return RI_OK;
+  }
+  // Who sums the scores (dist_kernel / the selecting workgroups, us): 32 groups of 4 heads, 8192 clusters 47.4 / 50.3, 5760 39.1 /
+  // 41.8; of 1, 8192 46.1 / 47.4; 8 of 7, 3808 28.0 / 26.7; 8 of 8, 4096 27.1 / 27.2, 32 of 8 33.2 / 33.8; 8 of 16, 2048 28.9 /
+  // 27.9; 12 of 7, 1920 27.5 / 26.2; 32 of 8, 2048 26.8 / 25.3; 64 of 16, 1024 31.4 / 28.9.  (512 threads: eight clusters each
+  // past 2048, and with sixteen heads that is more than the registers hold.)
+  const bool keys = S.nc > (S.gs <= 4 ? 4096 : S.gs <= 8 ? min(4096, 28 * 1024 / S.gs) : 2048);
+  rc = ri_launch_select_inputs(S, s->BG, s->half, keys, stream);
+  if (rc) return rc;
+  if (keys) {
+    if (S.nc <= 4096) launch_select_attend<8, SEL_KEYS>(S, A, s->BG, s->half, stream);
+    else if (S.nc <= 8192) launch_select_attend<16, SEL_KEYS>(S, A, s->BG, s->half, stream);
+    else launch_select_attend<32, SEL_KEYS>(S, A, s->BG, s->half, stream);
+  } else if (S.nc <= 1024) launch_select_attend<2, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  else if (S.nc <= 2048) launch_select_attend<4, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  else launch_select_attend<8, SEL_LOGITS>(S, A, s->BG, s->half, stream);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
 
 extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int static_len, void* out, ri_stream_t stream) {
   if (!s) return RI_ERR_ARG;
-  if (step_is_short(s, static_len)) return step_short(s, q, static_len, out, (hipStream_t)stream);
+  if (step_is_joined(s))
+    return step_joined(s, q, static_len, step_is_short(s, static_len) && step_is_alone(s, static_len), out, (hipStream_t)stream);
   auto* select = s->half ? ri_score_select_f16 : ri_score_select;
   auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
   const int rc = select(q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,

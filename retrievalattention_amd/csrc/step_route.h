@@ -1,5 +1,5 @@
-// Which decode steps one workgroup per group makes in one launch (step_kernel) and which are scoring + selection and
-// attention in launches of their own.  Host code only.
+// Which decode steps one workgroup per group makes in one launch (step_kernel), which several do, and which are scoring +
+// selection and attention in launches of their own.  Host code only.
 #pragma once
 #include <stdint.h>
 
@@ -12,8 +12,9 @@ static inline int gs_pad_of(int gs) { return gs <= 4 ? 4 : (gs <= 8 ? 8 : 16); }
 // compute unit left for a second one.
 static inline bool attend_alone(int64_t rows, int gs, int BG) { return rows * gs_pad_of(gs) <= 384 * 4 || BG > 128; }
 
-// Short: what one workgroup scores for itself (select.hip), and usually (16 tokens per retrieved cluster) no more rows than
-// one workgroup attends as fast as several: 8 groups of 8 heads 424 rows 14.6 us against 15.5, 488: 14.8 / 15.7, 552: 15.9 /
+// Short: what one workgroup may have to itself (step_is_alone: and does).  It scores for itself (select.hip), and usually (16
+// tokens per retrieved cluster) has no more rows than it attends as fast as two launches do (figures of both, before
+// step_is_joined): 8 groups of 8 heads 424 rows 14.6 us against 15.5, 488: 14.8 / 15.7, 552: 15.9 /
 // 15.5; of 4 heads 488: 13.8 / 15.0, 552: 15.4 / 14.8; one group of 8 heads 488: 14.5 / 15.0, 552: 15.6 / 14.9.
 // The rows are not known here when the kernel reads the zone's length from the device, as a captured step does until the
 // zone is full, and never what the retrieved clusters hold:
@@ -35,4 +36,27 @@ static inline bool step_is_short(const ri_decode_step_t* s, int static_len) {
   const int64_t zone = s->static_len_dev ? s->steady_stride : static_len;
   const int64_t pages = (int64_t)s->max_pages * s->page, held = pages < s->store_stride ? pages : s->store_stride;
   return zone + usual <= STEP_ROWS && zone + s->es + held <= STEP_ROWS_CROWDED;
+}
+
+// Selection and attention in one launch, and the scoring too up to STEP_CLUSTERS: what step.hip's kernels hold.  (512 probes:
+// a thread each; 16384 clusters: 32 a thread; with sixteen heads 32 KB of LDS are left for the tables; without sizes and
+// first rows there are none.  A workgroup that scores has a compute unit to itself: 264 groups of 4 heads, 512 clusters 32.5 us
+// in two launches, 37.3 in one.)
+static inline bool step_is_joined(const ri_decode_step_t* s) {
+  if (!s->cluster_size_i32 || !s->cluster_start || s->np > 512) return false;
+  if (s->nc <= STEP_CLUSTERS) return s->gs <= 8 && s->BG <= 256;
+  return s->nc <= 16384 && (s->gs <= 8 || 3 * s->np + s->es <= 8000);
+}
+
+// Of the short steps those that one workgroup per group makes as fast as several, which take the same at any length (us, one /
+// several).  8 groups of 8 heads 225 rows 13.4 / 14.2, 321: 14.1 / 14.2, 353: 14.5 / 14.2, 417: 15.1 / 14.2; of 4 heads 225: 12.7
+// / 13.5, 321: 13.4 / 13.5, 353: 13.7 / 13.5, with 512 clusters 331: 13.9 / 13.8 (a step, 15.2 either way), 523: 16.0 / 13.8; of 1 head 321: 13.0 / 13.1; 32
+// groups of 4 heads 321: 14.2 / 14.2, 417: 15.3 / 14.6.  With two workgroups per group only: 128 groups of 4 heads 417: 16.4 / 17.7,
+// of 8 heads, 512 clusters 587: 21.0 / 21.1; past 128 there is no second one.  A captured step, which starts at the length at hand
+// and ends at the zone's, may grow by a quarter past the line.
+static inline bool step_is_alone(const ri_decode_step_t* s, int static_len) {
+  if (s->BG > 128) return true;
+  const int64_t usual = (int64_t)s->np * 16 + s->es, zone = s->static_len_dev ? s->steady_stride : static_len;
+  const int64_t line = s->BG > 64 ? 640 : 336;
+  return static_len + usual <= line && zone + usual <= line * 5 / 4;
 }

@@ -72,3 +72,21 @@ def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static
             assert torch.equal(a[name], b[name]), name
     wf, gf = want.float(), got.float()
     assert (wf - gf).norm() <= (4e-3 if dtype == torch.bfloat16 else 5e-4) * wf.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BG,gs,nc,np_,es,static,pages,on_device", [
+    # several workgroups per group that score for themselves: many rows, few clusters, no estimation zone, cut pages
+    (3, 8, 512, 51, 119, 98, 1000, False), (2, 4, 504, 512 - 8, 0, 700, 2000, True), (1, 1, 8, 1, 7, 900, 100, False),
+    (5, 7, 384, 38, 100, 300, 20, False), (128, 3, 64, 12, 30, 700, 100, True), (256, 8, 32, 4, 20, 400, 100, False),
+    # scored before: every number of clusters a thread takes, with remainders; who sums the scores; heads padded and not
+    (2, 4, 520, 9, 100, 69, 100, False), (3, 8, 1024, 18, 237, 70, 200, True), (2, 16, 1032, 40, 300, 69, 300, False),
+    (1, 12, 2048, 36, 475, 500, 200, False), (2, 9, 2056, 512, 300, 69, 2000, False), (1, 3, 4096, 73, 950, 0, 300, True),
+    (2, 7, 4096, 20, 0, 69, 9, False), (1, 8, 3584, 70, 800, 69, 300, False), (1, 4, 4104, 73, 950, 69, 300, False),
+    (1, 1, 8192, 147, 1900, 69, 700, True), (2, 5, 8200, 512, 1900, 69, 2000, False), (1, 16, 16384, 300, 7000, 69, 2000, False),
+    (1, 8, 16384, 512, 15872, 69, 3000, False), (300, 2, 520, 5, 50, 20, 100, False),
+    # past the limits
+    (1, 2, 16392, 20, 300, 69, 100, False), (1, 2, 2048, 513, 300, 69, 3000, False), (1, 16, 16384, 300, 7200, 69, 2000, False)])
+def test_joined_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
+    """Steps whose attention's workgroups make the selection: the same lists, and outputs as above."""
+    test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
