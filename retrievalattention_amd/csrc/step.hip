@@ -107,9 +107,14 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
 // 4, 2048 22.3 -> 20.2; 1 of 4, 8192 27.5 -> 25.8; 8 of 8, 4096 28.0 -> 25.9; 32 of 16, 4096 41.2 -> 38.6; 4 of 12, 8192 35.0 ->
 // 33.2; 16 of 1, 1920 22.2 -> 20.0; 320 of 8, 1280 70.2 -> 65.2; 512 of 4, 1024 71.2 -> 68.0.
 // What bounds it is the selection's chain (see select_body.h), then what bounds the attention.
+// NT: threads that select; the attention is eight waves' always (with sixteen 16 groups of 4 heads, 1024 clusters take 20.6 us
+// instead of 18.8, 64 of 8, 16384 139.3), and the others leave before it (a barrier counts the waves there are).  512 up to 8192
+// clusters (1024 threads: 16 of 4, 1024 19.2, 32 of 8, 4096 33.9 instead of 32.9, 32 of 4, 8192 48.1 / 47.8), 1024 past them (64 of
+// 8, 16384 138.1 -> 137.5, 8 of 4 39.1 -> 38.5) and for more than 512 probes (in launches of their own -> joined: 32 of 4, 8192
+// clusters, 819 probes 85.9 -> 84.2; 12 of 7, 5760, 576 45.4 -> 43.7; 64 of 8, 8192, 819 157.4 -> 155.2).
 // ------------------------------------------------------------------------------------
-template <int E, int GSM, bool HALF, int SRC>
-__global__ __launch_bounds__(64 * ATT_WAVES, 2) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int4 m, SelectArgs S0,
+template <int NT, int E, int GSM, bool HALF, int SRC>
+__global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int4 m, SelectArgs S0,
                                                                           AttendParams A0) {
   extern __shared__ __attribute__((aligned(16))) int sh_kept[];
   SelectArgs S = S0;
@@ -133,20 +138,24 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void select_attend_kernel(ri_ptr
   int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
   const SelectKept kept = {nullptr, est, off, start, ids, meta};
   const AttendKept known = {nullptr, est, off, start, att_query_piece(A, g), att_steady_rows(A)};
-  select_group<64 * ATT_WAVES, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept);
+  select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept);
   lds_barrier();
+  if (NT > 64 * ATT_WAVES && threadIdx.x >= 64 * ATT_WAVES) return;
   attend_group<GSM, HALF, KEPT_TABLES>(A, g, blockIdx.y, known);
   if (blockIdx.y == 0) store_selection(S, g, kept);
 }
 
-template <int E, int SRC>
+template <int NT, int E, int SRC>
 static void launch_select_attend(const SelectArgs& S, const AttendParams& A, int BG, bool half, hipStream_t stream) {
   const void* a = SRC == SEL_KEYS ? (const void*)S.keys : (const void*)S.logits;
-  auto* kernel = S.gs <= 4   ? (half ? select_attend_kernel<E, 4, true, SRC> : select_attend_kernel<E, 4, false, SRC>)
-                 : S.gs <= 8 ? (half ? select_attend_kernel<E, 8, true, SRC> : select_attend_kernel<E, 8, false, SRC>)
-                             : (half ? select_attend_kernel<E, 16, true, SRC> : select_attend_kernel<E, 16, false, SRC>);
+  // (sixteen heads: up to 512 threads; more than 8192 clusters in so few: sixteen heads)
+  constexpr int LEAST = NT == 512 && E == 32 ? 16 : 4, MOST = NT == 512 ? 16 : 8;
+  constexpr int G4 = LEAST > 4 ? LEAST : 4, G8 = LEAST > 8 ? LEAST : 8, G16 = MOST;
+  auto* kernel = S.gs <= 4   ? (half ? select_attend_kernel<NT, E, G4, true, SRC> : select_attend_kernel<NT, E, G4, false, SRC>)
+                 : S.gs <= 8 ? (half ? select_attend_kernel<NT, E, G8, true, SRC> : select_attend_kernel<NT, E, G8, false, SRC>)
+                             : (half ? select_attend_kernel<NT, E, G16, true, SRC> : select_attend_kernel<NT, E, G16, false, SRC>);
   const size_t lds = (size_t)(4 + 3 * S.np + 1 + S.es) * sizeof(int);
-  kernel<<<dim3(BG, A.S), 64 * ATT_WAVES, lds, stream>>>(ri_pack_ptrs(a, S.tile_max, S.tile_sum, S.mask),
+  kernel<<<dim3(BG, A.S), NT, lds, stream>>>(ri_pack_ptrs(a, S.tile_max, S.tile_sum, S.mask),
                                                          (ri_int4){S.nc, S.gs, S.np, S.es}, (ri_int4){S.ntiles, A.S, A.W_kv, 0}, S,
                                                          A);
 }
@@ -167,6 +176,7 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
                              s->np, s->es, s->page, s->max_pages, s->scale, s->score_workspace, s->score_workspace_bytes);
   if (rc) return rc;
   if (s->attn_workspace && s->attn_workspace_bytes < ri_wave_attention_workspace_bytes(s->BG, s->gs)) return RI_ERR_WORKSPACE;
+  const bool wide = step_is_wide(s);
   AttendParams A;
   rc = ri_prepare_wave_attention(&A, q, s->steady_k, s->steady_v, s->steady_stride, static_len, s->static_len_dev, s->store_k,
                                  s->store_v, s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta,
@@ -187,13 +197,18 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
   const bool keys = S.nc > (S.gs <= 4 ? 4096 : S.gs <= 8 ? min(4096, 28 * 1024 / S.gs) : 2048);
   rc = ri_launch_select_inputs(S, s->BG, s->half, keys, stream);
   if (rc) return rc;
-  if (keys) {
-    if (S.nc <= 4096) launch_select_attend<8, SEL_KEYS>(S, A, s->BG, s->half, stream);
-    else if (S.nc <= 8192) launch_select_attend<16, SEL_KEYS>(S, A, s->BG, s->half, stream);
-    else launch_select_attend<32, SEL_KEYS>(S, A, s->BG, s->half, stream);
-  } else if (S.nc <= 1024) launch_select_attend<2, SEL_LOGITS>(S, A, s->BG, s->half, stream);
-  else if (S.nc <= 2048) launch_select_attend<4, SEL_LOGITS>(S, A, s->BG, s->half, stream);
-  else launch_select_attend<8, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  if (wide) {
+    if (keys) {
+      if (S.nc <= 8192) launch_select_attend<1024, 8, SEL_KEYS>(S, A, s->BG, s->half, stream);
+      else launch_select_attend<1024, 16, SEL_KEYS>(S, A, s->BG, s->half, stream);
+    } else launch_select_attend<1024, 4, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  } else if (keys) {
+    if (S.nc <= 4096) launch_select_attend<512, 8, SEL_KEYS>(S, A, s->BG, s->half, stream);
+    else if (S.nc <= 8192) launch_select_attend<512, 16, SEL_KEYS>(S, A, s->BG, s->half, stream);
+    else launch_select_attend<512, 32, SEL_KEYS>(S, A, s->BG, s->half, stream);
+  } else if (S.nc <= 1024) launch_select_attend<512, 2, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  else if (S.nc <= 2048) launch_select_attend<512, 4, SEL_LOGITS>(S, A, s->BG, s->half, stream);
+  else launch_select_attend<512, 8, SEL_LOGITS>(S, A, s->BG, s->half, stream);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

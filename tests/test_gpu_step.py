@@ -85,8 +85,12 @@ def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static
     (2, 7, 4096, 20, 0, 69, 9, False), (1, 8, 3584, 70, 800, 69, 300, False), (1, 4, 4104, 73, 950, 69, 300, False),
     (1, 1, 8192, 147, 1900, 69, 700, True), (2, 5, 8200, 512, 1900, 69, 2000, False), (1, 16, 16384, 300, 7000, 69, 2000, False),
     (1, 8, 16384, 512, 15872, 69, 3000, False), (300, 2, 520, 5, 50, 20, 100, False),
+    # 1024 threads that select
+    (1, 2, 1024, 513, 300, 69, 3000, False), (2, 8, 4096, 1024, 3000, 69, 5000, True), (1, 4, 4104, 700, 0, 69, 50, False),
+    (1, 7, 8192, 1024, 7168, 69, 5000, False), (2, 3, 8200, 9, 2000, 300, 5000, False), (1, 8, 16384, 1024, 15360, 69, 9000, False),
     # past the limits
-    (1, 2, 16392, 20, 300, 69, 100, False), (1, 2, 2048, 513, 300, 69, 3000, False), (1, 16, 16384, 300, 7200, 69, 2000, False)])
+    (1, 2, 16392, 20, 300, 69, 100, False), (1, 2, 2048, 1025, 300, 69, 6000, False), (1, 9, 2048, 513, 300, 69, 3000, False),
+    (1, 16, 16384, 300, 7200, 69, 2000, False)])
 def test_joined_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
     """Steps whose attention's workgroups make the selection: the same lists, and outputs as above."""
     test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
