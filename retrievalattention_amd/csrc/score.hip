@@ -11,7 +11,7 @@
 #define SCORE_TILE RI_SCORE_TILE  // centroids per workgroup == width of one softmax partial
 
 // ------------------------------------------------------------------------------------
-// score_kernel: grid (ntiles, BG), 256 threads = 4 waves, each wave owns 64 centroids.
+// score_kernel: grid (ntiles, BG), 256 threads = 4 waves, each wave owns 64 or 16 centroids.
 // MFMA 16x16x32: A = 16 centroid rows, B = query heads (columns >= gs are zero).
 // Accumulator register i of lane l holds row 4*(l/16)+i, column l%16.
 // ------------------------------------------------------------------------------------
@@ -20,25 +20,25 @@
 template <bool HALF>
 __device__ __forceinline__ uint16_t score_f32_to_16(float f) { return ri_f32_to_e16<HALF>(f); }
 
-// TPW = 16-row centroid tiles per wave: a workgroup covers SCORE_TILE = 256 centroids with 16 / TPW waves.
-// Launched with 4 (four waves, sixteen loads in flight per lane); eight waves with eight loads and sixteen with
-// four were slower (29.96 and 32.1 us against 29.6 us for scoring + selection at 32 groups of 8192 centroids).
-// Softmax partials of the 256 columns with one barrier: every wave reduces its own columns to a maximum and a
+// TPW = 16-row centroid tiles per wave, NWV waves: a workgroup covers 16 TPW NWV centroids.
+// Launched with 4 and 4 (SCORE_TILE, sixteen loads in flight per lane); eight waves with eight loads and sixteen with
+// four were slower (29.96 and 32.1 us against 29.6 us for scoring + selection at 32 groups of 8192 centroids); where those
+// workgroups are few with 1 and 4 (score_tile in select.hip).
+// Softmax partials of the columns with one barrier: every wave reduces its own columns to a maximum and a
 // sum of exponentials relative to that maximum, and after the barrier one thread per head folds the wave pairs
 // (max of the maxima, sums rescaled by exp(m_w - M)).
-template <bool HALF, int TPW, bool STREAM>
+template <bool HALF, int TPW, int NWV, bool STREAM>
 __device__ __forceinline__ void score_body(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cent, float* __restrict__ logits,
     uint16_t* __restrict__ logits_bf16, float* __restrict__ tile_max, float* __restrict__ tile_sum,
     int gs, int nc, int ntiles, float scale) {
-  constexpr int NWV = 16 / TPW;
   const int tile = blockIdx.x;
   const int g = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int r = lane & 15;
   const int h = lane >> 4;
-  const int c0 = tile * SCORE_TILE + wave * (16 * TPW);
+  const int c0 = (tile * NWV + wave) * (16 * TPW);
 
   const uint16_t* cg = cent + (size_t)g * nc * RI_DIM;
   // Rows past the last centroid and query heads past gs read a valid row instead (their columns are never used): a load
@@ -142,12 +142,12 @@ __device__ __forceinline__ void score_body(
   }
 }
 
-template <bool HALF, int TPW, bool STREAM>
-__global__ __launch_bounds__(1024 / TPW) void score_kernel(
+template <bool HALF, int TPW, int NWV, bool STREAM>
+__global__ __launch_bounds__(64 * NWV) void score_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cent, float* __restrict__ logits,
     uint16_t* __restrict__ logits16, float* __restrict__ tile_max, float* __restrict__ tile_sum,
     int gs, int nc, int ntiles, float scale) {
-  score_body<HALF, TPW, STREAM>(q, cent, logits, logits16, tile_max, tile_sum, gs, nc, ntiles, scale);
+  score_body<HALF, TPW, NWV, STREAM>(q, cent, logits, logits16, tile_max, tile_sum, gs, nc, ntiles, scale);
 }
 
 // Row statistics and softmax, a workgroup per row: every wave reduces the row's partials, with the workgroup's first 8
@@ -203,7 +203,7 @@ static int batch_gemm_softmax_impl(const void* A, const void* B, void* D, float*
   const int ntiles = (n + SCORE_TILE - 1) / SCORE_TILE;
   // fp32 logits are not part of this interface: the partial statistics come from the fp32
   // accumulators inside the kernel, the softmax from the 16-bit D, as in the reference.
-  score_kernel<HALF, 4, false><<<dim3(ntiles, batch_count), 256, 0, s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
+  score_kernel<HALF, 4, 4, false><<<dim3(ntiles, batch_count), 256, 0, s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
                                                                   (uint16_t*)D, Norm, Sum, m, n, ntiles, alpha);
   RI_HIP_CHECK_LAUNCH();
   const int threads = min(1024, (n / 8 + 63) / 64 * 64);
@@ -228,15 +228,16 @@ extern "C" int ri_batch_gemm_softmax_f16(const void* A, const void* B, void* D, 
 
 // scoring pass used by the fused selection (select.hip)
 int ri_launch_score(const void* q, const void* centroids, float* logits, float* tile_max, float* tile_sum,
-                    int BG, int gs, int nc, float scale, bool half, hipStream_t s) {
-  const int ntiles = (nc + SCORE_TILE - 1) / SCORE_TILE;
+                    int BG, int gs, int nc, int tile, float scale, bool half, hipStream_t s) {
+  const int ntiles = (nc + tile - 1) / tile;
   const uint16_t *qq = (const uint16_t*)q, *cc = (const uint16_t*)centroids;
   // Up to 32 MB of centroids the logits are better left where the next kernels find them (whole steps: 8 groups of 8 heads,
   // 4096 centroids 25.9 -> 25.0 us, 16 of 16, 2048 32.0 -> 30.9, 12 of 7, 1856 24.8 -> 24.4; 16 of 4, 8192 34.7 either way);
   // with more the write-back is longer than that (32 of 4, 8192 46.1 streamed, 46.4 not).
   const bool stream = (size_t)BG * nc > 128 * 1024;
-  auto* kernel = half ? (stream ? score_kernel<true, 4, true> : score_kernel<true, 4, false>)
-                      : (stream ? score_kernel<false, 4, true> : score_kernel<false, 4, false>);
+  auto* kernel = half ? (stream ? score_kernel<true, 4, 4, true> : score_kernel<true, 4, 4, false>)
+                      : (stream ? score_kernel<false, 4, 4, true> : score_kernel<false, 4, 4, false>);
+  if (tile == RI_SCORE_TILE_FEW) kernel = half ? score_kernel<true, 1, 4, false> : score_kernel<false, 1, 4, false>;
   kernel<<<dim3(ntiles, BG), 256, 0, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc, ntiles, scale);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;

@@ -459,10 +459,24 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(ri_ptr4 in, ri_int4 n,
 // ------------------------------------------------------------------------------------
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Centroids per scoring workgroup.  One compute unit reads 20 .. 25 KB per microsecond from memory, so the 64 KB of a wide
+// tile take it three, and while wide tiles do not give every unit one, narrow ones are read by four times as many (whole
+// captured steps, wide / narrow: 8 groups of 4 heads, 1024 clusters 18.0 / 16.7 us, 16: 18.6 / 17.7; 16 of 8, 2048 23.7 / 22.5; 12
+// of 7, 1920 25.7 / 24.9; 8 of 8, 4096 26.2 / 25.4; 16 of 4, 4096 25.8 / 25.3; 32 of 4, 2048 23.0 / 22.5; 64 of 4, 1024 22.0 either
+// way).  Past 64 partials a head's statistics are more than one load per lane, for every workgroup that wants them (1 group of
+// 8 heads, 16384 clusters 33.3 / 34.9; 2 of 16, 8192 33.8 / 34.5).
+static int score_tile(int BG, int nc) {
+  const bool few = nc <= 64 * RI_SCORE_TILE_FEW && (int64_t)BG * ((nc + RI_SCORE_TILE - 1) / RI_SCORE_TILE) <= 256;
+  return few ? RI_SCORE_TILE_FEW : RI_SCORE_TILE;
+}
+static size_t select_space(int BG, int gs, int nc, int tile) {
+  const size_t ntiles = (size_t)(nc + tile - 1) / tile;
+  return 2 * align256((size_t)BG * ntiles * gs * sizeof(float)) + align256((size_t)BG * nc * sizeof(uint16_t));
+}
+
 extern "C" size_t ri_score_select_workspace_bytes(int BG, int gs, int nc) {
   if (BG <= 0 || gs <= 0 || nc <= 0) return 0;
-  const size_t ntiles = (size_t)(nc + RI_SCORE_TILE - 1) / RI_SCORE_TILE;
-  return 2 * align256((size_t)BG * ntiles * gs * sizeof(float)) + align256((size_t)BG * nc * sizeof(uint16_t));
+  return select_space(BG, gs, nc, score_tile(BG, nc));
 }
 
 template <int NT, int E, int GSM, int SRC>
@@ -490,8 +504,10 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
   if (np <= 0 || np > SEL_MAX_PROBES || es < 0 || np + es > nc || nc > 65536) return RI_ERR_ARG;
   if (es > 0 && !est_ids) return RI_ERR_ARG;
   if (cluster_size_i32 && (!ret_tok_off || !meta || page <= 0 || max_pages <= 0)) return RI_ERR_ARG;
-  if (workspace_bytes < ri_score_select_workspace_bytes(BG, gs, nc)) return RI_ERR_WORKSPACE;
-  const int ntiles = (nc + RI_SCORE_TILE - 1) / RI_SCORE_TILE;
+  int tile = score_tile(BG, nc);
+  if (workspace_bytes < select_space(BG, gs, nc, tile)) tile = RI_SCORE_TILE;   // (room for the partials of wide tiles only)
+  if (workspace_bytes < select_space(BG, gs, nc, tile)) return RI_ERR_WORKSPACE;
+  const int ntiles = (nc + tile - 1) / tile;
   char* w = (char*)workspace;
   float* tmax = (float*)w;
   w += align256((size_t)BG * ntiles * gs * sizeof(float));
@@ -499,7 +515,7 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
   w += align256((size_t)BG * ntiles * gs * sizeof(float));
   *P = {(uint16_t*)w, (const uint16_t*)q, (const uint16_t*)centroids, logits, tmax, tsum, mask, cluster_size_i32,
         cluster_start, (uint16_t*)dist, cI, ret_ids, est_ids, ret_tok_off, ret_start, row_src, meta, row_src_stride, gs, nc,
-        ntiles, np, es, page, max_pages, scale};
+        ntiles, np, es, page, max_pages, tile, scale};
   return RI_OK;
 }
 
@@ -514,7 +530,7 @@ static int launch_dist(const SelectArgs& P, int BG, bool half, hipStream_t s) {
 }
 
 int ri_launch_select_inputs(const SelectArgs& P, int BG, bool half, bool keys, hipStream_t s) {
-  const int rc = ri_launch_score(P.q, P.cent, P.logits, P.tile_max, P.tile_sum, BG, P.gs, P.nc, P.scale, half, s);
+  const int rc = ri_launch_score(P.q, P.cent, P.logits, P.tile_max, P.tile_sum, BG, P.gs, P.nc, P.tile, P.scale, half, s);
   return rc || !keys ? rc : launch_dist(P, BG, half, s);
 }
 
@@ -549,7 +565,7 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }
-  rc = ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, scale, half, s);
+  rc = ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, P.tile, scale, half, s);
   if (rc) return rc;
   if (nc <= (gs <= 4 ? min(8192, 28 * 1024 / gs) : gs <= 8 ? 4096 : 2048) && np <= SEL_THREADS) {
     // as few waves as the clusters and the probes leave room for: what a wave does once costs all of them
@@ -618,11 +634,13 @@ static int score_logits_impl(const void* q, const void* centroids, float* logits
   if (!q || !centroids || !logits || !workspace) return RI_ERR_ARG;
   if (ri_any_misaligned16(q, centroids, logits, workspace)) return RI_ERR_ARG;
   if (BG <= 0 || gs <= 0 || gs > 16 || nc <= 0 || (nc % 4) != 0) return RI_ERR_ARG;
-  if (workspace_bytes < ri_score_select_workspace_bytes(BG, gs, nc)) return RI_ERR_WORKSPACE;
-  const int ntiles = (nc + RI_SCORE_TILE - 1) / RI_SCORE_TILE;
+  int tile = score_tile(BG, nc);
+  if (workspace_bytes < select_space(BG, gs, nc, tile)) tile = RI_SCORE_TILE;
+  if (workspace_bytes < select_space(BG, gs, nc, tile)) return RI_ERR_WORKSPACE;
+  const int ntiles = (nc + tile - 1) / tile;
   float* tmax = (float*)workspace;
   float* tsum = (float*)((char*)workspace + align256((size_t)BG * ntiles * gs * sizeof(float)));
-  return ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, scale, half, (hipStream_t)stream);
+  return ri_launch_score(q, centroids, logits, tmax, tsum, BG, gs, nc, tile, scale, half, (hipStream_t)stream);
 }
 
 extern "C" int ri_score_logits(const void* q, const void* centroids, float* logits, int BG, int gs, int nc,

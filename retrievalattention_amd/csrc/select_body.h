@@ -43,7 +43,7 @@ struct SelectArgs {
   int32_t* ret_start;
   int32_t* row_src;
   int32_t* meta;
-  int row_src_stride, gs, nc, ntiles, np, es, page, max_pages;
+  int row_src_stride, gs, nc, ntiles, np, es, page, max_pages, tile;
   float scale;
 };
 

@@ -364,3 +364,34 @@ def test_score_select_every_head_counts(dev, gs, nc):
     6): the selection must not make score sums here with the variant that holds four heads."""
     test_score_select(dev, 2, gs, nc, nc // 56, nc // 4, 3100 + nc + gs)
     test_score_select(dev, 2, gs, nc, nc // 56, nc // 4, 3200 + nc + gs, dt=torch.float16)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("BG,gs,nc", [(1, 4, 520), (3, 7, 1032), (1, 16, 4096), (16, 2, 4096), (17, 2, 4096), (64, 3, 1024),
+                                      (65, 3, 1024), (1, 2, 4104)])
+def test_score_select_narrow_tiles(dev, BG, gs, nc, dt):
+    """Few scoring workgroups: narrow tiles with remainders, as many partials as lanes, and the shapes just past either."""
+    test_score_select(dev, BG, gs, nc, nc // 50, nc // 4, BG + nc, dt=dt)
+
+
+def test_score_select_without_room_for_narrow_tiles(dev):
+    """A workspace for the partials of wide tiles is enough; the logits do not depend on it."""
+    from retrievalattention_amd import _lib
+    lib = _lib.lib()
+    BG, gs, nc, np_ = 2, 4, 1024, 18
+    q, cent = _mixture(BG, gs, nc, 5)
+    q, cent = q.to(dev), cent.to(dev)
+    room = lib.ri_score_select_workspace_bytes(BG, gs, nc)
+    wide = 2 * ((BG * 4 * gs * 4 + 255) // 256 * 256) + BG * nc * 2
+    assert wide < room
+    got = []
+    for nbytes in (room, wide, wide - 1):
+        logits = torch.zeros(BG, gs, nc, device=dev)
+        ids = torch.zeros(BG, np_, dtype=torch.int32, device=dev)
+        ws = torch.empty(room, dtype=torch.uint8, device=dev)
+        none = [None] * 3
+        rc = lib.ri_score_select(q.data_ptr(), cent.data_ptr(), *none, logits.data_ptr(), None, None, ids.data_ptr(), None, None,
+                                 None, None, 0, None, BG, gs, nc, np_, 0, 0, 0, 128 ** -0.5, ws.data_ptr(), nbytes, 0)
+        got.append((rc, logits, ids.sort(dim=1)[0]))
+    assert [r[0] for r in got[:2]] == [0, 0] and got[2][0] != 0
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
