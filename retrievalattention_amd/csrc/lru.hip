@@ -25,7 +25,7 @@
 // misses, row table) is its first half; the second (eviction, admission) only has to be done before the admission copy.
 // So the two are also launched apart, the second beside the copy of the missed rows from the host, which is bound by the
 // link and leaves the compute units idle (32 groups, 3840 clusters, 10 MB of misses: access and update in one launch in
-// front of the copy 27.8 + 200 us, access alone 7 and both others together 187).
+// front of the copy 27.8 + 200 us, access alone 7 and both others together 187, all with a copy that took as long by itself).
 #include "ri_common.h"
 
 #define LRU_THREADS 1024
@@ -33,6 +33,7 @@
 #define LRU_DIGIT 256
 #define LRU_COPIES 8        // of the age histogram: a step's clusters share their age
 #define LRU_HELD 4          // clusters per thread whose stamps and blocks stay in registers
+#define LRU_COPIERS 64      // waves that copy missed rows, for blocks of eight rows or more
 
 enum { LRU_BOTH, LRU_ACCESS, LRU_UPDATE };
 
@@ -424,28 +425,47 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(ri_lru_t P) {
   lru_group<R, PHASE>(P, blockIdx.x);
 }
 
-// grid (1 + X, groups): workgroup 0 of a group updates the cache's books, the others copy the group's missed rows from the
-// host store into the staging rows, eight items of at most `block` rows at a time (16 lanes per row).
+// grid groups + copiers: the first workgroups, one per group, update the cache's books; the others copy the missed rows of all
+// groups from the host store into the staging rows, the first wave of each (the rest of its threads leave).  The items, of at
+// most `block` rows, are numbered through all groups and a wave takes every copiers-th: eight rows at a time, 16 lanes per row,
+// with both halves requested before either is stored.  What is in flight is what counts: the link wants about 256 KB of it and
+// carries less the more there is (32 groups, 2830 blocks of up to 8 rows, 10.2 MB, GB/s by waves: 48 55.5, 64 55.7, 128 52.1,
+// 256 55.1, 512 54.3, 2048 49.6; a workgroup of sixteen waves to every eight items of a group, as many as there may be, 53.1;
+// plain reads of as much in a row 55.9).
 template <int R>
-__global__ __launch_bounds__(LRU_THREADS) void lru_stage_kernel(ri_lru_t P) {
-  const int g = blockIdx.y;
-  if (blockIdx.x == 0) {
-    lru_group<R, LRU_UPDATE>(P, g);
+__global__ __launch_bounds__(LRU_THREADS) void lru_stage_kernel(ri_lru_t P, int copiers) {
+  if ((int)blockIdx.x < P.BG) {
+    lru_group<R, LRU_UPDATE>(P, blockIdx.x);
     return;
   }
-  const int n = P.miss_num[g];
-  const size_t lists = (size_t)g * P.buffer_size;
-  const int sub = threadIdx.x >> 7, vec = (threadIdx.x & 127) >> 4, piece = threadIdx.x & 15;
-  for (int j = (blockIdx.x - 1) * 8 + sub; j < n; j += (gridDim.x - 1) * 8) {
-    const int rows = P.miss_sizes[lists + j];
-    const size_t src = (size_t)g * P.host_stride + P.miss_ids[lists + j];
-    const size_t dst = (size_t)g * P.cache_stride + P.stage_row0 + P.miss_cumsum[lists + j];
-    for (int r = vec; r < rows; r += 8) {
-      const uint4 k = reinterpret_cast<const uint4*>(P.host_k)[(src + r) * 16 + piece];
-      const uint4 v = reinterpret_cast<const uint4*>(P.host_v)[(src + r) * 16 + piece];
-      reinterpret_cast<uint4*>(P.cache_k)[(dst + r) * 16 + piece] = k;
-      reinterpret_cast<uint4*>(P.cache_v)[(dst + r) * 16 + piece] = v;
+  const int lane = threadIdx.x, vec = lane >> 4, piece = lane & 15;
+  if (lane >= 64) return;
+  int item = blockIdx.x - P.BG, first = 0;   // the item's number; that of the window's first
+  for (int g0 = 0; g0 < P.BG; g0 += 64) {
+    const int own = g0 + lane < P.BG ? P.miss_num[g0 + lane] : 0;
+    const int upto = (int)ri_wave_incl_scan((uint32_t)own), last = first + __builtin_amdgcn_readlane(upto, 63);
+    for (; item < last; item += copiers) {
+      const int in = __popcll(__ballot(upto <= item - first));   // the item's group in the window
+      const int g = g0 + in, j = item - first - __builtin_amdgcn_readlane(upto - own, in);
+      const size_t at = (size_t)g * P.buffer_size + j;
+      const int rows = P.miss_sizes[at];
+      const size_t src = (size_t)g * P.host_stride + P.miss_ids[at];
+      const size_t dst = (size_t)g * P.cache_stride + P.stage_row0 + P.miss_cumsum[at];
+      for (int r = vec; r < rows; r += 8) {
+        const int r2 = min(r + 4, rows - 1);
+        const uint4 k = reinterpret_cast<const uint4*>(P.host_k)[(src + r) * 16 + piece];
+        const uint4 v = reinterpret_cast<const uint4*>(P.host_v)[(src + r) * 16 + piece];
+        const uint4 k2 = reinterpret_cast<const uint4*>(P.host_k)[(src + r2) * 16 + piece];
+        const uint4 v2 = reinterpret_cast<const uint4*>(P.host_v)[(src + r2) * 16 + piece];
+        reinterpret_cast<uint4*>(P.cache_k)[(dst + r) * 16 + piece] = k;
+        reinterpret_cast<uint4*>(P.cache_v)[(dst + r) * 16 + piece] = v;
+        if (r + 4 < rows) {
+          reinterpret_cast<uint4*>(P.cache_k)[(dst + r2) * 16 + piece] = k2;
+          reinterpret_cast<uint4*>(P.cache_v)[(dst + r2) * 16 + piece] = v2;
+        }
+      }
     }
+    first = last;
   }
 }
 
@@ -510,11 +530,10 @@ extern "C" int ri_lru_stage_update(const ri_lru_t* s, ri_stream_t stream) {
       s->cache_stride < (int64_t)s->stage_row0 + (int64_t)s->buffer_size * s->block)
     return RI_ERR_ARG;
   if (ri_any_misaligned16(s->host_k, s->host_v, s->cache_k, s->cache_v)) return RI_ERR_ARG;
-  // A workgroup takes eight blocks at a time.  Many per group, most of them without work: the groups then start one after
-  // the other, and the link carries 54.9 GB/s; with at most sixteen, all groups' reads are mixed and it carries 50.0.
-  const dim3 grid(1 + min(64, (s->buffer_size + 7) / 8), s->BG);
-  if (s->np < LRU_THREADS) lru_stage_kernel<1><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
-  else lru_stage_kernel<4><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
+  const int copiers = LRU_COPIERS * 8 / min(s->block, 8);   // (a wave's share of what is in flight shrinks with its rows)
+  const dim3 grid(s->BG + copiers);
+  if (s->np < LRU_THREADS) lru_stage_kernel<1><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s, copiers);
+  else lru_stage_kernel<4><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s, copiers);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

@@ -209,3 +209,36 @@ def test_access_and_stage_update_equal_the_one_launch(dev, ncl, nprobe, capacity
                 row, k, at = (int(lists[4 + x][b, j]) for x in range(3))
                 for h, c in zip(host, cache):
                     assert torch.equal(c[b, stage0 + at:stage0 + at + k].cpu(), h[b, row:row + k])
+
+
+@pytest.mark.parametrize("BG,block", [(1, 8), (3, 1), (63, 3), (65, 8), (130, 16)])
+def test_missed_rows_are_staged_in_rank_order(dev, BG, block):
+    """Items numbered through all groups, sixty-four groups at a time: groups without misses, partial blocks, blocks shorter and
+    longer than the eight rows a wave copies at a time; nothing is written behind the rows."""
+    import ctypes
+    from retrievalattention_amd import kernels
+    from retrievalattention_amd._lib import lib
+    g = torch.Generator().manual_seed(BG)
+    ncl, nprobe = 24, 7
+    sz = torch.randint(0, 40, (BG, ncl), generator=g, dtype=torch.int32)
+    sz[1::5] = 0
+    st = (torch.cumsum(sz.long(), 1) - sz.long()).to(torch.int32)
+    n = max(1, int(sz.sum(1).max()))
+    buffer_size = nprobe * ((39 + block - 1) // block)
+    host = [torch.randn(BG, n, 128, generator=g).to(torch.bfloat16).pin_memory() for _ in range(2)]
+    cache = [torch.zeros(BG, buffer_size * block + 1, 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    lru = kernels.DeviceLru(BG, ncl, int(((sz + block - 1) // block).sum(1).max()) + 1, 0, buffer_size, block, dev)
+    lru.set_sizes(sz.to(dev))
+    lists = [torch.zeros((BG,) if i % 4 == 3 else (BG, buffer_size), dtype=torch.int32, device=dev) for i in range(12)]
+    row_src = torch.zeros(BG, buffer_size * block, dtype=torch.int32, device=dev)
+    ids = torch.stack([torch.randperm(ncl, generator=g)[:nprobe] for _ in range(BG)]).to(torch.int32)
+    s = lru.prepared(ids.to(dev), sz.to(dev), st.to(dev), lists, row_src, 0, torch.zeros(BG, 4, dtype=torch.int32, device=dev),
+                     *host, *cache)
+    for fn in (lib().ri_lru_access, lib().ri_lru_stage_update):
+        assert fn(ctypes.addressof(s), kernels._stream()) == 0
+    for h, c in zip(host, cache):
+        want = torch.zeros(c.shape, dtype=c.dtype)
+        for b in range(BG):
+            rows = torch.cat([torch.arange(st[b, i], st[b, i] + sz[b, i]) for i in ids[b].tolist()])
+            want[b, :len(rows)] = h[b, rows]
+        assert torch.equal(c.cpu(), want)
