@@ -4,7 +4,6 @@
 // index add :176-221) with a fixed summation order instead of fp32 atomics.
 #include "ri_common.h"
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void* km_lds_ptr;
 typedef const __attribute__((address_space(1))) void* km_glb_ptr;
 
@@ -32,125 +31,137 @@ static int km_together(int P) { return P % 8 == 0 ? 3 : P % 4 == 0 ? 2 : P % 2 =
 static dim3 km_grid(int T, int P) { return dim3((unsigned)T << km_together(P), P >> km_together(P)); }
 
 // ------------------------------------------------------------------------------------
-// assign: grid km_grid(ceil(N / (KM_W * 32 * KM_TT)), P), KM_W waves; a wave keeps KM_TT columns of 32
-// tokens in registers for the whole kernel (KM_TT independent accumulator chains).  Centroid
-// tiles of KM_CT rows go through KM_NB LDS buffers shared by all waves of the workgroup: a tile
+// assign: grid km_grid(ceil(N / (W * 32 * TT)), P), W waves; a wave keeps TT columns of 32
+// tokens in registers for the whole kernel.  Centroid
+// tiles of CT rows go through NB LDS buffers shared by all waves of the workgroup: a tile
 // is requested from global memory straight into its buffer (no registers, no LDS
-// stores) KM_NB - 1 tiles ahead, one wait and one barrier per tile.
-// MFMA 32x32x16: A = centroid rows, B = token columns; accumulator i of lane l is
-// row (i/4)*8 + (l/32)*4 + i%4, column l%32.  nc is a multiple of 32; the last tile may hold
-// fewer sub-tiles.  (Which tiling serves which shape: km_assign below.)
+// stores) NB - 1 tiles ahead, one wait and one barrier per tile.
+// MFMA 16x16x32: A = centroid rows, B = token columns; accumulator i of lane l is
+// row (l/16)*4 + i, column l%16.  nc is a multiple of 32; the last tile may hold
+// fewer sub-tiles.  (Which tiling serves which shape: km_assign_launch below.)
+// Long passes are bound by what the card's power lets the matrix cores do, and a product of sixteen rows reads and writes
+// half the sums per multiplication that one of 32 does: loops over registers alone hold 2.05 - 2.12 PFLOP/s against 1.75 -
+// 1.86 with 32x32x16, and 8 x 131072 tokens, 8192 centroids take 1378 us against 1504 (1.60 and 1.46 PFLOP/s; the matrix
+// cores were busy 73 % of the time, at a clock that fell with it).
 // HALF: keys and centroids are IEEE half instead of bfloat16.
 // ------------------------------------------------------------------------------------
 template <int V>
 __device__ __forceinline__ void km_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(V) : "memory"); }
 
-// base + the row, past the lane's first one in a sub-tile, of the first of a lane's sixteen scores that equals m: the half
-// that holds m is selected, then its half, down to one score.  low8 and low4 are the maxima of best and the first eight
-// and four scores, high4 of best and scores 8 .. 11; m is above best in every lane whose answer counts.  26 instructions,
-// of which four compare; comparing and selecting one score after the other takes 30, and leaves two slots idle between
-// each comparison and the select that reads its mask.  Written out because the compiler turns a select between two scores
-// into a search by index.  (The hardware wants two slots between a comparison and a select that reads it.  The scores have
-// been read by the maxima before: no matrix result is outstanding when this runs.)
-__device__ __forceinline__ int km_first_of(const f32x16_t& x, float m, float best, float low8, float low4, float high4,
-                                           int base) {
-  float y0, y1, y2, y3, y4, y5, y6, y7, t;
-  uint64_t e, e8;
+// (the compiler would quiet a NaN in front of its own maximum; these have none)
+__device__ __forceinline__ float km_max(float a, float b) {
+  float m;
+  asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+__device__ __forceinline__ float km_max3(float a, float b, float c) {
+  float m;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+  return m;
+}
+
+typedef uint32_t km_pair __attribute__((ext_vector_type(2)));
+// o[u] (+)= a b[u]: sixteen rows with twice sixteen tokens, 32 dims.  Written out so that the sums stay where they are: left to
+// the compiler every product gets another register for its sum, 64 more than there are.  Hazards are its own: two slots from a
+// register move to a product that reads it (in the shadow of the product before), and, behind the last one, km_products_wait.
+template <bool HALF, bool TIED, bool FIRST>
+__device__ __forceinline__ void km_products(f32x4_t& o0, f32x4_t& o1, const uint4& a, const uint4& b0, const uint4& b1) {
+  if (!TIED) {
+    const f32x4_t c0 = FIRST ? f32x4_t{0.f, 0.f, 0.f, 0.f} : o0, c1 = FIRST ? f32x4_t{0.f, 0.f, 0.f, 0.f} : o1;
+    if (HALF) {
+      o0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b0), c0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b1), c1, 0, 0, 0);
+    } else {
+      o0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b0), c0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b1), c1, 0, 0, 0);
+    }
+    return;
+  }
+  typedef uint32_t op_t __attribute__((ext_vector_type(4)));
+  const op_t x = __builtin_bit_cast(op_t, a), y0 = __builtin_bit_cast(op_t, b0), y1 = __builtin_bit_cast(op_t, b1);
+#define KM_TWO(TYPE, C0, C1)                                                                                            \
+  "s_nop 1\n\tv_mfma_f32_16x16x32_" TYPE " %0, %2, %3, " C0 "\n\tv_mfma_f32_16x16x32_" TYPE " %1, %2, %4, " C1
+  if (FIRST) {
+    if (HALF) asm volatile(KM_TWO("f16", "0", "0") : "=&v"(o0), "=&v"(o1) : "v"(x), "v"(y0), "v"(y1));
+    else asm volatile(KM_TWO("bf16", "0", "0") : "=&v"(o0), "=&v"(o1) : "v"(x), "v"(y0), "v"(y1));
+  } else {
+    if (HALF) asm volatile(KM_TWO("f16", "%0", "%1") : "+v"(o0), "+v"(o1) : "v"(x), "v"(y0), "v"(y1));
+    else asm volatile(KM_TWO("bf16", "%0", "%1") : "+v"(o0), "+v"(o1) : "v"(x), "v"(y0), "v"(y1));
+  }
+#undef KM_TWO
+}
+// eight slots from a product to whoever reads its sum: nobody does in front of this
+template <int TT>
+__device__ __forceinline__ void km_products_wait(f32x4_t (&o)[TT][2][2]) {
+  asm volatile("s_nop 7\n\ts_nop 1");
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) asm volatile("" : "+v"(o[tt][0][0]), "+v"(o[tt][0][1]), "+v"(o[tt][1][0]), "+v"(o[tt][1][1]));
+}
+
+// base + the row, past the lane's first one in a sub-tile, of the first of a lane's eight scores (x: rows 0 .. 3, y: 16 .. 19)
+// that equals m: the half that holds m is selected, then its half, down to one score.  low4 is the maximum of best and x; m is
+// above best in every lane whose answer counts.  Written out because the compiler turns a select between two scores into a
+// search by index.  (The hardware wants two slots between a comparison and a select that reads it.  The scores have been read
+// by the maxima before: no matrix result is outstanding when this runs.)
+__device__ __forceinline__ int km_first_of(const f32x4_t& x, const f32x4_t& y, float m, float low4, int base) {
+  float z0, z1, z2, z3, t;
+  uint64_t e, e4;
   int row;
   asm volatile(
-      "v_cmp_eq_f32_e64 %8, %25, %26\n\t"
+      "v_cmp_eq_f32_e64 %6, %16, %17\n\t"
       "s_nop 1\n\t"
-      "v_cndmask_b32_e64 %0, %17, %9, %8\n\t"
-      "v_cndmask_b32_e64 %1, %18, %10, %8\n\t"
-      "v_cndmask_b32_e64 %2, %19, %11, %8\n\t"
-      "v_cndmask_b32_e64 %3, %20, %12, %8\n\t"
-      "v_cndmask_b32_e64 %4, %21, %13, %8\n\t"
-      "v_cndmask_b32_e64 %5, %22, %14, %8\n\t"
-      "v_cndmask_b32_e64 %6, %23, %15, %8\n\t"
-      "v_cndmask_b32_e64 %7, %24, %16, %8"
-      : "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7), "=&s"(e8)
-      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]),
-        "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(low8), "v"(m));
-  // (accumulator i is row (i / 4) * 8 + i % 4)
-  asm volatile(
-      "v_cndmask_b32_e64 %8, %13, %12, %10\n\t"
-      "v_cmp_eq_f32_e64 %11, %8, %15\n\t"
-      "v_cndmask_b32_e64 %9, 16, 0, %10\n\t"
+      "v_cndmask_b32_e64 %0, %12, %8, %6\n\t"
+      "v_cndmask_b32_e64 %1, %13, %9, %6\n\t"
+      "v_cndmask_b32_e64 %2, %14, %10, %6\n\t"
+      "v_cndmask_b32_e64 %3, %15, %11, %6\n\t"
+      "v_max_f32_e32 %4, %0, %1\n\t"
+      "v_cmp_eq_f32_e64 %7, %4, %17\n\t"
+      "v_cndmask_b32_e64 %5, 16, 0, %6\n\t"
+      "v_add_u32_e32 %5, %18, %5\n\t"
+      "v_cndmask_b32_e64 %0, %2, %0, %7\n\t"
+      "v_cmp_eq_f32_e64 %6, %0, %17\n\t"
+      "v_cndmask_b32_e64 %1, 2, 0, %7\n\t"
       "s_nop 0\n\t"
-      "v_cndmask_b32_e64 %0, %4, %0, %11\n\t"
-      "v_cndmask_b32_e64 %1, %5, %1, %11\n\t"
-      "v_cndmask_b32_e64 %2, %6, %2, %11\n\t"
-      "v_cndmask_b32_e64 %3, %7, %3, %11\n\t"
-      "v_max3_f32 %8, %14, %0, %1\n\t"
-      "v_cmp_eq_f32_e64 %10, %8, %15\n\t"
-      "v_cndmask_b32_e64 %4, 8, 0, %11\n\t"
-      "s_nop 0\n\t"
-      "v_cndmask_b32_e64 %0, %2, %0, %10\n\t"
-      "v_cmp_eq_f32_e64 %11, %0, %15\n\t"
-      "v_cndmask_b32_e64 %5, 2, 0, %10\n\t"
-      "v_add3_u32 %9, %9, %4, %5\n\t"
-      "v_cndmask_b32_e64 %6, 1, 0, %11\n\t"
-      "v_add3_u32 %9, %9, %6, %16"
-      : "+v"(y0), "+v"(y1), "+v"(y2), "+v"(y3), "+v"(y4), "+v"(y5), "+v"(y6), "+v"(y7), "=&v"(t), "=&v"(row), "+s"(e8),
-        "=&s"(e)
-      : "v"(low4), "v"(high4), "v"(best), "v"(m), "v"(base));
+      "v_cndmask_b32_e64 %2, 1, 0, %6\n\t"
+      "v_add3_u32 %5, %5, %1, %2"
+      : "=&v"(z0), "=&v"(z1), "=&v"(z2), "=&v"(z3), "=&v"(t), "=&v"(row), "=&s"(e4), "=&s"(e)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(low4), "v"(m),
+        "v"(base));
   return row;
 }
 
-// The same with the largest of the other fifteen scores and of what low8, low4, high8 and high4 started from, in `second`:
-// what each halving leaves behind.  Ten instructions more.
-__device__ __forceinline__ int km_first_two(const f32x16_t& x, float m, float low8, float high8, float low4, float high4,
-                                            int base, float& second) {
-  float y0, y1, y2, y3, y4, y5, y6, y7, t, u;
-  uint64_t e, e8;
+// The same with the largest of the other seven scores and of what low4 and high4 started from, in `second`: what each halving
+// leaves behind.
+__device__ __forceinline__ int km_first_two(const f32x4_t& x, const f32x4_t& y, float m, float low4, float high4, int base,
+                                            float& second) {
+  float z0, z1, z2, z3, t, u;
+  uint64_t e, e4;
   int row;
   asm volatile(
-      "v_cmp_eq_f32_e64 %9, %26, %28\n\t"
+      "v_cmp_eq_f32_e64 %8, %18, %20\n\t"
       "s_nop 1\n\t"
-      "v_cndmask_b32_e64 %0, %18, %10, %9\n\t"
-      "v_cndmask_b32_e64 %1, %19, %11, %9\n\t"
-      "v_cndmask_b32_e64 %2, %20, %12, %9\n\t"
-      "v_cndmask_b32_e64 %3, %21, %13, %9\n\t"
-      "v_cndmask_b32_e64 %4, %22, %14, %9\n\t"
-      "v_cndmask_b32_e64 %5, %23, %15, %9\n\t"
-      "v_cndmask_b32_e64 %6, %24, %16, %9\n\t"
-      "v_cndmask_b32_e64 %7, %25, %17, %9\n\t"
-      "v_cndmask_b32_e64 %8, %26, %27, %9"
-      : "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7), "=&v"(second), "=&s"(e8)
-      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]),
-        "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(low8), "v"(high8), "v"(m));
-  asm volatile(
-      "v_cndmask_b32_e64 %5, %14, %13, %8\n\t"
-      "v_cmp_eq_f32_e64 %9, %5, %15\n\t"
-      "v_cndmask_b32_e64 %7, 16, 0, %8\n\t"
-      "v_max3_f32 %6, %4, %10, %11\n\t"
-      "v_max_f32_e32 %6, %6, %12\n\t"
-      "v_cndmask_b32_e64 %0, %4, %0, %9\n\t"
-      "v_cndmask_b32_e64 %1, %10, %1, %9\n\t"
-      "v_cndmask_b32_e64 %2, %11, %2, %9\n\t"
-      "v_cndmask_b32_e64 %3, %12, %3, %9\n\t"
-      "v_cndmask_b32_e64 %5, %5, %6, %9\n\t"
-      "v_cndmask_b32_e64 %4, 8, 0, %9"
-      : "+&v"(y0), "+&v"(y1), "+&v"(y2), "+&v"(y3), "+&v"(y4), "=&v"(t), "=&v"(u), "=&v"(row), "+s"(e8), "=&s"(e)
-      : "v"(y5), "v"(y6), "v"(y7), "v"(low4), "v"(high4), "v"(m));
-  asm volatile(
+      "v_cndmask_b32_e64 %0, %14, %10, %8\n\t"
+      "v_cndmask_b32_e64 %1, %15, %11, %8\n\t"
+      "v_cndmask_b32_e64 %2, %16, %12, %8\n\t"
+      "v_cndmask_b32_e64 %3, %17, %13, %8\n\t"
+      "v_cndmask_b32_e64 %6, %18, %19, %8\n\t"
       "v_max_f32_e32 %4, %0, %1\n\t"
-      "v_cmp_eq_f32_e64 %8, %4, %11\n\t"
-      "v_add_u32_e32 %7, %7, %10\n\t"
+      "v_cmp_eq_f32_e64 %9, %4, %20\n\t"
+      "v_cndmask_b32_e64 %7, 16, 0, %8\n\t"
       "v_max_f32_e32 %5, %2, %3\n\t"
-      "v_cndmask_b32_e64 %0, %2, %0, %8\n\t"
-      "v_cmp_eq_f32_e64 %9, %0, %11\n\t"
-      "v_cndmask_b32_e64 %1, %3, %1, %8\n\t"
-      "v_cndmask_b32_e64 %4, %4, %5, %8\n\t"
-      "v_cndmask_b32_e64 %5, 2, 0, %8\n\t"
-      "v_cndmask_b32_e64 %1, %0, %1, %9\n\t"
-      "v_max3_f32 %6, %6, %12, %4\n\t"
-      "v_cndmask_b32_e64 %4, 1, 0, %9\n\t"
-      "v_max_f32_e32 %6, %6, %1\n\t"
+      "v_cndmask_b32_e64 %0, %2, %0, %9\n\t"
+      "v_cmp_eq_f32_e64 %8, %0, %20\n\t"
+      "v_cndmask_b32_e64 %1, %3, %1, %9\n\t"
+      "v_cndmask_b32_e64 %4, %4, %5, %9\n\t"
+      "v_cndmask_b32_e64 %1, %0, %1, %8\n\t"
+      "v_cndmask_b32_e64 %5, 2, 0, %9\n\t"
+      "v_max3_f32 %6, %6, %4, %1\n\t"
+      "v_cndmask_b32_e64 %4, 1, 0, %8\n\t"
       "v_add3_u32 %7, %7, %5, %4\n\t"
-      "v_add_u32_e32 %7, %7, %13"
-      : "+&v"(y0), "+&v"(y1), "+&v"(y2), "+&v"(y3), "=&v"(y5), "=&v"(y6), "+&v"(second), "+&v"(row), "=&s"(e8), "=&s"(e)
-      : "v"(y4), "v"(m), "v"(t), "v"(base));
+      "v_add_u32_e32 %7, %21, %7"
+      : "=&v"(z0), "=&v"(z1), "=&v"(z2), "=&v"(z3), "=&v"(t), "=&v"(u), "=&v"(second), "=&v"(row), "=&s"(e4), "=&s"(e)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(low4), "v"(high4), "v"(m),
+        "v"(base));
   return row;
 }
 
@@ -207,34 +218,34 @@ struct KmScan {
   static_assert(W % 4 == 0, "an instruction's first row modulo 16 is the wave's");
   static constexpr int TOKENS = W * 32 * TT;
   static constexpr int L = CT / 4 / W;   // loads of a wave per tile
-  // Tokens as operands: lane: token r, dims 16 kk + 8 hh.  A load whose lanes touch 32 tokens keeps the compute unit's address
-  // path busy for 64 cycles, one of four whole tokens for 18; with eight waves that start together that is in front of the
-  // first product.  Their tokens are loaded whole and turned in the wave's part of the last tile buffer, which no tile is on
-  // its way to yet, 16 at a time, piece k of token t at place k ^ t of its row (8 x 8192 tokens, 512 centroids: 11.4 -> 10.3
-  // us, 16 x 8200 22.8 -> 20.8, 4 x 15000, 928 17.0 -> 16.0; 4 x 48719, 3072 120.6 and 121.4; four columns of long loops the
-  // same, so they stay).  The small tiles of four
-  // waves leave room for eight tokens at a time, and other workgroups run beside: as operands (128 x 8192: 121.9 us, turned
-  // 124.1).
+  // Tokens as operands: lane: token c, dims 32 kk + 8 g.  A load whose lanes touch sixteen tokens keeps the compute unit's address
+  // path busy longer than one of four whole tokens; where waves start together that is in front of the first product.  Their
+  // tokens are loaded whole and turned in the wave's part of the last tile buffer, which no tile is on
+  // its way to yet, 16 at a time, piece k of token t at place k ^ t of its row.  Tiles of 32 rows leave no room for sixteen
+  // tokens, and other workgroups run beside: as operands.
   static constexpr int WR = CT / W;
-  static constexpr bool TURN = WR == 16 && TT < 4;
-  // Operands from LDS: each is requested AHEAD products before its own, into the register that a product has just read, across
-  // sub-tiles where a tile has several.  (The compiler has two on their way and waits for each; as many more as the
-  // registers hold.  8 x 8192 tokens, 512 centroids: 10.2 -> 9.3 us, 16 x 8200 22.4 -> 20.7, 4 x 48719, 3072 119 -> 118,
-  // 128 x 8192 120.6 -> 117.6, 8 x 131072, 8192 1531 -> 1512.)
-  static constexpr int AHEAD = TT == 2 ? 3 : CT == 32 ? 0 : TT == 4 ? 4 : 8;
+  static constexpr bool TURN = WR == 16;
+  // Operands from LDS: each is requested AHEAD steps before its own, into the register that a product has just read, across
+  // sub-tiles where a tile has several.  Us with none / 2 or 4 / 3, 6 or 7 ahead: 8 x 8192 tokens, 512 centroids 8.7 / 8.2 / 8.5,
+  // 4 x 8192, 512 7.5 / 7.2 / 6.9, 28 x 8192 28.2 / 27.4 / 27.5, 8 x 131072, 8192 1405 / 1378 / 1378 (and 1410 with four, where a
+  // register too many leaves three workgroups to a compute unit).
+  static constexpr int AHEAD = TT == 2 ? 2 : CT == 64 ? 6 : 4;
+
+  static constexpr bool TIED = TT > 1;   // (registers are short)
 
   uint16_t (*sh)[CT][RI_DIM];   // [NB] tile buffers
   const uint16_t* cp;           // the problem's centroids
   const uint16_t* list;
-  int nc, lane, wave, r, hh;
+  int nc, lane, wave, r, hh;    // r, hh: this lane's token of a column's 32, and which half's answer (merged)
+  int c, g;                     // its token of sixteen, and its quarter of the products' dims and rows
   uint32_t next[L];             // LISTED: this lane's rows of the tile that is requested next
-  uint4 b[TT][8];
-  float best[TT], second[TT];
-  int at[TT];                   // where best was scored: the centroid, or its place in the list
+  uint4 b[TT][2][4];            // [column][sixteen tokens of it][products of 32 dims]
+  float best[TT][2], second[TT][2];
+  int at[TT][2];                // where best was scored: the centroid, or its place in the list
 
   __device__ __forceinline__ KmScan(uint16_t (*sh_c)[CT][RI_DIM], const uint16_t* centroids, int n)
       : sh(sh_c), cp(centroids), list(nullptr), nc(n), lane(threadIdx.x & 63),
-        wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), r(lane & 31), hh(lane >> 5) {}
+        wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), r(lane & 31), hh(lane >> 5), c(lane & 15), g(lane >> 4) {}
 
   // A tile goes from global memory straight into LDS, 16 bytes per lane and 1 KiB (four rows)
   // per wave instruction: lane l lands at byte l * 16 of the instruction's LDS window, and which
@@ -271,22 +282,26 @@ struct KmScan {
   }
   __device__ __forceinline__ void nothing_yet() {
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      best[tt] = second[tt] = -INFINITY;
-      at[tt] = 0;
-    }
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        best[tt][u] = second[tt][u] = -INFINITY;
+        at[tt][u] = 0;
+      }
   }
   // rows t0 .. of dp, the last one `last` (open: the rows named there)
   __device__ __forceinline__ void request_tokens(const uint16_t* dp, int t0, int last, const int32_t* open = nullptr) {
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int tok = min(t0 + tt * 32 + r, last);
-      const uint16_t* q = dp + (size_t)(open ? open[tok] : tok) * RI_DIM + hh * 8;
+    for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        b[tt][i] = TURN ? ri_ld16(dp + (size_t)min(t0 + tt * 32 + 4 * i + (lane >> 4), last) * RI_DIM + (lane & 15) * 8)
-                        : ri_ld16(q + i * 16);
-    }
+      for (int u = 0; u < 2; ++u) {
+        const int tok = min(t0 + tt * 32 + u * 16 + c, last);
+        const uint16_t* q = dp + (size_t)(open ? open[tok] : tok) * RI_DIM + g * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          b[tt][u][i] = TURN ? ri_ld16(dp + (size_t)min(t0 + tt * 32 + u * 16 + 4 * i + g, last) * RI_DIM + c * 8)
+                             : ri_ld16(q + i * 32);
+      }
   }
   // (The token registers are consumed here so that the compiler's own wait for their loads sits in front of the loop and not
   // inside it, where it would also wait for the tile in flight.)
@@ -294,35 +309,30 @@ struct KmScan {
     uint4* const turn = reinterpret_cast<uint4*>(&sh[NB - 1][wave * WR][0]);
     km_wait_vm<(NB - 1) * L>();
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      if (TURN) {
-        uint4 o[8];
+    for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int w = 0; w < 2; ++w) {
+      for (int u = 0; u < 2; ++u) {
+        if (TURN) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int row = 4 * i + (lane >> 4);
-            turn[row * 16 + ((lane & 15) ^ row)] = b[tt][w * 4 + i];
+            const int row = 4 * i + g;
+            turn[row * 16 + (c ^ row)] = b[tt][u][i];
           }
           ri_wave_sync();
-          if (r >> 4 == w) {
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) o[kk] = turn[(r & 15) * 16 + ((kk * 2 + hh) ^ (r & 15))];
-          }
+          for (int kk = 0; kk < 4; ++kk) b[tt][u][kk] = turn[c * 16 + ((kk * 4 + g) ^ c)];
           ri_wave_sync();   // (a wave's LDS accesses happen in order)
         }
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) b[tt][kk] = o[kk];
+        for (int kk = 0; kk < 4; ++kk)
+          asm volatile("" : "+v"(b[tt][u][kk].x), "+v"(b[tt][u][kk].y), "+v"(b[tt][u][kk].z), "+v"(b[tt][u][kk].w));
       }
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[tt][kk].x), "+v"(b[tt][kk].y), "+v"(b[tt][kk].z), "+v"(b[tt][kk].w));
-    }
   }
   // centroids (or places of the list) from .. end-1 against the tokens; track: with the second best
   __device__ __forceinline__ void score(int from, int end, bool track) {
-    const uint16_t* row_at[8];   // this lane's pieces of its row of a sub-tile
+    const uint16_t* row_at[8];   // this lane's pieces of its two rows of a sub-tile
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) row_at[kk] = &sh[0][r][((kk * 2 + hh) ^ (r & 15)) * 8];
+    for (int k = 0; k < 8; ++k) row_at[k] = &sh[0][k % 2 * 16 + c][((k / 2 * 4 + g) ^ c) * 8];
     for (int ct0 = from; ct0 < end; ct0 += NB * CT) {
 #pragma unroll
       for (int buf = 0; buf < NB; ++buf) {   // (unrolled: the buffer is in the offset of every LDS read)
@@ -344,83 +354,99 @@ struct KmScan {
 #pragma unroll
         for (int half = 0; half < CT / 32; ++half) {
           if (ct + half * 32 < end) {  // uniform: only the last tile can lack sub-tiles
-            f32x16_t acc[TT];
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-              for (int i = 0; i < 16; ++i) acc[tt][i] = 0.f;
+            f32x4_t acc[TT][2][2];
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) {
               const int k = half * 8 + kk;
               const uint4 a = AHEAD ? rows[k % (AHEAD ? AHEAD : 1)] : operand(k);
 #pragma unroll
-              for (int tt = 0; tt < TT; ++tt)
-                acc[tt] = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
-                                                                        __builtin_bit_cast(f16x8_t, b[tt][kk]), acc[tt], 0, 0, 0)
-                               : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[tt][kk]), acc[tt], 0,
-                                                                         0, 0);
+              for (int tt = 0; tt < TT; ++tt) {
+                if (kk < 2)
+                  km_products<HALF, TIED, true>(acc[tt][0][kk % 2], acc[tt][1][kk % 2], a, b[tt][0][kk / 2], b[tt][1][kk / 2]);
+                else
+                  km_products<HALF, TIED, false>(acc[tt][0][kk % 2], acc[tt][1][kk % 2], a, b[tt][0][kk / 2], b[tt][1][kk / 2]);
+              }
               if (AHEAD) {
                 if (k + AHEAD < CT / 4) rows[k % (AHEAD ? AHEAD : 1)] = operand(k + AHEAD);
                 __builtin_amdgcn_sched_barrier(0);
               }
             }
+            if (TIED) km_products_wait<TT>(acc);
             if (LISTED && ct + half * 32 + 32 > end) {   // uniform: rows past the last score nothing
-              const int left = end - (ct + half * 32) - hh * 4;
+              const int left = end - (ct + half * 32) - g * 4;
 #pragma unroll
               for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[tt][i] = i / 4 * 8 + i % 4 < left ? acc[tt][i] : -INFINITY;
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                  for (int i = 0; i < 8; ++i)
+                    acc[tt][u][i / 4][i % 4] = i / 4 * 16 + i % 4 < left ? acc[tt][u][i / 4][i % 4] : -INFINITY;
             }
-            // argmax epilogue: the lane's 16 scores are in ascending row order, so the first score
+            // argmax epilogue: the lane's eight scores are in ascending row order, so the first score
             // equal to their maximum is the lowest row; the index search only runs when some lane
             // of the wave improves on its best (about half of the sub-tiles of a full-size pass)
 #pragma unroll
-            for (int tt = 0; tt < TT; ++tt) {
-              // (both halves from a score seen before, which is no NaN: nine instructions.  From the second best where that is
-              // wanted: it then is the larger of the two wherever the best stays.)
-              float low8 = track ? second[tt] : best[tt], high8 = low8, low4 = low8, high4 = low8;
+            for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-              for (int i = 0; i < 8; ++i) {
-                low8 = fmaxf(low8, acc[tt][i]);
-                high8 = fmaxf(high8, acc[tt][8 + i]);
-                if (i == 3) low4 = low8, high4 = high8;
-              }
-              float m;
-              asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(low8), "v"(high8));   // (no NaN: the compiler would quiet one first)
-              const bool upd = m > best[tt];
-              if (!track) {
-                if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
-                  const int k = km_first_of(acc[tt], m, best[tt], low8, low4, high4, hh * 4 + ct + half * 32);
-                  at[tt] = upd ? k : at[tt];
-                  best[tt] = m;
+              for (int u = 0; u < 2; ++u) {
+                // (from a score seen before, which is no NaN.  From the second best where that is wanted: it then is the larger
+                // of the two wherever the best stays.)
+                const f32x4_t &x = acc[tt][u][0], &y = acc[tt][u][1];
+                float &top = best[tt][u], &next_best = second[tt][u];
+                const float seen = track ? next_best : top;
+                const float low4 = fmaxf(fmaxf(fmaxf(fmaxf(seen, x[0]), x[1]), x[2]), x[3]);
+                if (!track) {
+                  const float m = fmaxf(fmaxf(fmaxf(fmaxf(low4, y[0]), y[1]), y[2]), y[3]);
+                  const bool upd = m > top;
+                  if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+                    const int k = km_first_of(x, y, m, low4, g * 4 + ct + half * 32);
+                    at[tt][u] = upd ? k : at[tt][u];
+                  }
+                  top = m;   // (the same where no lane improves)
+                } else {
+                  const float high4 = fmaxf(fmaxf(fmaxf(fmaxf(seen, y[0]), y[1]), y[2]), y[3]);
+                  const float m = km_max(low4, high4);
+                  const bool upd = m > top;
+                  if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+                    float s;
+                    const int k = km_first_two(x, y, m, low4, high4, g * 4 + ct + half * 32, s);
+                    s = km_max(s, top);
+                    next_best = upd ? s : m;
+                    at[tt][u] = upd ? k : at[tt][u];
+                    top = upd ? m : top;
+                  } else {
+                    next_best = m;
+                  }
                 }
-              } else if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
-                float s;
-                const int k = km_first_two(acc[tt], m, low8, high8, low4, high4, hh * 4 + ct + half * 32, s);
-                asm("v_max_f32_e32 %0, %1, %2" : "=v"(s) : "v"(s), "v"(best[tt]));
-                second[tt] = upd ? s : m;
-                at[tt] = upd ? k : at[tt];
-                best[tt] = upd ? m : best[tt];
-              } else {
-                second[tt] = m;
               }
-            }
           }
         }
       }
     }
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) asm volatile("" : "+v"(best[tt]), "+v"(at[tt]));   // (one register each, whichever way out)
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) asm volatile("" : "+v"(best[tt][u]), "+v"(at[tt][u]));   // (one register each, whichever way out)
     km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's, or that another turn fills)
   }
-  // both halves of a wave have scored every other four rows for the same tokens: best, its place and second best of all
+  // The quarters of a wave have scored every other four rows for the same tokens: best, its place and second best of all of them
+  // for token r of a column, in both halves.  (The first exchange brings each row of lanes two quarters' answers for the
+  // sixteen tokens that are its own.)
   __device__ __forceinline__ void merged(int tt, float& top, int& place, float& next_best) {
-    const float ob = km_other(best[tt], hh);
-    const int oi = __float_as_int(km_other(__int_as_float(at[tt]), hh));
-    const bool other = ob > best[tt] || (ob == best[tt] && oi < at[tt]);
-    next_best = fmaxf(fminf(ob, best[tt]), ri_xor_max<32>(second[tt]));
-    top = other ? ob : best[tt];
-    place = other ? oi : at[tt];
+    const auto pair = [](uint32_t x, uint32_t y) { return __builtin_bit_cast(km_pair, __builtin_amdgcn_permlane16_swap(x, y, false, false)); };
+    const km_pair pb = pair(__float_as_uint(best[tt][0]), __float_as_uint(best[tt][1])), pa = pair(at[tt][0], at[tt][1]),
+                  ps = pair(__float_as_uint(second[tt][0]), __float_as_uint(second[tt][1]));
+    const auto first = [](float x, int i, float y, int j) { return y > x || (y == x && j < i); };   // the other one's
+    const float x0 = __uint_as_float(pb.x), x1 = __uint_as_float(pb.y);
+    const bool o = first(x0, (int)pa.x, x1, (int)pa.y);
+    const float b = o ? x1 : x0, s = fmaxf(fminf(x0, x1), fmaxf(__uint_as_float(ps.x), __uint_as_float(ps.y)));
+    const int a = o ? (int)pa.y : (int)pa.x;
+    const float ob = km_other(b, hh);
+    const int oa = __float_as_int(km_other(__int_as_float(a), hh));
+    const bool other = first(b, a, ob, oa);
+    next_best = fmaxf(fminf(ob, b), ri_xor_max<32>(s));
+    top = other ? ob : b;
+    place = other ? oa : a;
   }
 };
 
@@ -451,12 +477,12 @@ __global__ __launch_bounds__(W * 64) void km_assign_kernel(const uint16_t* __res
 // A pass of a clustering that knows the pass before (KmBounds), grid (ceil(N / TOKENS), P).  The clusters that no token has
 // joined or left keep their centroids, most keys win against unit vectors by their norm, and a token whose second best score
 // is known needs no more than the centroids that were written since: the same scores, hence the same assignment, of far fewer
-// products.  8 x 131072 tokens, 8192 centroids, us of ten passes: 10 x 1524 -> 1524 (all), 1308, 585, 105 and 73 + 391 (keys
-// left: 81, 38, 4 and 0.1 %; a fifth of the tokens is left open by the last), 1700 (all, with the second best: its search is
-// what a full pass loses by it), 1481 + 67, 722 + 61, 463 + 54 and 324 + 40 (90, 46, 28 and 19 % of the centroids written, 3 to
+// products.  8 x 131072 tokens, 8192 centroids, us of ten passes: 10 x 1383 -> 1383 (all), 1252, 569, 103 and 69 + 400 (keys
+// left: 81, 38, 4 and 0.1 %; a fifth of the tokens is left open by the last), 1684 (all, with the second best: its search is
+// what a full pass loses by it), 1395 + 69, 678 + 62, 438 + 55 and 313 + 43 (90, 46, 28 and 19 % of the centroids written, 3 to
 // 1.6 % of the tokens open).  Two columns of tokens and small tiles: with a short list the load of the tokens is the launch, and
-// three workgroups per compute unit overlap it (19 % of 8192: 324, of which 55 are the bytes; four columns, 8 waves: 393;
-// one column: 450).  The problems' workgroups are dealt over all chiplets, unlike those of a plain pass: problems take unequal
+// three workgroups per compute unit overlap it (19 % of 8192, with products of 32 rows: 324, of which 55 are the bytes; four
+// columns, 8 waves: 393; one column: 450).  The problems' workgroups are dealt over all chiplets, unlike those of a plain pass: problems take unequal
 // time (12943 -> 14059 with a problem to a chiplet).
 template <int TT, int CT, int W, int NB, bool HALF>
 __global__ __launch_bounds__(W * 64, TT == 2 ? 3 : 2) void km_assign_again_kernel(
@@ -479,10 +505,12 @@ __global__ __launch_bounds__(W * 64, TT == 2 ? 3 : 2) void km_assign_again_kerne
   s.nothing_yet();
   if (mode == KM_NEW) {   // (scores up to the bound are of no interest)
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      s.best[tt] = s.second[tt] = B.bound[first_token + min(t0 + tt * 32 + s.r, N - 1)];
-      s.at[tt] = nc - 1;   // (unless one does: uncertain below)
-    }
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        s.best[tt][u] = s.second[tt][u] = B.bound[first_token + min(t0 + tt * 32 + u * 16 + s.c, N - 1)];
+        s.at[tt][u] = nc - 1;   // (unless one does: uncertain below)
+      }
   }
   __syncthreads();
   s.start(0, max(n1, 1));
@@ -521,18 +549,20 @@ __global__ __launch_bounds__(W * 64, TT == 2 ? 3 : 2) void km_assign_again_kerne
       } else if (mode == KM_KEYS) {
         // |x c| <= |x| |c|, and a centroid that an update has written is a unit vector rounded to 16 bits (and this sum,
         // like the scores, to 32: far inside the hundredth)
-        float sq = 0.f;
+        float part_sq[2] = {0.f, 0.f};
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
+          for (int kk = 0; kk < 16; ++kk) {
             float lo, hi;
-            uint32_t word = (&s.b[tt][kk].x)[i];
+            uint32_t word = (&s.b[tt][u][kk / 4].x)[kk % 4];
             asm volatile("" : "+v"(word));   // (here, and not ahead of the loop: the registers are full)
             ri_unpack2<HALF>(word, lo, hi);
-            sq = fmaf(lo, lo, fmaf(hi, hi, sq));
+            part_sq[u] = fmaf(lo, lo, fmaf(hi, hi, part_sq[u]));
           }
-        ok = top[tt] > 1.01f * sqrtf(ri_xor_sum<32>(sq)) + 1e-17f && !B.odd[p];   // (1e-17: squares too small for a float)
+        const km_pair sq = __builtin_bit_cast(km_pair, __builtin_amdgcn_permlane16_swap(   // (as in `merged`)
+                               __float_as_uint(part_sq[0]), __float_as_uint(part_sq[1]), false, false));
+        ok = top[tt] > 1.01f * sqrtf(ri_xor_sum<32>(__uint_as_float(sq.x) + __uint_as_float(sq.y))) + 1e-17f && !B.odd[p];   // (1e-17: squares too small for a float)
       }
       __builtin_amdgcn_sched_barrier(0);
       if (ok) sure |= 1u << tt;
@@ -583,7 +613,7 @@ using KmOpenScan = KmScan<2, 32, 4, 4, HALF, false>;
 // The tokens that a pass left open (a few in a hundred), against all centroids, grid KM_OPEN_WGS: blocks of a problem's open tokens, each cut into
 // as many parts of the centroids as there are workgroups for; the last of a block's parts to arrive puts them together.
 // (What the others wrote reaches it by write-through stores that are complete before they arrive.)  Bound by the matrix cores
-// where there are many (210000 of 8 x 131072, 8192 centroids: 391 us, a full pass's rate), else by its chain: 400 tokens of
+// where there are many (210000 of 8 x 131072, 8192 centroids: 400 us), else by its chain: 400 tokens of
 // eight problems, 640 centroids: 10.5 us, 17 while the parts were put together one after the other.
 template <bool HALF>
 __global__ __launch_bounds__(256) void km_assign_open_kernel(const uint16_t* __restrict__ data,
@@ -1702,33 +1732,21 @@ static void km_assign_launch(const void* data, const void* centroids, int32_t* a
 #define KM_ASSIGN_LAUNCH(TT, CT, W, NB)                                                                                  \
   km_assign_kernel<TT, CT, W, NB, HALF><<<km_grid((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, stream>>>( \
       (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P))
-  const long long wgs128 = (long long)P * ((N + 127) / 128), wgs256 = (long long)P * ((N + 255) / 256);
-  const long long wgs768 = (long long)P * ((N + 767) / 768);
-  const long long wgs1024 = (long long)P * ((N + 1023) / 1024), rounds1024 = (wgs1024 + 255) / 256;
-  // A launch that does not fill the chip wants its waves spread: one token column per wave and, once there are two
-  // workgroups per compute unit of it, eight waves that share long tiles (8 x 8192 tokens, 512 centroids: 12.9 us
-  // against 18.9 with two columns when they were compared, now 8.7 against 11.8; 2 x 1708 tokens, 96 centroids: 4.9
-  // against 6.7).
-  if (wgs128 <= 256) KM_ASSIGN_LAUNCH(1, 32, 4, 2);
-  // A little more than those two per compute unit is a second round for a few: three columns per wave then do it in one
-  // round, the longer the loop the further.  By centroids, workgroups of one column and us with three columns / one: 512
-  // centroids, 520 21.5 / 22.2, 576 22.7 / 22.8; 768, 520 27.9 / 29.8, 576 30.6 / 31.4, 624 32.5 / 31.9; 1024, 520 35.9 / 39.0,
-  // 640 41.2 / 41.2, 688 43.1 / 42.8; 1536, 520 51.0 / 56.2, 720 63.0 / 63.1, 752 66.6 / 65.4; 2048, 520 65.9 / 74.3, 752 84.3 /
-  // 85.2; 3072, 520 95.5 / 109.2, 752 121.6 / 123.6.  (92 shapes of 4, 8 and 16 problems; the ones between lie between.)
-  else if (nc >= 512 && wgs256 > 512 && wgs256 <= 440 + nc / 5 && wgs256 <= 768 && wgs768 <= 256) KM_ASSIGN_LAUNCH(3, 128, 8, 2);
-  // (up to three of them: 22 x 8192 tokens, 512 centroids: 24.4 us against 25.4 with two columns, 26.5 with three; 24 x 8119:
-  // 25.2 against 25.7; 24 x 8192, 256: 16.4 either way; 28 x 8192: 30.8 against 30.0)
-  else if (wgs256 <= 768) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
-  // Long centroid loops: most reuse of every LDS read, eight waves of four columns on a compute unit of their own (8 x
-  // 131072 tokens, 8192 centroids: 1607 us against 1646 for two workgroups of four waves, now 1512; 4 x 61440, 3840: 177
-  // against 178 with two columns, 4 x 51000, 3200: 136 against 139, 4 x 65536, 2048: 104.2 against 102.7), provided the
-  // last round of these large workgroups is not mostly empty.
-  else if (nc > 2048 && (wgs1024 <= 256 || wgs1024 * 100 >= rounds1024 * 256 * 87)) KM_ASSIGN_LAUNCH(4, 128, 8, 2);
-  // Otherwise the load of the tokens in front of the loop is a large part of the kernel, and 128 registers and 32 KB of
-  // LDS let four workgroups per compute unit overlap one's loads with the others' products (128 x 8192 tokens, 512
-  // centroids: 111.3 us, one column 124, four 130, three 142, two in eight waves and tiles of 128 136; 32 x 8192: 31.6,
-  // 32.7, 34.6, 43.9, 36.5).
-  else KM_ASSIGN_LAUNCH(2, 32, 4, 4);
+  // Long launches: two columns, 128 registers and 32 KB of LDS, four workgroups to a compute unit; the load of one's tokens runs
+  // under the others' products.  (8 x 131072 tokens, 8192 centroids: 1393 us, four columns in eight waves 1397; 8 x 96000, 3072:
+  // 419 and 435; 128 x 8192, 512: 118 and 132.)  Short ones by how their 256-token pieces fall on 256 compute units: a last
+  // round that is more than half full is best made of eight waves that share long tiles, one that is emptier of half as many
+  // tokens per workgroup, with more LDS for each while there is one round.  Us by 256-token pieces, 512 centroids, <1, 64, 4, 2>
+  // / <1, 32, 4, 3> / <1, 128, 8, 2> / <2, 32, 4, 4>: 128 7.2 / 8.1 / 8.6 / 12.4, 256 9.1 / 10.0 / 9.1 / 12.7, 350 12.7 / 13.9 /
+  // 14.3 / 17.1, 420 15.3 / 17.1 / 14.6 / 17.1, 576 22.0 / 21.7 / 23.7 / 24.8, 768 27.1 / 26.6 / 26.0 / 26.8, 896 30.0 / 29.3 /
+  // 31.0 / 31.4, 1024 34.3 / 33.3 / 32.8 / 34.5, 1100 36.1 / 35.1 / 37.8 / 37.8, 1400 43.7 / 43.6 / 44.9 / 43.0, 3000 89.7 / 85.6 /
+  // 87.0 / 82.2; 4096 centroids: 128 40.9 / 45.5 / 47.6 / 71.3, 640 137.8 / 136.3 / 141.6 / 145.7, 1024 209.7 / 210.7 / 196.6 /
+  // 196.0; 128 centroids, 1024 15.5 / 16.0 / 19.0 / 17.5.  (270 shapes of eight problems.)
+  const long long pieces = (long long)P * ((N + 255) / 256);
+  if (pieces > 1152) KM_ASSIGN_LAUNCH(2, 32, 4, 4);
+  else if ((pieces - 1) % 256 >= 128 && (nc >= 256 || pieces <= 768)) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
+  else if (pieces <= 384) KM_ASSIGN_LAUNCH(1, 64, 4, 2);
+  else KM_ASSIGN_LAUNCH(1, 32, 4, 3);
 #undef KM_ASSIGN_LAUNCH
 }
 

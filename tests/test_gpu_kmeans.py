@@ -123,6 +123,16 @@ def test_assign_long_loops_and_three_columns(dev, P, N, nc, dt):
     test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt)
 
 
+# Which tiling serves a launch follows its 256-token pieces: both sides of every line.
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("pieces,nc", [(128, 96), (129, 96), (256, 96), (257, 96), (384, 96), (385, 96), (512, 96), (513, 96),
+                                       (640, 96), (641, 96), (768, 96), (769, 96), (1024, 96), (1024, 288), (1152, 96),
+                                       (1153, 96)])
+def test_assign_at_the_lines_between_tilings(dev, pieces, nc, dt):
+    test_assign_tilings(dev, 1, pieces * 256 - 3, nc, dt)
+    test_assign_ties_go_to_the_lowest_id(dev, 1, pieces * 256 - 3, nc, dt)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("P,N,nc", [(5, 1001, 32), (8, 8193, 544), (16, 8200, 544), (20, 9757, 608), (33, 8200, 512),
                                     (2, 32768, 2048)])
