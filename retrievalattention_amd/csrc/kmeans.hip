@@ -1981,14 +1981,14 @@ extern "C" int ri_kmeans_update_direct_f16(const void* data, const int32_t* assi
 // Whether passes know the ones before.  They read every token again (8 x 131072: 55 us), which short passes are bound by
 // anyway, and each is one launch more (5 us, 10 with a few tokens open).  Ten assignments and nine updates, us without / with,
 // by problems, tokens and centroids, keys in clusters (as many as centroids) with four large dimensions | without any structure:
-// 8 x 16400, 512: 486 / 569 | 432 / 510; 8 x 20000, 640: 611 / 648 | 529 / 588; 1 x 65536, 2048: 687 / 753 | 518 / 645; 8 x
-// 20000, 1248: 807 / 775 | 727 / 610; 8 x 32768, 1024: 971 / 947 | 861 / 860; 2 x 65536, 2048: 976 / 890 | 824 / 798; 1 x
-// 131072, 2720: 1161 / 1045 | 1010 / 1074; 4 x 32768, 2048: 893 / 785 | 818 / 647; 2 x 65536, 4096: 1422 / 1094 | 1343 / 921;
-// 8 x 65536, 1376: 1922 / 1640 | 1810 / 1828; 1 x 131072, 8192: 2563 / 1804 | 2365 / 1455; 8 x 131072, 8192: 15863 / 9751 |
-// two of those 4125 / 2345.  So from 2^28 scores a pass on.  (Up to 16384 tokens the lists never leave a workgroup, and a pass is
+// 8 x 16400, 512: 473 / 586 | 419 / 530; 8 x 20000, 640: 572 / 664 | 498 / 598; 1 x 65536, 2048: 657 / 791 | 487 / 700; 8 x
+// 20000, 1248: 760 / 796 | 684 / 616; 8 x 32768, 1024: 934 / 976 | 828 / 893; 2 x 65536, 2048: 901 / 898 | 756 / 807; 4 x 32768,
+// 2048: 827 / 793 | 752 / 649; 1 x 131072, 2720: 1069 / 1058 | 926 / 1086; 2 x 65536, 4096: 1295 / 1097 | 1214 / 927; 8 x 65536,
+// 1376: 1847 / 1648 | 1742 / 1807; 1 x 131072, 8192: 2325 / 1782 | 2135 / 1465; 8 x 131072, 8192: 14806 / 9586 | 14456 /
+// 7570.  So from 2^29 scores a pass on.  (Up to 16384 tokens the lists never leave a workgroup, and a pass is
 // bound by its keys.  64 problems: a lane each where the open tokens are dealt out; 16384 centroids: their order in LDS.)
 static bool km_bounded(int P, int N, int nc) {
-  return N > KM_DIRECT_MAX && P <= 64 && nc <= 16384 && (int64_t)P * N * nc >= 1ll << 28;
+  return N > KM_DIRECT_MAX && P <= 64 && nc <= 16384 && (int64_t)P * N * nc >= 1ll << 29;
 }
 
 __global__ __launch_bounds__(KM_OPEN_WGS + 64) void km_clear_kernel(int32_t* p, int n) {

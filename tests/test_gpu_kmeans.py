@@ -440,7 +440,7 @@ def _passes_one_by_one(keys, cent, seg, updates, last):
 # centroids, the most problems, segments with tokens left over; and shapes on the other side of the line.
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("kind", ["mixture", "normal", "ties", "odd"])
-@pytest.mark.parametrize("G,N,nc,seg", [(3, 45001, 2080, 1), (1, 17001, 16384, 1), (64, 16385, 288, 1), (2, 50003, 8192, 2),
+@pytest.mark.parametrize("G,N,nc,seg", [(6, 45001, 2080, 1), (2, 17001, 16384, 1), (64, 16385, 544, 1), (2, 70003, 8192, 2),
                                         (1, 20001, 64, 1), (2, 3001, 192, 3)])
 def test_iterate_equals_its_passes(dev, G, N, nc, seg, kind, dt):
     """Bit for bit the centroids and the assignment of the passes run one by one."""
