@@ -217,7 +217,8 @@ def bench_kmeans(cfg, dev, iters=10, reps=3):
     t_un = time_region(lambda: segment_k_means_csr(K, V, nc, iters, 1, init_indices=init, reuse_graph=True), reps)
     flops_un = 2.0 * 128 * Hkv * N * iters * nc
     unseg = {"ms_per_sequence": t_un * 1e3, "algorithmic_flops": flops_un, "achieved": flops_un / t_un / 1e12,
-             "frac": flops_un / t_un / MFMA_BF16_PEAK, "init": "seeded random tokens"}
+             "frac": flops_un / t_un / MFMA_BF16_PEAK, "init": "seeded random tokens",
+             "note": "flops of every pass over all centroids; passes leave out scores that cannot change an assignment"}
     return {"unsegmented": unseg, "ms_per_sequence": t * 1e3, "tokens": N, "kv_heads": Hkv, "centroids": nc, "segments": S,
             "iterations": iters, "algorithmic_flops": flops, "bound": "mfma", "achieved": flops / t / 1e12,
             "peak": MFMA_BF16_PEAK / 1e12, "unit": "TFLOP/s", "frac": flops / t / MFMA_BF16_PEAK,
@@ -714,25 +715,40 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
     reps_t.sort()
     t_step = reps_t[len(reps_t) // 2]
 
-    # the dominant kernel's duration inside the replayed step: the same layer cycle without its launch
-    # (score_kernel + dist_kernel + select_kernel only), both cycles timed by one event pair each on the
-    # launch stream; the difference is attend_kernel plus the gap in front of it
+    # the attention's duration behind a selection: in the step the attention's workgroups make the selection themselves
+    # (select_attend_kernel), so a layer cycle of both as launches of their own and one of the selection alone are timed by
+    # one event pair each on the launch stream; the difference is attend_kernel plus the gap in front of it
+    from retrievalattention_amd import kernels, _lib
+    out_tmp = torch.empty((BG, gs, 128), dtype=DT, device=dev)
+
+    def attend(l, slot):
+        kernels.wave_attention(
+            queries[l].view(BG, gs, 128), cache.steady_zone_keys[l], cache.steady_zone_values[l], static_len,
+            cache.list_keys[l], cache.list_values[l], None, cache.meta, cache.est_ids[slot], cache.logits,
+            cache.value_sum[l], cache.cluster_size[l], out_tmp, cache.valid_lengths[slot], es, cache.RSQRT_DIM,
+            ret_tok_off=cache.ret_tok_off, ret_start=cache.ret_start)
+
     t_attn_in_step = None
     if graphs is not None:
         sel_cycle = torch.cuda.CUDAGraph()
         with torch.cuda.graph(sel_cycle):
             for i in range(CL):
                 cache._select(queries[i % L], i % L, i % 2, True)
+        apart = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(apart):
+            for i in range(CL):
+                cache._select(queries[i % L], i % L, i % 2, True)
+                attend(i % L, i % 2)
         torch.cuda.synchronize()
         e0, e1, e2 = (torch.cuda.Event(enable_timing=True) for _ in range(3))
         best = [float("inf"), float("inf")]
         n_cyc = max(1, args.steps // CL)
         for _ in range(3):
             for _ in range(2):
-                cycle.replay()
+                apart.replay()
             e0.record()
             for _ in range(n_cyc):
-                cycle.replay()
+                apart.replay()
             e1.record()
             for _ in range(n_cyc):
                 sel_cycle.replay()
@@ -744,19 +760,9 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
 
     # per-kernel pass: the same layer cycle launched eagerly, one event pair around each entry point's
     # launches on the launch stream (cold caches as in the timed region: every step is another layer)
-    from retrievalattention_amd import kernels, _lib
     stream = torch.cuda.current_stream().cuda_stream
     n_k = min(args.steps, 256)
     ev = [[torch.cuda.Event(enable_timing=True) for _ in range(4)] for _ in range(n_k)]
-    out_tmp = torch.empty((BG, gs, 128), dtype=DT, device=dev)
-
-    def attend(l, slot):
-        kernels.wave_attention(
-            queries[l].view(BG, gs, 128), cache.steady_zone_keys[l], cache.steady_zone_values[l], static_len,
-            cache.list_keys[l], cache.list_values[l], None, cache.meta, cache.est_ids[slot], cache.logits,
-            cache.value_sum[l], cache.cluster_size[l], out_tmp, cache.valid_lengths[slot], es, cache.RSQRT_DIM,
-            ret_tok_off=cache.ret_tok_off, ret_start=cache.ret_start)
-
     for i in range(n_k + 8):
         l, slot = i % L, i % 2
         e = ev[max(i - 8, 0)]
@@ -803,10 +809,10 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
                                "GBps": attn_bytes / t_attn / 1e9},
         },
     }
-    # dominant kernel: attend_kernel, the one launch of ri_wave_attention (longest kernel, and the one that
-    # moves the K/V bytes).  Its duration is taken inside the replayed step (step cycle minus the cycle
-    # without it); an event pair around one eager launch also counts the dispatch of the launch
-    # (eager_event_us; null_launch_us is what the same pair reads around an empty kernel).
+    # dominant kernel: the attention (the one that moves the K/V bytes), as a launch of its own, attend_kernel.  Its duration is
+    # taken in a replayed cycle behind the selection's launches (that cycle minus the one without it); an event pair around one
+    # eager launch also counts the dispatch of the launch (eager_event_us; null_launch_us is what the same pair reads around an
+    # empty kernel).  The timed step itself has one launch for selection and attention.
     t_dom = t_attn_in_step if t_attn_in_step else t_attn
     traffic, traffic_source = measured_traffic(config_name)
     result["roofline"] = {"bound": "hbm", "kernel": "attend_kernel (ri_wave_attention)",
