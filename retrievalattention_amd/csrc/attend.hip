@@ -124,10 +124,12 @@ static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int e
   per_group = min(per_group, (int64_t)max_splits);
   if (per_group > 8 && per_group % 8 * 5 <= per_group && rows <= 64 * ATT_WAVES * per_group) per_group -= per_group % 8;
   if ((!several && attend_alone(rows, gs, BG)) || per_group < 1) per_group = 1;
-  const int waves = (int)per_group * ATT_WAVES;
+  const auto with_keys = [&](int64_t waves) {
+    return (int)(es_rows > 0 ? min(max((wk * waves + (wk + we) / 2) / (wk + we), (int64_t)1), waves - 1) : waves);
+  };
   P.S = (int)per_group;
-  P.W_kv = waves;
-  if (es_rows > 0) P.W_kv = (int)min(max((wk * waves + (wk + we) / 2) / (wk + we), (int64_t)1), (int64_t)(waves - 1));
+  P.W_kv = with_keys(per_group * ATT_WAVES);
+  P.W_one = with_keys(ATT_WAVES);
 }
 
 static int flash_decoding_impl(const void* q, const void* k, const void* v, const void* weight,

@@ -173,6 +173,7 @@ struct AttendParams {
   int* counters;    // [BG]
   int S;     // workgroups per group
   int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
+  int W_one; // the same of one workgroup's waves, if it takes the whole group
   int gs;
   float scale;
   // epilogue

@@ -62,12 +62,17 @@ __device__ __forceinline__ void store_selection(const SelectArgs& S, int g, cons
 // the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 523 / 843 / 1099 rows:
 // 15.0 / 17.3 / 19.8 / 22.7 us with one workgroup, 14.6 / 14.6 / 14.8 / 16.5 with several (16.3 .. 18.8 in two launches); the
 // retrieval of 10 % of the clusters, 8 groups of 8 heads 20.7 -> 19.0 (two launches -> SPLIT), 16 of 4 20.8 -> 19.4, 128 of 8
-// 33.6 -> 31.7.  step_route.h says which step takes which form.
+// 33.6 -> 31.7.  step_route.h says which step takes which form.  The rows that the clusters hold, and the zone's in a captured
+// step, are known behind the selection only: where they turn out to be few, one workgroup attends them all and hands no partial
+// over, and another stores the results (captured, 8 groups of 1 head, 4000 tokens 14.6 -> 13.4 us, 1 of 4, 8192 15.0 -> 14.5, 8 of
+// 8, 8192 16.3 -> 16.1, 128 of 8, 8192 23.3 -> 22.4).  With one workgroup the query's pieces ahead of the selection cost more
+// than they save: 8 groups of 4 heads 13.3 -> 13.15, 32 of 4, 3000 tokens 12.3 -> 12.1 without.
 // ------------------------------------------------------------------------------------
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
 template <int GSM, bool HALF, bool SPLIT>
-__global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int4 n, float scale, SelectArgs S0, AttendParams A0) {
+__global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int4 n, float scale, int one_rows,
+                                                           SelectArgs S0, AttendParams A0) {
   static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
   __shared__ __attribute__((aligned(16))) float sh_logits[STEP_CLUSTERS * GSM];
   static_assert(__alignof__(sh_logits) == 16, "read four heads at a time");
@@ -85,11 +90,24 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.es = A.es = n[3];
   S.scale = A.scale = scale;
   const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta};
-  const AttendKept known = {sh_logits, sh_est, sh_off, sh_start, att_query_piece(A, blockIdx.x), att_steady_rows(A)};
+  AttendKept known = {sh_logits, sh_est, sh_off, sh_start};
+  const auto ahead = [&]() {
+    known.q = att_query_piece(A, blockIdx.x);
+    known.lenA = att_steady_rows(A);
+  };
+  if (SPLIT) ahead();
   select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, SPLIT ? KEEP_TABLES : KEEP_ALL>(S, blockIdx.x, kept);
   lds_barrier();
-  attend_group<GSM, HALF, SPLIT ? KEPT_LOGITS : KEPT_ALL>(A, blockIdx.x, SPLIT ? blockIdx.y : 0, known);
-  if (SPLIT && blockIdx.y == 0) {
+  if (!SPLIT) ahead();
+  // (the same in all of the group's workgroups)
+  const bool one = SPLIT && known.lenA + sh_off[S.np] + S.es <= one_rows;
+  if (one) {
+    A.S = 1;
+    A.W_kv = A.W_one;
+  }
+  if (!one || blockIdx.y == 0)
+    attend_group<GSM, HALF, SPLIT ? KEPT_LOGITS : KEPT_ALL>(A, blockIdx.x, SPLIT ? blockIdx.y : 0, known);
+  if (SPLIT && blockIdx.y == (one && gridDim.y > 1 ? 1 : 0)) {
     store_selection(S, blockIdx.x, kept);
     const int nc = S.nc;
     for (int j = 0; j < S.gs; ++j)
@@ -165,7 +183,8 @@ static void launch_step(const SelectArgs& S, const AttendParams& A, int BG, bool
   auto* kernel = S.gs <= 4 ? (half ? step_kernel<4, true, SPLIT> : step_kernel<4, false, SPLIT>)
                            : (half ? step_kernel<8, true, SPLIT> : step_kernel<8, false, SPLIT>);
   kernel<<<dim3(BG, A.S), 64 * ATT_WAVES, 0, stream>>>(ri_pack_ptrs(S.cent, S.q, S.mask, S.cluster_size),
-                                                       (ri_int4){S.nc, S.gs, S.np, S.es}, S.scale, S, A);
+                                                       (ri_int4){S.nc, S.gs, S.np, S.es}, S.scale, step_alone_rows(BG), S,
+                                                       A);
 }
 
 // The step in one launch (nc <= STEP_CLUSTERS, up to eight heads), or in scoring and one more.

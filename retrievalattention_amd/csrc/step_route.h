@@ -57,10 +57,12 @@ static inline bool step_is_joined(const ri_decode_step_t* s) {
 // / 13.5, 321: 13.4 / 13.5, 353: 13.7 / 13.5, with 512 clusters 331: 13.9 / 13.8 (a step, 15.2 either way), 523: 16.0 / 13.8; of 1 head 321: 13.0 / 13.1; 32
 // groups of 4 heads 321: 14.2 / 14.2, 417: 15.3 / 14.6.  With two workgroups per group only: 128 groups of 4 heads 417: 16.4 / 17.7,
 // of 8 heads, 512 clusters 587: 21.0 / 21.1; past 128 there is no second one.  A captured step, which starts at the length at hand
-// and ends at the zone's, may grow by a quarter past the line.
+// and ends at the zone's, may grow by a quarter past the line.  (Several workgroups that find fewer rows than the line leave them
+// to one: step_kernel.)
+static inline int step_alone_rows(int BG) { return BG > 64 ? 640 : 336; }
 static inline bool step_is_alone(const ri_decode_step_t* s, int static_len) {
   if (s->BG > 128) return true;
   const int64_t usual = (int64_t)s->np * 16 + s->es, zone = s->static_len_dev ? s->steady_stride : static_len;
-  const int64_t line = s->BG > 64 ? 640 : 336;
+  const int64_t line = step_alone_rows(s->BG);
   return static_len + usual <= line && zone + usual <= line * 5 / 4;
 }

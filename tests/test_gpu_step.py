@@ -79,6 +79,10 @@ def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static
     # several workgroups per group that score for themselves: many rows, few clusters, no estimation zone, cut pages
     (3, 8, 512, 51, 119, 98, 1000, False), (2, 4, 504, 512 - 8, 0, 700, 2000, True), (1, 1, 8, 1, 7, 900, 100, False),
     (5, 7, 384, 38, 100, 300, 20, False), (128, 3, 64, 12, 30, 700, 100, True), (256, 8, 32, 4, 20, 400, 100, False),
+    # of which one has all rows where they are few after all: on both sides of the line, and of the one for many groups
+    (3, 8, 512, 51, 119, 98, 4, True), (2, 4, 512, 20, 200, 128, 1, False), (2, 4, 512, 20, 200, 137, 1, False),
+    (5, 1, 384, 38, 0, 69, 10, True), (80, 4, 256, 40, 60, 69, 10, False), (80, 4, 256, 40, 60, 572, 1, True),
+    (80, 4, 256, 40, 60, 581, 1, True),
     # scored before: every number of clusters a thread takes, with remainders; who sums the scores; heads padded and not
     (2, 4, 520, 9, 100, 69, 100, False), (3, 8, 1024, 18, 237, 70, 200, True), (2, 16, 1032, 40, 300, 69, 300, False),
     (1, 12, 2048, 36, 475, 500, 200, False), (2, 9, 2056, 512, 300, 69, 2000, False), (1, 3, 4096, 73, 950, 0, 300, True),
