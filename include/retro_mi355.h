@@ -263,7 +263,9 @@ int ri_wave_attention_part_f16(const void* q, const void* steady_k, const void* 
 /* The decode step of one layer over a device-resident cluster store: ri_score_select, then ri_wave_attention, with
  * everything but the query, the steady zone's length and the output in one struct (host memory, read during the call)
  * that a caller fills once per layer (steps 1-8 of compute(), cache_hub/retroinfer_cache.py:549-697).  Fields are the
- * arguments of those two entry points under the same names; `half` selects IEEE half instead of bfloat16. */
+ * arguments of those two entry points under the same names; `half` selects IEEE half instead of bfloat16.
+ * Every step may count arrivals and leave partials in attn_workspace, also where one workgroup per group would do: steps
+ * that may overlap on the device must not share score_workspace or attn_workspace (nor any other buffer written here). */
 typedef struct ri_decode_step_t {
   const void* centroids;
   const uint8_t* mask;

@@ -35,6 +35,10 @@ def _pinned(shape, dtype, fill=None):
 
 
 class retroinfer_cache(KV_Cache):
+    """Calls of one cache work in buffers of the cache and follow one another on a stream.  Decode steps of two caches
+    share nothing and may run on two streams at a time."""
+    _scratch = None   # kernels.Scratch (None: the process's)
+
     def __init__(self, valid_start, layer_num, batch_size, max_length, num_key_value_heads, num_heads,
                  head_dim, dtype, layer_mapping, max_new_length, static_pattern_start, static_pattern_end, core,
                  n_centroids, n_segment, nprobe, max_compute_cluster_num, cache_unit_size, cache_cluster_num,
@@ -249,6 +253,8 @@ class retroinfer_cache(KV_Cache):
         BG, D, gs = self.batch_groups, self.head_dim, self.group_size
         i32 = lambda *s: torch.zeros(s, dtype=torch.int32, device=d0)
         self.logits = torch.zeros((BG, gs, self.n_centroids), dtype=torch.float32, device=d0)
+        self._scratch = kernels.Scratch()
+        self._allocate_scratch()
         # int64 id lists [BG, nprobe + es] as the reference keeps them: real tensors on the staged
         # operator path (gather_copy_vectors and the host id copy read them), views put together from the
         # int32 lists on demand elsewhere
@@ -283,6 +289,12 @@ class retroinfer_cache(KV_Cache):
             self.es_value_sum = torch.zeros((BG, es, 1, D), dtype=self.dtype, device=d0)
             self.es_cluster_size = torch.zeros((BG, 1, 1, es), dtype=self.dtype, device=d0)
 
+    def _allocate_scratch(self):
+        """The cache's own scratch areas, before anything captures a step: decode steps of other caches, on other
+        streams, count arrivals and leave partials in theirs."""
+        for device in {c.device for c in self.centroids}:
+            self._scratch.decoding(self.batch_groups, self.group_size, self.n_centroids, device)
+
     def pre_allocate_decision(self):
         """Kept for callers of the reference API; this build always pre-allocates."""
         return True
@@ -301,7 +313,7 @@ class retroinfer_cache(KV_Cache):
         self.temp_keys = self.temp_values = None
         self._centred_keys.clear()
         # the clusterings captured during this prefill replay with the addresses of the buffers just dropped
-        # (scratch tensors that were outgrown stay: a decode graph of another cache may still replay with them)
+        # (scratch tensors that were outgrown stay: a graph captured over operators may still replay with them)
         if not torch.cuda.is_current_stream_capturing():
             kernels.release_cached_graphs(retired_workspaces=False)
 
@@ -474,6 +486,7 @@ class retroinfer_cache(KV_Cache):
         torch.cuda.set_device(self.layer_mapping[str(0)])
         self.n_centroids += ncu
         self._plans.clear()
+        self._allocate_scratch()
         self.logits = torch.zeros((BG, self.group_size, self.n_centroids), dtype=torch.float32,
                                   device=self.layer_mapping[str(0)])
         self.static_pattern_total = sps + spe
@@ -572,7 +585,7 @@ class retroinfer_cache(KV_Cache):
             self.cluster_size_i32[layer] if dev_mode else None, self.cluster_start[layer] if dev_mode else None,
             self.logits, None, cI, self.ret_ids[buf], self.est_ids[buf] if es > 0 else None,
             ret_tok_off, None, meta, self.nprobe, es, self.page_size, self.buffer_size, self.RSQRT_DIM,
-            ret_start=ret_start)
+            ret_start=ret_start, scratch=self._scratch)
 
     def compute(self, queries, layer_idx, queries_next=None):
         """Decode attention of one layer (reference: retroinfer_cache.py:549-697).
@@ -629,7 +642,7 @@ class retroinfer_cache(KV_Cache):
             self.est_ids[buf] if es > 0 else None, self.logits if es > 0 else None, self.value_sum[layer_idx],
             self.cluster_size[layer_idx], out, self.valid_lengths[buf], es, self.RSQRT_DIM,
             ret_tok_off=self.ret_tok_off, ret_start=self.ret_start,
-            static_len_dev=self.steady_len_dev if self.device_positions else None)
+            static_len_dev=self.steady_len_dev if self.device_positions else None, scratch=self._scratch)
         return out.view(self.batch_size, 1, self.num_heads, D)
 
     def _plan(self, layer, buf):
@@ -651,7 +664,7 @@ class retroinfer_cache(KV_Cache):
             tensors = dict(zip(names, t), static_len_dev=length)
             plan = self._plans[(layer, buf)] = kernels.DecodeStepPlan(
                 key, self.dtype, tensors, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
-                self.RSQRT_DIM)
+                self.RSQRT_DIM, self._scratch)
         return plan
 
     def _host_plan(self, layer, buf):
@@ -673,7 +686,7 @@ class retroinfer_cache(KV_Cache):
             plan = self._plans[(layer, buf)] = kernels.HostStepPlan(
                 key, self.dtype, dict(zip(names, t)), self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size,
                 self.RSQRT_DIM, lru, other[0], other[1], lists, row_src, other[3], other[4],
-                self.cache_size * self.page_size)
+                self.cache_size * self.page_size, self._scratch)
         return plan
 
     def block_cache_stats(self, layer_idx):
@@ -732,7 +745,7 @@ class retroinfer_cache(KV_Cache):
             else:
                 self._stage_misses(layer_idx, buf)
         elif es > 0:   # zones came from the predicted query: the estimation zone is scored by the true one
-            kernels.score_logits(q, self.centroids[layer_idx], self.logits, self.RSQRT_DIM)
+            kernels.score_logits(q, self.centroids[layer_idx], self.logits, self.RSQRT_DIM, scratch=self._scratch)
         _, _, row_src, meta = self.layouts[buf if self.use_cluster_estimation else 0]
         out = torch.empty((BG, gs, D), dtype=self.dtype, device=queries.device)
         ck = self.cache_keys[layer_idx].view(BG, rows, D)
@@ -745,19 +758,20 @@ class retroinfer_cache(KV_Cache):
             kernels.wave_attention_part(
                 q, self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx], static_len, ck, cv, row_src,
                 0, stage0, meta, est_ids, logits, self.value_sum[layer_idx], self.cluster_size[layer_idx],
-                self._part_out, self._part_lse, es, self.RSQRT_DIM, valid_lengths=self.valid_lengths[buf])
+                self._part_out, self._part_lse, es, self.RSQRT_DIM, valid_lengths=self.valid_lengths[buf],
+                scratch=self._scratch)
             cur.wait_stream(self.copystream)
             kernels.wave_attention_part(
                 q, self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx], 0, ck, cv, row_src,
                 stage0, rows, meta, None, None, self.value_sum[layer_idx], self.cluster_size[layer_idx], out, None, 0,
-                self.RSQRT_DIM, prev_out=self._part_out, prev_lse=self._part_lse)
+                self.RSQRT_DIM, prev_out=self._part_out, prev_lse=self._part_lse, scratch=self._scratch)
         else:
             if staged_on_copystream:
                 cur.wait_stream(self.copystream)
             kernels.wave_attention(
                 q, self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx], static_len, ck, cv, row_src,
                 meta, est_ids, logits, self.value_sum[layer_idx], self.cluster_size[layer_idx], out,
-                self.valid_lengths[buf], es, self.RSQRT_DIM)
+                self.valid_lengths[buf], es, self.RSQRT_DIM, scratch=self._scratch)
         # admission: staged blocks of the admitted misses into the cache blocks handed out for them
         kernels.gather_copy_and_scatter(
             ck[:, stage0:], self.cache_keys[layer_idx], cv[:, stage0:], self.cache_values[layer_idx],
@@ -824,7 +838,8 @@ class retroinfer_cache(KV_Cache):
                 self.cluster_size[layer_idx], self.es_cluster_size, self._cI[buf], BG, self.n_centroids,
                 self.es_cluster_num, self.max_compute_cluster_num, self.nprobe, self.es_cluster_num)
             es_out, es_lse = kernels.weighted_flash_decoding(q4, self.es_centroids, self.es_value_sum,
-                                                             self.es_cluster_size, return_softmax_lse=True)
+                                                             self.es_cluster_size, return_softmax_lse=True,
+                                                             scratch=self._scratch)
         else:
             es_out = es_lse = None
         if search_here:
@@ -855,11 +870,11 @@ class retroinfer_cache(KV_Cache):
             kernels.buffer_attention(
                 queries.view(BG, gs, D), self.execution_buffer_keys[buf], self.execution_buffer_values[buf],
                 self.valid_lengths[buf], self.est_ids[buf], self.logits, self.value_sum[layer_idx],
-                self.cluster_size[layer_idx], attn, self.es_cluster_num, self.RSQRT_DIM)
+                self.cluster_size[layer_idx], attn, self.es_cluster_num, self.RSQRT_DIM, scratch=self._scratch)
         else:
             attn = kernels.weighted_flash_decoding(
                 q4, self.execution_buffer_keys[buf], self.execution_buffer_values[buf], previous_out=es_out,
-                previous_lse=es_lse, cache_seqlens=self.valid_lengths[buf])
+                previous_lse=es_lse, cache_seqlens=self.valid_lengths[buf], scratch=self._scratch)
         if self.block_cache == "host":
             self.wave_buffer[layer_idx].sync()
         kernels.gather_copy_and_scatter(
@@ -895,7 +910,7 @@ class retroinfer_cache(KV_Cache):
             self.est_ids[buf] if es > 0 else None, self.logits if own else None, self.value_sum[layer_idx],
             self.cluster_size[layer_idx], out, self.valid_lengths[buf], es, self.RSQRT_DIM,
             ret_tok_off=ret_tok_off, ret_start=ret_start,
-            est_centroids=self.centroids[layer_idx] if es > 0 and not own else None)
+            est_centroids=self.centroids[layer_idx] if es > 0 and not own else None, scratch=self._scratch)
         if search_next:
             self._select(queries_next, layer_idx + 1, nbuf, True, layout=nbuf)
         return out.view(self.batch_size, 1, self.num_heads, D)

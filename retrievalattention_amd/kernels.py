@@ -9,6 +9,8 @@ import contextlib
 import ctypes
 import functools
 import math
+import threading
+import weakref
 
 import torch
 
@@ -84,41 +86,66 @@ def _need_all(tensors, dtype, names):
                 _need(x, dtype, nm)
 
 
-_workspaces = {}
-_workspace_generation = 0  # moves on whenever a scratch tensor is replaced: holders of an address look again
-_retired_workspaces = []   # superseded scratch tensors: captured HIP graphs may still hold their addresses
+_scratches = weakref.WeakSet()   # every Scratch there is
+_scratches_lock = threading.Lock()
 
 
-def _workspace(nbytes, device, tag):
-    """Per-(device, tag) scratch tensor, grown on demand and reused across calls.  It starts
-    zeroed: the attention kernels keep arrival counters in it that they leave at zero.
-    A scratch tensor that is outgrown is never freed: a HIP graph captured earlier replays with its
-    address, so handing the block back to the allocator would let that replay write into someone else's
-    memory.  Growing (or first use) during a capture is refused: the allocation would land in the graph's
-    private pool and its zero fill would become a memset node of the graph."""
-    key = (device, tag)
-    w = _workspaces.get(key)
-    if w is None or w.numel() < nbytes:
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError(f"scratch area '{tag}' must grow to {nbytes} bytes during a stream capture: run the "
-                               "same call once before capturing")
-        if w is not None:
-            _retired_workspaces.append(w)
-            nbytes = max(nbytes, w.numel() * 3 // 2)
-        w = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
-        _workspaces[key] = w
-        global _workspace_generation
-        _workspace_generation += 1
-    return w
+class Scratch:
+    """Scratch tensors by device and purpose, grown on demand and reused from call to call.  They start zeroed: the
+    attention kernels keep arrival counters in them that they leave at zero, so calls that may overlap on the device
+    (different streams) must not share one.  A cache has one of its own; calls that name none take the process's.
+    A tensor that is outgrown is kept as long as its owner: a HIP graph captured earlier replays with its address, so
+    handing the block back to the allocator would let that replay write into someone else's memory.  Growing (or first
+    use) during a capture is refused: the allocation would land in the graph's private pool and its zero fill would
+    become a memset node of the graph."""
+
+    def __init__(self):
+        self.areas, self.retired = {}, []
+        self.generation = 0   # moves on whenever a tensor is replaced: holders of an address look again
+        with _scratches_lock:
+            _scratches.add(self)
+
+    def area(self, nbytes, device, tag):
+        key = (device, tag)
+        w = self.areas.get(key)
+        if w is None or w.numel() < nbytes:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError(f"scratch area '{tag}' must grow to {nbytes} bytes during a stream capture: run the "
+                                   "same call once before capturing")
+            if w is not None:
+                self.retired.append(w)
+                nbytes = max(nbytes, w.numel() * 3 // 2)
+            w = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
+            self.areas[key] = w
+            self.generation += 1
+        return w
+
+    def decoding(self, BG, gs, nc, device):
+        """The areas of a decode step of BG groups of gs query heads over nc clusters: of the selection, of the attention."""
+        return (self.area(lib().ri_score_select_workspace_bytes(BG, gs, nc), device, "score0"),
+                self.area(lib().ri_wave_attention_workspace_bytes(BG, gs), device, "attn0"))
+
+
+_shared_scratch = Scratch()
+
+
+def _workspace(nbytes, device, tag, scratch=None):
+    return (_shared_scratch if scratch is None else scratch).area(nbytes, device, tag)
+
+
+def _all_scratch():
+    with _scratches_lock:
+        return list(_scratches)
 
 
 def reset_attention_workspaces():
     """Clears the arrival counters of every attention scratch tensor (on the current stream of its device).
     The attention launches leave them at zero; call this after a launch that did not run to its end."""
-    for (dev, tag), w in _workspaces.items():
-        if tag.startswith("attn"):
-            with torch.cuda.device(w.device):
-                check(lib().ri_attention_workspace_reset(_p(w), w.numel(), _stream()), "attention_workspace_reset")
+    for scratch in _all_scratch():
+        for (dev, tag), w in list(scratch.areas.items()):
+            if tag.startswith("attn"):
+                with torch.cuda.device(w.device):
+                    check(lib().ri_attention_workspace_reset(_p(w), w.numel(), _stream()), "attention_workspace_reset")
 
 
 def release_cached_graphs(retired_workspaces=True):
@@ -133,7 +160,8 @@ def release_cached_graphs(retired_workspaces=True):
     _km._GRAPHS.clear()
     _km._SEEN.clear()
     if retired_workspaces:
-        _retired_workspaces.clear()
+        for scratch in _all_scratch():
+            scratch.retired.clear()
 
 
 # limits of the fused decode path (checked by the entry points; callers can check them up front)
@@ -224,10 +252,11 @@ def _flash_workspace_bytes(BG, gs):
 
 @_ranged("flash_attention")
 def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_lse=None, cache_seqlens=None,
-                            return_softmax_lse=False):
+                            return_softmax_lse=False, scratch=None):
     """Signature of the calls at cache_hub/retroinfer_cache.py:611-617 and :666-674.
     q [BG, 1, gs, D]; k, v [BG, S, 1, D]; weight [BG, 1, 1, S]; previous_out [BG, 1, gs, D];
-    previous_lse [BG, gs] (any shape with BG*gs elements); cache_seqlens [BG] int32."""
+    previous_lse [BG, gs] (any shape with BG*gs elements); cache_seqlens [BG] int32.
+    `scratch`: the caller's own Scratch, where calls may overlap others."""
     BG, one, gs, D = q.shape
     S = k.shape[1]
     if one != 1 or D != 128 or k.shape[2] != 1:
@@ -244,7 +273,7 @@ def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_ls
         _need(cache_seqlens, torch.int32, "cache_seqlens")
     out = torch.empty_like(q)
     lse = torch.empty((BG, gs), dtype=torch.float32, device=q.device) if return_softmax_lse else None
-    ws = _workspace(_flash_workspace_bytes(BG, gs), q.device, "attn")
+    ws = _workspace(_flash_workspace_bytes(BG, gs), q.device, "attn", scratch)
     check(_fn("ri_weighted_flash_decoding", dt)(_p(q), _p(k), _p(v), _p(weight), _p(cache_seqlens), _p(previous_out),
                                            _p(previous_lse), _p(out), _p(lse), BG, gs, S, S,
                                            1.0 / math.sqrt(D), _p(ws), ws.numel(), _stream()),
@@ -345,14 +374,15 @@ class WaveBufferCPU:
 # ----------------------------------------------------------------------------------------
 @_ranged("search_topk_clusters")
 def score_select(q, centroids, mask, cluster_size_i32, cluster_start, logits, dist, cI, ret_ids, est_ids,
-                 ret_tok_off, row_src, meta, nprobe, es, page, max_pages, scale, slot=0, ret_start=None):
+                 ret_tok_off, row_src, meta, nprobe, es, page, max_pages, scale, slot=0, ret_start=None, scratch=None):
     """Centroid scoring + retrieval/estimation selection + token layout.  `slot` names the
-    scratch area: calls that may run concurrently (different streams) must use different slots.
+    scratch area in `scratch` (None: the process's): calls that may run concurrently (different streams) must use
+    different ones.
     The layout goes out as a row table (row_src), as rank tables (ret_tok_off + ret_start), or both."""
     BG, gs, D = q.shape
     nc = centroids.shape[1]
     nb = lib().ri_score_select_workspace_bytes(BG, gs, nc)
-    ws = _workspace(nb, q.device, f"score{slot}")
+    ws = _workspace(nb, q.device, f"score{slot}", scratch)
     _need(centroids, q.dtype, "centroids")
     check(_fn("ri_score_select", q.dtype)(_p(q), _p(centroids), _p(mask), _p(cluster_size_i32), _p(cluster_start),
                                 _p(logits), _p(dist), _p(cI), _p(ret_ids), _p(est_ids), _p(ret_tok_off),
@@ -362,11 +392,11 @@ def score_select(q, centroids, mask, cluster_size_i32, cluster_start, logits, di
           "score_select")
 
 
-def score_logits(q, centroids, logits, scale, slot=0):
+def score_logits(q, centroids, logits, scale, slot=0, scratch=None):
     """logits [BG, gs, nc] fp32 = scale * q . centroids^T, no selection."""
     BG, gs, D = q.shape
     nc = centroids.shape[1]
-    ws = _workspace(lib().ri_score_select_workspace_bytes(BG, gs, nc), q.device, f"score{slot}")
+    ws = _workspace(lib().ri_score_select_workspace_bytes(BG, gs, nc), q.device, f"score{slot}", scratch)
     _need(centroids, q.dtype, "centroids")
     check(_fn("ri_score_logits", q.dtype)(_p(q), _p(centroids), _p(logits), BG, gs, nc, float(scale), _p(ws), ws.numel(),
                                 _stream()), "score_logits")
@@ -375,18 +405,18 @@ def score_logits(q, centroids, logits, scale, slot=0):
 @_ranged("flash_attention")
 def wave_attention(q, steady_k, steady_v, static_len, store_k, store_v, row_src, meta, est_ids, logits,
                    value_sum, cluster_size_bf16, out, valid_lengths, es, scale, slot=0, ret_tok_off=None,
-                   ret_start=None, est_centroids=None, static_len_dev=None):
+                   ret_start=None, est_centroids=None, static_len_dev=None, scratch=None):
     """Attention over steady zone + retrieved clusters (read in place) + estimation zone.
     The retrieved rows come from a row table (row_src) or, with row_src None, from the rank tables
     ret_tok_off [BG, np+1] and ret_start [BG, np].  The estimation zone's scores are read from `logits`
     or, with logits None, computed in the launch from the rows of `est_centroids` [BG, nc, 128].
     With static_len_dev (int32 tensor of one element on the device) the number of steady rows is read
     from it when the kernel runs; static_len then only sizes the split.
-    `slot`: scratch area, one per concurrent call."""
+    `slot`: scratch area in `scratch` (None: the process's), one per concurrent call."""
     BG, gs, D = q.shape
     nc = value_sum.shape[1]
     nb = lib().ri_wave_attention_workspace_bytes(BG, gs)
-    ws = _workspace(nb, q.device, f"attn{slot}")
+    ws = _workspace(nb, q.device, f"attn{slot}", scratch)
     for t, nm in ((steady_k, "steady_k"), (store_k, "store_k"), (value_sum, "value_sum"), (out, "out")):
         _need(t, q.dtype, nm)
     check(_fn("ri_wave_attention", q.dtype)(_p(q), _p(steady_k), _p(steady_v), steady_k.shape[-2], static_len,
@@ -403,19 +433,20 @@ class DecodeStepPlan:
     """score_select + wave_attention of one layer over a device-resident store as one call (ri_decode_step): the
     addresses and sizes, which stay the same from token to token, are checked and laid down once.  `tensors`: the
     fields of ri_decode_step_t that are addresses (None: not given); `key` is what the holder compares to see whether
-    they still are what it would hand over now."""
+    they still are what it would hand over now.  `scratch`: whose areas the step works in (None: the process's).  Every
+    step may use the attention's arrival counters and partials, also of the shortest contexts: steps that may overlap
+    on the device need plans over different Scratch objects."""
 
-    def __init__(self, key, dtype, tensors, nprobe, es, page, max_pages, scale):
+    def __init__(self, key, dtype, tensors, nprobe, es, page, max_pages, scale, scratch=None):
         c = tensors["centroids"]
         BG, nc, _ = c.shape
         gs = tensors["logits"].shape[1]
         for nm in ("centroids", "steady_k", "steady_v", "store_k", "store_v", "value_sum", "cluster_size"):
             _need(tensors[nm], dtype, nm)
-        device = c.device
-        tensors = dict(tensors,
-                       score_workspace=_workspace(lib().ri_score_select_workspace_bytes(BG, gs, nc), device, "score0"),
-                       attn_workspace=_workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), device, "attn0"))
-        self.key, self.generation = key, _workspace_generation
+        self._scratch = _shared_scratch if scratch is None else scratch
+        score, attn = self._scratch.decoding(BG, gs, nc, c.device)
+        tensors = dict(tensors, score_workspace=score, attn_workspace=attn)
+        self.key, self.generation = key, self._scratch.generation
         self._tensors = tensors
         self._step = DecodeStep(
             steady_stride=tensors["steady_k"].shape[-2], store_stride=tensors["store_k"].shape[-2],
@@ -427,7 +458,7 @@ class DecodeStepPlan:
         self._call = lib().ri_decode_step
 
     def valid(self, key):
-        return self.key == key and self.generation == _workspace_generation
+        return self.key == key and self.generation == self._scratch.generation
 
     def run(self, q, static_len, out):
         status = self._call(self._address, q.data_ptr(), static_len, out.data_ptr(), _stream())
@@ -441,11 +472,11 @@ class HostStepPlan(DecodeStepPlan):
     [.., rows, 128] pinned; stage_row0: first staging row of the cache tensors."""
 
     def __init__(self, key, dtype, tensors, nprobe, es, page, max_pages, scale, lru, sizes, starts, lists, row_src, host_k,
-                 host_v, stage_row0):
+                 host_v, stage_row0, scratch=None):
         rows = tensors["store_k"].numel() // (lru.BG * 128)
         tensors = dict(tensors, store_k=tensors["store_k"].view(lru.BG, rows, 128),
                        store_v=tensors["store_v"].view(lru.BG, rows, 128))
-        super().__init__(key, dtype, tensors, nprobe, es, page, max_pages, scale)
+        super().__init__(key, dtype, tensors, nprobe, es, page, max_pages, scale, scratch)
         self._lru = lru.prepared(tensors["ret_ids"], sizes, starts, lists, row_src, stage_row0, tensors["meta"], host_k,
                                  host_v, tensors["store_k"], tensors["store_v"])
         self._lru_address = ctypes.addressof(self._lru)
@@ -469,12 +500,12 @@ def append_kv(key, value, steady_k, steady_v, pos, pos_dev=None):
 @_ranged("flash_attention")
 def wave_attention_part(q, steady_k, steady_v, static_len, store_k, store_v, row_src, src_row_lo, src_row_hi, meta,
                         est_ids, logits, value_sum, cluster_size_bf16, out, lse_out, es, scale, prev_out=None,
-                        prev_lse=None, valid_lengths=None, slot=0):
+                        prev_lse=None, valid_lengths=None, slot=0, scratch=None):
     """wave_attention over the rows of the row table whose source row lies in [src_row_lo, src_row_hi), merging an
     earlier part's (prev_out, prev_lse) and returning this part's log-sum-exp in lse_out [BG, gs] fp32."""
     BG, gs, D = q.shape
     nc = value_sum.shape[1]
-    ws = _workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), q.device, f"attn{slot}")
+    ws = _workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), q.device, f"attn{slot}", scratch)
     check(_fn("ri_wave_attention_part", q.dtype)(
         _p(q), _p(steady_k), _p(steady_v), steady_k.shape[-2], static_len, None, _p(store_k), _p(store_v),
         store_k.shape[-2], _p(row_src), row_src.shape[1], int(src_row_lo), int(src_row_hi), _p(meta), _p(est_ids),
@@ -499,13 +530,13 @@ def wave_attention_static(q, steady_k, steady_v, static_len, store_k, store_v, r
 
 
 def buffer_attention(q, buf_k, buf_v, cache_seqlens, est_ids, logits, value_sum, cluster_size_bf16, out, es, scale,
-                     slot=0):
+                     slot=0, scratch=None):
     """Attention over the rows [0, cache_seqlens[g]) of an execution buffer [BG, stride, 128] with the
     estimation zone (ids and logits from score_select) merged in the same launch."""
     BG, gs, D = q.shape
     nc = value_sum.shape[1]
     stride = buf_k.shape[-3] if buf_k.dim() == 4 else buf_k.shape[-2]
-    ws = _workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), q.device, f"attn{slot}")
+    ws = _workspace(lib().ri_wave_attention_workspace_bytes(BG, gs), q.device, f"attn{slot}", scratch)
     check(_fn("ri_buffer_attention", q.dtype)(_p(q), _p(buf_k), _p(buf_v), stride, _p(cache_seqlens), stride, _p(est_ids),
                                     _p(logits), _p(value_sum), _p(cluster_size_bf16), _p(out), BG, gs, nc, es,
                                     float(scale), _p(ws), ws.numel(), _stream()), "buffer_attention")
