@@ -33,7 +33,7 @@
 #define LRU_DIGIT 256
 #define LRU_COPIES 8        // of the age histogram: a step's clusters share their age
 #define LRU_HELD 4          // clusters per thread whose stamps and blocks stay in registers
-#define LRU_COPIERS 64      // waves that copy missed rows, for blocks of eight rows or more
+#define LRU_COPIERS 64      // workgroups that copy missed rows
 
 enum { LRU_BOTH, LRU_ACCESS, LRU_UPDATE };
 
@@ -425,46 +425,74 @@ __global__ __launch_bounds__(LRU_THREADS) void lru_kernel(ri_lru_t P) {
   lru_group<R, PHASE>(P, blockIdx.x);
 }
 
-// grid groups + copiers: the first workgroups, one per group, update the cache's books; the others copy the missed rows of all
-// groups from the host store into the staging rows, the first wave of each (the rest of its threads leave).  The items, of at
-// most `block` rows, are numbered through all groups and a wave takes every copiers-th: eight rows at a time, 16 lanes per row,
+// grid groups + LRU_COPIERS: the first workgroups, one per group, update the cache's books; the others copy the missed rows of all
+// groups from the host store into the staging rows, with one wave each where the items have eight rows on average, and with up to
+// eight where they have fewer (the rest of a workgroup's threads leave).  The items, of at most `block` rows, are numbered through
+// all groups and dealt out to the waves in turn: eight rows at a time, 16 lanes per row,
 // with both halves requested before either is stored.  What is in flight is what counts: the link wants about 256 KB of it and
 // carries less the more there is (32 groups, 2830 blocks of up to 8 rows, 10.2 MB, GB/s by waves: 48 55.5, 64 55.7, 128 52.1,
 // 256 55.1, 512 54.3, 2048 49.6; a workgroup of sixteen waves to every eight items of a group, as many as there may be, 53.1;
-// plain reads of as much in a row 55.9).
+// plain reads of as much in a row 55.9).  Hence the waves for short items, each of which keeps less in flight: 2880 items of 32
+// groups, us with one wave to a workgroup / as many as taken here: one row 74.3 / 33.6, two rows 76.3 / 58.8, three 85.1 / 84.7, four
+// 109.4 / 109.6 (one; two are 110.3 - 112.9), eight 211.1 / 211.6; 46294 rows of all lengths 420.6 / 421.2.
 template <int R>
-__global__ __launch_bounds__(LRU_THREADS) void lru_stage_kernel(ri_lru_t P, int copiers) {
+__global__ __launch_bounds__(LRU_THREADS) void lru_stage_kernel(ri_lru_t P) {
   if ((int)blockIdx.x < P.BG) {
     lru_group<R, LRU_UPDATE>(P, blockIdx.x);
     return;
   }
-  const int lane = threadIdx.x, vec = lane >> 4, piece = lane & 15;
-  if (lane >= 64) return;
-  int item = blockIdx.x - P.BG, first = 0;   // the item's number; that of the window's first
-  for (int g0 = 0; g0 < P.BG; g0 += 64) {
-    const int own = g0 + lane < P.BG ? P.miss_num[g0 + lane] : 0;
-    const int upto = (int)ri_wave_incl_scan((uint32_t)own), last = first + __builtin_amdgcn_readlane(upto, 63);
-    for (; item < last; item += copiers) {
-      const int in = __popcll(__ballot(upto <= item - first));   // the item's group in the window
-      const int g = g0 + in, j = item - first - __builtin_amdgcn_readlane(upto - own, in);
-      const size_t at = (size_t)g * P.buffer_size + j;
-      const int rows = P.miss_sizes[at];
-      const size_t src = (size_t)g * P.host_stride + P.miss_ids[at];
-      const size_t dst = (size_t)g * P.cache_stride + P.stage_row0 + P.miss_cumsum[at];
-      for (int r = vec; r < rows; r += 8) {
-        const int r2 = min(r + 4, rows - 1);
-        const uint4 k = reinterpret_cast<const uint4*>(P.host_k)[(src + r) * 16 + piece];
-        const uint4 v = reinterpret_cast<const uint4*>(P.host_v)[(src + r) * 16 + piece];
-        const uint4 k2 = reinterpret_cast<const uint4*>(P.host_k)[(src + r2) * 16 + piece];
-        const uint4 v2 = reinterpret_cast<const uint4*>(P.host_v)[(src + r2) * 16 + piece];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), vec = lane >> 4, piece = lane & 15;
+  if (wave >= 8) return;
+  const auto copy = [&](int g, int j) {
+    const size_t at = (size_t)g * P.buffer_size + j;
+    const int rows = P.miss_sizes[at];
+    const size_t src = (size_t)g * P.host_stride + P.miss_ids[at];
+    const size_t dst = (size_t)g * P.cache_stride + P.stage_row0 + P.miss_cumsum[at];
+    for (int r0 = 0; r0 < rows; r0 += 8) {   // (rows that there are not are not read: they would cross the link)
+      const int r = r0 + vec, r2 = r + 4;
+      uint4 k, v, k2, v2;
+      if (r < rows) {
+        k = reinterpret_cast<const uint4*>(P.host_k)[(src + r) * 16 + piece];
+        v = reinterpret_cast<const uint4*>(P.host_v)[(src + r) * 16 + piece];
+      }
+      if (r2 < rows) {
+        k2 = reinterpret_cast<const uint4*>(P.host_k)[(src + r2) * 16 + piece];
+        v2 = reinterpret_cast<const uint4*>(P.host_v)[(src + r2) * 16 + piece];
+      }
+      if (r < rows) {
         reinterpret_cast<uint4*>(P.cache_k)[(dst + r) * 16 + piece] = k;
         reinterpret_cast<uint4*>(P.cache_v)[(dst + r) * 16 + piece] = v;
-        if (r + 4 < rows) {
-          reinterpret_cast<uint4*>(P.cache_k)[(dst + r2) * 16 + piece] = k2;
-          reinterpret_cast<uint4*>(P.cache_v)[(dst + r2) * 16 + piece] = v2;
-        }
+      }
+      if (r2 < rows) {
+        reinterpret_cast<uint4*>(P.cache_k)[(dst + r2) * 16 + piece] = k2;
+        reinterpret_cast<uint4*>(P.cache_v)[(dst + r2) * 16 + piece] = v2;
       }
     }
+  };
+  int item = blockIdx.x - P.BG, step = 0, first = 0;   // the item's number; that of the window's first
+  for (int g0 = 0; g0 < P.BG; g0 += 64) {
+    const int g = g0 + lane, own = g < P.BG ? P.miss_num[g] : 0;
+    const int upto = (int)ri_wave_incl_scan((uint32_t)own), last = first + __builtin_amdgcn_readlane(upto, 63);
+    const auto next = [&]() {
+      const int in = __popcll(__ballot(upto <= item - first));   // the item's group in the window
+      copy(g0 + in, item - first - __builtin_amdgcn_readlane(upto - own, in));
+    };
+    if (g0 == 0) {
+      // How many waves, by the first window's rows, while the first wave's first item is on its way: that is its own in any case.
+      int rows = 0;
+      if (own > 0) {
+        const size_t end = (size_t)g * P.buffer_size + own - 1;
+        rows = P.miss_cumsum[end] + P.miss_sizes[end];
+      }
+      const bool begun = wave == 0 && item < last;
+      if (begun) next();
+      rows = __builtin_amdgcn_readlane((int)ri_wave_incl_scan((uint32_t)rows), 63);
+      const int waves = rows < 4 * last ? min((8 * last + rows - 1) / max(rows, 1), 8) : 1;
+      if (wave >= waves) return;
+      step = LRU_COPIERS * waves;
+      item += begun ? step : LRU_COPIERS * wave;
+    }
+    for (; item < last; item += step) next();
     first = last;
   }
 }
@@ -530,10 +558,9 @@ extern "C" int ri_lru_stage_update(const ri_lru_t* s, ri_stream_t stream) {
       s->cache_stride < (int64_t)s->stage_row0 + (int64_t)s->buffer_size * s->block)
     return RI_ERR_ARG;
   if (ri_any_misaligned16(s->host_k, s->host_v, s->cache_k, s->cache_v)) return RI_ERR_ARG;
-  const int copiers = LRU_COPIERS * 8 / min(s->block, 8);   // (a wave's share of what is in flight shrinks with its rows)
-  const dim3 grid(s->BG + copiers);
-  if (s->np < LRU_THREADS) lru_stage_kernel<1><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s, copiers);
-  else lru_stage_kernel<4><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s, copiers);
+  const dim3 grid(s->BG + LRU_COPIERS);
+  if (s->np < LRU_THREADS) lru_stage_kernel<1><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
+  else lru_stage_kernel<4><<<grid, LRU_THREADS, 0, (hipStream_t)stream>>>(*s);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

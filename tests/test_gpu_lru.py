@@ -212,7 +212,7 @@ def test_access_and_stage_update_equal_the_one_launch(dev, ncl, nprobe, capacity
 
 
 @pytest.mark.parametrize("BG,block", [(1, 8), (3, 1), (63, 3), (65, 8), (130, 16)])
-def test_missed_rows_are_staged_in_rank_order(dev, BG, block):
+def test_missed_rows_are_staged_in_rank_order(dev, BG, block, most=39):
     """Items numbered through all groups, sixty-four groups at a time: groups without misses, partial blocks, blocks shorter and
     longer than the eight rows a wave copies at a time; nothing is written behind the rows."""
     import ctypes
@@ -220,11 +220,11 @@ def test_missed_rows_are_staged_in_rank_order(dev, BG, block):
     from retrievalattention_amd._lib import lib
     g = torch.Generator().manual_seed(BG)
     ncl, nprobe = 24, 7
-    sz = torch.randint(0, 40, (BG, ncl), generator=g, dtype=torch.int32)
+    sz = torch.randint(0, most + 1, (BG, ncl), generator=g, dtype=torch.int32)
     sz[1::5] = 0
     st = (torch.cumsum(sz.long(), 1) - sz.long()).to(torch.int32)
     n = max(1, int(sz.sum(1).max()))
-    buffer_size = nprobe * ((39 + block - 1) // block)
+    buffer_size = nprobe * ((most + block - 1) // block)
     host = [torch.randn(BG, n, 128, generator=g).to(torch.bfloat16).pin_memory() for _ in range(2)]
     cache = [torch.zeros(BG, buffer_size * block + 1, 128, dtype=torch.bfloat16, device=dev) for _ in range(2)]
     lru = kernels.DeviceLru(BG, ncl, int(((sz + block - 1) // block).sum(1).max()) + 1, 0, buffer_size, block, dev)
@@ -242,3 +242,10 @@ def test_missed_rows_are_staged_in_rank_order(dev, BG, block):
             rows = torch.cat([torch.arange(st[b, i], st[b, i] + sz[b, i]) for i in ids[b].tolist()])
             want[b, :len(rows)] = h[b, rows]
         assert torch.equal(c.cpu(), want)
+
+
+@pytest.mark.parametrize("BG,block,most", [(1, 8, 1), (40, 8, 1), (40, 8, 2), (64, 8, 3), (70, 8, 5), (40, 2, 7), (200, 8, 1),
+                                           (33, 8, 8)])
+def test_short_blocks_are_staged_in_rank_order(dev, BG, block, most):
+    """Blocks of few rows, which more waves than one of a workgroup copy: from eight down to two of them."""
+    test_missed_rows_are_staged_in_rank_order(dev, BG, block, most)
