@@ -56,13 +56,18 @@ static inline bool step_is_joined(const ri_decode_step_t* s) {
 // several).  8 groups of 8 heads 225 rows 13.4 / 14.2, 321: 14.1 / 14.2, 353: 14.5 / 14.2, 417: 15.1 / 14.2; of 4 heads 225: 12.7
 // / 13.5, 321: 13.4 / 13.5, 353: 13.7 / 13.5, with 512 clusters 331: 13.9 / 13.8 (a step, 15.2 either way), 523: 16.0 / 13.8; of 1 head 321: 13.0 / 13.1; 32
 // groups of 4 heads 321: 14.2 / 14.2, 417: 15.3 / 14.6.  With two workgroups per group only: 128 groups of 4 heads 417: 16.4 / 17.7,
-// of 8 heads, 512 clusters 587: 21.0 / 21.1; past 128 there is no second one.  A captured step, which starts at the length at hand
-// and ends at the zone's, may grow by a quarter past the line.  (Several workgroups that find fewer rows than the line leave them
-// to one: step_kernel.)
+// of 8 heads, 512 clusters 587: 21.0 / 21.1; past 128 there is no second one.  (Several workgroups that find fewer rows than
+// the line leave them to one: step_kernel.)
+// A captured step starts at the length at hand and ends at the zone's, and may grow past the line.  One wins at first, several
+// later; from sixteen groups on every workgroup more shows in the start of the launch.  Zones of 323 rows, us a layer at the
+// first length, on average and at the last, several | one: 16 groups of 4 heads, up to 508 rows 15.2, 17.0, 18.2 | 15.2, 16.8,
+// 18.4; 32 of 4, 508 16.4, 17.6, 18.3 | 16.0, 17.5, 18.9; 64 of 4, 477 15.9, 17.2, 18.2 | 15.6, 17.1, 18.5; 32 of 8, 446 16.2,
+// 17.7, 18.4 | 16.0, 17.5, 19.0; 40 of 2, 477 15.3, 16.5, 17.4 | 15.2, 16.7, 18.5.  Past the line 24 of 4, 531 16.6, 17.4, 18.1 |
+// 16.2, 17.7, 19.1; 64 of 4, 554 17.1, 18.2, 18.7 | 16.5, 18.3, 19.9; 8 of 4, 477 14.1, 15.3, 16.3 | 14.2, 15.5, 17.1.
 static inline int step_alone_rows(int BG) { return BG > 64 ? 640 : 336; }
+static inline int step_alone_end(int BG) { return BG > 64 ? 800 : BG >= 16 ? 512 : 420; }
 static inline bool step_is_alone(const ri_decode_step_t* s, int static_len) {
   if (s->BG > 128) return true;
   const int64_t usual = (int64_t)s->np * 16 + s->es, zone = s->static_len_dev ? s->steady_stride : static_len;
-  const int64_t line = step_alone_rows(s->BG);
-  return static_len + usual <= line && zone + usual <= line * 5 / 4;
+  return static_len + usual <= step_alone_rows(s->BG) && zone + usual <= step_alone_end(s->BG);
 }

@@ -11,17 +11,16 @@ from retrievalattention_amd._lib import DecodeStep
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.fixture(scope="module")
-def is_short(tmp_path_factory):
+def _route(tmp_path_factory, name):
     if shutil.which("g++") is None:
         pytest.skip("no g++")
     where = tmp_path_factory.mktemp("route")
-    (where / "route.cpp").write_text('#include "step_route.h"\nextern "C" int is_short(const ri_decode_step_t* s, int n) '
-                                     '{ return step_is_short(s, n); }\n')
+    (where / "route.cpp").write_text('#include "step_route.h"\nextern "C" int ask(const ri_decode_step_t* s, int n) '
+                                     f'{{ return step_{name}(s, n); }}\n')
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "retrievalattention_amd", "csrc"), str(where / "route.cpp"), "-o",
                     str(where / "route.so")], check=True)
-    call = ctypes.CDLL(str(where / "route.so")).is_short
+    call = ctypes.CDLL(str(where / "route.so")).ask
 
     def short(static_len, zone=323, on_device=False, BG=8, gs=4, nc=512, np=9, es=118, page=8, max_pages=72, store=8192,
               sizes=True):
@@ -30,6 +29,16 @@ def is_short(tmp_path_factory):
                           cluster_size_i32=1 if sizes else None, cluster_start=1 if sizes else None)
         return bool(call(ctypes.byref(step), static_len))
     return short
+
+
+@pytest.fixture(scope="module")
+def is_short(tmp_path_factory):
+    return _route(tmp_path_factory, "is_short")
+
+
+@pytest.fixture(scope="module")
+def is_alone(tmp_path_factory):
+    return _route(tmp_path_factory, "is_alone")
 
 
 def test_limits(is_short):
@@ -61,3 +70,13 @@ def test_clusters_may_hold_what_the_page_limit_lets_them(is_short, gs):
     assert is_short(at, gs=gs, max_pages=1 << 30, store=608) and not is_short(at, gs=gs, max_pages=1 << 30, store=609)
     assert is_short(at, gs=gs, max_pages=1 << 30, BG=129)
     assert is_short(98, gs=gs, max_pages=1 << 30) == (gs == 4)
+
+
+def test_captured_steps_of_many_groups_keep_one_workgroup_for_longer(is_alone):
+    """Which short steps one workgroup per group makes: by the rows at hand, and captured ones by the zone's too."""
+    for BG, line, end in ((1, 336, 420), (15, 336, 420), (16, 336, 512), (64, 336, 512), (65, 640, 800), (128, 640, 800)):
+        assert is_alone(line - 90, BG=BG, np=4, es=26) and not is_alone(line - 89, BG=BG, np=4, es=26)
+        assert is_alone(69, zone=end - 90, on_device=True, BG=BG, np=4, es=26)
+        assert not is_alone(69, zone=end - 89, on_device=True, BG=BG, np=4, es=26)
+        assert not is_alone(line - 89, zone=end - 90, on_device=True, BG=BG, np=4, es=26)
+    assert is_alone(5000, BG=129)
