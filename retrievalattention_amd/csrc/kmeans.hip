@@ -61,6 +61,7 @@ __device__ __forceinline__ float km_max3(float a, float b, float c) {
 }
 
 typedef uint32_t km_pair __attribute__((ext_vector_type(2)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // o[u] (+)= a b[u]: sixteen rows with twice sixteen tokens, 32 dims.  Written out so that the sums stay where they are: left to
 // the compiler every product gets another register for its sum, 64 more than there are.  Hazards are its own: two slots from a
 // register move to a product that reads it (in the shadow of the product before), and, behind the last one, km_products_wait.
@@ -490,6 +491,153 @@ __global__ __launch_bounds__(W * 64) void km_assign_kernel(const uint16_t* __res
     const int tok = t0 + tt * 32 + s.r;
     if (s.hh == 0 && tok < N) assign[(size_t)p * N + tok] = place;
   }
+}
+
+// base + the row, past the lane's first one in a sub-tile, of the first of a lane's sixteen scores that equals m, found as
+// km_first_of finds one of eight.  low8 and low4 are the maxima of best and the first eight and four scores, high4 of best and
+// scores 8 .. 11.
+__device__ __forceinline__ int km_first_of16(const f32x16_t& x, float m, float best, float low8, float low4, float high4,
+                                             int base) {
+  float y0, y1, y2, y3, y4, y5, y6, y7, t;
+  uint64_t e, e8;
+  int row;
+  asm volatile(
+      "v_cmp_eq_f32_e64 %8, %25, %26\n\t"
+      "s_nop 1\n\t"
+      "v_cndmask_b32_e64 %0, %17, %9, %8\n\t"
+      "v_cndmask_b32_e64 %1, %18, %10, %8\n\t"
+      "v_cndmask_b32_e64 %2, %19, %11, %8\n\t"
+      "v_cndmask_b32_e64 %3, %20, %12, %8\n\t"
+      "v_cndmask_b32_e64 %4, %21, %13, %8\n\t"
+      "v_cndmask_b32_e64 %5, %22, %14, %8\n\t"
+      "v_cndmask_b32_e64 %6, %23, %15, %8\n\t"
+      "v_cndmask_b32_e64 %7, %24, %16, %8"
+      : "=&v"(y0), "=&v"(y1), "=&v"(y2), "=&v"(y3), "=&v"(y4), "=&v"(y5), "=&v"(y6), "=&v"(y7), "=&s"(e8)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]), "v"(x[9]),
+        "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "v"(low8), "v"(m));
+  // (sum i is row (i / 4) * 8 + i % 4)
+  asm volatile(
+      "v_cndmask_b32_e64 %8, %13, %12, %10\n\t"
+      "v_cmp_eq_f32_e64 %11, %8, %15\n\t"
+      "v_cndmask_b32_e64 %9, 16, 0, %10\n\t"
+      "s_nop 0\n\t"
+      "v_cndmask_b32_e64 %0, %4, %0, %11\n\t"
+      "v_cndmask_b32_e64 %1, %5, %1, %11\n\t"
+      "v_cndmask_b32_e64 %2, %6, %2, %11\n\t"
+      "v_cndmask_b32_e64 %3, %7, %3, %11\n\t"
+      "v_max3_f32 %8, %14, %0, %1\n\t"
+      "v_cmp_eq_f32_e64 %10, %8, %15\n\t"
+      "v_cndmask_b32_e64 %4, 8, 0, %11\n\t"
+      "s_nop 0\n\t"
+      "v_cndmask_b32_e64 %0, %2, %0, %10\n\t"
+      "v_cmp_eq_f32_e64 %11, %0, %15\n\t"
+      "v_cndmask_b32_e64 %5, 2, 0, %10\n\t"
+      "v_add3_u32 %9, %9, %4, %5\n\t"
+      "v_cndmask_b32_e64 %6, 1, 0, %11\n\t"
+      "v_add3_u32 %9, %9, %6, %16"
+      : "+v"(y0), "+v"(y1), "+v"(y2), "+v"(y3), "+v"(y4), "+v"(y5), "+v"(y6), "+v"(y7), "=&v"(t), "=&v"(row), "+s"(e8),
+        "=&s"(e)
+      : "v"(low4), "v"(high4), "v"(best), "v"(m), "v"(base));
+  return row;
+}
+
+// The same pass for launches that leave many compute units without work: there power bounds nothing, and half as many products,
+// each of 32 rows with 32 tokens, and one search of sixteen scores are fewer instructions than two of each with eight.  (Figures
+// at km_assign_launch.)  Eight waves of 32 tokens, tiles of 128 rows in two buffers; a lane has token r, dims 16 kk + 8 hh.
+template <bool HALF>
+__global__ __launch_bounds__(512) void km_assign_few_kernel(const uint16_t* __restrict__ data, const uint16_t* __restrict__ cent,
+                                                            int32_t* __restrict__ assign, int N, int nc, int seg,
+                                                            int64_t head_rows, int sh) {
+  constexpr int CT = 128, AHEAD = 8;
+  typedef KmScan<1, CT, 8, 2, HALF, false> Scan;
+  static_assert(Scan::TURN && Scan::WR == 16, "room for sixteen tokens of a wave");
+  __shared__ __attribute__((aligned(1024))) uint16_t sh_c[2][CT][RI_DIM];
+  const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
+  Scan s(sh_c, cent + (size_t)p * nc * RI_DIM, nc);
+  const int t0 = (blockIdx.x >> sh) * Scan::TOKENS + s.wave * 32, r = s.r, hh = s.hh;
+  const uint16_t* dp = data + km_row0(p, seg, head_rows, N) * RI_DIM;
+  uint4 in[8], b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) in[i] = ri_ld16(dp + (size_t)min(t0 + 4 * i + s.g, N - 1) * RI_DIM + s.c * 8);
+  s.start(0, nc);
+  uint4* const turn = reinterpret_cast<uint4*>(&sh_c[1][s.wave * Scan::WR][0]);
+  km_wait_vm<Scan::L>();
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + s.g;
+      turn[row * 16 + (s.c ^ row)] = in[w * 4 + i];
+    }
+    ri_wave_sync();
+    if (r >> 4 == w) {
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) b[kk] = turn[s.c * 16 + ((kk * 2 + hh) ^ s.c)];
+    }
+    ri_wave_sync();   // (a wave's LDS accesses happen in order)
+  }
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(b[kk].x), "+v"(b[kk].y), "+v"(b[kk].z), "+v"(b[kk].w));
+  float best = -INFINITY;
+  int at = 0;
+  const uint16_t* row_at[8];   // this lane's pieces of its row of a sub-tile
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) row_at[kk] = &sh_c[0][r][((kk * 2 + hh) ^ s.c) * 8];
+  for (int ct0 = 0; ct0 < nc; ct0 += 2 * CT) {
+#pragma unroll
+    for (int buf = 0; buf < 2; ++buf) {   // (unrolled: the buffer is in the offset of every LDS read)
+      const int ct = ct0 + buf * CT;
+      if (ct >= nc) break;
+      km_wait_vm<0>();   // this tile's loads of this wave have landed ...
+      asm volatile("s_barrier" ::: "memory");   // ... and every wave's; and every wave is done with the tile before
+      s.tile_load(ct + CT, 1 - buf);
+      uint4 rows[AHEAD];
+      const auto operand = [&](int k) {
+        return *reinterpret_cast<const uint4*>(row_at[k % 8] + (buf * CT + k / 8 * 32) * RI_DIM);
+      };
+#pragma unroll
+      for (int kk = 0; kk < AHEAD; ++kk) rows[kk] = operand(kk);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int half = 0; half < CT / 32; ++half) {
+        if (ct + half * 32 < nc) {  // uniform: only the last tile can lack sub-tiles
+          f32x16_t acc;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+          for (int kk = 0; kk < 8; ++kk) {
+            const int k = half * 8 + kk;
+            const uint4 a = rows[k % AHEAD];
+            acc = HALF ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
+                                                                __builtin_bit_cast(f16x8_t, b[kk]), acc, 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ri_as_bf16x8(a), ri_as_bf16x8(b[kk]), acc, 0, 0, 0);
+            if (k + AHEAD < CT / 4) rows[k % AHEAD] = operand(k + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          float low8 = best, high8 = best, low4 = best, high4 = best;   // (from the best so far, which is no NaN)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            low8 = fmaxf(low8, acc[i]);
+            high8 = fmaxf(high8, acc[8 + i]);
+            if (i == 3) low4 = low8, high4 = high8;
+          }
+          const float m = km_max(low8, high8);
+          const bool upd = m > best;
+          if (__builtin_amdgcn_ballot_w64(upd) != 0ull) {
+            const int k = km_first_of16(acc, m, best, low8, low4, high4, hh * 4 + ct + half * 32);
+            at = upd ? k : at;
+            best = m;
+          }
+        }
+      }
+    }
+  }
+  km_wait_vm<0>();   // (no load may land in LDS that is no longer this workgroup's)
+  const float other = km_other(best, hh);
+  const int other_at = __float_as_int(km_other(__int_as_float(at), hh));
+  if (other > best || (other == best && other_at < at)) at = other_at;
+  const int tok = t0 + r;
+  if (hh == 0 && tok < N) assign[(size_t)p * N + tok] = at;
 }
 
 // A pass of a clustering that knows the pass before (KmBounds), grid (ceil(N / TOKENS), P).  The clusters that no token has
@@ -1759,9 +1907,18 @@ static void km_assign_launch(const void* data, const void* centroids, int32_t* a
   // 14.3 / 17.1, 420 15.3 / 17.1 / 14.6 / 17.1, 576 22.0 / 21.7 / 23.7 / 24.8, 768 27.1 / 26.6 / 26.0 / 26.8, 896 30.0 / 29.3 /
   // 31.0 / 31.4, 1024 34.3 / 33.3 / 32.8 / 34.5, 1100 36.1 / 35.1 / 37.8 / 37.8, 1400 43.7 / 43.6 / 44.9 / 43.0, 3000 89.7 / 85.6 /
   // 87.0 / 82.2; 4096 centroids: 128 40.9 / 45.5 / 47.6 / 71.3, 640 137.8 / 136.3 / 141.6 / 145.7, 1024 209.7 / 210.7 / 196.6 /
-  // 196.0; 128 centroids, 1024 15.5 / 16.0 / 19.0 / 17.5.  (270 shapes of eight problems.)
+  // 196.0; 128 centroids, 1024 15.5 / 16.0 / 19.0 / 17.5.  (270 shapes of eight problems.)  Around the lines, on another card:
+  // 136 8.9 / 10.1 / 8.5 / 13.2, 160 9.1 / 10.0 / 8.4 / 13.1, 192 9.1 / 10.1 / 8.5 / 13.1, 224 9.3 / 10.1 / 8.7 / 13.1; 1200 39.4 /
+  // 38.1 / 37.6 / 38.9, 1280 40.3 / 39.0 / 38.1 / 40.0, 1344 42.7 / 41.4 / 43.1 / 43.8; 128 centroids, 1200 16.4 / 16.8 / 17.6 / 18.2.
+  // One round that leaves compute units without work: products of 32 rows (km_assign_few_kernel / <1, 128, 8, 2>), the further
+  // the longer the loop: 256 centroids, 136 pieces 5.63 / 5.72, 216 5.77 / 5.82; 512, 136 8.13 / 8.48, 176 8.12 / 8.45, 216 8.29 /
+  // 8.49, 256 8.71 / 8.68; 1024, 136 13.3 / 13.9, 192 13.8 / 14.2, 208 13.9 / 14.2, 232 14.8 / 14.7; 2048, 136 24.4 / 24.9, 192 24.9 /
+  // 24.9, 216 26.0 / 25.3; 4096, 136 45.4 / 45.7, 192 46.6 / 46.3; 128, 136 4.46 / 4.45.
   const long long pieces = (long long)P * ((N + 255) / 256);
-  if (pieces > 1152) KM_ASSIGN_LAUNCH(2, 32, 4, 4);
+  if (pieces > 128 && nc >= 256 && pieces + nc / 64 <= 224)
+    km_assign_few_kernel<HALF><<<km_grid((N + 255) / 256, P), 512, 0, stream>>>(
+        (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P));
+  else if (pieces > 1280) KM_ASSIGN_LAUNCH(2, 32, 4, 4);
   else if ((pieces - 1) % 256 >= 128 && (nc >= 256 || pieces <= 768)) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
   else if (pieces <= 384) KM_ASSIGN_LAUNCH(1, 64, 4, 2);
   else KM_ASSIGN_LAUNCH(1, 32, 4, 3);

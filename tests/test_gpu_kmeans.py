@@ -133,6 +133,18 @@ def test_assign_at_the_lines_between_tilings(dev, pieces, nc, dt):
     test_assign_ties_go_to_the_lowest_id(dev, 1, pieces * 256 - 3, nc, dt)
 
 
+# Launches with a piece for 129 to about 200 compute units, by pieces and centroids, and the lines of the longest ones.
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("pieces,nc", [(129, 224), (129, 256), (220, 256), (221, 256), (129, 288), (208, 1024), (209, 1024),
+                                       (192, 2048), (193, 2048), (130, 6016), (130, 6048), (1280, 96), (1281, 96), (1280, 288),
+                                       (1281, 288)])
+def test_assign_with_work_for_half_the_units(dev, pieces, nc, dt):
+    test_assign_tilings(dev, 1, pieces * 256 - 3, nc, dt)
+    test_assign_ties_go_to_the_lowest_id(dev, 1, pieces * 256 - 3, nc, dt)
+    if pieces < 256:
+        test_assign_finds_every_row(dev, 2, (pieces + 1) // 2 * 256 - 255, nc, dt)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("P,N,nc", [(5, 1001, 32), (8, 8193, 544), (16, 8200, 544), (20, 9757, 608), (33, 8200, 512),
                                     (2, 32768, 2048)])
