@@ -2144,8 +2144,14 @@ extern "C" int ri_kmeans_update_direct_f16(const void* data, const int32_t* assi
 // 1376: 1847 / 1648 | 1742 / 1807; 1 x 131072, 8192: 2325 / 1782 | 2135 / 1465; 8 x 131072, 8192: 14806 / 9586 | 14456 /
 // 7570.  So from 2^29 scores a pass on.  (Up to 16384 tokens the lists never leave a workgroup, and a pass is
 // bound by its keys.  64 problems: a lane each where the open tokens are dealt out; 16384 centroids: their order in LDS.)
+// The more tokens a cluster has, the fewer clusters no token joins or leaves, the later; without structure none.  Without /
+// with, by tokens to a centroid: 8 x 131072, 48: 5803 / 4703 | 5481 / 5407, 56: 5084 / 4266 | 4862 / 5110, 64: 4616 / 3960 | 4393 /
+// 4868, 95: 3510 / 3309 | 3308 / 3972, 128: 3012 / 3007 | 2720 / 3352; 4 x 131072, 48: 3150 / 2673 | 2879 / 2922, 64: 2571 / 2323 |
+// 2335 / 2635, 128: 1664 / 1731 | 1512 / 1880; 8 x 65536, 47: 1904 / 1741 | 1782 / 1875, 64: 1624 / 1579 | 1496 / 1744; 1 x 262144,
+// 47: 3175 / 2731 | 2883 / 3114, 64: 2747 / 2508 | 2245 / 2697, 128: 1552 / 1615 | 1386 / 1808.  Up to 50 keys with structure
+// gain more than others lose, and those lose little; past it they lose up to 30 %.
 static bool km_bounded(int P, int N, int nc) {
-  return N > KM_DIRECT_MAX && P <= 64 && nc <= 16384 && (int64_t)P * N * nc >= 1ll << 29;
+  return N > KM_DIRECT_MAX && N <= 50ll * nc && P <= 64 && nc <= 16384 && (int64_t)P * N * nc >= 1ll << 29;
 }
 
 __global__ __launch_bounds__(KM_OPEN_WGS + 64) void km_clear_kernel(int32_t* p, int n) {

@@ -39,6 +39,17 @@ def test_status_strings_and_version():
     assert l.ri_flash_decoding_workspace_bytes(0, 4) == 0
 
 
+def test_passes_know_each_other_where_clusters_are_small():
+    """What the passes of a clustering keep of each token (at least twelve bytes) is only asked for up to fifty tokens to a
+    centroid, from 2^29 scores a pass on."""
+    from retrievalattention_amd import _lib
+    l = _lib.lib()
+    P, nc = 8, 2048
+    bytes_ = lambda n, c=nc: l.ri_kmeans_iterate_workspace_bytes(P, n, c)  # noqa: E731
+    assert bytes_(50 * nc) - bytes_(50 * nc + 1) > 12 * P * 50 * nc - (1 << 20)
+    assert bytes_(2 * 16384, nc) > bytes_(2 * 16384, nc - 32) + 12 * P * 2 * 16384
+
+
 def test_missing_library_is_a_loud_error(monkeypatch, tmp_path):
     from retrievalattention_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)

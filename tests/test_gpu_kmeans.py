@@ -483,6 +483,11 @@ def test_iterate_equals_its_passes(dev, G, N, nc, seg, kind, dt):
         assert torch.equal(mine.view(torch.int16), cent.view(torch.int16))
 
 
+@pytest.mark.parametrize("G,N,nc,seg", [(3, 102400, 2048, 1), (3, 102401, 2048, 1)])
+def test_iterate_on_both_sides_of_fifty_tokens_a_centroid(dev, G, N, nc, seg):
+    test_iterate_equals_its_passes(dev, G, N, nc, seg, "mixture", torch.bfloat16)
+
+
 def test_iterate_refuses(dev):
     from retrievalattention_amd import _lib
     lib = _lib.lib()
