@@ -438,7 +438,7 @@ struct KmScan {
               }
           }
         }
-        if (((ct + CT) & 511) == 0 && ct + CT < end) share(track);
+        if (((ct + CT - from) & 511) == 0 && ct + CT < end) share(track);   // (a second turn starts anywhere in the list)
       }
     }
 #pragma unroll
