@@ -54,11 +54,6 @@ __device__ __forceinline__ float km_max(float a, float b) {
   asm("v_max_f32_e32 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
   return m;
 }
-__device__ __forceinline__ float km_max3(float a, float b, float c) {
-  float m;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
-  return m;
-}
 
 typedef uint32_t km_pair __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));

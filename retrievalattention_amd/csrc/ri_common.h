@@ -233,13 +233,13 @@ static inline ri_ptr4 ri_pack_ptrs(const void* a, const void* b, const void* c, 
 }
 
 // ---- shared between score.hip and select.hip ----
-#define RI_SCORE_TILE 256          // centroids per softmax partial
-#define RI_SCORE_TILE_FEW 64       // where that is few workgroups
-// tile: centroids per workgroup and softmax partial, RI_SCORE_TILE or RI_SCORE_TILE_FEW
+#define RI_SCORE_TILE 256          // centroids per scoring workgroup and softmax partial
+#define RI_SCORE_TILE_FEW 64       // where that is few workgroups (score_tile in select.hip)
+// tile: RI_SCORE_TILE or RI_SCORE_TILE_FEW
 int ri_launch_score(const void* q, const void* centroids, float* logits, float* tile_max, float* tile_sum,
                     int BG, int gs, int nc, int tile, float scale, bool half, hipStream_t s);
 
-// Row statistics from the per-256-column partials [ntiles, gs]: one wave per row, lanes over
+// Row statistics from the partials of a row's tiles [ntiles, gs]: one wave per row, lanes over
 // tiles, xor-butterfly reductions (fixed order, so the result is reproducible).
 __device__ __forceinline__ void ri_wave_reduce_partials(const float* pm, const float* ps, int ntiles, int gs,
                                                         int j, int lane, float* m_out, float* invz_out) {

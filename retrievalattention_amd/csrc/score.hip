@@ -1,14 +1,14 @@
 // Centroid scoring and cluster selection for the decode step (gfx950).
 //
 // score_kernel    : logits[g,j,c] = scale * <q[g,j,:], centroid[g,c,:]> on bf16 MFMA, streamed
-//                   once over the centroids, plus per-256-column softmax partials.
-// reduce/apply    : the two small kernels that complete the batch_gemm_softmax interface.
+//                   once over the centroids, plus softmax partials per 256 or 64 columns.
+// softmax_kernel  : the rest of the batch_gemm_softmax interface.
 //
 // Follows cache_hub/retroinfer_cache.py:569-575 and
 // library/retroinfer/retroinfer_kernels/src/batch_gemm_softmax.h:222-243 (rounding pipeline).
 #include "ri_common.h"
 
-#define SCORE_TILE RI_SCORE_TILE  // centroids per workgroup == width of one softmax partial
+#define SCORE_TILE RI_SCORE_TILE  // columns of one softmax partial of the batch_gemm_softmax interface
 
 // ------------------------------------------------------------------------------------
 // score_kernel: grid (ntiles, BG), 256 threads = 4 waves, each wave owns 64 or 16 centroids.

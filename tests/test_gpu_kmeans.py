@@ -115,10 +115,10 @@ def test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt):
         assert torch.equal(assign[p].long(), first)
 
 
-# Four columns of tokens per wave (more than 2048 centroids), and the line between one and three columns, on either side.
+# Loops over more than two thousand centroids, and launches a little past two and three rounds of workgroups.
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("P,N,nc", [(3, 66001, 2080), (8, 17001, 544), (8, 18001, 544), (24, 8001, 1056)])
-def test_assign_long_loops_and_three_columns(dev, P, N, nc, dt):
+def test_assign_long_loops_and_short_last_rounds(dev, P, N, nc, dt):
     test_assign_tilings(dev, P, N, nc, dt)
     test_assign_ties_go_to_the_lowest_id(dev, P, N, nc, dt)
 
