@@ -291,9 +291,11 @@ class retroinfer_cache(KV_Cache):
 
     def _allocate_scratch(self):
         """The cache's own scratch areas, before anything captures a step: decode steps of other caches, on other
-        streams, count arrivals and leave partials in theirs."""
+        streams, count arrivals and leave partials in theirs.  The process's areas grow with them: the operators can be
+        captured by themselves wherever a cache of their shape has been set up."""
         for device in {c.device for c in self.centroids}:
-            self._scratch.decoding(self.batch_groups, self.group_size, self.n_centroids, device)
+            for scratch in (self._scratch, kernels.shared_scratch):
+                scratch.decoding(self.batch_groups, self.group_size, self.n_centroids, device)
 
     def pre_allocate_decision(self):
         """Kept for callers of the reference API; this build always pre-allocates."""

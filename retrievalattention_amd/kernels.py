@@ -126,11 +126,11 @@ class Scratch:
                 self.area(lib().ri_wave_attention_workspace_bytes(BG, gs), device, "attn0"))
 
 
-_shared_scratch = Scratch()
+shared_scratch = Scratch()   # the process's
 
 
 def _workspace(nbytes, device, tag, scratch=None):
-    return (_shared_scratch if scratch is None else scratch).area(nbytes, device, tag)
+    return (shared_scratch if scratch is None else scratch).area(nbytes, device, tag)
 
 
 def _all_scratch():
@@ -443,7 +443,7 @@ class DecodeStepPlan:
         gs = tensors["logits"].shape[1]
         for nm in ("centroids", "steady_k", "steady_v", "store_k", "store_v", "value_sum", "cluster_size"):
             _need(tensors[nm], dtype, nm)
-        self._scratch = _shared_scratch if scratch is None else scratch
+        self._scratch = shared_scratch if scratch is None else scratch
         score, attn = self._scratch.decoding(BG, gs, nc, c.device)
         tensors = dict(tensors, score_workspace=score, attn_workspace=attn)
         self.key, self.generation = key, self._scratch.generation

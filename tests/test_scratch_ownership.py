@@ -48,7 +48,9 @@ def test_caches_have_scratch_of_their_own(no_gpu):
 def test_nothing_of_a_step_is_allocated_during_its_capture(no_gpu, monkeypatch):
     c = _host_cache()
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
-    c._plan(0, 0)
+    areas = _areas(c._plan(0, 0))
+    for tag, mine in zip(("score0", "attn0"), areas):   # nor of the same operators by themselves
+        assert kernels._workspace(mine.numel(), torch.device("cpu"), tag).data_ptr() != mine.data_ptr()
     with pytest.raises(RuntimeError, match="during a stream capture"):
         c._scratch.area(1 << 30, torch.device("cpu"), "attn0")
 
