@@ -25,36 +25,62 @@ HBM_PEAK = 8.0e12  # bytes/s, MI355X
 # the default of the reference's harnesses (simple_test.py:29, throughput_eval/test.py:28)
 DT, DT_NAME = torch.bfloat16, "bf16"
 
-# HBM bytes per attend_kernel launch come from rocprofv3 counter runs of this script (FETCH_SIZE and
+# HBM bytes per launch come from rocprofv3 counter runs of this script (FETCH_SIZE and
 # WRITE_SIZE, each scaled by what the counter reads for the known-size copy of --copy-probe): the figures
-# sit in a small data file next to the summary they were taken from, with a hash of the kernel source
-# they were measured on; a figure measured on another version of the kernel is not reported.
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "attend_kernel_traffic.json")
-ATTEND_SOURCES = [os.path.join(ROOT, "retrievalattention_amd", "csrc", f) for f in ("attend.hip", "attend_common.h")]
+# sit in a small data file next to the summary they were taken from, with a hash of the kernels' sources
+# they were measured on; a figure measured on another version of a kernel is not reported.
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "decode_kernel_traffic.json")
+ATTEND_SOURCES = ("attend.hip", "attend_common.h")
+KERNEL_SOURCES = {"attend_kernel": ATTEND_SOURCES, "dist_kernel": ("select.hip", "ri_common.h"),
+                  "select_attend_kernel": ATTEND_SOURCES + ("select_body.h", "step.hip"),
+                  "step_kernel": ATTEND_SOURCES + ("select_body.h", "step.hip")}
 
 
-def kernel_source_hash():
+def kernel_source_hash(kernel):
     import hashlib
     h = hashlib.sha256()
-    for f in ATTEND_SOURCES:
-        with open(f, "rb") as fh:
+    for f in KERNEL_SOURCES[kernel]:
+        with open(os.path.join(ROOT, "retrievalattention_amd", "csrc", f), "rb") as fh:
             h.update(fh.read())
     return h.hexdigest()[:16]
 
 
-def measured_traffic(config):
-    """(bytes per attend_kernel launch or None, where the figure comes from)."""
+def measured_traffic(config, kernels):
+    """(bytes of one launch of each of `kernels` together or None, where the figure comes from)."""
+    name = os.path.relpath(TRAFFIC_FILE, ROOT)
     try:
         with open(TRAFFIC_FILE) as fh:
-            rec = json.load(fh).get(config)
+            rec = json.load(fh).get(config, {})
     except (OSError, ValueError):
-        return None, f"{os.path.relpath(TRAFFIC_FILE, ROOT)} missing"
-    if not rec:
-        return None, f"no counter run recorded for {config}"
-    if rec.get("kernel_source_sha256_16") != kernel_source_hash():
-        return None, f"{rec['source']}: measured on another version of the kernel (stale, not reported)"
-    nbytes = int((rec["fetch_kib"] * rec["fetch_scale"] + rec["write_kib"] * rec["write_scale"]) * 1024)
-    return nbytes, rec["source"]
+        return None, f"{name} missing"
+    nbytes, sources = 0, []
+    for k in kernels:
+        r = rec.get(k)
+        if not r:
+            return None, f"no counter run of {k} recorded for {config}"
+        if r.get("kernel_source_sha256_16") != kernel_source_hash(k):
+            return None, f"{r['source']}: measured on another version of {k} (stale, not reported)"
+        nbytes += int((r["fetch_kib"] * r["fetch_scale"] + r["write_kib"] * r["write_scale"]) * 1024)
+        if r["source"] not in sources:
+            sources.append(r["source"])
+    return nbytes, ", ".join(sources)
+
+
+def attending_launches(cfg):
+    """The launches of a step over a device-resident store from the selection on, as the library makes them for the
+    configurations below: one for the whole step with few clusters (then the scoring is in it too), else one behind the
+    scoring, in front of which the scores are summed by a launch of their own where there are many."""
+    if cfg["nc"] <= 512:
+        return ["step_kernel"]
+    return (["dist_kernel"] if cfg["nc"] > 4096 else []) + ["select_attend_kernel"]
+
+
+def drift_cycles(steps, layers):
+    """(untimed, timed) cycles of drifting queries, which come from a pool of eight: whole rounds of the pool, two of them
+    untimed, after which the block cache's content repeats from round to round, so that rows counted in a round behind the
+    timed ones are those of a timed round."""
+    return 16, 8 * max(1, steps // (8 * layers))
+
 
 CONFIGS = {
     # name: batch, kv heads, group size, clustered tokens, mixture centres, centroids, segments, outliers, layers
@@ -216,9 +242,10 @@ def bench_kmeans(cfg, dev, iters=10, reps=3):
         segment_k_means_csr(K, V, nc, iters, 1, init_indices=init, reuse_graph=True)
     t_un = time_region(lambda: segment_k_means_csr(K, V, nc, iters, 1, init_indices=init, reuse_graph=True), reps)
     flops_un = 2.0 * 128 * Hkv * N * iters * nc
-    unseg = {"ms_per_sequence": t_un * 1e3, "algorithmic_flops": flops_un, "achieved": flops_un / t_un / 1e12,
-             "frac": flops_un / t_un / MFMA_BF16_PEAK, "init": "seeded random tokens",
-             "note": "flops of every pass over all centroids; passes leave out scores that cannot change an assignment"}
+    unseg = {"ms_per_sequence": t_un * 1e3, "flops_of_all_scores": flops_un, "equivalent_tflops": flops_un / t_un / 1e12,
+             "init": "seeded random tokens",
+             "note": "equivalent: as if every pass scored all centroids; passes leave out scores that cannot change an "
+                     "assignment, so this is no rate of the matrix cores"}
     return {"unsegmented": unseg, "ms_per_sequence": t * 1e3, "tokens": N, "kv_heads": Hkv, "centroids": nc, "segments": S,
             "iterations": iters, "algorithmic_flops": flops, "bound": "mfma", "achieved": flops / t / 1e12,
             "peak": MFMA_BF16_PEAK / 1e12, "unit": "TFLOP/s", "frac": flops / t / MFMA_BF16_PEAK,
@@ -451,8 +478,8 @@ def bench_host(args, cfg, cache, queries, L, nprobe, es, static_len, config_name
                 queries[l].copy_(pool[l][c % 8])
             run_cycle()
 
-        n_cyc = max(1, args.steps // L)
-        for c in range(max(1, args.warmup // L)):
+        n_warm, n_cyc = drift_cycles(args.steps, L)
+        for c in range(n_warm):
             drift_cycle(c)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -460,9 +487,9 @@ def bench_host(args, cfg, cache, queries, L, nprobe, es, static_len, config_name
             drift_cycle(c)
         torch.cuda.synchronize()
         t_d = (time.perf_counter() - t0) / (n_cyc * L)
-        # hit and miss blocks and missed rows of 8 more (untimed) cycles
+        # hit and miss blocks and missed rows of one more (untimed) round of the pool
         dh = dm = dr = 0
-        for c in range(n_cyc, n_cyc + 8):
+        for c in range(8):
             drift_cycle(c)
             torch.cuda.synchronize()
             for l in range(L):
@@ -538,7 +565,7 @@ def bench_host(args, cfg, cache, queries, L, nprobe, es, static_len, config_name
         t_attn = stage_us["attention"] * 1e-6
         where = ("ri_wave_attention over the block cache, every block a hit" if cache.block_cache == "device"
                  else "ri_buffer_attention over the assembled execution buffer")
-        traffic, traffic_source = measured_traffic(f"{config_name or args.config}_host")
+        traffic, traffic_source = measured_traffic(f"{config_name or args.config}_host", ["attend_kernel"])
         roofline = {"bound": "hbm", "kernel": f"attend_kernel ({where})",
                     "achieved": attn_bytes / t_attn / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                     "frac": attn_bytes / t_attn / HBM_PEAK, "traffic": traffic,
@@ -608,7 +635,9 @@ def compact(rec):
         out["cpu_us_per_layer_step"] = cpu["us_per_layer_step"]
         out["cpu_sample"] = cpu["sample"]
     if "stages" in rec:
-        out["stages_us"] = {k: v.get("us_in_step", v["us"]) for k, v in rec["stages"].items()}
+        out["stages_apart_us"] = {k: v.get("us_apart", v["us"]) for k, v in rec["stages"].items()}
+    if "attention_apart" in rec:
+        out["attention_apart"] = rec["attention_apart"]
     return out
 
 
@@ -715,9 +744,10 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
     reps_t.sort()
     t_step = reps_t[len(reps_t) // 2]
 
-    # the attention's duration behind a selection: in the step the attention's workgroups make the selection themselves
-    # (select_attend_kernel), so a layer cycle of both as launches of their own and one of the selection alone are timed by
-    # one event pair each on the launch stream; the difference is attend_kernel plus the gap in front of it
+    # Durations inside replayed cycles, one event pair per cycle on the launch stream.  What attends in the step: the step's cycle
+    # minus one of the scoring alone (attending_launches: the step itself where that is one launch).  The attention as a launch
+    # of its own, which the step does not make (its workgroups make the selection): a cycle of selection and attention minus one
+    # of the selection; attend_kernel plus the gap in front of it.
     from retrievalattention_amd import kernels, _lib
     out_tmp = torch.empty((BG, gs, 128), dtype=DT, device=dev)
 
@@ -728,35 +758,45 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
             cache.value_sum[l], cache.cluster_size[l], out_tmp, cache.valid_lengths[slot], es, cache.RSQRT_DIM,
             ret_tok_off=cache.ret_tok_off, ret_start=cache.ret_start)
 
-    t_attn_in_step = None
+    t_attending = t_attn_apart = None
+    launches = attending_launches(cfg)
     if graphs is not None:
-        sel_cycle = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(sel_cycle):
-            for i in range(CL):
-                cache._select(queries[i % L], i % L, i % 2, True)
-        apart = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(apart):
-            for i in range(CL):
-                cache._select(queries[i % L], i % L, i % 2, True)
-                attend(i % L, i % 2)
+        def captured(body):
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                for i in range(CL):
+                    body(i % L, i % 2)
+            return g
+
+        def selected(l, slot):
+            cache._select(queries[l], l, slot, True)
+
+        def apart(l, slot):
+            selected(l, slot)
+            attend(l, slot)
+
+        def scored(l, slot):
+            kernels.score_logits(queries[l].view(BG, gs, 128), cache.centroids[l], cache.logits, cache.RSQRT_DIM,
+                                 scratch=cache._scratch)
+
+        cycles = [cycle, captured(scored), captured(apart), captured(selected)]
         torch.cuda.synchronize()
-        e0, e1, e2 = (torch.cuda.Event(enable_timing=True) for _ in range(3))
-        best = [float("inf"), float("inf")]
+        marks = [torch.cuda.Event(enable_timing=True) for _ in range(len(cycles) + 1)]
+        best = [float("inf")] * len(cycles)
         n_cyc = max(1, args.steps // CL)
         for _ in range(3):
             for _ in range(2):
-                apart.replay()
-            e0.record()
-            for _ in range(n_cyc):
-                apart.replay()
-            e1.record()
-            for _ in range(n_cyc):
-                sel_cycle.replay()
-            e2.record()
+                cycles[-1].replay()
+            marks[0].record()
+            for g, mark in zip(cycles, marks[1:]):
+                for _ in range(n_cyc):
+                    g.replay()
+                mark.record()
             torch.cuda.synchronize()
-            best = [min(best[0], e0.elapsed_time(e1)), min(best[1], e1.elapsed_time(e2))]
-        t_attn_in_step = (best[0] - best[1]) * 1e-3 / (n_cyc * CL)
-        t_select_in_step = best[1] * 1e-3 / (n_cyc * CL)
+            best = [min(t, a.elapsed_time(b)) for t, a, b in zip(best, marks, marks[1:])]
+        t_cycle, t_scored, t_apart, t_selected = (t * 1e-3 / (n_cyc * CL) for t in best)
+        t_attending = t_cycle if launches == ["step_kernel"] else t_cycle - t_scored
+        t_attn_apart, t_select_apart = t_apart - t_selected, t_selected
 
     # per-kernel pass: the same layer cycle launched eagerly, one event pair around each entry point's
     # launches on the launch stream (cold caches as in the timed region: every step is another layer)
@@ -809,21 +849,26 @@ def bench_device(args, cfg, config_name, L, dev, extras=True):
                                "GBps": attn_bytes / t_attn / 1e9},
         },
     }
-    # dominant kernel: the attention (the one that moves the K/V bytes), as a launch of its own, attend_kernel.  Its duration is
-    # taken in a replayed cycle behind the selection's launches (that cycle minus the one without it); an event pair around one
-    # eager launch also counts the dispatch of the launch (eager_event_us; null_launch_us is what the same pair reads around an
-    # empty kernel).  The timed step itself has one launch for selection and attention.
-    t_dom = t_attn_in_step if t_attn_in_step else t_attn
-    traffic, traffic_source = measured_traffic(config_name)
-    result["roofline"] = {"bound": "hbm", "kernel": "attend_kernel (ri_wave_attention)",
-                          "achieved": attn_bytes / t_dom / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
-                          "frac": attn_bytes / t_dom / HBM_PEAK, "traffic": traffic, "traffic_source": traffic_source,
-                          "launch_us": t_dom * 1e6, "eager_event_us": t_attn * 1e6, "null_launch_us": t_null * 1e6,
-                          "algorithmic_bytes": attn_bytes,
-                          "launches_timed": max(1, args.steps // CL) * CL if t_attn_in_step else n_k}
-    if t_attn_in_step:
-        result["stages"]["score_select"]["us_in_step"] = t_select_in_step * 1e6
-        result["stages"]["wave_attention"]["us_in_step"] = t_attn_in_step * 1e6
+    # dominant: what attends in the timed step (the launches that move the K/V bytes; with eager launches only the attention by
+    # itself is timed).  attention_apart: attend_kernel behind launches that select.  An event pair around one eager launch also
+    # counts its dispatch (eager_event_us; null_launch_us is what the same pair reads around an empty kernel).
+    def roofline(names, nbytes, t, **more):
+        traffic, traffic_source = measured_traffic(config_name, names)
+        return {"bound": "hbm", "kernel": " + ".join(names), "achieved": nbytes / t / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
+                "frac": nbytes / t / HBM_PEAK, "traffic": traffic, "traffic_source": traffic_source, "launch_us": t * 1e6,
+                "algorithmic_bytes": nbytes, **more}
+
+    in_cycles = max(1, args.steps // CL) * CL
+    alone = roofline(["attend_kernel"], attn_bytes, t_attn_apart or t_attn, eager_event_us=t_attn * 1e6,
+                     null_launch_us=t_null * 1e6, launches_timed=in_cycles if t_attn_apart else n_k)
+    if t_attending:
+        result["roofline"] = roofline(launches, total_bytes if launches == ["step_kernel"] else attn_bytes, t_attending,
+                                      launches_timed=in_cycles)
+        result["attention_apart"] = alone
+        result["stages"]["score_select"]["us_apart"] = t_select_apart * 1e6
+        result["stages"]["wave_attention"]["us_apart"] = t_attn_apart * 1e6
+    else:
+        result["roofline"] = alone
     if est_next:
         result["next_layer_estimation"] = bench_estimate_next(args, cache, queries, outs, L, static_len)
     if extras and not args.no_read_probe:
