@@ -53,9 +53,12 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, r
 #define RI_MAX_PROBES 4096  // rank tables of a launch: (2 * np + 1) * 4 bytes of LDS (what the selection lays out)
 #define RI_MAX_GROUPS 4096  // size of the counter area at the head of the workspace
 
+// workgroups per group at most: one per compute unit for all groups together (plan_splits)
+static int attn_max_splits(int BG) { return min(RI_MAX_SPLITS, max(256 / BG, 1)); }
+
 static size_t attn_workspace_bytes(int BG, int gs) {
   if (BG <= 0 || BG > RI_MAX_GROUPS || gs <= 0 || gs > 16) return 0;
-  const size_t per = (size_t)BG * RI_MAX_SPLITS * gs_pad_of(gs);
+  const size_t per = (size_t)BG * attn_max_splits(BG) * gs_pad_of(gs);
   return RI_MAX_GROUPS * sizeof(int) + per * (2 + RI_DIM) * sizeof(float);
 }
 
@@ -118,7 +121,7 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
                         int max_splits = RI_MAX_SPLITS, bool several = false) {
   const int64_t rows = kv_rows + es_rows, wk = kv_rows * 512, we = es_rows * es_row_bytes;
-  int64_t per_group = 256 / BG;
+  int64_t per_group = attn_max_splits(BG);
   per_group = min(per_group, (int64_t)sqrt((double)(wk + we) / (double)(gs * 800)));
   per_group = min(per_group, (rows + 8 * ATT_WAVES - 1) / (8 * ATT_WAVES));   // half a chunk per wave at least
   per_group = min(per_group, (int64_t)max_splits);
