@@ -254,7 +254,6 @@ class retroinfer_cache(KV_Cache):
         i32 = lambda *s: torch.zeros(s, dtype=torch.int32, device=d0)
         self.logits = torch.zeros((BG, gs, self.n_centroids), dtype=torch.float32, device=d0)
         self._scratch = kernels.Scratch()
-        self._allocate_scratch()
         # int64 id lists [BG, nprobe + es] as the reference keeps them: real tensors on the staged
         # operator path (gather_copy_vectors and the host id copy read them), views put together from the
         # int32 lists on demand elsewhere
@@ -303,6 +302,7 @@ class retroinfer_cache(KV_Cache):
 
     def prepare_cache(self):
         """End of prefill (reference: retroinfer_cache.py:336-365)."""
+        self._allocate_scratch()   # (its clearing is done before any stream decodes)
         torch.cuda.synchronize()
         if self.kv_residency == "host":
             if self.block_cache == "host":

@@ -12,6 +12,7 @@ from retrievalattention_amd.cache_hub import retroinfer_cache
 @pytest.fixture
 def no_gpu(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
     monkeypatch.setattr(kernels, "_need", lambda *a, **k: None)
 
 
@@ -24,11 +25,12 @@ def _host_cache(nc=64):
         layer_num=1, layer_mapping={"0": "cpu"}, batch_size=1, batch_groups=2, head_dim=128, group_size=4, n_centroids=nc,
         nprobe=2, es_cluster_num=3, max_compute_cluster_num=5, kv_residency="device", block_cache="device",
         use_cluster_estimation=False, device_positions=False, page_size=8, buffer_size=64, dtype=torch.bfloat16,
-        RSQRT_DIM=128 ** -0.5, _plans={}, centroids=z(2, nc, 128), centroids_mask=z(2, nc, dt=torch.bool),
+        RSQRT_DIM=128 ** -0.5, _plans={}, _centred_keys={}, centroids=z(2, nc, 128), centroids_mask=z(2, nc, dt=torch.bool),
         cluster_size_i32=z(2, nc, dt=i32), cluster_start=z(2, nc, dt=i32), value_sum=z(2, nc, 128), cluster_size=z(2, nc),
         steady_zone_keys=z(1, 2, 70, 128), steady_zone_values=z(1, 2, 70, 128), list_keys=z(1, 2, 99, 128),
         list_values=z(1, 2, 99, 128))
     c.allocate_computation_buffer()
+    c.prepare_cache()
     return c
 
 
