@@ -349,6 +349,13 @@ struct AttendKept {
   int lenA;              // the steady zone's rows
 };
 
+// The waves' value tiles.  (Of a workgroup that makes the selection first: what that lays in them is dead by then.)
+__device__ __forceinline__ uint16_t (*att_tiles())[16 * ATT_VT_STRIDE] {
+  __shared__ __attribute__((aligned(16))) uint16_t sh_vt[ATT_WAVES][16 * ATT_VT_STRIDE];
+  static_assert(__alignof__(sh_vt) == 16, "pieces of 16 bytes");
+  return sh_vt;
+}
+
 // piece threadIdx.x % 16 of the query of head threadIdx.x / 16
 __device__ __forceinline__ uint4 att_query_piece(const AttendParams& P, int g) {
   const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
@@ -363,7 +370,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   constexpr int NW = ATT_WAVES;
   constexpr int NH = GS_PAD / 4;
   constexpr int NT = 64 * NW;
-  __shared__ __attribute__((aligned(16))) uint16_t sh_vt[NW][16 * ATT_VT_STRIDE];
+  uint16_t (*const sh_vt)[16 * ATT_VT_STRIDE] = att_tiles();
   __shared__ __attribute__((aligned(16))) uint16_t sh_pb[NW][16 * 16];
   __shared__ float sh_al[NW][16];
   __shared__ float sh_m[NW][GS_PAD];
@@ -373,7 +380,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   // unit (sixteen heads: 116 KB, one workgroup)
   constexpr bool ACC_OVER_VT = GS_PAD * RI_DIM * sizeof(float) <= 16 * ATT_VT_STRIDE * sizeof(uint16_t);
   __shared__ __attribute__((aligned(16))) float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
-  static_assert(__alignof__(sh_acc_own) == 16 && __alignof__(sh_vt) == 16, "read two dims at a time");
+  static_assert(__alignof__(sh_acc_own) == 16, "read two dims at a time");
   auto acc_of = [&](int w) -> float* {
     return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : &sh_acc_own[ACC_OVER_VT ? 0 : w][0][0];
   };

@@ -9,10 +9,13 @@
 // first half of step_kernel).
 //
 // One compute unit works for a group, so what bounds it is the number of instructions its waves issue, then the barriers
-// between the phases.  The rank thresholds come from two small histograms instead of one with a bin per key: 4 NT coarse
-// bins (the key's upper bits; one 16-byte LDS access per thread to clear and to read them), then the keys inside the two
-// threshold bins by their lower bits, which every wave scans for itself.  The retrieval zone (np of nc clusters) is
-// gathered and sorted as (key, id) pairs in registers, so the rank order needs no histogram either.
+// between the phases.  The rank thresholds come from one histogram with a bin per key over the octaves that scores are found in
+// (SEL_SPAN below), or from the keys' upper bits and then the lower ones of the two threshold bins; bins of one key are also hit
+// by fewer lanes at once.  The places above a bin stay in its word, so a key of the retrieval zone (np of nc) takes its place by
+// one atomic, and the few that share a bin are put in order by looking at each other.  In two histograms always, with the
+// retrieval zone sorted as pairs (36 exchanges for 256 of them), cycles of one of two waves of a SIMD: 32 groups of 4 heads, 8192
+// clusters, 147 probes 18800 -> 14000 from the first load to the tables, steps of four layers 187.8 -> 179.3 us; 64 of 8, 16384,
+// 294: 27300 -> 19500, a step 131.9 -> 128.4.
 // SRC says where the keys come from:
 //   SEL_KEYS    16-bit keys of a preceding dist_kernel (many clusters times heads: the score sums want many compute units)
 //   SEL_LOGITS  the logits and tile partials of a preceding score_kernel: the score sums are made here, one launch less
@@ -110,8 +113,32 @@ struct SelectKept {
   int* start;      // [np]
   int* ids;        // [np] KEEP_TABLES
   int* meta;       // [4] KEEP_TABLES
+  uint32_t* scratch;   // [SEL_SCRATCH<NT>] what the attention has not laid anything in yet
 };
 enum { KEEP_NONE, KEEP_TABLES, KEEP_ALL };
+
+// Bins of the rank search.  Scores are sums of at most sixteen probabilities: in bfloat16 (128 keys to an octave) a bin for
+// each of the 4094 keys up to that of 16, 2^-28 the lowest, finds a rank in one pass; the first bin and the last hold what lies
+// beyond, and where a rank falls there the search is made again by the keys' upper bits.  Half has too many keys for that.
+#define SEL_SPAN 4096
+#define SEL_WINDOW 0xB182u   // bin 0: keys up to this one; bin SEL_SPAN - 2: the key of 16.0, 0xC180
+#define SEL_SHIFT 4          // by the upper bits: lower bits of a key
+#define SEL_RUN 32u          // longest run of a bin that its entries put in order by looking at all of it
+template <int NT>
+constexpr int SEL_SCRATCH = SEL_SPAN + 3 * NT;
+
+typedef uint16_t sel_pair __attribute__((ext_vector_type(2)));
+// the bins of two keys
+__device__ __forceinline__ uint32_t sel_bins(uint32_t keys, bool window) {
+  const sel_pair k = __builtin_bit_cast(sel_pair, keys), lo = {SEL_WINDOW, SEL_WINDOW}, last = {SEL_SPAN - 1, SEL_SPAN - 1};
+  const sel_pair w = __builtin_elementwise_min(__builtin_elementwise_sub_sat(k, lo), last), u = k >> (sel_pair){SEL_SHIFT, SEL_SHIFT};
+  return __builtin_bit_cast(uint32_t, window ? w : u);
+}
+// 1 in the halves where a is above b
+__device__ __forceinline__ uint32_t sel_above(sel_pair a, sel_pair b) {
+  const sel_pair one = {1, 1};
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_sub_sat(a, b), one));
+}
 
 // GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well, with
 // KEEP_TABLES in place of memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
@@ -122,9 +149,12 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   constexpr bool STORE = KEEP != KEEP_TABLES;
   constexpr int NW = NT / 64, IDS = NT * E;
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
-  constexpr int SHIFT = 16 - (LOGT + 2), FB = 1 << SHIFT;   // lower bits of a key, fine bins
-  __shared__ __attribute__((aligned(16))) uint32_t hist[4 * NT];   // coarse bins; later the exchange area of the sort
-  __shared__ uint32_t sh_fine[2][64], sh_scan[3][16], sh_sel[4], sh_tot[3], sh_ret[NT];
+  constexpr int BPT = SEL_SPAN / NT, FB = 1 << SEL_SHIFT;   // bins of a thread, fine bins
+  static_assert(IDS <= 16384 * 2 && E <= 32, "counts in half a word, owned keys in one");
+  __shared__ __attribute__((aligned(16))) uint32_t sh_own[KEEP ? 4 : SEL_SCRATCH<NT>];
+  uint32_t* const hist = KEEP ? K.scratch : sh_own;   // bins; also the exchange area of the sort
+  uint32_t* const sh_rank = hist + SEL_SPAN;          // [3][NT] entries, sizes and first rows in rank order
+  __shared__ uint32_t sh_fine[2][FB], sh_scan[3][16], sh_sel[5], sh_tot[3], sh_ret[NT];
   // Sizes and first rows of all clusters, requested with the first loads: the ones of the retrieval zone are only known
   // after the sort, and a round trip for them there is a tenth of the kernel.  (With more clusters that is more than it saves:
   // 16 groups of 1024 10.4 us either way.)
@@ -138,11 +168,16 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nc = P.nc, np = P.np, es = P.es, k2 = np + es, gs = P.gs;
   const int cbeg = tid * E;   // nc % 8 == 0: a thread's ids exist together, from E = 16 on in eights
-  typedef typename std::conditional<(E <= 32), uint32_t, uint64_t>::type mask_t;
+  typedef uint32_t mask_t;
 
-  *reinterpret_cast<uint4*>(&hist[4 * tid]) = ri_zero16();
-  if (tid < 128) sh_fine[tid >> 6][lane] = 0u;
+  const auto clear_bins = [&]() {
+#pragma unroll
+    for (int i = 0; i < BPT; i += 4) *reinterpret_cast<uint4*>(&hist[BPT * tid + i]) = ri_zero16();
+  };
+  clear_bins();
+  if (tid < 2 * FB) sh_fine[tid / FB][tid % FB] = 0u;
   if (tid < 3) sh_tot[tid] = 0u;
+  if (tid == 3) sh_sel[4] = 0u;
   sh_ret[tid] = 0u;
 
   int32_t own_size = 0, own_row = 0;
@@ -326,117 +361,177 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     for (int i = 0; i < (E + 1) / 2; ++i)
       kw[i] = ri_bf16_sort_key(bits[2 * i]) | ri_bf16_sort_key(bits[2 * i + 1]) << 16;
   }
-  const int nown = min(max(nc - cbeg, 0), E);
   const auto key_of = [&](int i) { return (i & 1) ? kw[i >> 1] >> 16 : kw[i >> 1] & 0xffffu; };
+  const int nown = min(max(nc - cbeg, 0), E);
+  constexpr int KW = (E + 1) / 2, EIGHTS = (E + 7) / 8;   // (nc % 8 == 0: a thread's keys exist together, or eight by eight)
   lds_barrier();
 
   // ---- rank thresholds: T1 = key of descending rank np-1, T2 = key of rank k2-1 ----
+  // Afterwards a bin's word holds the keys above the bin, and in the upper half its own.
+  bool window = !HALF;
+  uint32_t C1, s1, C2, s2;
+  for (;;) {   // (twice at most: by the window, then by the upper bits)
 #pragma unroll
-  for (int i = 0; i < E; ++i)
-    if (i < nown) atomicAdd(&hist[key_of(i) >> SHIFT], 1u);
-  lds_barrier();
-  {
-    const uint4 h4 = *reinterpret_cast<const uint4*>(&hist[4 * tid]);
-    const uint32_t mine = h4.x + h4.y + h4.z + h4.w;
-    const uint32_t inc = ri_wave_incl_scan(mine);
-    if (lane == 63) sh_scan[0][wave] = inc;
-    lds_barrier();
-    uint32_t tot;
-    const uint32_t above = (uint32_t)nc - wave_offset<NW>(sh_scan[0], &tot) - inc;   // keys in bins above this thread's
-    // the thread whose bins hold the rank publishes the bin and the keys above it
-    const auto find = [&](uint32_t rank, uint32_t* out) {
-      if (rank - above < mine) {   // (unsigned: above <= rank < above + mine)
-        const uint32_t hb[4] = {h4.x, h4.y, h4.z, h4.w};
-        uint32_t a = above;
-        int at = 3;
+    for (int o = 0; o < EIGHTS; ++o)
+      if (8 * o < nown) {
 #pragma unroll
-        for (int i = 3; i > 0; --i)
-          if (at == i && rank - a >= hb[i]) { a += hb[i]; at = i - 1; }
-        out[0] = tid * 4 + at;
-        out[1] = a;
+        for (int v = 4 * o; v < 4 * o + 4 && v < KW; ++v) {
+          const uint32_t b = sel_bins(kw[v], window);
+          atomicAdd(&hist[b & 0xffffu], 1u);
+          if (E > 1) atomicAdd(&hist[b >> 16], 1u);
+        }
       }
-    };
-    find((uint32_t)(np - 1), sh_sel);
-    find((uint32_t)(k2 - 1), sh_sel + 2);
-  }
-  lds_barrier();
-  const uint32_t C1 = __builtin_amdgcn_readfirstlane(sh_sel[0]), C2 = __builtin_amdgcn_readfirstlane(sh_sel[2]);
+    lds_barrier();
+    {
+      uint32_t h[BPT], mine = 0;
 #pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const uint32_t k = key_of(i), c = k >> SHIFT;
-    if (i < nown && (c == C1 || c == C2)) atomicAdd(&sh_fine[c == C1 ? 0 : 1][k & (FB - 1)], 1u);
+      for (int i = 0; i < BPT; i += 4) {
+        const uint4 h4 = *reinterpret_cast<const uint4*>(&hist[BPT * tid + i]);
+        h[i] = h4.x; h[i + 1] = h4.y; h[i + 2] = h4.z; h[i + 3] = h4.w;
+      }
+#pragma unroll
+      for (int i = 0; i < BPT; ++i) mine += h[i];
+      const uint32_t inc = ri_wave_incl_scan(mine);
+      if (lane == 63) sh_scan[0][wave] = inc;
+      lds_barrier();
+      uint32_t tot;
+      const uint32_t above = (uint32_t)nc - wave_offset<NW>(sh_scan[0], &tot) - inc;   // keys in bins above this thread's
+      uint32_t a[BPT];
+      a[BPT - 1] = above;
+#pragma unroll
+      for (int i = BPT - 1; i > 0; --i) a[i - 1] = a[i] + h[i];
+#pragma unroll
+      for (int i = 0; i < BPT; i += 4)
+        *reinterpret_cast<uint4*>(&hist[BPT * tid + i]) = make_uint4(a[i] | h[i] << 16, a[i + 1] | h[i + 1] << 16,
+                                                                     a[i + 2] | h[i + 2] << 16, a[i + 3] | h[i + 3] << 16);
+      // the thread whose bins hold the rank publishes the bin and the keys above it
+      const auto find = [&](uint32_t rank, uint32_t* out) {
+        if (rank - above < mine) {   // (unsigned: above <= rank < above + mine)
+          int at = 0;
+          uint32_t up = 0;
+#pragma unroll
+          for (int i = 0; i < BPT; ++i)
+            if (rank - a[i] < h[i]) { at = i; up = a[i]; }
+          out[0] = tid * BPT + at;
+          out[1] = up;
+        }
+      };
+      find((uint32_t)(np - 1), sh_sel);
+      find((uint32_t)(k2 - 1), sh_sel + 2);
+      if (above < (uint32_t)np && mine > SEL_RUN) {   // a bin of the retrieval zone that is long to put in order
+#pragma unroll
+        for (int i = 0; i < BPT; ++i)
+          if (h[i] > SEL_RUN && a[i] + h[i] < (uint32_t)np) sh_sel[4] = 1u;
+      }
+    }
+    lds_barrier();
+    C1 = __builtin_amdgcn_readfirstlane(sh_sel[0]);
+    s1 = __builtin_amdgcn_readfirstlane(sh_sel[1]);
+    C2 = __builtin_amdgcn_readfirstlane(sh_sel[2]);
+    s2 = __builtin_amdgcn_readfirstlane(sh_sel[3]);
+    // (the first and the last bin of the window hold everything beyond it)
+    if (!window || (C2 > 0 && C1 < SEL_SPAN - 1)) break;
+    window = false;
+    clear_bins();
+    lds_barrier();
   }
-  lds_barrier();
-  // the fine bin of rank `rank` counted from the top of the coarse bin, and the keys above it
-  const auto fine_bin = [&](const uint32_t* f, uint32_t rank, uint32_t& above) {
-    const uint32_t c = lane < FB ? f[FB - 1 - (lane & (FB - 1))] : 0u;   // lane l: bin FB-1-l
-    const uint32_t inc = ri_wave_incl_scan(c);
-    const int at = __ffsll((long long)__ballot(inc > rank)) - 1;
-    above = (uint32_t)__builtin_amdgcn_readlane((int)(inc - c), at);
-    return (uint32_t)(FB - 1 - at);
-  };
-  const uint32_t s1 = __builtin_amdgcn_readfirstlane(sh_sel[1]), s2 = __builtin_amdgcn_readfirstlane(sh_sel[3]);
-  uint32_t a1, a2;
-  const uint32_t T1 = (C1 << SHIFT) | fine_bin(sh_fine[0], (uint32_t)(np - 1) - s1, a1);
-  const uint32_t T2 = (C2 << SHIFT) | fine_bin(sh_fine[C1 == C2 ? 0 : 1], (uint32_t)(k2 - 1) - s2, a2);
-  const uint32_t g1 = s1 + a1, g2 = s2 + a2;   // keys strictly above T1 / T2
+  uint32_t T1, T2, g1, g2;   // g1, g2: keys strictly above T1 / T2
+  if (window) {
+    T1 = SEL_WINDOW + C1;
+    T2 = SEL_WINDOW + C2;
+    g1 = s1;
+    g2 = s2;
+  } else {
+#pragma unroll
+    for (int o = 0; o < EIGHTS; ++o)
+      if (8 * o < nown) {
+#pragma unroll
+        for (int i = 8 * o; i < 8 * o + 8 && i < E; ++i) {
+          const uint32_t k = key_of(i), c = k >> SEL_SHIFT;
+          if (c == C1 || c == C2) atomicAdd(&sh_fine[c == C1 ? 0 : 1][k & (FB - 1)], 1u);
+        }
+      }
+    lds_barrier();
+    // the fine bin of rank `rank` counted from the top of the coarse bin, and the keys above it
+    const auto fine_bin = [&](const uint32_t* f, uint32_t rank, uint32_t& above) {
+      const uint32_t c = lane < FB ? f[FB - 1 - (lane & (FB - 1))] : 0u;   // lane l: bin FB-1-l
+      const uint32_t inc = ri_wave_incl_scan(c);
+      const int at = __ffsll((long long)__ballot(inc > rank)) - 1;
+      above = (uint32_t)__builtin_amdgcn_readlane((int)(inc - c), at);
+      return (uint32_t)(FB - 1 - at);
+    };
+    uint32_t a1, a2;
+    T1 = (C1 << SEL_SHIFT) | fine_bin(sh_fine[0], (uint32_t)(np - 1) - s1, a1);
+    T2 = (C2 << SEL_SHIFT) | fine_bin(sh_fine[C1 == C2 ? 0 : 1], (uint32_t)(k2 - 1) - s2, a2);
+    g1 = s1 + a1;
+    g2 = s2 + a2;
+  }
 
-  // ---- one scan places everything: keys above T1, ties at T1, ties at T2 and the keys strictly between ----
+  // ---- one scan places the ties and the keys between the thresholds ----
   // Tied keys are taken in ascending id order: tie rank r at T1 belongs to the retrieval zone
   // while g1 + r < np, then to the estimation zone while g1 + r < k2; at T2 while g2 + r < k2.
-  // The owned keys are classified once, without branches, into bit masks (bit i = owned key i); the rare cases
-  // (keys of the retrieval zone: np of nc; ties at a threshold) are then walked bit by bit.
-  mask_t m_gt1 = 0, m_eq1 = 0, m_gt2 = 0, m_eq2 = 0;
-#pragma unroll
-  for (int i = 0; i < E; ++i) {
-    const uint32_t k = key_of(i);
-    m_gt1 |= (mask_t)(k > T1) << i;
-    m_eq1 |= (mask_t)(k == T1) << i;
-    m_gt2 |= (mask_t)(k > T2) << i;
-    m_eq2 |= (mask_t)(k == T2) << i;
-  }
+  // The owned keys are classified once, two at a time and without branches, into bit masks (bit i = owned key i); the rare
+  // cases (keys of the retrieval zone: np of nc; ties at a threshold) are then walked bit by bit.
+  mask_t m_gt1 = 0, m_lt1 = 0, m_gt2 = 0, m_lt2 = 0;
   {
-    const mask_t ok = nown >= (int)(8 * sizeof(mask_t)) ? ~(mask_t)0 : ((mask_t)1 << nown) - 1;
-    m_gt1 &= ok; m_eq1 &= ok; m_gt2 &= ok;
-    m_eq2 &= T2 == T1 ? 0 : ok;
-  }
-  const mask_t m_mid = m_gt2 & ~m_gt1 & ~m_eq1;  // strictly between the thresholds: estimation zone
-  const auto popc = [](mask_t m) { return (uint32_t)(sizeof(mask_t) == 8 ? __popcll((unsigned long long)m) : __popc((unsigned)m)); };
-  const auto lowest = [](mask_t m) { return sizeof(mask_t) == 8 ? __ffsll((long long)m) - 1 : __ffs((int)m) - 1; };
-  // keys above T1 are fewer than NT <= 1024, everything else is at most nc
-  constexpr int NS = IDS <= 32768 ? 2 : 3;   // words: two counts share one while they fit
-  uint32_t cnt[3] = {popc(m_gt1) | popc(m_eq1) << 12, popc(m_eq2), popc(m_mid)}, pre[3];
-  if (NS == 2) cnt[1] |= cnt[2] << 16;
+    const sel_pair t1 = {(uint16_t)T1, (uint16_t)T1}, t2 = {(uint16_t)T2, (uint16_t)T2};
 #pragma unroll
-  for (int k = 0; k < NS; ++k) {
+    for (int w = 0; w < KW; w += 8) {
+      uint32_t gt1 = 0, lt1 = 0, gt2 = 0, lt2 = 0;   // bit 2 v: key 2 v, bit 16 + 2 v: key 2 v + 1
+#pragma unroll
+      for (int v = 0; v < 8 && w + v < KW; ++v) {
+        const sel_pair k = __builtin_bit_cast(sel_pair, kw[w + v]);
+        gt1 |= sel_above(k, t1) << (2 * v);
+        lt1 |= sel_above(t1, k) << (2 * v);
+        gt2 |= sel_above(k, t2) << (2 * v);
+        lt2 |= sel_above(t2, k) << (2 * v);
+      }
+      const auto in_order = [&](uint32_t m) { return (mask_t)((m & 0x5555u) | m >> 15) << (2 * w); };
+      m_gt1 |= in_order(gt1);
+      m_lt1 |= in_order(lt1);
+      m_gt2 |= in_order(gt2);
+      m_lt2 |= in_order(lt2);
+    }
+  }
+  const mask_t ok = nown >= (int)(8 * sizeof(mask_t)) ? ~(mask_t)0 : ((mask_t)1 << nown) - 1;
+  const mask_t m_eq1 = ~(m_gt1 | m_lt1) & ok, m_eq2 = T2 == T1 ? 0 : ~(m_gt2 | m_lt2) & ok;
+  m_gt1 &= ok;
+  const mask_t m_mid = m_gt2 & ~m_gt1 & ~m_eq1 & ok;  // strictly between the thresholds: estimation zone
+  const auto popc = [](mask_t m) { return (uint32_t)__popc((unsigned)m); };
+  const auto lowest = [](mask_t m) { return __ffs((int)m) - 1; };
+  uint32_t cnt[2] = {popc(m_eq1), popc(m_eq2) | popc(m_mid) << 16}, pre[2];   // (each at most nc <= 16384)
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
     pre[k] = ri_wave_incl_scan(cnt[k]);
-    if (lane == 63) sh_scan[k][wave] = pre[k];
+    if (lane == 63) sh_scan[k + 1][wave] = pre[k];
   }
-  lds_barrier();
-#pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    uint32_t tot;
-    pre[k] += wave_offset<NW>(sh_scan[k], &tot) - cnt[k];
-  }
-  const uint32_t r1 = pre[0] >> 12, r2 = NS == 2 ? pre[1] & 0xffffu : pre[1], mid_before = NS == 2 ? pre[1] >> 16 : pre[2];
-  const uint32_t lo1 = (uint32_t)np - g1;                            // first tie rank of T1 in the est zone
-  const uint32_t hi1r = (uint32_t)k2 > g1 ? (uint32_t)k2 - g1 : 0u;  // one past the last
-  const uint32_t hi2r = (uint32_t)k2 > g2 ? (uint32_t)k2 - g2 : 0u;
-  const uint32_t est_first = mid_before + (min(max(r1, lo1), hi1r) - lo1) + min(r2, hi2r);
   // owned key i (a register half chosen at run time: only the rare walks below need it)
   const auto key_at = [&](int i) {
     uint32_t w = 0;
 #pragma unroll
-    for (int v = 0; v < (E + 1) / 2; ++v) w = ((i >> 1) == v) ? kw[v] : w;
+    for (int v = 0; v < KW; ++v) w = ((i >> 1) == v) ? kw[v] : w;
     return (i & 1) ? (w >> 16) : (w & 0xffffu);
   };
+  // keys above T1 take the places of their bin in whatever order they come
+  for (mask_t m = m_gt1; m; m &= m - 1) {
+    const int i = lowest(m);
+    const uint32_t k = key_at(i);
+    const uint32_t slot = atomicAdd(&hist[sel_bins(k, window) & 0xffffu], 1u) & 0xffffu;
+    sh_ret[slot] = (k << 16) | (0xffffu - (uint32_t)(cbeg + i));
+  }
+  lds_barrier();
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    uint32_t tot;
+    pre[k] += wave_offset<NW>(sh_scan[k + 1], &tot) - cnt[k];
+  }
+  const uint32_t r1 = pre[0], r2 = pre[1] & 0xffffu, mid_before = pre[1] >> 16;
+  const uint32_t lo1 = (uint32_t)np - g1;                            // first tie rank of T1 in the est zone
+  const uint32_t hi1r = (uint32_t)k2 > g1 ? (uint32_t)k2 - g1 : 0u;  // one past the last
+  const uint32_t hi2r = (uint32_t)k2 > g2 ? (uint32_t)k2 - g2 : 0u;
+  const uint32_t est_first = mid_before + (min(max(r1, lo1), hi1r) - lo1) + min(r2, hi2r);
   mask_t est_bits = m_mid;  // bit i: owned key i is in the estimation zone
   {
-    uint32_t slot = pre[0] & 0xfffu;
-    for (mask_t m = m_gt1; m; m &= m - 1, ++slot) {
-      const int i = lowest(m);
-      sh_ret[slot] = (key_at(i) << 16) | (0xffffu - (uint32_t)(cbeg + i));
-    }
     uint32_t rk = r1;  // ties at T1 enter in id order
     for (mask_t m = m_eq1; m && rk < hi1r; m &= m - 1, ++rk) {
       const int i = lowest(m);
@@ -452,22 +547,67 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   uint32_t v = sh_ret[tid];
   const bool in = tid < np;
   const auto id_of = [](uint32_t pair) { return (int)(0xffffu - (pair & 0xffffu)); };
-  // (the sizes and first rows are requested for the unsorted entries, so that the loads behind the sort find them near)
-  int32_t warm_size = 0, warm_start = 0;
-  if (!STAGED && in && P.cluster_size) {
-    warm_size = P.cluster_size[(size_t)g * nc + id_of(v)];
-    if (P.cluster_start) warm_start = P.cluster_start[(size_t)g * nc + id_of(v)];
-  }
-  int n = 64;
-  while (n < np) n <<= 1;
-  block_sort_desc<LOGT>(v, n, hist);
-  if (!STAGED) asm volatile("" : : "v"(warm_size), "v"(warm_start));
-  const int my_c = id_of(v);
+  // (the sizes and first rows are requested for the unsorted entries: they go to the entry's rank with it, or the loads behind
+  // the sort find them near)
   uint32_t sz = 0;
   int32_t st = 0;
-  if (in && P.cluster_size) {
-    sz = (uint32_t)(STAGED ? sh_size[my_c] : P.cluster_size[(size_t)g * nc + my_c]);
-    if (P.cluster_start) st = STAGED ? sh_row[my_c] : P.cluster_start[(size_t)g * nc + my_c];
+  if (!STAGED && in && P.cluster_size) {
+    sz = (uint32_t)P.cluster_size[(size_t)g * nc + id_of(v)];
+    if (P.cluster_start) st = P.cluster_start[(size_t)g * nc + id_of(v)];
+  }
+  if (KEEP) {   // (in front of the wait for them)
+    uint32_t at = est_first;
+    for (mask_t m = est_bits; m; m &= m - 1) K.est[at++] = cbeg + lowest(m);
+  }
+  const bool sorted = __builtin_amdgcn_readfirstlane(sh_sel[4]) != 0 || g1 - s1 > SEL_RUN;   // uniform
+  int my_c;
+  if (!sorted) {
+    // An entry above T1 is in its bin's run of places already; its place there is the number of entries that come before it.
+    // (Ties at T1 are in theirs.)
+    int rank = tid;
+    if (tid < (int)g1) {
+      const uint32_t b = sel_bins(v >> 16, window) & 0xffffu, w = hist[b];
+      const bool cut = !window && b == C1;   // (its keys above T1 only)
+      const int end = cut ? (int)g1 : (int)(w & 0xffffu), start = cut ? (int)s1 : end - (int)(w >> 16);
+      if (end - start > 1) {
+        rank = start;
+        for (int e = start; e < end; e += 4) {
+          uint32_t o[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[u] = sh_ret[min(e + u, end - 1)];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) rank += e + u < end && o[u] > v;
+        }
+      }
+    }
+    if (in) {
+      sh_rank[rank] = v;
+      if (!STAGED) {
+        sh_rank[NT + rank] = sz;
+        sh_rank[2 * NT + rank] = (uint32_t)st;
+      }
+    }
+    lds_barrier();
+    v = in ? sh_rank[tid] : 0u;
+    my_c = id_of(v);
+    if (!STAGED && in) {
+      sz = sh_rank[NT + tid];
+      st = (int32_t)sh_rank[2 * NT + tid];
+    }
+  } else {
+    int n = 64;
+    while (n < np) n <<= 1;
+    block_sort_desc<LOGT>(v, n, hist);
+    if (!STAGED) asm volatile("" : : "v"(sz), "v"(st));
+    my_c = id_of(v);
+    if (!STAGED && in && P.cluster_size) {
+      sz = (uint32_t)P.cluster_size[(size_t)g * nc + my_c];
+      if (P.cluster_start) st = P.cluster_start[(size_t)g * nc + my_c];
+    }
+  }
+  if (STAGED && in && P.cluster_size) {
+    sz = (uint32_t)sh_size[my_c];
+    if (P.cluster_start) st = sh_row[my_c];
   }
 
   // ---- token layout of the retrieved clusters with the page cut-off ----
@@ -511,16 +651,12 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     else K.ids[tid] = my_c;
     if (STORE && P.cI) P.cI[(size_t)g * k2 + tid] = my_c;
   }
-  {
+  if (STORE) {
     uint32_t at = est_first;
-#pragma unroll
-    for (int i = 0; i < E; ++i) {
-      if ((est_bits >> i) & 1u) {
-        if (STORE) P.est_ids[(size_t)g * es + at] = cbeg + i;
-        if (KEEP) K.est[at] = cbeg + i;
-        if (STORE && P.cI) P.cI[(size_t)g * k2 + np + at] = cbeg + i;
-        ++at;
-      }
+    for (mask_t m = est_bits; m; m &= m - 1, ++at) {
+      const int c = cbeg + lowest(m);
+      P.est_ids[(size_t)g * es + at] = c;
+      if (P.cI) P.cI[(size_t)g * k2 + np + at] = c;
     }
   }
   if (!P.cluster_size) return;

@@ -37,6 +37,13 @@ extern "C" int ri_append_kv(const void* key, const void* value, void* steady_k, 
   return RI_OK;
 }
 
+// The selection's bins and rank arrays lie where the attention's value tiles will.
+template <int NT>
+__device__ __forceinline__ uint32_t* select_scratch() {
+  static_assert(SEL_SCRATCH<NT> * sizeof(uint32_t) <= ATT_WAVES * 16 * ATT_VT_STRIDE * sizeof(uint16_t), "room for them");
+  return reinterpret_cast<uint32_t*>(att_tiles());
+}
+
 // What a selection with KEEP_TABLES left in LDS goes to memory, by one of the workgroups that made it and when its rows are
 // attended.
 __device__ __forceinline__ void store_selection(const SelectArgs& S, int g, const SelectKept& K) {
@@ -89,7 +96,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.np = A.np = n[2];
   S.es = A.es = n[3];
   S.scale = A.scale = scale;
-  const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta};
+  const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta, select_scratch<STEP_CLUSTERS>()};
   AttendKept known = {sh_logits, sh_est, sh_off, sh_start};
   const auto ahead = [&]() {
     known.q = att_query_piece(A, blockIdx.x);
@@ -154,7 +161,7 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
   A.W_kv = m[2];
   const int np = S.np, g = blockIdx.x;
   int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
-  const SelectKept kept = {nullptr, est, off, start, ids, meta};
+  const SelectKept kept = {nullptr, est, off, start, ids, meta, select_scratch<NT>()};
   const AttendKept known = {nullptr, est, off, start, att_query_piece(A, g), att_steady_rows(A)};
   select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept);
   lds_barrier();

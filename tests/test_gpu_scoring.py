@@ -271,6 +271,31 @@ def test_score_select_degenerate_scores(dev, kind):
     assert torch.equal(meta.cpu()[:, 0].long(), kept) and torch.equal(off.cpu().long(), offs)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("gs,nc,nprobe,es", [(4, 256, 20, 60), (3, 512, 51, 119), (4, 1024, 100, 240), (8, 4096, 900, 950),
+                                             (4, 8192, 147, 1900), (1, 16384, 1024, 3800)])
+@pytest.mark.parametrize("spread", [0.0, 0.01, 0.2, 1.0, 8.0, 60.0])
+def test_score_select_rank_search(dev, spread, gs, nc, nprobe, es, dt):
+    """Scores from all but equal (long runs of equal keys, at the thresholds and above them) to ones of which most lie
+    below 2^-28 or are 0: wherever a rank falls the zones are the oracle's on the kernel's own scores, to the id."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(nc + int(100 * spread))
+    q = torch.randn(2, gs, 128, generator=g).to(dt).to(dev)
+    cent = (spread * torch.randn(2, nc, 128, generator=g)).to(dt).to(dev)
+    size = torch.randint(0, 20, (2, nc), generator=g, dtype=torch.int32)
+    mask = size == 0
+    start = (torch.cumsum(size, 1) - size).to(torch.int32)
+    i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)
+    ret, est, off, meta = i32(2, nprobe), i32(2, es), i32(2, nprobe + 1), i32(2, 4)
+    dist = torch.empty(2, nc, dtype=dt, device=dev)
+    kernels.score_select(q, cent, mask.to(torch.uint8).to(dev), size.to(dev), start.to(dev), torch.empty(2, gs, nc, device=dev),
+                         dist, None, ret, est, off, None, meta, nprobe, es, 8, 8192, 128 ** -0.5)
+    ret_x, est_x = scoring.select(dist.cpu(), nprobe, es)
+    assert torch.equal(ret.cpu().long(), ret_x) and torch.equal(est.cpu().long(), est_x)
+    kept, offs = scoring.retrieval_layout(ret_x, size, 8, 8192)
+    assert torch.equal(meta.cpu()[:, 0].long(), kept) and torch.equal(off.cpu().long(), offs)
+
+
 def test_score_select_page_cutoff(dev):
     """A tiny execution buffer forces the reference's cut-off: clusters after the first one that
     does not fit are dropped (wave_buffer_cpu.cpp:207-216)."""
