@@ -14,8 +14,8 @@
 // value tile row-major, and eight MFMA 16x16x16 (B operands read with LDS transpose loads) add the chunk
 // to fp32 accumulators that hold, per lane, four heads of one dimension per 16-wide tile.  A group with few
 // rows has one workgroup, which writes the output; otherwise every workgroup writes a (max, denominator, numerator)
-// partial, and the workgroup that finishes last for a group merges the partials (and an optional previous result) with
-// the log-sum-exp rule and writes the output, so the whole call is one launch.
+// partial, and of each share of the heads the wave that finishes last for a group merges the partials (and an optional
+// previous result) with the log-sum-exp rule and writes the output, so the whole call is one launch.
 //
 // Semantics follow the weighted_flash_decoding call sites at
 // cache_hub/retroinfer_cache.py:611-617 and :666-674.
@@ -51,10 +51,11 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, r
 // ------------------------------------------------------------------------------------
 #define RI_MAX_SPLITS 64
 #define RI_MAX_PROBES 4096  // rank tables of a launch: (2 * np + 1) * 4 bytes of LDS (what the selection lays out)
-#define RI_MAX_GROUPS 4096  // size of the counter area at the head of the workspace
+#define RI_MAX_GROUPS 4096  // groups of a launch; words of the counter area at the head of the workspace
 
 // workgroups per group at most: one per compute unit for all groups together (plan_splits)
 static int attn_max_splits(int BG) { return min(RI_MAX_SPLITS, max(256 / BG, 1)); }
+static_assert(128 * ATT_WAVES * ATT_COUNTER_PITCH <= RI_MAX_GROUPS, "more than one workgroup per group: up to 128 groups");
 
 static size_t attn_workspace_bytes(int BG, int gs) {
   if (BG <= 0 || BG > RI_MAX_GROUPS || gs <= 0 || gs > 16) return 0;
@@ -276,7 +277,7 @@ static int wave_attention_impl(const void* q, const void* steady_k, const void* 
   P.prev_lse = prev_lse;
   P.lse_out = lse_out;
   if (clear_counters) {
-    attend_clear_counters_kernel<<<(BG + 255) / 256, 256, 0, stream>>>(P.counters, BG);
+    attend_clear_counters_kernel<<<RI_MAX_GROUPS / 256, 256, 0, stream>>>(P.counters, RI_MAX_GROUPS);
     RI_HIP_CHECK_LAUNCH();
   }
   return launch_attend(P, BG, gs, half, stream);

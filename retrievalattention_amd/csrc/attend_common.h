@@ -127,6 +127,7 @@ __device__ __forceinline__ float2 ri_ld_partial(const float* p) {
 }
 
 #define ATT_WAVES 8                // waves of a workgroup
+#define ATT_COUNTER_PITCH 4        // words between arrival counters: four to a line of 64 bytes
 #define ATT_FLAG_A 0x40000000     // descriptor bit: row lives in region A
 #define ATT_SKIP (int)0x80000000  // descriptor bit (the sign): the row is read but not attended
 
@@ -167,10 +168,10 @@ struct AttendParams {
   const uint16_t* csize;      // [BG, nc] bf16
   int nc;
   int es;
-  // partials and the per-group arrival counters (zero between launches)
+  // partials and the arrival counters (zero between launches)
   float* part_ml;   // [BG, S, GS_PAD, 2]
   float* part_acc;  // [BG, S, GS_PAD, 128]
-  int* counters;    // [BG]
+  int* counters;    // [BG, ATT_WAVES] ATT_COUNTER_PITCH apart
   int S;     // workgroups per group
   int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
   int W_one; // the same of one workgroup's waves, if it takes the whole group
@@ -192,62 +193,87 @@ __device__ __forceinline__ void wave_rows(int total, int nwaves, int wid, int* r
   *r1 = min(total, *r0 + rpw);
 }
 
-// The output rows of head j: A / L merged with an earlier part (its output po, its log-sum-exp pl) under the maximum M.
-// Lane l holds dims 2l and 2l + 1.
-template <bool HALF>
-__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, float M, float L, float A0, float A1) {
-  const int lane = threadIdx.x & 63;
-  const size_t o = (size_t)g * P.gs + j;
+// A piece of the output row of head j, dims d .. d + N-1: A / L merged with an earlier part (its output po, its log-sum-exp pl)
+// under the maximum M.
+template <bool HALF, int N>
+__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, int d, float M, float L, const float (&A)[N]) {
+  static_assert(N == 1 || N == 2, "an element or a pair of them");
+  const size_t o = (size_t)g * P.gs + j, at = o * RI_DIM + d;
+  float x[2] = {A[0], N == 2 ? A[N - 1] : 0.f};
   if (P.prev_lse) {
     const float pl = P.prev_lse[o];
     if (pl != -INFINITY) {  // an empty earlier part carries no weight, whatever its output holds
       float p0, p1;
-      ri_unpack2<HALF>(*reinterpret_cast<const uint32_t*>(P.prev_out + o * RI_DIM + 2 * lane), p0, p1);
+      ri_unpack2<HALF>(N == 2 ? *reinterpret_cast<const uint32_t*>(P.prev_out + at) : (uint32_t)P.prev_out[at], p0, p1);
       const float M2 = fmaxf(M, pl);
       const float f = M == -INFINITY ? 0.f : __expf(M - M2), fp = __expf(pl - M2);
       L = L * f + fp;
-      A0 = A0 * f + fp * p0;
-      A1 = A1 * f + fp * p1;
+      x[0] = x[0] * f + fp * p0;
+      x[1] = x[1] * f + fp * p1;
       M = M2;
     }
   }
   // nothing attended at all (an empty part): zeros and a log-sum-exp of -inf, not 0/0
   const bool any = L > 0.f;
-  *reinterpret_cast<uint32_t*>(P.out + o * RI_DIM + 2 * lane) =
-      (uint32_t)ri_f32_to_e16<HALF>(any ? A0 / L : 0.f) | ((uint32_t)ri_f32_to_e16<HALF>(any ? A1 / L : 0.f) << 16);
-  if (lane == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
+  const uint16_t lo = ri_f32_to_e16<HALF>(any ? x[0] / L : 0.f);
+  if (N == 2)
+    *reinterpret_cast<uint32_t*>(P.out + at) = (uint32_t)lo | ((uint32_t)ri_f32_to_e16<HALF>(any ? x[1] / L : 0.f) << 16);
+  else
+    P.out[at] = lo;
+  if (d == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
 }
 
-// Merges the S split partials of group g (and the optional previous result) and writes the
-// output: wave w of the calling workgroup takes heads w, w+NW, ...; lanes first cover the splits
-// (statistics), then two dims each.
-// The partials come from the memory side, where a load takes about a microsecond and one compute unit gets 20 KB per
-// microsecond: every wave requests the statistics of all its heads and then eight splits of all of them at a time.
+// How the eight waves share the heads when they merge: N dims per lane, PARTS waves to a head of up to four (one past that),
+// HPW heads of a wave.
+template <int GS_PAD>
+struct HeadShare {
+  static constexpr int PARTS = GS_PAD < ATT_WAVES ? ATT_WAVES / GS_PAD : 1;
+  static constexpr int N = RI_DIM / 64 / PARTS;
+  static constexpr int HPW = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;
+  static_assert(N == 1 || N == 2, "a wave covers a head or half of one");
+  static __device__ __forceinline__ int head(int wave, int k) { return PARTS > 1 ? wave % GS_PAD : wave + k * ATT_WAVES; }
+  static __device__ __forceinline__ int dim(int wave, int lane) { return N * ((PARTS > 1 ? wave / GS_PAD * 64 : 0) + lane); }
+};
+
+// Merges a wave's share of the S split partials of group g (and the optional previous result) and writes the output: lanes
+// first cover the splits (statistics), then N dims each.
+// The partials come from the memory side, where a load takes about a microsecond: a wave requests the statistics of its
+// heads and sixteen splits of them at a time before it looks at any.
 // (One head after the other: 13600 cycles for 16 heads over 3 splits.)
 template <int GS_PAD, bool HALF>
-__device__ __forceinline__ void combine_group(const AttendParams& P, int g) {
-  constexpr int NW = ATT_WAVES;
-  constexpr int HPW = (GS_PAD + NW - 1) / NW;   // heads of a wave
-  constexpr int U = HPW > 2 ? 4 : 8;            // splits requested at a time
+__device__ __forceinline__ void combine_share(const AttendParams& P, int g, int wave) {
+  typedef HeadShare<GS_PAD> Share;
+  constexpr int HPW = Share::HPW, N = Share::N, U = 8;   // U: splits requested without a condition
   const int gs = P.gs, S = P.S;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (wave >= gs) return;
+  const int lane = threadIdx.x & 63;
+  const int d = Share::dim(wave, lane);
+  int head[HPW];
+#pragma unroll
+  for (int k = 0; k < HPW; ++k) head[k] = min(Share::head(wave, k), gs - 1);
   const float* ml = P.part_ml + (size_t)g * S * GS_PAD * 2;
-  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + 2 * lane;
+  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + d;
   float2 ms[HPW];
 #pragma unroll
-  for (int k = 0; k < HPW; ++k)
-    ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * 2);
-  float2 a[U][HPW];
-  const auto request = [&](int s0) {
+  for (int k = 0; k < HPW; ++k) ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + head[k]) * 2);
+  float a[2][U][HPW][N];
+  const auto request = [&](int b, int s0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int k = 0; k < HPW; ++k)
-        a[u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + min(wave + k * NW, gs - 1)) * RI_DIM);
+      for (int k = 0; k < HPW; ++k) {
+        const float* p = pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + head[k]) * RI_DIM;
+        if (N == 2) {
+          const float2 x = ri_ld_partial(p);
+          a[b][u][k][0] = x.x;
+          a[b][u][k][N - 1] = x.y;
+        } else {
+          a[b][u][k][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
   };
-  request(0);
-  float f[HPW], M[HPW], L[HPW], A0[HPW], A1[HPW];
+  request(0, 0);
+  if (S > U) request(1, U);
+  float f[HPW], M[HPW], L[HPW], A[HPW][N];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
     const float m = lane < S ? ms[k].x : -INFINITY;
@@ -256,23 +282,31 @@ __device__ __forceinline__ void combine_group(const AttendParams& P, int g) {
     f[k] = m == -INFINITY ? 0.f : __expf(m - M[k]);
     L[k] = ri_row_sum(ms[k].y * f[k]);
     L[k] = ri_xor_sum<32>(ri_xor_sum<16>(L[k]));
-    A0[k] = A1[k] = 0.f;
+#pragma unroll
+    for (int n = 0; n < N; ++n) A[k][n] = 0.f;
   }
-  for (int s0 = 0; s0 < S; s0 += U) {   // (a split past the last has no weight: f of its lane is 0)
-    if (s0) request(s0);
+  const auto add = [&](int b, int s0) {   // (a split past the last has no weight: f of its lane is 0)
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int k = 0; k < HPW; ++k) {
         const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[k]), (s0 + u) & 63));
         const float w = s0 + u < S ? fs : 0.f;
-        A0[k] += a[u][k].x * w;
-        A1[k] += a[u][k].y * w;
+#pragma unroll
+        for (int n = 0; n < N; ++n) A[k][n] += a[b][u][k][n] * w;
       }
+  };
+  for (int s0 = 0;; s0 += 2 * U) {
+    add(0, s0);
+    if (s0 + U >= S) break;
+    if (s0 + 2 * U < S) request(0, s0 + 2 * U);
+    add(1, s0 + U);
+    if (s0 + 2 * U >= S) break;
+    if (s0 + 3 * U < S) request(1, s0 + 3 * U);
   }
 #pragma unroll
   for (int k = 0; k < HPW; ++k)
-    if (wave + k * NW < gs) write_head<HALF>(P, g, wave + k * NW, M[k], L[k], A0[k], A1[k]);
+    if (Share::head(wave, k) < gs) write_head<HALF, N>(P, g, head[k], d, M[k], L[k], A[k]);
 }
 
 #define ATT_DESC_MAX 64  // rows of one wave whose descriptors are staged in LDS at a time (32 and 128 measured slower)
@@ -365,6 +399,32 @@ __device__ __forceinline__ int att_steady_rows(const AttendParams& P) {
   return P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
 }
 
+// The last of n ranks whose first row off[rank] is <= row (ranks of empty clusters share a first row with the next rank, which
+// is the one found); off[0] is 0.  For whole waves, whose rows ascend with the lane and are at most a batch apart: the wave
+// looks for the first one's rank together, 64 ranks per read, and counts on from there, the few ranks that begin behind it and
+// not behind the last row.  (Every lane by bisection took eight reads one after the other, 2000 .. 2500 cycles of each
+// wave's chain for 150 .. 300 ranks.)
+__device__ __forceinline__ int rank_of(const int* off, int n, int row) {
+  const int lane = threadIdx.x & 63;
+  const int first = __builtin_amdgcn_readfirstlane(row), last = __builtin_amdgcn_readlane(row, 63);
+  int base = 0, span = n;   // uniform: off[base] <= first < off[base + span]
+  while (span > 64) {
+    const int step = (span + 63) >> 6, at = lane * step;
+    const uint64_t below = __builtin_amdgcn_ballot_w64(at < span && off[base + min(at, span - 1)] <= first);
+    const int found = (__builtin_popcountll(below) - 1) * step;
+    base += found;
+    span = min(step, span - found);
+  }
+  int rank = base - 1;
+  for (;;) {   // uniform: 64 ranks from base on, until one begins behind the last row
+    const int o = base + lane < n ? off[base + lane] : 0x7fffffff;
+    const uint64_t here = __builtin_amdgcn_ballot_w64(o <= last);
+    for (uint64_t m = here; m; m &= m - 1) rank += __builtin_amdgcn_readlane(o, __builtin_ctzll(m)) <= row;
+    if (~here) return rank;
+    base += 64;
+  }
+}
+
 template <int GS_PAD, bool HALF, int KEPT>
 __device__ __forceinline__ void attend_group(const AttendParams& P, const int g, const int split, const AttendKept& K) {
   constexpr int NW = ATT_WAVES;
@@ -387,7 +447,6 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   __shared__ __attribute__((aligned(16))) uint16_t sh_q[GS_PAD][RI_DIM];
   __shared__ int sh_desc[NW][ATT_DESC_MAX];
   __shared__ float sh_w[NW][ATT_DESC_MAX];
-  __shared__ int sh_last;
   extern __shared__ __attribute__((aligned(16))) int sh_tab[];
   int* const sh_roff = KEPT ? K.off : sh_tab;                // [np + 1]
   int* const sh_rst = KEPT ? K.start : sh_tab + P.np + 1;    // [np]
@@ -481,22 +540,17 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
     attend_rows<GS_PAD, HALF, Keys>(
         st, sh, r0, r1,
         [&](int row, float& w) {
-          if (row < lead) return row | ATT_FLAG_A;
-          const int rb = row - lead;
           int d;
           if (KEPT || (!est && P.ret_off)) {
-            // the last rank whose first row is <= rb (ranks of empty clusters share a first row
-            // with the next rank, which is the one found)
-            int lo = 0, hi = P.np;
-            while (lo + 1 < hi) {
-              const int mid = (lo + hi) >> 1;
-              if (sh_roff[mid] <= rb) lo = mid; else hi = mid;
-            }
-            d = sh_rst[lo] + rb - sh_roff[lo];
-          } else {
-            d = rs ? rs[rb] : rb;
-            if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d = ATT_SKIP;   // row 0, not attended
+            if (__builtin_amdgcn_readlane(row, 63) < lead) return row | ATT_FLAG_A;   // (the batch's last row)
+            const int rb = max(row - lead, 0), rank = rank_of(sh_roff, P.np, rb);
+            d = sh_rst[rank] + rb - sh_roff[rank];
+            return row < lead ? row | ATT_FLAG_A : d;   // (no weights with rank tables)
           }
+          if (row < lead) return row | ATT_FLAG_A;
+          const int rb = row - lead;
+          d = rs ? rs[rb] : rb;
+          if (!est && P.row_src && (d < P.src_lo || d >= P.src_hi)) d = ATT_SKIP;   // row 0, not attended
           if (wB) w = ri_e16_to_f32<HALF>(wB[rb]);
           if (wsrc) w = ri_e16_to_f32<HALF>(wsrc[d]);
           return d;
@@ -580,9 +634,14 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   }
   __syncthreads();
 
-  // ---------------- merge the waves: wave w takes heads w, w + NW, ..., a lane two dims ----------------
-  for (int j = wave; j < gs; j += NW) {
-    float m[NW], M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
+  // ---------------- merge the waves: each takes its share of the heads ----------------
+  typedef HeadShare<GS_PAD> Share;
+  const int d = Share::dim(wave, lane);
+#pragma unroll
+  for (int k = 0; k < Share::HPW; ++k) {
+    const int j = Share::head(wave, k);
+    if (j >= gs) break;
+    float m[NW], M = -INFINITY, a[Share::N] = {}, l = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       m[w] = sh_m[w][j];
@@ -591,21 +650,24 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float f = m[w] == -INFINITY ? 0.f : __expf(m[w] - M);
-      const float2 x = *reinterpret_cast<const float2*>(acc_of(w) + j * RI_DIM + 2 * lane);
-      a0 += x.x * f;
-      a1 += x.y * f;
+      const float* x = acc_of(w) + j * RI_DIM + d;
+#pragma unroll
+      for (int n = 0; n < Share::N; ++n) a[n] += x[n] * f;
       l += sh_l[w][j] * f;
     }
     if (S == 1) {   // the workgroup has the whole group: no partial leaves it
-      write_head<HALF>(P, g, j, M, l, a0, a1);
+      write_head<HALF, Share::N>(P, g, j, d, M, l, a);
       continue;
     }
     const size_t o = ((size_t)g * S + split) * GS_PAD + j;
     // device-coherent stores: another workgroup of this launch reads them
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + 2 * lane]),
-                       (uint64_t)__float_as_uint(a0) | (uint64_t)__float_as_uint(a1) << 32, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    if (lane == 0)
+    if (Share::N == 2)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + d]),
+                         (uint64_t)__float_as_uint(a[0]) | (uint64_t)__float_as_uint(a[Share::N - 1]) << 32, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    else
+      __hip_atomic_store(&P.part_acc[o * RI_DIM + d], a[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0)   // (of a head's waves each for itself: the last of its own kind reads it)
       __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_ml[o * 2]),
                          (uint64_t)__float_as_uint(M) | (uint64_t)__float_as_uint(l) << 32, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
@@ -616,37 +678,38 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   }
   if constexpr (KEPT != KEPT_ALL) {
 
-  // ---------------- last workgroup of the group merges all splits ----------------
-  // Hand-off of the partials between workgroups of one launch, without fences:
+  // ---------------- the last wave of its share over all splits merges them ----------------
+  // Hand-off of the partials between workgroups of one launch, wave by wave (no barrier, and a group's heads are merged
+  // beside each other, by whichever workgroups come last: with the ranks found by whole waves, see rank_of, a layer of 16 groups
+  // of 4 heads, 1024 clusters 17.8 -> 17.6 us, of 32 of 4, 8192 44.8 -> 44.4, of 64 of 8, 16384 128.4 -> 127.5) and without fences:
   //  * the partial was written above with agent-scope atomic stores: on gfx950 those are write-through
   //    stores (sc1) that complete in the memory-side cache every compute unit shares, not in this
   //    compute unit's L1 or this chiplet's L2;
-  //  * s_waitcnt(0) returns when all of this wave's stores have been acknowledged there, the barrier
-  //    makes that true for the whole workgroup, and only then does one thread announce the arrival with
-  //    an agent-scope atomic increment (performed at the same shared level);
-  //  * the workgroup that sees the count complete reads the partials with agent-scope atomic loads
-  //    (combine_group), which bypass the non-coherent cache levels.
+  //  * s_waitcnt(0) returns when all of this wave's stores have been acknowledged there, and only then does the wave announce
+  //    the arrival of its share with an agent-scope atomic increment (performed at the same shared level);
+  //  * the wave that sees the count complete reads the partials of this share, and of no other, with agent-scope atomic
+  //    loads (combine_share), which bypass the non-coherent cache levels.
   // So every partial is globally visible before its arrival can be counted, and the reader cannot hit a
   // stale line.  The C++ memory model would express this with a release increment and an acquire on the
   // last arriver; at agent scope those compile to a write-back and an invalidate of the whole L2, which
   // was measured at +15 us per launch (35.2 us instead of 20.0 us at the benchmark shape), while the
-  // data that must be ordered is only this workgroup's own 2 KB.  The asm statement keeps the compiler
+  // data that must be ordered is only this wave's own 2 KB.  The asm statement keeps the compiler
   // from moving the stores below the wait.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "the partial hand-off below relies on gfx950 cache behaviour: build this file for gfx950 only"
 #endif
+  if (Share::head(wave, 0) >= gs) return;
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0)
-    sh_last = (__hip_atomic_fetch_add(&P.counters[g], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1);
-  __syncthreads();
-  if (!sh_last) return;
-  combine_group<GS_PAD, HALF>(P, g);
+  int* const arrived = P.counters + (g * NW + wave) * ATT_COUNTER_PITCH;
+  int before = 0;
+  if (lane == 0) before = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(before) != S - 1) return;
+  combine_share<GS_PAD, HALF>(P, g, wave);
   if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
   // ready for the next launch (every arrival of this launch has been counted; launches that share the
   // workspace do not overlap)
-  if (threadIdx.x == 0) __hip_atomic_store(&P.counters[g], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane == 0) __hip_atomic_store(arrived, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 

@@ -616,9 +616,14 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   uint32_t T_ret = 0, pages = 0;
   bool keep = false;
   if (P.cluster_size) {
-    const uint32_t pg = (sz + P.page - 1) / P.page;
-    uint32_t pg_pre = ri_wave_incl_scan(pg);
-    tok = ri_wave_incl_scan(sz);
+    // (a division by what is not known when this is built takes forty instructions)
+    const uint32_t up = sz + P.page - 1;
+    const uint32_t pg = (P.page & (P.page - 1)) == 0 ? up >> __builtin_ctz(P.page) : up / P.page;
+    uint32_t pg_pre = 0;
+    if (wave * 64 < np) {   // uniform
+      pg_pre = ri_wave_incl_scan(pg);
+      tok = ri_wave_incl_scan(sz);
+    }
     if (lane == 63) {
       sh_scan[0][wave] = pg_pre;
       sh_scan[1][wave] = tok;

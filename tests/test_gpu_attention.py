@@ -356,6 +356,70 @@ def _hide_rows(gen, S, runs):
     return hidden
 
 
+@pytest.mark.parametrize("BG,gs", [(1, 1), (2, 4), (3, 5), (8, 8), (11, 16), (128, 3), (129, 3)])
+def test_split_merge_shares(dev, BG, gs):
+    """Every head's share of the merge (two waves to a head, one, two heads to a wave; with up to 64 splits, and none past 128
+    groups), over and over on one workspace, with an earlier part and the log-sum-exp: against fp32 over the same rows.
+    Probabilities and outputs are 16 bits wide: 2^-8 of a value each, of which a norm sees a fraction."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(BG + gs)
+    for S in (700, 5003):
+        S = S if BG < 100 else S // 10
+        q, k, v = (torch.randn(BG, *s, 128, generator=g).to(torch.bfloat16) for s in ((1, gs), (S, 1), (S, 1)))
+        x = torch.einsum("bhd,bsd->bhs", q[:, 0].float(), k[:, :, 0].float()) / math.sqrt(128)
+        want = torch.einsum("bhs,bsd->bhd", x.softmax(-1), v[:, :, 0].float())
+        q, k, v = q.to(dev), k.to(dev), v.to(dev)
+        for cut in (S // 3, 16, S - 1):
+            o1, l1 = kernels.weighted_flash_decoding(q, k[:, :cut].contiguous(), v[:, :cut].contiguous(), return_softmax_lse=True)
+            out, lse = kernels.weighted_flash_decoding(q, k[:, cut:].contiguous(), v[:, cut:].contiguous(), previous_out=o1,
+                                                       previous_lse=l1, return_softmax_lse=True)
+            got = out.float().cpu().reshape(BG, gs, 128)
+            assert (got - want).norm() <= 4e-3 * want.norm()
+            assert torch.allclose(lse.cpu().reshape(BG, gs), x.logsumexp(-1), rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("n_clusters,np_", [(40, 3), (300, 64), (300, 65), (600, 129), (4096, 4096)])
+def test_rank_tables_of_empty_and_crowded_clusters(dev, n_clusters, np_):
+    """Ranks found by whole waves: runs of empty clusters longer than a wave, clusters of thousands of rows, one to 64 ranks per
+    read and more, a cut list; against the same rows through a row table."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(np_)
+    BG, gs = 2, 4
+    size = torch.randint(0, 3, (BG, n_clusters), generator=g)
+    size[torch.rand(BG, n_clusters, generator=g) < 0.6] = 0
+    size[:, np_ // 2] = 1500
+    size[:, :min(2, np_)] = 0
+    if np_ > 200:
+        size[:, 20:160] = 0
+    size[1, np_ - 1] = 70
+    start = size.cumsum(1) - size
+    rows = int(size.sum(1).max())
+    ids = torch.stack([torch.randperm(n_clusters, generator=g)[:np_] for _ in range(BG)])
+    n, first = torch.gather(size, 1, ids), torch.gather(start, 1, ids)
+    off = torch.cat([torch.zeros(BG, 1, dtype=torch.long), n.cumsum(1)], 1)
+    keep = np_ - np_ // 8
+    off[:, keep + 1:] = off[:, keep:keep + 1]                    # a cut list: constant from the last kept rank on
+    total = off[:, -1]
+    table = torch.full((BG, int(total.max()) + 1), -1, dtype=torch.int32)
+    for b in range(BG):
+        at = torch.cat([first[b, r] + torch.arange(int(n[b, r])) for r in range(keep)])
+        table[b, :at.numel()] = at.int()
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dev)
+    q, zk, zv, sk, sv = bf(BG, gs, 128), bf(BG, 80, 128), bf(BG, 80, 128), bf(BG, rows, 128), bf(BG, rows, 128)
+    sums = bf(BG, 8, 128)
+    meta = torch.stack([torch.full((BG,), keep), total, total * 0, total * 0], 1).int().to(dev)
+    outs = []
+    for tables in (True, False):
+        out, valid = torch.empty(BG, gs, 128, dtype=torch.bfloat16, device=dev), torch.empty(BG, dtype=torch.int32, device=dev)
+        kernels.wave_attention(q, zk, zv, 71, sk, sv, None if tables else table.to(dev), meta, None, None, sums, None, out, valid,
+                               0, 128 ** -0.5, ret_tok_off=off.int().to(dev) if tables else None,
+                               ret_start=first.int().to(dev) if tables else None)
+        assert torch.equal(valid.cpu().long(), total + 71)
+        outs.append(out.float())
+    # (the two plan their splits for another number of rows: roundings of 16-bit probabilities and outputs)
+    assert (outs[0] - outs[1]).norm() <= 4e-3 * outs[1].norm()
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("gs,S,runs", [(4, 40, True), (4, 1000, True), (7, 130, False), (8, 3001, True), (12, 640, True)])
 def test_infinite_key_elements(dev, gs, S, runs, dt):
