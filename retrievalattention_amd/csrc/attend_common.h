@@ -395,8 +395,13 @@ __device__ __forceinline__ uint4 att_query_piece(const AttendParams& P, int g) {
   const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
   return ri_ld16(P.q + ((size_t)g * P.gs + min(head, P.gs - 1)) * RI_DIM + piece * 8);
 }
+// the steady zone's rows (a vector load: the wait for a scalar one is a wait for every access to LDS as well)
 __device__ __forceinline__ int att_steady_rows(const AttendParams& P) {
-  return P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA;
+  int none = 0;
+  asm("" : "+v"(none));
+  const int32_t* const at = P.lenA_ptr ? P.lenA_ptr : reinterpret_cast<const int32_t*>(P.q);   // (any valid place)
+  const int there = at[none];
+  return P.lenA_ptr ? min(max(there, 0), (int)P.strideA) : P.lenA;
 }
 
 // The last of n ranks whose first row off[rank] is <= row (ranks of empty clusters share a first row with the next rank, which
@@ -467,7 +472,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(sh.pb)[i] = 0u;
   if (lane < 16) sh.al[lane] = 1.f;
   const int lenB = KEPT ? K.off[P.np] : P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  const int lenA = KEPT ? K.lenA : att_steady_rows(P);
+  const int lenA = __builtin_amdgcn_readfirstlane(KEPT ? K.lenA : att_steady_rows(P));
 
   const int wid = split * NW + wave;            // wave of the group
   const bool kv_wave = wid < P.W_kv;

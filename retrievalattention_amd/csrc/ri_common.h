@@ -256,6 +256,13 @@ __device__ __forceinline__ void ri_wave_reduce_partials(const float* pm, const f
   *invz_out = 1.0f / ri_wave_sum(z);
 }
 
+// The same from at most 64 partials, a lane's own (-inf, 0 past the last).
+__device__ __forceinline__ void ri_wave_reduce_partials(float pm, float ps, float* m_out, float* invz_out) {
+  const float m = ri_wave_max(pm);
+  *m_out = m;
+  *invz_out = 1.0f / ri_wave_sum(ps * __expf(pm - m));
+}
+
 // Inclusive prefix sum over the 64 lanes of a wave with DPP row shifts and row broadcasts
 // (no LDS traffic): shifts by 1, 2, 3 build sums of four neighbours, shifts by 4 and 8 finish the
 // 16-lane rows, the two broadcasts carry row totals into the rows behind.

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(NT) void select_radix_kernel(ri_ptr4 in, ri_int4 n,
   P.np = n[2];
   P.es = n[3];
   P.ntiles = ntiles;
-  select_group<NT, E, GSM, HALF, SRC, KEEP_NONE>(P, blockIdx.x, SelectKept{});
+  select_group<NT, E, GSM, HALF, SRC, KEEP_NONE>(P, blockIdx.x, SelectKept{}, [] {});
 }
 
 // ------------------------------------------------------------------------------------

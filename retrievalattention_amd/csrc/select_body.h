@@ -134,16 +134,18 @@ __device__ __forceinline__ uint32_t sel_bins(uint32_t keys, bool window) {
   const sel_pair w = __builtin_elementwise_min(__builtin_elementwise_sub_sat(k, lo), last), u = k >> (sel_pair){SEL_SHIFT, SEL_SHIFT};
   return __builtin_bit_cast(uint32_t, window ? w : u);
 }
-// 1 in the halves where a is above b
-__device__ __forceinline__ uint32_t sel_above(sel_pair a, sel_pair b) {
-  const sel_pair one = {1, 1};
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_sub_sat(a, b), one));
+// 1 in the halves where a is above b (written out: the compiler makes two comparisons and two selects of it)
+__device__ __forceinline__ uint32_t sel_above(uint32_t a, uint32_t b) {
+  uint32_t m;
+  asm("v_pk_sub_u16 %0, %1, %2 clamp\n\tv_pk_min_u16 %0, %0, 1 op_sel_hi:[1,0]" : "=&v"(m) : "v"(a), "v"(b));
+  return m;
 }
 
 // GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well, with
 // KEEP_TABLES in place of memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
-template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP>
-__device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K) {
+// ahead(): what the caller wants on its way behind the selection's first loads.
+template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP, typename Ahead>
+__device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K, Ahead&& ahead) {
   static_assert(KEEP == KEEP_NONE || SRC != SEL_SCORE || GSM <= 8, "the logits are in LDS");
   static_assert(KEEP != KEEP_ALL || SRC == SEL_SCORE, "what is not kept is in memory");
   constexpr bool STORE = KEEP != KEEP_TABLES;
@@ -194,6 +196,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       const uint4 k = *reinterpret_cast<const uint4*>(P.keys + (size_t)g * nc + min(cbeg + 8 * i, nc - 8));
       kw[4 * i] = k.x; kw[4 * i + 1] = k.y; kw[4 * i + 2] = k.z; kw[4 * i + 3] = k.w;
     }
+    ahead();
   } else {
     float d[E];
     const int cc = min(cbeg, nc - E);
@@ -222,6 +225,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) bq[kk] = ri_ld16(p + kk * 32);
       }
+      ahead();
       __builtin_amdgcn_sched_barrier(0);   // every load is in flight before the first product
       f32x4_t acc[4];
 #pragma unroll
@@ -321,18 +325,32 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       constexpr int V = E < 4 ? E : 4;   // columns per load
       typedef float vec_t __attribute__((ext_vector_type(V)));
       vec_t x[GSM][E / V];
+      // (a group's logits lie within 1 MB: 32-bit offsets from one base)
+      const char* const lg = reinterpret_cast<const char*>(P.logits + (size_t)g * gs * nc);
 #pragma unroll
       for (int j = 0; j < GSM; ++j)
 #pragma unroll
         for (int i = 0; i < E / V; ++i)
-          x[j][i] = *reinterpret_cast<const vec_t*>(P.logits + ((size_t)g * gs + min(j, gs - 1)) * nc + cc + V * i);
-      for (int j = wave; j < gs; j += NW) {
+          x[j][i] = *reinterpret_cast<const vec_t*>(lg + (uint32_t)(min(j, gs - 1) * nc + cc + V * i) * 4u);
+      // (at most 64 partials: narrow tiles up to 4096 clusters, wide ones past them.  All on their way before any is looked at.)
+      constexpr int HPW = (GSM + NW - 1) / NW;
+      const size_t part = (size_t)g * P.ntiles * gs;
+      const char *const pm = reinterpret_cast<const char*>(P.tile_max + part), *const ps = reinterpret_cast<const char*>(P.tile_sum + part);
+      float pm0[HPW], ps0[HPW];
+#pragma unroll
+      for (int k = 0; k < HPW; ++k) {
+        const uint32_t at = (uint32_t)(min(lane, P.ntiles - 1) * gs + min(wave + k * NW, gs - 1)) * 4u;
+        pm0[k] = *reinterpret_cast<const float*>(pm + at);
+        ps0[k] = *reinterpret_cast<const float*>(ps + at);
+      }
+      ahead();
+#pragma unroll
+      for (int k = 0; k < HPW; ++k) {
         float m, iz;
-        ri_wave_reduce_partials(P.tile_max + (size_t)g * P.ntiles * gs, P.tile_sum + (size_t)g * P.ntiles * gs,
-                                P.ntiles, gs, j, lane, &m, &iz);
-        if (lane == 0) {
-          sh_a[0][j] = m;
-          sh_b[0][j] = iz;
+        ri_wave_reduce_partials(lane < P.ntiles ? pm0[k] : -INFINITY, lane < P.ntiles ? ps0[k] : 0.f, &m, &iz);
+        if (lane == 0 && wave + k * NW < gs) {
+          sh_a[0][wave + k * NW] = m;
+          sh_b[0][wave + k * NW] = iz;
         }
       }
       lds_barrier();
@@ -355,7 +373,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     for (int i = 0; i < E; ++i) {
       bits[i] = ri_f32_to_e16<HALF>(d[i]);
       if ((mk[i / MB] >> (8 * (i % MB))) & 0xffu) bits[i] = ri_e16_lowest<HALF>();  // finfo(type).min
-      if (P.dist_out && cbeg < nc) P.dist_out[(size_t)g * nc + cbeg + i] = bits[i];
+      if (!KEEP && P.dist_out && cbeg < nc) P.dist_out[(size_t)g * nc + cbeg + i] = bits[i];
     }
 #pragma unroll
     for (int i = 0; i < (E + 1) / 2; ++i)
@@ -407,22 +425,23 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       // the thread whose bins hold the rank publishes the bin and the keys above it
       const auto find = [&](uint32_t rank, uint32_t* out) {
         if (rank - above < mine) {   // (unsigned: above <= rank < above + mine)
-          int at = 0;
-          uint32_t up = 0;
+          uint32_t at = 0, up = a[0];
 #pragma unroll
-          for (int i = 0; i < BPT; ++i)
-            if (rank - a[i] < h[i]) { at = i; up = a[i]; }
+          for (int i = 1; i < BPT; ++i) {
+            at += rank < a[i - 1];
+            up = rank < a[i - 1] ? a[i] : up;
+          }
           out[0] = tid * BPT + at;
           out[1] = up;
         }
       };
       find((uint32_t)(np - 1), sh_sel);
       find((uint32_t)(k2 - 1), sh_sel + 2);
-      if (above < (uint32_t)np && mine > SEL_RUN) {   // a bin of the retrieval zone that is long to put in order
+      uint32_t most = h[0];
 #pragma unroll
-        for (int i = 0; i < BPT; ++i)
-          if (h[i] > SEL_RUN && a[i] + h[i] < (uint32_t)np) sh_sel[4] = 1u;
-      }
+      for (int i = 1; i < BPT; ++i) most = max(most, h[i]);
+      // a bin of the retrieval zone that is long to put in order (or one just below it)
+      if (above < (uint32_t)np && most > SEL_RUN) sh_sel[4] = 1u;
     }
     lds_barrier();
     C1 = __builtin_amdgcn_readfirstlane(sh_sel[0]);
@@ -474,13 +493,13 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   // cases (keys of the retrieval zone: np of nc; ties at a threshold) are then walked bit by bit.
   mask_t m_gt1 = 0, m_lt1 = 0, m_gt2 = 0, m_lt2 = 0;
   {
-    const sel_pair t1 = {(uint16_t)T1, (uint16_t)T1}, t2 = {(uint16_t)T2, (uint16_t)T2};
+    const uint32_t t1 = T1 | T1 << 16, t2 = T2 | T2 << 16;
 #pragma unroll
     for (int w = 0; w < KW; w += 8) {
       uint32_t gt1 = 0, lt1 = 0, gt2 = 0, lt2 = 0;   // bit 2 v: key 2 v, bit 16 + 2 v: key 2 v + 1
 #pragma unroll
       for (int v = 0; v < 8 && w + v < KW; ++v) {
-        const sel_pair k = __builtin_bit_cast(sel_pair, kw[w + v]);
+        const uint32_t k = kw[w + v];
         gt1 |= sel_above(k, t1) << (2 * v);
         lt1 |= sel_above(t1, k) << (2 * v);
         gt2 |= sel_above(k, t2) << (2 * v);

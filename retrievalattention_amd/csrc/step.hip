@@ -102,12 +102,13 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
     known.q = att_query_piece(A, blockIdx.x);
     known.lenA = att_steady_rows(A);
   };
-  if (SPLIT) ahead();
-  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, SPLIT ? KEEP_TABLES : KEEP_ALL>(S, blockIdx.x, kept);
+  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, SPLIT ? KEEP_TABLES : KEEP_ALL>(S, blockIdx.x, kept, [&] {
+    if (SPLIT) ahead();
+  });
   lds_barrier();
   if (!SPLIT) ahead();
   // (the same in all of the group's workgroups)
-  const bool one = SPLIT && known.lenA + sh_off[S.np] + S.es <= one_rows;
+  const bool one = SPLIT && __builtin_amdgcn_readfirstlane(known.lenA + sh_off[S.np]) + S.es <= one_rows;
   if (one) {
     A.S = 1;
     A.W_kv = A.W_one;
@@ -125,7 +126,10 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
 // ------------------------------------------------------------------------------------
 // select + attend, behind the scoring: the attention's workgroups of a group each make the group's selection and go on with its
 // tables in LDS.  The compute units that repeat it would wait for it otherwise; a launch, and the tables' way through memory, are
-// left out.  The query's pieces and the zone's length are requested ahead of the selection, and one of the workgroups stores its
+// left out.  The query's pieces and the zone's length are requested before the selection looks at anything (behind its own first
+// loads: in front of them, with a wait for the struct's words and a load per head's partials under a condition, steps took 17.6
+// instead of 17.15 us in the first of the shapes below, 44.5 / 43.6 in the second, 22.5 / 21.7 for 12 of 7 heads, 1856 in half,
+// 127.5 / 126.0 in the fourth), and one of the workgroups stores its
 // results when its rows are attended (a load's wait covers the stores in front of it): without both 19.0, 47.5 and 26.2 us in
 // the first, second and third of these steps (captured, 4 layers a graph; in launches of their own -> joined): 16 groups of 4
 // heads, 1024 clusters 21.0 -> 18.9; 32 of 4, 8192 48.8 -> 47.0; 12 of 7, 1920 27.5 -> 25.6; 64 of 8, 16384 139.9 -> 138.2; 8 of
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
 // clusters, 819 probes 85.9 -> 84.2; 12 of 7, 5760, 576 45.4 -> 43.7; 64 of 8, 8192, 819 157.4 -> 155.2).
 // ------------------------------------------------------------------------------------
 template <int NT, int E, int GSM, bool HALF, int SRC>
-__global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int4 m, SelectArgs S0,
+__global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int2 m, SelectArgs S0,
                                                                           AttendParams A0) {
   extern __shared__ __attribute__((aligned(16))) int sh_kept[];
   SelectArgs S = S0;
@@ -156,14 +160,17 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
   S.gs = A.gs = n[1];
   S.np = A.np = n[2];
   S.es = A.es = n[3];
-  S.ntiles = m[0];
-  A.S = m[1];
-  A.W_kv = m[2];
+  S.ntiles = m[0] & 0xffff;
+  A.S = m[0] >> 16;
+  A.W_kv = m[1];
   const int np = S.np, g = blockIdx.x;
   int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
   const SelectKept kept = {nullptr, est, off, start, ids, meta, select_scratch<NT>()};
-  const AttendKept known = {nullptr, est, off, start, att_query_piece(A, g), att_steady_rows(A)};
-  select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept);
+  AttendKept known = {nullptr, est, off, start};
+  select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept, [&] {
+    known.q = att_query_piece(A, g);
+    known.lenA = att_steady_rows(A);
+  });
   lds_barrier();
   if (NT > 64 * ATT_WAVES && threadIdx.x >= 64 * ATT_WAVES) return;
   attend_group<GSM, HALF, KEPT_TABLES>(A, g, blockIdx.y, known);
@@ -181,7 +188,7 @@ static void launch_select_attend(const SelectArgs& S, const AttendParams& A, int
                              : (half ? select_attend_kernel<NT, E, G16, true, SRC> : select_attend_kernel<NT, E, G16, false, SRC>);
   const size_t lds = (size_t)(4 + 3 * S.np + 1 + S.es) * sizeof(int);
   kernel<<<dim3(BG, A.S), NT, lds, stream>>>(ri_pack_ptrs(a, S.tile_max, S.tile_sum, S.mask),
-                                                         (ri_int4){S.nc, S.gs, S.np, S.es}, (ri_int4){S.ntiles, A.S, A.W_kv, 0}, S,
+                                                         (ri_int4){S.nc, S.gs, S.np, S.es}, (ri_int2){S.ntiles | A.S << 16, A.W_kv}, S,
                                                          A);
 }
 
