@@ -134,6 +134,11 @@ static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int e
   P.S = (int)per_group;
   P.W_kv = with_keys(per_group * ATT_WAVES);
   P.W_one = with_keys(ATT_WAVES);
+  const auto inverse = [](int64_t waves) { return ATT_INVERSE(max(waves, (int64_t)1)); };
+  P.inv_kv = inverse(P.W_kv);
+  P.inv_es = inverse(per_group * ATT_WAVES - P.W_kv);
+  P.inv_kv_one = inverse(P.W_one);
+  P.inv_es_one = inverse(ATT_WAVES - P.W_one);
 }
 
 static int flash_decoding_impl(const void* q, const void* k, const void* v, const void* weight,

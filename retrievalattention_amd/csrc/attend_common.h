@@ -175,6 +175,8 @@ struct AttendParams {
   int S;     // workgroups per group
   int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
   int W_one; // the same of one workgroup's waves, if it takes the whole group
+  uint32_t inv_kv, inv_es;           // ATT_INVERSE of the waves of either kind
+  uint32_t inv_kv_one, inv_es_one;   // and of one workgroup's
   int gs;
   float scale;
   // epilogue
@@ -185,10 +187,12 @@ struct AttendParams {
   int32_t* valid_lengths;    // [BG] or null: lenA + lenB(g)
 };
 
-// rows of a wave: the group's `total` rows are cut into `nwaves` runs of a multiple of 16 rows
-__device__ __forceinline__ void wave_rows(int total, int nwaves, int wid, int* r0, int* r1) {
-  int rpw = (total + nwaves - 1) / nwaves;
-  rpw = (rpw + 15) & ~15;
+// Rows of a wave: the group's `total` rows are cut into `nwaves` runs of a multiple of 16 rows.  inv: ATT_INVERSE(nwaves), made by
+// the host, because a division by what is not known when this is built is thirty instructions in front of a wave's first load.
+#define ATT_INVERSE(nwaves) ((uint32_t)((0x80000000u + (uint32_t)(nwaves) - 1u) / (uint32_t)(nwaves)))
+__device__ __forceinline__ void wave_rows(int total, int nwaves, uint32_t inv, int wid, int* r0, int* r1) {
+  const uint32_t n = ((uint32_t)(total + 15) >> 4) + nwaves - 1;   // (exact below 2^31 / nwaves, of which there are 512)
+  const int rpw = 16 * (int)(n < (1u << 22) ? (uint32_t)(((uint64_t)n * inv) >> 31) : n / (uint32_t)nwaves);
   *r0 = min(total, wid * rpw);
   *r1 = min(total, *r0 + rpw);
 }
@@ -528,8 +532,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
     // value = value sum, weight = cluster size, located through the id list.
     const bool est = !kv_wave;
     int r0, r1;
-    if (est) wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
-    else wave_rows(lenA + lenB, P.W_kv, wid, &r0, &r1);
+    if (est) wave_rows(P.es, W_es, P.inv_es, wid - P.W_kv, &r0, &r1);
+    else wave_rows(lenA + lenB, P.W_kv, P.inv_kv, wid, &r0, &r1);
     const uint16_t* qrow = &sh_q[n % GS_PAD][h * 8];
     const uint16_t* kA = P.kA + (size_t)g * P.strideA * RI_DIM;
     const uint16_t* vA = P.vA + (size_t)g * P.strideA * RI_DIM;
@@ -594,7 +598,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   } else {
     // ---------------- estimation rows with their logits at hand ----------------
     int r0, r1;
-    wave_rows(P.es, W_es, wid - P.W_kv, &r0, &r1);
+    wave_rows(P.es, W_es, P.inv_es, wid - P.W_kv, &r0, &r1);
     const int32_t* ids = P.est_ids + (size_t)g * P.es;
     const uint16_t* vs = P.value_sum + (size_t)g * P.nc * RI_DIM;
     const uint16_t* cs = P.csize + (size_t)g * P.nc;

@@ -112,6 +112,8 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   if (one) {
     A.S = 1;
     A.W_kv = A.W_one;
+    A.inv_kv = A.inv_kv_one;
+    A.inv_es = A.inv_es_one;
   }
   if (!one || blockIdx.y == 0)
     attend_group<GSM, HALF, SPLIT ? KEPT_LOGITS : KEPT_ALL>(A, blockIdx.x, SPLIT ? blockIdx.y : 0, known);
