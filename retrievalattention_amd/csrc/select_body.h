@@ -111,11 +111,11 @@ struct SelectKept {
   int* est;        // [es]
   int* off;        // [np + 1]
   int* start;      // [np]
-  int* ids;        // [np] KEEP_TABLES
-  int* meta;       // [4] KEEP_TABLES
+  int* ids;        // [np]
+  int* meta;       // [4]
   uint32_t* scratch;   // [SEL_SCRATCH<NT>] what the attention has not laid anything in yet
 };
-enum { KEEP_NONE, KEEP_TABLES, KEEP_ALL };
+enum { KEEP_NONE, KEEP_TABLES };
 
 // Bins of the rank search.  Scores are sums of at most sixteen probabilities: in bfloat16 (128 keys to an octave) a bin for
 // each of the 4094 keys up to that of 16, 2^-28 the lowest, finds a rank in one pass; the first bin and the last hold what lies
@@ -141,14 +141,13 @@ __device__ __forceinline__ uint32_t sel_above(uint32_t a, uint32_t b) {
   return m;
 }
 
-// GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: what the attention reads is left in K as well, with
-// KEEP_TABLES in place of memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
+// GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: the results are left in K in place of
+// memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
 // ahead(): what the caller wants on its way behind the selection's first loads.
 template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP, typename Ahead>
 __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K, Ahead&& ahead) {
   static_assert(KEEP == KEEP_NONE || SRC != SEL_SCORE || GSM <= 8, "the logits are in LDS");
-  static_assert(KEEP != KEEP_ALL || SRC == SEL_SCORE, "what is not kept is in memory");
-  constexpr bool STORE = KEEP != KEEP_TABLES;
+  constexpr bool STORE = !KEEP;
   constexpr int NW = NT / 64, IDS = NT * E;
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
   constexpr int BPT = SEL_SPAN / NT, FB = 1 << SEL_SHIFT;   // bins of a thread, fine bins
@@ -212,6 +211,11 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       const int r = lane & 15, h = lane >> 4;
       const uint16_t* cg = P.cent + (size_t)g * nc * RI_DIM;
       uint4 a[4][4], bq[4];
+      {
+        const uint16_t* p = P.q + ((size_t)g * gs + min(r, gs - 1)) * RI_DIM + h * 8;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) bq[kk] = ri_ld16(p + kk * 32);
+      }
       // tile t of this wave: rows [16 * (wave + NW * t), + 16), so that few clusters still occupy every wave; rows past
       // the last centroid and heads past gs read a valid row (never used)
 #pragma unroll
@@ -219,11 +223,6 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           a[t][i] = ri_ld16(cg + (size_t)min(16 * (wave + NW * t) + 4 * i + h, nc - 1) * RI_DIM + r * 8);
-      }
-      {
-        const uint16_t* p = P.q + ((size_t)g * gs + min(r, gs - 1)) * RI_DIM + h * 8;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) bq[kk] = ri_ld16(p + kk * 32);
       }
       ahead();
       __builtin_amdgcn_sched_barrier(0);   // every load is in flight before the first product
@@ -243,19 +242,25 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(ri_as_bf16x8(at[kk]), ri_as_bf16x8(bq[kk]), x, 0, 0, 0);
         acc[t] = x * P.scale;
       }
-      // softmax statistics: every wave's maximum and sum relative to it, folded by every lane for its head
+      // softmax statistics: every wave's maximum and sum relative to it, folded by every lane for its head.  (No branches: a
+      // row past the last centroid scores -inf and weighs 0; nc % 4 == 0, the four rows are valid together.)
       float lmax = -INFINITY, lsum = 0.f;
+      f32x4_t there[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        if (16 * (wave + NW * t) + 4 * h < nc)   // nc % 4 == 0: the four rows are valid together
+      for (int t = 0; t < 4; ++t) {
+        const bool in = 16 * (wave + NW * t) + 4 * h < nc;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) lmax = fmaxf(lmax, acc[t][i]);
+        for (int i = 0; i < 4; ++i) {
+          there[t][i] = in ? acc[t][i] : -INFINITY;
+          lmax = fmaxf(lmax, there[t][i]);
+        }
+      }
       lmax = ri_xor_max<32>(ri_xor_max<16>(lmax));
+      const float base = lmax == -INFINITY ? 0.f : lmax;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        if (16 * (wave + NW * t) + 4 * h < nc)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) lsum += __expf(acc[t][i] - lmax);
+        for (int i = 0; i < 4; ++i) lsum += __expf(there[t][i] - base);
       lsum = ri_xor_sum<32>(ri_xor_sum<16>(lsum));
       if (h == 0) {
         sh_a[wave][r] = lmax;
@@ -265,26 +270,30 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       // nothing, so the scores go through LDS to the thread that owns the cluster, which computes gs probabilities (8 groups
       // of 4 heads, 512 clusters with the sizes at hand: 7.9 -> 7.7 us, 256: 6.9 -> 6.6); with more heads the lanes that have
       // the scores compute sixteen each (8 groups of 12: 8.4, the other way 9.3).
-      float* const xs = KEEP ? K.logits : sh_x;   // [cluster][GSM]
-      if (OWN) {
+      float* const xs = KEEP ? K.logits : sh_x;   // [cluster][GSM], of as many clusters as there are threads
+      if (OWN && r < gs) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int c = 16 * (wave + NW * t) + 4 * h;
-          if (r < gs && c < nc)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xs[(c + i) * GSM + r] = acc[t][i];
-        }
+          for (int i = 0; i < 4; ++i) xs[(16 * (wave + NW * t) + 4 * h + i) * GSM + r] = acc[t][i];
       }
       sh_size[tid] = own_size;
       sh_row[tid] = own_row;
       lds_barrier();
-      float m = sh_a[0][r], z = 0.f;   // of head r
-#pragma unroll
-      for (int w = 1; w < NW; ++w) m = fmaxf(m, sh_a[w][r]);
+      float mw[NW], zw[NW], m, z = 0.f;   // of head r
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        const float mw = sh_a[w][r];
-        z += (mw == -INFINITY) ? 0.f : sh_b[w][r] * __expf(mw - m);   // a wave past the last centroid holds nothing
+        mw[w] = sh_a[w][r];
+        zw[w] = sh_b[w][r];
+      }
+      m = mw[0];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) m = fmaxf(m, mw[w]);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        float part = zw[w] * __expf(mw[w] - m);
+        asm("" : "+v"(part));   // (else each becomes a branch with its own wait)
+        z += (mw[w] == -INFINITY) ? 0.f : part;   // a wave past the last centroid holds nothing
       }
       const float iz = 1.0f / z;
       d[0] = 0.f;
@@ -297,12 +306,15 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
         }
 #pragma unroll
         for (int j = 0; j < GSM; ++j) {
-          if (j >= gs) break;   // uniform
           const float mj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), j));
           const float izj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iz), j));
-          d[0] += ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[j]) - mj) * izj);
-          if (STORE && cbeg < nc) P.logits[((size_t)g * gs + j) * nc + cbeg] = x[j];
+          const float p = ri_round_e16<HALF>(__expf(ri_round_e16<HALF>(x[j]) - mj) * izj);
+          d[0] += j < gs ? p : 0.f;
         }
+        if (STORE && cbeg < nc)
+#pragma unroll
+          for (int j = 0; j < GSM; ++j)
+            if (j < gs) P.logits[((size_t)g * gs + j) * nc + cbeg] = x[j];
       } else {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -368,6 +380,8 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
         }
       }
     }
+    // (looked at here: the compiler compares where it loads, which is a wait in front of every other load)
+    if (SRC == SEL_SCORE) asm volatile("" : "+v"(mk[0]));
     uint16_t bits[E + 1] = {};
 #pragma unroll
     for (int i = 0; i < E; ++i) {

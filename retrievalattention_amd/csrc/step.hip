@@ -62,18 +62,21 @@ __device__ __forceinline__ void store_selection(const SelectArgs& S, int g, cons
 // With up to 512 clusters the selection is one workgroup per group that scores for itself: as one kernel with the attention
 // the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
 // host as well.  What bounds it is the chain of either half on one compute unit.  8 groups of 4 heads, 512 clusters, 331
-// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  110060 bytes of LDS (119532 with 8 heads): one
+// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  103564 bytes of LDS (113036 with 8 heads): one
 // workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.
 // SPLIT: several workgroups per group, which all make the same selection and attend a part of the rows each (see
-// select_attend_kernel): with the query and the zone's length requested ahead of the selection and its results stored behind
+// select_attend_kernel): with the query and the zone's length requested behind the first loads and the results stored behind
 // the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 523 / 843 / 1099 rows:
 // 15.0 / 17.3 / 19.8 / 22.7 us with one workgroup, 14.6 / 14.6 / 14.8 / 16.5 with several (16.3 .. 18.8 in two launches); the
 // retrieval of 10 % of the clusters, 8 groups of 8 heads 20.7 -> 19.0 (two launches -> SPLIT), 16 of 4 20.8 -> 19.4, 128 of 8
 // 33.6 -> 31.7.  step_route.h says which step takes which form.  The rows that the clusters hold, and the zone's in a captured
 // step, are known behind the selection only: where they turn out to be few, one workgroup attends them all and hands no partial
 // over, and another stores the results (captured, 8 groups of 1 head, 4000 tokens 14.6 -> 13.4 us, 1 of 4, 8192 15.0 -> 14.5, 8 of
-// 8, 8192 16.3 -> 16.1, 128 of 8, 8192 23.3 -> 22.4).  With one workgroup the query's pieces ahead of the selection cost more
-// than they save: 8 groups of 4 heads 13.3 -> 13.15, 32 of 4, 3000 tokens 12.3 -> 12.1 without.
+// 8, 8192 16.3 -> 16.1, 128 of 8, 8192 23.3 -> 22.4).
+// The scoring half is bound by its instructions and waits, not by the centroids' bytes (a quarter of them takes as long): with
+// its own statistics and those of the eight waves made without branches, the clusters' masks not looked at in front of the other
+// loads, and the results stored behind the attention by one workgroup as by several, captured layers took 16.05 -> 15.5 us (8
+// groups of 4 heads, 8192 tokens), 17.3 -> 16.4 (8 of 8), 16.55 -> 15.95 (16 of 4), 17.35 -> 16.7 (32 of 4, 8000).
 // ------------------------------------------------------------------------------------
 // (what the first loads want stands before the structs: in registers at the start; 64 groups of 8 heads 15.3 -> 15.0 us, 8 of 4
 // the same)
@@ -83,7 +86,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   static_assert(64 * ATT_WAVES == STEP_CLUSTERS, "a cluster per thread");
   __shared__ __attribute__((aligned(16))) float sh_logits[STEP_CLUSTERS * GSM];
   static_assert(__alignof__(sh_logits) == 16, "read four heads at a time");
-  __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS], sh_ids[SPLIT ? STEP_CLUSTERS : 1],
+  __shared__ int sh_est[STEP_CLUSTERS], sh_off[STEP_CLUSTERS + 1], sh_start[STEP_CLUSTERS], sh_ids[STEP_CLUSTERS],
       sh_meta[4];
   SelectArgs S = S0;
   AttendParams A = A0;
@@ -98,15 +101,11 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.scale = A.scale = scale;
   const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta, select_scratch<STEP_CLUSTERS>()};
   AttendKept known = {sh_logits, sh_est, sh_off, sh_start};
-  const auto ahead = [&]() {
+  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, KEEP_TABLES>(S, blockIdx.x, kept, [&] {
     known.q = att_query_piece(A, blockIdx.x);
     known.lenA = att_steady_rows(A);
-  };
-  select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, SPLIT ? KEEP_TABLES : KEEP_ALL>(S, blockIdx.x, kept, [&] {
-    if (SPLIT) ahead();
   });
   lds_barrier();
-  if (!SPLIT) ahead();
   // (the same in all of the group's workgroups)
   const bool one = SPLIT && __builtin_amdgcn_readfirstlane(known.lenA + sh_off[S.np]) + S.es <= one_rows;
   if (one) {
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   }
   if (!one || blockIdx.y == 0)
     attend_group<GSM, HALF, SPLIT ? KEPT_LOGITS : KEPT_ALL>(A, blockIdx.x, SPLIT ? blockIdx.y : 0, known);
-  if (SPLIT && blockIdx.y == (one && gridDim.y > 1 ? 1 : 0)) {
+  if (blockIdx.y == (one && gridDim.y > 1 ? 1 : 0)) {
     store_selection(S, blockIdx.x, kept);
     const int nc = S.nc;
     for (int j = 0; j < S.gs; ++j)
