@@ -375,15 +375,14 @@ __device__ __forceinline__ void attend_rows(WaveState<GS_PAD>& st, const WaveLds
 // The rank tables of the retrieval zone (np + 1 token offsets, np first rows) live in dynamic LDS, sized by
 // the launch, so that any number of probes the selection accepts can be attended.
 // HALF: q, K, V, value sums, cluster sizes, weights and outputs are IEEE half instead of bfloat16.
-// KEPT: the workgroup has just made the selection, whose tables and ids are in LDS (K), from KEPT_LOGITS on the logits too.
-// KEPT_ALL: it has the whole group.
+// KEPT: the workgroup has just made the selection, whose tables and ids are in LDS (K), from KEPT_LOGITS on the logits too, and
+// has laid down what att_clear and att_put_query do.  KEPT_ALL: it has the whole group.
 enum { KEPT_NONE, KEPT_TABLES, KEPT_LOGITS, KEPT_ALL };
 struct AttendKept {
   const float* logits;   // [nc][GS_PAD]
   const int* est;        // [es]
   int* off;              // [np + 1]
   int* start;            // [np]
-  uint4 q;               // this thread's piece of the query (att_query_piece), requested ahead of the selection
   int lenA;              // the steady zone's rows
 };
 
@@ -392,6 +391,35 @@ __device__ __forceinline__ uint16_t (*att_tiles())[16 * ATT_VT_STRIDE] {
   __shared__ __attribute__((aligned(16))) uint16_t sh_vt[ATT_WAVES][16 * ATT_VT_STRIDE];
   static_assert(__alignof__(sh_vt) == 16, "pieces of 16 bytes");
   return sh_vt;
+}
+
+// What else a workgroup lays down in LDS before its rows: probabilities (of heads that do not exist they stay zero) and factors
+// (theirs must not scale by garbage), a wave's own, and the query, read again per chunk so that the registers go to the loads.
+template <int GS_PAD>
+struct AttendLds {
+  __attribute__((aligned(16))) uint16_t pb[ATT_WAVES][16 * 16];
+  __attribute__((aligned(16))) uint16_t q[GS_PAD][RI_DIM];
+  float al[ATT_WAVES][16];
+};
+template <int GS_PAD>
+__device__ __forceinline__ AttendLds<GS_PAD>& att_lds() {
+  __shared__ __attribute__((aligned(16))) AttendLds<GS_PAD> sh;
+  return sh;
+}
+template <int GS_PAD>
+__device__ __forceinline__ void att_clear() {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wave >= ATT_WAVES) return;
+  AttendLds<GS_PAD>& sh = att_lds<GS_PAD>();
+  reinterpret_cast<uint2*>(sh.pb[wave])[lane] = make_uint2(0u, 0u);
+  if (lane < 16) sh.al[wave][lane] = 1.f;
+}
+// row m of the MFMA holds head m % GS_PAD, zero if >= gs
+template <int GS_PAD>
+__device__ __forceinline__ void att_put_query(uint4 piece_of, int gs) {
+  static_assert(GS_PAD * (RI_DIM / 8) <= 64 * ATT_WAVES, "one piece of the query per thread");
+  const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
+  if (head < GS_PAD) *reinterpret_cast<uint4*>(&att_lds<GS_PAD>().q[head][piece * 8]) = head < gs ? piece_of : ri_zero16();
 }
 
 // piece threadIdx.x % 16 of the query of head threadIdx.x / 16
@@ -440,8 +468,9 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   constexpr int NH = GS_PAD / 4;
   constexpr int NT = 64 * NW;
   uint16_t (*const sh_vt)[16 * ATT_VT_STRIDE] = att_tiles();
-  __shared__ __attribute__((aligned(16))) uint16_t sh_pb[NW][16 * 16];
-  __shared__ float sh_al[NW][16];
+  auto& sh_pb = att_lds<GS_PAD>().pb;
+  auto& sh_al = att_lds<GS_PAD>().al;
+  auto& sh_q = att_lds<GS_PAD>().q;
   __shared__ float sh_m[NW][GS_PAD];
   __shared__ float sh_l[NW][GS_PAD];
   // the waves' numerators for the merge: up to eight heads they are laid over the wave's own value tile (dead once its
@@ -453,7 +482,6 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   auto acc_of = [&](int w) -> float* {
     return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : &sh_acc_own[ACC_OVER_VT ? 0 : w][0][0];
   };
-  __shared__ __attribute__((aligned(16))) uint16_t sh_q[GS_PAD][RI_DIM];
   __shared__ int sh_desc[NW][ATT_DESC_MAX];
   __shared__ float sh_w[NW][ATT_DESC_MAX];
   extern __shared__ __attribute__((aligned(16))) int sh_tab[];
@@ -472,9 +500,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   for (int dt = 0; dt < 8; ++dt) st.acc[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 
   const WaveLds sh = {sh_vt[wave], sh_pb[wave], sh_al[wave], sh_desc[wave], sh_w[wave]};
-  // P rows of heads that do not exist stay zero; alpha of such heads must not scale by garbage
-  for (int i = lane; i < 16 * 16 / 2; i += 64) reinterpret_cast<uint32_t*>(sh.pb)[i] = 0u;
-  if (lane < 16) sh.al[lane] = 1.f;
+  if (!KEPT) att_clear<GS_PAD>();
   const int lenB = KEPT ? K.off[P.np] : P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
   const int lenA = __builtin_amdgcn_readfirstlane(KEPT ? K.lenA : att_steady_rows(P));
 
@@ -484,8 +510,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   const int W_es = S * NW - P.W_kv;
 
   // ---------------- prologue: query and rank tables to LDS ----------------
-  if (kv_wg || P.est_cent) {
-    const bool tab = !KEPT && kv_wg && P.ret_off != nullptr;
+  if (!KEPT && (kv_wg || P.est_cent)) {
+    const bool tab = kv_wg && P.ret_off != nullptr;
     // every global load of the prologue is requested before the first of them is consumed
     // (up to 1023 probes the table entries pass through registers, TAB_U per thread; longer tables are
     // staged by a plain loop after the query)
@@ -500,15 +526,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
         t_st[u] = P.ret_start[(size_t)g * P.np + min(i, P.np - 1)];
       }
     }
-    // A operand: query heads through LDS (read again per chunk: registers go to the loads);
-    // row m of the MFMA holds head m % GS_PAD, zero if >= gs
-    static_assert(GS_PAD * (RI_DIM / 8) <= NT, "one piece of the query per thread");
-    {
-      const int head = threadIdx.x / (RI_DIM / 8), piece = threadIdx.x % (RI_DIM / 8);
-      uint4 qv = KEPT ? K.q : att_query_piece(P, g);
-      if (head >= gs) qv = ri_zero16();
-      if (head < GS_PAD) *reinterpret_cast<uint4*>(&sh_q[head][piece * 8]) = qv;
-    }
+    att_put_query<GS_PAD>(att_query_piece(P, g), gs);
     if (tab_fast) {
 #pragma unroll
       for (int u = 0; u < TAB_U; ++u) {
@@ -522,8 +540,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
         if (i < P.np) sh_rst[i] = P.ret_start[(size_t)g * P.np + i];
       }
     }
-    if (KEPT) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (the selection's stores stay in flight)
-    else __syncthreads();
+    __syncthreads();
   }
 
   if (kv_wave || (!KEPT && P.est_cent)) {

@@ -101,10 +101,13 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.scale = A.scale = scale;
   const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta, select_scratch<STEP_CLUSTERS>()};
   AttendKept known = {sh_logits, sh_est, sh_off, sh_start};
+  uint4 query;
   select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, KEEP_TABLES>(S, blockIdx.x, kept, [&] {
-    known.q = att_query_piece(A, blockIdx.x);
+    query = att_query_piece(A, blockIdx.x);
     known.lenA = att_steady_rows(A);
+    att_clear<GSM>();
   });
+  att_put_query<GSM>(query, S.gs);
   lds_barrier();
   // (the same in all of the group's workgroups)
   const bool one = SPLIT && __builtin_amdgcn_readfirstlane(known.lenA + sh_off[S.np]) + S.es <= one_rows;
@@ -168,10 +171,13 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
   int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
   const SelectKept kept = {nullptr, est, off, start, ids, meta, select_scratch<NT>()};
   AttendKept known = {nullptr, est, off, start};
+  uint4 query;
   select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept, [&] {
-    known.q = att_query_piece(A, g);
+    query = att_query_piece(A, g);
     known.lenA = att_steady_rows(A);
+    att_clear<GSM>();
   });
+  att_put_query<GSM>(query, S.gs);
   lds_barrier();
   if (NT > 64 * ATT_WAVES && threadIdx.x >= 64 * ATT_WAVES) return;
   attend_group<GSM, HALF, KEPT_TABLES>(A, g, blockIdx.y, known);
