@@ -462,7 +462,7 @@ int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, int32_t* offs
 /* `updates` times ri_kmeans_assign and the normalised update of that assignment, then (last != 0) one more assignment:
  * the same centroids and the same assign [P, N] bit for bit.  Between the passes the library keeps, in the workspace, what
  * a token's best and second best scores were and which centroids have moved, and scores again only where the best can have
- * changed.  centroids [P, nc, 128] as the clustering starts from them (nc % 32 == 0); workspace:
+ * changed; what `assign` holds between the passes is the library's.  centroids [P, nc, 128] as the clustering starts from them (nc % 32 == 0); workspace:
  * ri_kmeans_iterate_workspace_bytes, no initialisation needed. */
 size_t ri_kmeans_iterate_workspace_bytes(int P, int N, int nc);
 int ri_kmeans_iterate(const void* data, void* centroids, int32_t* assign, int P, int N, int nc, int seg, int64_t head_rows,

@@ -464,12 +464,21 @@ struct KmScan {
   }
 };
 
+// Between the passes of ri_kmeans_iterate a problem's assignment lies as 16-bit words in the first half of its row of `assign`,
+// where km_direct_kernel takes it from (narrow; figures there).
+#define KM_NARROW 4   // beside the shift of km_grid in the kernels' `shape`
+__device__ __forceinline__ void km_put_place(int32_t* row, int tok, int place, int narrow) {
+  if (narrow) reinterpret_cast<uint16_t*>(row)[tok] = (uint16_t)place;
+  else row[tok] = place;
+}
+
 template <int TT, int CT, int W, int NB, bool HALF>
 __global__ __launch_bounds__(W * 64) void km_assign_kernel(const uint16_t* __restrict__ data, const uint16_t* __restrict__ cent,
                                                            int32_t* __restrict__ assign, int N, int nc, int seg,
-                                                           int64_t head_rows, int sh) {
+                                                           int64_t head_rows, int shape) {
   typedef KmScan<TT, CT, W, NB, HALF, false> Scan;
   __shared__ __attribute__((aligned(1024))) uint16_t sh_c[NB][CT][RI_DIM];
+  const int sh = shape & 3;
   const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
   Scan s(sh_c, cent + (size_t)p * nc * RI_DIM, nc);
   const int t0 = (blockIdx.x >> sh) * Scan::TOKENS + s.wave * (32 * TT);
@@ -484,7 +493,7 @@ __global__ __launch_bounds__(W * 64) void km_assign_kernel(const uint16_t* __res
     int place;
     s.merged(tt, top, place, second);
     const int tok = t0 + tt * 32 + s.r;
-    if (s.hh == 0 && tok < N) assign[(size_t)p * N + tok] = place;
+    if (s.hh == 0 && tok < N) km_put_place(assign + (size_t)p * N, tok, place, shape & KM_NARROW);
   }
 }
 
@@ -542,11 +551,12 @@ __device__ __forceinline__ int km_first_of16(const f32x16_t& x, float m, float b
 template <bool HALF>
 __global__ __launch_bounds__(512) void km_assign_few_kernel(const uint16_t* __restrict__ data, const uint16_t* __restrict__ cent,
                                                             int32_t* __restrict__ assign, int N, int nc, int seg,
-                                                            int64_t head_rows, int sh) {
+                                                            int64_t head_rows, int shape) {
   constexpr int CT = 128, AHEAD = 8;
   typedef KmScan<1, CT, 8, 2, HALF, false> Scan;
   static_assert(Scan::TURN && Scan::WR == 16, "room for sixteen tokens of a wave");
   __shared__ __attribute__((aligned(1024))) uint16_t sh_c[2][CT][RI_DIM];
+  const int sh = shape & 3;
   const int p = (blockIdx.y << sh) + (blockIdx.x & ((1 << sh) - 1));
   Scan s(sh_c, cent + (size_t)p * nc * RI_DIM, nc);
   const int t0 = (blockIdx.x >> sh) * Scan::TOKENS + s.wave * 32, r = s.r, hh = s.hh;
@@ -632,7 +642,7 @@ __global__ __launch_bounds__(512) void km_assign_few_kernel(const uint16_t* __re
   const int other_at = __float_as_int(km_other(__int_as_float(at), hh));
   if (other > best || (other == best && other_at < at)) at = other_at;
   const int tok = t0 + r;
-  if (hh == 0 && tok < N) assign[(size_t)p * N + tok] = at;
+  if (hh == 0 && tok < N) km_put_place(assign + (size_t)p * N, tok, at, shape & KM_NARROW);
 }
 
 // A pass of a clustering that knows the pass before (KmBounds), grid (ceil(N / TOKENS), P).  The clusters that no token has
@@ -1545,15 +1555,20 @@ __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmSto
 // grid km_grid(ceil(nc / CPW), P), eight waves: a workgroup owns CPW consecutive clusters.  Every wave takes a contiguous run of
 // the problem's tokens, compacts those of the workgroup's clusters into LDS (in token order), counts them, and after a
 // scan in (cluster, wave) order scatters them to the workgroup's list in LDS, ranking equal clusters inside a round of 64
-// with ballots: the stable order of the list kernels, hence the same sums.  The run is read four tokens to a lane, up to
+// with ballots: the stable order of the list kernels, hence the same sums.  The run is read four tokens to a lane (eight in 16 bits), up to
 // 1024 requested at once; a token costs three instructions (its cluster in a byte, all others' flagged), positions come
 // from one wave scan per 512 and only the few hits are looped over.  A ballot, a rank and a branch for every 64 tokens
 // were most of a late update: 8 x 8192 tokens, 512 clusters 8.2 -> 7.5 us, 4 x 15000, 928 clusters 10.8 -> 9.2, 1 x 16384
 // 8.5 -> 6.9, 128 x 8192 52.0 -> 49.8.  Then a wave sums whole clusters of at most
 // KM_BLK rows; the blocks of longer ones are spread over the waves and folded in block order.
-// Reading all assignments of the problem per workgroup (4 N bytes) is what the split costs: 32 KB at 8192 tokens, about a
-// microsecond.  128 x 8192 tokens, 512 clusters each: 50 us, bound by reading the keys, against 13 + 70 + 5 us of list
-// sort, sums and fold; 8 x 8192: 7.5 us against 12 + 11 + 4.5.
+// Reading all assignments of the problem per workgroup is what the split costs: 32 KB at 8192 tokens in 32 bits, a third of
+// a late update's time.  NARROW: an earlier pass left them as 16-bit words (km_put_place); twice eight tokens to a lane, two
+// words to an instruction, one scan per 1024.  Loads are made without a condition, what they bring too much is put out
+// afterwards (behind a condition each waited for the one before), and what the rows' address takes, a division and four
+// arguments, is done while they are on their way (after the lists it took 400 ns).  Late updates by the two, us: 8 x 8192 tokens, 512
+// clusters 7.1 -> 5.8, 24 x 8119 half 12.7 -> 11.5, 128 x 8192 49.7 -> 47.0 (50.5 in 32 bits).
+// 128 x 8192 tokens, 512 clusters each: 47 us, bound by reading the keys, against 13 + 70 + 5 us of list
+// sort, sums and fold; 8 x 8192: 5.8 us against 12 + 11 + 4.5.
 // counts / offsets / members (CSR, as km_sort_small_kernel writes them) only when asked for, and then alone if there is
 // no `cent`: the last pass of a prefill, whose means come with the stores (8 x 8192 tokens, whole prefill 367 -> 363 us).
 // ------------------------------------------------------------------------------------
@@ -1645,22 +1660,27 @@ __device__ __forceinline__ void km_sum_listed(__amdgpu_buffer_rsrc_t rows, uint3
 
 // four consecutive assignments; a problem's first one lies on four bytes only
 typedef int32_t km_quad __attribute__((ext_vector_type(4), aligned(4)));
+// eight consecutive ones in 16 bits (a problem's row of `assign` starts on four bytes)
+typedef uint32_t km_eight __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t km_u16x2 __attribute__((ext_vector_type(2)));
 // tokens of a wave's run: whole quads of 64 lanes
 __host__ __device__ constexpr int km_direct_run(int N) {
   return (N + KM_DIRECT_WAVES * 256 - 1) / (KM_DIRECT_WAVES * 256) * 256;
 }
 
-template <bool HALF, int CPW>
+template <bool HALF, int CPW, bool NARROW>
 __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
-    const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent,
-    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int seg,
-    int64_t head_rows, int normalize, int sh) {
+    const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent, int N, int nc,
+    int shape, int seg, int64_t head_rows, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ listed) {
   constexpr int NW = KM_DIRECT_WAVES, E = CPW * NW / 64;   // E: (cluster, wave) counters per lane
   static_assert((CPW & (CPW - 1)) == 0 && CPW * NW % 64 == 0 && CPW <= 64, "counters dealt to the lanes, a cluster in a byte");
   __shared__ int32_t sh_run[CPW * NW], sh_at[NW][CPW], sh_off[CPW + 1], sh_below[NW];
   extern __shared__ __attribute__((aligned(16))) uint32_t sh_buf[];   // NW * run_len words: compacted tokens, later block sums
+  int32_t* const members = NARROW ? nullptr : listed;
+  const int sh = shape & 3, normalize = shape >> 2 & 1;
   // (last problem first: its keys are what the assignment pass has just left in the memory-side cache)
-  const int p = ((gridDim.y - 1 - blockIdx.y) << sh) + (blockIdx.x & ((1 << sh) - 1)), c0 = (blockIdx.x >> sh) * CPW;
+  const int p = (((shape >> 3) - (int)blockIdx.y) << sh) + (blockIdx.x & ((1 << sh) - 1)), c0 = (blockIdx.x >> sh) * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int run_len = km_direct_run(N);
   uint32_t* const mine = sh_buf + wave * run_len;
@@ -1670,56 +1690,106 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
   const int32_t* as = assign + (size_t)p * N;
   const int t1 = min((wave + 1) * run_len, N);
   int cnt = 0, below = 0;   // tokens of this wave in the workgroup's clusters, (per lane) in lower ones
-  for (int t0 = wave * run_len; t0 < t1; t0 += 1024) {
-    // four quads of consecutive tokens per lane, all requested before the first is looked at
-    km_quad a[4];
+  const auto take = [&](uint32_t c, int token, int at) {
+    mine[at] = c << 16 | (uint32_t)token;
+    atomicAdd(&sh_run[c * NW + wave], 1);
+  };
+  size_t row0;
+  const auto find_rows = [&]() {   // a division, while the assignments are on their way
+    __builtin_amdgcn_sched_barrier(0);
+    int problem = p, segments = seg;
+    asm volatile("" : "+s"(problem), "+s"(segments));   // (else it moves ahead of them)
+    row0 = km_row0(problem, segments, head_rows, N);
+    asm volatile("" : "+s"(row0));
+  };
+  int t0 = wave * run_len;
+  do {   // (once for a wave without tokens, too)
+    if constexpr (NARROW) {
+      // twice eight consecutive tokens per lane, without a condition: what lies past the problem's N words is still its own row
+      km_eight a[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = t0 + q * 256 + lane * 4;
-      if (t0 + q * 256 + 256 <= t1) {
-        a[q] = *reinterpret_cast<const km_quad*>(as + i);
-      } else if (t0 + q * 256 < t1) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int x = as[min(i + j, N - 1)];
-          a[q][j] = i + j < t1 ? x : 0x7fffffff;
-        }
-      } else {
-        a[q] = km_quad(0x7fffffff);
-      }
-    }
-#pragma unroll
-    for (int q0 = 0; q0 < 4; q0 += 2) {
-      if (t0 + q0 * 256 >= t1) break;
-      uint32_t loc[2], hit[2], at[2];   // a byte per token: its cluster from c0 on, CPW for all others
+      for (int q = 0; q < 2; ++q)
+        a[q] = *reinterpret_cast<const km_eight*>(reinterpret_cast<const uint16_t*>(as) + min(t0 + q * 512 + lane * 8, 2 * N - 8));
+      find_rows();
+      uint64_t loc[2], hit[2];   // a byte per token: its cluster from c0 on, CPW for all others
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        loc[q] = 0;
+        uint32_t d[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const uint32_t d = (uint32_t)(a[q0 + q][j] - c0);
-          loc[q] |= min(d, (uint32_t)CPW) << (8 * j);
-          if (members) below += (int)(d >> 31);
+          const uint32_t w = a[q][j];   // (a cast of the element itself takes the first one's)
+          const km_u16x2 x = __builtin_bit_cast(km_u16x2, w) - km_u16x2((uint16_t)c0);
+          d[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(x, km_u16x2((uint16_t)CPW)));
         }
-        hit[q] = ~loc[q] & (uint32_t)CPW * 0x01010101u;
+        loc[q] = (uint64_t)__builtin_amdgcn_perm(d[3], d[2], 0x06040200) << 32 | __builtin_amdgcn_perm(d[1], d[0], 0x06040200);
+        const int left = t1 - (t0 + q * 512 + lane * 8);
+        if (t0 + q * 512 + 512 > t1)   // (uniform)
+          loc[q] = left >= 8 ? loc[q] : loc[q] | (uint64_t)CPW * 0x0101010101010101ull << 8 * max(left, 0);
+        hit[q] = ~loc[q] & (uint64_t)CPW * 0x0101010101010101ull;
       }
-      // positions of a lane's first hits in both quads, in one scan (at most 256 each)
-      const uint32_t n = (uint32_t)__popc(hit[0]) | (uint32_t)__popc(hit[1]) << 16, inc = ri_wave_incl_scan(n);
+      // positions of a lane's first hits in both eights, in one scan (at most 512 each)
+      const uint32_t n = (uint32_t)__popcll(hit[0]) | (uint32_t)__popcll(hit[1]) << 16, inc = ri_wave_incl_scan(n);
       const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
-      at[0] = cnt + ((inc - n) & 0xffffu);
-      at[1] = cnt + (int)(all & 0xffffu) + ((inc - n) >> 16);
+      int at[2] = {cnt + (int)((inc - n) & 0xffffu), cnt + (int)(all & 0xffffu) + (int)((inc - n) >> 16)};
       cnt += (int)(all & 0xffffu) + (int)(all >> 16);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        for (uint32_t h = hit[q]; h; h &= h - 1) {
-          const int j = (__ffs((int)h) - 1) >> 3;
-          const uint32_t c = loc[q] >> (8 * j) & (uint32_t)(CPW - 1);
-          mine[at[q]++] = c << 16 | (uint32_t)(t0 + (q0 + q) * 256 + lane * 4 + j);
-          atomicAdd(&sh_run[c * NW + wave], 1);
+      for (int q = 0; q < 2; ++q)
+        for (uint64_t h = hit[q]; h; h &= h - 1) {
+          const int j = (__ffsll((long long)h) - 1) >> 3;
+          take((uint32_t)(loc[q] >> (8 * j)) & (uint32_t)(CPW - 1), t0 + q * 512 + lane * 8 + j, at[q]++);
         }
+    } else {
+      // four quads of consecutive tokens per lane; the one that would pass the problem's end begins at its last four tokens
+      km_quad a[4];
+      if (N >= 4) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const km_quad*>(as + min(t0 + q * 256 + lane * 4, N - 4));
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a[q][j] = as[min(j, N - 1)];
+      }
+      find_rows();
+#pragma unroll
+      for (int q0 = 0; q0 < 4; q0 += 2) {
+        if (t0 + q0 * 256 >= t1) break;
+        uint32_t loc[2], hit[2], at[2];
+        int first[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int i = t0 + (q0 + q) * 256 + lane * 4;
+          first[q] = min(i, max(N - 4, 0));
+          if (t0 + (q0 + q) * 256 + 256 > t1) {   // (uniform)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (first[q] + j < i || first[q] + j >= t1) a[q0 + q][j] = 0x7fffffff;
+          }
+          loc[q] = 0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t d = (uint32_t)(a[q0 + q][j] - c0);
+            loc[q] |= min(d, (uint32_t)CPW) << (8 * j);
+            if (members) below += (int)(d >> 31);
+          }
+          hit[q] = ~loc[q] & (uint32_t)CPW * 0x01010101u;
+        }
+        // positions of a lane's first hits in both quads, in one scan (at most 256 each)
+        const uint32_t n = (uint32_t)__popc(hit[0]) | (uint32_t)__popc(hit[1]) << 16, inc = ri_wave_incl_scan(n);
+        const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        at[0] = cnt + ((inc - n) & 0xffffu);
+        at[1] = cnt + (int)(all & 0xffffu) + ((inc - n) >> 16);
+        cnt += (int)(all & 0xffffu) + (int)(all >> 16);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          for (uint32_t h = hit[q]; h; h &= h - 1) {
+            const int j = (__ffs((int)h) - 1) >> 3;
+            take(loc[q] >> (8 * j) & (uint32_t)(CPW - 1), first[q] + j, at[q]++);
+          }
       }
     }
-  }
+    t0 += 1024;
+  } while (t0 < t1);
   if (members) {
     below = (int)ri_wave_incl_scan((uint32_t)below);
     if (lane == 63) sh_below[wave] = below;
@@ -1775,7 +1845,7 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
     if (!cent) return;
   }
   const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(rows + km_row0(p, seg, head_rows, N) * RI_DIM), 0, N * RI_DIM * 2, 0x00020000);
+      const_cast<uint16_t*>(rows + row0 * RI_DIM), 0, N * RI_DIM * 2, 0x00020000);
   uint32_t* op = reinterpret_cast<uint32_t*>(cent + ((size_t)p * nc + c0) * RI_DIM) + lane;
   // Work items for the waves in turn: the blocks of the long lists first (early iterations have lists of thousands), then
   // the short lists; no barrier between them.  Block sums go to LDS: the compacted tokens are dead, and lists longer than
@@ -1785,8 +1855,12 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
   float* const part = reinterpret_cast<float*>(sh_buf);
   const int my_o = sh_off[min(lane, CPW - 1)], my_s = lane < CPW ? sh_off[min(lane, CPW - 1) + 1] - my_o : 0;
   const int my_nb = my_s > KM_DIRECT_SHORT ? (my_s + KM_BLK - 1) / KM_BLK : 0;
-  const int nb_incl = (int)ri_wave_incl_scan((uint32_t)my_nb);
-  const int nblocks = __builtin_amdgcn_readlane(nb_incl, 63);
+  uint64_t big = __builtin_amdgcn_ballot_w64(my_nb > 0);
+  int nb_incl = 0, nblocks = 0;
+  if (big) {
+    nb_incl = (int)ri_wave_incl_scan((uint32_t)my_nb);
+    nblocks = __builtin_amdgcn_readlane(nb_incl, 63);
+  }
   const int halves = 2 * nblocks <= NW ? 2 : 1, items = halves * nblocks;
   for (int k = wave; k < items; k += NW) {
     const int blk = halves == 2 ? k >> 1 : k;
@@ -1813,7 +1887,6 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
   }
   if (nblocks == 0) return;   // uniform over the workgroup
   __syncthreads();
-  uint64_t big = __builtin_amdgcn_ballot_w64(my_nb > 0);
   for (int i = 0; big; big &= big - 1, ++i) {   // a wave folds every eighth long list in block order
     if ((i & (NW - 1)) != wave) continue;
     const int c = __ffsll((long long)big) - 1;
@@ -1889,10 +1962,11 @@ static int km_assign_args(const void* data, const void* centroids, const int32_t
 
 template <bool HALF>
 static void km_assign_launch(const void* data, const void* centroids, int32_t* assign, int P, int N, int nc, int seg,
-                             int64_t head_rows, hipStream_t stream) {
+                             int64_t head_rows, bool narrow, hipStream_t stream) {
+  const int shape = km_together(P) | (narrow ? KM_NARROW : 0);
 #define KM_ASSIGN_LAUNCH(TT, CT, W, NB)                                                                                  \
   km_assign_kernel<TT, CT, W, NB, HALF><<<km_grid((N + W * 32 * TT - 1) / (W * 32 * TT), P), W * 64, 0, stream>>>( \
-      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P))
+      (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, shape)
   // Long launches: two columns, 128 registers and 32 KB of LDS, four workgroups to a compute unit; the load of one's tokens runs
   // under the others' products.  (8 x 131072 tokens, 8192 centroids: 1393 us, four columns in eight waves 1397; 8 x 96000, 3072:
   // 419 and 435; 128 x 8192, 512: 118 and 132.)  Short ones by how their 256-token pieces fall on 256 compute units: a last
@@ -1912,7 +1986,7 @@ static void km_assign_launch(const void* data, const void* centroids, int32_t* a
   const long long pieces = (long long)P * ((N + 255) / 256);
   if (pieces > 128 && nc >= 256 && pieces + nc / 64 <= 224)
     km_assign_few_kernel<HALF><<<km_grid((N + 255) / 256, P), 512, 0, stream>>>(
-        (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, km_together(P));
+        (const uint16_t*)data, (const uint16_t*)centroids, assign, N, nc, seg, head_rows, shape);
   else if (pieces > 1280) KM_ASSIGN_LAUNCH(2, 32, 4, 4);
   else if ((pieces - 1) % 256 >= 128 && (nc >= 256 || pieces <= 768)) KM_ASSIGN_LAUNCH(1, 128, 8, 2);
   else if (pieces <= 384) KM_ASSIGN_LAUNCH(1, 64, 4, 2);
@@ -1936,7 +2010,7 @@ static int km_assign(const void* data, const void* centroids, int32_t* assign, i
                      int64_t head_rows, ri_stream_t stream) {
   int rc = km_assign_args(data, centroids, assign, P, N, nc, seg);
   if (rc) return rc;
-  km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, (hipStream_t)stream);
+  km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, false, (hipStream_t)stream);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
@@ -2066,15 +2140,19 @@ extern "C" int ri_kmeans_update_f16(const void* data, const int32_t* counts, con
 
 template <bool HALF>
 static int km_direct_launch(const void* data, const int32_t* assign, void* centroids, int32_t* counts, int32_t* offsets,
-                            int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize,
+                            int32_t* members, int P, int N, int nc, int seg, int64_t head_rows, int normalize, bool narrow,
                             ri_stream_t stream) {
   // tokens compacted (4 bytes) and listed (2 bytes); block sums of a long cluster (512 bytes per KM_BLK rows) fit there too
   const size_t lds = (size_t)km_direct_run(N) * KM_DIRECT_WAVES * 6 + 512;
-#define KM_DIRECT_LAUNCH(CPW)                                                                                         \
-  do {                                                                                                                \
-    km_direct_kernel<HALF, CPW><<<km_grid((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>( \
-        (const uint16_t*)data, assign, (uint16_t*)centroids, counts, offsets, members, N, nc, seg, head_rows,         \
-        normalize, km_together(P));                                                                                                   \
+  const int shape = km_together(P) | (normalize ? 4 : 0) | ((P >> km_together(P)) - 1) << 3;
+#define KM_DIRECT_LAUNCH_AS(CPW, NARROW)                                                                              \
+  km_direct_kernel<HALF, CPW, NARROW>                                                                                 \
+      <<<km_grid((nc + CPW - 1) / CPW, P), KM_DIRECT_WAVES * 64, lds, (hipStream_t)stream>>>(                         \
+          (const uint16_t*)data, assign, (uint16_t*)centroids, N, nc, shape, seg, head_rows, counts, offsets, members)
+#define KM_DIRECT_LAUNCH(CPW)                     \
+  do {                                            \
+    if (narrow) KM_DIRECT_LAUNCH_AS(CPW, true);   \
+    else KM_DIRECT_LAUNCH_AS(CPW, false);         \
   } while (0)
   // As many workgroups as are resident at once (four of 512 threads, as many as the LDS of a compute unit holds): more
   // of them read the assignments more often and wait for a second round (24 x 8119 tokens, 512 clusters each: 8
@@ -2087,6 +2165,7 @@ static int km_direct_launch(const void* data, const int32_t* assign, void* centr
   else if (fits(16)) KM_DIRECT_LAUNCH(16);
   else KM_DIRECT_LAUNCH(32);
 #undef KM_DIRECT_LAUNCH
+#undef KM_DIRECT_LAUNCH_AS
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }
@@ -2101,7 +2180,7 @@ static int km_update_direct(const void* data, const int32_t* assign, void* centr
   if (rc) return rc;
   if (N > KM_DIRECT_MAX || seg <= 0 || P % seg != 0) return RI_ERR_ARG;
   return km_direct_launch<HALF>(data, assign, centroids, counts, offsets, members, P, N, nc, seg, head_rows, normalize,
-                                stream);
+                                false, stream);
 }
 
 extern "C" int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P,
@@ -2110,7 +2189,7 @@ extern "C" int ri_kmeans_lists_direct(const int32_t* assign, int32_t* counts, in
   int rc = km_check(P, N, nc);
   if (rc) return rc;
   if (N > KM_DIRECT_MAX) return RI_ERR_ARG;
-  return km_direct_launch<false>(nullptr, assign, nullptr, counts, offsets, members, P, N, nc, 1, N, 0, stream);
+  return km_direct_launch<false>(nullptr, assign, nullptr, counts, offsets, members, P, N, nc, 1, N, 0, false, stream);
 }
 
 extern "C" int ri_kmeans_update_direct(const void* data, const int32_t* assign, void* centroids, int32_t* counts,
@@ -2200,6 +2279,7 @@ static int km_iterate(const void* data, void* centroids, int32_t* assign, int P,
   const KmIterateSpace w = km_iterate_space(P, N, nc);
   if (workspace_bytes < w.all) return RI_ERR_WORKSPACE;
   const bool bounded = km_bounded(P, N, nc);
+  const bool narrows = N <= KM_DIRECT_MAX && N >= 8 && nc < 65536;   // (eight words, and ids that leave one over)
   hipStream_t s = (hipStream_t)stream;
   char* const base = (char*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   const KmBounds B = {(float*)(base + w.best), (float*)(base + w.bound), (const int32_t*)(base + w.state),
@@ -2213,12 +2293,13 @@ static int km_iterate(const void* data, void* centroids, int32_t* assign, int P,
     RI_HIP_CHECK_LAUNCH();
   }
   for (int i = 0; i < updates + (last ? 1 : 0); ++i) {
+    const bool narrow = narrows && i + (last ? 0 : 1) < updates;   // (the last assignment is the caller's)
     if (bounded && i > 0) km_assign_again<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, B, s);
-    else km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, s);
+    else km_assign_launch<HALF>(data, centroids, assign, P, N, nc, seg, head_rows, narrow, s);
     RI_HIP_CHECK_LAUNCH();
     if (i == updates) break;
     if (N <= KM_DIRECT_MAX) {
-      rc = km_direct_launch<HALF>(data, assign, centroids, nullptr, nullptr, nullptr, P, N, nc, seg, head_rows, 1, stream);
+      rc = km_direct_launch<HALF>(data, assign, centroids, nullptr, nullptr, nullptr, P, N, nc, seg, head_rows, 1, narrow, stream);
       if (rc) return rc;
       continue;
     }

@@ -500,3 +500,14 @@ def test_iterate_refuses(dev):
         keys.data_ptr(), cent.data_ptr(), assign.data_ptr(), 1, 64, nc, 1, 64, updates, 1, p, room, 0)
     assert call() == 0
     assert call(nc=33) != 0 and call(updates=-1) != 0 and call(room=nbytes - 1) != 0 and call(p=None) != 0
+
+
+# The assignments that passes hand over in 16 bits, eight to a lane: problems of fewer than eight tokens, runs of a wave that
+# end inside a lane's eight or that no token is left for, second rounds, odd starts of a problem's row, 8, 16 and 32 clusters to
+# a workgroup, and the most centroids whose ids leave a word over.
+@pytest.mark.parametrize("G,N,nc,seg", [(1, 7, 32, 1), (3, 8, 32, 1), (5, 9, 64, 1), (1, 255, 64, 1), (3, 1025, 96, 3),
+                                        (2, 2049, 96, 1), (8, 8191, 512, 1), (3, 15 * 1001, 480, 15), (130, 4099, 256, 1),
+                                        (2, 16384, 1024, 1), (1, 16383, 65504, 1), (1, 300, 65536, 1)])
+@pytest.mark.parametrize("kind", ["mixture", "ties"])
+def test_iterate_hands_assignments_over(dev, G, N, nc, seg, kind):
+    test_iterate_equals_its_passes(dev, G, N, nc, seg, kind, torch.bfloat16)
