@@ -382,6 +382,14 @@ def test_score_select_all_scores_equal(dev, nc, gs):
     assert torch.equal(est.cpu(), torch.arange(nprobe, nprobe + es, dtype=torch.int32).expand(2, -1))
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("gs", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("nc", [8200, 16384, 16392, 16640])
+def test_score_select_sums_of_many_tiles(dev, gs, nc, dt):
+    """The heads' statistics from 33, 64 (a lane each) and 65 tiles of partials, with and without heads that only pad."""
+    test_score_select(dev, 2, gs, nc, 60, 300, 40 + gs, dt)
+
+
 @pytest.mark.parametrize("gs", [5, 6])
 @pytest.mark.parametrize("nc", [4104, 4768, 4776, 5728, 5736])
 def test_score_select_every_head_counts(dev, gs, nc):
