@@ -76,13 +76,14 @@ _MAX_GRAPHS = 4
 
 def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1, init_indices=None,
                         reuse_graph=False, value_sum=None, value_store=None, store_stride=0, key_rows=None, key_mean=None,
-                        key_store=None):
+                        key_store=None, index=None):
     """Runs the clustering and returns a KMeansResult (no dense cluster lists, no host copy).
     key/value [G, N, 128] bfloat16 or float16 device tensors, keys contiguous.
 
     value_sum: [G, nc, 128] tensor for the sums (else a new one).  value_store: where the value rows are also
     written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
-    key_rows, the [G, N, 128] keys before key_mean was subtracted.
+    key_rows, the [G, N, 128] keys before key_mean was subtracted; index (with key_store): the tensors of
+    kernels.prefill_index, filled on the way.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and of the same
     type, shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -128,7 +129,7 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device) if value_sum is None else value_sum
     if key_store is not None:
         kernels.kmeans_store_rows(kernels.aligned_rows(value), key_rows, key_mean, r.counts, r.offsets, r.members,
-                                  r.value_sum, r.centroids, value_store, key_store, G, N, nc, store_stride)
+                                  r.value_sum, r.centroids, value_store, key_store, G, N, nc, store_stride, index)
         return r
     kernels.kmeans_value_sum(kernels.aligned_rows(value), r.counts, r.offsets, r.members, r.value_sum, G, N, nc,
                              store=value_store, store_stride=store_stride)

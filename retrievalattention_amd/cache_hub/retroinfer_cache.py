@@ -389,13 +389,15 @@ class retroinfer_cache(KV_Cache):
                 self.stage_keys = torch.empty((H, n_in, self.head_dim), dtype=self.dtype, device=keys.device)
                 self.stage_values = torch.empty_like(self.stage_keys)
             store_k, store_v, stride = self.stage_keys, self.stage_values, self.stage_keys.shape[1]
+        index = (self.centroids[layer_idx][rows], self.centroids_mask[layer_idx][rows], self.cluster_size[layer_idx][rows],
+                 self.cluster_size_i32[layer_idx][rows], self.cluster_start[layer_idx][rows])
         km = segment_k_means_csr(ck, head_values, self.n_centroids, num_segments=self.n_segment,
                                  reuse_graph=True,   # results are consumed below, before the next call
                                  value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride,
-                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k)
-        kernels.prefill_index(km.centroids, mean_key, km.counts, km.offsets, self.centroids[layer_idx][rows],
-                              self.centroids_mask[layer_idx][rows], self.cluster_size[layer_idx][rows],
-                              self.cluster_size_i32[layer_idx][rows], self.cluster_start[layer_idx][rows])
+                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k,
+                                 index=None if store_k is None else index)
+        if store_k is None:
+            kernels.prefill_index(km.centroids, mean_key, km.counts, km.offsets, *index)
         self.store_rows[layer_idx][rows] = [valid_length] * H
         if dev_organise:
             self.mainevents[dkey].record()

@@ -1294,8 +1294,8 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
 
 // odd (where it is asked for): set if the squares underflow or are no numbers, so that the result's norm need not be one
 template <bool MEAN, bool HALF>
-__device__ __forceinline__ void km_finish(float s0, float s1, int count, int normalize, uint32_t* op,
-                                          int32_t* odd = nullptr) {
+__device__ __forceinline__ uint32_t km_finish(float s0, float s1, int count, int normalize, uint32_t* op,
+                                              int32_t* odd = nullptr) {
   if (MEAN) {
     const float cnt = (float)count;
     s0 = s0 / cnt;
@@ -1307,7 +1307,9 @@ __device__ __forceinline__ void km_finish(float s0, float s1, int count, int nor
       s1 = s1 / nrm;
     }
   }
-  *op = (uint32_t)ri_f32_to_e16<HALF>(s0) | ((uint32_t)ri_f32_to_e16<HALF>(s1) << 16);
+  const uint32_t word = (uint32_t)ri_f32_to_e16<HALF>(s0) | ((uint32_t)ri_f32_to_e16<HALF>(s1) << 16);
+  *op = word;
+  return word;
 }
 
 // slots of one problem: the last list starts below N and a slot index is at most 2 (N / KM_BLK) + 1
@@ -1403,6 +1405,27 @@ __device__ __forceinline__ void km_plan(const KmMoves& M, int p, int N, int nc) 
   }
 }
 
+// A cache's entries of the clusters, made where their means are (out == nullptr: none): mean + the keys' mean, whether empty,
+// sizes, first rows, as index_kernel makes them of finished means.
+struct KmIndex {
+  uint32_t* out;   // [P, nc, 64] words
+  uint8_t* mask;
+  uint16_t* size16;
+  int32_t *size, *start;
+};
+// (behind the rows: a load's wait covers the stores in front of it)
+template <bool HALF>
+__device__ __forceinline__ void km_entry(const KmIndex& X, size_t at, int size, int start, uint32_t word, uint32_t mean) {
+  const int lane = threadIdx.x & 63;
+  X.out[at * (RI_DIM / 2) + lane] = ri_sum2<HALF>(word, mean);
+  if (lane == 0) {
+    X.mask[at] = size == 0;
+    X.size16[at] = ri_f32_to_e16<HALF>((float)size);
+    X.size[at] = size;
+    X.start[at] = start;
+  }
+}
+
 // grid (item workgroups + ceil(nc / 4), P), four waves each.  The first item_wgs workgroups take
 // one slot per wave (blocks of long lists, their fp32 sums go to partial[p][slot]); the others one
 // cluster per wave.
@@ -1415,7 +1438,8 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
                                                float2* __restrict__ partial, int item_wgs, int cap, int N, int nc,
                                                int seg, int64_t head_stride, int normalize,
                                                uint16_t* __restrict__ copy, int64_t copy_stride,
-                                               const uint16_t* __restrict__ mean, const KmMoves& M = KmMoves{}) {
+                                               const uint16_t* __restrict__ mean, const KmMoves& M = KmMoves{},
+                                               const KmIndex& X = KmIndex{}) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int32_t* off = offsets + (size_t)p * (nc + 1);
@@ -1446,15 +1470,18 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
     if (!touched) return;   // the tokens of the update before, in the same order: it has their mean
   }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
+  const int o = off[c];
   if (s == 0) {
     if (!MEAN) *op = 0u;  // empty cluster: zero value sum; the centroid is left untouched
+    else if (CENTER && X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, *op, mw);
     return;
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + off[c], 0, s, s0, s1, pitch,
-                                      COPY ? wp + (size_t)off[c] * (RI_DIM / 2) : nullptr, mw);
-  km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);
+  km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + o, 0, s, s0, s1, pitch,
+                                      COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
+  const uint32_t word = km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);
+  if (CENTER && X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, word, mw);
 }
 
 template <bool MEAN, bool HALF, bool COPY>
@@ -1486,13 +1513,13 @@ __global__ __launch_bounds__(256) void km_store_kernel(KmStoreArgs V, KmStoreArg
                                                        const int32_t* __restrict__ counts,
                                                        const int32_t* __restrict__ offsets,
                                                        const int32_t* __restrict__ members, int item_wgs, int cap, int N,
-                                                       int nc, int64_t copy_stride) {
+                                                       int nc, int64_t copy_stride, KmIndex X) {
   if (blockIdx.z == 0)
     km_reduce_rows<false, HALF, true, false>(V.rows, V.pitch, counts, offsets, members, V.out, V.partial, item_wgs, cap, N,
                                              nc, 1, V.head_stride, 0, V.copy, copy_stride, nullptr);
   else
     km_reduce_rows<true, HALF, true, true>(K.rows, K.pitch, counts, offsets, members, K.out, K.partial, item_wgs, cap, N,
-                                           nc, 1, K.head_stride, 0, K.copy, copy_stride, mean);
+                                           nc, 1, K.head_stride, 0, K.copy, copy_stride, mean, KmMoves{}, X);
 }
 
 // grid (item workgroups, P): the wave of a long list's first slot adds the block sums in block
@@ -1500,7 +1527,8 @@ __global__ __launch_bounds__(256) void km_store_kernel(KmStoreArgs V, KmStoreArg
 template <bool MEAN, bool HALF>
 __device__ __forceinline__ void km_fold(const int32_t* __restrict__ offsets, const float2* __restrict__ partial,
                                         uint16_t* __restrict__ out, int cap, int nc, int normalize,
-                                        const KmMoves& M = KmMoves{}) {
+                                        const KmMoves& M = KmMoves{}, const uint32_t* mean = nullptr,
+                                        const KmIndex& X = KmIndex{}) {
   const int p = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1530,7 +1558,8 @@ __device__ __forceinline__ void km_fold(const int32_t* __restrict__ offsets, con
     t.y += v.y;
   }
   uint32_t* op = reinterpret_cast<uint32_t*>(out + ((size_t)p * nc + c) * RI_DIM) + lane;
-  km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op, M.state ? M.odd + p : nullptr);
+  const uint32_t word = km_finish<MEAN, HALF>(t.x, t.y, s, normalize, op, M.state ? M.odd + p : nullptr);
+  if (X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, word, mean[p * (RI_DIM / 2) + lane]);
 }
 
 template <bool MEAN, bool HALF>
@@ -1544,9 +1573,10 @@ __global__ __launch_bounds__(256) void km_reduce_fold_kernel(const int32_t* __re
 
 template <bool HALF>
 __global__ __launch_bounds__(256) void km_store_fold_kernel(KmStoreArgs V, KmStoreArgs K,
-                                                            const int32_t* __restrict__ offsets, int cap, int nc) {
+                                                            const uint16_t* __restrict__ mean,
+                                                            const int32_t* __restrict__ offsets, int cap, int nc, KmIndex X) {
   if (blockIdx.z == 0) km_fold<false, HALF>(offsets, V.partial, V.out, cap, nc, 0);
-  else km_fold<true, HALF>(offsets, K.partial, K.out, cap, nc, 0);
+  else km_fold<true, HALF>(offsets, K.partial, K.out, cap, nc, 0, KmMoves{}, reinterpret_cast<const uint32_t*>(mean), X);
 }
 
 // ------------------------------------------------------------------------------------
@@ -2365,7 +2395,8 @@ template <bool HALF>
 static int km_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
                          const void* mean, const int32_t* counts, const int32_t* offsets, const int32_t* members,
                          void* value_sum, void* centroids, void* value_store, void* key_store, int64_t store_stride_rows,
-                         int P, int N, int nc, void* workspace, size_t workspace_bytes, hipStream_t s) {
+                         int P, int N, int nc, void* workspace, size_t workspace_bytes, hipStream_t s,
+                         const KmIndex& X = KmIndex{}) {
   if (!values || !keys || !mean || !counts || !offsets || !members || !value_sum || !centroids || !value_store ||
       !key_store || !workspace)
     return RI_ERR_ARG;
@@ -2388,11 +2419,45 @@ static int km_store_rows(const void* values, int64_t v_head, int64_t v_row, cons
                          partial + (size_t)P * cap * (RI_DIM / 2), (size_t)k_row / 2, k_head / 2};
   km_store_kernel<HALF><<<dim3(item_wgs + (nc + 3) / 4, P, 2), 256, 0, s>>>(V, K, (const uint16_t*)mean, counts, offsets,
                                                                             members, item_wgs, cap, N, nc,
-                                                                            store_stride_rows);
+                                                                            store_stride_rows, X);
   RI_HIP_CHECK_LAUNCH();
-  km_store_fold_kernel<HALF><<<dim3(item_wgs, P, 2), 256, 0, s>>>(V, K, offsets, cap, nc);
+  km_store_fold_kernel<HALF><<<dim3(item_wgs, P, 2), 256, 0, s>>>(V, K, (const uint16_t*)mean, offsets, cap, nc, X);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
+}
+
+template <bool HALF>
+static int km_store_index(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
+                          const void* mean, const int32_t* counts, const int32_t* offsets, const int32_t* members,
+                          void* value_sum, void* centroids, void* value_store, void* key_store, int64_t store_stride_rows,
+                          void* out, uint8_t* mask, void* size16, int32_t* size, int32_t* start, int P, int N, int nc,
+                          void* workspace, size_t workspace_bytes, hipStream_t s) {
+  if (!out || !mask || !size16 || !size || !start || ri_any_misaligned16(out)) return RI_ERR_ARG;
+  const KmIndex X = {(uint32_t*)out, mask, (uint16_t*)size16, size, start};
+  return km_store_rows<HALF>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum, centroids,
+                             value_store, key_store, store_stride_rows, P, N, nc, workspace, workspace_bytes, s, X);
+}
+
+extern "C" int ri_kmeans_store_index(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,
+                                     int64_t k_row, const void* mean, const int32_t* counts, const int32_t* offsets,
+                                     const int32_t* members, void* value_sum, void* centroids, void* value_store,
+                                     void* key_store, int64_t store_stride_rows, void* out, uint8_t* mask, void* size16,
+                                     int32_t* size, int32_t* start, int P, int N, int nc, void* workspace,
+                                     size_t workspace_bytes, ri_stream_t stream) {
+  return km_store_index<false>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum,
+                               centroids, value_store, key_store, store_stride_rows, out, mask, size16, size, start, P, N, nc,
+                               workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" int ri_kmeans_store_index_f16(const void* values, int64_t v_head, int64_t v_row, const void* keys,
+                                         int64_t k_head, int64_t k_row, const void* mean, const int32_t* counts,
+                                         const int32_t* offsets, const int32_t* members, void* value_sum, void* centroids,
+                                         void* value_store, void* key_store, int64_t store_stride_rows, void* out,
+                                         uint8_t* mask, void* size16, int32_t* size, int32_t* start, int P, int N, int nc,
+                                         void* workspace, size_t workspace_bytes, ri_stream_t stream) {
+  return km_store_index<true>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum,
+                              centroids, value_store, key_store, store_stride_rows, out, mask, size16, size, start, P, N, nc,
+                              workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int ri_kmeans_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,

@@ -298,17 +298,10 @@ extern "C" int ri_prefill_center_f16(void* keys, const void* mean, int H, int N,
 }
 
 // ------------------------------------------------------------------------------------
-// index: the cache's entries of a finished clustering, one launch for all of them.
+// index: the cache's entries of a finished clustering, one launch for all of them, where they are not made with the stores
+// (km_store_kernel).
 // grid (ceil(nc / 16), H), 16 lanes per cluster.
 // ------------------------------------------------------------------------------------
-template <bool HALF>
-__device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
-  float a0, a1, b0, b1;
-  ri_unpack2<HALF>(a, a0, a1);
-  ri_unpack2<HALF>(b, b0, b1);
-  return (uint32_t)ri_f32_to_e16<HALF>(a0 + b0) | ((uint32_t)ri_f32_to_e16<HALF>(a1 + b1) << 16);
-}
-
 template <bool HALF>
 __global__ __launch_bounds__(256) void index_kernel(const uint4* __restrict__ cent, const uint4* __restrict__ mean,
                                                     const int32_t* __restrict__ counts,
@@ -319,7 +312,8 @@ __global__ __launch_bounds__(256) void index_kernel(const uint4* __restrict__ ce
   if (c >= nc) return;
   const size_t at = (size_t)h * nc + c;
   const uint4 x = cent[at * 16 + piece], m = mean[(size_t)h * 16 + piece];
-  out[at * 16 + piece] = make_uint4(add2<HALF>(x.x, m.x), add2<HALF>(x.y, m.y), add2<HALF>(x.z, m.z), add2<HALF>(x.w, m.w));
+  out[at * 16 + piece] =
+      make_uint4(ri_sum2<HALF>(x.x, m.x), ri_sum2<HALF>(x.y, m.y), ri_sum2<HALF>(x.z, m.z), ri_sum2<HALF>(x.w, m.w));
   if (piece == 0) {
     const int32_t n = counts[at];
     mask[at] = n == 0;

@@ -101,6 +101,14 @@ __device__ __forceinline__ uint32_t ri_sub2(uint32_t a, uint32_t b) {
   ri_unpack2<HALF>(b, b0, b1);
   return (uint32_t)ri_f32_to_e16<HALF>(a0 - b0) | ((uint32_t)ri_f32_to_e16<HALF>(a1 - b1) << 16);
 }
+// a + b, as ri_sub2
+template <bool HALF>
+__device__ __forceinline__ uint32_t ri_sum2(uint32_t a, uint32_t b) {
+  float a0, a1, b0, b1;
+  ri_unpack2<HALF>(a, a0, a1);
+  ri_unpack2<HALF>(b, b0, b1);
+  return (uint32_t)ri_f32_to_e16<HALF>(a0 + b0) | ((uint32_t)ri_f32_to_e16<HALF>(a1 + b1) << 16);
+}
 // finfo(type).min as a bit pattern: the score of a masked (empty) cluster
 template <bool HALF>
 __host__ __device__ __forceinline__ uint16_t ri_e16_lowest() { return HALF ? 0xfbff : 0xff7f; }

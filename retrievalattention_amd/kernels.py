@@ -673,17 +673,18 @@ def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot
 
 
 def kmeans_store_rows(values, keys, mean, counts, offsets, members, value_sum, centroids, value_store, key_store, P, N, nc,
-                      store_stride):
-    """Value sums and means of the centred keys, with both stores; values/keys [P, N, 128], strided or not."""
+                      store_stride, index=None):
+    """Value sums and means of the centred keys, with both stores; values/keys [P, N, 128], strided or not.
+    index: (out, mask, size16, size, start) of prefill_index, filled as well."""
     ws = _workspace(2 * lib().ri_kmeans_reduce_workspace_bytes(P, N, nc), values.device, "kmeans_store")
     vh, vr = _row_strides(values, "kmeans_store_rows")
     kh, kr = _row_strides(keys, "kmeans_store_rows")
     if not values.dtype == keys.dtype == mean.dtype == value_store.dtype == key_store.dtype:
         raise TypeError("kmeans_store_rows: values, keys and the stores must have the same element type")
-    check(_fn("ri_kmeans_store_rows", values.dtype)(_p(values), vh, vr, _p(keys), kh, kr, _p(mean), _p(counts),
-                                                    _p(offsets), _p(members), _p(value_sum), _p(centroids),
-                                                    _p(value_store), _p(key_store), store_stride, P, N, nc, _p(ws),
-                                                    ws.numel(), _stream()), "kmeans_store_rows")
+    fn = _fn("ri_kmeans_store_rows" if index is None else "ri_kmeans_store_index", values.dtype)
+    check(fn(_p(values), vh, vr, _p(keys), kh, kr, _p(mean), _p(counts), _p(offsets), _p(members), _p(value_sum),
+             _p(centroids), _p(value_store), _p(key_store), store_stride, *(_p(t) for t in index or ()), P, N, nc, _p(ws),
+             ws.numel(), _stream()), "kmeans_store_rows")
 
 
 def permute_rows_strided(src, members, dst, P, N, out_stride_rows):

@@ -74,6 +74,40 @@ def test_prefill_passes(dev, dtype, H, N, nc, fused):
     assert torch.equal(size, counts) and torch.equal(start, offsets[:, :nc])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,nc", [(1, 1, 32), (3, 257, 64), (8, 1000, 96), (2, 20001, 1088)])
+def test_index_entries_on_the_way_to_the_stores(dev, dtype, H, N, nc):
+    """The entries that the stores' launches fill are those of the finished means: of short lists, of long ones, whose
+    means are folded later, and of empty clusters, which keep their centroids."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(H * N + nc)
+    rows = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)
+    K, V, mean, cent = rows(N, H, 128), rows(N, H, 128), rows(H, 1, 128), rows(H, nc, 128)
+    hk, hv = K.transpose(0, 1), V.transpose(0, 1)
+    assign = torch.randint(0, nc - 1, (H, N), generator=g, dtype=torch.int32)
+    assign[:, : N // 2] = 3
+    assign = assign.to(dev)
+    counts, offsets, members = (torch.empty(s, dtype=torch.int32, device=dev) for s in ((H, nc), (H, nc + 1), (H, N)))
+    kernels.kmeans_build_lists(assign, counts, offsets, members, H, N, nc)
+
+    def stored(**options):
+        means, sums = cent.clone(), torch.zeros_like(cent)
+        stores = [torch.zeros((H, N + 7, 128), dtype=dtype, device=dev) for _ in range(2)]
+        kernels.kmeans_store_rows(hv, hk, mean, counts, offsets, members, sums, means, *stores, H, N, nc, N + 7, **options)
+        return means, sums, *stores
+
+    def entries():
+        return (torch.zeros_like(cent), torch.zeros((H, nc), dtype=torch.bool, device=dev),
+                torch.zeros((H, nc), dtype=dtype, device=dev), torch.zeros_like(counts), torch.zeros_like(counts))
+
+    apart, filled = entries(), entries()
+    plain = stored()
+    kernels.prefill_index(plain[0], mean, counts, offsets, *apart)
+    assert all(torch.equal(a, b) for a, b in zip(stored(index=filled), plain))
+    assert all(torch.equal(a, b) for a, b in zip(filled, apart))
+    assert torch.equal(filled[0], plain[0] + mean) and torch.equal(filled[1], counts == 0)
+
+
 # where the order of the sum changes (one part, four, eight, sixteen ...; one head has a rule of its own), and around it
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,N", [(1, 1), (1, 1020), (1, 1021), (1, 8193), (1, 16384), (1, 16385), (1, 40007), (2, 3),
