@@ -183,6 +183,13 @@ __global__ __launch_bounds__(1024) void softmax_kernel(const uint4* __restrict__
   }
 }
 
+// LDS that a scoring launch asks for and does not use: from three rounds of workgroups on, two to a compute unit stream faster
+// than the four that fit (128 KB of rows on their way to a unit, not 256; a kernel that only reads shows the same).  A step, us,
+// four / two / one: 64 groups of 8 heads, 16384 clusters 125.7 / 123.1 / 140; four / two: 64 of 4, 16384 122.9 / 119.9, 128 of 4, 8192
+// 121.1 / 118.3, 48 of 8, 16384 104.5 / 103.0, 64 of 12, 16384 138.3 / 137.3; two rounds: 64 of 4, 8192 70.3 / 69.7, 32 of 4, 16384 71.3 /
+// 70.9, but 128 of 8, 4096 74.3 / 74.9; less: 24 of 4, 16384 59.7 / 59.9, 32 of 8, 8192 44.3 / 45.1.  (Three to a unit 126.2 in the first.)
+static size_t score_spread(int64_t workgroups) { return workgroups >= 3 * 1024 ? 56 * 1024 : 0; }
+
 // ------------------------------------------------------------------------------------
 // C entry points
 // ------------------------------------------------------------------------------------
@@ -203,7 +210,7 @@ static int batch_gemm_softmax_impl(const void* A, const void* B, void* D, float*
   const int ntiles = (n + SCORE_TILE - 1) / SCORE_TILE;
   // fp32 logits are not part of this interface: the partial statistics come from the fp32
   // accumulators inside the kernel, the softmax from the 16-bit D, as in the reference.
-  score_kernel<HALF, 4, 4, false><<<dim3(ntiles, batch_count), 256, 0, s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
+  score_kernel<HALF, 4, 4, false><<<dim3(ntiles, batch_count), 256, score_spread((int64_t)ntiles * batch_count), s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
                                                                   (uint16_t*)D, Norm, Sum, m, n, ntiles, alpha);
   RI_HIP_CHECK_LAUNCH();
   const int threads = min(1024, (n / 8 + 63) / 64 * 64);
@@ -238,7 +245,8 @@ int ri_launch_score(const void* q, const void* centroids, float* logits, float* 
   auto* kernel = half ? (stream ? score_kernel<true, 4, 4, true> : score_kernel<true, 4, 4, false>)
                       : (stream ? score_kernel<false, 4, 4, true> : score_kernel<false, 4, 4, false>);
   if (tile == RI_SCORE_TILE_FEW) kernel = half ? score_kernel<true, 1, 4, false> : score_kernel<false, 1, 4, false>;
-  kernel<<<dim3(ntiles, BG), 256, 0, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc, ntiles, scale);
+  const size_t spread = tile == RI_SCORE_TILE_FEW ? 0 : score_spread((int64_t)ntiles * BG);
+  kernel<<<dim3(ntiles, BG), 256, spread, s>>>(qq, cc, logits, nullptr, tile_max, tile_sum, gs, nc, ntiles, scale);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
 }

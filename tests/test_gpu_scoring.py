@@ -428,3 +428,34 @@ def test_score_select_without_room_for_narrow_tiles(dev):
         got.append((rc, logits, ids.sort(dim=1)[0]))
     assert [r[0] for r in got[:2]] == [0, 0] and got[2][0] != 0
     assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+
+
+# Both sides of the line from which a scoring launch has fewer workgroups to a compute unit (3072 tiles), the last tile with a remainder.
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("BG,gs,nc", [(96, 5, 7688), (96, 5, 8168), (192, 2, 4000)])
+def test_scores_of_long_launches(dev, BG, gs, nc, dt):
+    """The same logits and softmax as of the groups by themselves, half of them at a time, and those of a product in float32."""
+    from retrievalattention_amd import _lib, kernels
+    lib = _lib.lib()
+    g = torch.Generator(device=dev).manual_seed(BG + nc)
+    q, cent = (torch.randn(BG, n, 128, generator=g, device=dev).to(dt) for n in (gs, nc))
+    scale, tiles = 128 ** -0.5, (nc + 255) // 256
+    call = getattr(lib, "ri_score_logits" + ("_f16" if dt == torch.float16 else ""))
+
+    def scores(a, b):
+        n = b - a
+        logits = torch.zeros(n, gs, nc, device=dev)
+        room = lib.ri_score_select_workspace_bytes(n, gs, nc)
+        ws = torch.empty(room, dtype=torch.uint8, device=dev)
+        assert call(q[a:].data_ptr(), cent[a:].data_ptr(), logits.data_ptr(), n, gs, nc, scale, ws.data_ptr(), room, 0) == 0
+        d, soft = (torch.zeros(n, gs, nc, dtype=dt, device=dev) for _ in range(2))
+        norm, total = (torch.zeros(n, tiles, gs, device=dev) for _ in range(2))
+        kernels.batch_gemm_softmax(q[a:b].view(n, 1, gs, 128), cent[a:b], d, norm, total, soft, n, gs, nc, 128, scale)
+        return logits, d, soft
+
+    whole, halves = scores(0, BG), [scores(0, BG // 2), scores(BG // 2, BG)]
+    for i in range(3):
+        assert torch.equal(whole[i], torch.cat([h[i] for h in halves]))
+    want = torch.stack([q[i].float() @ cent[i].float().t() for i in range(BG)]) * scale
+    # 128 products of 16-bit numbers in 32-bit sums: 128 roundings of the largest partial sum at most (|scores| below 8 here)
+    assert (whole[0] - want).abs().max() < 128 * 8 * 2 ** -24 * 2
