@@ -1248,7 +1248,11 @@ __global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
 // wave's instructions bound this as much as the bytes: three fetch a row (address arithmetic per row took seven, and a
 // select per row is left to the last eight: 8 x 131072 tokens, 8192 clusters 71.3 -> 57.0 us, with 64 rows in flight 67.4;
 // half the tokens in seven clusters of 4 x 20000 tokens 27.7 -> 19.7).
-// pitch: words between rows.  With wp the rows are also copied: row k of the list to wp + k * 64.
+// pitch: words between rows.  With wp the rows are also copied: row k of the list to wp + k * 64, with stores that do not stay in
+// the caches, which nobody reads them from soon.  Copies take sixteen rows a round: the addresses of the stores are registers
+// too, and of 84 a SIMD holds five waves where of 58 it holds eight.  Keys and values of 8 x 131072 tokens, us with 32 / 24 / 16 / 8
+// rows 214.5 / 222 / 199.5 / 211.5, a prefill 3240 / - / 3225, with sixteen and such stores 204.4 and 3196; 4 x 50021 half 37.4 / 43.0 / 36.5 /
+// 37.6, 34.8 with such stores, 8 x 8192 17.5 / 20.2 / 17.7 / 19.9, 16.7.  (Loads past the caches as well: 38.3 and 19.8 in these two.)
 // CENTER: the sum is of the rows minus `mean` (this lane's two dims), as ri_prefill_center leaves them.
 template <bool HALF, int U, bool COPY = false, bool CENTER = false>
 __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, const int32_t* mem, int k0, int k1, float& s0,
@@ -1279,13 +1283,13 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
 #pragma unroll
         for (int j = e; j < e + 8; ++j) {
           add(term(v[j]));
-          if (COPY) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
+          if (COPY) __builtin_nontemporal_store(v[j], wp + (size_t)(k + j) * (RI_DIM / 2));
         }
       } else if (e < n) {
 #pragma unroll
         for (int j = e; j < e + 8; ++j) {
           add(j < n ? term(v[j]) : 0u);   // the word 0 is (+0, +0) in either type
-          if (COPY && j < n) wp[(size_t)(k + j) * (RI_DIM / 2)] = v[j];
+          if (COPY && j < n) __builtin_nontemporal_store(v[j], wp + (size_t)(k + j) * (RI_DIM / 2));
         }
       }
     }
@@ -1455,7 +1459,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
     const int c = km_slot_owner(off, nc, slot, s, o, j);
     if (c < 0 || (M.state && !M.first && !M.touched[(size_t)p * nc + c])) return;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1,
+    km_sum_rows<HALF, COPY ? 16 : 32, COPY, CENTER>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1,
                                         pitch, COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
     partial[((size_t)p * cap + slot) * 64 + lane] = make_float2(s0, s1);
     return;
@@ -1478,7 +1482,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF, 32, COPY, CENTER>(rp, members + (size_t)p * N + o, 0, s, s0, s1, pitch,
+  km_sum_rows<HALF, COPY ? 16 : 32, COPY, CENTER>(rp, members + (size_t)p * N + o, 0, s, s0, s1, pitch,
                                       COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
   const uint32_t word = km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);
   if (CENTER && X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, word, mw);
