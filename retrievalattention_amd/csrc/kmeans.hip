@@ -880,9 +880,9 @@ __global__ __launch_bounds__(256) void km_assign_open_kernel(const uint16_t* __r
 // ------------------------------------------------------------------------------------
 // inverted lists
 // ------------------------------------------------------------------------------------
-// Inverted lists are a stable sort of the token ids by cluster id.  Ids of at most 9 bits take one counting pass, three
-// launches: per-chunk digit histograms (KM_SORT_CHUNK tokens, LDS counters), an exclusive scan of the [digit][chunk]
-// table per problem, and a scatter in which every wave walks its part of a chunk in token order, ranks equal digits
+// Inverted lists are a stable sort of the token ids by cluster id.  Ids of at most 9 bits take one counting pass, two
+// launches, three with a large table: per-chunk digit histograms (KM_SORT_CHUNK tokens, LDS counters), an exclusive scan of the
+// [digit][chunk] table per problem, and a scatter in which every wave walks its part of a chunk in token order, ranks equal digits
 // inside each 64-token round with ballots and keeps running positions in LDS.  Longer ids take that pass over their upper
 // digit and one launch that sorts every bucket of it by the lower digit in a workgroup and writes offsets and counts on
 // the way.  Stability makes every list ascending without any per-list sort, and no global atomics are involved, so the
@@ -899,10 +899,10 @@ __device__ __forceinline__ void km_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// chunk_hist[p][digit][chunk] = tokens of the chunk whose key has that digit; a workgroup per chunk
+// chunk_hist[p][digit][chunk] (by_chunk: [p][chunk][digit]) = tokens of the chunk whose key has that digit; a workgroup per chunk
 __global__ __launch_bounds__(256) void km_sort_hist_kernel(const int32_t* __restrict__ keys,
                                                            int32_t* __restrict__ chunk_hist, int N, int nchunks,
-                                                           int shift, int bits) {
+                                                           int shift, int bits, bool by_chunk) {
   __shared__ int32_t h[KM_SORT_MAX_BINS];
   const int p = blockIdx.y, chunk = blockIdx.x, bins = 1 << bits;
   const int i0 = chunk * KM_SORT_CHUNK + threadIdx.x;
@@ -915,7 +915,8 @@ __global__ __launch_bounds__(256) void km_sort_hist_kernel(const int32_t* __rest
   for (int r = 0; r < KM_SORT_ROUNDS; ++r)
     if (i0 + r * 256 < N) atomicAdd(&h[(k[r] >> shift) & (bins - 1)], 1);
   __syncthreads();
-  for (int b = threadIdx.x; b < bins; b += 256) chunk_hist[((size_t)p * bins + b) * nchunks + chunk] = h[b];
+  for (int b = threadIdx.x; b < bins; b += 256)
+    chunk_hist[by_chunk ? ((size_t)p * nchunks + chunk) * bins + b : ((size_t)p * bins + b) * nchunks + chunk] = h[b];
 }
 
 // in-place exclusive prefix sum over the n = bins * nchunks entries of each problem.
@@ -973,12 +974,74 @@ __global__ __launch_bounds__(1024) void km_sort_scan_kernel(int32_t* __restrict_
   }
 }
 
+// What a scatter without a scan in front of it writes besides: where every digit starts (starts), or, of whole ids, offsets and
+// counts.
+struct KmFirsts {
+  int32_t *starts, *offsets, *counts;
+  int nc;
+};
+// Up to KM_SORT_TABLE counts the scatter's workgroups add up the table themselves, which is one round trip more for each
+// where the scan is a launch of one workgroup per problem; the first chunk's writes where the digits start.
+// at: [bins] where this chunk's tokens of each digit go.  16 <= bins / 4 <= 128 pieces to a row of the table, sixteen per thread.
+#define KM_SORT_TABLE 16384
+__device__ __forceinline__ void km_sort_places(const int32_t* __restrict__ table, int32_t* at, int p, int chunk, int nchunks,
+                                               int bits, int N, const KmFirsts& F) {
+  __shared__ __attribute__((aligned(16))) int32_t sh_all[KM_SORT_TABLE / 16], sh_before[KM_SORT_TABLE / 16];
+  __shared__ int32_t sh_w[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, bins = 1 << bits;
+  const int row0 = tid >> (bits - 2), quad = tid & ((bins >> 2) - 1), rows = 1024 >> bits;   // rows that the workgroup reads at a time
+  const int4* const in = reinterpret_cast<const int4*>(table + (size_t)p * nchunks * bins) + quad;
+  int4 v[16], all = make_int4(0, 0, 0, 0), before = all;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) v[u] = in[(size_t)min(row0 + u * rows, nchunks - 1) << (bits - 2)];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int row = row0 + u * rows, there = row < nchunks ? -1 : 0, ahead = row < chunk ? -1 : 0;
+    all.x += v[u].x & there; all.y += v[u].y & there; all.z += v[u].z & there; all.w += v[u].w & there;
+    before.x += v[u].x & ahead; before.y += v[u].y & ahead; before.z += v[u].z & ahead; before.w += v[u].w & ahead;
+  }
+  *reinterpret_cast<int4*>(&sh_all[tid * 4]) = all;   // [row0][digit]
+  *reinterpret_cast<int4*>(&sh_before[tid * 4]) = before;
+  __syncthreads();
+  // a thread's digits: tid, or with 512 of them 2 tid and the next
+  const int each = bits == 9 ? 2 : 1, b0 = tid * each;
+  int32_t n[2] = {0, 0}, ex[2] = {0, 0};
+  for (int e = 0; e < each; ++e)
+    if (b0 + e < bins)
+      for (int r = 0; r < rows; ++r) {
+        n[e] += sh_all[(r << bits) + b0 + e];
+        ex[e] += sh_before[(r << bits) + b0 + e];
+      }
+  const int inc = (int)ri_wave_incl_scan((uint32_t)(n[0] + n[1]));
+  if (lane == 63) sh_w[wave] = inc;
+  __syncthreads();
+  int start = inc - n[0] - n[1];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) start += w < wave ? sh_w[w] : 0;
+  for (int e = 0; e < each; ++e) {
+    const int b = b0 + e;
+    if (b < bins) at[b] = start + ex[e];
+    if (chunk == 0) {
+      if (F.starts && b < bins) F.starts[p * bins + b] = start;
+      if (F.offsets && b < F.nc) {
+        F.offsets[(size_t)p * (F.nc + 1) + b] = start;
+        F.counts[(size_t)p * F.nc + b] = n[e];
+      }
+    }
+    start += n[e];
+  }
+  if (chunk == 0 && F.offsets && tid == 0) F.offsets[(size_t)p * (F.nc + 1) + F.nc] = N;
+  __syncthreads();
+}
+
 // A workgroup per chunk; its four waves take 256 consecutive tokens each and count their digits first, so that each knows
-// where it starts.  low >= 0: token << low | the id's low bits, else the token.
+// where it starts.  low >= 0: token << low | the id's low bits, else the token.  SCANNED: chunk_hist is, else by chunks.
+template <bool SCANNED>
 __global__ __launch_bounds__(256) void km_sort_scatter_kernel(const int32_t* __restrict__ keys,
                                                               const int32_t* __restrict__ chunk_hist,
                                                               int32_t* __restrict__ out_toks, int N, int nchunks,
-                                                              int shift, int bits, int low) {
+                                                              int shift, int bits, int low, KmFirsts F) {
+  __shared__ int32_t sh_at[SCANNED ? 1 : KM_SORT_MAX_BINS];
   __shared__ int32_t sh[4][KM_SORT_MAX_BINS];
   const int p = blockIdx.y, chunk = blockIdx.x, bins = 1 << bits;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -989,9 +1052,12 @@ __global__ __launch_bounds__(256) void km_sort_scatter_kernel(const int32_t* __r
   for (int r = 0; r < KM_SORT_ROUNDS; ++r) k[r] = keys[(size_t)p * N + min(i0 + r * 64, N - 1)];
   for (int b = lane; b < bins; b += 64) run[b] = 0;
   int32_t first[KM_SORT_MAX_BINS / 256];
+  if (!SCANNED) km_sort_places(chunk_hist, sh_at, p, chunk, nchunks, bits, N, F);
 #pragma unroll
-  for (int u = 0; u < KM_SORT_MAX_BINS / 256; ++u)
-    first[u] = chunk_hist[((size_t)p * bins + min((int)threadIdx.x + u * 256, bins - 1)) * nchunks + chunk];
+  for (int u = 0; u < KM_SORT_MAX_BINS / 256; ++u) {
+    const int b = min((int)threadIdx.x + u * 256, bins - 1);
+    first[u] = SCANNED ? chunk_hist[((size_t)p * bins + b) * nchunks + chunk] : sh_at[b];
+  }
   km_wave_lds_sync();
 #pragma unroll
   for (int r = 0; r < KM_SORT_ROUNDS; ++r)
@@ -1135,8 +1201,8 @@ __global__ __launch_bounds__(KM_SMALL_WAVES * 64) void km_sort_small_kernel(cons
 #define KM_BUCKET_HELD 4   // rounds of 64 tokens per wave kept in registers between the two walks
 
 __global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
-    const int32_t* __restrict__ assign, const int32_t* __restrict__ toks, const int32_t* __restrict__ chunk_hist,
-    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int nchunks,
+    const int32_t* __restrict__ assign, const int32_t* __restrict__ toks, const int32_t* __restrict__ starts,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ members, int N, int nc, int pitch,
     int bits, int buckets, int bins, bool packed) {
   constexpr int NW = KM_BUCKET_WAVES, HELD = KM_BUCKET_HELD;
   __shared__ int32_t sh_run[KM_SORT_MAX_BINS][NW];
@@ -1144,9 +1210,9 @@ __global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
   const int p = blockIdx.y, bucket = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int C = 1 << bits, c0 = bucket << bits;
-  const int32_t* first = chunk_hist + (size_t)p * bins * nchunks;
-  const int start = first[(size_t)bucket * nchunks];
-  const int end = bucket + 1 < buckets ? first[(size_t)(bucket + 1) * nchunks] : N;
+  const int32_t* first = starts + (size_t)p * bins * pitch;   // a digit's start every `pitch` words
+  const int start = first[(size_t)bucket * pitch];
+  const int end = bucket + 1 < buckets ? first[(size_t)(bucket + 1) * pitch] : N;
   const int rounds = (end - start + NW * 64 - 1) / (NW * 64);   // of 64 tokens per wave
   const int32_t* as = assign + (size_t)p * N;
   const int32_t* tk = toks + (size_t)p * N;
@@ -2061,8 +2127,8 @@ extern "C" int ri_kmeans_assign_f16(const void* data, const void* centroids, int
 
 extern "C" size_t ri_kmeans_workspace_bytes(int P, int N, int nc) {
   if (P <= 0 || N <= 0 || nc <= 0) return 0;
-  // digit table [P, 512, chunks] + the tokens by bucket [P, N] for ids of two digits
-  return ((size_t)P * KM_SORT_MAX_BINS * km_sort_chunks(N) + (size_t)P * N) * sizeof(int32_t);
+  // digit table [P, 512, chunks] + the tokens by bucket [P, N] for ids of two digits + where the buckets start [P, 512]
+  return ((size_t)P * KM_SORT_MAX_BINS * (km_sort_chunks(N) + 1) + (size_t)P * N) * sizeof(int32_t);
 }
 
 static int km_build_lists(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P, int N,
@@ -2078,21 +2144,35 @@ static int km_build_lists(const int32_t* assign, int32_t* counts, int32_t* offse
     return RI_OK;
   }
   const dim3 cgrid(nchunks, P);
-  km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, N, nchunks, lo_bits, hi_bits);
-  RI_HIP_CHECK_LAUNCH();
-  // (a single digit: the scan itself yields offsets and counts)
+  // (a single digit: its starts are offsets, and its counts theirs)
   const bool single = lo_bits == 0;
-  km_sort_scan_kernel<<<P, 1024, 0, s>>>(chunk_hist, nchunks << hi_bits, single ? offsets : nullptr,
-                                         single ? counts : nullptr, nchunks, nc, N);
-  RI_HIP_CHECK_LAUNCH();
   const bool packed = (uint64_t)N << lo_bits <= 1ull << 32;
-  km_sort_scatter_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, single ? members : toks, N, nchunks, lo_bits, hi_bits,
-                                               single || !packed ? -1 : lo_bits);
+  const int low = single || !packed ? -1 : lo_bits;
+  // Without the scan's launch, whole clusterings of ten lists, us: 1 x 20000 tokens, 512 centroids 349.4 -> 333.4, 1 x 40000, 2496 592.2 ->
+  // 582.8, 4 x 32768, 2048 894.2 -> 884.8, 8 x 17000, 544 571.4 -> 567.7, 8 x 20000, 640 631.3 -> 630.0, 8 x 131072, 8192 (a table of 16384)
+  // 10093 -> 10071, prefills (one list) the same.  Larger tables would be another round of every workgroup's loads, ids of less
+  // than 6 bits more rows than threads add up.
+  const bool table = hi_bits >= 6 && (long long)nchunks << hi_bits <= KM_SORT_TABLE && !ri_misaligned16(chunk_hist);
+  int32_t* const starts = table ? toks + (size_t)P * N : chunk_hist;
+  km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, N, nchunks, lo_bits, hi_bits, table);
+  RI_HIP_CHECK_LAUNCH();
+  if (table) {
+    km_sort_scatter_kernel<false><<<cgrid, 256, 0, s>>>(
+        assign, chunk_hist, single ? members : toks, N, nchunks, lo_bits, hi_bits, low,
+        KmFirsts{single ? nullptr : starts, single ? offsets : nullptr, counts, nc});
+  } else {
+    km_sort_scan_kernel<<<P, 1024, 0, s>>>(chunk_hist, nchunks << hi_bits, single ? offsets : nullptr,
+                                           single ? counts : nullptr, nchunks, nc, N);
+    RI_HIP_CHECK_LAUNCH();
+    km_sort_scatter_kernel<true><<<cgrid, 256, 0, s>>>(assign, chunk_hist, single ? members : toks, N, nchunks, lo_bits,
+                                                       hi_bits, low, KmFirsts{});
+  }
   RI_HIP_CHECK_LAUNCH();
   if (!single) {
     const int buckets = ((nc - 1) >> lo_bits) + 1;
-    km_bucket_kernel<<<dim3(buckets, P), KM_BUCKET_WAVES * 64, 0, s>>>(assign, toks, chunk_hist, counts, offsets, members, N,
-                                                                       nc, nchunks, lo_bits, buckets, 1 << hi_bits, packed);
+    km_bucket_kernel<<<dim3(buckets, P), KM_BUCKET_WAVES * 64, 0, s>>>(assign, toks, starts, counts, offsets, members, N, nc,
+                                                                       table ? 1 : nchunks, lo_bits, buckets, 1 << hi_bits,
+                                                                       packed);
     RI_HIP_CHECK_LAUNCH();
   }
   return RI_OK;
