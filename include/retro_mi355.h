@@ -600,6 +600,19 @@ int ri_kmeans_store_index_f16(const void* values, int64_t v_head_stride, int64_t
                               void* size16, int32_t* size, int32_t* start, int P, int N, int nc, void* workspace,
                               size_t workspace_bytes, ri_stream_t stream);
 
+/* ri_kmeans_lists_direct (counts, offsets and members are written) and ri_kmeans_store_index, or without `out` ri_kmeans_store_rows,
+ * over its lists in one launch, for at most 16384 tokens per head. */
+int ri_kmeans_store_direct(const void* values, int64_t v_head_stride, int64_t v_row_stride, const void* keys,
+                           int64_t k_head_stride, int64_t k_row_stride, const void* mean, const int32_t* assign,
+                           int32_t* counts, int32_t* offsets, int32_t* members, void* value_sum, void* centroids,
+                           void* value_store, void* key_store, int64_t store_stride_rows, void* out, uint8_t* mask,
+                           void* size16, int32_t* size, int32_t* start, int P, int N, int nc, ri_stream_t stream);
+int ri_kmeans_store_direct_f16(const void* values, int64_t v_head_stride, int64_t v_row_stride, const void* keys,
+                               int64_t k_head_stride, int64_t k_row_stride, const void* mean, const int32_t* assign,
+                               int32_t* counts, int32_t* offsets, int32_t* members, void* value_sum, void* centroids,
+                               void* value_store, void* key_store, int64_t store_stride_rows, void* out, uint8_t* mask,
+                               void* size16, int32_t* size, int32_t* start, int P, int N, int nc, ri_stream_t stream);
+
 /* Initial centroids: row trunc(c * (N / nc) + N / nc / 2) of every problem, in float32 (kmeans.py:234-236). */
 int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_stream_t stream);
 

@@ -92,6 +92,8 @@ SIGNATURES = {
     "ri_kmeans_store_rows_f16": (I, [P, I64, I64, P, I64, I64] + [P] * 8 + [I64, I, I, I, P, SZ, P]),
     "ri_kmeans_store_index": (I, [P, I64, I64, P, I64, I64] + [P] * 8 + [I64] + [P] * 5 + [I, I, I, P, SZ, P]),
     "ri_kmeans_store_index_f16": (I, [P, I64, I64, P, I64, I64] + [P] * 8 + [I64] + [P] * 5 + [I, I, I, P, SZ, P]),
+    "ri_kmeans_store_direct": (I, [P, I64, I64, P, I64, I64] + [P] * 9 + [I64] + [P] * 5 + [I, I, I, P]),
+    "ri_kmeans_store_direct_f16": (I, [P, I64, I64, P, I64, I64] + [P] * 9 + [I64] + [P] * 5 + [I, I, I, P]),
     "ri_kmeans_init": (I, [P, P, I, I, I, P]),
     "ri_prefill_split": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, I64, P]),
     "ri_prefill_split_centred": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, P, I64, P]),

@@ -29,7 +29,7 @@ class KMeansResult:
 
 def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_means=True):
     """Everything of the clustering that reads the keys: centroids, assignment, inverted lists.  final_means off: the
-    caller takes the last means over the lists."""
+    caller takes the last means over the lists, which it makes itself where kmeans_store_makes_lists says so."""
     G, N, D = key.shape
     dev = key.device
     nc, S = num_centroids, num_segments
@@ -53,7 +53,9 @@ def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_me
     else:
         r.assign = torch.empty((G, N), dtype=torch.int32, device=dev)
         kernels.kmeans_assign(key, centroids, r.assign, G, N, nc, 1, N)
-    if N <= kernels.KMEANS_DIRECT_MAX_TOKENS and not final_means:
+    if not final_means and kernels.kmeans_store_makes_lists(G, N, nc):
+        pass
+    elif N <= kernels.KMEANS_DIRECT_MAX_TOKENS and not final_means:
         kernels.kmeans_lists_direct(r.assign, r.counts, r.offsets, r.members, G, N, nc)
     elif N <= kernels.KMEANS_DIRECT_MAX_TOKENS:
         kernels.kmeans_update_direct(key, r.assign, centroids, G, N, nc, 1, N, False,
@@ -129,7 +131,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device) if value_sum is None else value_sum
     if key_store is not None:
         kernels.kmeans_store_rows(kernels.aligned_rows(value), key_rows, key_mean, r.counts, r.offsets, r.members,
-                                  r.value_sum, r.centroids, value_store, key_store, G, N, nc, store_stride, index)
+                                  r.value_sum, r.centroids, value_store, key_store, G, N, nc, store_stride, index,
+                                  r.assign if kernels.kmeans_store_makes_lists(G, N, nc) else None)
         return r
     kernels.kmeans_value_sum(kernels.aligned_rows(value), r.counts, r.offsets, r.members, r.value_sum, G, N, nc,
                              store=value_store, store_stride=store_stride)

@@ -1768,11 +1768,56 @@ __host__ __device__ constexpr int km_direct_run(int N) {
   return (N + KM_DIRECT_WAVES * 256 - 1) / (KM_DIRECT_WAVES * 256) * 256;
 }
 
-template <bool HALF, int CPW, bool NARROW>
-__global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
+// The values and keys of a list, tokens list[k0 .. k1-1], in sums and copies as km_sum_rows makes them (s: two dims of the values,
+// two of the keys less their mean).  Both rows of sixteen tokens are on their way before the first is added: a load's wait covers
+// the stores in front of it.  VALUES, KEYS: both or one of them.
+struct KmStoreDirect {
+  KmStoreArgs v, k;        // (no partials)
+  const uint16_t* mean;
+  int64_t stride;          // rows of the stores from problem to problem
+  KmIndex X;
+};
+template <bool HALF, bool VALUES, bool KEYS>
+__device__ __forceinline__ void km_store_listed(const uint32_t* rv, size_t pv, const uint32_t* rk, size_t pk, const uint16_t* list,
+                                                int k0, int k1, float (&s)[4], uint32_t* wv, uint32_t* wk, uint32_t mean) {
+  const int lane = threadIdx.x & 63;
+  for (int k = k0; k < k1; k += 16) {
+    const int n = min(16, k1 - k), token = list[k + min(lane & 15, n - 1)];
+    uint32_t v[16], x[16];
+#pragma unroll
+    for (int e = 0; e < 16; e += 8)
+      if (e < n) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) {
+          const size_t t = (uint32_t)__builtin_amdgcn_readlane(token, j);
+          if (VALUES) v[j] = (rv + t * pv)[(uint32_t)lane];
+          if (KEYS) x[j] = (rk + t * pk)[(uint32_t)lane];
+        }
+      }
+#pragma unroll
+    for (int e = 0; e < 16; e += 8) {
+      if (e >= n) break;
+#pragma unroll
+      for (int j = e; j < e + 8; ++j) {
+        if (VALUES) ri_add2<HALF>(j < n ? v[j] : 0u, s[0], s[1]);
+        if (KEYS) ri_add2<HALF>(j < n ? ri_sub2<HALF>(x[j], mean) : 0u, s[2], s[3]);
+      }
+#pragma unroll
+      for (int j = e; j < e + 8; ++j)
+        if (j < n) {
+          if (VALUES) __builtin_nontemporal_store(v[j], wv + (size_t)(k + j) * (RI_DIM / 2));
+          if (KEYS) __builtin_nontemporal_store(x[j], wk + (size_t)(k + j) * (RI_DIM / 2));
+        }
+    }
+  }
+}
+
+// STORE: the lists' values and keys are summed and stored as ri_kmeans_store_rows does it, see km_store_direct_kernel.
+template <bool HALF, int CPW, bool NARROW, bool STORE>
+__device__ __forceinline__ void km_direct_group(
     const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent, int N, int nc,
     int shape, int seg, int64_t head_rows, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-    int32_t* __restrict__ listed) {
+    int32_t* __restrict__ listed, const KmStoreDirect& T) {
   constexpr int NW = KM_DIRECT_WAVES, E = CPW * NW / 64;   // E: (cluster, wave) counters per lane
   static_assert((CPW & (CPW - 1)) == 0 && CPW * NW % 64 == 0 && CPW <= 64, "counters dealt to the lanes, a cluster in a byte");
   __shared__ int32_t sh_run[CPW * NW], sh_at[NW][CPW], sh_off[CPW + 1], sh_below[NW];
@@ -1932,16 +1977,88 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
   }
   __syncthreads();
 
-  if (members) {
-    int base = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) base += sh_below[w];
+  int base = 0;   // tokens of lower clusters
+  const auto write_lists = [&]() {
     for (int k = tid; k < sh_off[CPW]; k += NW * 64) members[(size_t)p * N + base + k] = list[k];
     if (tid < CPW && c0 + tid < nc) {
       offsets[(size_t)p * (nc + 1) + c0 + tid] = base + sh_off[tid];
       counts[(size_t)p * nc + c0 + tid] = sh_off[tid + 1] - sh_off[tid];
     }
     if (tid == 0 && c0 + CPW >= nc) offsets[(size_t)p * (nc + 1) + nc] = N;
+  };
+  if (members) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) base += sh_below[w];
+  }
+  if constexpr (STORE) {
+    const uint32_t* const rv = reinterpret_cast<const uint32_t*>(T.v.rows) + (size_t)p * T.v.head_stride;
+    const uint32_t* const rk = reinterpret_cast<const uint32_t*>(T.k.rows) + (size_t)p * T.k.head_stride;
+    const size_t first = ((size_t)p * T.stride + base) * (RI_DIM / 2) + lane, clusters = (size_t)p * nc + c0;
+    uint32_t* const wv = reinterpret_cast<uint32_t*>(T.v.copy) + first;
+    uint32_t* const wk = reinterpret_cast<uint32_t*>(T.k.copy) + first;
+    uint32_t* const sums = reinterpret_cast<uint32_t*>(T.v.out) + clusters * (RI_DIM / 2) + lane;
+    uint32_t* const means = reinterpret_cast<uint32_t*>(T.k.out) + clusters * (RI_DIM / 2) + lane;
+    const uint32_t mean = reinterpret_cast<const uint32_t*>(T.mean)[p * (RI_DIM / 2) + lane];
+    const auto finish_keys = [&](int c, int o, int s, float s0, float s1) {
+      const uint32_t word = km_finish<true, HALF>(s0, s1, s, 0, means + c * (RI_DIM / 2));
+      if (T.X.out) km_entry<HALF>(T.X, clusters + c, s, base + o, word, mean);
+    };
+    bool longer = false;
+    for (int c = wave; c < CPW && c0 + c < nc; c += NW) {
+      const int o = sh_off[c], s = sh_off[c + 1] - o;
+      if (s == 0) {   // zero value sum; the centroid stays
+        sums[c * (RI_DIM / 2)] = 0u;
+        if (T.X.out) km_entry<HALF>(T.X, clusters + c, 0, base + o, means[c * (RI_DIM / 2)], mean);
+        continue;
+      }
+      if (s > KM_BLK) {
+        longer = true;
+        continue;
+      }
+      float x[4] = {0.f, 0.f, 0.f, 0.f};
+      km_store_listed<HALF, true, true>(rv, T.v.pitch, rk, T.k.pitch, list, o, o + s, x, wv, wk, mean);
+      km_finish<false, HALF>(x[0], x[1], s, 0, sums + c * (RI_DIM / 2));
+      finish_keys(c, o, s, x[2], x[3]);
+    }
+    write_lists();
+    if (!__syncthreads_or(longer)) return;
+    // Lists of several blocks, values then keys: the blocks dealt to the waves, their sums (512 bytes each, at most N / 128 of
+    // them) where the compacted tokens were, then added in order.
+    float2* const part = reinterpret_cast<float2*>(sh_buf);
+    const auto blocks = [&](auto keys) {
+      constexpr bool KEYS = decltype(keys)::value;
+      for (int fold = 0; fold < 2; ++fold) {
+        for (int c = 0, item = 0; c < CPW; ++c) {
+          const int o = sh_off[c], s = sh_off[c + 1] - o, nb = (s + KM_BLK - 1) / KM_BLK;
+          if (nb < 2) continue;
+          if (!fold) {
+            for (int b = 0; b < nb; ++b)
+              if (((item + b) & (NW - 1)) == wave) {
+                float x[4] = {0.f, 0.f, 0.f, 0.f};
+                km_store_listed<HALF, !KEYS, KEYS>(rv, T.v.pitch, rk, T.k.pitch, list, o + b * KM_BLK, o + min(s, (b + 1) * KM_BLK), x,
+                                                   wv, wk, mean);
+                part[(item + b) * 64 + lane] = KEYS ? make_float2(x[2], x[3]) : make_float2(x[0], x[1]);
+              }
+          } else if ((c & (NW - 1)) == wave) {
+            float2 t = part[item * 64 + lane];
+            for (int b = 1; b < nb; ++b) {
+              t.x += part[(item + b) * 64 + lane].x;
+              t.y += part[(item + b) * 64 + lane].y;
+            }
+            if (KEYS) finish_keys(c, o, s, t.x, t.y);
+            else km_finish<false, HALF>(t.x, t.y, s, 0, sums + c * (RI_DIM / 2));
+          }
+          item += nb;
+        }
+        __syncthreads();
+      }
+    };
+    blocks(std::false_type{});
+    blocks(std::true_type{});
+    return;
+  }
+  if (members) {
+    write_lists();
     if (!cent) return;
   }
   const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
@@ -1999,6 +2116,28 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
     }
     km_finish<true, HALF>(t.x, t.y, s, normalize, op + c * (RI_DIM / 2));
   }
+}
+
+template <bool HALF, int CPW, bool NARROW>
+__global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
+    const uint16_t* __restrict__ rows, const int32_t* __restrict__ assign, uint16_t* __restrict__ cent, int N, int nc,
+    int shape, int seg, int64_t head_rows, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ listed) {
+  km_direct_group<HALF, CPW, NARROW, false>(rows, assign, cent, N, nc, shape, seg, head_rows, counts, offsets, listed,
+                                            KmStoreDirect{});
+}
+
+// Lists, value sums, means, stores and index entries of short problems in one launch, where lists, rows and a fold of long lists'
+// blocks are three: the lists stay in LDS, and what bounds it is one chain of assignments, rows and stores instead of
+// three.  Worth it while all workgroups of eight clusters are resident at once (kernels.py); the launch against the three and a prefill, us: 8 x
+// 8192 tokens, 512 clusters 21.1 / 4 + 17.5 + 2.5 to 4, 217.4 -> 214.5; 8 x 2001, 128 12.9 / 3.8 + 8.7 + 2.4, 120.9 -> 118.9; 4 x 1500 113.9 ->
+// 112.1; 4 x 16384 224.2 both; more clusters to a workgroup: 8 x 12000 350.4 -> 353.6, 8 x 16384 346.4 -> 352.4.
+template <bool HALF>
+__global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 4) void km_store_direct_kernel(const int32_t* __restrict__ assign, int N, int nc,
+                                                                                  int shape, int32_t* __restrict__ counts,
+                                                                                  int32_t* __restrict__ offsets,
+                                                                                  int32_t* __restrict__ members, KmStoreDirect T) {
+  km_direct_group<HALF, 8, false, true>(nullptr, assign, nullptr, N, nc, shape, 1, N, counts, offsets, members, T);
 }
 
 // out[p, i, :] = in[p, members[p, i], :]; 16 lanes per row; strides in 16-byte pieces
@@ -2475,23 +2614,32 @@ extern "C" int ri_kmeans_value_rows_f16(const void* values, int64_t head_stride,
                              store_stride_rows, P, N, nc, workspace, workspace_bytes, stream);
 }
 
-template <bool HALF>
-static int km_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
-                         const void* mean, const int32_t* counts, const int32_t* offsets, const int32_t* members,
-                         void* value_sum, void* centroids, void* value_store, void* key_store, int64_t store_stride_rows,
-                         int P, int N, int nc, void* workspace, size_t workspace_bytes, hipStream_t s,
-                         const KmIndex& X = KmIndex{}) {
-  if (!values || !keys || !mean || !counts || !offsets || !members || !value_sum || !centroids || !value_store ||
-      !key_store || !workspace)
+static int km_store_args(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
+                         const void* mean, const void* counts, const void* offsets, const void* members, const void* value_sum,
+                         const void* centroids, const void* value_store, const void* key_store, int64_t store_stride_rows, int P,
+                         int N, int nc) {
+  if (!values || !keys || !mean || !counts || !offsets || !members || !value_sum || !centroids || !value_store || !key_store)
     return RI_ERR_ARG;
-  if (ri_any_misaligned16(values, value_sum, value_store, workspace) ||
-      ri_any_misaligned16(keys, centroids, key_store, mean))
+  if (ri_any_misaligned16(values, value_sum, value_store) || ri_any_misaligned16(keys, centroids, key_store, mean))
     return RI_ERR_ARG;
   int rc = km_check(P, N, nc);
   if (rc) return rc;
   if (v_head < 0 || k_head < 0 || v_row < RI_DIM || k_row < RI_DIM || (v_head | v_row | k_head | k_row) % 8 != 0 ||
       store_stride_rows < N)
     return RI_ERR_ARG;
+  return RI_OK;
+}
+
+template <bool HALF>
+static int km_store_rows(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head, int64_t k_row,
+                         const void* mean, const int32_t* counts, const int32_t* offsets, const int32_t* members,
+                         void* value_sum, void* centroids, void* value_store, void* key_store, int64_t store_stride_rows,
+                         int P, int N, int nc, void* workspace, size_t workspace_bytes, hipStream_t s,
+                         const KmIndex& X = KmIndex{}) {
+  int rc = km_store_args(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum, centroids,
+                         value_store, key_store, store_stride_rows, P, N, nc);
+  if (rc) return rc;
+  if (!workspace || ri_misaligned16(workspace)) return RI_ERR_ARG;
   const size_t each = ri_kmeans_reduce_workspace_bytes(P, N, nc);
   if (workspace_bytes < 2 * each) return RI_ERR_WORKSPACE;
   const int cap = km_item_cap(N), item_wgs = (cap + 3) / 4;
@@ -2520,6 +2668,47 @@ static int km_store_index(const void* values, int64_t v_head, int64_t v_row, con
   const KmIndex X = {(uint32_t*)out, mask, (uint16_t*)size16, size, start};
   return km_store_rows<HALF>(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum, centroids,
                              value_store, key_store, store_stride_rows, P, N, nc, workspace, workspace_bytes, s, X);
+}
+
+template <bool HALF>
+static int km_store_direct(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,
+                           int64_t k_row, const void* mean, const int32_t* assign, int32_t* counts, int32_t* offsets,
+                           int32_t* members, void* value_sum, void* centroids, void* value_store, void* key_store,
+                           int64_t store_stride_rows, void* out, uint8_t* mask, void* size16, int32_t* size,
+                           int32_t* start, int P, int N, int nc, hipStream_t s) {
+  int rc = km_store_args(values, v_head, v_row, keys, k_head, k_row, mean, counts, offsets, members, value_sum, centroids,
+                         value_store, key_store, store_stride_rows, P, N, nc);
+  if (rc) return rc;
+  if (!assign || N > KM_DIRECT_MAX || (out && (!mask || !size16 || !size || !start || ri_misaligned16(out)))) return RI_ERR_ARG;
+  const KmStoreDirect T = {{(const uint16_t*)values, (uint16_t*)value_sum, (uint16_t*)value_store, nullptr, (size_t)v_row / 2, v_head / 2},
+                           {(const uint16_t*)keys, (uint16_t*)centroids, (uint16_t*)key_store, nullptr, (size_t)k_row / 2, k_head / 2},
+                           (const uint16_t*)mean, store_stride_rows, {(uint32_t*)out, mask, (uint16_t*)size16, size, start}};
+  const size_t lds = (size_t)km_direct_run(N) * KM_DIRECT_WAVES * 6 + 512;
+  const int shape = km_together(P) | ((P >> km_together(P)) - 1) << 3;
+  km_store_direct_kernel<HALF><<<km_grid((nc + 7) / 8, P), KM_DIRECT_WAVES * 64, lds, s>>>(assign, N, nc, shape, counts, offsets,
+                                                                                            members, T);
+  RI_HIP_CHECK_LAUNCH();
+  return RI_OK;
+}
+
+extern "C" int ri_kmeans_store_direct(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,
+                                      int64_t k_row, const void* mean, const int32_t* assign, int32_t* counts, int32_t* offsets,
+                                      int32_t* members, void* value_sum, void* centroids, void* value_store, void* key_store,
+                                      int64_t store_stride_rows, void* out, uint8_t* mask, void* size16, int32_t* size,
+                                      int32_t* start, int P, int N, int nc, ri_stream_t stream) {
+  return km_store_direct<false>(values, v_head, v_row, keys, k_head, k_row, mean, assign, counts, offsets, members, value_sum,
+                                centroids, value_store, key_store, store_stride_rows, out, mask, size16, size, start, P, N, nc,
+                                (hipStream_t)stream);
+}
+
+extern "C" int ri_kmeans_store_direct_f16(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,
+                                          int64_t k_row, const void* mean, const int32_t* assign, int32_t* counts, int32_t* offsets,
+                                          int32_t* members, void* value_sum, void* centroids, void* value_store, void* key_store,
+                                          int64_t store_stride_rows, void* out, uint8_t* mask, void* size16, int32_t* size,
+                                          int32_t* start, int P, int N, int nc, ri_stream_t stream) {
+  return km_store_direct<true>(values, v_head, v_row, keys, k_head, k_row, mean, assign, counts, offsets, members, value_sum,
+                               centroids, value_store, key_store, store_stride_rows, out, mask, size16, size, start, P, N, nc,
+                               (hipStream_t)stream);
 }
 
 extern "C" int ri_kmeans_store_index(const void* values, int64_t v_head, int64_t v_row, const void* keys, int64_t k_head,

@@ -672,15 +672,29 @@ def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot
                                                     _stream()), "kmeans_value_sum")
 
 
+def kmeans_store_makes_lists(P, N, nc):
+    """Whether the stores are made from the assignment, with the lists, in one launch: short problems whose workgroups of eight
+    clusters are resident at once, two to each of 256 compute units (8 x 8192 tokens, 512 clusters: a prefill 217.4 -> 214.5 us;
+    of twice as many clusters 346 -> 352)."""
+    return N <= KMEANS_DIRECT_MAX_TOKENS and P * ((nc + 7) // 8) <= 512
+
+
 def kmeans_store_rows(values, keys, mean, counts, offsets, members, value_sum, centroids, value_store, key_store, P, N, nc,
-                      store_stride, index=None):
+                      store_stride, index=None, assign=None):
     """Value sums and means of the centred keys, with both stores; values/keys [P, N, 128], strided or not.
-    index: (out, mask, size16, size, start) of prefill_index, filled as well."""
-    ws = _workspace(2 * lib().ri_kmeans_reduce_workspace_bytes(P, N, nc), values.device, "kmeans_store")
+    index: (out, mask, size16, size, start) of prefill_index, filled as well.  assign (up to KMEANS_DIRECT_MAX_TOKENS tokens): the
+    lists are made from it and written on the way."""
     vh, vr = _row_strides(values, "kmeans_store_rows")
     kh, kr = _row_strides(keys, "kmeans_store_rows")
     if not values.dtype == keys.dtype == mean.dtype == value_store.dtype == key_store.dtype:
         raise TypeError("kmeans_store_rows: values, keys and the stores must have the same element type")
+    if assign is not None:
+        check(_fn("ri_kmeans_store_direct", values.dtype)(
+            _p(values), vh, vr, _p(keys), kh, kr, _p(mean), _p(assign), _p(counts), _p(offsets), _p(members), _p(value_sum),
+            _p(centroids), _p(value_store), _p(key_store), store_stride, *(_p(t) for t in index or (None,) * 5), P, N, nc,
+            _stream()), "kmeans_store_rows")
+        return
+    ws = _workspace(2 * lib().ri_kmeans_reduce_workspace_bytes(P, N, nc), values.device, "kmeans_store")
     fn = _fn("ri_kmeans_store_rows" if index is None else "ri_kmeans_store_index", values.dtype)
     check(fn(_p(values), vh, vr, _p(keys), kh, kr, _p(mean), _p(counts), _p(offsets), _p(members), _p(value_sum),
              _p(centroids), _p(value_store), _p(key_store), store_stride, *(_p(t) for t in index or ()), P, N, nc, _p(ws),

@@ -108,6 +108,43 @@ def test_index_entries_on_the_way_to_the_stores(dev, dtype, H, N, nc):
     assert torch.equal(filled[0], plain[0] + mean) and torch.equal(filled[1], counts == 0)
 
 
+# Lists made in the launch that stores their rows: problems of fewer tokens than a load takes, lists of one block, of just more and
+# of a whole problem, last workgroups of few clusters, the most tokens; rows with strides of their own.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,nc", [(1, 1, 32), (3, 3, 32), (2, 255, 32), (8, 1000, 96), (3, 2051, 128), (8, 8191, 512), (16, 8192, 512),
+                                    (5, 16383, 1024), (33, 2000, 540), (2, 16384, 32)])
+@pytest.mark.parametrize("kind", ["even", "blocks", "one"])
+def test_stores_that_make_the_lists(dev, dtype, H, N, nc, kind):
+    """The lists of ri_kmeans_lists_direct, and over them what the launches that take lists write, bit for bit."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(H * N + nc)
+    rows = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)
+    kv, mean, cent = rows(N, 2, H, 128), rows(H, 1, 128), rows(H, nc, 128)
+    hk, hv = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
+    assign = torch.randint(0, nc - 1, (H, N), generator=g, dtype=torch.int32)
+    if kind == "blocks":   # lists of 256 and 257 tokens, and one of several blocks in the same workgroup's clusters
+        for first, last, c in ((0, 256, nc - 1), (256, 513, 2), (513, 1400, 5), (1400, 2800, 6)):
+            assign[:, first:last] = c
+    elif kind == "one":
+        assign[:] = nc - 2
+    assign = assign[:, torch.randperm(N, generator=g)].contiguous().to(dev)
+
+    def stored(index, made):
+        lists = [torch.full(s, -1, dtype=torch.int32, device=dev) for s in ((H, nc), (H, nc + 1), (H, N))]
+        if not made:
+            kernels.kmeans_lists_direct(assign, *lists, H, N, nc)
+        means, sums = cent.clone(), torch.full_like(cent, 7)
+        stores = [torch.zeros((H, N + 7, 128), dtype=dtype, device=dev) for _ in range(2)]
+        entries = (torch.zeros_like(cent), torch.zeros((H, nc), dtype=torch.bool, device=dev),
+                   torch.zeros((H, nc), dtype=dtype, device=dev), torch.zeros_like(lists[0]), torch.zeros_like(lists[0]))
+        kernels.kmeans_store_rows(hv, hk, mean, *lists, sums, means, *stores, H, N, nc, N + 7, entries if index else None,
+                                  assign if made else None)
+        return (*lists, means, sums, *stores, *entries)
+
+    for index in (True, False):
+        assert all(torch.equal(a, b) for a, b in zip(stored(index, True), stored(index, False)))
+
+
 # where the order of the sum changes (one part, four, eight, sixteen ...; one head has a rule of its own), and around it
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,N", [(1, 1), (1, 1020), (1, 1021), (1, 8193), (1, 16384), (1, 16385), (1, 40007), (2, 3),
