@@ -502,7 +502,9 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   const WaveLds sh = {sh_vt[wave], sh_pb[wave], sh_al[wave], sh_desc[wave], sh_w[wave]};
   if (!KEPT) att_clear<GS_PAD>();
   const int lenB = KEPT ? K.off[P.np] : P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  const int lenA = __builtin_amdgcn_readfirstlane(KEPT ? K.lenA : att_steady_rows(P));
+  // (by itself the attention asks for the zone's length only where there is one to ask for: a round trip in front of its rows, 11.3 ->
+  // 11.6 us of 32 groups of 4 heads, 1900 rows)
+  const int lenA = __builtin_amdgcn_readfirstlane(KEPT ? K.lenA : P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA);
 
   const int wid = split * NW + wave;            // wave of the group
   const bool kv_wave = wid < P.W_kv;
