@@ -197,87 +197,70 @@ __device__ __forceinline__ void wave_rows(int total, int nwaves, uint32_t inv, i
   *r1 = min(total, *r0 + rpw);
 }
 
-// A piece of the output row of head j, dims d .. d + N-1: A / L merged with an earlier part (its output po, its log-sum-exp pl)
-// under the maximum M.
-template <bool HALF, int N>
-__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, int d, float M, float L, const float (&A)[N]) {
-  static_assert(N == 1 || N == 2, "an element or a pair of them");
-  const size_t o = (size_t)g * P.gs + j, at = o * RI_DIM + d;
-  float x[2] = {A[0], N == 2 ? A[N - 1] : 0.f};
+// The output row of head j: A / L merged with an earlier part (its output po, its log-sum-exp pl) under the maximum M.
+// Lane l holds dims 2l and 2l + 1.
+template <bool HALF>
+__device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, float M, float L, float A0, float A1) {
+  const int lane = threadIdx.x & 63;
+  const size_t o = (size_t)g * P.gs + j, at = o * RI_DIM + 2 * lane;
   if (P.prev_lse) {
     const float pl = P.prev_lse[o];
     if (pl != -INFINITY) {  // an empty earlier part carries no weight, whatever its output holds
       float p0, p1;
-      ri_unpack2<HALF>(N == 2 ? *reinterpret_cast<const uint32_t*>(P.prev_out + at) : (uint32_t)P.prev_out[at], p0, p1);
+      ri_unpack2<HALF>(*reinterpret_cast<const uint32_t*>(P.prev_out + at), p0, p1);
       const float M2 = fmaxf(M, pl);
       const float f = M == -INFINITY ? 0.f : __expf(M - M2), fp = __expf(pl - M2);
       L = L * f + fp;
-      x[0] = x[0] * f + fp * p0;
-      x[1] = x[1] * f + fp * p1;
+      A0 = A0 * f + fp * p0;
+      A1 = A1 * f + fp * p1;
       M = M2;
     }
   }
   // nothing attended at all (an empty part): zeros and a log-sum-exp of -inf, not 0/0
   const bool any = L > 0.f;
-  const uint16_t lo = ri_f32_to_e16<HALF>(any ? x[0] / L : 0.f);
-  if (N == 2)
-    *reinterpret_cast<uint32_t*>(P.out + at) = (uint32_t)lo | ((uint32_t)ri_f32_to_e16<HALF>(any ? x[1] / L : 0.f) << 16);
-  else
-    P.out[at] = lo;
-  if (d == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
+  *reinterpret_cast<uint32_t*>(P.out + at) =
+      (uint32_t)ri_f32_to_e16<HALF>(any ? A0 / L : 0.f) | ((uint32_t)ri_f32_to_e16<HALF>(any ? A1 / L : 0.f) << 16);
+  if (lane == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
 }
 
-// How the eight waves share the heads when they merge: N dims per lane, PARTS waves to a head of up to four (one past that),
-// HPW heads of a wave.
+// How the eight waves share the heads when they merge: wave w takes heads w, w + ATT_WAVES, ..., a lane two dims.  (With up to four
+// heads two waves to a head, a dim per lane, are twice the stores, arrivals and requests: eight captured layers of 16 groups of 4
+// heads, 1024 clusters 134.3 -> 136.0 us, the operators' two calls over 32 groups 62.6 -> 63.1.)
 template <int GS_PAD>
 struct HeadShare {
-  static constexpr int PARTS = GS_PAD < ATT_WAVES ? ATT_WAVES / GS_PAD : 1;
-  static constexpr int N = RI_DIM / 64 / PARTS;
-  static constexpr int HPW = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;
-  static_assert(N == 1 || N == 2, "a wave covers a head or half of one");
-  static __device__ __forceinline__ int head(int wave, int k) { return PARTS > 1 ? wave % GS_PAD : wave + k * ATT_WAVES; }
-  static __device__ __forceinline__ int dim(int wave, int lane) { return N * ((PARTS > 1 ? wave / GS_PAD * 64 : 0) + lane); }
+  static constexpr int HPW = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;   // heads of a wave
+  static __device__ __forceinline__ int head(int wave, int k) { return wave + k * ATT_WAVES; }
 };
 
 // Merges a wave's share of the S split partials of group g (and the optional previous result) and writes the output: lanes
-// first cover the splits (statistics), then N dims each.
+// first cover the splits (statistics), then two dims each.
 // The partials come from the memory side, where a load takes about a microsecond: a wave requests the statistics of its
 // heads and sixteen splits of them at a time before it looks at any.
 // (One head after the other: 13600 cycles for 16 heads over 3 splits.)
 template <int GS_PAD, bool HALF>
 __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int wave) {
   typedef HeadShare<GS_PAD> Share;
-  constexpr int HPW = Share::HPW, N = Share::N, U = 8;   // U: splits requested without a condition
+  constexpr int HPW = Share::HPW, U = 8;   // U: splits requested without a condition
   const int gs = P.gs, S = P.S;
   const int lane = threadIdx.x & 63;
-  const int d = Share::dim(wave, lane);
   int head[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) head[k] = min(Share::head(wave, k), gs - 1);
   const float* ml = P.part_ml + (size_t)g * S * GS_PAD * 2;
-  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + d;
+  const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + 2 * lane;
   float2 ms[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + head[k]) * 2);
-  float a[2][U][HPW][N];
+  float2 a[2][U][HPW];
   const auto request = [&](int b, int s0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int k = 0; k < HPW; ++k) {
-        const float* p = pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + head[k]) * RI_DIM;
-        if (N == 2) {
-          const float2 x = ri_ld_partial(p);
-          a[b][u][k][0] = x.x;
-          a[b][u][k][N - 1] = x.y;
-        } else {
-          a[b][u][k][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
+      for (int k = 0; k < HPW; ++k) a[b][u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + head[k]) * RI_DIM);
   };
   request(0, 0);
   if (S > U) request(1, U);
-  float f[HPW], M[HPW], L[HPW], A[HPW][N];
+  float f[HPW], M[HPW], L[HPW], A0[HPW], A1[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
     const float m = lane < S ? ms[k].x : -INFINITY;
@@ -286,8 +269,7 @@ __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int 
     f[k] = m == -INFINITY ? 0.f : __expf(m - M[k]);
     L[k] = ri_row_sum(ms[k].y * f[k]);
     L[k] = ri_xor_sum<32>(ri_xor_sum<16>(L[k]));
-#pragma unroll
-    for (int n = 0; n < N; ++n) A[k][n] = 0.f;
+    A0[k] = A1[k] = 0.f;
   }
   const auto add = [&](int b, int s0) {   // (a split past the last has no weight: f of its lane is 0)
 #pragma unroll
@@ -296,8 +278,8 @@ __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int 
       for (int k = 0; k < HPW; ++k) {
         const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[k]), (s0 + u) & 63));
         const float w = s0 + u < S ? fs : 0.f;
-#pragma unroll
-        for (int n = 0; n < N; ++n) A[k][n] += a[b][u][k][n] * w;
+        A0[k] += a[b][u][k].x * w;
+        A1[k] += a[b][u][k].y * w;
       }
   };
   for (int s0 = 0;; s0 += 2 * U) {
@@ -310,7 +292,7 @@ __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int 
   }
 #pragma unroll
   for (int k = 0; k < HPW; ++k)
-    if (Share::head(wave, k) < gs) write_head<HALF, N>(P, g, head[k], d, M[k], L[k], A[k]);
+    if (Share::head(wave, k) < gs) write_head<HALF>(P, g, head[k], M[k], L[k], A0[k], A1[k]);
 }
 
 #define ATT_DESC_MAX 64  // rows of one wave whose descriptors are staged in LDS at a time (32 and 128 measured slower)
@@ -664,12 +646,11 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
 
   // ---------------- merge the waves: each takes its share of the heads ----------------
   typedef HeadShare<GS_PAD> Share;
-  const int d = Share::dim(wave, lane);
 #pragma unroll
   for (int k = 0; k < Share::HPW; ++k) {
     const int j = Share::head(wave, k);
     if (j >= gs) break;
-    float m[NW], M = -INFINITY, a[Share::N] = {}, l = 0.f;
+    float m[NW], M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       m[w] = sh_m[w][j];
@@ -678,24 +659,21 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float f = m[w] == -INFINITY ? 0.f : __expf(m[w] - M);
-      const float* x = acc_of(w) + j * RI_DIM + d;
-#pragma unroll
-      for (int n = 0; n < Share::N; ++n) a[n] += x[n] * f;
+      const float2 x = *reinterpret_cast<const float2*>(acc_of(w) + j * RI_DIM + 2 * lane);
+      a0 += x.x * f;
+      a1 += x.y * f;
       l += sh_l[w][j] * f;
     }
     if (S == 1) {   // the workgroup has the whole group: no partial leaves it
-      write_head<HALF, Share::N>(P, g, j, d, M, l, a);
+      write_head<HALF>(P, g, j, M, l, a0, a1);
       continue;
     }
     const size_t o = ((size_t)g * S + split) * GS_PAD + j;
     // device-coherent stores: another workgroup of this launch reads them
-    if (Share::N == 2)
-      __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + d]),
-                         (uint64_t)__float_as_uint(a[0]) | (uint64_t)__float_as_uint(a[Share::N - 1]) << 32, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    else
-      __hip_atomic_store(&P.part_acc[o * RI_DIM + d], a[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (lane == 0)   // (of a head's waves each for itself: the last of its own kind reads it)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_acc[o * RI_DIM + 2 * lane]),
+                       (uint64_t)__float_as_uint(a0) | (uint64_t)__float_as_uint(a1) << 32, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0)
       __hip_atomic_store(reinterpret_cast<uint64_t*>(&P.part_ml[o * 2]),
                          (uint64_t)__float_as_uint(M) | (uint64_t)__float_as_uint(l) << 32, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
