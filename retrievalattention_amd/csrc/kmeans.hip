@@ -2266,8 +2266,8 @@ extern "C" int ri_kmeans_assign_f16(const void* data, const void* centroids, int
 
 extern "C" size_t ri_kmeans_workspace_bytes(int P, int N, int nc) {
   if (P <= 0 || N <= 0 || nc <= 0) return 0;
-  // digit table [P, 512, chunks] + the tokens by bucket [P, N] for ids of two digits + where the buckets start [P, 512]
-  return ((size_t)P * KM_SORT_MAX_BINS * (km_sort_chunks(N) + 1) + (size_t)P * N) * sizeof(int32_t);
+  // digit table [P, 512, chunks] + the tokens by bucket [P, N] for ids of two digits
+  return ((size_t)P * KM_SORT_MAX_BINS * km_sort_chunks(N) + (size_t)P * N) * sizeof(int32_t);
 }
 
 static int km_build_lists(const int32_t* assign, int32_t* counts, int32_t* offsets, int32_t* members, int P, int N,
@@ -2291,8 +2291,9 @@ static int km_build_lists(const int32_t* assign, int32_t* counts, int32_t* offse
   // 582.8, 4 x 32768, 2048 894.2 -> 884.8, 8 x 17000, 544 571.4 -> 567.7, 8 x 20000, 640 631.3 -> 630.0, 8 x 131072, 8192 (a table of 16384)
   // 10093 -> 10071, prefills (one list) the same.  Larger tables would be another round of every workgroup's loads, ids of less
   // than 6 bits more rows than threads add up.
-  const bool table = hi_bits >= 6 && (long long)nchunks << hi_bits <= KM_SORT_TABLE && !ri_misaligned16(chunk_hist);
-  int32_t* const starts = table ? toks + (size_t)P * N : chunk_hist;
+  // (Where the buckets start lies behind the table, whose room is for 512 digits; 512 buckets leave none.)
+  const bool table = hi_bits >= 6 && (single || hi_bits < 9) && (long long)nchunks << hi_bits <= KM_SORT_TABLE && !ri_misaligned16(chunk_hist);
+  int32_t* const starts = table ? chunk_hist + ((size_t)P * nchunks << hi_bits) : chunk_hist;
   km_sort_hist_kernel<<<cgrid, 256, 0, s>>>(assign, chunk_hist, N, nchunks, lo_bits, hi_bits, table);
   RI_HIP_CHECK_LAUNCH();
   if (table) {

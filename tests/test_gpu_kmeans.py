@@ -514,8 +514,8 @@ def test_iterate_hands_assignments_over(dev, G, N, nc, seg, kind):
 
 
 # Tables of digit counts that the scatter adds up itself and the smallest that a launch scans: whole ids of 6, 7 and 9 bits and
-# ids of two digits on both sides of 16384 counts, fewer than 64 digits, last chunks of one token.
+# ids of two digits on both sides of 16384 counts, fewer than 64 digits, 512 buckets, last chunks of one token.
 @pytest.mark.parametrize("P,N,nc", [(2, 262144, 64), (2, 262145, 64), (1, 131073, 100), (3, 32768, 512), (3, 32769, 512), (2, 131072, 8192),
-                                    (2, 131073, 8192), (5, 16385, 33), (2, 20000, 32), (3, 17409, 544), (1, 33793, 16384)])
+                                    (2, 131073, 8192), (5, 16385, 33), (2, 20000, 32), (3, 17409, 544), (1, 33793, 16384), (2, 32768, 16384)])
 def test_build_lists_on_both_sides_of_the_table(dev, P, N, nc):
     test_build_lists_is_a_stable_sort(dev, P, N, nc, N % 97)
