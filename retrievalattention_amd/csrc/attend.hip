@@ -55,7 +55,8 @@ __global__ __launch_bounds__(64 * ATT_WAVES, 2) void attend_kernel(ri_ptr4 in, r
 
 // workgroups per group at most: one per compute unit for all groups together (plan_splits)
 static int attn_max_splits(int BG) { return min(RI_MAX_SPLITS, max(256 / BG, 1)); }
-static_assert(128 * ATT_WAVES * ATT_COUNTER_PITCH <= RI_MAX_GROUPS, "more than one workgroup per group: up to 128 groups");
+static constexpr bool counters_fit(int BG) { return BG * ATT_WAVES * attend_counter_pitch(BG) <= RI_MAX_GROUPS; }
+static_assert(counters_fit(16) && counters_fit(32) && counters_fit(64) && counters_fit(128), "more than one workgroup per group: up to 128 groups");
 
 static size_t attn_workspace_bytes(int BG, int gs) {
   if (BG <= 0 || BG > RI_MAX_GROUPS || gs <= 0 || gs > 16) return 0;
@@ -74,6 +75,7 @@ static size_t attn_scratch_used(int BG, int gp, int S) {
 
 static void carve_workspace(AttendParams& P, void* workspace, int BG, int gp) {
   P.counters = (int*)workspace;
+  P.pitch = attend_counter_pitch(BG);
   P.part_ml = (float*)((char*)workspace + RI_MAX_GROUPS * sizeof(int));
   P.part_acc = P.part_ml + (size_t)BG * P.S * gp * 2;
 }

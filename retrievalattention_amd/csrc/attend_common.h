@@ -127,7 +127,6 @@ __device__ __forceinline__ float2 ri_ld_partial(const float* p) {
 }
 
 #define ATT_WAVES 8                // waves of a workgroup
-#define ATT_COUNTER_PITCH 4        // words between arrival counters: four to a line of 64 bytes
 #define ATT_FLAG_A 0x40000000     // descriptor bit: row lives in region A
 #define ATT_SKIP (int)0x80000000  // descriptor bit (the sign): the row is read but not attended
 
@@ -171,7 +170,8 @@ struct AttendParams {
   // partials and the arrival counters (zero between launches)
   float* part_ml;   // [BG, S, GS_PAD, 2]
   float* part_acc;  // [BG, S, GS_PAD, 128]
-  int* counters;    // [BG, ATT_WAVES] ATT_COUNTER_PITCH apart
+  int* counters;    // [BG, ATT_WAVES] pitch words apart (attend_counter_pitch)
+  int pitch;
   int S;     // workgroups per group
   int W_kv;  // of the group's S * ATT_WAVES waves the first W_kv take key/value rows, the others estimation rows
   int W_one; // the same of one workgroup's waves, if it takes the whole group
@@ -707,7 +707,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   if (Share::head(wave, 0) >= gs) return;
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0);
-  int* const arrived = P.counters + (g * NW + wave) * ATT_COUNTER_PITCH;
+  int* const arrived = P.counters + (g * NW + wave) * P.pitch;
   int before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(before) != S - 1) return;

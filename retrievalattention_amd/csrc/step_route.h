@@ -1,5 +1,5 @@
 // Which decode steps one workgroup per group makes in one launch (step_kernel), which several do, and which are scoring +
-// selection and attention in launches of their own.  Host code only.
+// selection and attention in launches of their own; where an attention's workgroups count their arrivals.  Host code only.
 #pragma once
 #include <stdint.h>
 
@@ -11,6 +11,12 @@ static inline int gs_pad_of(int gs) { return gs <= 4 ? 4 : (gs <= 8 ? 8 : 16); }
 // Groups that an attention launch gives one workgroup each: few rows (fewer the more heads share their arithmetic), or no
 // compute unit left for a second one.
 static inline bool attend_alone(int64_t rows, int gs, int BG) { return rows * gs_pad_of(gs) <= 384 * 4 || BG > 128; }
+
+// Words between the arrival counters of a launch's waves, eight to a group of more than one workgroup, which up to 128 groups
+// have (attend_common.h).  Every arrival is an atomic at the memory side, where those on one line wait for each other: counters have
+// lines of their own while there is room.  Four counters to 64 bytes / one to a line of 128, us: 2 groups of 8 heads, 15100 rows
+// 13.8 / 12.4, 1 of 8, 40000 18.0 / 16.5, 8 of 8, 20000 21.2 / 19.3, 6 of 8, 3000 9.4 / 9.1; half a line the same.
+static constexpr int attend_counter_pitch(int BG) { return BG <= 16 ? 32 : BG <= 32 ? 16 : BG <= 64 ? 8 : 4; }
 
 // Short: what one workgroup may have to itself (step_is_alone: and does).  It scores for itself (select.hip), and usually (16
 // tokens per retrieved cluster) has no more rows than it attends as fast as two launches do (figures of both, before

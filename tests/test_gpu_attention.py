@@ -378,6 +378,22 @@ def test_split_merge_shares(dev, BG, gs):
             assert torch.allclose(lse.cpu().reshape(BG, gs), x.logsumexp(-1), rtol=0, atol=1e-4)
 
 
+def test_workspace_serves_other_group_counts(dev):
+    """Arrivals of few groups are counted elsewhere than those of many: one workspace, launches of all distances in turn, against
+    fp32 over the same rows (2^-8 of a value each, of which a norm sees a fraction)."""
+    from retrievalattention_amd import kernels
+    scratch, g = kernels.Scratch(), torch.Generator().manual_seed(1)
+    S = 900
+    q, k, v = (torch.randn(128, *s, 128, generator=g).to(torch.bfloat16) for s in ((1, 4), (S, 1), (S, 1)))
+    x = torch.matmul(q[:, 0].float(), k[:, :, 0].float().transpose(1, 2).contiguous()) / math.sqrt(128)
+    want = torch.matmul(x.softmax(-1), v[:, :, 0].float())
+    q, k, v = q.to(dev), k.to(dev), v.to(dev)
+    for BG in (128, 1, 65, 16, 64, 17, 33, 2, 32, 128):
+        for _ in range(2):
+            out = kernels.weighted_flash_decoding(q[:BG], k[:BG], v[:BG], scratch=scratch)
+            assert (out.float().cpu().view(BG, 4, 128) - want[:BG]).norm() <= 4e-3 * want[:BG].norm()
+
+
 @pytest.mark.parametrize("n_clusters,np_", [(40, 3), (300, 64), (300, 65), (600, 129), (4096, 4096)])
 def test_rank_tables_of_empty_and_crowded_clusters(dev, n_clusters, np_):
     """Ranks found by whole waves: runs of empty clusters longer than a wave, clusters of thousands of rows, one to 64 ranks per

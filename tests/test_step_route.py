@@ -1,4 +1,5 @@
-"""Which decode steps one workgroup per group makes (csrc/step_route.h, host code: compiled here by g++)."""
+"""Which decode steps one workgroup per group makes, and where arrivals are counted (csrc/step_route.h, host code: compiled here by
+g++)."""
 import ctypes
 import os
 import shutil
@@ -11,16 +12,19 @@ from retrievalattention_amd._lib import DecodeStep
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def _route(tmp_path_factory, name):
+def _compiled(tmp_path_factory, function):
     if shutil.which("g++") is None:
         pytest.skip("no g++")
     where = tmp_path_factory.mktemp("route")
-    (where / "route.cpp").write_text('#include "step_route.h"\nextern "C" int ask(const ri_decode_step_t* s, int n) '
-                                     f'{{ return step_{name}(s, n); }}\n')
+    (where / "route.cpp").write_text(f'#include "step_route.h"\nextern "C" int ask{function}\n')
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "retrievalattention_amd", "csrc"), str(where / "route.cpp"), "-o",
                     str(where / "route.so")], check=True)
-    call = ctypes.CDLL(str(where / "route.so")).ask
+    return ctypes.CDLL(str(where / "route.so")).ask
+
+
+def _route(tmp_path_factory, name):
+    call = _compiled(tmp_path_factory, f"(const ri_decode_step_t* s, int n) {{ return step_{name}(s, n); }}")
 
     def short(static_len, zone=323, on_device=False, BG=8, gs=4, nc=512, np=9, es=118, page=8, max_pages=72, store=8192,
               sizes=True):
@@ -80,3 +84,12 @@ def test_captured_steps_of_many_groups_keep_one_workgroup_for_longer(is_alone):
         assert not is_alone(69, zone=end - 89, on_device=True, BG=BG, np=4, es=26)
         assert not is_alone(line - 89, zone=end - 90, on_device=True, BG=BG, np=4, es=26)
     assert is_alone(5000, BG=129)
+
+
+def test_arrival_counters_have_lines_of_their_own(tmp_path_factory):
+    """Eight counters a group for the up to 128 groups that have more than one workgroup, in 4096 words: a line of 128 bytes each up
+    to 16 groups, half a line up to 32."""
+    pitch = _compiled(tmp_path_factory, "(int groups) { return attend_counter_pitch(groups); }")
+    for groups in range(1, 129):
+        assert groups * 8 * pitch(groups) <= 4096
+        assert pitch(groups) >= (32 if groups <= 16 else 16 if groups <= 32 else 4)
