@@ -223,43 +223,39 @@ __device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, 
   if (lane == 0 && P.lse_out) P.lse_out[o] = M + __logf(L);
 }
 
-// How the eight waves share the heads when they merge: wave w takes heads w, w + ATT_WAVES, ..., a lane two dims.  (With up to four
+// The eight waves share the heads when they merge: wave w takes heads w, w + ATT_WAVES, ..., a lane two dims.  (With up to four
 // heads two waves to a head, a dim per lane, are twice the stores, arrivals and requests: eight captured layers of 16 groups of 4
 // heads, 1024 clusters 134.3 -> 136.0 us, the operators' two calls over 32 groups 62.6 -> 63.1.)
 template <int GS_PAD>
-struct HeadShare {
-  static constexpr int HPW = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;   // heads of a wave
-  static __device__ __forceinline__ int head(int wave, int k) { return wave + k * ATT_WAVES; }
-};
+constexpr int ATT_HEADS_OF_WAVE = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;
 
 // Merges a wave's share of the S split partials of group g (and the optional previous result) and writes the output: lanes
 // first cover the splits (statistics), then two dims each.
-// The partials come from the memory side, where a load takes about a microsecond: a wave requests the statistics of its
-// heads and sixteen splits of them at a time before it looks at any.
-// (One head after the other: 13600 cycles for 16 heads over 3 splits.)
+// The partials come from the memory side, where a load takes about a microsecond and one compute unit gets 20 KB per
+// microsecond: a wave requests the statistics of its heads and then eight splits of them at a time.  (One head after the other:
+// 13600 cycles for 16 heads over 3 splits.  Sixteen splits on their way: their registers and conditions cost more than the round trips,
+// the attention by itself 1 group of 16 heads, 100000 rows 30.9 -> 32.8 us, 4 of 12, 24000 19.4 -> 20.3, 8 of 8, 6000 10.5 -> 10.9.)
 template <int GS_PAD, bool HALF>
 __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int wave) {
-  typedef HeadShare<GS_PAD> Share;
-  constexpr int HPW = Share::HPW, U = 8;   // U: splits requested without a condition
+  constexpr int HPW = ATT_HEADS_OF_WAVE<GS_PAD>, U = 8;   // U: splits requested at a time
   const int gs = P.gs, S = P.S;
   const int lane = threadIdx.x & 63;
   int head[HPW];
 #pragma unroll
-  for (int k = 0; k < HPW; ++k) head[k] = min(Share::head(wave, k), gs - 1);
+  for (int k = 0; k < HPW; ++k) head[k] = min(wave + k * ATT_WAVES, gs - 1);
   const float* ml = P.part_ml + (size_t)g * S * GS_PAD * 2;
   const float* pa = P.part_acc + (size_t)g * S * GS_PAD * RI_DIM + 2 * lane;
   float2 ms[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) ms[k] = ri_ld_partial(ml + ((size_t)min(lane, S - 1) * GS_PAD + head[k]) * 2);
-  float2 a[2][U][HPW];
-  const auto request = [&](int b, int s0) {
+  float2 a[U][HPW];
+  const auto request = [&](int s0) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int k = 0; k < HPW; ++k) a[b][u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + head[k]) * RI_DIM);
+      for (int k = 0; k < HPW; ++k) a[u][k] = ri_ld_partial(pa + ((size_t)min(s0 + u, S - 1) * GS_PAD + head[k]) * RI_DIM);
   };
-  request(0, 0);
-  if (S > U) request(1, U);
+  request(0);
   float f[HPW], M[HPW], L[HPW], A0[HPW], A1[HPW];
 #pragma unroll
   for (int k = 0; k < HPW; ++k) {
@@ -271,28 +267,21 @@ __device__ __forceinline__ void combine_share(const AttendParams& P, int g, int 
     L[k] = ri_xor_sum<32>(ri_xor_sum<16>(L[k]));
     A0[k] = A1[k] = 0.f;
   }
-  const auto add = [&](int b, int s0) {   // (a split past the last has no weight: f of its lane is 0)
+  for (int s0 = 0; s0 < S; s0 += U) {   // (a split past the last has no weight: f of its lane is 0)
+    if (s0) request(s0);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int k = 0; k < HPW; ++k) {
         const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f[k]), (s0 + u) & 63));
         const float w = s0 + u < S ? fs : 0.f;
-        A0[k] += a[b][u][k].x * w;
-        A1[k] += a[b][u][k].y * w;
+        A0[k] += a[u][k].x * w;
+        A1[k] += a[u][k].y * w;
       }
-  };
-  for (int s0 = 0;; s0 += 2 * U) {
-    add(0, s0);
-    if (s0 + U >= S) break;
-    if (s0 + 2 * U < S) request(0, s0 + 2 * U);
-    add(1, s0 + U);
-    if (s0 + 2 * U >= S) break;
-    if (s0 + 3 * U < S) request(1, s0 + 3 * U);
   }
 #pragma unroll
   for (int k = 0; k < HPW; ++k)
-    if (Share::head(wave, k) < gs) write_head<HALF>(P, g, head[k], M[k], L[k], A0[k], A1[k]);
+    if (wave + k * ATT_WAVES < gs) write_head<HALF>(P, g, head[k], M[k], L[k], A0[k], A1[k]);
 }
 
 #define ATT_DESC_MAX 64  // rows of one wave whose descriptors are staged in LDS at a time (32 and 128 measured slower)
@@ -645,10 +634,9 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   __syncthreads();
 
   // ---------------- merge the waves: each takes its share of the heads ----------------
-  typedef HeadShare<GS_PAD> Share;
 #pragma unroll
-  for (int k = 0; k < Share::HPW; ++k) {
-    const int j = Share::head(wave, k);
+  for (int k = 0; k < ATT_HEADS_OF_WAVE<GS_PAD>; ++k) {
+    const int j = wave + k * NW;
     if (j >= gs) break;
     float m[NW], M = -INFINITY, a0 = 0.f, a1 = 0.f, l = 0.f;
 #pragma unroll
@@ -704,7 +692,7 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "the partial hand-off below relies on gfx950 cache behaviour: build this file for gfx950 only"
 #endif
-  if (Share::head(wave, 0) >= gs) return;
+  if (wave >= gs) return;
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0);
   int* const arrived = P.counters + (g * NW + wave) * P.pitch;

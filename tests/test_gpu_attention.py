@@ -358,12 +358,12 @@ def _hide_rows(gen, S, runs):
 
 @pytest.mark.parametrize("BG,gs", [(1, 1), (2, 4), (3, 5), (8, 8), (11, 16), (128, 3), (129, 3)])
 def test_split_merge_shares(dev, BG, gs):
-    """Every head's share of the merge (two waves to a head, one, two heads to a wave; with up to 64 splits, and none past 128
+    """Every head's share of the merge (a head to a wave, two with sixteen heads; with up to all 64 splits, and none past 128
     groups), over and over on one workspace, with an earlier part and the log-sum-exp: against fp32 over the same rows.
     Probabilities and outputs are 16 bits wide: 2^-8 of a value each, of which a norm sees a fraction."""
     from retrievalattention_amd import kernels
     g = torch.Generator().manual_seed(BG + gs)
-    for S in (700, 5003):
+    for S in (700, 5003, 20011):
         S = S if BG < 100 else S // 10
         q, k, v = (torch.randn(BG, *s, 128, generator=g).to(torch.bfloat16) for s in ((1, gs), (S, 1), (S, 1)))
         x = torch.einsum("bhd,bsd->bhs", q[:, 0].float(), k[:, :, 0].float()) / math.sqrt(128)
