@@ -687,18 +687,21 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   // stale line.  The C++ memory model would express this with a release increment and an acquire on the
   // last arriver; at agent scope those compile to a write-back and an invalidate of the whole L2, which
   // was measured at +15 us per launch (35.2 us instead of 20.0 us at the benchmark shape), while the
-  // data that must be ordered is only this wave's own 2 KB.  The asm statement keeps the compiler
-  // from moving the stores below the wait.
+  // data that must be ordered is only this wave's own 2 KB.  Neither the wait nor relaxed atomics keep the compiler from moving
+  // memory accesses over them, so empty asm statements do: the first keeps the stores above the wait, the second the increment
+  // below it, the third the loads of the partials below the test of the count.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
 #error "the partial hand-off below relies on gfx950 cache behaviour: build this file for gfx950 only"
 #endif
   if (wave >= gs) return;
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0);
+  asm volatile("" ::: "memory");
   int* const arrived = P.counters + (g * NW + wave) * P.pitch;
   int before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(before) != S - 1) return;
+  asm volatile("" ::: "memory");
   combine_share<GS_PAD, HALF>(P, g, wave);
   if (threadIdx.x == 0 && P.valid_lengths) P.valid_lengths[g] = lenA + lenB;
   // ready for the next launch (every arrival of this launch has been counted; launches that share the
