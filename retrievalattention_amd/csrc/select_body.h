@@ -118,10 +118,18 @@ struct SelectKept {
 enum { KEEP_NONE, KEEP_TABLES };
 
 // Bins of the rank search.  Scores are sums of at most sixteen probabilities: in bfloat16 (128 keys to an octave) a bin for
-// each of the 4094 keys up to that of 16, 2^-28 the lowest, finds a rank in one pass; the first bin and the last hold what lies
-// beyond, and where a rank falls there the search is made again by the keys' upper bits.  Half has too many keys for that.
+// each of the 4031 keys up to that of 16, 1.5 * 2^-28 the lowest, finds a rank in one pass; the first 64 bins and the last hold what
+// lies beyond, and where a rank falls there the search is made again by the keys' upper bits.  Half has too many keys for that.
+// 64: what lies below is dealt to them by lane.  Peaked heads leave most of their clusters there, and on one bin those are one
+// atomic after the other.  Where only the estimation zone's rank falls there and a thread has one key or two (BYTES), the keys below
+// are searched by their upper bytes and then by the lower ones, which is less than the whole search again; of more keys the code of it
+// costs all other steps more (16 groups of 2 heads, 10 % of 2496 clusters 25.2 -> 25.5).  Captured layers whose heads are as
+// peaked, us, always two histograms / one bin below and the whole search again / as it is: 2 groups of 8 heads, 8192 clusters 27.7 / 33.3 /
+// 27.0; 32 of 4, 8192 47.1 / 52.7 / 45.0; 16 of 4, 1024 18.8 / 19.9 / 18.9; 8 of 4, 512 17.2 / 17.7 / 16.7; a selection by itself, 8 of
+// 8, 4096 14.1 / 18.4 / 15.3.  Keys inside cost an instruction for two.
 #define SEL_SPAN 4096
-#define SEL_WINDOW 0xB182u   // bin 0: keys up to this one; bin SEL_SPAN - 2: the key of 16.0, 0xC180
+#define SEL_WINDOW 0xB182u   // keys from here on have a bin, but see SEL_BELOW; bin SEL_SPAN - 2: the key of 16.0, 0xC180
+#define SEL_BELOW 64         // bins that what lies below the next one's key shares
 #define SEL_SHIFT 4          // by the upper bits: lower bits of a key
 #define SEL_RUN 32u          // longest run of a bin that its entries put in order by looking at all of it
 template <int NT>
@@ -152,6 +160,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
   constexpr int BPT = SEL_SPAN / NT, FB = 1 << SEL_SHIFT;   // bins of a thread, fine bins
   static_assert(IDS <= 16384 * 2 && E <= 32, "counts in half a word, owned keys in one");
+  constexpr bool BYTES = E <= 2;   // the estimation zone's rank below the window is found by two small passes, see SEL_BELOW
   __shared__ __attribute__((aligned(16))) uint32_t sh_own[KEEP ? 4 : SEL_SCRATCH<NT>];
   uint32_t* const hist = KEEP ? K.scratch : sh_own;   // bins; also the exchange area of the sort
   uint32_t* const sh_rank = hist + SEL_SPAN;          // [3][NT] entries, sizes and first rows in rank order
@@ -401,6 +410,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
   // ---- rank thresholds: T1 = key of descending rank np-1, T2 = key of rank k2-1 ----
   // Afterwards a bin's word holds the keys above the bin, and in the upper half its own.
   bool window = !HALF;
+  uint32_t spread = window ? (uint32_t)lane * 0x10001u : 0u;   // the least bin of either key
   uint32_t C1, s1, C2, s2;
   for (;;) {   // (twice at most: by the window, then by the upper bits)
 #pragma unroll
@@ -408,7 +418,8 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       if (8 * o < nown) {
 #pragma unroll
         for (int v = 4 * o; v < 4 * o + 4 && v < KW; ++v) {
-          const uint32_t b = sel_bins(kw[v], window);
+          const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(sel_pair, sel_bins(kw[v], window)),
+                                                                                     __builtin_bit_cast(sel_pair, spread)));
           atomicAdd(&hist[b & 0xffffu], 1u);
           if (E > 1) atomicAdd(&hist[b >> 16], 1u);
         }
@@ -462,10 +473,12 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     s1 = __builtin_amdgcn_readfirstlane(sh_sel[1]);
     C2 = __builtin_amdgcn_readfirstlane(sh_sel[2]);
     s2 = __builtin_amdgcn_readfirstlane(sh_sel[3]);
-    // (the first and the last bin of the window hold everything beyond it)
-    if (!window || (C2 > 0 && C1 < SEL_SPAN - 1)) break;
+    // (the last bin holds everything above the window, the first ones everything below)
+    if (__builtin_expect(!window || ((BYTES ? C1 : C2) >= SEL_BELOW && C1 < SEL_SPAN - 1), 1)) break;
     window = false;
+    spread = 0u;
     clear_bins();
+    if (tid == 0) sh_sel[4] = 0u;
     lds_barrier();
   }
   uint32_t T1, T2, g1, g2;   // g1, g2: keys strictly above T1 / T2
@@ -474,6 +487,40 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     T2 = SEL_WINDOW + C2;
     g1 = s1;
     g2 = s2;
+    if (BYTES && __builtin_expect(C2 < SEL_BELOW, 0)) {   // of the keys below, by their upper bytes, then the lower ones of the rank's
+      uint32_t* const byte = sh_rank;   // [2][256]
+      static_assert(3 * NT >= 512, "room for them");
+      for (int i = tid; i < 512; i += NT) byte[i] = 0u;
+      lds_barrier();
+      const auto count = [&](auto&& at) {
+#pragma unroll
+        for (int o = 0; o < EIGHTS; ++o)
+          if (8 * o < nown) {
+#pragma unroll
+            for (int i = 8 * o; i < 8 * o + 8 && i < E; ++i)
+              if (key_of(i) < SEL_WINDOW + SEL_BELOW) at(key_of(i));
+          }
+        lds_barrier();
+      };
+      // the bin of rank `rank` counted from the top, which becomes the rank in the bin
+      const auto find = [&](const uint32_t* f, uint32_t& rank) {
+        const uint4 x = *reinterpret_cast<const uint4*>(f + 252 - 4 * lane);   // lane l: bins 255 - 4 l to 252 - 4 l
+        const uint32_t n = x.x + x.y + x.z + x.w, inc = ri_wave_incl_scan(n);
+        const int l = __ffsll((long long)__ballot(inc > rank)) - 1;
+        rank -= (uint32_t)__builtin_amdgcn_readlane((int)(inc - n), l);
+        uint32_t bin = 255 - 4 * l;
+        const uint32_t c[3] = {(uint32_t)__builtin_amdgcn_readlane((int)x.w, l), (uint32_t)__builtin_amdgcn_readlane((int)x.z, l),
+                               (uint32_t)__builtin_amdgcn_readlane((int)x.y, l)};
+        for (int i = 0; i < 3 && rank >= c[i]; ++i) { rank -= c[i]; --bin; }
+        return bin;
+      };
+      uint32_t rank = (uint32_t)k2 - 1 - (hist[SEL_BELOW - 1] & 0xffffu);   // (keys above the last of the shared bins)
+      count([&](uint32_t k) { atomicAdd(&byte[k >> 8], 1u); });
+      const uint32_t upper = find(byte, rank);
+      count([&](uint32_t k) { if (k >> 8 == upper) atomicAdd(&byte[256 + (k & 255)], 1u); });
+      T2 = upper << 8 | find(byte + 256, rank);
+      g2 = (uint32_t)k2 - 1 - rank;   // (rank: of the last key among those equal to T2)
+    }
   } else {
 #pragma unroll
     for (int o = 0; o < EIGHTS; ++o)

@@ -296,6 +296,27 @@ def test_score_select_rank_search(dev, spread, gs, nc, nprobe, es, dt):
     assert torch.equal(meta.cpu()[:, 0].long(), kept) and torch.equal(off.cpu().long(), offs)
 
 
+@pytest.mark.parametrize("gs,nc,nprobe,es", [(4, 512, 20, 119), (8, 1024, 40, 240), (4, 8192, 147, 1900), (1, 16384, 1024, 3800)])
+@pytest.mark.parametrize("octave", [27.0, 27.3, 27.41, 27.5, 27.9, 28.1, 30.0])
+def test_score_select_around_the_lowest_score_with_a_bin(dev, octave, gs, nc, nprobe, es):
+    """A few clusters that hold all the probability and the others around 2^-octave, on both sides of the lowest score that the
+    rank search has a bin for, some masked: the zones are the oracle's on the kernel's own scores, to the id."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator().manual_seed(nc + int(100 * octave))
+    u = torch.randint(0, 2, (2, 1, 128), generator=g) * 2.0 - 1     # a logit is the centroid's factor times sqrt(128)
+    tops = nprobe // 2
+    factor = 0.03 * torch.randn(2, nc, 1, generator=g)
+    factor[:, torch.randperm(nc, generator=g)[:tops]] = (octave * math.log(2) + math.log(gs / tops)) / 128 ** 0.5
+    q, cent = u.expand(2, gs, 128).to(torch.bfloat16).to(dev), (factor * u).to(torch.bfloat16).to(dev)
+    mask = (torch.rand(2, nc, generator=g) < 0.3).to(torch.uint8)
+    ret, est = (torch.empty(2, n, dtype=torch.int32, device=dev) for n in (nprobe, es))
+    dist = torch.empty(2, nc, dtype=torch.bfloat16, device=dev)
+    kernels.score_select(q, cent, mask.to(dev), None, None, torch.empty(2, gs, nc, device=dev), dist, None, ret, est, None, None,
+                         None, nprobe, es, 8, 8192, 128 ** -0.5)
+    ret_x, est_x = scoring.select(dist.cpu(), nprobe, es)
+    assert torch.equal(ret.cpu().long(), ret_x) and torch.equal(est.cpu().long(), est_x)
+
+
 def test_score_select_page_cutoff(dev):
     """A tiny execution buffer forces the reference's cut-off: clusters after the first one that
     does not fit are dropped (wave_buffer_cpu.cpp:207-216)."""
