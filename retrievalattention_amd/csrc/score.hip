@@ -188,6 +188,9 @@ __global__ __launch_bounds__(1024) void softmax_kernel(const uint4* __restrict__
 // four / two / one: 64 groups of 8 heads, 16384 clusters 125.7 / 123.1 / 140; four / two: 64 of 4, 16384 122.9 / 119.9, 128 of 4, 8192
 // 121.1 / 118.3, 48 of 8, 16384 104.5 / 103.0, 64 of 12, 16384 138.3 / 137.3; two rounds: 64 of 4, 8192 70.3 / 69.7, 32 of 4, 16384 71.3 /
 // 70.9, but 128 of 8, 4096 74.3 / 74.9; less: 24 of 4, 16384 59.7 / 59.9, 32 of 8, 8192 44.3 / 45.1.  (Three to a unit 126.2 in the first.)
+// Where the scores go out in 16 bits and a softmax reads them back, only up to four heads, or from six rounds on.  Four / two to a
+// unit, inputs in turn: 64 of 4, 16384 56.2 / 54.0, 96 of 4, 8192 43.6 / 42.9, but 96 of 8, 8192 47.8 / 48.0, 48 of 12, 16384 51.0 / 51.9, 128 of
+// 16, 8192 71.9 / 72.3 (the same input again, 64 of 8, 16384 51.8 / 53.5); six rounds, 96 of 8, 16384 90.1 / 87.2, of 12 96.8 / 95.5.
 static size_t score_spread(int64_t workgroups) { return workgroups >= 3 * 1024 ? 56 * 1024 : 0; }
 
 // ------------------------------------------------------------------------------------
@@ -210,8 +213,10 @@ static int batch_gemm_softmax_impl(const void* A, const void* B, void* D, float*
   const int ntiles = (n + SCORE_TILE - 1) / SCORE_TILE;
   // fp32 logits are not part of this interface: the partial statistics come from the fp32
   // accumulators inside the kernel, the softmax from the 16-bit D, as in the reference.
-  score_kernel<HALF, 4, 4, false><<<dim3(ntiles, batch_count), 256, score_spread((int64_t)ntiles * batch_count), s>>>((const uint16_t*)A, (const uint16_t*)B, nullptr,
-                                                                  (uint16_t*)D, Norm, Sum, m, n, ntiles, alpha);
+  const int64_t workgroups = (int64_t)ntiles * batch_count;
+  const size_t spread = m <= 4 || workgroups >= 6 * 1024 ? score_spread(workgroups) : 0;
+  score_kernel<HALF, 4, 4, false><<<dim3(ntiles, batch_count), 256, spread, s>>>(
+      (const uint16_t*)A, (const uint16_t*)B, nullptr, (uint16_t*)D, Norm, Sum, m, n, ntiles, alpha);
   RI_HIP_CHECK_LAUNCH();
   const int threads = min(1024, (n / 8 + 63) / 64 * 64);
   softmax_kernel<HALF><<<dim3(m, batch_count), threads, 0, s>>>((const uint4*)D, Norm, Sum, (uint4*)Softmax, ntiles, m,
