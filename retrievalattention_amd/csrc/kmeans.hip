@@ -2129,9 +2129,11 @@ __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 6) void km_direct_kernel(
 
 // Lists, value sums, means, stores and index entries of short problems in one launch, where lists, rows and a fold of long lists'
 // blocks are three: the lists stay in LDS, and what bounds it is one chain of assignments, rows and stores instead of
-// three.  Worth it while all workgroups of eight clusters are resident at once (kernels.py); the launch against the three and a prefill, us: 8 x
-// 8192 tokens, 512 clusters 21.1 / 4 + 17.5 + 2.5 to 4, 217.4 -> 214.5; 8 x 2001, 128 12.9 / 3.8 + 8.7 + 2.4, 120.9 -> 118.9; 4 x 1500 113.9 ->
-// 112.1; 4 x 16384 224.2 both; more clusters to a workgroup: 8 x 12000 350.4 -> 353.6, 8 x 16384 346.4 -> 352.4.
+// three.  Worth it while all workgroups of eight clusters are resident at once: 512 up to 12288 tokens, past them, where one's LDS is
+// 87 KB and more, 256 (kernels.py).  This launch / the three, captured, us: 8 x 8192 tokens, 512 clusters 20.2 / 23.7, 4 x 12288, 768 18.0 /
+// 20.6, 8 x 12288, 512 30.3 / 32.3, 2 x 16384, 1024 14.2 / 15.7; fewer workgroups 2 x 8192 14.2 / 13.8, 1 x 4000 12.2 / 11.9, which
+// whole prefills do not show; more of them than fit 4 x 12300, 768 25.5 / 21.5, 4 x 16384, 1024 25.5 / 22.3, 2 x 16384, 1088 24.0 / 18.4.
+// More clusters to a workgroup, prefills: 8 x 12000 350.4 -> 353.6, 8 x 16384 346.4 -> 352.4.
 template <bool HALF>
 __global__ __launch_bounds__(KM_DIRECT_WAVES * 64, 4) void km_store_direct_kernel(const int32_t* __restrict__ assign, int N, int nc,
                                                                                   int shape, int32_t* __restrict__ counts,

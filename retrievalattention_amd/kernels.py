@@ -674,9 +674,9 @@ def kmeans_value_sum(values, counts, offsets, members, value_sum, P, N, nc, slot
 
 def kmeans_store_makes_lists(P, N, nc):
     """Whether the stores are made from the assignment, with the lists, in one launch: short problems whose workgroups of eight
-    clusters are resident at once, two to each of 256 compute units (8 x 8192 tokens, 512 clusters: a prefill 217.4 -> 214.5 us;
-    of twice as many clusters 346 -> 352)."""
-    return N <= KMEANS_DIRECT_MAX_TOKENS and P * ((nc + 7) // 8) <= 512
+    clusters are resident at once, two to each of 256 compute units up to 12288 tokens, whose lists take 74 KB of LDS, and one to a
+    unit past them (figures at km_store_direct_kernel)."""
+    return N <= KMEANS_DIRECT_MAX_TOKENS and P * ((nc + 7) // 8) <= (512 if N <= 12288 else 256)
 
 
 def kmeans_store_rows(values, keys, mean, counts, offsets, members, value_sum, centroids, value_store, key_store, P, N, nc,

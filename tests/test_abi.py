@@ -54,6 +54,16 @@ def test_passes_know_each_other_where_clusters_are_small():
     assert bytes_(2 * 16384, nc) > bytes_(2 * 16384, nc - 32) + 12 * P * 2 * 16384
 
 
+def test_stores_make_lists_while_their_workgroups_are_resident():
+    """A workgroup for eight clusters, whose LDS lets two to each of 256 compute units up to 12288 tokens and one past them."""
+    from retrievalattention_amd.kernels import kmeans_store_makes_lists as made
+    for N in (1, 8192, 12288):
+        assert made(4, N, 1024) and made(512, N, 8) and not made(4, N, 1025) and not made(513, N, 8)
+    for N in (12289, 16384):
+        assert made(2, N, 1024) and made(256, N, 8) and not made(2, N, 1025) and not made(4, N, 1024)
+    assert not made(1, 16385, 8)
+
+
 def test_missing_library_is_a_loud_error(monkeypatch, tmp_path):
     from retrievalattention_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)
