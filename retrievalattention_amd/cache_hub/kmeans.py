@@ -84,8 +84,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
 
     value_sum: [G, nc, 128] tensor for the sums (else a new one).  value_store: where the value rows are also
     written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
-    key_rows, the [G, N, 128] keys before key_mean was subtracted; index (with key_store): the tensors of
-    kernels.prefill_index, filled on the way.
+    key_rows, the [G, N, 128] keys before key_mean was subtracted.  index (with key_mean): the tensors that
+    kernels.prefill_index fills, filled here, with key_store in its launches.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and of the same
     type, shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -136,6 +136,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
         return r
     kernels.kmeans_value_sum(kernels.aligned_rows(value), r.counts, r.offsets, r.members, r.value_sum, G, N, nc,
                              store=value_store, store_stride=store_stride)
+    if index is not None:
+        kernels.prefill_index(r.centroids, key_mean, r.counts, r.offsets, *index)
     return r
 
 

@@ -394,10 +394,7 @@ class retroinfer_cache(KV_Cache):
         km = segment_k_means_csr(ck, head_values, self.n_centroids, num_segments=self.n_segment,
                                  reuse_graph=True,   # results are consumed below, before the next call
                                  value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride,
-                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k,
-                                 index=None if store_k is None else index)
-        if store_k is None:
-            kernels.prefill_index(km.centroids, mean_key, km.counts, km.offsets, *index)
+                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k, index=index)
         self.store_rows[layer_idx][rows] = [valid_length] * H
         if dev_organise:
             self.mainevents[dkey].record()

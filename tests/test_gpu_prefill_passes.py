@@ -145,6 +145,27 @@ def test_stores_that_make_the_lists(dev, dtype, H, N, nc, kind):
         assert all(torch.equal(a, b) for a, b in zip(stored(index, True), stored(index, False)))
 
 
+@pytest.mark.parametrize("N,nc", [(2000, 128), (20000, 128)])
+def test_clustering_fills_the_index_with_stores_or_without(dev, N, nc):
+    """The index entries that a clustering is handed hold the same, whether it writes the stores as well or not."""
+    from retrievalattention_amd.cache_hub.kmeans import segment_k_means_csr
+    H, dtype = 2, torch.bfloat16
+    g = torch.Generator().manual_seed(N)
+    rows = [torch.randn(H, N, 128, generator=g).to(dtype).to(dev) for _ in range(2)]
+    mean = rows[0].float().mean(dim=1, keepdim=True).to(dtype)
+    got = []
+    for stores in (True, False):
+        entries = (torch.full((H, nc, 128), 7, dtype=dtype, device=dev), torch.ones((H, nc), dtype=torch.bool, device=dev),
+                   *(torch.full((H, nc), -1, dtype=t, device=dev) for t in (dtype, torch.int32, torch.int32)))
+        more = dict(key_rows=rows[0], key_store=torch.empty_like(rows[0]), value_store=torch.empty_like(rows[1]),
+                    store_stride=N) if stores else {}
+        r = segment_k_means_csr(rows[0] - mean, rows[1], nc, 3, key_mean=mean, index=entries, **more)
+        assert torch.equal(entries[0], r.centroids + mean) and torch.equal(entries[3], r.counts)
+        assert torch.equal(entries[4], r.offsets[:, :-1])
+        got.append(entries)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 # where the order of the sum changes (one part, four, eight, sixteen ...; one head has a rule of its own), and around it
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,N", [(1, 1), (1, 1020), (1, 1021), (1, 8193), (1, 16384), (1, 16385), (1, 40007), (2, 3),
