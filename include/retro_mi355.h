@@ -150,8 +150,8 @@ int ri_score_logits_f16(const void* q, const void* centroids, float* logits, int
  *   out = (e^{prev_lse}·prev_out + Σ_r e^{s_r} v_r) / (e^{prev_lse} + Σ_r w_r e^{s_r}),
  *   s_r = scale·q·k_r;  lse_out = log of that denominator.
  *   workspace: ri_flash_decoding_workspace_bytes(BG, gs) bytes of device memory that the
- *   caller zeroes once after allocating it (its head holds per-group arrival counters which
- *   every call leaves at zero again); calls sharing a workspace must not overlap in time.
+ *   caller zeroes once after allocating it (its head holds arrival counters, eight to a group,
+ *   which every call leaves at zero again); calls sharing a workspace must not overlap in time.
  *   BG <= 4096. */
 size_t ri_flash_decoding_workspace_bytes(int BG, int gs);
 /* Clears the arrival counters at the head of an attention workspace (of ri_weighted_flash_decoding,

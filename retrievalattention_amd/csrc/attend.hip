@@ -111,16 +111,19 @@ static int est_row_bytes(int gs, bool scored_here) { return 256 + 32 + (scored_h
 //    leaves units without work between 86 and 255 groups (4 heads over 8192 clusters: 100 groups 33.8 us, 128: 42.0, 160:
 //    58.6, 200: 67.0, 256: 88.8), and is still ahead of the two or more workgroups of four waves per group that it
 //    replaced (42.4, 46.7, 78.7, 86.8, 101.8 us).
-//  * A compute unit reads about 25 KB per microsecond, so more workgroups stream a group's rows faster, but the last
-//    one to arrive reads the partials of all of them at that same rate: the sum of both is least near
-//    sqrt(bytes of the group / bytes of a partial), flat towards fewer (12 groups of 7 heads, 3550 rows: 15 workgroups
-//    11.6 us, 21: 12.0).
-//  * The last one reads the partials eight at a time, so one or two past a multiple of eight cost a round trip: 9 -> 8
-//    workgroups 8.5 -> 7.9 us (16 groups of 4 heads, 623 rows), 17 -> 16 12.1 -> 11.5 (12 groups of 7, 3488), 25 -> 24 10.6 ->
-//    10.2 (4 of 4, 4350), 34 -> 32 14.1 -> 13.7 (2 of 8, 15100).  More than a fifth is not worth giving up, nor
-//    any of them once a wave has more than four chunks (24 groups of 3, 24200 rows: 10 -> 8 took 1.5 % of the step).
+//  * A compute unit reads about 25 KB per microsecond, so more workgroups stream a group's rows faster, but the waves
+//    that come last read the partials of all of them at that same rate: the sum of both is least near
+//    sqrt(bytes of the group / bytes of a partial), flat towards fewer (12 groups of 7 heads in half, 3488 rows: 12 workgroups
+//    9.9 us, 15 and 16 8.9, 21 9.3; 8 of 8, 4000: 12 9.8, 16 8.8, 21 9.3).
+//  * A wave requests eight splits at a time, whether there are as many or not (combine_share), so one or two past a multiple of eight
+//    cost as much as eight: 9 -> 8 workgroups 7.2 -> 6.8 us (16 groups of 4 heads, 623 rows), 17 -> 16 9.3 -> 8.9 (12 of 7, 3488), 26 -> 24
+//    9.2 -> 8.8 (4 of 4, 4350), 34 -> 32 12.2 -> 11.8 (2 of 8, 15100), 20 -> 16 13.8 -> 12.8 (4 of 12, 8000); layers of captured
+//    steps, 16 groups of 4 heads, 1024 clusters 18.4 -> 17.9, 8 of 8, 8192 28.6 -> 28.2, 4 of 4, 8192 24.7 -> 24.3.  It loses where a wave
+//    gets a second chunk of rows by it: 20 -> 16 7.8 -> 8.3 (8 of 4, 2500), a layer of 1 of 8, 8192 24.6 -> 25.4, 12 of 7 24.2 -> 24.5.
+//    More than a fifth is not worth giving up, nor any of them once a wave has more than four chunks.
 //  * A few rows (less of them the more heads share their arithmetic) stay with one workgroup, which hands no partial to
-//    another: 8 groups of 4 heads, 331 rows: 6.7 us against 7.2 for three workgroups.
+//    another: one, two and three workgroups, 8 groups of 4 heads, 331 rows 6.7, 7.5, 6.6 us; of 8 heads, 200 rows 5.9, 7.0, 7.1, 331
+//    7.1, 8.1, 7.1.
 static void plan_splits(AttendParams& P, int64_t kv_rows, int64_t es_rows, int es_row_bytes, int BG, int gs,
                         int max_splits = RI_MAX_SPLITS, bool several = false) {
   const int64_t rows = kv_rows + es_rows, wk = kv_rows * 512, we = es_rows * es_row_bytes;

@@ -224,8 +224,8 @@ __device__ __forceinline__ void write_head(const AttendParams& P, int g, int j, 
 }
 
 // The eight waves share the heads when they merge: wave w takes heads w, w + ATT_WAVES, ..., a lane two dims.  (With up to four
-// heads two waves to a head, a dim per lane, are twice the stores, arrivals and requests: eight captured layers of 16 groups of 4
-// heads, 1024 clusters 134.3 -> 136.0 us, the operators' two calls over 32 groups 62.6 -> 63.1.)
+// heads, two waves to a head and a dim per lane would be twice the stores, arrivals and requests: eight captured layers of 16
+// groups of 4 heads, 1024 clusters 136.0 us instead of 134.3, the five operators over 32 groups 63.1 instead of 62.6.)
 template <int GS_PAD>
 constexpr int ATT_HEADS_OF_WAVE = (GS_PAD + ATT_WAVES - 1) / ATT_WAVES;
 
@@ -342,7 +342,7 @@ __device__ __forceinline__ void attend_rows(WaveState<GS_PAD>& st, const WaveLds
   }
 }
 
-// The eight waves of a workgroup merge in LDS, so a group split over S workgroups hands S partials to its last arriver.
+// The eight waves of a workgroup merge in LDS, so a group split over S workgroups hands S partials to whichever waves come last.
 // The rank tables of the retrieval zone (np + 1 token offsets, np first rows) live in dynamic LDS, sized by
 // the launch, so that any number of probes the selection accepts can be attended.
 // HALF: q, K, V, value sums, cluster sizes, weights and outputs are IEEE half instead of bfloat16.
@@ -473,8 +473,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   const WaveLds sh = {sh_vt[wave], sh_pb[wave], sh_al[wave], sh_desc[wave], sh_w[wave]};
   if (!KEPT) att_clear<GS_PAD>();
   const int lenB = KEPT ? K.off[P.np] : P.lenB_ptr ? P.lenB_ptr[(size_t)g * P.lenB_ptr_stride] : P.lenB_const;
-  // (by itself the attention asks for the zone's length only where there is one to ask for: a round trip in front of its rows, 11.3 ->
-  // 11.6 us of 32 groups of 4 heads, 1900 rows)
+  // (by itself the attention asks for the zone's length only where there is one to ask for: asked for always it is a round trip in
+  // front of its rows, 11.6 instead of 11.3 us of 32 groups of 4 heads, 1900 rows)
   const int lenA = __builtin_amdgcn_readfirstlane(KEPT ? K.lenA : P.lenA_ptr ? min(max(P.lenA_ptr[0], 0), (int)P.strideA) : P.lenA);
 
   const int wid = split * NW + wave;            // wave of the group

@@ -575,15 +575,12 @@ static int score_select_impl(const void* q, const void* centroids, const uint8_t
   float *const tmax = P.tile_max, *const tsum = P.tile_sum;
   uint16_t* const keys = P.keys;
   // One compute unit reads 20 KB per microsecond from memory and up to 100 from its L2.  Its own scoring therefore pays up to
-  // 512 clusters (8 groups of 4 heads: 8.0 us; 640 clusters 10.3 against 10.0 for two launches, 16 groups of 1024 11.8
-  // against 10.7; for 128 groups of 8 heads it is still ahead there, 14.0 against 16.0, but not by what the rule would
-  // cost), its own score sums up to about 112 KB of logits of up to four heads (8 groups of 4, 4096 clusters: 14.4 against
-  // 15.5 us; 32 groups of 4, 7168 clusters 24.5 either way, 8192 28.1 against 27.4; one head, 8192 clusters 16.3 against
-  // 17.3).  Past 4096 clusters a thread holds eight of them: with more than four heads that is 64 logits in registers, and
-  // many compute units are the faster ones again (4 .. 32 groups of 5 and 6 heads, 4104 .. 5728 clusters: 16.1 .. 22.6 us
-  // with dist_kernel, 20.0 .. 26.2 without; 8 heads, 4096 clusters 15.9 without, 16.4 with); so it is past 2048 with more
-  // than eight (8 groups of 9 heads, 3000 clusters 16.2 us with dist_kernel, 18.3 without; 16 of 16, 2048 16.6 without,
-  // 17.7 with).
+  // 512 clusters, what its threads hold (own / two launches, us: 8 groups of 4 heads 7.2 / 7.8, of 8 7.7 / 8.4, of 12 7.8 / 9.8, 128 of 8 8.4 /
+  // 10.6), its own score sums where the logits are few (own / dist_kernel: 16 groups of 4 heads, 1024 clusters 8.2 / 9.8; 8 of 4, 4096 11.0
+  // either way; 16 of 16, 2048 13.3 / 13.6, 8 of 12 12.0 / 12.2).  Past 4096 clusters a thread holds eight of them: with more than
+  // four heads that is 64 logits in registers, and many compute units are the faster ones (4 of 5, 4104 14.5 / 11.8, 32 of 6, 5728 23.2
+  // / 18.6); so it is past 2048 with more than eight (8 of 9, 3000 15.3 / 12.8).  Between those the lines are an earlier dist_kernel's,
+  // and the present one is ahead: 32 of 4, 7168 22.8 / 20.3, 8 of 8, 4096 13.4 / 12.1, one head, 8192 12.5 / 12.4.
   if (nc <= 512) {
     if (nc <= 256) launch_select_heads<256, 1, SEL_SCORE>(P, BG, half, s);
     else launch_select_heads<512, 1, SEL_SCORE>(P, BG, half, s);

@@ -61,18 +61,18 @@ __device__ __forceinline__ void store_selection(const SelectArgs& S, int g, cons
 // step: scoring, selection and attention of a group in one launch, for short contexts.
 // With up to 512 clusters the selection is one workgroup per group that scores for itself: as one kernel with the attention
 // the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
-// host as well.  What bounds it is the chain of either half on one compute unit.  8 groups of 4 heads, 512 clusters, 331
-// rows: 14.9 -> 13.5 us; 8 heads 16.3 -> 14.7; 128 groups 17.6 -> 15.8.  103564 bytes of LDS (113036 with 8 heads): one
-// workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.
+// host as well.  What bounds it is the chain of either half on one compute unit.  Captured layers with their appends, in launches of
+// their own -> one, us: 8 groups of 4 heads, 512 clusters, 331 rows 18.0 -> 16.3; 8 heads 19.0 -> 17.8; 128 groups of 4 20.7 -> 18.7.
+// 103564 bytes of LDS (113036 with 8 heads): one workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.
 // SPLIT: several workgroups per group, which all make the same selection and attend a part of the rows each (see
 // select_attend_kernel): with the query and the zone's length requested behind the first loads and the results stored behind
-// the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 523 / 843 / 1099 rows:
-// 15.0 / 17.3 / 19.8 / 22.7 us with one workgroup, 14.6 / 14.6 / 14.8 / 16.5 with several (16.3 .. 18.8 in two launches); the
-// retrieval of 10 % of the clusters, 8 groups of 8 heads 20.7 -> 19.0 (two launches -> SPLIT), 16 of 4 20.8 -> 19.4, 128 of 8
-// 33.6 -> 31.7.  step_route.h says which step takes which form.  The rows that the clusters hold, and the zone's in a captured
+// the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 521 / 831 / 1331 rows:
+// 17.8 / 20.2 / 21.9 / 27.3 us with one workgroup, 17.0 / 17.1 / 17.0 / 18.6 with several (19.0 / 19.2 / 19.0 / 20.3 in launches of their own);
+// the retrieval of 10 % of the clusters, launches of their own -> SPLIT, 8 groups of 8 heads 22.1 -> 20.1, 16 of 4 21.3 -> 19.5, 128 of 8
+// 35.0 -> 32.4.  step_route.h says which step takes which form.  The rows that the clusters hold, and the zone's in a captured
 // step, are known behind the selection only: where they turn out to be few, one workgroup attends them all and hands no partial
-// over, and another stores the results (captured, 8 groups of 1 head, 4000 tokens 14.6 -> 13.4 us, 1 of 4, 8192 15.0 -> 14.5, 8 of
-// 8, 8192 16.3 -> 16.1, 128 of 8, 8192 23.3 -> 22.4).
+// over, and another stores the results (8 groups of 1 head, 256 clusters 15.8 -> 14.8 us, of 4 heads 16.2 -> 15.0, 128 of 8, 512 23.9 ->
+// 22.9; 8 of 8, 512 17.1 either way).
 // The scoring half is bound by its instructions and waits, not by the centroids' bytes (a quarter of them takes as long): with
 // its own statistics and those of the eight waves made without branches, the clusters' masks not looked at in front of the other
 // loads, and the results stored behind the attention by one workgroup as by several, captured layers took 16.05 -> 15.5 us (8
@@ -136,15 +136,16 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
 // 127.5 / 126.0 in the fourth), and one of the workgroups stores its
 // results when its rows are attended (a load's wait covers the stores in front of it): without both 19.0, 47.5 and 26.2 us in
 // the first, second and third of these steps (captured, 4 layers a graph; in launches of their own -> joined): 16 groups of 4
-// heads, 1024 clusters 21.0 -> 18.9; 32 of 4, 8192 48.8 -> 47.0; 12 of 7, 1920 27.5 -> 25.6; 64 of 8, 16384 139.9 -> 138.2; 8 of
-// 4, 2048 22.3 -> 20.2; 1 of 4, 8192 27.5 -> 25.8; 8 of 8, 4096 28.0 -> 25.9; 32 of 16, 4096 41.2 -> 38.6; 4 of 12, 8192 35.0 ->
-// 33.2; 16 of 1, 1920 22.2 -> 20.0; 320 of 8, 1280 70.2 -> 65.2; 512 of 4, 1024 71.2 -> 68.0.
+// heads, 1024 clusters 20.4 -> 18.0; 32 of 4, 8192 48.0 -> 45.1; 12 of 7, 1920 half 24.8 -> 22.6; 64 of 8, 16384 130.8 -> 128.1; 8 of
+// 4, 2048 21.7 -> 19.6; 1 of 4, 8192 25.2 -> 23.0; 8 of 8, 4096 27.6 -> 23.8; 32 of 16, 4096 38.9 -> 36.2; 4 of 12, 8192 32.4 ->
+// 30.2; 16 of 1, 1920 22.2 -> 19.7; 320 of 8, 1280 72.6 -> 67.4; 512 of 4, 1024 74.4 -> 70.5.
 // What bounds it is the selection's chain (see select_body.h), then what bounds the attention.
-// NT: threads that select; the attention is eight waves' always (with sixteen 16 groups of 4 heads, 1024 clusters take 20.6 us
-// instead of 18.8, 64 of 8, 16384 139.3), and the others leave before it (a barrier counts the waves there are).  512 up to 8192
-// clusters (1024 threads: 16 of 4, 1024 19.2, 32 of 8, 4096 33.9 instead of 32.9, 32 of 4, 8192 48.1 / 47.8), 1024 past them (64 of
-// 8, 16384 138.1 -> 137.5, 8 of 4 39.1 -> 38.5) and for more than 512 probes (in launches of their own -> joined: 32 of 4, 8192
-// clusters, 819 probes 85.9 -> 84.2; 12 of 7, 5760, 576 45.4 -> 43.7; 64 of 8, 8192, 819 157.4 -> 155.2).
+// NT: threads that select; the attention is eight waves' always, and the others leave before it (a barrier counts the waves
+// there are).  512 up to 8192 clusters (512 / 1024 threads: 16 groups of 4 heads, 1024 17.9 / 19.6, 8 of 4, 2048 19.4 / 20.7, 12 of 7, 1920 22.0
+// / 23.8, 32 of 8, 4096 31.1 / 31.6, 32 of 4, 8192 44.0 / 44.3, 8 of 4 25.8 / 25.9), 1024 past them, where it makes no difference any
+// more (64 of 8, 16384 127.9 / 128.2, 8 of 4 33.4 / 33.2), and for more than 512 probes, which 512 threads do not hold (in launches of
+// their own -> joined: 32 of 4, 8192 clusters, 819 probes 85.5 -> 81.9; 12 of 7, 5632, 563 42.2 -> 39.2; 64 of 8, 8192, 819 150.8 ->
+// 146.9).
 // ------------------------------------------------------------------------------------
 template <int NT, int E, int GSM, bool HALF, int SRC>
 __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in, ri_int4 n, ri_int2 m, SelectArgs S0,
@@ -230,10 +231,11 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }
-  // Who sums the scores (dist_kernel / the selecting workgroups, us): 32 groups of 4 heads, 8192 clusters 47.4 / 50.3, 5760 39.1 /
-  // 41.8; of 1, 8192 46.1 / 47.4; 8 of 7, 3808 28.0 / 26.7; 8 of 8, 4096 27.1 / 27.2, 32 of 8 33.2 / 33.8; 8 of 16, 2048 28.9 /
-  // 27.9; 12 of 7, 1920 27.5 / 26.2; 32 of 8, 2048 26.8 / 25.3; 64 of 16, 1024 31.4 / 28.9.  (512 threads: eight clusters each
-  // past 2048, and with sixteen heads that is more than the registers hold.)
+  // Who sums the scores (dist_kernel / the selecting workgroups, captured layers with their appends, us): 32 groups of 4 heads, 8192
+  // clusters 44.8 / 47.6, 5632 36.1 / 38.7, 4096 29.5 / 29.2; 8 of 4, 5632 24.3 / 26.5; of 1, 32 of 8192 42.9 / 44.0; 8 of 16, 2048 26.0 / 25.9;
+  // 64 of 16, 1024 28.8 / 27.6; 12 of 7, 1920 23.0 / 22.0; 32 of 8, 2048 25.7 / 24.7.  Between 2048 and 4096 clusters of five to eight heads
+  // the line is an earlier dist_kernel's, and the present one is ahead: 8 of 7, 3808 23.5 / 24.2; 8 of 8, 4096 23.8 / 24.9, 32 of 8 31.0 / 31.9.
+  // (512 threads: eight clusters each past 2048, and with sixteen heads that is more than the registers hold.)
   const bool keys = S.nc > (S.gs <= 4 ? 4096 : S.gs <= 8 ? min(4096, 28 * 1024 / S.gs) : 2048);
   rc = ri_launch_select_inputs(S, s->BG, s->half, keys, stream);
   if (rc) return rc;

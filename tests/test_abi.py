@@ -37,8 +37,8 @@ def test_status_strings_and_version():
     # two fp32 tile partials per (group, 256-centroid tile, head) and one 16-bit sort key per centroid
     assert l.ri_score_select_workspace_bytes(32, 4, 8192) == 2 * 32 * 32 * 4 * 4 + 32 * 8192 * 2
     assert l.ri_flash_decoding_workspace_bytes(0, 4) == 0
-    # an arrival counter per group that there may be, and two statistics and 128 sums in fp32 per workgroup and (padded) head:
-    # at most a workgroup per compute unit, or one per group, and 64 per group
+    # a word per group that there may be for arrival counters (eight to each of up to 128 groups), and two statistics and 128 sums in
+    # fp32 per workgroup and (padded) head: at most a workgroup per compute unit, or one per group, and 64 per group
     for BG, gs, workgroups, heads in ((32, 4, 256, 4), (24, 7, 240, 8), (300, 16, 300, 16), (1, 1, 64, 4), (4096, 9, 4096, 16)):
         assert l.ri_wave_attention_workspace_bytes(BG, gs) == 4 * 4096 + workgroups * heads * 130 * 4
 
