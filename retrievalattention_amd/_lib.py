@@ -142,6 +142,19 @@ def lib():
     return _lib
 
 
+_step_calls = None
+
+
+def step_calls():
+    """The native module that makes a decode step's calls."""
+    global _step_calls
+    if _step_calls is None:
+        lib()
+        from . import _step_calls as module
+        _step_calls = module
+    return _step_calls
+
+
 def check(status, what):
     if status != 0:
         l = lib()

@@ -1,4 +1,5 @@
-"""Builds libretro_mi355.so (HIP kernels + host wave buffer) for gfx950 with hipcc.
+"""Builds libretro_mi355.so (HIP kernels + host wave buffer) for gfx950 with hipcc, and _step_calls.so (the calls of a decode
+step from Python) with g++.
 
     python -m retrievalattention_amd.build
 
@@ -7,6 +8,7 @@ The library is written next to this file so that it travels with the source tree
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -57,8 +59,25 @@ def build(verbose=False):
                 print(o)
     objs = [j[1] for j in jobs]
     _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB] + objs + ["-pthread"])
+    _run(step_calls_command())
     build_capi_example(hipcc)
     return LIB
+
+
+# The Python calls of a decode step (csrc/step_calls.cpp): a module of its own, because it is bound to this interpreter and to
+# torch, which the library is not.
+STEP_CALLS = os.path.join(HERE, "_step_calls.so")
+
+
+def step_calls_command():
+    import torch
+    from torch.utils import cpp_extension
+    include = [f"-I{d}" for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    libs = [f"-L{d}" for d in cpp_extension.library_paths("cuda") + [HERE]]
+    return ["g++", *CPP_FLAGS, "-O2", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *include,
+            os.path.join(CSRC, "step_calls.cpp"), "-o", STEP_CALLS, *libs, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+            "-lc10_hip", "-l:libretro_mi355.so", "-Wl,-rpath,$ORIGIN"]
 
 
 # A plain HIP program that drives a decode step through the C ABI (no Python, no torch); tests/test_gpu_capi.py

@@ -15,6 +15,7 @@ Two residencies of the clustered K/V:
 Buffer names follow the reference so that code poking at them keeps working.
 """
 import math
+import types
 import warnings
 
 import torch
@@ -38,6 +39,7 @@ class retroinfer_cache(KV_Cache):
     """Calls of one cache work in buffers of the cache and follow one another on a stream.  Decode steps of two caches
     share nothing and may run on two streams at a time."""
     _scratch = None   # kernels.Scratch (None: the process's)
+    _plans = types.MappingProxyType({})   # (layer, buffer) -> prepared step, of an instance
 
     def __init__(self, valid_start, layer_num, batch_size, max_length, num_key_value_heads, num_heads,
                  head_dim, dtype, layer_mapping, max_new_length, static_pattern_start, static_pattern_end, core,
@@ -155,6 +157,7 @@ class retroinfer_cache(KV_Cache):
         self.store_rows = [[0] * BG for _ in L]  # rows of the store in use, per group
         self._plans = {}                         # (layer, buffer) -> DecodeStepPlan of the device-resident step
         self._row_shape = (batch_size, 1, self.kv_head, self.head_dim)
+        self._out_shape = (batch_size, 1, self.num_heads, self.head_dim)
         self._centred_keys = {}                  # (device, tokens) -> buffer of centred keys for the clustering
         if self.kv_residency == "device":
             self._init_device_store()
@@ -527,6 +530,8 @@ class retroinfer_cache(KV_Cache):
         them over (another type, layout, shape or device, a full zone): torch's copies then convert, broadcast or
         raise."""
         k, v = self.steady_zone_keys[layer_idx], self.steady_zone_values[layer_idx]
+        if kernels.append_row(key_states, value_states, k, v, self.static_pattern_total, pos_dev, self._row_shape):
+            return True
         device = k.get_device()
         if device < 0 or self.static_pattern_total >= k.shape[2]:
             return False
@@ -629,10 +634,17 @@ class retroinfer_cache(KV_Cache):
             queries.numel() == self.batch_groups * self.group_size * self.head_dim
 
     def _compute_device(self, queries, layer_idx, static_len, buf):
+        plan = self._plans.get((layer_idx, buf))
+        if plan is not None:
+            out = plan.step(queries, static_len, self._out_shape, self._step_buffers(layer_idx, buf), self._step_numbers())
+            if out is not None:
+                return out
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
         if self._prepared_takes(queries, layer_idx):
             out = queries.new_empty((self.batch_size, 1, self.num_heads, D))
-            self._plan(layer_idx, buf).run(queries, static_len, out)
+            plan = self._plan(layer_idx, buf)
+            plan.run(queries, static_len, out)
+            plan.prepare(self._step_buffers(layer_idx, buf), self._step_numbers())
             return out
         self._select(queries, layer_idx, buf, True)
         out = torch.empty((BG, gs, D), dtype=self.dtype, device=queries.device)
@@ -646,14 +658,21 @@ class retroinfer_cache(KV_Cache):
             static_len_dev=self.steady_len_dev if self.device_positions else None, scratch=self._scratch)
         return out.view(self.batch_size, 1, self.num_heads, D)
 
+    def _step_numbers(self):
+        return self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size
+
+    def _step_buffers(self, layer, buf):
+        """The buffers of a layer's step over a device-resident store, the zone's length on the device (or None) last."""
+        return (self.centroids[layer], self.centroids_mask[layer], self.cluster_size_i32[layer], self.cluster_start[layer],
+                self.logits, self.ret_ids[buf], self.est_ids[buf], self.ret_tok_off, self.ret_start, self.meta,
+                self.steady_zone_keys[layer], self.steady_zone_values[layer], self.list_keys[layer],
+                self.list_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf],
+                self.steady_len_dev if self.device_positions else None)
+
     def _plan(self, layer, buf):
         """The layer's step as one prepared call.  It is prepared again when any buffer has moved since (buffers are
         attributes that the index growth and callers replace)."""
-        t = (self.centroids[layer], self.centroids_mask[layer], self.cluster_size_i32[layer], self.cluster_start[layer],
-             self.logits, self.ret_ids[buf], self.est_ids[buf], self.ret_tok_off, self.ret_start, self.meta,
-             self.steady_zone_keys[layer], self.steady_zone_values[layer], self.list_keys[layer],
-             self.list_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
-        length = self.steady_len_dev if self.device_positions else None
+        *t, length = self._step_buffers(layer, buf)
         key = [x.data_ptr() for x in t]
         key += (None if length is None else length.data_ptr(), self.nprobe, self.es_cluster_num, self.page_size,
                 self.buffer_size)
@@ -668,17 +687,27 @@ class retroinfer_cache(KV_Cache):
                 self.RSQRT_DIM, self._scratch)
         return plan
 
+    def _host_step_buffers(self, layer, buf):
+        """_step_buffers for a host-resident store with the device-side block cache: those of the step, others, the lists, the
+        block cache's state."""
+        _, _, row_src, meta = self.layouts[buf if self.use_cluster_estimation else 0]
+        return (self.centroids[layer], self.centroids_mask[layer], self.logits, self.ret_ids[buf], self.est_ids[buf], meta,
+                self.steady_zone_keys[layer], self.steady_zone_values[layer], self.cache_keys[layer],
+                self.cache_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf],
+                self.cluster_size_i32[layer], self.cluster_start[layer], row_src, self.list_keys[layer],
+                self.list_values[layer], *self._lists(layer), *self.device_lru[layer].state())
+
+    def _host_step_numbers(self, layer):
+        # (a plan keeps its manager, so that no other one has its id)
+        return id(self.device_lru[layer]), self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size
+
     def _host_plan(self, layer, buf):
         """_plan for a host-resident store with the device-side block cache."""
         lru = self.device_lru[layer]
-        _, _, row_src, meta = self.layouts[buf if self.use_cluster_estimation else 0]
-        t = (self.centroids[layer], self.centroids_mask[layer], self.logits, self.ret_ids[buf], self.est_ids[buf], meta,
-             self.steady_zone_keys[layer], self.steady_zone_values[layer], self.cache_keys[layer],
-             self.cache_values[layer], self.value_sum[layer], self.cluster_size[layer], self.valid_lengths[buf])
-        other = (self.cluster_size_i32[layer], self.cluster_start[layer], row_src, self.list_keys[layer],
-                 self.list_values[layer])
-        lists = self._lists(layer)
-        key = [x.data_ptr() for x in (*t, *other, *lists, *lru.state())]
+        buffers = self._host_step_buffers(layer, buf)
+        t, other, lists = buffers[:13], buffers[13:18], buffers[18:30]
+        row_src = other[2]
+        key = [x.data_ptr() for x in buffers]
         key += (lru, self.nprobe, self.es_cluster_num, self.page_size, self.buffer_size)
         plan = self._plans.get((layer, buf))
         if plan is None or not plan.valid(key):
@@ -725,11 +754,19 @@ class retroinfer_cache(KV_Cache):
                                search_next):
         BG, gs, D = self.batch_groups, self.group_size, self.head_dim
         es = self.es_cluster_num
-        if search_here and not search_next and not self.overlap_miss_staging and \
-                self._prepared_takes(queries, layer_idx):
-            out = queries.new_empty((self.batch_size, 1, self.num_heads, D))
-            self._host_plan(layer_idx, buf).run(queries, static_len, out)
-            return out
+        if search_here and not search_next and not self.overlap_miss_staging:
+            plan = self._plans.get((layer_idx, buf))
+            if plan is not None:
+                out = plan.step(queries, static_len, self._out_shape, self._host_step_buffers(layer_idx, buf),
+                                self._host_step_numbers(layer_idx))
+                if out is not None:
+                    return out
+            if self._prepared_takes(queries, layer_idx):
+                out = queries.new_empty((self.batch_size, 1, self.num_heads, D))
+                plan = self._host_plan(layer_idx, buf)
+                plan.run(queries, static_len, out)
+                plan.prepare(self._host_step_buffers(layer_idx, buf), self._host_step_numbers(layer_idx))
+                return out
         q = queries.view(BG, gs, D)
         rows = self.cache_blocks * self.page_size
         stage0 = self.cache_size * self.page_size

@@ -14,7 +14,7 @@ import weakref
 
 import torch
 
-from ._lib import DecodeStep, Lru, lib, check
+from ._lib import DecodeStep, Lru, lib, check, step_calls
 
 # 16-bit element types of the reference's operators and cache (batch_gemm_softmax.cu:185-197,
 # gather_copy.cu:63-67): every wrapper takes either and calls the entry point of that type (name or name_f16).
@@ -176,6 +176,9 @@ MAX_GROUPS = 4096          # ri_wave_attention / ri_weighted_flash_decoding: bat
 # ----------------------------------------------------------------------------------------
 def batch_gemm_softmax(A, B, D, Norm, Sum, Softmax, batch_count, m, n, k, alpha=1.0, beta=0.0):
     """batch_gemm_softmax.cu:201-209.  A [bc, m, k], B [bc, n, k]; D/Softmax [bc, m, n]."""
+    status = step_calls().gemm_softmax(A, B, D, Softmax, Norm, Sum, batch_count, m, n, k, alpha, beta)
+    if status is not None:
+        return check(status, "batch_gemm_softmax") if status else None
     if A.dtype not in _DT:
         raise RuntimeError("Only Half and BFloat16 are supported")      # batch_gemm_softmax.cu:196
     _need_all((A, B, D, Softmax), A.dtype, ("A", "B", "D", "Softmax"))
@@ -193,6 +196,10 @@ def batch_gemm_softmax(A, B, D, Norm, Sum, Softmax, batch_count, m, n, k, alpha=
 def gather_copy_vectors(key_data, key_buffer, value_data, value_buffer, src_metadata, dst_metadata,
                         data_offsets, groups, data_length, buffer_length, index_size, copy_start, copy_num):
     """gather_copy.cu:288-292.  The rows are moved as 16-bit elements: Half or BFloat16 (gather_copy.cu:63-67)."""
+    status = step_calls().gather_vectors(key_data, key_buffer, value_data, value_buffer, src_metadata, dst_metadata, data_offsets,
+                                         groups, data_length, buffer_length, index_size, copy_start, copy_num)
+    if status is not None:
+        return check(status, "gather_copy_vectors") if status else None
     if key_data.dtype not in _DT:
         raise RuntimeError("Only Half and BFloat16 are supported")
     _need_all((key_data, key_buffer, value_data, value_buffer, src_metadata, dst_metadata), key_data.dtype,
@@ -258,6 +265,12 @@ def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_ls
     previous_lse [BG, gs] (any shape with BG*gs elements); cache_seqlens [BG] int32.
     `scratch`: the caller's own Scratch, where calls may overlap others."""
     BG, one, gs, D = q.shape
+    if q.__class__ is torch.Tensor and q.is_cuda and one == 1 and D == 128 and q.dtype in _DT:
+        ws = _workspace(_flash_workspace_bytes(BG, gs), q.device, "attn", scratch)
+        out = step_calls().flash(q, k, v, weight, previous_out, previous_lse, cache_seqlens, ws, 1.0 / math.sqrt(D),
+                                 return_softmax_lse)
+        if out is not None:
+            return check(out, "weighted_flash_decoding") if out.__class__ is int else out
     S = k.shape[1]
     if one != 1 or D != 128 or k.shape[2] != 1:
         raise ValueError("weighted_flash_decoding: expected q [BG,1,gs,128], k/v [BG,S,1,128]")
@@ -455,10 +468,28 @@ class DecodeStepPlan:
             max_pages=max_pages, half=int(dtype == torch.float16), scale=scale,
             **{nm: _p(t) for nm, t in tensors.items()})
         self._address = ctypes.addressof(self._step)
+        self._lru_address = 0
         self._call = lib().ri_decode_step
+        self._native = None
 
     def valid(self, key):
         return self.key == key and self.generation == self._scratch.generation
+
+    def prepare(self, buffers, numbers):
+        """Behind the first call: what `step` compares.  buffers, numbers: tuples of everything that this was prepared from."""
+        if self._native is None and all(t is None or type(t) is torch.Tensor for t in buffers):
+            self._native = step_calls().Step(self._address, self._lru_address, self._tensors["centroids"], buffers,
+                                             (*numbers, self.generation))
+
+    def step(self, q, static_len, out_shape, buffers, numbers):
+        """The call with a new output of out_shape, in native code; None, and nothing launched, where q is not what a prepared
+        call reads or anything of buffers and numbers is not what it was prepared from."""
+        if self._native is None or PROFILER_RANGES:
+            return None
+        out = self._native.run(q, static_len, out_shape, buffers, (*numbers, self._scratch.generation))
+        if out.__class__ is int:
+            check(out, "step")
+        return out
 
     def run(self, q, static_len, out):
         status = self._call(self._address, q.data_ptr(), static_len, out.data_ptr(), _stream())
@@ -486,6 +517,15 @@ class HostStepPlan(DecodeStepPlan):
         status = self._call(self._address, self._lru_address, q.data_ptr(), static_len, out.data_ptr(), _stream())
         if status:
             check(status, "host_step")
+
+
+def append_row(key, value, steady_k, steady_v, pos, pos_dev, row_shape):
+    """append_kv in native code where rows of row_shape and zones [batch, heads, rows, 128] are plain contiguous tensors of one
+    type and device, with room for pos; else False, and nothing launched."""
+    status = step_calls().append(key, value, steady_k, steady_v, pos, pos_dev, row_shape)
+    if status:
+        check(status, "append_kv")
+    return status is not None
 
 
 def append_kv(key, value, steady_k, steady_v, pos, pos_dev=None):

@@ -1,0 +1,113 @@
+"""The native calls of a decode step and of the operators (csrc/step_calls.cpp): what they leave to the general way, and that
+both ways do the same."""
+import math
+
+import pytest
+import torch
+
+from retrievalattention_amd import kernels
+from retrievalattention_amd._lib import step_calls
+
+ROW = (2, 1, 3, 128)
+
+
+def _rows(**change):
+    t = dict(k=torch.zeros(ROW, dtype=torch.bfloat16), v=torch.zeros(ROW, dtype=torch.bfloat16),
+             zk=torch.zeros(2, 3, 5, 128, dtype=torch.bfloat16), zv=torch.zeros(2, 3, 5, 128, dtype=torch.bfloat16), pos=1,
+             at=None, shape=ROW)
+    t.update(change)
+    return t.values()
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_what_is_no_plain_device_tensor_is_left_to_the_general_way():
+    """Host tensors, subclasses and other objects: nothing is launched, and nothing is raised."""
+    native = step_calls()
+    assert native.append(*_rows()) is None
+    assert native.append(*_rows(k=torch.zeros(ROW, dtype=torch.bfloat16).as_subclass(_Sub))) is None
+    assert native.append(*_rows(k=object())) is None and native.append(*_rows(at=3)) is None
+    x = torch.zeros(8, dtype=torch.bfloat16)
+    assert native.gemm_softmax(x, x, x, x, x, x, 1, 1, 1, 128, 1.0, 0.0) is None
+    assert native.gather_vectors(x, x, x, x, x, x, x, 1, 1, 1, 1, 0, 1) is None
+    assert native.flash(x, x, x, None, None, None, None, x, 1.0, False) is None
+    with pytest.raises(TypeError):
+        native.append(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change,takes", [
+    (dict(), True), (dict(pos=4), True), (dict(pos=5), False), (dict(shape=(2, 1, 3)), False), (dict(shape=(2, 3, 1, 128)), False),
+    (dict(zk=torch.zeros(2, 3, 5, 128)), False), (dict(zk=torch.zeros(2, 5, 3, 128, dtype=torch.bfloat16).transpose(1, 2)), False),
+    (dict(k=torch.zeros(2, 3, 1, 128, dtype=torch.bfloat16).transpose(1, 2)), True),
+    (dict(k=torch.zeros(2, 1, 128, 3, dtype=torch.bfloat16).transpose(2, 3)), False),
+    (dict(v=torch.zeros(2 * 3 * 128 + 4, dtype=torch.bfloat16)[4:].view(ROW)), False),
+    (dict(at=torch.tensor([2])), True), (dict(at=torch.tensor([2], dtype=torch.int32)), False),
+    (dict(at=torch.tensor([7])), True)])
+def test_append_takes_rows_as_a_layer_hands_them_over(dev, change, takes):
+    args = [x.to(dev) if isinstance(x, torch.Tensor) else x for x in _rows(**change)]
+    if "v" in change:   # (a copy would be aligned)
+        args[1] = torch.zeros(2 * 3 * 128 + 4, dtype=torch.bfloat16, device=dev)[4:].view(ROW)
+    k, v, zk, zv, pos, at, shape = args
+    k.normal_(), v.normal_()
+    before = zk.clone(), zv.clone()
+    assert kernels.append_row(k, v, zk, zv, pos, at, shape) is takes
+    row = pos if at is None else int(at)
+    if takes and row < 5:
+        before[0][:, :, row], before[1][:, :, row] = k[:, 0], v[:, 0]
+    assert torch.equal(zk, before[0]) and torch.equal(zv, before[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("residency", ["device", "device-pos", "host"])
+def test_step_follows_its_buffers(dev, residency):
+    """A prepared step in native code gives what the general way gives, also behind a buffer that was replaced, another number
+    of probes, and queries of a subclass."""
+    from tests.test_gpu_cache import _gen, _make_cache, _prefill
+    ctx = 1024 + 68
+    cache = _make_cache(dev, residency, 1, 2, 2, 4, ctx, 64, 1, 8, 16)
+    _prefill(cache, *_gen(1, 2, 2, 4, ctx, 64, dev, 5), 1, 2)
+    cache.layer_num = 2   # (no layer is the last one: the same token again)
+    q = torch.randn(2, 1, 8, 128, device=dev).bfloat16()
+    plan = lambda: cache._plans[(0, 0)]
+    general, native = cache.compute(q, 0), cache.compute(q, 0)
+    assert torch.equal(general, native) and native.shape == general.shape and plan()._native is not None
+    first = plan()
+    cache.value_sum[0] = cache.value_sum[0].clone() * 2
+    moved = cache.compute(q, 0)
+    assert plan() is not first and not torch.equal(moved, general)
+    assert torch.equal(cache.compute(q, 0), moved)
+    assert torch.equal(cache.compute(q.as_subclass(_Sub), 0).as_subclass(torch.Tensor), moved)
+    cache.nprobe -= 1
+    other = cache.compute(q, 0)
+    assert not torch.equal(other, moved) and torch.equal(cache.compute(q, 0), other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_operators_natively_and_in_general(dev, dtype):
+    """The same call with plain tensors and with a subclass, which takes the general way."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    r = lambda *s, dt=dtype: torch.randn(s, generator=g, device=dev).to(dt)
+    BG, gs, n, rows = 3, 5, 264, 40
+    q, cent, keys, values, weight = r(BG, 1, gs, 128), r(BG, n, 128), r(BG, rows, 1, 128), r(BG, rows, 1, 128), \
+        r(BG, 1, 1, rows).abs()
+    lengths = torch.tensor([40, 7, 23], dtype=torch.int32, device=dev)
+    ids = torch.stack([torch.randperm(n, generator=g, device=dev) for _ in range(BG)])
+    results = []
+    for of in (lambda t: t, lambda t: t.as_subclass(_Sub)):
+        product, softmax = (torch.zeros(BG, gs, n, dtype=dtype, device=dev) for _ in range(2))
+        norm, total = (torch.zeros(BG, 2, gs, device=dev) for _ in range(2))
+        kernels.batch_gemm_softmax(of(q), cent, product, norm, total, softmax, BG, gs, n, 128, 1 / math.sqrt(128))
+        bk, bv, bs = torch.zeros_like(keys), torch.zeros_like(values), torch.zeros_like(weight)
+        kernels.gather_copy_vectors(of(cent), bk, cent, bv, r(BG, n) * 0 + 1, bs, ids, BG, n, rows, n, 3, rows)
+        a, lse = kernels.weighted_flash_decoding(of(q), keys, values, weight, return_softmax_lse=True)
+        b = kernels.weighted_flash_decoding(of(q), keys, values, previous_out=a.as_subclass(torch.Tensor),
+                                            previous_lse=lse.as_subclass(torch.Tensor), cache_seqlens=lengths)
+        results.append([x.as_subclass(torch.Tensor) for x in (product, softmax, norm, total, bk, bv, bs, a, lse, b)])
+    for x, y in zip(*results):
+        assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
+    with pytest.raises(ValueError):
+        kernels.batch_gemm_softmax(q, cent, product, norm[:1], total, softmax, BG, gs, n, 128)
