@@ -624,6 +624,7 @@ int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_s
    is rounded to half, or to fp32 and then to bfloat16: the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144 tokens, and 2 GiB of them together; beyond that
    ri_prefill_mean_workspace_bytes is 0 and the call refuses.
    ri_prefill_split_centred: ri_prefill_split with mean[h] taken off the rows of keys, as ri_prefill_center does.
+   ri_prefill_split_init: ri_prefill_split_centred, with what ri_kmeans_init gives for the rows of keys in centroids [H, nc, 128].
    ri_prefill_index: out = centroids + mean, mask = (count == 0), sizes as elements and as int32, first rows. */
 int ri_prefill_split(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
                      int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
@@ -637,6 +638,14 @@ int ri_prefill_split_centred_f16(const void* key, const void* value, int64_t key
                                  int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0,
                                  int n_start, int end0, int n_end, int H, const void* mean, void* keys, void* steady_k,
                                  void* steady_v, int64_t steady_stride, ri_stream_t stream);
+int ri_prefill_split_init(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                          int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
+                          int end0, int n_end, int H, const void* mean, void* keys, void* steady_k, void* steady_v,
+                          int64_t steady_stride, void* centroids, int nc, ri_stream_t stream);
+int ri_prefill_split_init_f16(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                              int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0,
+                              int n_start, int end0, int n_end, int H, const void* mean, void* keys, void* steady_k,
+                              void* steady_v, int64_t steady_stride, void* centroids, int nc, ri_stream_t stream);
 size_t ri_prefill_mean_workspace_bytes(int H, int N);
 int ri_prefill_mean(const void* key, int64_t key_row_stride, int64_t key_head_stride, int first, int N, int H, void* mean,
                     void* workspace, size_t workspace_bytes, ri_stream_t stream);

@@ -98,6 +98,8 @@ SIGNATURES = {
     "ri_prefill_split": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, I64, P]),
     "ri_prefill_split_centred": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, P, I64, P]),
     "ri_prefill_split_centred_f16": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, P, I64, P]),
+    "ri_prefill_split_init": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, P, I64, P, I, P]),
+    "ri_prefill_split_init_f16": (I, [P, P] + [I64] * 4 + [I] * 7 + [P, P, P, P, I64, P, I, P]),
     "ri_prefill_mean_workspace_bytes": (SZ, [I, I]),
     "ri_prefill_mean": (I, [P, I64, I64, I, I, I, P, P, SZ, P]),
     "ri_prefill_mean_f16": (I, [P, I64, I64, I, I, I, P, P, SZ, P]),

@@ -27,13 +27,16 @@ class KMeansResult:
     __slots__ = ("centroids", "value_sum", "assign", "counts", "offsets", "members")
 
 
-def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_means=True):
+def _cluster(key, num_centroids, num_iters, num_segments, init_indices, final_means=True, centroids=None):
     """Everything of the clustering that reads the keys: centroids, assignment, inverted lists.  final_means off: the
-    caller takes the last means over the lists, which it makes itself where kmeans_store_makes_lists says so."""
+    caller takes the last means over the lists, which it makes itself where kmeans_store_makes_lists says so.
+    centroids: the initial ones, which become the result's."""
     G, N, D = key.shape
     dev = key.device
     nc, S = num_centroids, num_segments
-    if init_indices is None:
+    if centroids is not None:
+        pass
+    elif init_indices is None:
         centroids = torch.empty((G, nc, D), dtype=key.dtype, device=dev)
         kernels.kmeans_init(key, centroids, G, N, nc)
     else:
@@ -78,14 +81,15 @@ _MAX_GRAPHS = 4
 
 def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1, init_indices=None,
                         reuse_graph=False, value_sum=None, value_store=None, store_stride=0, key_rows=None, key_mean=None,
-                        key_store=None, index=None):
+                        key_store=None, index=None, centroids=None):
     """Runs the clustering and returns a KMeansResult (no dense cluster lists, no host copy).
     key/value [G, N, 128] bfloat16 or float16 device tensors, keys contiguous.
 
     value_sum: [G, nc, 128] tensor for the sums (else a new one).  value_store: where the value rows are also
     written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
     key_rows, the [G, N, 128] keys before key_mean was subtracted.  index (with key_mean): the tensors that
-    kernels.prefill_index fills, filled here, with key_store in its launches.
+    kernels.prefill_index fills, filled here, with key_store in its launches.  centroids: [G, nc, 128] tensor with what
+    kernels.kmeans_init gives for the keys; the result's centroids are in it.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and of the same
     type, shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -106,13 +110,13 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     r = None
     if reuse_graph and not torch.cuda.is_current_stream_capturing():
         gkey = (key.data_ptr(), key.dtype, tuple(key.shape), str(key.device), nc, num_iters, S, key_store is None,
-                None if init_indices is None else init_indices.data_ptr())
+                None if init_indices is None else init_indices.data_ptr(), None if centroids is None else centroids.data_ptr())
         hit = _GRAPHS.get(gkey)
         if hit is None and gkey in _SEEN:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
-                res = _cluster(key, nc, num_iters, S, init_indices, key_store is None)
-            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph)
+                res = _cluster(key, nc, num_iters, S, init_indices, key_store is None, centroids)
+            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph, as the result's are)
             _GRAPHS[gkey] = hit
             while len(_GRAPHS) > _MAX_GRAPHS:
                 _GRAPHS.popitem(last=False)
@@ -127,7 +131,7 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
             while len(_SEEN) > 64:
                 _SEEN.popitem(last=False)
     if r is None:
-        r = _cluster(key, nc, num_iters, S, init_indices, key_store is None)
+        r = _cluster(key, nc, num_iters, S, init_indices, key_store is None, centroids)
     r.value_sum = torch.empty((G, nc, D), dtype=value.dtype, device=key.device) if value_sum is None else value_sum
     if key_store is not None:
         kernels.kmeans_store_rows(kernels.aligned_rows(value), key_rows, key_mean, r.counts, r.offsets, r.members,

@@ -158,7 +158,7 @@ class retroinfer_cache(KV_Cache):
         self._plans = {}                         # (layer, buffer) -> DecodeStepPlan of the device-resident step
         self._row_shape = (batch_size, 1, self.kv_head, self.head_dim)
         self._out_shape = (batch_size, 1, self.num_heads, self.head_dim)
-        self._centred_keys = {}                  # (device, tokens) -> buffer of centred keys for the clustering
+        self._centred_keys = {}                  # (device, tokens, clusters) -> the clustering's keys and centroids
         if self.kv_residency == "device":
             self._init_device_store()
         else:
@@ -362,16 +362,20 @@ class retroinfer_cache(KV_Cache):
 
         # the centred keys go to a buffer that keeps its address from call to call: the clustering of
         # every further layer and sequence of this length then replays one captured graph
-        ck = self._centred_keys.get((dkey, valid_length))
+        buffers = (dkey, valid_length, self.n_centroids)
+        ck, cc = self._centred_keys.get(buffers, (None, None))
         if ck is None:
             if len(self._centred_keys) >= 2:
                 self._centred_keys.clear()
-            ck = torch.empty((H, valid_length, head_dim), dtype=keys.dtype, device=keys.device)
-            self._centred_keys[(dkey, valid_length)] = ck
+            ck, cc = (torch.empty((H, n, head_dim), dtype=keys.dtype, device=keys.device)
+                      for n in (valid_length, self.n_centroids))
+            self._centred_keys[buffers] = ck, cc
         mean_key = kernels.prefill_mean(keys, lo, valid_length)
+        if mean_key is None:
+            cc = None
         kernels.prefill_split(keys, values, lo, valid_length, vs, sps, seq_len - spe, spe, ck,
                               self.steady_zone_keys[layer_idx][batch_idx], self.steady_zone_values[layer_idx][batch_idx],
-                              mean_key)
+                              mean_key, cc)
         if mean_key is None:
             mean_key = torch.mean(ck, dim=1, keepdim=True)
             kernels.prefill_center(ck, mean_key)
@@ -397,7 +401,7 @@ class retroinfer_cache(KV_Cache):
         km = segment_k_means_csr(ck, head_values, self.n_centroids, num_segments=self.n_segment,
                                  reuse_graph=True,   # results are consumed below, before the next call
                                  value_sum=self.value_sum[layer_idx][rows], value_store=store_v, store_stride=stride,
-                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k, index=index)
+                                 key_rows=head_keys, key_mean=mean_key, key_store=store_k, index=index, centroids=cc)
         self.store_rows[layer_idx][rows] = [valid_length] * H
         if dev_organise:
             self.mainevents[dkey].record()

@@ -2160,8 +2160,7 @@ __global__ __launch_bounds__(256) void km_init_kernel(const uint4* __restrict__ 
                                                       int nc, float ratio, float half) {
   const int c = blockIdx.x * 16 + (threadIdx.x >> 4), piece = threadIdx.x & 15;
   if (c >= nc) return;
-  const float x = (float)c * ratio;   // (two roundings: built without fp contraction)
-  const int row = min((int)(x + half), N - 1);
+  const int row = ri_kmeans_first_row(c, ratio, half, N);
   cent[((size_t)blockIdx.y * nc + c) * 16 + piece] = data[((size_t)blockIdx.y * N + row) * 16 + piece];
 }
 

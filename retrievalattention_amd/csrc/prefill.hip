@@ -179,7 +179,9 @@ extern "C" int ri_prefill_mean_f16(const void* key, int64_t key_row_stride, int6
 // and V.  16 lanes per row, a workgroup moves 16 rows of one head: occupancy keeps more loads in flight than several rows
 // per thread do (8 heads of 8K / 128K tokens: 6.7 / 93 us; two or four rows per thread 19 / 105).  Heads vary fastest over
 // the workgroups, so those in flight together read whole tokens.  Workgroups behind the clustered range move the steady
-// rows.
+// rows, and those behind them the rows that a clustering starts from, which is a launch less in front of it (prefills, us, with a
+// launch of their own / as it is: 4 heads x 50021 tokens in half 581.3 / 579.1, 8 x 131072 3192.0 / 3185.5; short ones 153.2 / 151.5, 241.4 /
+// 239.1).
 // ------------------------------------------------------------------------------------
 struct SplitParams {
   const uint4* k;
@@ -191,6 +193,9 @@ struct SplitParams {
   int64_t k_row, k_head, v_row, v_head;   // pieces between tokens and between heads
   int64_t zone_stride;                    // rows between heads
   int first, N, start0, end0, n_start, n_end, H, blocks;   // blocks: of 16 clustered rows
+  uint4* cent;      // [H, nc, 16] initial centroids (nc 0: none)
+  int nc;
+  float ratio, half;   // as ri_kmeans_first_row takes them
 };
 
 template <bool HALF>
@@ -209,6 +214,15 @@ __global__ __launch_bounds__(256) void split_kernel(SplitParams P) {
     P.keys[((int64_t)h * P.N + i) * 16 + piece] = CENTRE ? sub8<HALF>(x, P.mean[h * 16 + piece]) : x;
     return;
   }
+  const int steady = (P.n_start + P.n_end + 15) / 16;
+  if (blk >= P.blocks + steady) {
+    const int c = (blk - P.blocks - steady) * 16 + sub;
+    if (c >= P.nc) return;
+    const int64_t i = ri_kmeans_first_row(c, P.ratio, P.half, P.N);
+    const uint4 x = P.k[h * P.k_head + (P.first + i) * P.k_row + piece];
+    P.cent[((int64_t)h * P.nc + c) * 16 + piece] = CENTRE ? sub8<HALF>(x, P.mean[h * 16 + piece]) : x;
+    return;
+  }
   const int i = (blk - P.blocks) * 16 + sub;
   if (i >= P.n_start + P.n_end) return;
   const int64_t tok = i < P.n_start ? P.start0 + i : P.end0 + (i - P.n_start);
@@ -222,19 +236,22 @@ template <bool CENTRE, bool HALF>
 static int prefill_split(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
                          int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0, int n_start,
                          int end0, int n_end, int H, const void* mean, void* keys, void* steady_k, void* steady_v,
-                         int64_t steady_stride, ri_stream_t stream) {
+                         int64_t steady_stride, void* cent, int nc, ri_stream_t stream) {
   if (!key || !value || !keys || !steady_k || !steady_v || (CENTRE && !mean)) return RI_ERR_ARG;
-  if (ri_any_misaligned16(key, value, mean, keys, steady_k, steady_v)) return RI_ERR_ARG;
+  if (ri_any_misaligned16(key, value, mean, keys, steady_k, steady_v) || ri_any_misaligned16(cent)) return RI_ERR_ARG;
+  if (nc < 0 || (nc > 0 && !cent)) return RI_ERR_ARG;
   if (N <= 0 || H <= 0 || first < 0 || start0 < 0 || end0 < 0 || n_start < 0 || n_end < 0 ||
       steady_stride < n_start + n_end || key_row_stride < 0 || key_head_stride < 0 || value_row_stride < 0 ||
       value_head_stride < 0 || (key_row_stride | key_head_stride | value_row_stride | value_head_stride) % 8 != 0)
     return RI_ERR_ARG;
   const int blocks = N / 16 + (N % 16 != 0);
-  const int64_t wgs = ((int64_t)blocks + ((int64_t)n_start + n_end + 15) / 16) * H;
+  const int64_t wgs = ((int64_t)blocks + ((int64_t)n_start + n_end + 15) / 16 + ((int64_t)nc + 15) / 16) * H;
+  const double ratio = nc > 0 ? (double)N / nc : 0;
   if (wgs > 0x7fffffffLL) return RI_ERR_ARG;
   const SplitParams P = {(const uint4*)key, (const uint4*)value, (const uint4*)mean, (uint4*)keys, (uint4*)steady_k,
                          (uint4*)steady_v, key_row_stride / 8, key_head_stride / 8, value_row_stride / 8,
-                         value_head_stride / 8, steady_stride, first, N, start0, end0, n_start, n_end, H, blocks};
+                         value_head_stride / 8, steady_stride, first, N, start0, end0, n_start, n_end, H, blocks,
+                         (uint4*)cent, nc, (float)ratio, (float)(ratio / 2)};
   split_kernel<CENTRE, HALF><<<dim3((unsigned)wgs), 256, 0, (hipStream_t)stream>>>(P);
   RI_HIP_CHECK_LAUNCH();
   return RI_OK;
@@ -246,7 +263,7 @@ extern "C" int ri_prefill_split(const void* key, const void* value, int64_t key_
                                 int64_t steady_stride, ri_stream_t stream) {
   return prefill_split<false, false>(key, value, key_row_stride, key_head_stride, value_row_stride, value_head_stride, first,
                                      N, start0, n_start, end0, n_end, H, nullptr, keys, steady_k, steady_v, steady_stride,
-                                     stream);
+                                     nullptr, 0, stream);
 }
 
 extern "C" int ri_prefill_split_centred(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
@@ -255,7 +272,7 @@ extern "C" int ri_prefill_split_centred(const void* key, const void* value, int6
                                         void* steady_k, void* steady_v, int64_t steady_stride, ri_stream_t stream) {
   return prefill_split<true, false>(key, value, key_row_stride, key_head_stride, value_row_stride, value_head_stride, first,
                                     N, start0, n_start, end0, n_end, H, mean, keys, steady_k, steady_v, steady_stride,
-                                    stream);
+                                    nullptr, 0, stream);
 }
 
 extern "C" int ri_prefill_split_centred_f16(const void* key, const void* value, int64_t key_row_stride,
@@ -264,7 +281,27 @@ extern "C" int ri_prefill_split_centred_f16(const void* key, const void* value, 
                                             const void* mean, void* keys, void* steady_k, void* steady_v,
                                             int64_t steady_stride, ri_stream_t stream) {
   return prefill_split<true, true>(key, value, key_row_stride, key_head_stride, value_row_stride, value_head_stride, first, N,
-                                   start0, n_start, end0, n_end, H, mean, keys, steady_k, steady_v, steady_stride, stream);
+                                   start0, n_start, end0, n_end, H, mean, keys, steady_k, steady_v, steady_stride, nullptr, 0,
+                                   stream);
+}
+
+extern "C" int ri_prefill_split_init(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                                     int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0,
+                                     int n_start, int end0, int n_end, int H, const void* mean, void* keys, void* steady_k,
+                                     void* steady_v, int64_t steady_stride, void* centroids, int nc, ri_stream_t stream) {
+  return prefill_split<true, false>(key, value, key_row_stride, key_head_stride, value_row_stride, value_head_stride, first,
+                                    N, start0, n_start, end0, n_end, H, mean, keys, steady_k, steady_v, steady_stride,
+                                    centroids, nc, stream);
+}
+
+extern "C" int ri_prefill_split_init_f16(const void* key, const void* value, int64_t key_row_stride, int64_t key_head_stride,
+                                         int64_t value_row_stride, int64_t value_head_stride, int first, int N, int start0,
+                                         int n_start, int end0, int n_end, int H, const void* mean, void* keys,
+                                         void* steady_k, void* steady_v, int64_t steady_stride, void* centroids, int nc,
+                                         ri_stream_t stream) {
+  return prefill_split<true, true>(key, value, key_row_stride, key_head_stride, value_row_stride, value_head_stride, first, N,
+                                   start0, n_start, end0, n_end, H, mean, keys, steady_k, steady_v, steady_stride, centroids,
+                                   nc, stream);
 }
 
 // ------------------------------------------------------------------------------------

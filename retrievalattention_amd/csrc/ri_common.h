@@ -93,6 +93,12 @@ __device__ __forceinline__ void ri_add2(uint32_t w, float& s0, float& s1) {
   if (HALF) asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s1) : "v"(w));
   else s1 += __uint_as_float(w & 0xffff0000u);
 }
+// the row that centroid c of a clustering of N rows starts from: trunc(c * ratio + half) in fp32, ratio and half of N / nc
+// (two roundings: built without fp contraction)
+__device__ __forceinline__ int ri_kmeans_first_row(int c, float ratio, float half, int N) {
+  const float x = (float)c * ratio;
+  return min((int)(x + half), N - 1);
+}
 // a - b on packed pairs: both operands widened, the differences rounded
 template <bool HALF>
 __device__ __forceinline__ uint32_t ri_sub2(uint32_t a, uint32_t b) {

@@ -765,8 +765,9 @@ def prefill_mean(keys, first, N):
     return mean
 
 
-def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, steady_k, steady_v, mean=None):
-    """keys/values [T, H, 128]; out [H, N, 128], less mean [H, 1, 128] where given; steady_k/v [H, rows, 128]."""
+def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, steady_k, steady_v, mean=None, centroids=None):
+    """keys/values [T, H, 128]; out [H, N, 128], less mean [H, 1, 128] where given; steady_k/v [H, rows, 128].  centroids (with
+    mean): [H, nc, 128], which kmeans_init of out would fill."""
     kr, kh = _row_strides(keys, "prefill_split")
     vr, vh = _row_strides(values, "prefill_split")
     T, H = keys.shape[0], keys.shape[1]
@@ -778,6 +779,10 @@ def prefill_split(keys, values, first, N, start0, n_start, end0, n_end, out, ste
     tail = (_p(out), _p(steady_k), _p(steady_v), steady_k.stride(0) // 128, _stream())
     if mean is None:
         check(lib().ri_prefill_split(*lead, *tail), "prefill_split")
+    elif centroids is not None:
+        _need(centroids, keys.dtype, "centroids")
+        check(_fn("ri_prefill_split_init", keys.dtype)(*lead, _p(mean), *tail[:-1], _p(centroids), centroids.shape[1], tail[-1]),
+              "prefill_split")
     else:
         check(_fn("ri_prefill_split_centred", keys.dtype)(*lead, _p(mean), *tail), "prefill_split")
 

@@ -191,6 +191,26 @@ def test_prefill_mean(dev, dtype, H, N):
     assert torch.equal(ck, ref) and torch.equal(zones[0], zones[2]) and torch.equal(zones[1], zones[3])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,nc", [(1, 32, 32), (3, 100, 32), (2, 1000, 41), (8, 4099, 256), (1, 7, 33), (4, 50021, 3072)])
+def test_initial_centroids_come_with_the_split(dev, dtype, H, N, nc):
+    """What the split writes for the centroids are the rows that kmeans_init takes of the centred keys, and everything else is as
+    without them: whole and partial workgroups of centroids, more centroids than rows."""
+    from retrievalattention_amd import kernels
+    g = torch.Generator(device=dev).manual_seed(N)
+    vs, sps, spe = 3, 4, 20
+    K, V = torch.randn(2, vs + sps + N + spe, H, 128, generator=g, device=dev).to(dtype)
+    lo, mean = vs + sps, torch.randn(H, 1, 128, generator=g, device=dev).to(dtype)
+    keys = [torch.empty((H, N, 128), dtype=dtype, device=dev) for _ in range(2)]
+    zones = [torch.zeros((H, sps + spe, 128), dtype=dtype, device=dev) for _ in range(4)]
+    cent = [torch.zeros((H, nc + 1, 128), dtype=dtype, device=dev)[:, :nc].contiguous() for _ in range(2)]
+    kernels.prefill_split(K, V, lo, N, vs, sps, lo + N, spe, keys[0], *zones[:2], mean)
+    kernels.kmeans_init(keys[0], cent[0], H, N, nc)
+    kernels.prefill_split(K, V, lo, N, vs, sps, lo + N, spe, keys[1], *zones[2:], mean, cent[1])
+    assert torch.equal(keys[0], keys[1]) and torch.equal(zones[0], zones[2]) and torch.equal(zones[1], zones[3])
+    assert torch.equal(cent[0], cent[1])
+
+
 def test_prefill_mean_leaves_other_shapes(dev):
     from retrievalattention_amd import kernels
     assert kernels.prefill_mean(torch.empty((40, 33, 128), dtype=torch.bfloat16, device=dev), 0, 40) is None
