@@ -53,6 +53,7 @@ struct SelectArgs {
 // Barrier over LDS traffic only: global stores issued before it stay in flight (__syncthreads waits for them as well).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+
 // lanes whose bit K and bit D are equal: those that keep the larger value of an exchange over 2^D in a merge of 2^K
 constexpr uint64_t keep_mask(int K, int D) {
   uint64_t m = 0;
@@ -151,9 +152,10 @@ __device__ __forceinline__ uint32_t sel_above(uint32_t a, uint32_t b) {
 
 // GSM: query heads padded to 4, 8 or 16 (SEL_LOGITS, SEL_SCORE).  KEEP: the results are left in K in place of
 // memory (a load's wait covers the stores in front of it: the caller stores behind the attention).
-// ahead(): what the caller wants on its way behind the selection's first loads.
+// ahead(): what the caller wants on its way behind the selection's first loads.  Returns the cluster of the thread's rank, -1
+// past the list.
 template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP, typename Ahead>
-__device__ __forceinline__ void select_group(const SelectArgs& P, const int g, const SelectKept& K, Ahead&& ahead) {
+__device__ __forceinline__ int select_group(const SelectArgs& P, const int g, const SelectKept& K, Ahead&& ahead) {
   static_assert(KEEP == KEEP_NONE || SRC != SEL_SCORE || GSM <= 8, "the logits are in LDS");
   constexpr bool STORE = !KEEP;
   constexpr int NW = NT / 64, IDS = NT * E;
@@ -744,7 +746,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
       if (P.cI) P.cI[(size_t)g * k2 + np + at] = c;
     }
   }
-  if (!P.cluster_size) return;
+  if (!P.cluster_size) return in ? my_c : -1;
   if (in) {
     if (STORE) P.ret_tok_off[(size_t)g * (np + 1) + tid] = (int32_t)((tid < nkeep) ? tok : T_ret);
     if (STORE && P.ret_start) P.ret_start[(size_t)g * np + tid] = st;
@@ -767,6 +769,7 @@ __device__ __forceinline__ void select_group(const SelectArgs& P, const int g, c
     const int room = P.row_src_stride - (int)tok;
     for (int k = 0; k < (int)sz && k < room; ++k) dst[k] = st + k;
   }
+  return in ? my_c : -1;
 }
 
 // Checks the arguments of ri_score_select and lays them down (select.hip).
@@ -778,3 +781,7 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
 
 // Scoring, and the scores' sums and keys if `keys` (select.hip)
 int ri_launch_select_inputs(const SelectArgs& P, int BG, bool half, bool keys, hipStream_t s);
+
+// Scoring, selection and the block cache's look-up of the selected clusters (host_step.hip); `taken`: false, and nothing launched,
+// where that is not worth a launch of its own kind.
+int ri_launch_select_access(const SelectArgs& P, const ri_lru_t& lru, int BG, bool half, bool* taken, hipStream_t s);

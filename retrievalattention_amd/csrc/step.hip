@@ -5,6 +5,7 @@
 // wrapper call per stage a layer-step took 46 us of host time, of which the launches are 1 us each.  The addresses and
 // sizes of a layer do not change from token to token, so the caller keeps them in one struct and hands over its address.
 #include "attend_common.h"
+#include "lru_body.h"
 #include "select_body.h"
 #include "step_route.h"
 
@@ -277,11 +278,21 @@ extern "C" int ri_host_step(const ri_decode_step_t* s, const ri_lru_t* lru, cons
   if (!s || !lru) return RI_ERR_ARG;
   auto* select = s->half ? ri_score_select_f16 : ri_score_select;
   auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
-  int rc = select(q, s->centroids, s->mask, nullptr, nullptr, s->logits, nullptr, nullptr, s->ret_ids, s->est_ids, nullptr,
-                  nullptr, nullptr, 0, nullptr, s->BG, s->gs, s->nc, s->np, s->es, s->page, s->max_pages, s->scale,
-                  s->score_workspace, s->score_workspace_bytes, stream);
+  SelectArgs S;
+  int rc = ri_prepare_select(&S, q, s->centroids, s->mask, nullptr, nullptr, s->logits, nullptr, nullptr, s->ret_ids,
+                             s->est_ids, nullptr, nullptr, nullptr, 0, nullptr, s->BG, s->gs, s->nc, s->np, s->es, s->page,
+                             s->max_pages, s->scale, s->score_workspace, s->score_workspace_bytes);
   if (rc) return rc;
-  if ((rc = ri_lru_access(lru, stream))) return rc;
+  bool taken = false;
+  if (ri_lru_check(*lru) == RI_OK) rc = ri_launch_select_access(S, *lru, s->BG, s->half, &taken, (hipStream_t)stream);
+  if (rc) return rc;
+  if (!taken) {
+    rc = select(q, s->centroids, s->mask, nullptr, nullptr, s->logits, nullptr, nullptr, s->ret_ids, s->est_ids, nullptr,
+                nullptr, nullptr, 0, nullptr, s->BG, s->gs, s->nc, s->np, s->es, s->page, s->max_pages, s->scale,
+                s->score_workspace, s->score_workspace_bytes, stream);
+    if (rc) return rc;
+    if ((rc = ri_lru_access(lru, stream))) return rc;
+  }
   if ((rc = ri_lru_stage_update(lru, stream))) return rc;
   rc = attend(q, s->steady_k, s->steady_v, s->steady_stride, static_len, s->static_len_dev, s->store_k, s->store_v,
               s->store_stride, lru->row_src, lru->row_src_stride, nullptr, nullptr, 0, s->meta, s->est_ids,

@@ -249,3 +249,64 @@ def test_missed_rows_are_staged_in_rank_order(dev, BG, block, most=39):
 def test_short_blocks_are_staged_in_rank_order(dev, BG, block, most):
     """Blocks of few rows, which more waves than one of a workgroup copy: from eight down to two of them."""
     test_missed_rows_are_staged_in_rank_order(dev, BG, block, most)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BG,gs,nc,nprobe,es,buffer_blocks", [
+    # selection and look-up in one launch: every number of threads and of clusters to a thread, heads padded and not, no
+    # estimation zone, a probe list as long as the threads take, a buffer that cuts the list
+    (1, 1, 8, 3, 2, 100), (3, 8, 256, 255, 0, 2000), (2, 12, 256, 9, 100, 12), (2, 4, 264, 20, 60, 200), (5, 7, 512, 511, 1, 4000),
+    (2, 3, 520, 511, 9, 4000), (3, 16, 1024, 18, 237, 100), (2, 8, 1032, 30, 300, 40), (1, 9, 2048, 40, 500, 300),
+    (1, 4, 2048, 1023, 500, 8000), (2, 7, 2056, 600, 300, 5000), (2, 8, 4096, 74, 950, 400), (70, 4, 64, 5, 10, 30),
+    # past it
+    (2, 8, 256, 256, 0, 2000), (1, 4, 512, 512, 0, 4000), (2, 9, 2056, 40, 300, 300), (1, 4, 4104, 74, 950, 400),
+    (1, 2, 2048, 1024, 300, 8000), (1, 8, 8200, 20, 300, 200)])
+def test_host_step_equals_the_operators(dev, dtype, BG, gs, nc, nprobe, es, buffer_blocks):
+    """The prepared step against selection and look-up called by themselves: the same ids, lists, row table and books, and the
+    output of an attention over the step's own row table."""
+    from retrievalattention_amd import kernels
+    block, steps = 8, 4
+    g = torch.Generator().manual_seed(BG * nc + nprobe)
+    rn = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    sz = torch.randint(0, 21, (BG, nc), generator=g, dtype=torch.int32)
+    st = (torch.cumsum(sz.long(), 1) - sz.long()).to(torch.int32)
+    n, max_blocks = int(sz.sum(1).max()) + 1, int(((sz + 7) // 8).sum(1).max()) + 1
+    mask, size16 = (sz == 0).to(dev), sz.to(dtype).to(dev)
+    sz, st = sz.to(dev), st.to(dev)
+    capacity, stage0 = max_blocks, max_blocks * block
+    cent, vs, sk, sv = rn(BG, nc, 128).to(dev), rn(BG, nc, 128).to(dev), rn(BG, 70, 128).to(dev), rn(BG, 70, 128).to(dev)
+    host = [rn(BG, n, 128).pin_memory() for _ in range(2)]
+    scale = 128 ** -0.5
+    i32 = lambda *s: torch.full(s, -5, dtype=torch.int32, device=dev)
+    sides = []
+    for _ in range(2):
+        lru = kernels.DeviceLru(BG, nc, max_blocks, capacity, buffer_blocks, block, dev)
+        lru.set_sizes(sz)
+        lists = [torch.zeros((BG,) if i % 4 == 3 else (BG, buffer_blocks), dtype=torch.int32, device=dev) for i in range(12)]
+        sides.append(dict(lru=lru, lists=lists, row_src=i32(BG, buffer_blocks * block), meta=i32(BG, 4), ret=i32(BG, nprobe),
+                          est=i32(BG, max(es, 1)), logits=torch.zeros(BG, gs, nc, device=dev), valid=i32(BG)))
+    a, b = sides
+    cache = [torch.zeros(BG, stage0 + buffer_blocks * block, 128, dtype=dtype, device=dev) for _ in range(2)]
+    est = lambda d: d["est"] if es else None
+    plan = kernels.HostStepPlan(None, dtype, dict(
+        centroids=cent, mask=mask, logits=b["logits"], ret_ids=b["ret"], est_ids=est(b), meta=b["meta"], steady_k=sk, steady_v=sv,
+        store_k=cache[0], store_v=cache[1], value_sum=vs, cluster_size=size16, valid_lengths=b["valid"]), nprobe, es, 8,
+        buffer_blocks, scale, b["lru"], sz, st, b["lists"], b["row_src"], *host, stage0)
+    q0 = rn(BG, gs, 128).to(dev)
+    for step in range(steps):
+        q = q0 + 0.3 * step * rn(BG, gs, 128).to(dev)
+        kernels.score_select(q, cent, mask, None, None, a["logits"], None, None, a["ret"], est(a), None, None, None, nprobe, es, 8,
+                             buffer_blocks, scale)
+        a["lru"].access_update(a["ret"], sz, st, a["lists"], row_src=a["row_src"], stage_row0=stage0, meta=a["meta"])
+        got, want = (torch.empty(BG, gs, 128, dtype=dtype, device=dev) for _ in range(2))
+        plan.run(q, 70, got)
+        for name in ("ret", "est", "logits", "row_src", "meta"):
+            if es or name != "est":
+                assert torch.equal(a[name], b[name]), (step, name)
+        for x, y in zip(a["lists"], b["lists"]):
+            assert torch.equal(x, y), step
+        for name in ("stamp", "blk_ids", "free_list", "free_count", "epoch"):
+            assert torch.equal(getattr(a["lru"], name), getattr(b["lru"], name)), (step, name)
+        kernels.wave_attention(q, sk, sv, 70, *cache, b["row_src"], b["meta"], est(b), b["logits"] if es else None, vs, size16, want,
+                               b["valid"], es, scale)
+        assert torch.equal(got, want), step
