@@ -1362,6 +1362,80 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
   }
 }
 
+// The same sum without copies: sixty-four rows in flight at any time, each register
+// requested again as soon as its row is added, ids a round ahead, rows by buffer offsets (bytes within 31 bits: km_reduce).  A
+// round that is requested, waited for and added 32 rows at a time leaves a wave waiting for most of a block, and costs more than
+// the waves that its fewer registers make room for.  Updates over given lists, us, rounds / ahead, an early and a late iteration: 1 x 22198
+// tokens, 800 clusters 15.1, 9.8 / 9.8, 7.7; 2 x 20124, 448 16.1, 13.6 / 10.9, 9.6; 2 x 44152, 1536 20.0, 15.4 / 15.0, 10.4; 4 x 65536, 2048 25.0, 24.3
+// / 21.8, 19.4; 8 x 131072, 8192 59.0, 63.2 / 55.4, 60.3 (4.9 TB/s).
+template <bool HALF>
+__device__ __forceinline__ void km_sum_rows_ahead(__amdgpu_buffer_rsrc_t rows, uint32_t row_bytes, const int32_t* mem, int k0, int k1,
+                                                  float& s0, float& s1) {
+  constexpr int U = 64;
+  const int lane = threadIdx.x & 63;
+  const uint32_t byte = (uint32_t)lane * 4u;
+  uint32_t v[U];
+  int off, so[8];
+  const auto offsets = [&](int e) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) so[j] = __builtin_amdgcn_readlane(off, e + j);
+  };
+  const auto request = [&](int e) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[e + j] = __builtin_amdgcn_raw_buffer_load_b32(rows, byte, so[j], 0);
+  };
+  const auto add8 = [&](int e) {
+#pragma unroll
+    for (int j = e; j < e + 8; ++j) ri_add2<HALF>(v[j], s0, s1);
+  };
+  const auto rest = [&](int k) {
+#pragma unroll
+    for (int e = 0; e < U; e += 8) {
+      if (k + e + 8 <= k1) {
+        add8(e);
+      } else if (k + e < k1) {
+#pragma unroll
+        for (int j = e; j < e + 8; ++j) ri_add2<HALF>(k + j < k1 ? v[j] : 0u, s0, s1);   // the word 0 is (+0, +0) in either type
+      }
+    }
+  };
+  int k = k0;
+  off = (int)((uint32_t)mem[min(k + lane, k1 - 1)] * row_bytes);
+  if (k + U < k1) {
+    int next = mem[min(k + U + lane, k1 - 1)];
+#pragma unroll
+    for (int e = 0; e < U; e += 8) {
+      offsets(e);
+      __builtin_amdgcn_sched_barrier(0);
+      request(e);
+    }
+    do {   // (as in km_sum_listed: no branch around a load)
+      k += U;
+      off = (int)((uint32_t)next * row_bytes);
+      next = mem[min(k + U + lane, k1 - 1)];
+#pragma unroll
+      for (int e = 0; e < U; e += 8) {
+        offsets(e);
+        __builtin_amdgcn_sched_barrier(0);
+        add8(e);
+        __builtin_amdgcn_sched_barrier(0);
+        request(e);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } while (k + U < k1);
+    rest(k);
+  } else {
+#pragma unroll
+    for (int e = 0; e < U; e += 8)
+      if (k + e < k1) {
+        offsets(e);
+        __builtin_amdgcn_sched_barrier(0);
+        request(e);
+      }
+    rest(k);
+  }
+}
+
 // odd (where it is asked for): set if the squares underflow or are no numbers, so that the result's norm need not be one
 template <bool MEAN, bool HALF>
 __device__ __forceinline__ uint32_t km_finish(float s0, float s1, int count, int normalize, uint32_t* op,
@@ -1501,7 +1575,8 @@ __device__ __forceinline__ void km_entry(const KmIndex& X, size_t at, int size, 
 // cluster per wave.
 // COPY (sums of value rows): every row is also written where its list puts it, row off + k of problem p to
 // copy + (p * copy_stride + off + k) * 128: the cluster-contiguous store, without a second pass over the rows.
-template <bool MEAN, bool HALF, bool COPY, bool CENTER>
+// AHEAD (without copies): sums by km_sum_rows_ahead.
+template <bool MEAN, bool HALF, bool COPY, bool CENTER, bool AHEAD = false>
 __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows, size_t pitch,
                                                const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
                                                const int32_t* __restrict__ members, uint16_t* __restrict__ out,
@@ -1518,6 +1593,17 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
                        (size_t)(p % seg) * N * pitch;
   uint32_t* wp = COPY ? reinterpret_cast<uint32_t*>(copy) + (size_t)p * copy_stride * (RI_DIM / 2) + lane : nullptr;
   const uint32_t mw = CENTER ? reinterpret_cast<const uint32_t*>(mean)[p * (RI_DIM / 2) + lane] : 0u;
+  static_assert(!AHEAD || (!COPY && !CENTER), "sums alone");
+  const auto sum = [&](int o, int k0, int k1, float& s0, float& s1) {
+    const int32_t* const list = members + (size_t)p * N + o;
+    if constexpr (AHEAD) {
+      const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(rp), 0,
+                                                                           (int)(((N - 1) * pitch + RI_DIM / 2) * 4), 0x00020000);
+      km_sum_rows_ahead<HALF>(all, (uint32_t)pitch * 4u, list, k0, k1, s0, s1);
+    } else {
+      km_sum_rows<HALF, COPY ? 16 : 32, COPY, CENTER>(rp, list, k0, k1, s0, s1, pitch, COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
+    }
+  };
   if ((int)blockIdx.x < item_wgs) {
     const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (slot >= cap) return;
@@ -1525,8 +1611,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
     const int c = km_slot_owner(off, nc, slot, s, o, j);
     if (c < 0 || (M.state && !M.first && !M.touched[(size_t)p * nc + c])) return;
     float s0 = 0.f, s1 = 0.f;
-    km_sum_rows<HALF, COPY ? 16 : 32, COPY, CENTER>(rp, members + (size_t)p * N + o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1,
-                                        pitch, COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
+    sum(o, j * KM_BLK, min(s, (j + 1) * KM_BLK), s0, s1);
     partial[((size_t)p * cap + slot) * 64 + lane] = make_float2(s0, s1);
     return;
   }
@@ -1548,13 +1633,12 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
   }
   if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
-  km_sum_rows<HALF, COPY ? 16 : 32, COPY, CENTER>(rp, members + (size_t)p * N + o, 0, s, s0, s1, pitch,
-                                      COPY ? wp + (size_t)o * (RI_DIM / 2) : nullptr, mw);
+  sum(o, 0, s, s0, s1);
   const uint32_t word = km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);
   if (CENTER && X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, word, mw);
 }
 
-template <bool MEAN, bool HALF, bool COPY>
+template <bool MEAN, bool HALF, bool COPY, bool AHEAD>
 __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restrict__ rows, size_t pitch,
                                                         const int32_t* __restrict__ counts,
                                                         const int32_t* __restrict__ offsets,
@@ -1563,7 +1647,7 @@ __global__ __launch_bounds__(256) void km_reduce_kernel(const uint16_t* __restri
                                                         int item_wgs, int cap, int N, int nc, int seg,
                                                         int64_t head_stride, int normalize,
                                                         uint16_t* __restrict__ copy, int64_t copy_stride, KmMoves M) {
-  km_reduce_rows<MEAN, HALF, COPY, false>(rows, pitch, counts, offsets, members, out, partial, item_wgs, cap, N, nc, seg,
+  km_reduce_rows<MEAN, HALF, COPY, false, AHEAD>(rows, pitch, counts, offsets, members, out, partial, item_wgs, cap, N, nc, seg,
                                           head_stride, normalize, copy, copy_stride, nullptr, M);
 }
 
@@ -2354,7 +2438,9 @@ static int km_reduce(const void* rows, int64_t head_stride, int64_t row_stride, 
   float2* partial = (float2*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   const int item_wgs = (cap + 3) / 4;
   if ((long long)item_wgs + (nc + 3) / 4 > 0x7fffffffLL) return RI_ERR_ARG;
-  km_reduce_kernel<MEAN, HALF, COPY><<<dim3(item_wgs + (nc + 3) / 4, P), 256, 0, s>>>(
+  const bool ahead = !COPY && (int64_t)N * row_stride * 2 <= 0x7fffffffLL;   // (rows by offsets of 31 bits; others by address)
+  auto* kernel = ahead ? km_reduce_kernel<MEAN, HALF, COPY, !COPY> : km_reduce_kernel<MEAN, HALF, COPY, false>;
+  kernel<<<dim3(item_wgs + (nc + 3) / 4, P), 256, 0, s>>>(
       (const uint16_t*)rows, (size_t)row_stride / 2, counts, offsets, members, (uint16_t*)out, partial, item_wgs, cap, N,
       nc, seg, head_stride / 2, normalize, (uint16_t*)copy, copy_stride, M);
   RI_HIP_CHECK_LAUNCH();

@@ -519,3 +519,31 @@ def test_iterate_hands_assignments_over(dev, G, N, nc, seg, kind):
                                     (2, 131073, 8192), (5, 16385, 33), (2, 20000, 32), (3, 17409, 544), (1, 33793, 16384), (2, 32768, 16384)])
 def test_build_lists_on_both_sides_of_the_table(dev, P, N, nc):
     test_build_lists_is_a_stable_sort(dev, P, N, nc, N % 97)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("wide", [False, True])
+def test_sums_of_lists_of_every_length(dev, dt, wide):
+    """Lists whose lengths lie around the eights, the rounds of 64 rows and the blocks of 256 of a wave's sum, in rows that are
+    next to each other and in rows too far apart for offsets of 31 bits: the sums that the oracle defines."""
+    from retrievalattention_amd import kernels
+    lengths = [0, 1, 2, 7, 8, 9, 15, 31, 56, 57, 63, 64, 65, 71, 72, 127, 128, 129, 136, 191, 192, 193, 200, 255, 256, 257, 264, 319,
+               320, 321, 511, 512, 513, 576, 777, 1024, 1100, 3000, 5000, 6, 64, 16]
+    nc = len(lengths) + (-len(lengths)) % 32
+    g = torch.Generator().manual_seed(7)
+    a = torch.cat([torch.full((n,), c) for c, n in enumerate(lengths)])[torch.randperm(sum(lengths), generator=g)].int()
+    N = a.numel()
+    rows = torch.randn(N, 128, generator=g).to(dt)
+    counts, offsets, members = (torch.empty(1, n, dtype=torch.int32, device=dev) for n in (nc, nc + 1, N))
+    kernels.kmeans_build_lists(a[None].to(dev), counts, offsets, members, 1, N, nc)
+    assert counts[0, :len(lengths)].tolist() == lengths
+    if wide:
+        pitch = (1 << 30) // N // 8 * 8 + 128   # elements: N rows of it are past 2 GiB
+        values = torch.zeros(N * pitch, dtype=dt, device=dev).view(N, pitch)[:, :128]
+        values.copy_(rows)
+    else:
+        values = rows.to(dev)
+    sums = torch.empty(1, nc, 128, dtype=dt, device=dev)
+    kernels.kmeans_value_sum(values[None], counts, offsets, members, sums, 1, N, nc)
+    s, _ = okm.cluster_sums(rows, a.numpy().astype(np.int64), nc)
+    assert torch.equal(sums[0].cpu(), torch.from_numpy(s).to(dt))
