@@ -547,3 +547,11 @@ def test_sums_of_lists_of_every_length(dev, dt, wide):
     kernels.kmeans_value_sum(values[None], counts, offsets, members, sums, 1, N, nc)
     s, _ = okm.cluster_sums(rows, a.numpy().astype(np.int64), nc)
     assert torch.equal(sums[0].cpu(), torch.from_numpy(s).to(dt))
+
+
+@pytest.mark.parametrize("G,N,nc,seg", [(3, 40001, 96, 1), (1, 65600, 640, 1), (5, 17001, 32, 1), (2, 50003, 1024, 3), (1, 16640, 32, 1)])
+@pytest.mark.parametrize("kind", ["mixture", "ties", "odd"])
+def test_iterate_folds_long_lists_where_they_are_summed(dev, G, N, nc, seg, kind):
+    """Longer problems whose passes know nothing of each other: lists of two blocks, of hundreds, and one of all tokens."""
+    nc = nc if seg == 1 else nc // 32 // seg * 32 * seg
+    test_iterate_equals_its_passes(dev, G, N, nc, seg, kind, torch.bfloat16)
