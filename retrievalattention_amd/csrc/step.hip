@@ -258,8 +258,10 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
 
 extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int static_len, void* out, ri_stream_t stream) {
   if (!s) return RI_ERR_ARG;
-  if (step_is_joined(s))
-    return step_joined(s, q, static_len, step_is_short(s, static_len) && step_is_alone(s, static_len), out, (hipStream_t)stream);
+  if (step_is_joined(s)) {
+    const bool one = step_is_short(s, static_len) && s->BG > 128;   // (figures at step_is_alone)
+    return step_joined(s, q, static_len, one, out, (hipStream_t)stream);
+  }
   auto* select = s->half ? ri_score_select_f16 : ri_score_select;
   auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
   const int rc = select(q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,

@@ -18,7 +18,7 @@ static inline bool attend_alone(int64_t rows, int gs, int BG) { return rows * gs
 // 13.8 / 12.4, 1 of 8, 40000 18.0 / 16.5, 8 of 8, 20000 21.2 / 19.3, 6 of 8, 3000 9.4 / 9.1; half a line the same.
 static constexpr int attend_counter_pitch(int BG) { return BG <= 16 ? 32 : BG <= 32 ? 16 : BG <= 64 ? 8 : 4; }
 
-// Short: what one workgroup may have to itself (step_is_alone: and does).  It scores for itself (select.hip), and usually (16
+// Short: what one workgroup may have to itself.  It scores for itself (select.hip), and usually (16
 // tokens per retrieved cluster) has no more rows than it attends as fast as scoring + selection and attention in launches of their own
 // do.  Captured layers with their appends, us, by the rows, one workgroup / in launches of their own: 8 groups of 8 heads 391 rows 18.4 / 19.2,
 // 451 19.0 / 19.0, 521 20.2 / 19.2; of 4 heads 451 18.1 / 18.0, 521 18.8 / 18.2; one group of 8 heads 451 17.9 / 18.1, 521 19.8 / 18.4.
@@ -58,15 +58,12 @@ static inline bool step_is_joined(const ri_decode_step_t* s) {
   return step_is_wide(s) || (s->np <= 512 && (s->gs <= 8 || 3 * s->np + s->es <= 8000));
 }
 
-// Of the short steps those that one workgroup per group makes.  Several take the same at any length, and where they find no more rows
-// than the line they leave them to one of them (step_kernel).  The lines were drawn when that, and several that all work, were behind
-// one at the first lengths.  With the present kernels they are not, up to the line within 0.4 us of one workgroup and past it
-// ahead.  Captured layers with their appends, us, by the rows, one / several that all work / several that leave: 8 groups of 4 heads, 192
-// clusters 161 15.1 / 16.0 / 14.8, 281 15.9 / 16.2 / 15.6, 411 17.0 / 16.0 / 16.1, 512 clusters 331 16.3 / 16.1 / 16.1, 451 18.1 / 16.2 / 16.2; 8 of 8, 320
-// 223 16.2 / 16.9 / 15.8, 343 17.6 / 16.9 / 16.7; 32 of 4, 512 331 17.3 / 17.4 / 17.6, 451 19.4 / 17.6 / 17.8.  With two workgroups per group only: 128
-// groups of 4 heads, 512 331 18.7 / 20.1 / 18.9, 451 20.9 / 21.7 / 21.1, 581 22.3 / 22.4 / 22.3, of 8 heads 331 20.1 / 21.0 / 19.9, 581 23.3 / 23.0 / 22.9;
-// past 128 there is no second one.
-// A captured step starts at the length at hand and ends at the zone's, and may grow past the line.  Zones of 69 to 323 rows, us a layer
+// Of the short steps those that one workgroup per group holds its own in. Past 128 groups there is no second one, and it makes them; up
+// to them several that leave few rows to one of them (step_kernel, by step_alone_rows) are ahead everywhere and make all, inside
+// these lines too, which nothing but their test asks for any more. Captured layers with their appends, us, one / several: 8 groups of 4 heads, 512
+// clusters 13.85 / 13.35; of 1, 104 11.65 / 11.40; of 8, 256 13.30 / 12.90; 88 of 1, 120 12.10 / 11.85; 24 of 1, 104 11.95 / 11.65; 16 of 4, 256 12.35 /
+// 12.10; 32 of 4, 496 13.75 / 13.40; 128 of 4, 496 15.20 / 14.90, of 8, 256 14.10 / 13.70; 1 of 4, 320 11.90 / 11.60.
+// A captured step starts at the length at hand and ends at the zone's, and may grow past the line. Earlier kernels, zones of 69 to 323 rows, us a layer
 // at the first length, on average and at the last, several | one: 16 groups of 4 heads, up to 508 rows 15.6, 16.7, 17.7 | 15.8, 17.2, 18.8;
 // 32 of 4, 508 16.6, 17.8, 18.4 | 16.8, 18.3, 19.9; 64 of 4, 477 16.5, 17.8, 18.8 | 16.6, 18.0, 19.4; 32 of 8, 446 16.4, 18.1, 19.1 | 16.7, 18.4,
 // 20.2; 40 of 2, 477 16.1, 17.2, 18.1 | 16.4, 17.8, 19.2.  Past the line 24 of 4, 531 16.7, 17.4, 18.4 | 16.7, 18.3, 19.9; 64 of 4, 554 17.5, 18.6,
