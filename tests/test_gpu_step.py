@@ -98,3 +98,12 @@ def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static
 def test_joined_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
     """Steps whose attention's workgroups make the selection: the same lists, and outputs as above."""
     test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BG,gs,nc,np_,es,static,pages,on_device", [
+    # who sums the scores: on both sides of 2048 clusters for seven and eight heads, of 4096 for six, with 1024 selecting threads too
+    (2, 7, 2048, 36, 475, 69, 300, False), (2, 7, 2056, 36, 475, 69, 300, True), (3, 8, 2056, 600, 300, 69, 4000, False),
+    (2, 6, 2056, 37, 470, 69, 300, False), (2, 6, 4096, 73, 950, 69, 600, False), (2, 6, 4104, 73, 950, 69, 600, True)])
+def test_joined_step_at_the_line_of_the_sums(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
+    test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
