@@ -433,6 +433,15 @@ __device__ __forceinline__ int rank_of(const int* off, int n, int row) {
   }
 }
 
+// The waves' numerators for the merge where they do not fit the wave's own value tile (see attend_group): free until then.
+template <int GS_PAD>
+__device__ __forceinline__ float* att_numerators() {
+  constexpr bool OWN = GS_PAD * RI_DIM * sizeof(float) > 16 * ATT_VT_STRIDE * sizeof(uint16_t);
+  __shared__ __attribute__((aligned(16))) float sh_acc[OWN ? ATT_WAVES : 1][OWN ? GS_PAD : 1][RI_DIM];
+  static_assert(__alignof__(sh_acc) == 16, "read two dims at a time");
+  return &sh_acc[0][0][0];
+}
+
 template <int GS_PAD, bool HALF, int KEPT>
 __device__ __forceinline__ void attend_group(const AttendParams& P, const int g, const int split, const AttendKept& K) {
   constexpr int NW = ATT_WAVES;
@@ -448,10 +457,8 @@ __device__ __forceinline__ void attend_group(const AttendParams& P, const int g,
   // rows are done), which keeps a workgroup at 48 KB of LDS, so that the two its registers leave room for fit a compute
   // unit (sixteen heads: 116 KB, one workgroup)
   constexpr bool ACC_OVER_VT = GS_PAD * RI_DIM * sizeof(float) <= 16 * ATT_VT_STRIDE * sizeof(uint16_t);
-  __shared__ __attribute__((aligned(16))) float sh_acc_own[ACC_OVER_VT ? 1 : NW][ACC_OVER_VT ? 1 : GS_PAD][RI_DIM];
-  static_assert(__alignof__(sh_acc_own) == 16, "read two dims at a time");
   auto acc_of = [&](int w) -> float* {
-    return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : &sh_acc_own[ACC_OVER_VT ? 0 : w][0][0];
+    return ACC_OVER_VT ? reinterpret_cast<float*>(sh_vt[w]) : att_numerators<GS_PAD>() + (size_t)w * GS_PAD * RI_DIM;
   };
   __shared__ int sh_desc[NW][ATT_DESC_MAX];
   __shared__ float sh_w[NW][ATT_DESC_MAX];

@@ -115,7 +115,10 @@ struct SelectKept {
   int* ids;        // [np]
   int* meta;       // [4]
   uint32_t* scratch;   // [SEL_SCRATCH<NT>] what the attention has not laid anything in yet
+  uint4* area;         // SEL_SCORE of more than eight heads: SEL_AREA<NT, GSM> bytes, the same (their logits go to memory)
 };
+template <int NT, int GSM>
+constexpr size_t SEL_AREA = NT / 64 * 256 * sizeof(uint4) + (size_t)NT * GSM * sizeof(uint16_t);
 enum { KEEP_NONE, KEEP_TABLES };
 
 // Bins of the rank search.  Scores are sums of at most sixteen probabilities: in bfloat16 (128 keys to an octave) a bin for
@@ -156,7 +159,6 @@ __device__ __forceinline__ uint32_t sel_above(uint32_t a, uint32_t b) {
 // past the list.
 template <int NT, int E, int GSM, bool HALF, int SRC, int KEEP, typename Ahead>
 __device__ __forceinline__ int select_group(const SelectArgs& P, const int g, const SelectKept& K, Ahead&& ahead) {
-  static_assert(KEEP == KEEP_NONE || SRC != SEL_SCORE || GSM <= 8, "the logits are in LDS");
   constexpr bool STORE = !KEEP;
   constexpr int NW = NT / 64, IDS = NT * E;
   constexpr int LOGT = NT == 256 ? 8 : (NT == 512 ? 9 : 10);
@@ -174,9 +176,12 @@ __device__ __forceinline__ int select_group(const SelectArgs& P, const int g, co
   constexpr bool OWN = GSM <= 8;   // who computes the probabilities, see below
   __shared__ __attribute__((aligned(16))) int32_t sh_size[STAGED ? IDS : 4], sh_row[STAGED ? IDS : 4];
   __shared__ __attribute__((aligned(16))) float sh_x[SRC == SEL_SCORE && OWN && !KEEP ? IDS * GSM : 4];
-  __shared__ __attribute__((aligned(16))) uint16_t sh_p[SRC == SEL_SCORE && !OWN ? IDS * GSM : 8];
+  constexpr bool LENT = KEEP && SRC == SEL_SCORE && !OWN;   // the rows' turn and the probabilities lie in what the attention lends
+  __shared__ __attribute__((aligned(16))) uint16_t sh_p_own[SRC == SEL_SCORE && !OWN && !LENT ? IDS * GSM : 8];
   __shared__ float sh_a[SRC == SEL_SCORE ? NW : 1][16], sh_b[SRC == SEL_SCORE ? NW : 1][16];
-  __shared__ __attribute__((aligned(16))) uint4 sh_rows[SRC == SEL_SCORE ? NW : 1][SRC == SEL_SCORE ? 256 : 1];
+  __shared__ __attribute__((aligned(16))) uint4 sh_rows_own[SRC == SEL_SCORE && !LENT ? NW : 1][SRC == SEL_SCORE ? 256 : 1];
+  auto* const sh_rows = LENT ? reinterpret_cast<uint4 (*)[SRC == SEL_SCORE ? 256 : 1]>(K.area) : sh_rows_own;
+  uint16_t* const sh_p = LENT ? reinterpret_cast<uint16_t*>(K.area + NW * 256) : sh_p_own;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nc = P.nc, np = P.np, es = P.es, k2 = np + es, gs = P.gs;
   const int cbeg = tid * E;   // nc % 8 == 0: a thread's ids exist together, from E = 16 on in eights

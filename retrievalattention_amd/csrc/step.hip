@@ -64,7 +64,8 @@ __device__ __forceinline__ void store_selection(const SelectArgs& S, int g, cons
 // the second half finds ids, tables and logits in LDS, and a launch is left out, which counts on the
 // host as well.  What bounds it is the chain of either half on one compute unit.  Captured layers with their appends, in launches of
 // their own -> one, us: 8 groups of 4 heads, 512 clusters, 331 rows 18.0 -> 16.3; 8 heads 19.0 -> 17.8; 128 groups of 4 20.7 -> 18.7.
-// 103564 bytes of LDS (113036 with 8 heads): one workgroup per compute unit, hence at most 256 groups; sixteen heads would not fit.
+// 103564 bytes of LDS (113036 with 8 heads): one workgroup per compute unit, hence at most 256 groups; more
+// heads: launch_score_attend.
 // SPLIT: several workgroups per group, which all make the same selection and attend a part of the rows each (see
 // select_attend_kernel): with the query and the zone's length requested behind the first loads and the results stored behind
 // the attention, the launch takes much the same at any length.  8 groups of 8 heads, 512 clusters, 331 / 521 / 831 / 1331 rows:
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void step_kernel(ri_ptr4 in, ri_int
   S.np = A.np = n[2];
   S.es = A.es = n[3];
   S.scale = A.scale = scale;
-  const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta, select_scratch<STEP_CLUSTERS>()};
+  const SelectKept kept = {sh_logits, sh_est, sh_off, sh_start, sh_ids, sh_meta, select_scratch<STEP_CLUSTERS>(), nullptr};
   AttendKept known = {sh_logits, sh_est, sh_off, sh_start};
   uint4 query;
   select_group<STEP_CLUSTERS, 1, GSM, HALF, SEL_SCORE, KEEP_TABLES>(S, blockIdx.x, kept, [&] {
@@ -156,6 +157,10 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
   AttendParams A = A0;
   if (SRC == SEL_KEYS) {
     S.keys = ri_global<uint16_t>(in[0]);
+  } else if (SRC == SEL_SCORE) {
+    S.cent = ri_global<const uint16_t>(in[0]);
+    S.q = A.q = ri_global<const uint16_t>(in[1]);
+    S.cluster_size = ri_global<const int32_t>(in[2]);
   } else {
     S.logits = ri_global<float>(in[0]);
     S.tile_max = ri_global<float>(in[1]);
@@ -171,7 +176,10 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
   A.W_kv = m[1];
   const int np = S.np, g = blockIdx.x;
   int *const meta = sh_kept, *const off = meta + 4, *const start = off + np + 1, *const ids = start + np, *const est = ids + np;
-  const SelectKept kept = {nullptr, est, off, start, ids, meta, select_scratch<NT>()};
+  static_assert(SRC != SEL_SCORE || SEL_AREA<NT, GSM> <= (size_t)ATT_WAVES * GSM * RI_DIM * sizeof(float), "room in the numerators");
+  static_assert(SRC != SEL_SCORE || GSM == 16, "step_kernel's otherwise");
+  const SelectKept kept = {nullptr, est, off, start, ids, meta, select_scratch<NT>(),
+                           SRC == SEL_SCORE ? reinterpret_cast<uint4*>(att_numerators<GSM>()) : nullptr};
   AttendKept known = {nullptr, est, off, start};
   uint4 query;
   select_group<NT, E, GSM, HALF, SRC, KEEP_TABLES>(S, g, kept, [&] {
@@ -180,6 +188,7 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
     att_clear<GSM>();
   });
   att_put_query<GSM>(query, S.gs);
+  if (SRC == SEL_SCORE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the logits, which other waves read back)
   lds_barrier();
   if (NT > 64 * ATT_WAVES && threadIdx.x >= 64 * ATT_WAVES) return;
   attend_group<GSM, HALF, KEPT_TABLES>(A, g, blockIdx.y, known);
@@ -199,6 +208,18 @@ static void launch_select_attend(const SelectArgs& S, const AttendParams& A, int
   kernel<<<dim3(BG, A.S), NT, lds, stream>>>(ri_pack_ptrs(a, S.tile_max, S.tile_sum, S.mask),
                                                          (ri_int4){S.nc, S.gs, S.np, S.es}, (ri_int2){S.ntiles | A.S << 16, A.W_kv}, S,
                                                          A);
+}
+
+// More than eight heads over few clusters: scoring, selection and attention in one launch too, but the logits go to memory, from
+// which the attention's waves read them back (every workgroup of a group writes the same ones), and the selection's rows and
+// probabilities lie where the numerators will: LDS holds no more. What bounds it is the same chain as step_kernel's. Captured layers with their
+// appends, us, selection and attention in launches of their own / as it is: 8 groups of 16 heads, 480 clusters 19.15 / 17.25; of 12, 256 16.8 / 15.1;
+// 1 of 12, 192 15.7 / 14.3; 32 of 16, 512 20.0 / 17.9; 2 of 16, 160 16.6 / 15.2; 128 of 12, 384 19.9 / 17.8; 16 of 12, 448 17.65 / 15.7.
+static void launch_score_attend(const SelectArgs& S, const AttendParams& A, int BG, bool half, hipStream_t stream) {
+  auto* kernel = half ? select_attend_kernel<512, 1, 16, true, SEL_SCORE> : select_attend_kernel<512, 1, 16, false, SEL_SCORE>;
+  const size_t lds = (size_t)(4 + 3 * S.np + 1 + S.es) * sizeof(int);
+  kernel<<<dim3(BG, A.S), 512, lds, stream>>>(ri_pack_ptrs(S.cent, S.q, S.cluster_size, S.mask), (ri_int4){S.nc, S.gs, S.np, S.es},
+                                              (ri_int2){S.ntiles | A.S << 16, A.W_kv}, S, A);
 }
 
 template <bool SPLIT>
@@ -224,10 +245,11 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
                                  s->store_v, s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta,
                                  s->est_ids, s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out,
                                  s->valid_lengths, s->BG, s->gs, s->nc, s->es, s->scale, s->attn_workspace,
-                                 s->attn_workspace_bytes, alone ? ATT_ONE : S.nc <= STEP_CLUSTERS ? ATT_SEVERAL : ATT_PLAN);
+                                 s->attn_workspace_bytes, alone ? ATT_ONE : S.nc <= STEP_CLUSTERS && S.gs <= 8 ? ATT_SEVERAL : ATT_PLAN);
   if (rc) return rc;
   if (S.nc <= STEP_CLUSTERS) {
-    if (alone) launch_step<false>(S, A, s->BG, s->half, stream);
+    if (S.gs > 8) launch_score_attend(S, A, s->BG, s->half, stream);
+    else if (alone) launch_step<false>(S, A, s->BG, s->half, stream);
     else launch_step<true>(S, A, s->BG, s->half, stream);
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;

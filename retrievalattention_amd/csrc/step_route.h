@@ -46,14 +46,14 @@ static inline bool step_is_short(const ri_decode_step_t* s, int static_len) {
 
 // Selection and attention in one launch, and the scoring too up to STEP_CLUSTERS: what step.hip's kernels hold.  (A probe per
 // thread; 512 threads, or wide 1024, whose registers do not hold sixteen heads; up to 32 clusters a thread; with sixteen heads
-// 32 KB of LDS are left for the tables; without sizes and first rows there are none.  A workgroup that scores has a compute unit
+// 32 KB of LDS are left for the tables, of which those of up to 512 clusters take 8; without sizes and first rows there are none.  A workgroup that scores has a compute unit
 // to itself: 264 groups of 4 heads, 512 clusters, a captured layer 33.2 us in two launches, 36.4 in one.)
 static inline bool step_is_wide(const ri_decode_step_t* s) {
   return s->gs <= 8 && s->np <= 1024 && (s->nc > 8192 || s->np > 512);
 }
 static inline bool step_is_joined(const ri_decode_step_t* s) {
   if (!s->cluster_size_i32 || !s->cluster_start) return false;
-  if (s->nc <= STEP_CLUSTERS) return s->gs <= 8 && s->BG <= 256;
+  if (s->nc <= STEP_CLUSTERS) return s->BG <= 256;
   if (s->nc > 16384) return false;
   return step_is_wide(s) || (s->np <= 512 && (s->gs <= 8 || 3 * s->np + s->es <= 8000));
 }

@@ -107,3 +107,15 @@ def test_joined_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, stati
     (2, 6, 2056, 37, 470, 69, 300, False), (2, 6, 4096, 73, 950, 69, 600, False), (2, 6, 4104, 73, 950, 69, 600, True)])
 def test_joined_step_at_the_line_of_the_sums(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
     test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("BG,gs,nc,np_,es,static,pages,on_device", [
+    # more than eight heads over few clusters: one workgroup per group and several, few and many waves that score, no estimation zone,
+    # a probe list that is all clusters, cut pages, and past the limits
+    (1, 9, 8, 3, 2, 1, 100, False), (2, 16, 8, 8, 0, 0, 100, True), (5, 12, 40, 7, 33, 300, 100, False), (8, 16, 256, 5, 60, 70, 3, True),
+    (3, 10, 264, 30, 200, 69, 300, False), (8, 12, 480, 9, 110, 98, 100, False), (2, 16, 512, 512, 0, 69, 2000, False),
+    (1, 13, 512, 51, 461, 700, 500, True), (130, 9, 64, 6, 20, 90, 100, False), (256, 16, 32, 4, 8, 20, 100, False),
+    (257, 16, 32, 4, 8, 20, 100, False)])
+def test_few_clusters_of_many_heads(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
+    test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
