@@ -116,7 +116,9 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 res = _cluster(key, nc, num_iters, S, init_indices, key_store is None, centroids)
-            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph, as the result's are)
+            if centroids is not None:
+                res.centroids = None                  # (the caller's: kept by its address, as the keys are, and not alive)
+            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph)
             _GRAPHS[gkey] = hit
             while len(_GRAPHS) > _MAX_GRAPHS:
                 _GRAPHS.popitem(last=False)
@@ -126,6 +128,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
             r = KMeansResult()
             for f in ("centroids", "assign", "counts", "offsets", "members"):
                 setattr(r, f, getattr(hit[1], f))
+            if centroids is not None:
+                r.centroids = centroids
         else:
             _SEEN[gkey] = True
             while len(_SEEN) > 64:

@@ -367,8 +367,8 @@ class retroinfer_cache(KV_Cache):
         if ck is None:
             if len(self._centred_keys) >= 2:
                 self._centred_keys.clear()
-            ck, cc = (torch.empty((H, n, head_dim), dtype=keys.dtype, device=keys.device)
-                      for n in (valid_length, self.n_centroids))
+            both = torch.empty((H * (valid_length + self.n_centroids), head_dim), dtype=keys.dtype, device=keys.device)
+            ck, cc = (x.view(H, -1, head_dim) for x in both.split((H * valid_length, H * self.n_centroids)))
             self._centred_keys[buffers] = ck, cc
         mean_key = kernels.prefill_mean(keys, lo, valid_length)
         if mean_key is None:

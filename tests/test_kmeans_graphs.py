@@ -35,3 +35,26 @@ def test_a_captured_clustering_is_replayed_for_its_own_kind_of_call(monkeypatch,
     assert len(launched) == 2 and len(replayed) == 2     # launched, captured and replayed, replayed
     call(**change)
     assert len(launched) == 3 and len(replayed) == 2
+
+
+def test_a_captured_clustering_keeps_no_buffer_of_its_caller(monkeypatch):
+    """Initial centroids that the caller hands over are the result's, by their address: neither they nor the keys stay alive with
+    the graph, and other ones are another clustering."""
+    import weakref
+    monkeypatch.setattr(kmeans, "_GRAPHS", kmeans.collections.OrderedDict())
+    monkeypatch.setattr(kmeans, "_SEEN", kmeans.collections.OrderedDict())
+    replayed = []
+    monkeypatch.setattr(kmeans, "_cluster", lambda key, *a: SimpleNamespace(
+        centroids=a[-1], assign=None, counts=None, offsets=None, members=None))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: SimpleNamespace(replay=lambda: replayed.append(1)))
+    monkeypatch.setattr(torch.cuda, "graph", lambda g: contextlib.nullcontext())
+    monkeypatch.setattr(kernels, "kmeans_value_sum", lambda *a, **k: None)
+    key, centroids, other = (torch.zeros(1, 64, 128, dtype=torch.bfloat16) for _ in range(3))
+    call = lambda c: kmeans.segment_k_means_csr(key, key, 64, reuse_graph=True, centroids=c)
+    for _ in range(3):
+        assert call(centroids).centroids is centroids
+    assert len(replayed) == 2 and call(other).centroids is other and len(replayed) == 2
+    held = weakref.ref(centroids)
+    del centroids
+    assert held() is None
