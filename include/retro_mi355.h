@@ -546,8 +546,9 @@ int ri_lru_stage_update(const ri_lru_t* lru, ri_stream_t stream);
 
 /* The decode step of one layer over a host-resident store with the device-side block cache (compute(),
  * cache_hub/retroinfer_cache.py:549-697): what ri_score_select and ri_lru_access do (selection and look-up in
- * one launch where a thread has one probe and the selection sums the scores), ri_lru_stage_update, ri_wave_attention over the row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`, store_k / store_v are the cache tensors of
- * `lru` and ret_tok_off, ret_start, cluster_start are not used. */
+ * one launch where a thread has one probe and the selection sums the scores), ri_lru_stage_update,
+ * ri_wave_attention over the row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`,
+ * store_k / store_v are the cache tensors of `lru` and ret_tok_off, ret_start, cluster_start are not used. */
 int ri_host_step(const ri_decode_step_t* step, const ri_lru_t* lru, const void* q, int static_len, void* out,
                  ri_stream_t stream);
 

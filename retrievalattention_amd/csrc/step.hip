@@ -258,9 +258,11 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
   // clusters 44.8 / 47.6, 5632 36.1 / 38.7, 4096 29.5 / 29.2; 8 of 4, 5632 24.3 / 26.5; of 1, 32 of 8192 42.9 / 44.0; 8 of 16, 2048 26.0 / 25.9;
   // 64 of 16, 1024 28.8 / 27.6; 12 of 7, 1920 23.0 / 22.0; 32 of 8, 2048 25.7 / 24.7. Between 2048 and
   // 4096 clusters: 8 of 7, 2304 19.6 / 20.4, 2816 20.6 / 21.2; 8 of 8, 3328 21.6 / 22.3, 32 of 8, 2304 24.2 / 25.0, 2816 24.9 / 25.7, 64 of 8, 2816 31.8 / 32.5;
-  // 2 of 7, 2560 19.3 / 20.5; but 16 of 5, 2560 20.8 / 20.8, 128 of 6, 3104 52.8 / 52.4.
+  // 2 of 7, 2560 19.3 / 20.5, 64 of 7, 2560 30.1 / 30.9; but 16 of 5, 2560 20.8 / 20.8, 128 of 6, 3104 52.8 / 52.4. More groups fill
+  // the chip with selecting workgroups, and the second launch is not made up for: 128 of 7, 2304 42.7 / 42.3, 2816 51.8 / 50.7, 3328
+  // 56.9 / 56.7, of 8, 2304 43.9 / 43.6, 2816 52.2 / 52.5; 64 of 7, 2304 29.9 / 29.7.
   // (512 threads: eight clusters each past 2048, and with sixteen heads that is more than the registers hold.)
-  const bool keys = S.nc > (S.gs <= 6 ? 4096 : 2048);
+  const bool keys = S.nc > (S.gs <= 6 || s->BG > 64 ? 4096 : s->BG > 48 ? 2432 : 2048);
   rc = ri_launch_select_inputs(S, s->BG, s->half, keys, stream);
   if (rc) return rc;
   if (wide) {
