@@ -1,4 +1,4 @@
-// The group's half of the device-side block cache manager (see lru.hip), also behind a selection (host_step.hip).
+// The group's half of the device-side block cache manager (see lru.hip), also behind a selection.
 #pragma once
 #include "ri_common.h"
 

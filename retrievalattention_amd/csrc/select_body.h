@@ -787,6 +787,6 @@ int ri_prepare_select(SelectArgs* P, const void* q, const void* centroids, const
 // Scoring, and the scores' sums and keys if `keys` (select.hip)
 int ri_launch_select_inputs(const SelectArgs& P, int BG, bool half, bool keys, hipStream_t s);
 
-// Scoring, selection and the block cache's look-up of the selected clusters (host_step.hip); `taken`: false, and nothing launched,
+// Scoring, selection and the block cache's look-up of the selected clusters (lru.hip); `taken`: false, and nothing launched,
 // where that is not worth a launch of its own kind.
 int ri_launch_select_access(const SelectArgs& P, const ri_lru_t& lru, int BG, bool half, bool* taken, hipStream_t s);
