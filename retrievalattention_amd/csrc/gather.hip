@@ -99,7 +99,7 @@ extern "C" int ri_gather_copy_vectors(const void* src_keys, void* dst_keys, cons
                                       int index_size, int copy_start, int copy_num, ri_stream_t stream) {
   if (!src_keys || !dst_keys || !src_values || !dst_values || !src_meta || !dst_meta || !idx) return RI_ERR_ARG;
   if (ri_any_misaligned16(src_keys, dst_keys, src_values, dst_values)) return RI_ERR_ARG;
-  if (groups <= 0 || copy_num < 0 || copy_start < 0 || copy_start + copy_num > index_size ||
+  if (groups <= 0 || copy_num < 0 || copy_start < 0 || (int64_t)copy_start + copy_num > index_size ||
       copy_num > buffer_length)
     return RI_ERR_ARG;
   if (copy_num == 0) return RI_OK;

@@ -267,8 +267,9 @@ PyObject* gather_vectors(PyObject*, PyObject* const* args, Py_ssize_t n) {
       !device_tensors(args + 6, 1, at::kLong, t + 6) || !integers(args + 7, 6, x))
     Py_RETURN_NONE;
   const int64_t groups = x[0], data = x[1], buffer = x[2];
-  if (!holds(t[0], groups, data, 128) || !holds(t[1], groups, buffer, 128) || !holds(t[6], groups, x[3], 1) ||
-      !holds(t[4], groups, data, 1) || !holds(t[5], groups, buffer, 1))
+  if (!holds(t[0], groups, data, 128) || !holds(t[1], groups, buffer, 128) || !holds(t[2], groups, data, 128) ||
+      !holds(t[3], groups, buffer, 128) || !holds(t[4], groups, data, 1) || !holds(t[5], groups, buffer, 1) ||
+      !holds(t[6], groups, x[3], 1))
     Py_RETURN_NONE;
   void* p[7];
   for (int i = 0; i < 7; ++i) p[i] = address(t[i]);
@@ -283,7 +284,7 @@ PyObject* gather_vectors(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // flash(q, k, v, weight, previous_out, previous_lse, cache_seqlens, workspace, scale, return_lse): the output, or (output, lse);
-// a status that is not zero; None as above.  q [BG, 1, gs, 128], k [BG, S, 1, 128].
+// a status that is not zero; None as above.  q [BG, 1, gs, 128], k [BG, S, 1, 128]; the others by their elements.
 PyObject* flash(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   const at::Tensor *t[7], *ws;
@@ -296,6 +297,9 @@ PyObject* flash(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const at::Tensor &q = *t[0], &k = *t[1];
   if (q.dim() != 4 || k.dim() != 4 || q.size(1) != 1 || q.size(3) != 128 || k.size(2) != 1) Py_RETURN_NONE;
   const int64_t BG = q.size(0), gs = q.size(2), S = k.size(1);
+  if (!holds(t[1], BG, S, 128) || !holds(t[2], BG, S, 128) || (t[3] && !holds(t[3], BG, S, 1)) ||
+      (t[4] && (!holds(t[4], BG, gs, 128) || !holds(t[5], BG, gs, 1))) || (t[6] && !holds(t[6], BG, 1, 1)))
+    Py_RETURN_NONE;
   const double scale = PyFloat_AsDouble(args[8]);
   const int with_lse = PyObject_IsTrue(args[9]);
   if (PyErr_Occurred()) return nullptr;

@@ -206,6 +206,7 @@ def gather_copy_vectors(key_data, key_buffer, value_data, value_buffer, src_meta
               ("key_data", "key_buffer", "value_data", "value_buffer", "src_metadata", "dst_metadata"))
     _need(data_offsets, torch.int64, "data_offsets")
     if key_data.numel() < groups * data_length * 128 or key_buffer.numel() < groups * buffer_length * 128 or \
+            value_data.numel() < groups * data_length * 128 or value_buffer.numel() < groups * buffer_length * 128 or \
             data_offsets.numel() < groups * index_size or src_metadata.numel() < groups * data_length or \
             dst_metadata.numel() < groups * buffer_length:
         raise ValueError("gather_copy_vectors: a buffer is smaller than its shape arguments")
@@ -284,6 +285,10 @@ def weighted_flash_decoding(q, k, v, weight=None, previous_out=None, previous_ls
         _need(previous_lse, torch.float32, "previous_lse")
     if cache_seqlens is not None:
         _need(cache_seqlens, torch.int32, "cache_seqlens")
+    if k.numel() < BG * S * D or v.numel() < BG * S * D or (weight is not None and weight.numel() < BG * S) or \
+            (previous_out is not None and (previous_out.numel() < q.numel() or previous_lse.numel() < BG * gs)) or \
+            (cache_seqlens is not None and cache_seqlens.numel() < BG):
+        raise ValueError("weighted_flash_decoding: a tensor is smaller than the shapes of q and k ask for")
     out = torch.empty_like(q)
     lse = torch.empty((BG, gs), dtype=torch.float32, device=q.device) if return_softmax_lse else None
     ws = _workspace(_flash_workspace_bytes(BG, gs), q.device, "attn", scratch)

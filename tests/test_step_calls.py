@@ -37,6 +37,71 @@ def test_what_is_no_plain_device_tensor_is_left_to_the_general_way():
         native.append(x)
 
 
+def _gather_args(device="cpu", short=None):
+    """Two groups, 24 rows each, 5 of them gathered; `short`: the argument that has an element too few."""
+    e = lambda n, name, dt=torch.bfloat16: torch.zeros(n - (name == short), dtype=dt, device=device)  # noqa: E731
+    return (e(2 * 24 * 128, "key_data"), e(2 * 8 * 128, "key_buffer"), e(2 * 24 * 128, "value_data"),
+            e(2 * 8 * 128, "value_buffer"), e(2 * 24, "src_metadata"), e(2 * 8, "dst_metadata"),
+            e(2 * 10, "data_offsets", torch.int64), 2, 24, 8, 10, 3, 5)
+
+
+def _flash_args(device="cpu", short=None):
+    """q, k, v, weight, previous_out, previous_lse, cache_seqlens of two groups of three heads over 24 rows; `short`: the one that
+    has rows (k) or elements too few."""
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(s, dtype=dt, device=device)  # noqa: E731
+    e = lambda n, name, dt=torch.bfloat16: z(n - (name == short), dt=dt)  # noqa: E731
+    return (z(2, 1, 3, 128), z(2 - (short == "k"), 24, 1, 128), e(2 * 24 * 128, "v"), e(2 * 24, "weight"),
+            e(2 * 3 * 128, "previous_out"), e(2 * 3, "previous_lse", torch.float32), e(2, "cache_seqlens", torch.int32))
+
+
+GATHERED = ("key_data", "key_buffer", "value_data", "value_buffer", "src_metadata", "dst_metadata", "data_offsets")
+ATTENDED = ("k", "v", "weight", "previous_out", "previous_lse", "cache_seqlens")
+
+
+@pytest.mark.parametrize("short", (None,) + GATHERED + ATTENDED)
+def test_short_buffers_are_refused_before_a_launch(monkeypatch, short):
+    """The wrappers' general way, on host tensors that it is told to take: nothing is called with a buffer that is smaller than
+    the other arguments say."""
+    calls = []
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *a: calls.append(name) or 0
+    for name in ("_need", "_need_all"):
+        monkeypatch.setattr(kernels, name, lambda *a, **k: None)
+    monkeypatch.setattr(kernels, "lib", Library)
+    monkeypatch.setattr(kernels, "_stream", lambda: 0)
+    monkeypatch.setattr(kernels, "_workspace", lambda *a: torch.zeros(1))
+    monkeypatch.setattr(kernels, "_flash_workspace_bytes", lambda *a: 256)   # (it keeps what the library says)
+    for names, call in ((GATHERED, lambda: kernels.gather_copy_vectors(*_gather_args(short=short))),
+                        (ATTENDED, lambda: kernels.weighted_flash_decoding(*_flash_args(short=short)))):
+        calls.clear()
+        if short in names:
+            with pytest.raises(ValueError, match="smaller"):
+                call()
+            assert not calls
+        else:
+            call()
+            assert len(calls) == 1
+
+
+@pytest.mark.gpu
+def test_short_buffers_are_left_to_the_general_way(dev):
+    """The native calls launch nothing then, and the general way raises."""
+    native = step_calls()
+    assert native.gather_vectors(*_gather_args(dev)) == 0
+    ws = kernels._workspace(kernels._flash_workspace_bytes(2, 3), dev, "attn")
+    assert isinstance(native.flash(*_flash_args(dev), ws, 1.0, False), torch.Tensor)
+    for short in GATHERED:
+        assert native.gather_vectors(*_gather_args(dev, short)) is None, short
+        with pytest.raises(ValueError):
+            kernels.gather_copy_vectors(*_gather_args(dev, short))
+    for short in ATTENDED:
+        assert native.flash(*_flash_args(dev, short), ws, 1.0, False) is None, short
+        with pytest.raises(ValueError):
+            kernels.weighted_flash_decoding(*_flash_args(dev, short))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("change,takes", [
     (dict(), True), (dict(pos=4), True), (dict(pos=5), False), (dict(shape=(2, 1, 3)), False), (dict(shape=(2, 3, 1, 128)), False),
