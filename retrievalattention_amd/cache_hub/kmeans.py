@@ -79,6 +79,22 @@ _SEEN = collections.OrderedDict()
 _MAX_GRAPHS = 4
 
 
+def _graph_key(key, nc, num_iters, S, final_means, init_indices, given):
+    return (key.data_ptr(), key.dtype, key.shape, key.device, nc, num_iters, S, final_means,
+            None if init_indices is None else init_indices.data_ptr(), given)
+
+
+def initial_centroids(key, num_centroids, num_iters=10, num_segments=1, final_means=True):
+    """[G, nc, 128] tensor for the initial centroids of a call of segment_k_means_csr with reuse_graph (final_means: without
+    key_store): a captured clustering's own, which its replays start from and end in, else a new one."""
+    hit = None
+    if not torch.cuda.is_current_stream_capturing():
+        hit = _GRAPHS.get(_graph_key(key, num_centroids, num_iters, num_segments, final_means, None, True))
+    if hit is not None:
+        return hit[1].centroids
+    return torch.empty((key.shape[0], num_centroids, key.shape[2]), dtype=key.dtype, device=key.device)
+
+
 def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1, init_indices=None,
                         reuse_graph=False, value_sum=None, value_store=None, store_stride=0, key_rows=None, key_mean=None,
                         key_store=None, index=None, centroids=None):
@@ -89,7 +105,8 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
     written cluster by cluster, store_stride rows from group to group.  key_store (with value_store): the same for
     key_rows, the [G, N, 128] keys before key_mean was subtracted.  index (with key_mean): the tensors that
     kernels.prefill_index fills, filled here, with key_store in its launches.  centroids: [G, nc, 128] tensor with what
-    kernels.kmeans_init gives for the keys; the result's centroids are in it.
+    kernels.kmeans_init gives for the keys, best in an initial_centroids(); it is written over, and the result's centroids are
+    in it or in the captured clustering's.
 
     reuse_graph (off unless asked for): the second call with keys at the same address and of the same
     type, shape and parameters captures the launches into a HIP graph, and later such calls replay it.
@@ -109,27 +126,24 @@ def segment_k_means_csr(key, value, num_centroids, num_iters=10, num_segments=1,
         raise AssertionError("centroids per segment must be a multiple of 32")  # kmeans.py:99
     r = None
     if reuse_graph and not torch.cuda.is_current_stream_capturing():
-        gkey = (key.data_ptr(), key.dtype, tuple(key.shape), str(key.device), nc, num_iters, S, key_store is None,
-                None if init_indices is None else init_indices.data_ptr(), None if centroids is None else centroids.data_ptr())
+        gkey = _graph_key(key, nc, num_iters, S, key_store is None, init_indices, centroids is not None)
         hit = _GRAPHS.get(gkey)
         if hit is None and gkey in _SEEN:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 res = _cluster(key, nc, num_iters, S, init_indices, key_store is None, centroids)
-            if centroids is not None:
-                res.centroids = None                  # (the caller's: kept by its address, as the keys are, and not alive)
-            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph)
+            hit = (graph, res, init_indices)          # (the index tensor stays alive with the graph, as given centroids do)
             _GRAPHS[gkey] = hit
             while len(_GRAPHS) > _MAX_GRAPHS:
                 _GRAPHS.popitem(last=False)
         if hit is not None:
             _GRAPHS.move_to_end(gkey)
+            if centroids is not None and centroids is not hit[1].centroids:
+                hit[1].centroids.copy_(centroids)
             hit[0].replay()
             r = KMeansResult()
             for f in ("centroids", "assign", "counts", "offsets", "members"):
                 setattr(r, f, getattr(hit[1], f))
-            if centroids is not None:
-                r.centroids = centroids
         else:
             _SEEN[gkey] = True
             while len(_SEEN) > 64:

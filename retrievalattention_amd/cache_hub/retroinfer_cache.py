@@ -22,7 +22,7 @@ import torch
 
 from .. import kernels
 from .cache import KV_Cache
-from .kmeans import segment_k_means_csr, csr_to_dense
+from .kmeans import initial_centroids, segment_k_means_csr, csr_to_dense
 
 # generated tokens are folded into the index every THRESHOLD_LENGTH steps
 THRESHOLD_LENGTH = 1024
@@ -158,7 +158,7 @@ class retroinfer_cache(KV_Cache):
         self._plans = {}                         # (layer, buffer) -> DecodeStepPlan of the device-resident step
         self._row_shape = (batch_size, 1, self.kv_head, self.head_dim)
         self._out_shape = (batch_size, 1, self.num_heads, self.head_dim)
-        self._centred_keys = {}                  # (device, tokens, clusters) -> the clustering's keys and centroids
+        self._centred_keys = {}                  # (device, tokens) -> buffer of centred keys for the clustering
         if self.kv_residency == "device":
             self._init_device_store()
         else:
@@ -362,17 +362,14 @@ class retroinfer_cache(KV_Cache):
 
         # the centred keys go to a buffer that keeps its address from call to call: the clustering of
         # every further layer and sequence of this length then replays one captured graph
-        buffers = (dkey, valid_length, self.n_centroids)
-        ck, cc = self._centred_keys.get(buffers, (None, None))
+        ck = self._centred_keys.get((dkey, valid_length))
         if ck is None:
             if len(self._centred_keys) >= 2:
                 self._centred_keys.clear()
-            both = torch.empty((H * (valid_length + self.n_centroids), head_dim), dtype=keys.dtype, device=keys.device)
-            ck, cc = (x.view(H, -1, head_dim) for x in both.split((H * valid_length, H * self.n_centroids)))
-            self._centred_keys[buffers] = ck, cc
+            ck = torch.empty((H, valid_length, head_dim), dtype=keys.dtype, device=keys.device)
+            self._centred_keys[(dkey, valid_length)] = ck
         mean_key = kernels.prefill_mean(keys, lo, valid_length)
-        if mean_key is None:
-            cc = None
+        cc = None if mean_key is None else initial_centroids(ck, self.n_centroids, 10, self.n_segment, cpu_organise)
         kernels.prefill_split(keys, values, lo, valid_length, vs, sps, seq_len - spe, spe, ck,
                               self.steady_zone_keys[layer_idx][batch_idx], self.steady_zone_values[layer_idx][batch_idx],
                               mean_key, cc)

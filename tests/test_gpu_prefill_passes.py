@@ -215,3 +215,33 @@ def test_prefill_mean_leaves_other_shapes(dev):
     from retrievalattention_amd import kernels
     assert kernels.prefill_mean(torch.empty((40, 33, 128), dtype=torch.bfloat16, device=dev), 0, 40) is None
     assert kernels.prefill_mean(torch.empty((262145, 1, 128), dtype=torch.bfloat16, device=dev), 0, 262145) is None
+
+
+@pytest.mark.parametrize("residency", ["device", "host-cpu"])
+def test_captured_clusterings_serve_the_caches_that_follow(dev, residency):
+    """Layers of two caches in a row, launched, captured and replayed, with initial centroids in the captured clustering's own
+    tensor, against prefills of which each is launched kernel by kernel."""
+    from retrievalattention_amd.cache_hub import kmeans
+    from tests.test_gpu_cache import _gen, _make_cache
+    layers, ctx = 3, 2500 + 68
+    K, V = _gen(layers, 2, 2, 4, ctx, 64, dev, 3)
+
+    def prefilled(b, captured):
+        cache = _make_cache(dev, residency, layers, 1, 2, 4, ctx, 96, 1, 8, 16)
+        for layer in range(layers):
+            if not captured:
+                kmeans._GRAPHS.clear(), kmeans._SEEN.clear()
+            cache.prefill_update_kv_cache(None, K[layer][b], V[layer][b], layer, 0)
+            cache.sync(layer, 0)
+        torch.cuda.synchronize()
+        if residency != "device":
+            cache.prepare_cache()
+        return [[x[layer].clone() for x in (cache.centroids, cache.value_sum, cache.cluster_size_i32, cache.cluster_start,
+                                            cache.list_keys, cache.list_values)] for layer in range(layers)]
+    kmeans._GRAPHS.clear(), kmeans._SEEN.clear()
+    for b in range(2):
+        for got, want in zip(prefilled(b, True), prefilled(b, False)):
+            rows = int(want[2][0].sum())
+            for x, y in zip(got, want):
+                x, y = (t[..., :rows, :] if t.dim() == 4 else t for t in (x, y))
+                assert torch.equal(x, y)

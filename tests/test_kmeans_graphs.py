@@ -37,9 +37,10 @@ def test_a_captured_clustering_is_replayed_for_its_own_kind_of_call(monkeypatch,
     assert len(launched) == 3 and len(replayed) == 2
 
 
-def test_a_captured_clustering_keeps_no_buffer_of_its_caller(monkeypatch):
-    """Initial centroids that the caller hands over are the result's, by their address: neither they nor the keys stay alive with
-    the graph, and other ones are another clustering."""
+def test_a_captured_clustering_is_found_by_its_keys_alone(monkeypatch):
+    """Initial centroids that the caller hands over become a captured clustering's own, and later calls for the same keys are told
+    to use them: a caller that comes after another one, with keys at the same address, replays at once.  Other ones are copied.
+    The keys do not stay alive with the graph."""
     import weakref
     monkeypatch.setattr(kmeans, "_GRAPHS", kmeans.collections.OrderedDict())
     monkeypatch.setattr(kmeans, "_SEEN", kmeans.collections.OrderedDict())
@@ -50,11 +51,20 @@ def test_a_captured_clustering_keeps_no_buffer_of_its_caller(monkeypatch):
     monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: SimpleNamespace(replay=lambda: replayed.append(1)))
     monkeypatch.setattr(torch.cuda, "graph", lambda g: contextlib.nullcontext())
     monkeypatch.setattr(kernels, "kmeans_value_sum", lambda *a, **k: None)
-    key, centroids, other = (torch.zeros(1, 64, 128, dtype=torch.bfloat16) for _ in range(3))
-    call = lambda c: kmeans.segment_k_means_csr(key, key, 64, reuse_graph=True, centroids=c)
-    for _ in range(3):
-        assert call(centroids).centroids is centroids
-    assert len(replayed) == 2 and call(other).centroids is other and len(replayed) == 2
-    held = weakref.ref(centroids)
-    del centroids
+    key = torch.zeros(1, 64, 128, dtype=torch.bfloat16)
+    own = lambda: kmeans.initial_centroids(key, 64)
+    call = lambda c: kmeans.segment_k_means_csr(key, key, 64, reuse_graph=True, centroids=c).centroids
+    first, second = own(), own()
+    assert first is not second and first.shape == (1, 64, 128) and first.dtype == key.dtype
+    assert call(first) is first and call(second) is second and len(replayed) == 1   # launched; captured and replayed
+    assert own() is second and call(own()) is second and len(replayed) == 2
+    other = torch.ones(1, 64, 128, dtype=torch.bfloat16)
+    assert call(other) is second and len(replayed) == 3 and torch.equal(second, other)
+    for change in (dict(num_iters=9), dict(num_segments=2), dict(final_means=False)):
+        assert kmeans.initial_centroids(key, 64, **change) is not second
+    assert kmeans.initial_centroids(key, 32) is not second
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert own() is not second
+    held = weakref.ref(key)
+    del key
     assert held() is None
