@@ -198,8 +198,8 @@ __global__ __launch_bounds__(NT, NT / 256) void select_attend_kernel(ri_ptr4 in,
 template <int NT, int E, int SRC>
 static void launch_select_attend(const SelectArgs& S, const AttendParams& A, int BG, bool half, hipStream_t stream) {
   const void* a = SRC == SEL_KEYS ? (const void*)S.keys : (const void*)S.logits;
-  // (sixteen heads: up to 512 threads; more than 8192 clusters in so few: sixteen heads)
-  constexpr int LEAST = NT == 512 && E == 32 ? 16 : 4, MOST = NT == 512 ? 16 : 8;
+  // (sixteen heads: up to 512 threads, and no logits past 2048 clusters; more than 8192 clusters in so few: sixteen heads)
+  constexpr int LEAST = NT == 512 && E == 32 ? 16 : 4, MOST = NT == 512 && !(SRC == SEL_LOGITS && E == 8) ? 16 : 8;
   constexpr int G4 = LEAST > 4 ? LEAST : 4, G8 = LEAST > 8 ? LEAST : 8, G16 = MOST;
   auto* kernel = S.gs <= 4   ? (half ? select_attend_kernel<NT, E, G4, true, SRC> : select_attend_kernel<NT, E, G4, false, SRC>)
                  : S.gs <= 8 ? (half ? select_attend_kernel<NT, E, G8, true, SRC> : select_attend_kernel<NT, E, G8, false, SRC>)
@@ -254,15 +254,7 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
   }
-  // Who sums the scores (dist_kernel / the selecting workgroups, captured layers with their appends, us): 32 groups of 4 heads, 8192
-  // clusters 44.8 / 47.6, 5632 36.1 / 38.7, 4096 29.5 / 29.2; 8 of 4, 5632 24.3 / 26.5; of 1, 32 of 8192 42.9 / 44.0; 8 of 16, 2048 26.0 / 25.9;
-  // 64 of 16, 1024 28.8 / 27.6; 12 of 7, 1920 23.0 / 22.0; 32 of 8, 2048 25.7 / 24.7. Between 2048 and
-  // 4096 clusters: 8 of 7, 2304 19.6 / 20.4, 2816 20.6 / 21.2; 8 of 8, 3328 21.6 / 22.3, 32 of 8, 2304 24.2 / 25.0, 2816 24.9 / 25.7, 64 of 8, 2816 31.8 / 32.5;
-  // 2 of 7, 2560 19.3 / 20.5, 64 of 7, 2560 30.1 / 30.9; but 16 of 5, 2560 20.8 / 20.8, 128 of 6, 3104 52.8 / 52.4. More groups fill
-  // the chip with selecting workgroups, and the second launch is not made up for: 128 of 7, 2304 42.7 / 42.3, 2816 51.8 / 50.7, 3328
-  // 56.9 / 56.7, of 8, 2304 43.9 / 43.6, 2816 52.2 / 52.5; 64 of 7, 2304 29.9 / 29.7.
-  // (512 threads: eight clusters each past 2048, and with sixteen heads that is more than the registers hold.)
-  const bool keys = S.nc > (S.gs <= 6 || s->BG > 64 ? 4096 : s->BG > 48 ? 2432 : 2048);
+  const bool keys = step_sums_apart(S.gs, s->BG, S.nc);
   rc = ri_launch_select_inputs(S, s->BG, s->half, keys, stream);
   if (rc) return rc;
   if (wide) {

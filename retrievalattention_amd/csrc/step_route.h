@@ -58,6 +58,22 @@ static inline bool step_is_joined(const ri_decode_step_t* s) {
   return step_is_wide(s) || (s->np <= 512 && (s->gs <= 8 || 3 * s->np + s->es <= 8000));
 }
 
+// Who sums the scores of a step that is scored before: dist_kernel, which then hands keys over, or the workgroups that select, from
+// the logits.  dist_kernel / the selecting workgroups, captured layers with their appends, us:
+//  * Up to six heads dist_kernel past 4096 clusters: 32 groups of 4 heads, 8192 44.8 / 47.6, 5632 36.1 / 38.7, 4096 29.5 / 29.2; 8 of 4, 5632
+//    24.3 / 26.5; of 1, 32 of 8192 42.9 / 44.0; 16 of 5, 2560 20.8 / 20.8, 128 of 6, 3104 52.8 / 52.4.
+//  * Seven and eight heads past 2048 in up to 64 groups: 12 of 7, 1920 23.0 / 22.0, 32 of 8, 2048 25.7 / 24.7; 8 of 7, 2304 19.6 / 20.4, 8 of 8,
+//    3328 21.6 / 22.3, 32 of 8, 2816 24.9 / 25.7; 56 of 7, 2304 27.7 / 28.1, 3840 34.7 / 35.5, 64 of 7, 2304 28.9 / 29.5, 3328 36.4 / 37.0, 64 of
+//    8, 2304 29.8 / 30.4, 3840 37.4 / 38.2.  In more groups they fill the chip with selecting workgroups, and the second launch is made up
+//    for no longer: 80 of 7, 2304 33.1 / 33.7, 3328 40.4 / 40.0, 72 of 8, 3840 41.6 / 41.6, 96 of 7, 2816 45.1 / 45.0, of 8 42.9 / 42.7, 112 of
+//    7 47.9 / 47.3, 128 of 8 52.3 / 52.0, 3840 59.9 / 59.5, 192 of 7, 3328 78.9 / 78.4, 256 of 8, 2816 90.8 / 90.0, 3840 111.3 / 110.4.
+//  * More heads past 2048 in any number of groups: 8 of 16, 2048 26.0 / 25.9, 64 of 16, 1024 28.8 / 27.6; 56 of 9, 2304 30.6 / 33.7, of 12, 2816
+//    37.1 / 40.8, of 16, 4096 43.0 / 46.7, 72 of 9, 4096 47.1 / 48.5, of 16, 2816 43.7 / 47.0, 128 of 9, 2304 47.6 / 49.3, of 12, 3328 63.0 /
+//    65.5, of 16, 4096 78.0 / 80.0.  (Eight clusters of sixteen heads to a thread are 157 registers and 118 KB of LDS.)
+static inline bool step_sums_apart(int gs, int BG, int nc) {
+  return nc > (gs > 8 ? 2048 : gs > 6 && BG <= 64 ? 2048 : 4096);
+}
+
 // Of the short steps those that one workgroup per group holds its own in. Past 128 groups there is no second one, and it makes them; up
 // to them several that leave few rows to one of them (step_kernel, by step_alone_rows) are ahead everywhere and make all, inside
 // these lines too, which nothing but their test asks for any more. Captured layers with their appends, us, one / several: 8 groups of 4 heads, 512

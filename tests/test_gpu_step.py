@@ -105,7 +105,11 @@ def test_joined_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, stati
     # who sums the scores: on both sides of 2048 clusters for seven and eight heads, of 4096 for six, with 1024 selecting threads too
     (2, 7, 2048, 36, 475, 69, 300, False), (2, 7, 2056, 36, 475, 69, 300, True), (3, 8, 2056, 600, 300, 69, 4000, False),
     (2, 6, 2056, 37, 470, 69, 300, False), (2, 6, 4096, 73, 950, 69, 600, False), (2, 6, 4104, 73, 950, 69, 600, True),
-    (49, 7, 2432, 36, 475, 69, 300, True), (49, 7, 2440, 36, 475, 69, 300, True), (65, 8, 4096, 73, 950, 69, 600, False)])
+    (49, 7, 2432, 36, 475, 69, 300, True), (49, 7, 2440, 36, 475, 69, 300, True), (65, 8, 4096, 73, 950, 69, 600, False),
+    # of 2048 for more than eight heads in many groups too, and for eight in up to 64
+    (65, 16, 2048, 36, 475, 69, 300, False), (65, 16, 2056, 36, 475, 69, 300, False), (65, 9, 4096, 73, 950, 69, 600, True),
+    (49, 12, 2432, 43, 560, 69, 300, False), (130, 10, 2064, 37, 478, 69, 300, True), (64, 8, 2056, 37, 476, 69, 300, False),
+    (65, 8, 2056, 37, 476, 69, 300, False)])
 def test_joined_step_at_the_line_of_the_sums(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
     test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device)
 

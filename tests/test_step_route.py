@@ -86,6 +86,17 @@ def test_captured_steps_of_many_groups_keep_one_workgroup_for_longer(is_alone):
     assert is_alone(5000, BG=129)
 
 
+def test_who_sums_the_scores(tmp_path_factory):
+    """Clusters up to which the selecting workgroups sum the scores themselves, by the heads and the groups.  More than eight heads
+    have dist_kernel past 2048 clusters in any number of groups: eight clusters of sixteen heads to a thread are no form of
+    the kernel's."""
+    apart = _compiled(tmp_path_factory, "(int gs, int groups, int nc) { return step_sums_apart(gs, groups, nc); }")
+    for gs in range(1, 17):
+        for groups in (1, 8, 48, 49, 64, 65, 128, 129, 256, 4096):
+            line = 2048 if gs > 8 or (gs > 6 and groups <= 64) else 4096
+            assert not apart(gs, groups, line) and apart(gs, groups, line + 8), (gs, groups)
+
+
 def test_arrival_counters_have_lines_of_their_own(tmp_path_factory):
     """Eight counters a group for the up to 128 groups that have more than one workgroup, in 4096 words: a line of 128 bytes each up
     to 16 groups, half a line up to 32."""
