@@ -231,8 +231,8 @@ static void launch_step(const SelectArgs& S, const AttendParams& A, int BG, bool
                                                        A);
 }
 
-// The step in one launch (nc <= STEP_CLUSTERS, up to eight heads), or in scoring and one more.
-static int step_joined(const ri_decode_step_t* s, const void* q, int static_len, bool alone, void* out, hipStream_t stream) {
+// The step in one launch (nc <= STEP_CLUSTERS), or in scoring, perhaps the scores' sums, and one more.
+static int step_joined(const ri_decode_step_t* s, const void* q, int static_len, bool one, void* out, hipStream_t stream) {
   SelectArgs S;
   int rc = ri_prepare_select(&S, q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,
                              s->ret_ids, s->est_ids, s->ret_tok_off, s->ret_start, nullptr, 0, s->meta, s->BG, s->gs, s->nc,
@@ -245,11 +245,11 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
                                  s->store_v, s->store_stride, nullptr, 0, s->ret_tok_off, s->ret_start, s->np, s->meta,
                                  s->est_ids, s->es > 0 ? s->logits : nullptr, nullptr, s->value_sum, s->cluster_size, out,
                                  s->valid_lengths, s->BG, s->gs, s->nc, s->es, s->scale, s->attn_workspace,
-                                 s->attn_workspace_bytes, alone ? ATT_ONE : S.nc <= STEP_CLUSTERS && S.gs <= 8 ? ATT_SEVERAL : ATT_PLAN);
+                                 s->attn_workspace_bytes, one ? ATT_ONE : S.nc <= STEP_CLUSTERS && S.gs <= 8 ? ATT_SEVERAL : ATT_PLAN);
   if (rc) return rc;
   if (S.nc <= STEP_CLUSTERS) {
     if (S.gs > 8) launch_score_attend(S, A, s->BG, s->half, stream);
-    else if (alone) launch_step<false>(S, A, s->BG, s->half, stream);
+    else if (one) launch_step<false>(S, A, s->BG, s->half, stream);
     else launch_step<true>(S, A, s->BG, s->half, stream);
     RI_HIP_CHECK_LAUNCH();
     return RI_OK;
@@ -275,10 +275,7 @@ static int step_joined(const ri_decode_step_t* s, const void* q, int static_len,
 
 extern "C" int ri_decode_step(const ri_decode_step_t* s, const void* q, int static_len, void* out, ri_stream_t stream) {
   if (!s) return RI_ERR_ARG;
-  if (step_is_joined(s)) {
-    const bool one = step_is_short(s, static_len) && s->BG > 128;   // (figures at step_is_alone)
-    return step_joined(s, q, static_len, one, out, (hipStream_t)stream);
-  }
+  if (step_is_joined(s)) return step_joined(s, q, static_len, step_is_one(s, static_len), out, (hipStream_t)stream);
   auto* select = s->half ? ri_score_select_f16 : ri_score_select;
   auto* attend = s->half ? ri_wave_attention_f16 : ri_wave_attention;
   const int rc = select(q, s->centroids, s->mask, s->cluster_size_i32, s->cluster_start, s->logits, nullptr, nullptr,

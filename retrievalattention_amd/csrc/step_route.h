@@ -1,5 +1,5 @@
-// Which decode steps one workgroup per group makes in one launch (step_kernel), which several do, and which are scoring +
-// selection and attention in launches of their own; where an attention's workgroups count their arrivals.  Host code only.
+// Which decode steps are one launch (step_kernel), of one or of several workgroups per group, which are two or three, and which are
+// scoring + selection and attention in launches of their own; where an attention's workgroups count their arrivals.  Host code only.
 #pragma once
 #include <stdint.h>
 
@@ -18,36 +18,11 @@ static inline bool attend_alone(int64_t rows, int gs, int BG) { return rows * gs
 // 13.8 / 12.4, 1 of 8, 40000 18.0 / 16.5, 8 of 8, 20000 21.2 / 19.3, 6 of 8, 3000 9.4 / 9.1; half a line the same.
 static constexpr int attend_counter_pitch(int BG) { return BG <= 16 ? 32 : BG <= 32 ? 16 : BG <= 64 ? 8 : 4; }
 
-// Short: what one workgroup may have to itself.  It scores for itself (select.hip), and usually (16
-// tokens per retrieved cluster) has no more rows than it attends as fast as scoring + selection and attention in launches of their own
-// do.  Captured layers with their appends, us, by the rows, one workgroup / in launches of their own: 8 groups of 8 heads 391 rows 18.4 / 19.2,
-// 451 19.0 / 19.0, 521 20.2 / 19.2; of 4 heads 451 18.1 / 18.0, 521 18.8 / 18.2; one group of 8 heads 451 17.9 / 18.1, 521 19.8 / 18.4.
-// The rows are not known here when the kernel reads the zone's length from the device, as a captured step does until the
-// zone is full, and never what the retrieved clusters hold:
-//  * Where the attention by itself would be one workgroup per group all the same, one launch is faster whatever they turn
-//    out to be.  Captured with 331 rows, then 331, 762 and 1354: 8 groups of 4 heads 16.4, 20.8, 26.8 / 18.1, 22.3, 28.5, 128 groups
-//    19.0, 26.4, 35.4 / 20.9, 28.6, 39.1; with 64 tokens in each of 9 clusters (763 rows) 20.5 / 21.9 and 24.6 / 26.9.
-//  * Elsewhere the other route has more workgroups, so the rows that the zone can hold decide, and those of the clusters are
-//    bounded by the page limit and the store.  8 groups of 8 heads captured with 331 rows: then 17.8 / 18.8, at 458 rows 19.6 / 19.6,
-//    but at 762 23.2 / 19.8, 1062: 25.8 / 20.9, 1354: 30.0 / 22.3; with 64 tokens in each of 9 clusters 22.7 / 20.3.  At twice the limit
-//    the most crowded clusters cost what usual ones save.
 #define STEP_CLUSTERS 512
-#define STEP_ROWS 448
-#define STEP_ROWS_CROWDED (2 * STEP_ROWS)
-static inline bool step_is_short(const ri_decode_step_t* s, int static_len) {
-  if (s->nc > STEP_CLUSTERS || s->gs > 8 || s->BG > 256 || !s->cluster_size_i32 || !s->cluster_start) return false;
-  const int64_t usual = (int64_t)s->np * 16 + s->es;
-  if (static_len + usual > STEP_ROWS) return false;
-  if (attend_alone(static_len + usual, s->gs, s->BG)) return true;
-  const int64_t zone = s->static_len_dev ? s->steady_stride : static_len;
-  const int64_t pages = (int64_t)s->max_pages * s->page, held = pages < s->store_stride ? pages : s->store_stride;
-  return zone + usual <= STEP_ROWS && zone + s->es + held <= STEP_ROWS_CROWDED;
-}
-
 // Selection and attention in one launch, and the scoring too up to STEP_CLUSTERS: what step.hip's kernels hold.  (A probe per
 // thread; 512 threads, or wide 1024, whose registers do not hold sixteen heads; up to 32 clusters a thread; with sixteen heads
-// 32 KB of LDS are left for the tables, of which those of up to 512 clusters take 8; without sizes and first rows there are none.  A workgroup that scores has a compute unit
-// to itself: 264 groups of 4 heads, 512 clusters, a captured layer 33.2 us in two launches, 36.4 in one.)
+// 32 KB of LDS are left for the tables, of which those of up to 512 clusters take 8; without sizes and first rows there are none.  A
+// workgroup that scores has a compute unit to itself: 264 groups of 4 heads, 512 clusters, a captured layer 33.2 us in two launches, 36.4 in one.)
 static inline bool step_is_wide(const ri_decode_step_t* s) {
   return s->gs <= 8 && s->np <= 1024 && (s->nc > 8192 || s->np > 512);
 }
@@ -74,20 +49,21 @@ static inline bool step_sums_apart(int gs, int BG, int nc) {
   return nc > (gs > 8 ? 2048 : gs > 6 && BG <= 64 ? 2048 : 4096);
 }
 
-// Of the short steps those that one workgroup per group holds its own in. Past 128 groups there is no second one, and it makes them; up
-// to them several that leave few rows to one of them (step_kernel, by step_alone_rows) are ahead everywhere and make all, inside
-// these lines too, which nothing but their test asks for any more. Captured layers with their appends, us, one / several: 8 groups of 4 heads, 512
-// clusters 13.85 / 13.35; of 1, 104 11.65 / 11.40; of 8, 256 13.30 / 12.90; 88 of 1, 120 12.10 / 11.85; 24 of 1, 104 11.95 / 11.65; 16 of 4, 256 12.35 /
-// 12.10; 32 of 4, 496 13.75 / 13.40; 128 of 4, 496 15.20 / 14.90, of 8, 256 14.10 / 13.70; 1 of 4, 320 11.90 / 11.60.
-// A captured step starts at the length at hand and ends at the zone's, and may grow past the line. Earlier kernels, zones of 69 to 323 rows, us a layer
-// at the first length, on average and at the last, several | one: 16 groups of 4 heads, up to 508 rows 15.6, 16.7, 17.7 | 15.8, 17.2, 18.8;
-// 32 of 4, 508 16.6, 17.8, 18.4 | 16.8, 18.3, 19.9; 64 of 4, 477 16.5, 17.8, 18.8 | 16.6, 18.0, 19.4; 32 of 8, 446 16.4, 18.1, 19.1 | 16.7, 18.4,
-// 20.2; 40 of 2, 477 16.1, 17.2, 18.1 | 16.4, 17.8, 19.2.  Past the line 24 of 4, 531 16.7, 17.4, 18.4 | 16.7, 18.3, 19.9; 64 of 4, 554 17.5, 18.6,
-// 19.2 | 17.4, 19.1, 20.5; 8 of 4, 477 15.2, 16.2, 17.3 | 15.5, 16.7, 18.2.
-static inline int step_alone_rows(int BG) { return BG > 64 ? 640 : 336; }
-static inline int step_alone_end(int BG) { return BG > 64 ? 800 : BG >= 16 ? 512 : 420; }
-static inline bool step_is_alone(const ri_decode_step_t* s, int static_len) {
-  if (s->BG > 128) return true;
-  const int64_t usual = (int64_t)s->np * 16 + s->es, zone = s->static_len_dev ? s->steady_stride : static_len;
-  return static_len + usual <= step_alone_rows(s->BG) && zone + usual <= step_alone_end(s->BG);
+// Steps that score for themselves, of up to eight heads (step_kernel).  Up to 128 groups several workgroups per group make them.
+// Captured layers with their appends, us, one / several: 8 groups of 4 heads, 512 clusters 13.85 / 13.35; of 1, 104 11.65 / 11.40; of 8, 256
+// 13.30 / 12.90; 88 of 1, 120 12.10 / 11.85; 16 of 4, 256 12.35 / 12.10; 32 of 4, 496 13.75 / 13.40; 128 of 4, 496 15.20 / 14.90, of 8, 256
+// 14.10 / 13.70; 1 of 4, 320 11.90 / 11.60.  Past 128 there is no second one, and where the usual 16 tokens to a cluster make no more than STEP_ROWS
+// rows the kernel's form for one, which knows of no other, makes them: form for several / for one 136 groups of 4 heads, 96 clusters 12.4 / 12.3,
+// 256 13.35 / 13.15, of 8, 512 17.7 / 17.6; 192 of 8, 256 15.4 / 15.1; 256 of 4, 256 15.65 / 15.4, of 8, 512 22.6 / 22.4.
+#define STEP_ROWS 448
+static inline bool step_is_one(const ri_decode_step_t* s, int static_len) {
+  return s->BG > 128 && step_is_joined(s) && s->nc <= STEP_CLUSTERS && s->gs <= 8 &&
+         static_len + (int64_t)s->np * 16 + s->es <= STEP_ROWS;
 }
+
+// Rows up to which one of several workgroups attends them all and the others leave (step_kernel looks behind the selection, where
+// a captured step's length and what the clusters hold are known).  Earlier kernels' captured layers with their appends, us, by the rows, several
+// that all work / that leave: 8 groups of 4 heads, 192 clusters 161 16.0 / 14.8, 281 16.2 / 15.6, 411 16.0 / 16.1; 8 of 8, 320 223 16.9 / 15.8,
+// 343 16.9 / 16.7; 32 of 4, 512 331 17.4 / 17.6.  With two workgroups per group only: 128 groups of 4 heads, 512 331 20.1 / 18.9, 581 22.4 /
+// 22.3, of 8 331 21.0 / 19.9, 581 23.0 / 22.9.
+static inline int step_alone_rows(int BG) { return BG > 64 ? 640 : 336; }

@@ -29,11 +29,17 @@ def test_append_kv(dev, BG, stride, pos, on_device):
     (5, 8, 256, 4, 60, 70, 2, True), (4, 3, 264, 10, 100, 69, 100, False), (8, 4, 512, 9, 118, 98, 100, False),
     (2, 7, 504, 12, 150, 100, 3, True), (256, 2, 16, 2, 3, 5, 100, False), (257, 2, 16, 2, 3, 5, 100, False),
     (2, 4, 512, 13, 118, 98, 100, False), (2, 4, 512, 13, 118, 98, 40, False), (3, 8, 512, 9, 118, 98, 72, False),
-    (3, 8, 512, 9, 118, 98, 76, True)])
+    (3, 8, 512, 9, 118, 98, 76, True),
+    # one workgroup per group, past 128 groups: heads padded and not, every number of waves that score, no estimation zone, cut
+    # pages, the zone's length from the device, and both sides of 448 rows
+    (129, 1, 8, 1, 0, 0, 100, False), (129, 5, 40, 7, 33, 17, 100, False), (256, 7, 64, 2, 20, 69, 1, True),
+    (200, 8, 256, 4, 0, 70, 100, False), (256, 3, 128, 2, 30, 300, 100, True), (130, 8, 512, 9, 118, 98, 100, True),
+    (129, 8, 264, 13, 118, 122, 100, False), (129, 8, 264, 13, 118, 123, 100, False), (160, 4, 104, 18, 0, 160, 3, True),
+    (160, 4, 104, 18, 0, 161, 3, True)])
 def test_short_step_equals_the_operators(dev, dtype, BG, gs, nc, np_, es, static, pages, on_device):
-    """The step that one workgroup per group makes (and, past its limits, the launches one by one) against scoring +
-    selection and attention called by themselves: the same lists; outputs differ only where those split a group's rows,
-    by roundings of the 16-bit probabilities and of the output, each at most 2^-8 of a value (2^-11 in half), of which a
+    """The step in one launch, of several workgroups per group up to 128 groups and of one past them (and, past its limits, the
+    launches one by one), against scoring + selection and attention called by themselves: the same lists; outputs differ
+    only where the rows of a group are split in another way, by roundings of the 16-bit probabilities and of the output, each at most 2^-8 of a value (2^-11 in half), of which a
     norm over the output sees a fraction."""
     from retrievalattention_amd import kernels
     g = torch.Generator().manual_seed(BG * nc + gs)

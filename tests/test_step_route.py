@@ -1,5 +1,5 @@
-"""Which decode steps one workgroup per group makes, and where arrivals are counted (csrc/step_route.h, host code: compiled here by
-g++)."""
+"""Which decode steps one workgroup per group makes, who sums the scores of others, and where arrivals are counted
+(csrc/step_route.h, host code: compiled here by g++)."""
 import ctypes
 import os
 import shutil
@@ -23,67 +23,31 @@ def _compiled(tmp_path_factory, function):
     return ctypes.CDLL(str(where / "route.so")).ask
 
 
-def _route(tmp_path_factory, name):
-    call = _compiled(tmp_path_factory, f"(const ri_decode_step_t* s, int n) {{ return step_{name}(s, n); }}")
+@pytest.fixture(scope="module")
+def is_one(tmp_path_factory):
+    """What ri_decode_step asks: whether the kernel's form for one workgroup per group makes the step."""
+    call = _compiled(tmp_path_factory, "(const ri_decode_step_t* s, int n) { return step_is_one(s, n); }")
 
-    def short(static_len, zone=323, on_device=False, BG=8, gs=4, nc=512, np=9, es=118, page=8, max_pages=72, store=8192,
-              sizes=True):
+    def one(static_len, zone=323, on_device=False, BG=129, gs=4, nc=512, np=9, es=118, page=8, max_pages=72, store=8192,
+            sizes=True):
         step = DecodeStep(BG=BG, gs=gs, nc=nc, np=np, es=es, page=page, max_pages=max_pages, steady_stride=zone,
                           store_stride=store, static_len_dev=1 if on_device else None,
                           cluster_size_i32=1 if sizes else None, cluster_start=1 if sizes else None)
         return bool(call(ctypes.byref(step), static_len))
-    return short
-
-
-@pytest.fixture(scope="module")
-def is_short(tmp_path_factory):
-    return _route(tmp_path_factory, "is_short")
-
-
-@pytest.fixture(scope="module")
-def is_alone(tmp_path_factory):
-    return _route(tmp_path_factory, "is_alone")
-
-
-def test_limits(is_short):
-    assert is_short(98) and is_short(98, gs=8)
-    assert not is_short(98, nc=520) and not is_short(98, gs=9) and not is_short(98, BG=257) and not is_short(98, sizes=False)
-    assert is_short(186) and not is_short(187)                      # 448 rows
-    assert is_short(186, BG=256) and not is_short(187, BG=256)
+    return one
 
 
 @pytest.mark.parametrize("gs", [1, 4, 5, 8])
-def test_length_on_the_device_grows_to_the_zone(is_short, gs):
-    """A captured step serves every length up to the zone's: only where the attention by itself would have one workgroup
-    as well (384 rows of up to four heads, 192 of eight, more than 128 groups) does the length at hand decide."""
-    alone = gs <= 4
-    for zone in (69 + 256, 69 + 1024):
-        assert is_short(69, zone=zone, on_device=True, gs=gs) == alone
-        assert is_short(122, zone=zone, on_device=True, gs=gs) == alone
-        assert not is_short(123, zone=zone, on_device=True, gs=gs)
-        assert is_short(123, zone=zone, on_device=False, gs=gs)
-        assert is_short(123, zone=zone, on_device=True, gs=gs, BG=129)
-    assert is_short(123, zone=186, on_device=True, gs=gs) and not is_short(123, zone=187, on_device=True, gs=gs)
-    assert is_short(69, zone=1093, on_device=True, gs=gs, nc=128, np=2, es=30)
-
-
-@pytest.mark.parametrize("gs", [4, 8])
-def test_clusters_may_hold_what_the_page_limit_lets_them(is_short, gs):
-    at = 170   # 432 rows if the clusters have their usual size
-    assert is_short(at, gs=gs, max_pages=76) and not is_short(at, gs=gs, max_pages=77)     # 896 rows at most
-    assert is_short(at, gs=gs, max_pages=1 << 30, store=608) and not is_short(at, gs=gs, max_pages=1 << 30, store=609)
-    assert is_short(at, gs=gs, max_pages=1 << 30, BG=129)
-    assert is_short(98, gs=gs, max_pages=1 << 30) == (gs == 4)
-
-
-def test_captured_steps_of_many_groups_keep_one_workgroup_for_longer(is_alone):
-    """Which short steps one workgroup per group makes: by the rows at hand, and captured ones by the zone's too."""
-    for BG, line, end in ((1, 336, 420), (15, 336, 420), (16, 336, 512), (64, 336, 512), (65, 640, 800), (128, 640, 800)):
-        assert is_alone(line - 90, BG=BG, np=4, es=26) and not is_alone(line - 89, BG=BG, np=4, es=26)
-        assert is_alone(69, zone=end - 90, on_device=True, BG=BG, np=4, es=26)
-        assert not is_alone(69, zone=end - 89, on_device=True, BG=BG, np=4, es=26)
-        assert not is_alone(line - 89, zone=end - 90, on_device=True, BG=BG, np=4, es=26)
-    assert is_alone(5000, BG=129)
+def test_steps_that_one_workgroup_per_group_makes(is_one, gs):
+    """Those of 129 to 256 groups, up to 512 clusters and eight heads, with up to 448 rows by the length at hand and the usual
+    size of a cluster: the zone's end, pages and the store do not matter.  Up to 128 groups there are several workgroups."""
+    assert not any(is_one(at, BG=BG, gs=gs) for at in (0, 69, 186) for BG in (1, 8, 64, 65, 128))
+    for BG in (129, 200, 256):
+        assert is_one(0, BG=BG, gs=gs) and is_one(186, BG=BG, gs=gs) and not is_one(187, BG=BG, gs=gs)
+        assert is_one(186, BG=BG, gs=gs, zone=9000, on_device=True, max_pages=1 << 30, store=1 << 40)
+        assert is_one(400, BG=BG, gs=gs, np=1, es=32) and not is_one(401, BG=BG, gs=gs, np=1, es=32)
+        assert not is_one(98, BG=BG, gs=gs, nc=520) and not is_one(98, BG=BG, gs=gs, sizes=False)
+    assert not is_one(98, gs=9) and not is_one(98, BG=257, gs=gs)
 
 
 def test_who_sums_the_scores(tmp_path_factory):
