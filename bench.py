@@ -69,10 +69,12 @@ def measured_traffic(config, kernels):
 def attending_launches(cfg):
     """The launches of a step over a device-resident store from the selection on, as the library makes them for the
     configurations below: one for the whole step with few clusters (then the scoring is in it too), else one behind the
-    scoring, in front of which the scores are summed by a launch of their own where there are many."""
+    scoring, in front of which the scores are summed by a launch of their own where there are many (step_sums_apart in
+    csrc/step_route.h)."""
     if cfg["nc"] <= 512:
         return ["step_kernel"]
-    return (["dist_kernel"] if cfg["nc"] > 4096 else []) + ["select_attend_kernel"]
+    own = 2048 if cfg["gs"] > 8 or (cfg["gs"] > 6 and cfg["B"] * cfg["Hkv"] <= 64) else 4096
+    return (["dist_kernel"] if cfg["nc"] > own else []) + ["select_attend_kernel"]
 
 
 def drift_cycles(steps, layers):

@@ -24,7 +24,7 @@ def test_drifting_queries_are_timed_in_whole_rounds_of_their_pool():
 def test_traffic_is_of_the_launches_that_the_step_makes(monkeypatch, tmp_path):
     """Recorded for every launch of a step's attention, and on the sources at hand, or not reported."""
     assert bench.attending_launches(bench.CONFIGS["c1"]) == ["step_kernel"]
-    assert bench.attending_launches(bench.CONFIGS["c4"]) == ["select_attend_kernel"]
+    assert bench.attending_launches(bench.CONFIGS["c4"]) == ["dist_kernel", "select_attend_kernel"]
     assert bench.attending_launches(bench.CONFIGS["c2"]) == ["dist_kernel", "select_attend_kernel"]
     entry = lambda k: dict(fetch_kib=1000.0, fetch_scale=2.0, write_kib=24.0, write_scale=1.0, source="here",  # noqa: E731
                            kernel_source_sha256_16=bench.kernel_source_hash(k))

@@ -7,6 +7,7 @@ import subprocess
 
 import pytest
 
+import bench
 from retrievalattention_amd._lib import DecodeStep
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -59,6 +60,9 @@ def test_who_sums_the_scores(tmp_path_factory):
         for groups in (1, 8, 48, 49, 64, 65, 128, 129, 256, 4096):
             line = 2048 if gs > 8 or (gs > 6 and groups <= 64) else 4096
             assert not apart(gs, groups, line) and apart(gs, groups, line + 8), (gs, groups)
+            for nc in (520, 2048, 2056, 4096, 4104, 16384):   # the launches that the benchmark names
+                cfg = dict(B=groups, Hkv=1, gs=gs, nc=nc)
+                assert bench.attending_launches(cfg) == ["dist_kernel"] * apart(gs, groups, nc) + ["select_attend_kernel"]
 
 
 def test_arrival_counters_have_lines_of_their_own(tmp_path_factory):
