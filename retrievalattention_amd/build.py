@@ -1,5 +1,5 @@
-"""Builds libretro_mi355.so (HIP kernels + host wave buffer) for gfx950 with hipcc, and _step_calls.so (the calls of a decode
-step from Python) with g++.
+"""Builds libretro_mi355.so (HIP kernels + host wave buffer) for gfx950, the C example over it and _step_calls.so (the calls of a
+decode step from Python), all with hipcc.
 
     python -m retrievalattention_amd.build
 
@@ -59,8 +59,8 @@ def build(verbose=False):
                 print(o)
     objs = [j[1] for j in jobs]
     _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB] + objs + ["-pthread"])
-    _run(step_calls_command())
     build_capi_example(hipcc)
+    _run(step_calls_command(hipcc))   # (last: it alone needs torch's headers)
     return LIB
 
 
@@ -69,12 +69,12 @@ def build(verbose=False):
 STEP_CALLS = os.path.join(HERE, "_step_calls.so")
 
 
-def step_calls_command():
+def step_calls_command(hipcc):
     import torch
     from torch.utils import cpp_extension
-    include = [f"-I{d}" for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    include = [x for d in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]] for x in ("-isystem", d)]
     libs = [f"-L{d}" for d in cpp_extension.library_paths("cuda") + [HERE]]
-    return ["g++", *CPP_FLAGS, "-O2", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    return [hipcc, *CPP_FLAGS, "-Wall", "-shared", "-no-hip-rt", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *include,
             os.path.join(CSRC, "step_calls.cpp"), "-o", STEP_CALLS, *libs, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
             "-lc10_hip", "-l:libretro_mi355.so", "-Wl,-rpath,$ORIGIN"]
