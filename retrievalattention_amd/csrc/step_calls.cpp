@@ -215,9 +215,9 @@ void* address(const at::Tensor* t) { return t ? t->data_ptr() : nullptr; }
 bool integers(PyObject* const* args, int n, int64_t* out) {
   for (int i = 0; i < n; ++i) {
     if (!PyLong_Check(args[i])) return false;
-    out[i] = PyLong_AsLongLong(args[i]);
-    if (PyErr_Occurred()) throw python_error();
-    if (out[i] < 0 || out[i] > INT32_MAX) return false;
+    int over;
+    out[i] = PyLong_AsLongLongAndOverflow(args[i], &over);
+    if (over || out[i] < 0 || out[i] > INT32_MAX) return false;
   }
   return true;
 }
@@ -242,7 +242,10 @@ PyObject* gemm_softmax(PyObject*, PyObject* const* args, Py_ssize_t n) {
       !holds(t[4], bc, tiles, m) || !holds(t[5], bc, tiles, m))
     Py_RETURN_NONE;
   const double alpha = PyFloat_AsDouble(args[10]), beta = PyFloat_AsDouble(args[11]);
-  if (PyErr_Occurred()) return nullptr;
+  if (PyErr_Occurred()) {   // (float() takes more)
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
   void* p[6];
   for (int i = 0; i < 6; ++i) p[i] = address(t[i]);
   const ri_stream_t stream = current_stream();

@@ -176,3 +176,20 @@ def test_operators_natively_and_in_general(dev, dtype):
         assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
     with pytest.raises(ValueError):
         kernels.batch_gemm_softmax(q, cent, product, norm[:1], total, softmax, BG, gs, n, 128)
+
+
+@pytest.mark.gpu
+def test_numbers_that_the_native_call_does_not_take(dev):
+    """What float() takes and PyFloat does not goes the general way; sizes past 64 bits are refused as sizes past the buffers are."""
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(s, dtype=dt, device=dev)  # noqa: E731
+    a, b = z(1, 2, 128) + 1, z(1, 8, 128) + 1
+    out = []
+    for alpha, beta in ((0.5, 0.0), ("0.5", "0")):
+        out.append(z(1, 2, 8))
+        kernels.batch_gemm_softmax(a, b, out[-1], z(1, 1, 2, dt=torch.float32), z(1, 1, 2, dt=torch.float32), z(1, 2, 8), 1, 2, 8,
+                                   128, alpha, beta)
+    assert torch.equal(*out) and float(out[0][0, 0, 0]) == 64.0
+    for m, n in ((1 << 70, 8), (2, 1 << 70), (1 << 40, 8)):
+        with pytest.raises(ValueError):
+            kernels.batch_gemm_softmax(a, b, out[0], z(1, 1, 2, dt=torch.float32), z(1, 1, 2, dt=torch.float32), z(1, 2, 8), 1, m, n,
+                                       128)
