@@ -546,7 +546,7 @@ int ri_lru_stage_update(const ri_lru_t* lru, ri_stream_t stream);
 
 /* The decode step of one layer over a host-resident store with the device-side block cache (compute(),
  * cache_hub/retroinfer_cache.py:549-697): what ri_score_select and ri_lru_access do (selection and look-up in
- * one launch where a thread has one probe and the selection sums the scores), ri_lru_stage_update,
+ * one launch up to 4096 clusters, 2048 with more than eight heads, and 1023 probes, up to 512 clusters 255 or 511), ri_lru_stage_update,
  * ri_wave_attention over the row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`,
  * store_k / store_v are the cache tensors of `lru` and ret_tok_off, ret_start, cluster_start are not used. */
 int ri_host_step(const ri_decode_step_t* step, const ri_lru_t* lru, const void* q, int static_len, void* out,
@@ -622,8 +622,8 @@ int ri_kmeans_init(const void* data, void* centroids, int P, int N, int nc, ri_s
    of every head from tokens start0.., the following n_end from tokens end0..  Strides in elements, multiples of 8.
    ri_prefill_center: keys[h][i] -= mean[h], in the element type.
    ri_prefill_mean: mean[h] = the mean of key[first .. first + N - 1][h], summed in fp32 in a fixed order; the sum times 1 / N
-   is rounded to half, or to fp32 and then to bfloat16: the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144 tokens, and 2 GiB of them together; beyond that
-   ri_prefill_mean_workspace_bytes is 0 and the call refuses.
+   is rounded to half, or to fp32 and then to bfloat16: the bits torch.mean(keys, dim=1) gives.  Up to 32 heads and 262144
+   tokens, and 2 GiB of them together; beyond that ri_prefill_mean_workspace_bytes is 0 and the call refuses.
    ri_prefill_split_centred: ri_prefill_split with mean[h] taken off the rows of keys, as ri_prefill_center does.
    ri_prefill_split_init: ri_prefill_split_centred, with what ri_kmeans_init gives for the rows of keys in centroids [H, nc, 128].
    ri_prefill_index: out = centroids + mean, mask = (count == 0), sizes as elements and as int32, first rows. */

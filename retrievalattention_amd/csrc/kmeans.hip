@@ -1296,7 +1296,8 @@ __global__ __launch_bounds__(KM_BUCKET_WAVES * 64) void km_bucket_kernel(
 // starting from block 0's.  One wave per block, lane l owns dims 2l and 2l+1.  Lists of at
 // most KM_BLK rows (nearly all of them) are finished by their own wave.  A longer list (the first
 // Lloyd iterations produce a few huge ones) is split into its blocks, which other waves of the same
-// launch sum in parallel, and a second, small launch adds the block sums in order.
+// launch sum in parallel; who adds the block sums in order is a second, small launch, or, in a clustering's
+// later updates whose passes know nothing of each other, the wave whose block is the last to arrive.
 //
 // Which wave sums which block needs no queue and no counter: block j of a long list that starts at
 // list offset o owns slot 2 * (o / KM_BLK) + j of its problem.  Two long lists never share a slot (a
@@ -1365,9 +1366,11 @@ __device__ __forceinline__ void km_sum_rows(const uint32_t* __restrict__ rp, con
 // The same sum without copies: sixty-four rows in flight at any time, each register
 // requested again as soon as its row is added, ids a round ahead, rows by buffer offsets (bytes within 31 bits: km_reduce).  A
 // round that is requested, waited for and added 32 rows at a time leaves a wave waiting for most of a block, and costs more than
-// the waves that its fewer registers make room for.  Updates over given lists, us, rounds / ahead, an early and a late iteration: 1 x 22198
-// tokens, 800 clusters 15.1, 9.8 / 9.8, 7.7; 2 x 20124, 448 16.1, 13.6 / 10.9, 9.6; 2 x 44152, 1536 20.0, 15.4 / 15.0, 10.4; 4 x 65536, 2048 25.0, 24.3
-// / 21.8, 19.4; 8 x 131072, 8192 59.0, 63.2 / 55.4, 60.3 (4.9 TB/s).
+// the waves that its fewer registers make room for (72 to 82; five to a SIMD where seven were).  Updates over given lists, us, rounds /
+// ahead, an early and a late iteration: 1 x 22198 tokens, 800 clusters 15.1, 9.8 / 9.8, 7.7; 2 x 20124, 448 16.1, 13.6 / 10.9, 9.6; 2 x
+// 44152, 1536 20.0, 15.4 / 15.0, 10.4; 4 x 65536, 2048 25.0, 24.3 / 21.8, 19.4; 4 x 131072, 8192 37.3, 34.3 / 34.4, 32.6; 8 x 131072, 4096
+// 58.6, 56.2 / 55.0, 51.7; 8 x 200000, 8192 101.7, 100.8 / 98.8, 97.1.  Where the launch is at the memory's rate they are level: 8 x 131072, 8192
+// 61.2, 63.5 / 57.5, 65.8, and on average over a clustering of them 56.3 / 56.7 (keys), 68.4 / 67.0 (values).
 template <bool HALF>
 __device__ __forceinline__ void km_sum_rows_ahead(__amdgpu_buffer_rsrc_t rows, uint32_t row_bytes, const int32_t* mem, int k0, int k1,
                                                   float& s0, float& s1) {
@@ -1572,7 +1575,7 @@ __device__ __forceinline__ void km_entry(const KmIndex& X, size_t at, int size, 
 
 // grid (item workgroups + ceil(nc / 4), P), four waves each.  The first item_wgs workgroups take
 // one slot per wave (blocks of long lists, their fp32 sums go to partial[p][slot]); the others one
-// cluster per wave.
+// cluster per wave.  arrived: words that the blocks of a long list are counted in, the last of which finishes it (null: a launch does).
 // COPY (sums of value rows): every row is also written where its list puts it, row off + k of problem p to
 // copy + (p * copy_stride + off + k) * 128: the cluster-contiguous store, without a second pass over the rows.
 // AHEAD (without copies): sums by km_sum_rows_ahead.
@@ -1664,7 +1667,7 @@ __device__ __forceinline__ void km_reduce_rows(const uint16_t* __restrict__ rows
     else if (CENTER && X.out) km_entry<HALF>(X, (size_t)p * nc + c, s, o, *op, mw);
     return;
   }
-  if (s > KM_BLK) return;  // summed by the slot waves, finished by km_reduce_fold_kernel
+  if (s > KM_BLK) return;  // summed by the slot waves, finished by the last of them (arrived) or by km_reduce_fold_kernel
   float s0 = 0.f, s1 = 0.f;
   sum(o, 0, s, s0, s1);
   const uint32_t word = km_finish<MEAN, HALF>(s0, s1, s, normalize, op, M.state ? M.odd + p : nullptr);

@@ -221,7 +221,9 @@ static void launch_heads(const SelectArgs& P, const ri_lru_t& L, int BG, bool ha
   else launch_access<NT, E, 16, SRC>(P, L, BG, half, s);
 }
 
-// The selection's forms are those of ri_score_select, as far as it makes the scores' sums itself; a thread has one rank.
+// The selection's forms are those of ri_score_select where it makes the scores' sums itself, up to four clusters to a thread: 4096
+// clusters, 2048 with more than eight heads (with up to four heads ri_score_select sums further).  A thread has one rank, and
+// one thread at least has none: up to 255, 511 or 1023 probes.  *taken tells the caller of the rest to launch both halves apart.
 int ri_launch_select_access(const SelectArgs& P, const ri_lru_t& L, int BG, bool half, bool* taken, hipStream_t s) {
   *taken = false;
   const int nc = P.nc, np = P.np;

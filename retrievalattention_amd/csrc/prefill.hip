@@ -179,9 +179,9 @@ extern "C" int ri_prefill_mean_f16(const void* key, int64_t key_row_stride, int6
 // and V.  16 lanes per row, a workgroup moves 16 rows of one head: occupancy keeps more loads in flight than several rows
 // per thread do (8 heads of 8K / 128K tokens: 6.7 / 93 us; two or four rows per thread 19 / 105).  Heads vary fastest over
 // the workgroups, so those in flight together read whole tokens.  Workgroups behind the clustered range move the steady
-// rows, and those behind them the rows that a clustering starts from, which is a launch less in front of it (prefills, us, with a
-// launch of their own / as it is: 4 heads x 50021 tokens in half 581.3 / 579.1, 8 x 131072 3192.0 / 3185.5; short ones 153.2 / 151.5, 241.4 /
-// 239.1).
+// rows, and those behind them the rows that a clustering starts from, which is a launch less in front of it, most of which the split
+// takes longer where they are many (split + that launch / as it is: 8 heads x 8192 tokens 6.1 + 2.9 / 6.3 us, 8 x 131072 81.6 + 8.5 / 87.4;
+// prefills 219 / 216, 4 x 50021 in half 575 / 574, 8 x 16384 377 / 372).
 // ------------------------------------------------------------------------------------
 struct SplitParams {
   const uint4* k;

@@ -53,7 +53,6 @@ struct SelectArgs {
 // Barrier over LDS traffic only: global stores issued before it stay in flight (__syncthreads waits for them as well).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-
 // lanes whose bit K and bit D are equal: those that keep the larger value of an exchange over 2^D in a merge of 2^K
 constexpr uint64_t keep_mask(int K, int D) {
   uint64_t m = 0;
