@@ -546,8 +546,8 @@ int ri_lru_stage_update(const ri_lru_t* lru, ri_stream_t stream);
 
 /* The decode step of one layer over a host-resident store with the device-side block cache (compute(),
  * cache_hub/retroinfer_cache.py:549-697): what ri_score_select and ri_lru_access do (selection and look-up in
- * one launch up to 4096 clusters, 2048 with more than eight heads, and 1023 probes, up to 512 clusters 255 or 511), ri_lru_stage_update,
- * ri_wave_attention over the row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`,
+ * one launch up to 4096 clusters, 2048 with more than eight heads, and up to 1023 probes, 255 with 256 clusters, 511 with
+ * 512), ri_lru_stage_update, ri_wave_attention over the row table and ri_gather_copy_and_scatter of the admitted blocks.  In `step`,
  * store_k / store_v are the cache tensors of `lru` and ret_tok_off, ret_start, cluster_start are not used. */
 int ri_host_step(const ri_decode_step_t* step, const ri_lru_t* lru, const void* q, int static_len, void* out,
                  ri_stream_t stream);
